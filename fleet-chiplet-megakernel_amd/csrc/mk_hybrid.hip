@@ -396,20 +396,30 @@ __device__ __forceinline__ void stage_hy_route(CStage &st, Ctx &c, int M, char *
 }
 
 // ----------------------------------------------------------------------------- experts
-// Weights of an expert are operand tiles (see stage_mx_head_linear); a unit is a pair of 16-row tiles of one expert over all
-// tokens that visit it.  Few units: a workgroup per unit, its wavefronts split the reduction; many: a wavefront per unit.  MK_F_SILU: the pair is gate and up of the same 16 outputs, out =
-// silu(gate) up.  Expert e < num_experts takes row (token, s) of `in` where s is its place among the token's choices (ld_in_slot 0:
-// the token's one row) and writes row (token, s) of `out`; the shared expert has its own sizes and place topk.
-// st.n / n_shared: rows of a matrix (gate and up together), st.k / k_shared: reduction length (whole operand rows).
-// Units of the shared expert come first: they have the most tokens, and their weights are known before the routing is.
+// Weights of an expert are operand tiles (see stage_mx_head_linear); a unit is a pair of 16-row tiles of one expert over at most 16 of
+// the tokens that visit it.  MK_F_SILU: the pair is gate and up of the same 16 outputs, out = silu(gate) up.  Expert e < num_experts
+// takes row (token, s) of `in` where s is its place among the token's choices (ld_in_slot 0: the token's one row) and writes row
+// (token, s) of `out`; the shared expert has its own sizes and place topk.  st.n / n_shared: rows of a matrix (gate and up together),
+// st.k / k_shared: reduction length (whole operand rows).
+//
+// The stage is bound by streaming the weights.  Units are numbered expert by expert (the shared one first) and a workgroup takes a
+// contiguous range, so that a wavefront reads one contiguous stream per tile and share of the reduction, and the token rows of an
+// expert are staged in LDS once for all the units of it: between two units of a range the wavefronts issue nothing but weight
+// requests, a ring of D steps x 2 tiles that never drains (64 KB per CU at D = 8; 128 KB gained nothing).  The wavefronts split
+// the reduction, so a workgroup's share is balanced to one unit; sums meet in LDS, double-buffered, one workgroup barrier per unit.
+// Token rows read from L2 inside the loop had tied every step to a round trip behind the weights.  Before -> now, gate/up and down: 64
+// experts of 1536 on rows of 4096, 64 tokens 371 -> 268 and 175 -> 150 us (1.6 GB at 6.1 TB/s, 0.8 GB at 5.5), one token 64.7 -> 45.2
+// and 35.1 -> 26.4 us; 128 experts of 768 on rows of 2048, 16 tokens 91 -> 68 and 50 -> 42 us.
 struct HyLists {
-  unsigned long long tok[MK_MOE_MAX_EXPERTS];  // tokens that visit the expert
-  int active[MK_MOE_MAX_EXPERTS];
-  int n_active;
-  int pad[3];
-  unsigned char place[MK_MOE_MAX_EXPERTS][MK_MAX_TOKENS];
+  unsigned long long tok[MK_MOE_MAX_EXPERTS];   // tokens that visit the expert
+  unsigned short entry[896];                    // expert | group of tokens << 8: one entry per `rows that fit` tokens of an expert
+  int n_entries, pad[15];
+  unsigned place[MK_MOE_MAX_EXPERTS][MK_MAX_TOKENS / 8];  // place of the expert among a token's choices, 4 bits each
 };
-static_assert(sizeof(HyLists) <= MK_OUT_OFFSET, "the lists lie below the scratch of the routing and of the reduction");
+constexpr int HY_X = (sizeof(HyLists) + 63) / 64 * 64;            // staged token rows [16-byte word of the row][row]
+constexpr int HY_RED = MK_LDS_BYTES - 2 * MK_WAVES * 2 * 64 * 16; // partial sums of two units
+static_assert(HY_X <= MK_OUT_OFFSET && HY_RED - HY_X >= 128 * 1024, "16 rows of 8 KB fit; the routing's scratch is free by then");
+static_assert(MK_MOE_MAX_EXPERTS + MK_MAX_TOKENS * MK_MOE_MAX_TOPK / 2 <= 896 && MK_MOE_MAX_TOPK <= 16 && MK_MOE_MAX_EXPERTS <= 256, "entries with at least two rows each");
 template <typename E>
 __device__ __forceinline__ float hy_glu(E, CStage &st, bool shared, float a, float b) {
 #if MK_HAVE_DUAL
@@ -420,194 +430,285 @@ __device__ __forceinline__ float hy_glu(E, CStage &st, bool shared, float a, flo
 #endif
   return hy_silu(E(), a) * b;
 }
-template <typename E, int MT, bool SPLIT>
-__device__ __forceinline__ void hy_expert_unit(CStage &st, const HyLists *ls, bool shared, int e, int pair, unsigned long long toks, int n, int K, int wave, int lane,
-                                               const u32x4 *W, const u32x4 (&first)[2][4], f32x4 *red) {
-  constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW, KB = 4;
+// rows that LDS holds of one entry (at most 16: the columns of a matrix instruction); fewer than two: rows are read from memory
+template <typename E>
+__device__ __forceinline__ int hy_rows(int K) { return min(16, (HY_RED - HY_X) / (K * (int)sizeof(E))); }
+
+// What a workgroup walks: units [s0, s1) of the shared expert (gs groups of tokens, units_s each), then units [r0, r1) of the entries
+// (`units` each).
+struct HyRange {
+  int s0, s1, r0, r1, gs, units_s, units;
+};
+// The u-th unit of a range: D steps of the reduction are a block.
+struct HyUnit {
+  const u32x4 *w0, *w1;  // this lane's operands of the two tiles
+  int nks, kb, ke, nb;   // steps of the reduction, this wavefront's share of them, blocks it takes (alike for all wavefronts)
+  int i, pair, n;        // entry (negative: a group of the shared expert), pair of tiles (may lie behind the last one), outputs
+};
+template <typename E, int D>
+__device__ __forceinline__ HyUnit hy_unit(CStage &st, const HyLists *ls, const HyRange &rg, int u, int ks, int wave, int lane) {
+  HyUnit a;
+  const int ksl = ks == 4 ? 2 : ks - 1, ns = rg.s1 - rg.s0;  // (log2 of ks)
+  const bool shared = u < ns;
+  const int v = shared ? rg.s0 + u : rg.r0 + u - ns, per = shared ? rg.units_s : rg.units, q = v / per;
+  a.pair = ((v - q * per) << (2 - ksl)) + (wave >> ksl);
+  a.i = shared ? q - rg.gs : q;
+  a.n = shared ? st.n_shared : st.n;
+  a.nks = (shared ? st.k_shared : st.k) / FxType<E>::KW;
+  const int kq = (a.nks + ks - 1) >> ksl, p = (a.n + 31) / 32;
+  a.kb = min(a.nks, (wave & (ks - 1)) * kq);
+  a.ke = min(a.nks, a.kb + kq);
+  a.nb = (kq + D - 1) / D;
+  const int e = shared ? 0 : __builtin_amdgcn_readfirstlane(ls->entry[q]) & 255;
+  a.w0 = (shared ? (const u32x4 *)st.w_shared : (const u32x4 *)st.w.seg[0]) + ((size_t)e * p + min(a.pair, p - 1)) * 2 * a.nks * 64 + lane;
+  a.w1 = a.w0 + (size_t)a.nks * 64;
+  return a;
+}
+constexpr int HY_FIRST = 8;  // steps of the ring that may have been requested in advance
+
+// Walk the units of `rg`.  ks wavefronts (4, 2 or 1) split the reduction of a pair of tiles.  w: the ring, its first steps requested if
+// `early`.  row_words: 16-byte words per row where all rows of a single token lie in LDS (row of place p at p * row_words; 0: one row).
+template <typename E, int D, bool XLDS>
+__device__ __forceinline__ void hy_expert_walk(CStage &st, const HyLists *ls, int M, const HyRange rg, int ks, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
+  constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const bool glu = st.flags & MK_F_SILU;
-  const int lr = lane & 15, lg = lane >> 4, nks = K / KW, kq = SPLIT ? (nks + MK_WAVES - 1) / MK_WAVES : nks, kb = SPLIT ? min(nks, wave * kq) : 0, ke = min(nks, kb + kq);
-  const int cnt = __popcll(toks);
-  // lane r gets the r-th token of the list
-  const int mine = (toks >> lane) & 1 ? __popcll(toks & ((1ull << lane) - 1ull)) : 63;
-  int nth = __builtin_amdgcn_ds_permute(mine << 2, lane);  // (lane 63 may receive several: it is only read when the list holds 64)
-  if (cnt == 64) nth = lane;
-  int tok[MT], place[MT];
-  const E *xr[MT];
+  u32x4 *xl = (u32x4 *)(smem + HY_X);
+  f32x4 *red = (f32x4 *)(smem + HY_RED);
+  const int ns = rg.s1 - rg.s0, n_all = ns + rg.r1 - rg.r0;
+  HyUnit a = hy_unit<E, D>(st, ls, rg, 0, ks, wave, lane);
 #pragma unroll
-  for (int m = 0; m < MT; m++) {
-    tok[m] = __builtin_amdgcn_ds_bpermute(min(m * 16 + lr, cnt - 1) << 2, nth);
-    place[m] = shared ? st.topk : ls->place[e][tok[m]];
-    xr[m] = (const E *)st.in + (size_t)tok[m] * st.ld_in + (size_t)place[m] * st.ld_in_slot + lg * EPC;
-  }
-  f32x4 acc[2][MT];
-#pragma unroll
-  for (int h = 0; h < 2; h++)
-#pragma unroll
-    for (int m = 0; m < MT; m++) acc[h][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  const u32x4 *w0 = W + (size_t)(2 * pair) * nks * 64 + lane, *w1 = w0 + (size_t)nks * 64;
-  u32x4 a[2][KB];
-#pragma unroll
-  for (int h = 0; h < 2; h++)
-#pragma unroll
-    for (int q = 0; q < KB; q++) a[h][q] = first[h][q];
-  for (int k0 = kb; k0 < ke; k0 += KB) {
-    u32x4 an[2][KB], b[KB][MT];
-#pragma unroll
-    for (int q = 0; q < KB; q++)
-#pragma unroll
-      for (int m = 0; m < MT; m++) b[q][m] = *(const u32x4 *)(xr[m] + (size_t)min(k0 + q, nks - 1) * KW);
-#pragma unroll
-    for (int q = 0; q < KB; q++) {
-      an[0][q] = ldg_stream(w0 + (size_t)min(k0 + KB + q, nks - 1) * 64);
-      an[1][q] = ldg_stream(w1 + (size_t)min(k0 + KB + q, nks - 1) * 64);
+  for (int j = 0; j < D; j++)
+    if (j >= HY_FIRST || !early) {
+      w[0][j] = ldg_stream(a.w0 + (size_t)min(a.kb + j, a.nks - 1) * 64);
+      w[1][j] = ldg_stream(a.w1 + (size_t)min(a.kb + j, a.nks - 1) * 64);
     }
+  int staged = 0x7fffffff, cnt = 1, tok = 0, place = 0;  // rows in LDS belong to this entry; token and place of column lane & 15
+  const E *xr = nullptr;
+  const u32x4 *xb = xl + lg;
+  const int ksl = ks == 4 ? 2 : ks - 1;  // log2
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  for (int u = 0; u < n_all; u++) {
+    if (a.i != staged) {
+      // ---- the unit's token rows
+      staged = a.i;
+      const bool shared = a.i < 0;
+      if (rows_in) {
+        place = shared ? st.topk : a.i;
+        xb = xl + place * row_words + lg;
+      } else {
+        const int en = shared ? (a.i + rg.gs) << 8 : __builtin_amdgcn_readfirstlane(ls->entry[a.i]), e = en & 255, K = a.nks * KW;
+        unsigned long long toks = M >= 64 ? ~0ull : (1ull << M) - 1ull;
+        if (!shared) {
+          const unsigned long long t = ls->tok[e];
+          toks = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)t) | ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(t >> 32)) << 32);
+        }
+        const int per = XLDS ? hy_rows<E>(K) : 16, r0 = (en >> 8) * per;
+        cnt = min(per, __popcll(toks) - r0);
+        // lane r gets the r-th token of the group (lane 63 what is left over)
+        const int rank = (toks >> lane) & 1 ? __popcll(toks & ((1ull << lane) - 1ull)) - r0 : -1;
+        const int nth = __builtin_amdgcn_ds_permute((rank >= 0 && rank < cnt ? rank : 63) << 2, lane);
+        auto token = [&](int r) { return __builtin_amdgcn_ds_bpermute(r << 2, nth); };
+        auto place_of = [&](int t) { return shared ? st.topk : (int)(ls->place[e][t >> 3] >> ((t & 7) * 4) & 15u); };
+        tok = token(min(lr, cnt - 1));
+        place = place_of(tok);
+        xr = (const E *)st.in + (size_t)tok * st.ld_in + (size_t)place * st.ld_in_slot + lg * EPC;
+        xb = xl + lg * cnt + min(lr, cnt - 1);
+        if constexpr (XLDS) {
+          __syncthreads();  // (everybody is done with the rows of the entry before)
+          // word q: 16 bytes 4 b + (q & 3) of row r, (b, r) = q / 4 in steps of the grid: four lanes read 64 bytes of a row, and what a wavefront
+          // stores is one contiguous piece of LDS
+          const int total = cnt * (a.nks << 2), dr = (MK_THREADS / 4) % cnt, db = (MK_THREADS / 4) / cnt;
+          int r = (tid >> 2) % cnt, b = (tid >> 2) / cnt;
+          for (int q0 = 0; q0 < total; q0 += 8 * MK_THREADS) {
+            u32x4 v[8];
+            int at[8];
 #pragma unroll
-    for (int q = 0; q < KB; q++)
+            for (int z = 0; z < 8; z++) {
+              const bool in = q0 + z * MK_THREADS + tid < total;
+              const int t = token(in ? r : 0), j = in ? 4 * b + (tid & 3) : 0;
+              at[z] = in ? j * cnt + r : -1;
+              v[z] = *(const u32x4 *)((const E *)st.in + (size_t)t * st.ld_in + (size_t)place_of(t) * st.ld_in_slot + j * EPC);
+              r += dr;
+              b += db;
+              if (r >= cnt) {
+                r -= cnt;
+                b++;
+              }
+            }
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const u32x4 w = k0 + q < ke ? a[h][q] : zero;
-#pragma unroll
-        for (int m = 0; m < MT; m++) acc[h][m] = fx_mma_k(E(), w, b[q][m], acc[h][m]);
+            for (int z = 0; z < 8; z++)
+              if (at[z] >= 0) xl[at[z]] = v[z];
+          }
+          __syncthreads();
+        }
       }
+    }
+    const bool more = u + 1 < n_all;
+    const HyUnit nx = more ? hy_unit<E, D>(st, ls, rg, u + 1, ks, wave, lane) : a;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    for (int blk = 0; blk < a.nb; blk++) {
+      const bool last = blk + 1 == a.nb;
+      const int k0 = a.kb + blk * D;
+      u32x4 b[D];
 #pragma unroll
-    for (int h = 0; h < 2; h++)
+      for (int j = 0; j < D; j++) {
+        const int s = min(k0 + j, a.nks - 1);
+        if constexpr (XLDS) b[j] = xb[s * 4 * cnt];
+        else b[j] = *(const u32x4 *)(xr + (size_t)s * KW);
+      }
+      // what the ring takes next: this unit's block or the first one of the unit behind (behind the range: one line again and again)
+      const u32x4 *p0 = last ? nx.w0 : a.w0, *p1 = last ? nx.w1 : a.w1;
+      const int kn = last ? nx.kb : k0 + D, end = (last ? nx.nks : a.nks) - 1, kl = last && !more ? min(kn, end) : end;
 #pragma unroll
-      for (int q = 0; q < KB; q++) a[h][q] = an[h][q];
-  }
-  if constexpr (SPLIT) {
+      for (int j = 0; j < D; j++) {
+        const bool real = k0 + j < a.ke;
+#pragma unroll
+        for (int h = 0; h < 2; h++) acc[h] = fx_mma_k(E(), real ? w[h][j] : zero, b[j], acc[h]);
+        w[0][j] = ldg_stream(p0 + (size_t)min(kn + j, kl) * 64);
+        w[1][j] = ldg_stream(p1 + (size_t)min(kn + j, kl) * 64);
+      }
+    }
+    // ---- the wavefronts' sums
+    f32x4 *rb = red + (u & 1) * (MK_WAVES * 2 * 64);
+#pragma unroll
+    for (int h = 0; h < 2; h++) rb[(wave * 2 + h) * 64 + lane] = acc[h];
     __syncthreads();
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int m = 0; m < MT; m++) red[((wave * 2 + h) * MT + m) * 64 + lane] = acc[h][m];
-    __syncthreads();
-  }
-  auto total = [&](int h, int m) {
-    if constexpr (!SPLIT) return acc[h][m];
-    else return red[(h * MT + m) * 64 + lane] + red[((2 + h) * MT + m) * 64 + lane] + red[((4 + h) * MT + m) * 64 + lane] + red[((6 + h) * MT + m) * 64 + lane];
-  };
-#pragma unroll
-  for (int m = 0; m < MT; m++) {
+    const f32x4 *rw = rb + (wave >> ksl << ksl) * 2 * 64 + lane;
+    auto total = [&](int h) {
+      f32x4 v = rw[h * 64];
+      for (int q = 1; q < ks; q++) v += rw[(2 * q + h) * 64];
+      return v;
+    };
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      if ((SPLIT && ((2 * m + h) & (MK_WAVES - 1)) != wave) || m * 16 + lr >= cnt || (glu && h)) continue;
-      const f32x4 v = total(h, m);
+      if (((2 * u + h) & (ks - 1)) != (wave & (ks - 1)) || lr >= cnt || (glu && h) || a.pair * 32 >= a.n) continue;
+      const f32x4 v = total(h);
       float r[4] = {v[0], v[1], v[2], v[3]};
       if (glu) {
-        const f32x4 u = total(1, m);
+        const f32x4 g = total(1);
 #pragma unroll
-        for (int q = 0; q < 4; q++) r[q] = hy_glu(E(), st, shared, r[q], u[q]);
+        for (int q = 0; q < 4; q++) r[q] = hy_glu(E(), st, a.i < 0, r[q], g[q]);
       }
-      fx_stc4((E *)st.out + (size_t)tok[m] * st.ld_out + (size_t)place[m] * st.ld_out_slot, (glu ? pair : 2 * pair + h) * 16 + lg * 4, glu ? n / 2 : n, r);
+      fx_stc4((E *)st.out + (size_t)tok * st.ld_out + (size_t)place * st.ld_out_slot, (glu ? a.pair : 2 * a.pair + h) * 16 + lg * 4, glu ? a.n / 2 : a.n, r);
     }
+    a = nx;
   }
 }
 template <typename E, int MAXM>
 __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char *smem) {
-  constexpr int KW = FxType<E>::KW;
+  constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Ex = st.num_experts, topk = st.topk;
-  const int pairs = (st.n + 31) / 32, pairs_s = st.w_shared ? (st.n_shared + 31) / 32 : 0;
+  // short reductions are split among fewer wavefronts, so that each of them has a ring's worth of steps
+  const int nks = st.k / KW, ks = nks >= 48 ? 4 : nks >= 24 ? 2 : 1, ppu = MK_WAVES / ks;  // pairs of tiles per unit
   HyLists *ls = (HyLists *)smem;
-  f32x4 *red = (f32x4 *)(smem + MK_MOE_OFFSET);
-  struct Unit {
-    int e, pair, K, n;
-    const u32x4 *W;
-  };
-  auto unit = [&](int u) {
-    Unit a;
-    if (u < pairs_s) {
-      a = Unit{-1, u, st.k_shared, st.n_shared, (const u32x4 *)st.w_shared};
-    } else {
-      const int i = (u - pairs_s) / pairs;
-      a.pair = (u - pairs_s) - i * pairs;
-      a.e = __builtin_amdgcn_readfirstlane(ls->active[i]);
-      a.K = st.k;
-      a.n = st.n;
-      a.W = (const u32x4 *)st.w.seg[0] + (size_t)a.e * pairs * 2 * (st.k / KW) * 64;
-    }
-    return a;
-  };
-  u32x4 first[2][4];
-  auto load_first = [&](const Unit &a, bool split) {
-    const int nks = a.K / KW, kq = (nks + MK_WAVES - 1) / MK_WAVES, kb = split ? min(nks, wave * kq) : 0;
-    const u32x4 *w0 = a.W + (size_t)(2 * a.pair) * nks * 64 + lane, *w1 = w0 + (size_t)nks * 64;
+  const int fit = hy_rows<E>(st.k), fit_s = st.w_shared ? hy_rows<E>(st.k_shared) : 16;
+  const bool xlds = fit >= 2 && fit_s >= 2;
+  const int per = xlds ? fit : 16, per_s = xlds ? fit_s : 16;
+  HyRange rg;
+  rg.units = ((st.n + 31) / 32 + ppu - 1) / ppu;
+  rg.units_s = st.w_shared ? ((st.n_shared + 31) / 32 + ppu - 1) / ppu : 0;
+  rg.gs = st.w_shared ? (M + per_s - 1) / per_s : 0;
+  const int n_s = rg.gs * rg.units_s;
+  auto part = [&](int n, int v) { return (int)((long long)n * v / c.G); };
+  // a few tokens: every workgroup takes a share of the shared expert first, whose weights are known before the routing is (many tokens:
+  // its rows would be staged by everybody for a unit or two)
+  const bool deal = M <= 4;
+  rg.s0 = deal ? part(n_s, c.vid) : 0;
+  rg.s1 = deal ? part(n_s, c.vid + 1) : 0;
+  // rows of a single token: all of them in LDS at once
+  const int one_words = max(st.k, st.w_shared ? st.k_shared : 0) / EPC, one_rows = st.ld_in_slot ? topk + (st.w_shared ? 1 : 0) : 1;
+  const bool inline_route = M == 1 && (st.flags & MK_F_MOE_INLINE_TOPK);
+  const bool rows_in = M == 1 && one_rows * one_words * 16 <= (inline_route ? MK_OUT_OFFSET : HY_RED) - HY_X;
+  u32x4 w[2][12];
+  const bool early = rg.s0 < rg.s1 && wave != 0;  // (wavefront 0 polls and routes)
+  if (early) {
+    const HyUnit a = hy_unit<E, HY_FIRST>(st, ls, rg, 0, ks, wave, lane);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      first[0][q] = ldg_stream(w0 + (size_t)min(kb + q, nks - 1) * 64);
-      first[1][q] = ldg_stream(w1 + (size_t)min(kb + q, nks - 1) * 64);
+    for (int j = 0; j < HY_FIRST; j++) {
+      w[0][j] = ldg_stream(a.w0 + (size_t)min(a.kb + j, a.nks - 1) * 64);
+      w[1][j] = ldg_stream(a.w1 + (size_t)min(a.kb + j, a.nks - 1) * 64);
     }
-  };
-  const int u0 = mx_spread(c);
-  const bool early = u0 < pairs_s && wave != 0;
-  if (early) load_first(unit(u0), true);
+  }
+  if (M > 1 || !rows_in) {
+    for (int i = tid; i < Ex; i += MK_THREADS) ls->tok[i] = 0ull;
+    for (int i = tid; i < Ex * (MK_MAX_TOKENS / 8); i += MK_THREADS) ls->place[0][i] = 0u;
+  }
   if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
   // ---- which experts have which tokens
-  for (int i = tid; i < Ex; i += MK_THREADS) ls->tok[i] = 0ull;
-  __syncthreads();
-  if (M == 1 && (st.flags & MK_F_MOE_INLINE_TOPK)) {
-    if (wave == MK_WAVES - 1) {
-      float w;
-      int id;
-      hy_route_wave(st, (const float *)st.moe_logits, lane, w, id, (float *)(smem + MK_OUT_OFFSET));
-      if (lane < topk) {
-        ls->tok[id] = 1ull;
-        ls->place[id][0] = (unsigned char)lane;
+  if (rows_in) {
+    if (wave == 0) {
+      float f = 0.f;
+      int id = 0;
+      if (inline_route) {
+        hy_route_wave(st, (const float *)st.moe_logits, lane, f, id, (float *)(smem + MK_OUT_OFFSET));
+        if (c.vid == 0) hy_route_store(st, 0, lane, f, id);
+      } else if (lane < topk) {
+        id = ldc_i32(st.ids + lane);
       }
-      if (c.vid == 0) hy_route_store(st, 0, lane, w, id);
+      if (lane < topk) ls->entry[lane] = (unsigned short)id;
+    } else {
+      u32x4 *xl = (u32x4 *)(smem + HY_X);
+      const int total = one_rows * one_words;
+      for (int q = tid - 64; q < total; q += MK_THREADS - 64) {
+        const int p = q / one_words, j = q - p * one_words;
+        xl[q] = *(const u32x4 *)((const E *)st.in + (size_t)p * st.ld_in_slot + min(j, (p == topk ? st.k_shared : one_rows == 1 ? one_words * EPC : st.k) / EPC - 1) * EPC);
+      }
     }
+    __syncthreads();
+    rg.r0 = part(topk * rg.units, c.vid);
+    rg.r1 = part(topk * rg.units, c.vid + 1);
   } else {
-    for (int i = tid; i < M * topk; i += MK_THREADS) {
-      const int t = i / topk, id = ldc_i32(st.ids + i);
-      atomicOr(&ls->tok[id], 1ull << t);
-      ls->place[id][t] = (unsigned char)(i - t * topk);
-    }
-  }
-  __syncthreads();
-  if (wave == 0) {
-    int base = 0;
-    for (int q = 0; q < Ex; q += 64) {
-      const bool has = q + lane < Ex && ls->tok[q + lane] != 0ull;
-      const unsigned long long m = __ballot(has);
-      if (has) ls->active[base + __popcll(m & ((1ull << lane) - 1ull))] = q + lane;
-      base += __popcll(m);
-    }
-    if (lane == 0) ls->n_active = base;
-  }
-  __syncthreads();
-  const int n_units = pairs_s + __builtin_amdgcn_readfirstlane(ls->n_active) * pairs;
-  const unsigned long long all = M >= 64 ? ~0ull : (1ull << M) - 1ull;
-  auto walk = [&](auto split, int u, int stride, bool have) {
-    constexpr bool SPLIT = decltype(split)::value;
-    if (u < n_units && !have) load_first(unit(u), SPLIT);
-    for (; u < n_units; u += stride) {
-      const Unit a = unit(u);
-      u32x4 f[2][4];
-#pragma unroll
-      for (int h = 0; h < 2; h++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) f[h][q] = first[h][q];
-      if (u + stride < n_units) load_first(unit(u + stride), SPLIT);
-      const bool shared = a.e < 0;
-      unsigned long long toks = all;
-      if (!shared) {
-        const unsigned long long t = ls->tok[a.e];
-        toks = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)t) | ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(t >> 32)) << 32);
+    if (inline_route) {
+      if (wave == 0) {
+        float f;
+        int id;
+        hy_route_wave(st, (const float *)st.moe_logits, lane, f, id, (float *)(smem + MK_OUT_OFFSET));
+        if (lane < topk) {
+          ls->tok[id] = 1ull;
+          ls->place[id][0] = (unsigned)lane;
+        }
+        if (c.vid == 0) hy_route_store(st, 0, lane, f, id);
       }
-      const int cnt = __popcll(toks);
-      if constexpr (SPLIT) {  // 16 tokens at a time
-        const int rank = (toks >> lane) & 1 ? __popcll(toks & ((1ull << lane) - 1ull)) : -1;
-        for (int g = 0; g < cnt; g += 16) hy_expert_unit<E, 1, true>(st, ls, shared, a.e, a.pair, __ballot(rank >= g && rank < g + 16), a.n, a.K, wave, lane, a.W, f, red);
-      } else if (cnt <= 16) {
-        hy_expert_unit<E, 1, false>(st, ls, shared, a.e, a.pair, toks, a.n, a.K, wave, lane, a.W, f, red);
-      } else {
-        hy_expert_unit<E, 4, false>(st, ls, shared, a.e, a.pair, toks, a.n, a.K, wave, lane, a.W, f, red);
+    } else {
+      for (int i = tid; i < M * topk; i += MK_THREADS) {
+        const int t = i / topk, id = ldc_i32(st.ids + i);
+        atomicOr(&ls->tok[id], 1ull << t);
+        atomicOr(&ls->place[id][t >> 3], (unsigned)(i - t * topk) << ((t & 7) * 4));
       }
     }
-  };
-  if (MAXM == 1 || n_units < 3 * MK_WAVES * c.G) walk(std::true_type{}, u0, c.G, early);
-  else if constexpr (MAXM > 1) walk(std::false_type{}, mx_wave_item(c, wave), c.G * MK_WAVES, false);
+    __syncthreads();
+    if (wave == 0) {
+      int base = 0;
+      for (int q = 0; q < Ex; q += 64) {
+        const int g = q + lane < Ex ? (__popcll(ls->tok[q + lane]) + per - 1) / per : 0;
+        const int end = base + wave_incl_scan(g, lane);
+        for (int i = 0; i < g; i++) ls->entry[end - g + i] = (unsigned short)(q + lane | i << 8);
+        base = wave_bcast(end, 63);
+      }
+      if (lane == 0) ls->n_entries = base;
+    }
+    __syncthreads();
+    const int n_r = __builtin_amdgcn_readfirstlane(ls->n_entries) * rg.units;
+    if (deal) {
+      rg.r0 = part(n_r, c.vid);
+      rg.r1 = part(n_r, c.vid + 1);
+    } else {  // one range over the shared expert's units and the entries'
+      const int u0 = part(n_s + n_r, c.vid), u1 = part(n_s + n_r, c.vid + 1);
+      rg.s0 = min(u0, n_s);
+      rg.s1 = min(u1, n_s);
+      rg.r0 = max(u0 - n_s, 0);
+      rg.r1 = max(u1 - n_s, 0);
+    }
+  }
+  if (rg.s0 < rg.s1 || rg.r0 < rg.r1) {
+    // a ring of 8 steps per tile, or of 12 where a wavefront's share of the reduction is then walked with fewer empty steps
+    const int kq = (nks + ks - 1) / ks;
+    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, ls, M, rg, ks, early, w, false, 0, smem);
+    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    else hy_expert_walk<E, 12, true>(st, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+  }
   c.wrote_through = true;
 }

@@ -374,6 +374,17 @@ def test_experts_alone(dtype, rows, E, top, ff, shared, width):
     pk.finalize()
 
 
+@pytest.mark.parametrize("dtype,rows,E,top,ff,shared,width", [
+    # reductions split among four, two and no wavefronts, rings of 8 and of 12 steps, shares that end inside a block
+    (torch.bfloat16, 1, 5, 3, 768, 800, 1568), (torch.bfloat16, 4, 5, 3, 1536, 1504, 800), (torch.bfloat16, 5, 6, 2, 400, 768, 4096), (torch.float32, 3, 4, 2, 400, 200, 776),
+    # more tokens per expert than fit in LDS at once, experts without any
+    (torch.bfloat16, 64, 2, 1, 96, 64, 4096), (torch.bfloat16, 33, 40, 1, 64, None, 2048), (torch.float32, 64, 3, 2, 48, 40, 2064),
+    # single tokens whose rows do not all fit beside the routing; rows that do not fit in LDS at all
+    (torch.bfloat16, 1, 3, 2, 40, 24, 8192), (torch.float32, 1, 3, 2, 40, 24, 17024), (torch.float32, 18, 3, 2, 17024, 24, 64)])
+def test_experts_long_reductions(dtype, rows, E, top, ff, shared, width):
+    test_experts_alone(dtype, rows, E, top, ff, shared, width)
+
+
 # ---------------------------------------------------------------- whole models
 @BOTH
 @pytest.mark.parametrize("name", ["even", "odd", "wide"])
