@@ -133,6 +133,25 @@ size_t dtype_size(int dt) {
 
 }  // namespace
 
+// What a launch leaves behind, read by the host once the stream is through.
+struct LaunchStatus {
+  unsigned xcd_count[MK_MAX_XCD];
+  unsigned abort_flag, abort_where;
+  MkSched sched;
+};
+// Runs behind every launch: one workgroup puts the outcome in pinned host memory and leaves the barrier state zeroed for the next launch.
+// (Bound by the launch; a memset in front and two pageable copies behind cost 12 + 2 x 13 us per launch on MI355X, this adds about 1.)
+__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out) {
+  const unsigned t = threadIdx.x;
+  if (t < MK_MAX_XCD) out->xcd_count[t] = sync->xcd_count[t];
+  if (t == 32) out->abort_flag = sync->abort_flag;
+  if (t == 33) out->abort_where = sync->abort_where;
+  if (t >= 64 && t < 64 + sizeof(MkSched) / 4) ((unsigned *)&out->sched)[t - 64] = ((const unsigned *)sched)[t - 64];
+  __syncthreads();
+  for (unsigned i = t; i < sizeof(MkSync) / 4; i += blockDim.x) ((unsigned *)sync)[i] = 0u;
+}
+static_assert(sizeof(MkSched) % 4 == 0 && sizeof(MkSched) / 4 <= 192 && sizeof(MkSync) % 4 == 0, "copied word by word");
+
 struct mk_graph {
   mk_config cfg;
   int num_cus = 0;
@@ -156,7 +175,9 @@ struct mk_graph {
   std::string json, program_text;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool launch_pending = false;
-  MkSync *pending_sync = nullptr;  // barrier state of the pending / last launch (the graph's own or the static scratch)
+  LaunchStatus *h_status = nullptr;  // pinned host memory: what the last launch left (mk_launch_done_kernel)
+  hipStream_t launch_stream = nullptr;
+  bool ms_due = false;               // last_ms has not been read from the events yet
   int max_kv_heads = 1, max_qpk = 1;  // over the attention stages
   double last_ms = 0.0;
   int last_nxcd = 0, last_aborted = 0;
@@ -2611,7 +2632,7 @@ int upload_runtime(mk_graph *g) {
   return MK_OK;
 }
 
-// `rt` is the runtime block the kernel receives by value; `cleared_by_caller`: its barrier state has been zeroed already
+// `rt` is the runtime block the kernel receives by value; its barrier state is zero (from its allocation, or the launch before)
 // graphs with flex stages (mk_flex.hip) have kernels of their own; graphs that never run more than one token per iteration
 // use the instantiation for exactly that.  Null: not in this build of the library.
 static const void *kernel_of(const mk_graph *g) {
@@ -2667,37 +2688,35 @@ static const void *kernel_of(const mk_graph *g) {
   return k;
 }
 
-int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler, const MkRuntime *rt = nullptr, bool cleared_by_caller = false) {
+int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler, const MkRuntime *rt = nullptr) {
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending: call mk_wait first");
   HIP_TRY(hipSetDevice(g->cfg.device));
   if (!rt) rt = &g->h_rt;
-  if (!cleared_by_caller) HIP_TRY(hipMemsetAsync(rt->sync, 0, sizeof(MkSync), stream));
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
   HIP_TRY(hipEventRecord(g->ev0, stream));
   HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
   HIP_TRY(hipEventRecord(g->ev1, stream));
   g->launch_pending = true;
-  g->pending_sync = rt->sync;
+  g->launch_stream = stream;
+  g->ms_due = true;
+  hipLaunchKernelGGL(mk_launch_done_kernel, dim3(1), dim3(256), 0, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status);
+  HIP_TRY(hipGetLastError());
   return MK_OK;
 }
 
 int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   if (!g->launch_pending) return fail(MK_ESTATE, "no launch pending");
   HIP_TRY(hipStreamSynchronize(stream));
+  if (stream != g->launch_stream) HIP_TRY(hipStreamSynchronize(g->launch_stream));
   g->launch_pending = false;
-  float ms = 0.f;
-  HIP_TRY(hipEventElapsedTime(&ms, g->ev0, g->ev1));
-  g->last_ms = ms;
-  MkSync hs;
-  HIP_TRY(hipMemcpy(&hs, g->pending_sync ? g->pending_sync : g->d_sync, sizeof(MkSync), hipMemcpyDeviceToHost));
+  const LaunchStatus &hs = *g->h_status;
   int nx = 0;
   for (int i = 0; i < MK_MAX_XCD; i++) nx += hs.xcd_count[i] > 0;
   g->last_nxcd = nx;
   g->last_aborted = hs.abort_flag != 0;
-  MkSched sc;
-  HIP_TRY(hipMemcpy(&sc, g->d_sched, sizeof(MkSched), hipMemcpyDeviceToHost));
+  const MkSched &sc = hs.sched;
   if (finished_out) *finished_out = sc.finished;
   if (hs.abort_flag) {
     // workgroups that unwound mid-stage may have left the split-K and split-KV arrival counters mid-count (their last
@@ -2836,6 +2855,7 @@ int mk_graph_destroy(mk_graph *g) {
   if (g->launch_pending) (void)hipDeviceSynchronize();
   for (void *p : g->allocs) (void)hipFree(p);
   for (void *p : g->host_allocs) free(p);
+  if (g->h_status) (void)hipHostFree(g->h_status);
   if (g->ev0) (void)hipEventDestroy(g->ev0);
   if (g->ev1) (void)hipEventDestroy(g->ev1);
   delete g;
@@ -3198,6 +3218,8 @@ int mk_compile(mk_graph *g) {
   if ((rc = upload_runtime(g))) return rc;
   HIP_TRY(hipEventCreate(&g->ev0));
   HIP_TRY(hipEventCreate(&g->ev1));
+  HIP_TRY(hipHostMalloc((void **)&g->h_status, sizeof(LaunchStatus)));
+  memset(g->h_status, 0, sizeof(LaunchStatus));
   if ((rc = resolve_scratch(g->cfg.device))) return rc;  // set-up is where the static launch scratch's address is looked up
   g->compiled = true;
   return mk_init_requests(g);
@@ -3289,7 +3311,7 @@ int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations) {
   hipLaunchKernelGGL(mk_fill_zero_kernel, dim3(16), dim3(256), 0, (hipStream_t)stream, (uint4 *)base, SS_CLEARED_END / 16);
   HIP_TRY(hipGetLastError());
   const int sched = g->cfg.mode == MK_MODE_OFFLINE ? MK_SCHED_OFFLINE : (g->cfg.mode == MK_MODE_ONLINE ? MK_SCHED_ONLINE : MK_SCHED_FROM_META);
-  return do_launch(g, (hipStream_t)stream, sched == MK_SCHED_FROM_META ? 1 : max_iterations, sched, &rt, true);
+  return do_launch(g, (hipStream_t)stream, sched == MK_SCHED_FROM_META ? 1 : max_iterations, sched, &rt);
 }
 
 int mk_wait(mk_graph *g, void *stream, int *finished_out) {
@@ -3352,6 +3374,12 @@ int mk_get_stats(mk_graph *g, mk_stats *out) {
   out->weight_bytes = g->weight_bytes;
   out->packed_weight_bytes = g->packed_bytes;
   out->row_major_weight_bytes = g->row_major_bytes;
+  if (g->ms_due && !g->launch_pending) {
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, g->ev0, g->ev1));
+    g->last_ms = ms;
+    g->ms_due = false;
+  }
   out->last_launch_ms = g->last_ms;
   if (g->compiled && !g->launch_pending) {
     MkSched sc;

@@ -655,48 +655,48 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // rows [qo_indptr[i], qo_indptr[i+1]) and its sequence, new tokens included, is (pages - 1) * page_size + last_page_len
 // long, so its rows sit at the last positions of that sequence.  Derives the per-row slot / position / first-row arrays
 // on the device (no host round trip, so a serving loop can enqueue launches back to back).  Runs on one thread.
-__device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt) {
+// Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).
+__device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt, int lane) {
   const int R = rt.max_requests, B = rt.max_tokens;
   // A batch the stages cannot run as described is not run at all: truncating a request's rows would leave the rest with
   // the slot / position an earlier launch gave them, and they would append K/V rows to some other request's cache.
-  // bad: 1 = rows outside [0, max tokens), overlapping, or with gaps; 2 = more rows for one request than
-  // max_tokens_per_request; 3 = a sequence shorter than its new rows, longer than max_seq_length, or without pages.
-  int ntok = 0, bad = 0;
-  unsigned long long covered = 0ull;
-  for (int i = 0; i < R && !bad; i++) {
-    const int q0 = rt.qo_indptr[i], n = rt.qo_indptr[i + 1] - q0;
-    if (n <= 0) continue;  // an unused slot (hosts that fill only the first entries leave zeros behind them)
-    if (q0 < 0 || q0 + n > B) {
-      bad = 1;
-      break;
+  // bad, of the first slot that cannot run: 1 = rows outside [0, max tokens), overlapping, or with gaps; 2 = more rows for one
+  // request than max_tokens_per_request; 3 = a sequence shorter than its new rows, longer than max_seq_length, or without pages.
+  const int i = min(lane, R - 1);  // (at most 64 slots)
+  const int q0 = rt.qo_indptr[i], q1 = rt.qo_indptr[i + 1], pages = rt.kv_indptr[i + 1] - rt.kv_indptr[i], last = rt.kv_last_page_len[i];
+  const int n = lane < R ? q1 - q0 : 0;  // (<= 0: an unused slot; hosts that fill only the first entries leave zeros behind them)
+  const int len = (int)((long long)(pages - 1) * rt.page_size) + last;
+  const bool inside = n > 0 && q0 >= 0 && n <= B && q0 <= B - n;
+  const unsigned long long rows = inside ? (n >= 64 ? ~0ull : ((1ull << n) - 1ull)) << q0 : 0ull;
+  unsigned lo = (unsigned)rows, hi = (unsigned)(rows >> 32);  // rows of this slot and those in front of it
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned ul = (unsigned)__builtin_amdgcn_ds_bpermute(((lane - o) & 63) << 2, (int)lo), uh = (unsigned)__builtin_amdgcn_ds_bpermute(((lane - o) & 63) << 2, (int)hi);
+    if (lane >= o) {
+      lo |= ul;
+      hi |= uh;
     }
-    if (n > rt.max_new_per_req) {
-      bad = 2;
-      break;
-    }
-    const unsigned long long rows = (n >= 64 ? ~0ull : ((1ull << n) - 1ull)) << q0;
-    if (covered & rows) {
-      bad = 1;
-      break;
-    }
-    covered |= rows;
-    const int pages = rt.kv_indptr[i + 1] - rt.kv_indptr[i];
-    const int len = (pages - 1) * rt.page_size + rt.kv_last_page_len[i];
-    if (pages < 1 || len < n || len > rt.max_seq) {
-      bad = 3;
-      break;
-    }
+  }
+  const unsigned pl = (unsigned)__builtin_amdgcn_ds_bpermute(((lane - 1) & 63) << 2, (int)lo), ph = (unsigned)__builtin_amdgcn_ds_bpermute(((lane - 1) & 63) << 2, (int)hi);
+  const unsigned long long before = lane ? (unsigned long long)pl | ((unsigned long long)ph << 32) : 0ull;
+  const int why = n <= 0 ? 0 : !inside ? 1 : n > rt.max_new_per_req ? 2 : (before & rows) ? 1 : pages < 1 || len < n || len > rt.max_seq ? 3 : 0;
+  const unsigned long long which = __ballot(why != 0);
+  int bad = which ? wave_bcast(why, (int)__ffsll(which) - 1) : 0;
+  const unsigned long long covered = (unsigned long long)(unsigned)wave_bcast((int)lo, 63) | ((unsigned long long)(unsigned)wave_bcast((int)hi, 63) << 32);
+  int ntok = covered ? 64 - __clzll((long long)covered) : 0;
+  if (covered != (ntok >= 64 ? ~0ull : ((1ull << ntok) - 1ull)) && !bad) bad = 1;
+  if (!bad) {
     for (int j = 0; j < n; j++) {
       rt.tok_slot[q0 + j] = i;
       rt.tok_pos[q0 + j] = len - n + j;
       rt.tok_first[q0 + j] = q0;
     }
-    if (q0 + n > ntok) ntok = q0 + n;
   }
-  if (!bad && covered != (ntok >= 64 ? ~0ull : ((1ull << ntok) - 1ull))) bad = 1;
   if (bad) ntok = 0;
-  rt.sched->bad_batch = bad;
-  rt.sched->num_tokens = ntok;
+  if (lane == 0) {
+    rt.sched->bad_batch = bad;
+    rt.sched->num_tokens = ntok;
+  }
   return ntok;
 }
 
@@ -4446,13 +4446,14 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       // a handful of slots: one thread walks them; more: a wavefront, one lane per slot
       const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && rt.max_requests > 2 && rt.spec_len == 0;
       int ntok_w = 0;
+      const bool from_meta = run_scheduler == MK_SCHED_FROM_META;
       if (c.vid == 0 && threadIdx.x < 64 && wave_sched) ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x);
+      if (c.vid == 0 && threadIdx.x < 64 && from_meta) ntok_w = mk_batch_from_meta(*rtp, threadIdx.x);
       if (c.vid == 0 && threadIdx.x == 0) {
         int ntok;
-        if (wave_sched) ntok = ntok_w;
+        if (wave_sched || from_meta) ntok = ntok_w;
         else if (run_scheduler == MK_SCHED_OFFLINE) ntok = mk_prepare_next_batch(*rtp, (int *)smem);
-        else if (run_scheduler == MK_SCHED_ONLINE) ntok = mk_online_next_batch(*rtp);
-        else ntok = mk_batch_from_meta(*rtp);
+        else ntok = mk_online_next_batch(*rtp);
         if (ntok == 0) rt.sched->finished = 1;
         else rt.sched->iterations++;
         if (rt.timing && rt.sched->iterations <= rt.timing_cap) rt.timing[rt.sched->iterations] = (long long)wall_clock64();

@@ -151,3 +151,36 @@ def test_online_notoken_rejects_a_batch_it_cannot_run():
     assert on.mpk.stats()["aborted"] == 0
     assert not all(bool((c == 0.25).all()) for c in caches)
     on.mpk.finalize()
+
+
+def test_online_notoken_many_slots():
+    """All slots a wavefront has lanes for, unused ones among them: the rows are the same wherever the requests sit, and the first
+    slot that cannot run decides the reason."""
+    from mirage import _capi
+    from oracle.qwen3_ref import make_model_weights
+    cfg = _cfg()
+    w = make_model_weights(cfg, seed=44)
+    R, B, max_seq, PS = 64, 64, 48, 16
+    on = _decoder(cfg, w, max_num_batched_tokens=B, max_num_batched_requests=R, max_seq_length=max_seq, page_size=PS, total_requests=R, max_num_pages=R, kernel_mode="online_notoken")
+    m = on.meta
+
+    def run(rows, lens):
+        """rows, lens: new rows and length of every slot (a page each)"""
+        n = torch.tensor(rows)
+        m["input_tokens"].copy_((7 * torch.arange(B, dtype=torch.int64)).view(-1, 1) % cfg.vocab_size)
+        m["qo_indptr_buffer"].copy_(torch.cat([torch.zeros(1, dtype=torch.int64), n.cumsum(0)]).to(torch.int32))
+        m["paged_kv_indptr_buffer"].copy_(torch.cat([torch.zeros(1, dtype=torch.int64), (n > 0).cumsum(0)]).to(torch.int32))
+        m["paged_kv_indices_buffer"].copy_(torch.arange(R, dtype=torch.int32))
+        m["paged_kv_last_page_len_buffer"].copy_(torch.tensor(lens, dtype=torch.int32))
+        torch.cuda.synchronize()
+        on.mpk()
+        return on.logits()[:int(n.sum())].clone()
+
+    a = run([3] + [1] * 51 + [0] * 12, [3] + [1] * 51 + [0] * 12)
+    b = run([0] * 5 + [3] + [1] * 50 + [0] * 7 + [1], [0] * 5 + [3] + [1] * 50 + [0] * 7 + [1])
+    assert torch.equal(a, b)
+    with pytest.raises(_capi.MkError, match="shorter than its new rows"):
+        run([1] * 20 + [2] + [0] * 39 + [9] + [0] * 3, [1] * 20 + [1] + [0] * 39 + [9] + [0] * 3)
+    with pytest.raises(_capi.MkError, match="max_tokens_per_request"):
+        run([1] * 20 + [0] * 43 + [9], [1] * 20 + [0] * 43 + [9])
+    on.mpk.finalize()
