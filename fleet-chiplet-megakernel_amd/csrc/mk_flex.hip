@@ -979,75 +979,172 @@ __device__ __forceinline__ void stage_fx_attn(CStage &st, Ctx &c, const MkRuntim
 }
 
 // ----------------------------------------------------------------------------- 32-bit linear
-// out[m, n] = sum_k x[m, k] W[n, k] in true 32-bit (v_mfma_f32_16x16x4_f32), optional SwiGLU epilogue.  A workgroup owns a
-// range of 16-column output tiles and all rows; its wavefronts split K and are reduced through LDS in a fixed order.
 __device__ __forceinline__ float fx_glu_f32(CStage &st, float g, float u) {
 #if MK_HAVE_DUAL
   if (st.flags & MK_F_GELU) return 0.5f * g * (1.f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
 #endif
   return g / (1.f + expf(-g)) * u;
 }
-template <int MT>
-__device__ __forceinline__ void stage_fx_linear_f32(CStage &st, Ctx &c, int M, char *smem) {
-  if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+// out[m, n] = sum_k x[m, k] W[n, k] in true 32-bit (v_mfma_f32_16x16x4_f32), optional SwiGLU epilogue.
+//
+// Bound by the weights' stream with few tokens, by the matrix cores (157 TFLOP/s) and the CU's path to L2 with many.  A unit is a 16-column
+// output tile (a pair of them under SwiGLU) times MT tiles of 16 tokens; a workgroup walks a contiguous range of units, its wavefronts
+// split the reduction and are reduced through LDS in a fixed order.  Operands of D steps of 32 k are in flight per wavefront and never
+// drain between units; the weights of the first ones are requested before the previous stage's barrier.
+// Rows are read eight lanes to a whole 128-byte line and change into operand order in a wavefront's own LDS (16-byte words of a row
+// XORed with the row, so neither direction meets a bank twice): read in operand order, every lane another row, a CU takes in 16 bytes a
+// clock, a quarter of what it can.
+// MT is the number of token tiles that leaves the workgroup with the most units the least to multiply, the largest of them where they
+// tie: a weight row is then read once for more tokens.  The token groups of a tile are neighbours in a range, so that what they read
+// again comes from the die's L2.
+// Before -> now, 3 / 64 tokens, us: 5120 x 2048 34 -> 14 / 60 -> 33, 2048 x 4096 34 -> 13 / 56 -> 19, gate and up 12288 x 2048 46 -> 28 / 71
+// -> 48, 2048 x 6144 48 -> 17 / 80 -> 26, 32768 x 2048 129 -> 49 (5.5 TB/s) / 217 -> 120 (72 TFLOP/s; operand-order loads: 158).
+template <int MT, bool SILU>
+__device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M, char *smem) {
+  constexpr int NH = SILU ? 2 : 1, NT = NH + MT, D = MT == 1 ? 8 : 4;  // 16-row tiles of a step: weights, then tokens
+  constexpr bool DB = NH * MT < 8;                                       // sums of two units fit beside the operands
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4, l8 = lane >> 3, c8 = lane & 7;
+  const int K = st.k, n_out = SILU ? st.n / 2 : st.n, half = st.silu_half, nks = K / 16;  // (16 k of a tile are one operand)
+  const int ng = (M + 16 * MT - 1) / (16 * MT), n_units = (n_out + 15) / 16 * ng;
+  const int u0 = (int)(((long long)c.vid * n_units) / c.G), u1 = (int)(((long long)(c.vid + 1) * n_units) / c.G);
+  const int kq = (nks + MK_WAVES - 1) / MK_WAVES, kb = min(nks, wave * kq), ke = min(nks, kb + kq), nb = (kq + 2 * D - 1) / (2 * D);
+  f32x4 *red = (f32x4 *)smem;  // [DB ? 2 : 1][waves][NH][MT][64]
+  f32x4 *ops = red + (DB ? 2 : 1) * MK_WAVES * NH * MT * 64 + wave * 2 * NT * 128;  // [2][tile][8-row half][8 rows][8 words]
+  struct Unit {
+    const f32x4 *row[NT][2];  // this lane's row of either half of a tile
+    int tile, m0;
+  };
+  auto unit = [&](int u) {
+    Unit a;
+    a.tile = u / ng;
+    a.m0 = (u - a.tile * ng) * 16 * MT;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int o = min(a.tile * 16 + 8 * i + l8, n_out - 1);
+      const int vr = SILU ? (o / half) * 2 * half + (o % half) : o;
+#pragma unroll
+      for (int h = 0; h < NH; h++) a.row[h][i] = (const f32x4 *)weight_row(st.w, vr + h * half, K / 4);
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) a.row[NH + mt][i] = (const f32x4 *)((const float *)st.in + (size_t)min(a.m0 + mt * 16 + 8 * i + l8, M - 1) * st.ld_in);
+    }
+    return a;
+  };
+  f32x4 ring[D][NT][2];
+  Unit a{};
+  if (u0 < u1) a = unit(u0);
+  const bool early = u0 < u1 && wave != 0;
+  auto word = [&](int s) { return min(4 * s + c8, 4 * nks - 1); };  // this lane's 16-byte word of the step that begins at s (in units of 16 k)
+  auto request = [&](f32x4 (&r)[NT][2], const Unit &p, int s, int t0, int t1) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      if (t >= t0 && t < t1) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) r[t][i] = p.row[t][i][word(s)];
+      }
+  };
+  if (early) {
+#pragma unroll
+    for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, 0, NH);
+  }
+  if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
   c.wrote_through = true;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lr = lane & 15, lg = lane >> 4;
+  if (u0 >= u1) return;
+  if (!early) {
+#pragma unroll
+    for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, 0, NH);
+  }
+#pragma unroll
+  for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, NH, NT);
+  f32x4 op[2][NT][2];  // operands of two steps, [tile][16 k]
+  auto turn = [&](const f32x4 (&r)[NT][2], f32x4 (&o)[NT][2], int slot) {
+    f32x4 *b = ops + slot * NT * 128;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) b[t * 128 + i * 64 + l8 * 8 + (c8 ^ l8)] = r[t][i];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) o[t][h] = b[t * 128 + lr * 8 + ((h * 4 + lg) ^ (lr & 7))];
+  };
+  turn(ring[0], op[0], 0);
+  for (int u = u0; u < u1; u++) {
+    const bool more = u + 1 < u1;
+    const Unit nx = more ? unit(u + 1) : a;
+    f32x4 acc[NH][MT];
+#pragma unroll
+    for (int h = 0; h < NH; h++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) acc[h][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int blk = 0; blk < nb; blk++) {
+      const bool last = blk + 1 == nb;
+      const int k0 = kb + blk * 2 * D, kn = last ? kb : k0 + 2 * D, step = last && !more ? 0 : 2;  // (behind the range: one line again and again)
+      Unit p;
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) p.row[t][i] = last ? nx.row[t][i] : a.row[t][i];
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        // operands of the step behind this one, whose place in the ring is then free (the one behind a block's last is its successor's first)
+        request(ring[j], p, kn + step * j, 0, NT);
+        turn(ring[(j + 1) % D], op[(j + 1) & 1], (j + 1) & 1);
+        const int s = k0 + 2 * j;
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+          if (s + e < ke) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+              for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int h = 0; h < NH; h++) acc[h][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[j & 1][h][e][q], op[j & 1][NH + mt][e][q], acc[h][mt], 0, 0, 0);
+          }
+      }
+    }
+    f32x4 *rb = red + (DB ? u & 1 : 0) * (MK_WAVES * NH * MT * 64) + lane;
+    if (!DB) __syncthreads();
+#pragma unroll
+    for (int h = 0; h < NH; h++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) rb[((wave * NH + h) * MT + mt) * 64] = acc[h][mt];
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const int m = a.m0 + mt * 16 + lr;
+      if (((u * MT + mt) & (MK_WAVES - 1)) != wave || m >= M) continue;
+      f32x4 v[NH];
+#pragma unroll
+      for (int h = 0; h < NH; h++) {
+        v[h] = rb[(h * MT + mt) * 64];
+#pragma unroll
+        for (int q = 1; q < MK_WAVES; q++) v[h] += rb[((q * NH + h) * MT + mt) * 64];
+      }
+      float r[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) r[i] = SILU ? fx_glu_f32(st, v[0][i], v[NH - 1][i]) : linear_act(st, v[0][i]);
+      fx_stc4((float *)st.out + (size_t)m * st.ld_out, a.tile * 16 + lg * 4, n_out, r);
+    }
+    a = nx;
+  }
+}
+__device__ __forceinline__ void stage_fx_linear_f32(CStage &st, Ctx &c, int M, char *smem) {
   const bool silu = st.flags & MK_F_SILU;
-  const int K = st.k, n_out = silu ? st.n / 2 : st.n, half = st.silu_half;
-  const int ntiles = (n_out + 15) / 16;
-  const int t_begin = (int)(((long long)c.vid * ntiles) / c.G), t_end = (int)(((long long)(c.vid + 1) * ntiles) / c.G);
-  const int kq = ((K / 16 + MK_WAVES - 1) / MK_WAVES) * 16;
-  const int kbeg = min(K, wave * kq), kend = min(K, kbeg + kq);
-  f32x4 *red = (f32x4 *)smem;  // [waves][2][MT][64]
-  const float *xrow[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++) xrow[mt] = (const float *)st.in + (size_t)min(mt * 16 + lr, M - 1) * st.ld_in + lg * 4;
-  for (int ot = t_begin; ot < t_end; ot++) {
-    const int o = min(ot * 16 + lr, n_out - 1);
-    int vr = o;
-    if (silu) vr = (o / half) * 2 * half + (o % half);
-    const float *w0 = (const float *)weight_row(st.w, vr, K / 4) + lg * 4;
-    const float *w1 = silu ? (const float *)weight_row(st.w, vr + half, K / 4) + lg * 4 : w0;
-    f32x4 acc[2][MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[0][mt] = acc[1][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k = kbeg; k < kend; k += 16) {
-      const f32x4 a0 = *(const f32x4 *)(w0 + k), a1 = *(const f32x4 *)(w1 + k);
-      f32x4 b[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) b[mt] = *(const f32x4 *)(xrow[mt] + k);
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-          acc[0][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[j], b[mt][j], acc[0][mt], 0, 0, 0);
-          if (silu) acc[1][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[j], b[mt][j], acc[1][mt], 0, 0, 0);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) red[((wave * 2 + h) * MT + mt) * 64 + lane] = acc[h][mt];
-    __syncthreads();
-    for (int e = tid; e < MT * 64; e += MK_THREADS) {
-      const int l = e & 63, mt = e >> 6, m = mt * 16 + (l & 15);
-      f32x4 v = red[mt * 64 + l], g = red[(MT + mt) * 64 + l];
-#pragma unroll
-      for (int w = 1; w < MK_WAVES; w++) {
-        v += red[((w * 2) * MT + mt) * 64 + l];
-        g += red[((w * 2 + 1) * MT + mt) * 64 + l];
-      }
-      if (m < M) {
-        float r[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) r[i] = silu ? fx_glu_f32(st, v[i], g[i]) : linear_act(st, v[i]);
-        fx_stc4((float *)st.out + (size_t)m * st.ld_out, ot * 16 + (l >> 4) * 4, n_out, r);
-      }
-    }
+  const int tiles = ((silu ? st.n / 2 : st.n) + 15) / 16, mt = (M + 15) / 16;
+  auto rounds = [&](int per) { return (tiles * ((mt + per - 1) / per) + c.G - 1) / c.G * per; };  // token tiles of the busiest workgroup
+  const int r1 = rounds(1), r2 = mt > 1 ? rounds(2) : 1 << 30, r4 = mt > 2 ? rounds(4) : 1 << 30;
+  if (r4 <= r2 && r4 <= r1) {
+    if (silu) stage_fx_linear_f32_t<4, true>(st, c, M, smem);
+    else stage_fx_linear_f32_t<4, false>(st, c, M, smem);
+  } else if (r2 <= r1) {
+    if (silu) stage_fx_linear_f32_t<2, true>(st, c, M, smem);
+    else stage_fx_linear_f32_t<2, false>(st, c, M, smem);
+  } else if (silu) {
+    stage_fx_linear_f32_t<1, true>(st, c, M, smem);
+  } else {
+    stage_fx_linear_f32_t<1, false>(st, c, M, smem);
   }
 }
 

@@ -4217,11 +4217,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         case MK_OP_FX_PREP: if constexpr (FX) stage_fx_prep<E>(st, c, rt, M); break;
         case MK_OP_FX_ATTN: if constexpr (FX) stage_fx_attn<E>(st, c, rt, M, MAXM == 1 || single, smem); break;
         case MK_OP_LINEAR_F32:
-          if constexpr (F32) {
-            if (M <= 16) stage_fx_linear_f32<1>(st, c, M, smem);
-            else if (M <= 32) stage_fx_linear_f32<2>(st, c, M, smem);
-            else stage_fx_linear_f32<4>(st, c, M, smem);
-          }
+          if constexpr (F32) stage_fx_linear_f32(st, c, M, smem);
           break;
         case MK_OP_FX_ARGMAX_F32: if constexpr (F32) stage_fx_argmax_f32(st, c, rt, M); break;
 #endif

@@ -48,7 +48,7 @@ class ServingSession:
     state_slots = slots = None
     # sessions opened here: a pass's ids and description in pinned memory, the device tensor they are copied to, and a pinned place for the
     # sampled tokens, so that a pass waits for the device once (a pageable copy in either direction costs 12 to 16 us, of which a pass had
-    # three; one copy per wanted row of logits another 8 each: a decode step of 16 requests spent 280 us outside the launch, now 90)
+    # three; one copy per wanted row of logits another 8 each: a decode step of 16 requests spent 280 us outside the launch, now 85)
     _host = _dev = _sampled = None
 
     def __init__(self, mpk: MPK):

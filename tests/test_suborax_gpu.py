@@ -143,6 +143,12 @@ def test_32_bit_linear(k, n, silu):
     pk.finalize()
 
 
+# one, two and four token tiles per unit, workgroups with several units, shares of the reduction that are odd or empty
+@pytest.mark.parametrize("k,n,silu", [(96, 5120, False), (160, 2048, False), (352, 2064, False), (64, 32768, False), (96, 6144, True), (32, 16400, True)])
+def test_32_bit_linear_units(k, n, silu):
+    test_32_bit_linear(k, n, silu)
+
+
 def test_32_bit_sampling_takes_the_lowest_of_equal_maxima():
     import mirage as mi
     pk, V = _graph(8), 3001
