@@ -1904,6 +1904,7 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
 #endif
 struct XresPlan {
   int S;       // K slices per tile range (0: this form cannot run the stage)
+  int R;       // tile ranges a workgroup walks one after another (1 unless S is 1)
   int groups;  // tile ranges
   int wt;      // weight tiles of the stage
   int tpu;     // most tiles a range holds (decides tiles per wavefront and prefetch depth for every workgroup alike)
@@ -1921,9 +1922,20 @@ __device__ __forceinline__ XresPlan linear_xres_plan(CStage &st, const Ctx &c) {
     const int gs = c.G / S;
     int tpu = (p.wt + gs - 1) / gs;  // tiles per range
     tpu = (tpu + unit - 1) / unit * unit;
-    if (tpu > 6) break;              // two streaming wavefronts with three tiles each
-    if (tpu < 4) continue;           // too few tiles to occupy them: split K further
+    if (tpu < 4) continue;           // too few tiles to occupy two streaming wavefronts: split K further
     p.S = S;
+    p.R = 1;
+    if (tpu > 6) {
+      // more than three tiles each: several ranges of equal size, one after another, whose rows are staged anew (an eighth of the weights'
+      // bytes at 64 tokens).  The form for any shape, whose wavefronts read the rows in operand order at every step, took 66.6 / 56.7 us
+      // for 32768 x 4096 at 64 tokens / the last 5 of a prompt; this takes 55.1 / 45.6.
+      const int nun = p.wt / unit;
+      p.R = (nun * unit + 6 * c.G - 1) / (6 * c.G);
+      while ((nun + c.G * p.R - 1) / (c.G * p.R) * unit > 6) p.R++;
+      p.tpu = (nun + c.G * p.R - 1) / (c.G * p.R) * unit;
+      p.groups = min(nun, c.G * p.R);
+      return p;
+    }
     p.tpu = tpu;
     p.groups = (p.wt / unit + tpu / unit - 1) / (tpu / unit);
     return p;
@@ -1943,15 +1955,19 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   const int half = st.silu_half;
   const int S = plan.S;
   const int g = c.vid / S, sl = c.vid - g * S;
-  const bool active = g < plan.groups;  // workgroups beyond the last range only keep the barriers
-  const int nun = plan.wt / unit;       // balanced ranges of whole units
-  const int tb = active ? (int)(((long long)g * nun) / plan.groups) * unit : 0, te = active ? (int)(((long long)(g + 1) * nun) / plan.groups) * unit : 0;
+  // ranges [q0, q0 + nr) of this workgroup; workgroups beyond the last range only keep the barriers
+  const int q0 = plan.R > 1 ? (int)(((long long)c.vid * plan.groups) / c.G) : g, nr = plan.R > 1 ? (int)(((long long)(c.vid + 1) * plan.groups) / c.G) - q0 : (g < plan.groups ? 1 : 0);
+  const bool active = nr > 0;
+  const int nun = plan.wt / unit;  // balanced ranges of whole units
+  auto range_at = [&](int q) { return (int)(((long long)q * nun) / plan.groups) * unit; };
+  int tb = active ? range_at(q0) : 0, te = active ? range_at(q0 + 1) : 0;
   const int kslice = K / S, kbeg = sl * kslice, nsteps = kslice >> 6, npass = nsteps / NSP;
   const uint16_t *x = (st.flags & MK_F_NORM) ? (const uint16_t *)st.norm_out : (const uint16_t *)st.in;
   const int ldx = (st.flags & MK_F_NORM) ? st.ld_norm : st.ld_in;
   u32x4 *xl = (u32x4 *)smem;  // two buffers of [step of the pass][token tile][16 rows][8] 16-byte words
   constexpr int XBUF = NSP * MT * 128;  // 16-byte operands per buffer
   int *sflag = (int *)(smem + 2 * XBUF * 16);
+  u32x4 *xpair = xl + 2 * XBUF + 16;  // a gate/up pair that two wavefronts hold
   u32x4 *part = (u32x4 *)rt.splitk_part;
   // hand the K-slice sum to the norm stage that follows, if there is one and the rows fit the partial buffer
   const bool defer = (st.flags & MK_F_DEFER_SUM) && S > 1 && (size_t)S * (MT * 16) * st.n * 4 <= (size_t)c.G * 65536;
@@ -1986,9 +2002,9 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   // 8 r + (c ^ (r & 7)), so that the operand reads meet no bank twice.  `nw` wavefronts share the items: wavefront `w` of them takes
   // items w, w + nw, ...
   // (64 tokens, operand order -> lines, us: 24576 x 4096 41.9 -> 39.6, 4096 x 12288 28.9 -> 27.0, 6144 x 4096 17.3 -> 16.7.)
-  auto stage_pass = [&](int pass, int w, int nw) {
+  auto stage_pass = [&](int pass, int par, int w, int nw) {
     const uint16_t *base = x + kbeg + pass * (NSP * 64) + ((lane & 7) ^ (lane >> 3)) * 8;
-    u32x4 *buf = xl + (pass & 1) * XBUF;
+    u32x4 *buf = xl + (par & 1) * XBUF;
     for (int i = w; i < MT * NSP; i += nw) {
       const int step = i / MT, mt = i - step * MT, r0 = mt * 16 + (lane >> 3);
       __attribute__((address_space(3))) char *dst = (__attribute__((address_space(3))) char *)(buf + (size_t)i * 128);
@@ -2000,26 +2016,27 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   {
     constexpr int NB = 8, NSW = 2;    // ring depth in steps; streaming wavefronts
     const bool loader = wave >= NSW;  // stages token rows, holds no tiles
-    const int tw0 = tb + wave * TW;   // a streaming wavefront's first tile
-    const bool has_tile = active && !loader && tw0 < te;
+    int tw0 = tb + wave * TW;         // a streaming wavefront's first tile
+    // (between two ranges of a workgroup the ring stays full, so a wavefront without a tile in one of them reads the last one along)
+    const bool streams = active && !loader && (nr > 1 || tw0 < te);
     const u32x4 *wrow[TW];
 #pragma unroll
     for (int t = 0; t < TW; t++) wrow[t] = tile_base(max(min(tw0 + t, te - 1), 0));
     bf16x8 a[NB][TW][2];
-    auto w_load = [&](int step, bf16x8 (&aa)[TW][2]) {
+    auto w_load = [&](const u32x4 *const (&row)[TW], int step, bf16x8 (&aa)[TW][2]) {
 #pragma unroll
       for (int t = 0; t < TW; t++) {
-        aa[t][0] = __builtin_nontemporal_load((const bf16x8 *)(wrow[t] + step * step_stride));
-        aa[t][1] = __builtin_nontemporal_load((const bf16x8 *)(wrow[t] + step * step_stride + half_stride));
+        aa[t][0] = __builtin_nontemporal_load((const bf16x8 *)(row[t] + step * step_stride));
+        aa[t][1] = __builtin_nontemporal_load((const bf16x8 *)(row[t] + step * step_stride + half_stride));
       }
     };
     // weights do not depend on the previous stage: the first NBP steps are requested before its barrier is awaited, the
     // rest of the ring right after the first pass's token rows (what a CU has in flight sits in front of the barrier
     // poll and of the row requests)
     constexpr int NBP = MK_TUNE_XRES_PRE < NB ? MK_TUNE_XRES_PRE : NB;
-    if (has_tile) {
+    if (streams) {
 #pragma unroll
-      for (int j = 0; j < NBP; j++) w_load(j, a[j]);
+      for (int j = 0; j < NBP; j++) w_load(wrow, j, a[j]);
     }
     // Token rows come from other workgroups and are read with cached loads, so what this die's caches hold of them must
     // go first.  The invalidate is issued BEFORE the barrier is awaited: nothing on this die reads the stage's input
@@ -2036,10 +2053,6 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     barrier_done(c);
     MK_MARK(c, 0);
     f32x4 acc[TW][MT];
-#pragma unroll
-    for (int t = 0; t < TW; t++)
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) acc[t][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     auto compute = [&](const u32x4 *xb, const bf16x8 (&aa)[TW][2]) {
       u32x4 b[2][MT];
 #pragma unroll
@@ -2055,44 +2068,136 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
           for (int t = 0; t < TW; t++) acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa[t][h], __builtin_bit_cast(bf16x8, b[h][mt]), acc[t][mt], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     };
-    // Passes [0, n_refill) refill the ring as they go, the last one only consumes it.  Every pass starts with a workgroup
-    // barrier: its rows have landed (whoever requested them has waited for them) and everybody is done with the other
-    // buffer, into which the loader then requests the next pass's rows.
-    const int n_refill = npass - 1;
+    // All passes but the very last one refill the ring as they go, the last of a range with the first steps of the next range.  Every
+    // pass starts with a workgroup barrier: its rows have landed (whoever requested them has waited for them) and everybody is done with
+    // the other buffer, into which the loader then requests the next pass's rows.
+    const u32x4 *wnext[TW];
+    int par = 0;  // passes done
     auto do_pass = [&](int pass, auto refill_c) {
       constexpr bool REFILL = decltype(refill_c)::value;
-      if (pass == 0 && has_tile && NBP < NB) {
+      if (par == 0 && streams && NBP < NB) {
         // the token rows of pass 0 have landed once nothing but the ring steps requested after them is outstanding
         static_assert((NB - NBP) * TW * 2 <= 63, "vmcnt range");
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - NBP) * TW * 2) : "memory");
-      } else if (pass == 0 || loader) {
+      } else if (par == 0 || loader) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       __syncthreads();
-      if (pass == 0) MK_MARK(c, 1);
-      if (loader && active && pass + 1 < npass) stage_pass(pass + 1, wave - NSW, MK_WAVES - NSW);
+      if (par == 0) MK_MARK(c, 1);
+      const bool in_range = pass + 1 < npass;
+      if (loader && active && REFILL) stage_pass(in_range ? pass + 1 : 0, par + 1, wave - NSW, MK_WAVES - NSW);
       __builtin_amdgcn_sched_barrier(0);
-      if (has_tile) {
-        const u32x4 *xb = xl + (pass & 1) * XBUF;
+      if (streams) {
+        const u32x4 *xb = xl + (par & 1) * XBUF;
+        static_assert(NB == NSP, "a refill is the same step of the next pass");
+        const u32x4 *wr[TW];
+#pragma unroll
+        for (int t = 0; t < TW; t++) wr[t] = in_range ? wrow[t] : wnext[t];
+        const int s0 = in_range ? (pass + 1) * NSP : 0;
 #pragma unroll
         for (int j = 0; j < NSP; j++) {
           compute(xb + j * MT * 128, a[j]);
-          if (REFILL) w_load(pass * NSP + j + NB, a[j]);
+          if (REFILL) w_load(wr, s0 + j, a[j]);
+        }
+      }
+      par++;
+    };
+    if (active) stage_pass(0, 0, wave, MK_WAVES);
+    __builtin_amdgcn_sched_barrier(0);
+    if (streams) {
+#pragma unroll
+      for (int j = NBP; j < NB; j++) w_load(wrow, j, a[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto clear = [&]() {
+#pragma unroll
+      for (int t = 0; t < TW; t++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[t][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    };
+    // ---- epilogue of a range: lane l holds token m = mt * 16 + (l & 15), output columns tile * 16 + (l >> 4) * 4 .. + 3
+    auto finish = [&]() {
+      const bool has_tile = active && !loader && tw0 < te;
+      if (silu && (TW & 1)) {
+        // an odd tile count per wavefront leaves the middle gate/up pair split: wavefront 1 hands its first tile (an up
+        // tile) to wavefront 0, which holds the gate tile, through LDS
+        if (wave == 1 && has_tile) {
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++) xpair[mt * 64 + lane] = __builtin_bit_cast(u32x4, acc[0][mt]);
+        }
+        __syncthreads();
+      }
+      auto store_tile = [&](int otile, const f32x4 (&v)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+          const int m = mt * 16 + lr;
+          if (m < M) {
+            uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
+            const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
+            float rr[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const int n = otile * 16 + lg * 4 + i;
+              float r = v[mt][i];
+              if ((st.flags & MK_F_RES) && n < n_out) r += bf2f(rrow[n]);
+              rr[i] = linear_act(st, r);
+            }
+            stc_bf16x4(orow, otile * 16 + lg * 4, n_out, rr);
+          }
+        }
+      };
+      if (!has_tile) {
+        // (no tile in this range)
+      } else if (!silu) {
+#pragma unroll
+        for (int t = 0; t < TW; t++)
+          if (tw0 + t < te) store_tile(tw0 + t, acc[t]);
+      } else {
+        // tile index relative to the range start is even for gate tiles (ranges hold whole pairs)
+#pragma unroll
+        for (int t = 0; t < TW; t++) {
+          const int ti = tw0 + t;
+          if (ti >= te || ((ti - tb) & 1)) continue;  // pairs are stored by the holder of their gate tile
+          f32x4 v[MT];
+          if (t + 1 < TW) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+              for (int i = 0; i < 4; i++) v[mt][i] = linear_glu(st, acc[t][mt][i], acc[(t + 1) % TW][mt][i]);
+          } else {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+              const f32x4 up = __builtin_bit_cast(f32x4, xpair[mt * 64 + lane]);
+#pragma unroll
+              for (int i = 0; i < 4; i++) v[mt][i] = linear_glu(st, acc[t][mt][i], up[i]);
+            }
+          }
+          store_tile(ti >> 1, v);
         }
       }
     };
-    if (active) stage_pass(0, wave, MK_WAVES);
-    __builtin_amdgcn_sched_barrier(0);
-    if (has_tile) {
-#pragma unroll
-      for (int j = NBP; j < NB; j++) w_load(j, a[j]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
     int pass = 0;
-    for (; pass < n_refill; pass++) do_pass(pass, std::true_type{});
+    for (int r = 1; r < nr; r++) {  // all ranges but the last
+      const int nb_ = range_at(q0 + r), ne_ = range_at(q0 + r + 1);
+#pragma unroll
+      for (int t = 0; t < TW; t++) wnext[t] = tile_base(min(nb_ + wave * TW + t, ne_ - 1));
+      clear();
+      for (pass = 0; pass < npass; pass++) do_pass(pass, std::true_type{});
+      finish();
+      tb = nb_;
+      te = ne_;
+      tw0 = tb + wave * TW;
+#pragma unroll
+      for (int t = 0; t < TW; t++) wrow[t] = wnext[t];
+    }
+#pragma unroll
+    for (int t = 0; t < TW; t++) wnext[t] = wrow[t];
+    clear();
+    for (pass = 0; pass < npass - 1; pass++) do_pass(pass, std::true_type{});
     MK_MARK(c, 2);
     do_pass(pass, std::false_type{});
     MK_MARK(c, 3);
+    const bool has_tile = active && !loader && tw0 < te;
     if (defer) {
       // the consumer sums the slices: leave them as [slice][token][n] fp32 rows
       if (has_tile) {
@@ -2153,64 +2258,7 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
           }
       }
     }
-    // ---- epilogue: lane l holds token m = mt * 16 + (l & 15), output columns tile * 16 + (l >> 4) * 4 .. + 3
-    if (silu && (TW & 1)) {
-      // an odd tile count per wavefront leaves the middle gate/up pair split: wavefront 1 hands its first tile (an up
-      // tile) to wavefront 0, which holds the gate tile, through LDS
-      __syncthreads();  // everybody is done with the row buffers
-      if (wave == 1 && has_tile) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) xl[mt * 64 + lane] = __builtin_bit_cast(u32x4, acc[0][mt]);
-      }
-      __syncthreads();
-    }
-    if (!has_tile) return;
-    auto store_tile = [&](int otile, const f32x4 (&v)[MT]) {
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) {
-        const int m = mt * 16 + lr;
-        if (m < M) {
-          uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
-          const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
-          float rr[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const int n = otile * 16 + lg * 4 + i;
-            float r = v[mt][i];
-            if ((st.flags & MK_F_RES) && n < n_out) r += bf2f(rrow[n]);
-            rr[i] = linear_act(st, r);
-          }
-          stc_bf16x4(orow, otile * 16 + lg * 4, n_out, rr);
-        }
-      }
-    };
-    if (!silu) {
-#pragma unroll
-      for (int t = 0; t < TW; t++)
-        if (tw0 + t < te) store_tile(tw0 + t, acc[t]);
-    } else {
-      // tile index relative to the range start is even for gate tiles (ranges hold whole pairs)
-#pragma unroll
-      for (int t = 0; t < TW; t++) {
-        const int ti = tw0 + t;
-        if (ti >= te || ((ti - tb) & 1)) continue;  // pairs are stored by the holder of their gate tile
-        f32x4 v[MT];
-        if (t + 1 < TW) {
-#pragma unroll
-          for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[mt][i] = linear_glu(st, acc[t][mt][i], acc[(t + 1) % TW][mt][i]);
-        } else {
-#pragma unroll
-          for (int mt = 0; mt < MT; mt++) {
-            const f32x4 up = __builtin_bit_cast(f32x4, xl[mt * 64 + lane]);
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[mt][i] = linear_glu(st, acc[t][mt][i], up[i]);
-          }
-        }
-        store_tile(ti >> 1, v);
-      }
-    }
+    finish();
   }
 }
 

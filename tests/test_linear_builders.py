@@ -78,3 +78,34 @@ def test_linear_builder_matches_oracle(name, M, B):
     assert ulp <= 1.0 and frac < 0.02, f"{name}: {frac:.4f} of outputs differ, max {ulp} ulp ({mabs})"
     assert mpk.stats()["aborted"] == 0
     mpk.finalize()
+
+
+@pytest.mark.parametrize("rows", [3, 33, 64])
+@pytest.mark.parametrize("n,k,silu,res", [
+    # more tiles per workgroup than the streaming wavefronts hold: two ranges of three and four tiles, of six, three ranges with a ragged last
+    # tile; one, two and three passes over k; pairs of gate and up tiles
+    (16 * 1540, 512, False, False), (26688, 1024, False, True), (16 * 3072, 512, False, False), (16 * 3300 + 5, 1536, False, False), (13008, 1024, True, False), (16 * 1700, 512, True, False)])
+def test_wide_linear_in_ranges(n, k, silu, res, rows):
+    import mirage as mi
+    g = torch.Generator(device="cuda").manual_seed(n + rows)
+    mk = lambda *s: torch.empty(s, device="cuda").normal_(0.0, 1.0, generator=g)
+    x, W, r = mk(64, k).bfloat16(), (mk(2 * n if silu else n, k) / k ** 0.5).bfloat16(), mk(64, n).bfloat16()
+    mpk = make_mpk(make_meta(1, 64, 64, 64, 64), 64, 64, 64, 64, 64, mode="onepass")
+    a, y = mpk.attach_input, mpk.new_tensor((64, n), dtype=mi.bfloat16, name="y")
+    if silu:
+        w = mpk.shuffle_tensors(inputs=[a(W[:n], "gate"), a(W[n:], "up")], shuffled_dim=0, num_groups=1, name="gate_up")
+        mpk.gang_linear_silu_layer(input=a(x, "x"), weight=w, output=y, tile_n=2, output_stride=n, m_tiles=1)
+    elif res:
+        mpk.linear_with_residual_layer(input=a(x, "x"), weight=a(W, "W"), residual=a(r, "r"), output=y, grid_dim=(1, 1, 1), block_dim=(256, 1, 1))
+    else:
+        mpk.linear_layer(input=a(x, "x"), weight=a(W, "W"), output=y, grid_dim=(1, 1, 1), block_dim=(256, 1, 1))
+    mpk.compile()
+    mpk.run_once(list(range(rows)), [0] * rows)
+    want = x[:rows].double() @ W.double().T
+    if silu:
+        want = torch.nn.functional.silu(want[:, :n]) * want[:, n:]
+    if res:
+        want = want + r[:rows].double()
+    # one rounding to 8 bits of mantissa, behind 32-bit sums
+    torch.testing.assert_close(y.to_torch()[:rows].double(), want, rtol=2.0 ** -8, atol=2.0 ** -16 * k ** 0.5)
+    mpk.finalize()
