@@ -14,14 +14,14 @@
 // 32-bit rows (out2: steps, from column cols[2] on decays).
 template <typename E>
 __device__ __forceinline__ void stage_du_conv(CStage &st, Ctx &c, int M) {
-  const int n = st.n, n4 = n / 4, taps = st.taps, per = (n4 + MK_THREADS - 1) / MK_THREADS, lane = threadIdx.x & 63;
+  const int n = st.n, n4 = n / 4, taps = st.taps, per = (n4 + MK_THREADS - 1) / MK_THREADS, lane = c.tid & 63;
   const int H = st.step_bias ? st.num_q_heads : 0, hper = (H + MK_THREADS - 1) / MK_THREADS;
   const int first_of = c.sh_tok[2 * MK_MAX_TOKENS + lane];
   barrier_wait(c);
   const E *w = (const E *)st.conv_w;
   for (int i = mx_spread(c); i < M * (per + hper); i += c.G) {
     if (i >= M * per) {
-      const int k = i - M * per, t = k / hper, h = (k - t * hper) * MK_THREADS + threadIdx.x;
+      const int k = i - M * per, t = k / hper, h = (k - t * hper) * MK_THREADS + c.tid;
       if (h >= H) continue;
       const float z = fx_ldc((const E *)st.in + (size_t)t * st.ld_in + st.cols[1] + h) + st.step_bias[h];
       const float dt = z > 20.f ? z : log1pf(expf(z));
@@ -30,7 +30,7 @@ __device__ __forceinline__ void stage_du_conv(CStage &st, Ctx &c, int M) {
       stc_f32(o + st.cols[2], exp2f(st.a_tab[h] * dt));
       continue;
     }
-    const int t = i / per, q = (i - t * per) * MK_THREADS + threadIdx.x;
+    const int t = i / per, q = (i - t * per) * MK_THREADS + c.tid;
     const int t0 = __builtin_amdgcn_readfirstlane(c.sh_tok[2 * MK_MAX_TOKENS + t]), p0 = __builtin_amdgcn_readfirstlane(c.sh_tok[t0]), lead = t - t0;
     const int cnt = __popcll(__ballot(lane < M && first_of == t0));  // the request's tokens
     if (q >= n4 || (lead > 0 && lead < taps - 1)) continue;
@@ -115,7 +115,7 @@ struct DuUnit {
 template <int CH>
 __device__ __forceinline__ DuUnit du_unit(CStage &st, const Ctx &c, const MkRuntime &rt, const MxDeltaUnits &us, int u, int lg2) {
   const int GW = 64 >> lg2, CW = MK_WAVES * GW * CH, V = st.v_dim, H = st.num_q_heads, Np = (st.states + 3) / 4 * 4, nblk = (V + CW - 1) / CW;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), uh = u / nblk, ri = uh / H;
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6), uh = u / nblk, ri = uh / H;
   DuUnit a;
   a.h = uh - ri * H;
   a.v0 = (u - uh * nblk) * CW + wave * GW * CH + (lane >> lg2);
@@ -130,8 +130,8 @@ template <int Q>
 struct DuLanes {
   int at[Q], GW, V, Np;
   bool on[Q];
-  __device__ __forceinline__ DuLanes(CStage &st, int lg2) {
-    const int L = 1 << lg2, j = threadIdx.x & (L - 1);
+  __device__ __forceinline__ DuLanes(CStage &st, int tid, int lg2) {
+    const int L = 1 << lg2, j = tid & (L - 1);
     GW = 64 >> lg2;
     V = st.v_dim;
     Np = (st.states + 3) / 4 * 4;
@@ -188,9 +188,9 @@ template <typename E, int Q, int CH, int DEP>
 __device__ __forceinline__ void stage_du_scan_single(CStage &st, Ctx &c, const MkRuntime &rt, int M, int lg2) {
   static_assert(DEP == 1 || DEP == 2, "");
   static_assert(CH <= 4, "a lane finishes one output, four lanes or more share a value");
-  const int L = 1 << lg2, j = threadIdx.x & (L - 1), CW = MK_WAVES * (64 >> lg2) * CH;
+  const int L = 1 << lg2, j = c.tid & (L - 1), CW = MK_WAVES * (64 >> lg2) * CH;
   const int V = st.v_dim, H = st.num_q_heads, per_group = H / st.groups, nblk = (V + CW - 1) / CW;
-  const DuLanes<Q> ln(st, lg2);
+  const DuLanes<Q> ln(st, c.tid, lg2);
   const MxDeltaUnits us = mx_delta_units(c, M);
   const int n_units = us.nreq * H * nblk;
   struct Rows {
@@ -213,7 +213,7 @@ __device__ __forceinline__ void stage_du_scan_single(CStage &st, Ctx &c, const M
     r.z = fx_ldc((const E *)st.in + (size_t)a.t0 * st.ld_in + st.cols[3] + a.h * V + ln.value(a, min(j, CH - 1)));
   };
   const int u0 = mx_spread(c);
-  const bool have = u0 < n_units, early = have && threadIdx.x >= 64;
+  const bool have = u0 < n_units, early = have && c.tid >= 64;
   auto unit = [&](int u) { return du_unit<CH>(st, c, rt, us, min(u, n_units - 1 - (n_units - 1 - u0) % c.G), lg2); };  // (behind the last: the last again)
   // A ring of DEP + 1 units, unrolled so that registers which still wait for their loads are never copied.
   f32x4 S[DEP + 1][CH][Q];
@@ -269,9 +269,9 @@ __device__ __forceinline__ void stage_du_scan_single(CStage &st, Ctx &c, const M
 // some request brings several tokens: the rows of a unit's portion are put in LDS at once (32-bit), then every group of lanes walks them
 template <typename E, int Q, int CH>
 __device__ __forceinline__ void stage_du_scan_portions(CStage &st, Ctx &c, const MkRuntime &rt, int M, int lg2, char *smem) {
-  const int L = 1 << lg2, GW = 64 >> lg2, CW = MK_WAVES * GW * CH, tid = threadIdx.x, lane = tid & 63, j = lane & (L - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int L = 1 << lg2, GW = 64 >> lg2, CW = MK_WAVES * GW * CH, tid = c.tid, lane = tid & 63, j = lane & (L - 1), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int V = st.v_dim, H = st.num_q_heads, per_group = H / st.groups, nblk = (V + CW - 1) / CW;
-  const DuLanes<Q> ln(st, lg2);
+  const DuLanes<Q> ln(st, c.tid, lg2);
   const int Np = 4 * L * Q, n4 = Np / 4, real4 = ln.Np / 4;  // (rows in LDS are padded with zeros to what the lanes read)
   const MxDeltaUnits us = mx_delta_units(c, M);
   const int n_units = us.nreq * H * nblk;

@@ -97,13 +97,13 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
     if (st.pos_tab) {  // (the caller keeps positions inside the table)
       const E *pos = (const E *)st.pos_tab + (size_t)min(c.sh_tok[t], st.pos_rows - 1) * k;
       if ((k & 3) == 0) {
-        for (int i = threadIdx.x * 4; i < k; i += MK_THREADS * 4) {
+        for (int i = c.tid * 4; i < k; i += MK_THREADS * 4) {
           const f32x4 v = fx_ld_quad(src + i) * scale + fx_ld_quad(pos + i);
           if (out32) fx_stc_quad(out32 + i, v);
           fx_stc_quad(out + i, v);
         }
       } else {
-        for (int i = threadIdx.x; i < k; i += MK_THREADS) {
+        for (int i = c.tid; i < k; i += MK_THREADS) {
           const float v = fmaf(fx_val(src[i]), scale, fx_val(pos[i]));
           if (out32) stc_f32(out32 + i, v);
           fx_stc(out + i, fx_round<E>(v));
@@ -113,7 +113,7 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
     }
 #endif
     if ((k & 3) == 0) {
-      for (int i = threadIdx.x * 4; i < k; i += MK_THREADS * 4) {
+      for (int i = c.tid * 4; i < k; i += MK_THREADS * 4) {
         f32x4 v;
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = fx_val(src[i + e]) * scale;
@@ -121,7 +121,7 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
         fx_stc_quad(out + i, v);
       }
     } else {
-      for (int i = threadIdx.x; i < k; i += MK_THREADS) {
+      for (int i = c.tid; i < k; i += MK_THREADS) {
         const float v = fx_val(src[i]) * scale;
         if (out32) stc_f32(out32 + i, v);
         fx_stc(out + i, fx_round<E>(v));
@@ -138,7 +138,7 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
 // Rows of up to 4096 values, four quads per thread.  Bound by the barrier and one round trip for the row: the slices of all quads are
 // requested before the first value is waited for (a branch around each quad had made a round trip per quad of it).
 // 4096 values from four slices, as a stage: 8.9 -> 6.7 us at 4 rows, 9.5 -> 7.1 at 64.
-__device__ __forceinline__ int fx_quad_at(int c0, int j, int n4) { return min(c0 + (int)threadIdx.x + j * MK_THREADS, n4 - 1); }
+__device__ __forceinline__ int fx_quad_at(const Ctx &c, int c0, int j, int n4) { return min(c0 + c.tid + j * MK_THREADS, n4 - 1); }
 // v = alpha * x + y of four quads of a row
 template <typename E>
 __device__ __forceinline__ void fx_addnorm_sum(CStage &st, const Ctx &c, int dS, int t, int c0, int n4, const f32x4 (&x)[4], f32x4 (&v)[4]) {
@@ -151,7 +151,7 @@ __device__ __forceinline__ void fx_addnorm_sum(CStage &st, const Ctx &c, int dS,
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int b = 0; b < Q; b++) q[j][b] = fx_ldc_quad(p + b * slice + 4 * fx_quad_at(c0, j, n4));
+        for (int b = 0; b < Q; b++) q[j][b] = fx_ldc_quad(p + b * slice + 4 * fx_quad_at(c, c0, j, n4));
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         v[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -164,7 +164,7 @@ __device__ __forceinline__ void fx_addnorm_sum(CStage &st, const Ctx &c, int dS,
     else sum_slices(std::integral_constant<int, 8>{});
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = st.in ? fx_ldc_quad((const E *)st.in + (size_t)t * st.ld_in + 4 * fx_quad_at(c0, j, n4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 4; j++) v[j] = st.in ? fx_ldc_quad((const E *)st.in + (size_t)t * st.ld_in + 4 * fx_quad_at(c, c0, j, n4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -181,7 +181,7 @@ __device__ __forceinline__ void fx_addnorm_store(CStage &st, int t, int s, f32x4
 }
 template <typename E>
 __device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char *smem) {
-  const int tid = threadIdx.x, n4 = st.n / 4;
+  const int tid = c.tid, n4 = st.n / 4;
   float *red = (float *)smem;
   const f32x4 *w4 = (const f32x4 *)st.norm_w;
   const float *xr = (const float *)st.res;
@@ -189,7 +189,7 @@ __device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char
   f32x4 x[4], v[4];
   auto load_x = [&](int t, int c0) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) x[j] = fx_ldc_quad(xr + (size_t)t * st.ld_res + 4 * fx_quad_at(c0, j, n4));
+    for (int j = 0; j < 4; j++) x[j] = fx_ldc_quad(xr + (size_t)t * st.ld_res + 4 * fx_quad_at(c, c0, j, n4));
   };
   auto squares = [&](int c0) {
     float ss = 0.f;
@@ -202,7 +202,7 @@ __device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char
   if (n4 <= 4 * MK_THREADS) {
     f32x4 g[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) g[j] = w4[fx_quad_at(0, j, n4)];
+    for (int j = 0; j < 4; j++) g[j] = w4[fx_quad_at(c, 0, j, n4)];
     // the residual row was written at least one barrier earlier than y: requested before the barrier is awaited (not by the
     // wavefront that polls it)
     const bool pre = (st.flags & MK_F_RES_EARLY) && t0 < M && tid >= 64;
@@ -440,7 +440,7 @@ __device__ __forceinline__ void stage_fx_prep(CStage &st, Ctx &c, const MkRuntim
   barrier_wait(c);
   constexpr int KW = FxType<E>::KW;
   const FxRows<E> rows = fx_rows<E>(st, c);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   const int H = st.num_q_heads, nkv = st.num_kv_heads, D = st.head_dim, DV = st.v_dim;
   const int nkc = (D + KW - 1) / KW, nvb = (DV + 15) / 16, ps = rt.page_size;
   const int per = H + 2 * nkv, total = M * per;
@@ -532,7 +532,7 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
   using X = FxType<E>;
   constexpr int EPC = X::EPC, KW = X::KW, TP = X::TP, SUB = X::SUB;
   constexpr int PSTR = VB * 16 + 4, PST = VB * 16 + 32;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const int nkv = st.num_kv_heads, qpk = st.num_q_heads / nkv, D = st.head_dim, DV = st.v_dim;
   const int nkc = (D + KW - 1) / KW, nkg = (nkc + KC - 1) / KC, nvb = (DV + 15) / 16, nvs = (nvb + VB - 1) / VB;
@@ -1028,7 +1028,7 @@ template <int MT, bool SILU>
 __device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int NH = SILU ? 2 : 1, NT = NH + MT, D = MT == 1 ? 8 : 4;  // 16-row tiles of a step: weights, then tokens
   constexpr bool DB = NH * MT < 8;                                       // sums of two units fit beside the operands
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4, l8 = lane >> 3, c8 = lane & 7;
   const int K = st.k, n_out = SILU ? st.n / 2 : st.n, half = st.silu_half, nks = K / 16;  // (16 k of a tile are one operand)
   const int ng = (M + 16 * MT - 1) / (16 * MT), n_units = (n_out + 15) / 16 * ng;
@@ -1179,7 +1179,7 @@ __device__ __forceinline__ void stage_fx_argmax_f32(CStage &st, Ctx &c, const Mk
   const int n = st.n, per = (n + c.G - 1) / c.G, c0 = c.vid * per, c1 = min(n, c0 + per);
   float *pv = rt.argmax_pv ? rt.argmax_pv : (float *)st.aux0;
   int *pi = rt.argmax_pv ? rt.argmax_pi : (int *)st.aux1;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   for (int t = wave; t < M; t += MK_WAVES) {
     const float *row = (const float *)st.in + (size_t)t * st.ld_in;
     float best = -INFINITY;

@@ -21,7 +21,7 @@ __device__ __forceinline__ void stage_hy_conv(CStage &st, Ctx &c, const MkRuntim
   const int n = st.n, n4 = n / 4, taps = st.taps, per = (n4 + MK_THREADS - 1) / MK_THREADS;
   const float *w = (const float *)st.norm_w;
   for (int i = mx_spread(c); i < M * per; i += c.G) {
-    const int t = i / per, q = (i - t * per) * MK_THREADS + threadIdx.x;
+    const int t = i / per, q = (i - t * per) * MK_THREADS + c.tid;
     if (q >= n4) continue;
     const int t0 = __builtin_amdgcn_readfirstlane(c.sh_tok[2 * MK_MAX_TOKENS + t]), pos = __builtin_amdgcn_readfirstlane(c.sh_tok[t]);
     const int slot = __builtin_amdgcn_readfirstlane(rt.state_ids[__builtin_amdgcn_readfirstlane(c.sh_tok[MK_MAX_TOKENS + t])]);
@@ -67,7 +67,7 @@ template <typename E, int Q, int TB, int CH>
 __device__ __forceinline__ void stage_hy_scan_t(CStage &st, Ctx &c, const MkRuntime &rt, int M, int lg2) {
   constexpr int KK = (TB * CH + 3) / 4;  // (outputs a lane finishes, with the fewest lanes per channel)
   const int L = 1 << lg2, GW = 64 >> lg2, CW = MK_WAVES * GW * CH;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & (L - 1);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & (L - 1);
   const int n = st.n, Np = (st.states + 3) / 4 * 4, nblk = (n + CW - 1) / CW;
   const MxDeltaUnits us = mx_delta_units(c, M);
   const int n_units = us.nreq * nblk;
@@ -385,7 +385,7 @@ __device__ __forceinline__ void hy_route_store(CStage &st, int t, int lane, floa
 // (iterations of several tokens; a single token is routed by the expert stage itself)
 __device__ __forceinline__ void stage_hy_route(CStage &st, Ctx &c, int M, char *smem) {
   barrier_wait(c);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   for (int t = mx_wave_item(c, wave); t < M; t += c.G * MK_WAVES) {
     float w;
     int id;
@@ -469,9 +469,9 @@ constexpr int HY_FIRST = 8;  // steps of the ring that may have been requested i
 // Walk the units of `rg`.  ks wavefronts (4, 2 or 1) split the reduction of a pair of tiles.  w: the ring, its first steps requested if
 // `early`.  row_words: 16-byte words per row where all rows of a single token lie in LDS (row of place p at p * row_words; 0: one row).
 template <typename E, int D, bool XLDS>
-__device__ __forceinline__ void hy_expert_walk(CStage &st, const HyLists *ls, int M, const HyRange rg, int ks, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
+__device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const HyLists *ls, int M, const HyRange rg, int ks, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const bool glu = st.flags & MK_F_SILU;
   u32x4 *xl = (u32x4 *)(smem + HY_X);
   f32x4 *red = (f32x4 *)(smem + HY_RED);
@@ -598,7 +598,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const HyLists *ls, in
 template <typename E, int MAXM>
 __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Ex = st.num_experts, topk = st.topk;
   // short reductions are split among fewer wavefronts, so that each of them has a ring's worth of steps
   const int nks = st.k / KW, ks = nks >= 48 ? 4 : nks >= 24 ? 2 : 1, ppu = MK_WAVES / ks;  // pairs of tiles per unit
@@ -706,9 +706,9 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   if (rg.s0 < rg.s1 || rg.r0 < rg.r1) {
     // a ring of 8 steps per tile, or of 12 where a wavefront's share of the reduction is then walked with fewer empty steps
     const int kq = (nks + ks - 1) / ks;
-    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, ls, M, rg, ks, early, w, false, 0, smem);
-    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
-    else hy_expert_walk<E, 12, true>(st, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, c, ls, M, rg, ks, early, w, false, 0, smem);
+    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, c, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    else hy_expert_walk<E, 12, true>(st, c, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
   }
   c.wrote_through = true;
 }

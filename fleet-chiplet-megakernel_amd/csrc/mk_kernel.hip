@@ -91,6 +91,8 @@ typedef const __attribute__((address_space(4))) MkWeight CWeight;
 #endif
 
 struct Ctx {
+  int tid;   // threadIdx.x, made opaque for every stage that runs: see run_stage_program
+  CStage *st;  // descriptor of the stage that runs (null before the first one)
   int vid;   // virtual workgroup id: xcd-major, so vids [x*quota, (x+1)*quota) share an L2
   int G;     // workgroups in the grid
   int xcd;   // XCC_ID of the CU this workgroup landed on
@@ -364,7 +366,15 @@ __device__ __forceinline__ void barrier_done(Ctx &c) {
 
 __device__ __forceinline__ void barrier_wait(Ctx &c) {
   if (!c.pending) return;
-  if (threadIdx.x == 0) barrier_poll(c);
+  if (threadIdx.x == 0) {
+    // The polling wavefront brings the stage's descriptor into the scalar cache: its misses would otherwise follow one another behind the
+    // barrier.  (By every wavefront, ahead of the stage, it had held up the requests for weights: a prompt of qwen3-8b 68.0 -> 70.0 ms.)
+    typedef const __attribute__((address_space(4))) int CInt;
+    CInt *d = (CInt *)c.st;
+    static_assert(sizeof(MkStage) == 11 * 64, "one word of every line");
+    if (d) asm volatile("" ::"s"(d[0]), "s"(d[16]), "s"(d[32]), "s"(d[48]), "s"(d[64]), "s"(d[80]), "s"(d[96]), "s"(d[112]), "s"(d[128]), "s"(d[144]), "s"(d[160]));
+    barrier_poll(c);
+  }
   __syncthreads();
   barrier_done(c);
 }
@@ -786,7 +796,7 @@ __device__ __forceinline__ void stage_embed(CStage &st, Ctx &c, const MkRuntime 
     const u32x4 *src = (const u32x4 *)st.w.seg[0] + (size_t)(id < 0 ? 0 : id) * k8;
     u32x4 *dst = (u32x4 *)st.out + (size_t)t * (st.ld_out / 8);
     const u32x4 zero = {0u, 0u, 0u, 0u};
-    for (int i = threadIdx.x; i < k8; i += MK_THREADS) dst[i] = id < 0 ? zero : src[i];
+    for (int i = c.tid; i < k8; i += MK_THREADS) dst[i] = id < 0 ? zero : src[i];
   }
 }
 
@@ -810,7 +820,7 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 // 4096 values from four slices, as a stage: 8.4 -> 7.3 us.
 template <int NS>
 __device__ __forceinline__ void stage_norm_rows(CStage &st, Ctx &c, int M, char *smem) {
-  const int tid = threadIdx.x, k8 = st.k / 8;
+  const int tid = c.tid, k8 = st.k / 8;
   float *red = (float *)smem;
   const u32x4 *w4 = (const u32x4 *)st.norm_w;
   auto at = [&](int j) { return min(tid + j * MK_THREADS, k8 - 1); };
@@ -922,14 +932,14 @@ __device__ __forceinline__ void stage_norm(CStage &st, Ctx &c, int M, char *smem
     const uint32_t *w = (const uint32_t *)st.norm_w;
     uint32_t *y = (uint32_t *)st.out + (size_t)t * (st.ld_out / 2);
     float ss = 0.f;
-    for (int i = threadIdx.x; i < k2; i += MK_THREADS) {
+    for (int i = c.tid; i < k2; i += MK_THREADS) {
       const uint32_t u = ldc_u32(x + i);
       xs[i] = u;
       ss += bf_lo(u) * bf_lo(u) + bf_hi(u) * bf_hi(u);
     }
     ss = block_sum(ss, red);
     const float r = rsqrtf(ss / (float)st.k + st.eps);
-    for (int i = threadIdx.x; i < k2; i += MK_THREADS) {
+    for (int i = c.tid; i < k2; i += MK_THREADS) {
       const uint32_t u = xs[i], g = w[i];
       y[i] = pack2((bf_lo(u) * r) * bf_lo(g), (bf_hi(u) * r) * bf_hi(g));
     }
@@ -972,7 +982,7 @@ __device__ __forceinline__ bool mx_prenorm_by_wave(CStage &st) { return st.k <= 
 // FX: the norm in front may be an FX_ADDNORM (see mk_flex.hip): alpha * residual + y, both rows in memory, then the norm.
 template <bool FX>
 __device__ __forceinline__ void stage_x_m1(CStage &st, const Ctx &c, uint32_t *xs, float *red) {
-  const int tid = threadIdx.x, k4 = st.k / 4;
+  const int tid = c.tid, k4 = st.k / 4;
   const unsigned long long *xin = (const unsigned long long *)st.in;
   unsigned long long *xs2 = (unsigned long long *)xs;
   if constexpr (FX) {
@@ -1143,7 +1153,7 @@ __device__ __forceinline__ void stage_x_m1_addnorm_wave(CStage &st, Ctx &c, uint
 // (tasks/mi300/gang_linear_mi300.cuh:359-576).
 template <int KL, int R, bool SILU, bool W0OK, bool FX>
 __device__ __forceinline__ void stage_linear_m1_t(CStage &st, Ctx &c, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int K8 = KL * 64;
   constexpr int NROW = SILU ? 2 : 1;  // weight rows per output ([gate ; up] pair)
   constexpr int U = R / NROW;         // outputs in flight per worker wavefront
@@ -1327,7 +1337,7 @@ __device__ __forceinline__ void stage_linear_m1_t(CStage &st, Ctx &c, char *smem
 // instantiation: same arithmetic, no cross-barrier prefetch.
 template <bool FX>
 __device__ __forceinline__ void stage_linear_m1_generic(CStage &st, Ctx &c, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = st.k, k8 = K / 8;
   uint32_t *xs = (uint32_t *)smem;
   float *red = (float *)(smem + MK_RED_OFFSET);
@@ -1411,7 +1421,7 @@ __device__ __forceinline__ void stage_linear_m1(CStage &st, Ctx &c, char *smem) 
 // [token][output] and written through.
 template <int KL, int R, bool SILU, int MB>
 __device__ __forceinline__ void stage_linear_small(CStage &st, Ctx &c, int M, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int K8 = KL * 64;
   constexpr int NROW = SILU ? 2 : 1;
   constexpr int U = R / NROW;
@@ -1687,10 +1697,10 @@ template <int MT>
 __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, const MkRuntime &rt, int M, const TilePlan plan, char *smem) {
   barrier_wait(c);
   c.wrote_through = true;  // partial tiles and outputs are all written through: no L2 write-back at this stage's arrival
-  if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   __syncthreads();
   MK_MARK(c, 0);
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const bool silu = st.flags & MK_F_SILU;
   const int K = st.k, k8 = K / 8;
@@ -1967,7 +1977,7 @@ template <int MT, int TW>
 __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const MkRuntime &rt, int M, const XresPlan plan, char *smem) {
   c.wrote_through = true;  // partial tiles and outputs are all written through: no L2 write-back at this stage's arrival
   constexpr int NSP = MK_XRES_STEPS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const bool silu = st.flags & MK_F_SILU;
   const int K = st.k, k8 = K / 8;
@@ -2300,11 +2310,11 @@ __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, cha
   // activations were produced by other workgroups: drop what this die's caches hold of them once, then use cached loads
   // so the rows are shared through the die's L2.  (Issued before the barrier is awaited: nothing on this die reads
   // the stage's input buffers between their previous consumer and this barrier.)
-  if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
   c.wrote_through = true;  // outputs are written through: no L2 write-back at this stage's arrival
   MK_MARK(c, 0);
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const bool silu = st.flags & MK_F_SILU;
   const int K = st.k, k8 = K / 8;
@@ -2460,7 +2470,7 @@ __device__ __forceinline__ void stage_silu_mul(CStage &st, Ctx &c, int M) {
   const uint16_t *in = (const uint16_t *)st.in;
   uint16_t *out = (uint16_t *)st.out;
   const int total = M * (st.topk > 0 ? st.topk : 1) * n;  // MoE: topk rows per token, contiguous
-  for (int i = c.vid * MK_THREADS + threadIdx.x; i < total; i += c.G * MK_THREADS) {
+  for (int i = c.vid * MK_THREADS + c.tid; i < total; i += c.G * MK_THREADS) {
     const int t = i / n, j = i - t * n;
     const int g = j / half, jj = j - g * half;
     const uint16_t *row = in + (size_t)t * st.ld_in + (size_t)g * 2 * half;
@@ -2474,7 +2484,7 @@ __device__ __forceinline__ void stage_copy(CStage &st, Ctx &c, int M) {
   const uint16_t *in = (const uint16_t *)st.in;
   uint16_t *out = (uint16_t *)st.out;
   const long long total = (long long)M * st.n;
-  for (long long i = (long long)c.vid * MK_THREADS + threadIdx.x; i < total; i += (long long)c.G * MK_THREADS) stc_u16(out + i, ldc_u16(in + i));
+  for (long long i = (long long)c.vid * MK_THREADS + c.tid; i < total; i += (long long)c.G * MK_THREADS) stc_u16(out + i, ldc_u16(in + i));
   c.wrote_through = true;
 }
 
@@ -2585,7 +2595,7 @@ __device__ __forceinline__ void moe_route_wave(const uint16_t *logits, int E, in
 // column of the routing table.  Columns of tokens that are not part of the iteration are left alone.
 __device__ __forceinline__ void stage_moe_topk(CStage &st, Ctx &c, int M) {
   barrier_wait(c);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   const int E = st.num_experts;
   for (int t = c.vid * MK_WAVES + wave; t < M; t += c.G * MK_WAVES) {
     int sel[4];
@@ -2603,8 +2613,8 @@ __device__ __forceinline__ void stage_moe_topk(CStage &st, Ctx &c, int M) {
 // Build the active-expert list and the (token, slot) pairs of every active expert from the routing table.
 // Single-token iterations keep slot order (active expert s is the expert of slot s); multi-token iterations list
 // experts in ascending id with their tokens in ascending order.
-__device__ __forceinline__ void moe_build_lists(CStage &st, MoeLds *L, int M, bool r_in_lds) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+__device__ __forceinline__ void moe_build_lists(CStage &st, const Ctx &c, MoeLds *L, int M, bool r_in_lds) {
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int E = st.num_experts;
   if (M == 1) {
     if (tid <= st.topk) {  // slot s is "active expert" s; a slot no expert claims (caller-written table) stays empty
@@ -2683,7 +2693,7 @@ __device__ __forceinline__ void moe_build_lists(CStage &st, MoeLds *L, int M, bo
 template <int KL, int R, bool SILU>
 __device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int NROW = SILU ? 2 : 1;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
   const int k8 = st.k / 8;
   const bool combine = !SILU && (st.flags & MK_F_MOE_COMBINE) && M == 1;
@@ -2714,7 +2724,7 @@ __device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, int M, ch
   } else if (combine && tid < st.topk) {
     L->w[tid] = ldc_f32(st.moe_topk_w + tid);
   }
-  moe_build_lists(st, L, M, inline_topk);
+  moe_build_lists(st, c, L, M, inline_topk);
   const int n_act = L->n_act;
   if (c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)
     for (int i = tid; i < st.num_experts; i += MK_THREADS) st.moe_mask[i] = i < n_act ? L->act_e[i] : -1;
@@ -2831,7 +2841,7 @@ template <int KL, int R, bool SILU>
 __device__ __forceinline__ void stage_moe_linear_m1(CStage &st, Ctx &c, char *smem) {
   constexpr int TK = 8;
   constexpr int NSUB = SILU ? 2 : TK;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
   const int k8 = st.k / 8, topk = st.topk, E = st.num_experts;
   const bool ctrl = wave == 0;
@@ -3097,7 +3107,7 @@ template <int KL, int R, bool SILU>
 __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int NROW = SILU ? 2 : 1;
   constexpr int NARR = SILU ? 3 : 1;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = c.tid, lane = tid & 63;
   MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
   const int k8 = st.k / 8;
   const int n_act = L->n_act;
@@ -3335,13 +3345,13 @@ __device__ __forceinline__ void stage_moe_linear(CStage &st, Ctx &c, int M, char
     // common front: wait for the previous stage, one acquire (activation rows are read with cached loads), routing lists
     MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
     barrier_wait(c);
-    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
-    moe_build_lists(st, L, M, false);
+    moe_build_lists(st, c, L, M, false);
     if (c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)
       const int n_act = L->n_act;
-      for (int i = threadIdx.x; i < st.num_experts; i += MK_THREADS) st.moe_mask[i] = i < n_act ? L->act_e[i] : -1;
-      if (threadIdx.x == 0) st.moe_mask[st.num_experts] = n_act;
+      for (int i = c.tid; i < st.num_experts; i += MK_THREADS) st.moe_mask[i] = i < n_act ? L->act_e[i] : -1;
+      if (c.tid == 0) st.moe_mask[st.num_experts] = n_act;
     }
     if (st.k <= 1024) {
       if (silu) stage_moe_linear_multi<2, 4, true>(st, c, M, smem);
@@ -3375,7 +3385,7 @@ __device__ __forceinline__ void stage_moe_combine(CStage &st, Ctx &c, int M) {
   const int n = st.n, total = M * n;
   const uint16_t *in = (const uint16_t *)st.in, *res = (const uint16_t *)st.res;
   uint16_t *out = (uint16_t *)st.out;
-  for (int i = c.vid * MK_THREADS + threadIdx.x; i < total; i += c.G * MK_THREADS) {
+  for (int i = c.vid * MK_THREADS + c.tid; i < total; i += c.G * MK_THREADS) {
     const int t = i / n, j = i - t * n;
     float s = bf2f(ldc_u16(res + (size_t)t * st.ld_res + j));
     for (int k = 0; k < st.topk; k++)
@@ -3463,7 +3473,7 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
   constexpr int NPRE = MK_TUNE_NPRE;          // positions per lane group requested ahead
   constexpr int DPT = QPK * D / MK_THREADS;   // merged outputs per thread (all of one head)
   constexpr int TPH = D / DPT;                // threads per head in the merges
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j16 = lane & 15, gg = wave * 4 + (lane >> 4);
   const int nkv = st.num_kv_heads;
   // LDS: q rows, then the K and V rows of this iteration's new positions (a request ingests up to MK_MAX_NEW_PER_REQ prompt
@@ -4041,7 +4051,7 @@ __device__ __forceinline__ void stage_argmax_partial(CStage &st, Ctx &c, const M
   const int c0 = c.vid * per, c1 = min(n, c0 + per);
   float *pv = rt.argmax_pv ? rt.argmax_pv : (float *)st.aux0;
   int *pi = rt.argmax_pv ? rt.argmax_pi : (int *)st.aux1;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   constexpr int NDW = 5, TB = 4;  // dwords per lane per token, tokens in flight per wavefront
   const int nd = (c1 - c0 + 1) / 2;
   // one wavefront per token, TB tokens' slices requested together; slices longer than NDW * 64 dwords loop
@@ -4089,7 +4099,7 @@ __device__ __forceinline__ void stage_argmax_reduce(CStage &st, Ctx &c, const Mk
   const float *pv = rt.argmax_pv ? rt.argmax_pv : (const float *)st.aux0;
   const int *pi = rt.argmax_pv ? rt.argmax_pi : (const int *)st.aux1;
   long long *out = (long long *)st.out;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   for (int t = c.vid * MK_WAVES + wave; t < M; t += c.G * MK_WAVES) {
     float best = -INFINITY;
     int bi = 0x7fffffff;
@@ -4279,6 +4289,14 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         CStage &nx = ((CStage *)(unsigned long long)rt.stages)[s + 1];
         if (nx.op == MK_OP_LINEAR && (nx.flags & MK_F_NORM) && nx.in == st.in && linear_small_ok(nx, c, M)) continue;
       }
+      // Lane offsets that stages derive from the thread index would otherwise be computed once, ahead of all stages, and wait in scratch
+      // for the stage that wants them, which then starts with a chain of scratch loads.  Scratch per lane: 480 -> 0 bytes (fixed-shape
+      // stages), 640 -> 0 (flex), 1568 -> 0 (mix), 1648 -> 0 (hybrid), 2320 -> 624 (dual); vizonex-8b at 64 streams 95.5 -> 85.4 ms,
+      // bukatar-8b 57.0 -> 52.5, suborax-8b serving 135 -> 131.
+      c.tid = threadIdx.x;
+      asm volatile("" : "+v"(c.tid));
+      __builtin_assume(c.tid >= 0 && c.tid < MK_THREADS);
+      c.st = &st;
       const long long t_in = (long long)wall_clock64();
       switch (op) {
 #if MK_HAVE_FLEX
@@ -4453,6 +4471,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   c.state_ids = rt.state_ids;
 #endif
   c.prof_n = 0;
+  c.st = nullptr;
   c.defer_S = 0;
   c.wrote_through = false;
   c.arrive_w0 = false;

@@ -96,7 +96,7 @@ __device__ __forceinline__ f32x4 mx_ring_conv(CStage &st, const E *ring, int n, 
 // request brings one token also out3 = the normed row plus its convolution over time, which keeps the row in the request's ring.
 template <typename E, int NS>
 __device__ __forceinline__ void stage_mx_prenorm_t(CStage &st, Ctx &c, int M, bool single, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n4 = st.n / 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n4 = st.n / 4;
   float *red = (float *)smem, *gs = red + 64, *row = gs + MK_MX_MAX_GROUPS;
   const int ng = st.norm_groups, gl = ng ? st.k / ng : st.k;
   const f32x4 *w4 = (const f32x4 *)st.norm_w, *yw4 = (const f32x4 *)st.y_norm_w;
@@ -284,7 +284,7 @@ __device__ __forceinline__ void mx_norm_row(const E *src, const float *w, int n,
 template <typename E>
 __device__ __forceinline__ void stage_mx_norm_parts(CStage &st, Ctx &c, int M) {
   barrier_wait(c);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ng = st.norm_groups, gl = st.k / ng;
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6), ng = st.norm_groups, gl = st.k / ng;
   for (int i = mx_wave_item(c, wave); i < M * ng; i += c.G * MK_WAVES) {
     const int t = i / ng, q = i - t * ng;
     E *o = (E *)st.out + (size_t)t * st.ld_out + q * gl;
@@ -307,7 +307,7 @@ __device__ __forceinline__ void stage_mx_prenorm(CStage &st, Ctx &c, int M, bool
 
 // The same in front of a single-token bf16 linear, whose input row it leaves in LDS (virtual workgroup 0 also stores the rows).
 __device__ __forceinline__ void mx_x_m1_prenorm(CStage &st, const Ctx &c, uint32_t *xs, float *red) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), k4 = st.k / 4, ng = st.norm_groups, gl = st.k_real / ng;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), k4 = st.k / 4, ng = st.norm_groups, gl = st.k_real / ng;
   f32x4 *vs = (f32x4 *)((char *)xs + MK_MOE_OFFSET);  // the sum, 32-bit
   float *gs = (float *)((char *)xs + MK_MOE_OFFSET + 12 * 4 * 4 * MK_THREADS);
   float f = 1.f;
@@ -489,14 +489,15 @@ template <int NS>
 struct MxPrologue {
   f32x4 g[NS], x[NS], ys[NS], y2s[NS];
   unsigned long long cw[NS][MX_EARLY_TAPS], ring[NS][MX_EARLY_TAPS];
-  int pos, k4;
+  int tid, pos, k4;
   uint16_t *rows;
-  __device__ __forceinline__ int at(int j) const { return min((int)threadIdx.x + j * MK_THREADS, k4 - 1); }
+  __device__ __forceinline__ int at(int j) const { return min(tid + j * MK_THREADS, k4 - 1); }
   __device__ __forceinline__ void load_x(CStage &st) {
 #pragma unroll
     for (int j = 0; j < NS; j++) x[j] = fx_ldc_quad((const float *)st.res + 4 * at(j));
   }
   __device__ __forceinline__ void load(CStage &st, const Ctx &c) {
+    tid = c.tid;
     k4 = st.k / 4;
     pos = __builtin_amdgcn_readfirstlane(c.sh_tok[0]);
     const f32x4 one = {1.f, 1.f, 1.f, 1.f};
@@ -524,7 +525,6 @@ struct MxPrologue {
   __device__ __forceinline__ void finish(CStage &st, const Ctx &c, uint32_t *xs, float *red) {
     auto quad = [](unsigned long long u) { return (f32x4){bf_lo((uint32_t)u), bf_hi((uint32_t)u), bf_lo((uint32_t)(u >> 32)), bf_hi((uint32_t)(u >> 32))}; };
     auto pack = [](f32x4 o) { return (unsigned long long)pack2(o[0], o[1]) | ((unsigned long long)pack2(o[2], o[3]) << 32); };
-    const int tid = threadIdx.x;
     if (!(st.flags & MK_F_RES_EARLY)) load_x(st);
     if (st.y_in) {
       f32x4 y[NS], y2[NS];
@@ -586,7 +586,7 @@ __device__ __forceinline__ bool mx_dual_prenorm(CStage &) { return false; }
 // PRO: the row comes from an MxPrologue of that many quads per thread (dual kernels; 0: it does not).
 template <int R, int U, int PRO = 0>
 __device__ __forceinline__ void stage_mx_linear_m1_t(CStage &st, Ctx &c, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = st.k, k8 = K / 8, nkb = (k8 + 64 * U - 1) / (64 * U), n = st.n;
   u32x4 *xs4 = (u32x4 *)smem;
   const int nw = c.G * MK_WAVES, id = c.vid * MK_WAVES + wave, q = n / nw, rem = n - q * nw;
@@ -684,7 +684,7 @@ __device__ __forceinline__ void mx_glu(CStage &st, Ctx &c, int M) {
   const int n = st.glu_n, per = (n + 4 * MK_THREADS - 1) / (4 * MK_THREADS), total = M * per;
   const float lim = st.glu_limit, beta = st.glu_beta, bias = st.glu_bias;
   for (int i = c.G - 1 - mx_spread(c); i < total; i += c.G) {
-    const int t = i / per, d = (i - t * per) * 4 * MK_THREADS + 4 * threadIdx.x;
+    const int t = i / per, d = (i - t * per) * 4 * MK_THREADS + 4 * c.tid;
     if (d >= n) continue;
     const E *row = (const E *)st.in + (size_t)t * st.ld_in;
     const f32x4 a = fx_ldc_quad(row + st.glu_gate + d), b = fx_ldc_quad(row + st.glu_up + d);
@@ -735,7 +735,7 @@ template <typename E>
 __device__ __forceinline__ void stage_mx_latent_prep(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
   barrier_wait(c);
   constexpr int KW = FxType<E>::KW;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   const int R = st.rank, rot = st.rot_dims, half = rot / 2, nrc = (R + KW - 1) / KW, nkc = nrc + (rot + KW - 1) / KW, ps = rt.page_size;
   const int nq = st.n > 0, per = nq + (st.k_cache ? 1 : 0), total = M * per;  // (a model may form its queries without a latent)
   for (int i = mx_wave_item(c, wave); i < total; i += c.G * MK_WAVES) {
@@ -782,7 +782,7 @@ template <typename E, int MT, int EPI, bool SPLIT>
 __device__ __forceinline__ void stage_mx_head_linear_t(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW, KB = MT == 4 ? 4 : SPLIT ? 16 : EPI == MX_DECAY ? 4 : 8, B16 = sizeof(E) == 2;
   static_assert(!SPLIT || MT == 1, "");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int N = st.n, nks = st.k / KW, nt = (N + 15) / 16, mts = MT == 1 ? (M + 15) / 16 : 1, items = st.groups * nt * mts;
   const int kq = SPLIT ? (nks + MK_WAVES - 1) / MK_WAVES : nks;
   const int kb = SPLIT ? min(nks, wave * kq) : 0, ke = SPLIT ? min(nks, kb + kq) : nks;
@@ -924,7 +924,7 @@ struct MxLatentRows {
   int my_n, my_tiles, tiles_incl, total, cmax;
 };
 __device__ __forceinline__ MxLatentRows mx_latent_rows(const Ctx &c, int M, int H, int unit_rows) {
-  const int lane = threadIdx.x & 63;
+  const int lane = c.tid & 63;
   MxLatentRows r;
   const bool first = lane < M && c.sh_tok[2 * MK_MAX_TOKENS + lane] == lane;
   const unsigned long long fm = __ballot(first), later = lane < 63 ? fm >> (lane + 1) : 0ull;
@@ -967,7 +967,7 @@ __device__ __forceinline__ void stage_mx_latent_attn_t(CStage &st, Ctx &c, const
   constexpr int EPC = X::EPC, KW = X::KW, B16 = sizeof(E) == 2, TPOS = 16 * SUB, PARTS = MK_WAVES / SUB, KC = (NK + PARTS - 1) / PARTS;
   constexpr int QN = RT * NK * 64 / MK_THREADS, GRP = NK % 6 == 0 ? 6 : 5;
   static_assert(RT * NK % 4 == 0, "whole rounds of query operands");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int H = st.num_q_heads, R = st.rank, rot = st.rot_dims, half = rot / 2;
   const int nrc = (R + KW - 1) / KW, npc = (rot + KW - 1) / KW, nkc = nrc + npc, nvb = nrc * KW / 16, Rp = nrc * KW, PST = Rp + 32;
   const int ps = rt.page_size;
@@ -1270,7 +1270,7 @@ template <typename E>
 __device__ __forceinline__ void stage_mx_latent_merge(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
   barrier_wait(c);
   constexpr int KW = FxType<E>::KW;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int H = st.num_q_heads, Rp = (st.rank + KW - 1) / KW * KW, PST = Rp + 32, UR = 16 * st.v_tiles, TPOS = 16 * st.k_tiles;
   const MxLatentRows rw = mx_latent_rows(c, M, H, UR);
   const bool few = rw.cmax <= 8;
@@ -1346,7 +1346,7 @@ struct MxDeltaUnits {
   int my_n, rank_of, nreq;
 };
 __device__ __forceinline__ MxDeltaUnits mx_delta_units(const Ctx &c, int M) {
-  const int lane = threadIdx.x & 63;
+  const int lane = c.tid & 63;
   MxDeltaUnits r;
   r.first = lane < M && c.sh_tok[2 * MK_MAX_TOKENS + lane] == lane;
   const unsigned long long fm = __ballot(r.first), later = lane < 63 ? fm >> (lane + 1) : 0ull;
@@ -1426,7 +1426,7 @@ __device__ __forceinline__ void mx_delta_step(f32x4 (&S)[NC][NI], const MxDeltaV
 // every request brings one token
 template <typename E, int NI, int NC>
 __device__ __forceinline__ void stage_mx_delta_single(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int D = st.head_dim, Dp = (D + 15) / 16 * 16, H = st.num_q_heads, n_units = M * H, col = (wave * 4 + lg) * NC;
   const MxDeltaUnits us = mx_delta_units(c, M);
   const E *in = (const E *)st.in;
@@ -1533,7 +1533,7 @@ __device__ __forceinline__ void stage_mx_delta_single(CStage &st, Ctx &c, const 
 template <typename E, int NI, int NC>
 __device__ __forceinline__ void stage_mx_delta_multi(CStage &st, Ctx &c, const MkRuntime &rt, int M, int slices, char *smem) {
   constexpr int DPS = NI * 64 + 4, TW = MX_TB / MK_WAVES;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int D = st.head_dim, Dp = (D + 15) / 16 * 16, H = st.num_q_heads, cw = (wave * 4 + lg) * NC, d4 = min(4 * lane, Dp - 4);
   float *rv = (float *)smem, *kv = rv + MX_TB * DPS, *uv = kv + MX_TB * DPS, *av = uv + MX_TB * DPS, *wv = av + MX_TB * DPS, *vv = wv + MX_TB * DPS, *ov = vv + MX_TB * DPS;
   const MxDeltaUnits us = mx_delta_units(c, M);
@@ -1653,7 +1653,7 @@ __device__ __forceinline__ void stage_mx_delta_multi(CStage &st, Ctx &c, const M
 // Head outputs of an iteration whose units were dealt in slices: a wavefront per (token, head).
 template <typename E>
 __device__ __forceinline__ void stage_mx_delta_out(CStage &st, Ctx &c, int M) {
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
   const int D = st.head_dim, Dp = (D + 15) / 16 * 16, H = st.num_q_heads, d4 = min(4 * lane, Dp - 4);
   barrier_wait(c);
   for (int i = mx_wave_item(c, wave); i < M * H; i += c.G * MK_WAVES) {
