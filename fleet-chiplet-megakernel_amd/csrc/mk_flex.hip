@@ -252,14 +252,22 @@ template <typename E> struct FxRows {
   const float *part;
   size_t slice, ldp;
   const float *bias;  // (hybrid kernels) added to every row where it is used, null: none
-  template <int NS> __device__ __forceinline__ float get(int tok, int col) const {
+  // what one element is made of: the linear's output, or its slices ...
+  template <int NS> __device__ __forceinline__ void request(int tok, int col, float (&q)[NS ? NS : 1]) const {
     if constexpr (NS == 0) {
-      return fx_ldc(in + (size_t)tok * ld + col);
+      q[0] = fx_ldc(in + (size_t)tok * ld + col);
     } else {
       const float *p = part + (size_t)tok * ldp + col;
-      float q[NS], s = 0.f;
 #pragma unroll
       for (int b = 0; b < NS; b++) q[b] = ldc_f32(p + b * slice);
+    }
+  }
+  // ... and its value, rounded as the linear would have
+  template <int NS> static __device__ __forceinline__ float value(const float (&q)[NS ? NS : 1]) {
+    if constexpr (NS == 0) {
+      return q[0];
+    } else {
+      float s = 0.f;
 #pragma unroll
       for (int b = 0; b < NS; b++) s += q[b];
       return fx_val(fx_round<E>(s));
@@ -278,31 +286,42 @@ template <typename E> __device__ __forceinline__ FxRows<E> fx_rows(CStage &st, C
   c.defer_S = 0;
   return r;
 }
-#define MK_FX_HEAD_REGS (MK_FX_MAX_HEAD_DIM / 64)
-// One query or key head row by one wavefront: dims [0, rot) are rotated (dim i < rot / 2 pairs with i + rot / 2), then the
-// row is divided by sqrt(mean(x^2) + eps) when the stage asks for it.  Split in a half that requests everything and a half
-// that computes, so that a wavefront can have the requests of two rows in flight; put(d, value) for every d < D.
+// f(registers a head row takes per lane)
+template <typename F> __device__ __forceinline__ void fx_head_regs(int D, int DV, F f) {
+  if (max(D, DV) <= 128) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, MK_FX_MAX_HEAD_DIM / 64>{});
+}
+// One query or key head row by one wavefront, lane l holding every 64th column: dims [0, rot) are rotated (dim i < rot / 2 pairs with
+// i + rot / 2), then the row is divided by sqrt(mean(x^2) + eps) when the stage asks for it; put(d, value) for every d < D.  A value
+// row is copied as it is.
+//
+// Bound by round trips: a wavefront requests two rows with all their slices at once, and partners of the rotation change lanes in the
+// wavefront's own LDS.  (A branch around every 64 columns, and a second request for the partners, had made four to eight trips of a row.)
+// Heads of up to 128 columns have their own form (R = 2 registers a row): branches past six more blocks of every loop had each been a fetch
+// of instructions.  Rows ready after the barrier of the attention stage, 32 q / 8 kv heads of 128, four streams: 9.5 -> 5.0 us; prep stage
+// of 64 tokens 7.3 -> 4.0 us.
 //
 // Dual kernels, MK_F_ROW_NORM: the row's query heads (its key heads) are together divided by their root mean square and multiplied
 // by a weight per column instead; `r` is that factor, `w` the weights.
-struct FxHead {
-  float x[MK_FX_HEAD_REGS], xp[MK_FX_HEAD_REGS], cs[MK_FX_HEAD_REGS], sn[MK_FX_HEAD_REGS];
+template <int R> struct FxHead {
+  float x[R], cs[R], sn[R];
 #if MK_HAVE_HYB
-  float b[MK_FX_HEAD_REGS], bp[MK_FX_HEAD_REGS];  // bias of x and xp
+  float b[R];  // bias of x
 #endif
 #if MK_HAVE_DUAL
-  float r, w[MK_FX_HEAD_REGS];
+  float r, w[R];
 #endif
 };
 #if MK_HAVE_DUAL
 // Weights of the row norm for the head whose columns begin at `col`.
-__device__ __forceinline__ void fx_row_weights(CStage &st, int col, int lane, FxHead &h) {
+template <int R>
+__device__ __forceinline__ void fx_row_weights(CStage &st, int col, int lane, FxHead<R> &h) {
   if (!(st.flags & MK_F_ROW_NORM)) return;
   const int nq = st.num_q_heads * st.head_dim;
   const float *w = col < nq ? (const float *)st.q_norm_w + col : (const float *)st.k_norm_w + (col - nq);
 #pragma unroll
-  for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-    if (j * 64 < st.head_dim) h.w[j] = w[min(j * 64 + lane, st.head_dim - 1)];
+  for (int j = 0; j < R; j++)
+    if (R == 2 || j * 64 < st.head_dim) h.w[j] = w[min(j * 64 + lane, st.head_dim - 1)];
 }
 // This lane's part of the sum of squares over columns [c0, c1) of a row, lane `id` of `n`.
 template <typename E>
@@ -323,87 +342,100 @@ __device__ __forceinline__ float fx_row_squares(const E *row, int c0, int c1, in
   return ss;
 }
 #endif
-// Bias of a row's columns (hybrid kernels): requested beside the row, added when it is used.
-template <typename E>
-__device__ __forceinline__ void fx_bias_load(const FxRows<E> &rows, int col, int n, int rot, int lane, float (&b)[MK_FX_HEAD_REGS], float (&bp)[MK_FX_HEAD_REGS]) {
-#if MK_HAVE_HYB
-  const int half = rot >> 1;
-  const float *p = rows.bias;
-#pragma unroll
-  for (int j = 0; j < MK_FX_HEAD_REGS; j++) b[j] = bp[j] = 0.f;
-  if (!p) return;
-#pragma unroll
-  for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-    if (j * 64 < n) {
-      const int d = min(j * 64 + lane, n - 1);
-      b[j] = p[col + d];
-      if (j * 64 < rot) bp[j] = p[col + (d < rot ? (d < half ? d + half : d - half) : d)];
-    }
-#endif
-}
-template <typename E>
-__device__ __forceinline__ void fx_head_load(CStage &st, const FxRows<E> &rows, int tok, int col, int pos, int lane, FxHead &h) {
-  const int D = st.head_dim, rot = (st.flags & MK_F_ROPE) ? st.rot_dims : 0, half = rot >> 1;
-  const float *ct = (const float *)st.cos_tab + (size_t)pos * st.ld_cos, *sn = (const float *)st.sin_tab + (size_t)pos * st.ld_cos;
+// Columns [col, col + n) of row `tok`, by one wavefront.
+struct FxSpan {
+  int tok, col, n;
+};
+template <typename E, int R>
+__device__ __forceinline__ void fx_span_load2(const FxRows<E> &rows, const FxSpan &s0, const FxSpan &s1, int lane, FxHead<R> &h0, FxHead<R> &h1) {
   rows.with_slices([&](auto ns) {
     constexpr int NS = decltype(ns)::value;
 #pragma unroll
-    for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-      if (j * 64 < D) {
-        const int d = min(j * 64 + lane, D - 1);
-        h.x[j] = rows.template get<NS>(tok, col + d);
-        if (j * 64 < rot) {
-          const bool in = d < rot, lo = d < half;
-          h.xp[j] = rows.template get<NS>(tok, col + (in ? (lo ? d + half : d - half) : d));
-          const int ci = in ? (lo ? d : d - half) : 0;
-          h.cs[j] = ct[ci];
-          h.sn[j] = sn[ci];
+    for (int j = 0; j < R; j += 2)
+      if (R == 2 || j * 64 < max(s0.n, s1.n)) {
+        float q[2][2][NS ? NS : 1];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const int d = (j + i) * 64 + lane;
+          rows.template request<NS>(s0.tok, s0.col + min(d, s0.n - 1), q[0][i]);
+          rows.template request<NS>(s1.tok, s1.col + min(d, s1.n - 1), q[1][i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          h0.x[j + i] = rows.template value<NS>(q[0][i]);
+          h1.x[j + i] = rows.template value<NS>(q[1][i]);
         }
       }
   });
+}
+// What is requested beside a row: its bias (hybrid kernels; added when it is used), and a head's rotation at position `pos`.
+template <typename E, int R>
+__device__ __forceinline__ void fx_head_tables(CStage &st, const FxRows<E> &rows, const FxSpan &s, bool rotated, int pos, int lane, FxHead<R> &h) {
 #if MK_HAVE_HYB
-  fx_bias_load(rows, col, D, rot, lane, h.b, h.bp);
+#pragma unroll
+  for (int j = 0; j < R; j++) h.b[j] = 0.f;
+  if (rows.bias) {
+#pragma unroll
+    for (int j = 0; j < R; j++)
+      if (R == 2 || j * 64 < s.n) h.b[j] = rows.bias[s.col + min(j * 64 + lane, s.n - 1)];
+  }
+#endif
+  const int rot = rotated && (st.flags & MK_F_ROPE) ? st.rot_dims : 0, half = rot >> 1;
+  const float *ct = (const float *)st.cos_tab + (size_t)pos * st.ld_cos, *sn = (const float *)st.sin_tab + (size_t)pos * st.ld_cos;
+#pragma unroll
+  for (int j = 0; j < R; j++)
+    if (j * 64 < rot) {
+      const int d = j * 64 + lane, ci = d < rot ? (d < half ? d : d - half) : 0;
+      h.cs[j] = ct[ci];
+      h.sn[j] = sn[ci];
+    }
+}
+// element j of a value row
+template <int R>
+__device__ __forceinline__ float fx_value(const FxHead<R> &h, int j) {
+#if MK_HAVE_HYB
+  return h.x[j] + h.b[j];
+#else
+  return h.x[j];
 #endif
 }
-// ... and a value row, which is copied as it is: columns [0, n) of it, lane l holds every 64th
-template <typename E>
-__device__ __forceinline__ void fx_value_load(const FxRows<E> &rows, int tok, int col, int n, int lane, float (&v)[MK_FX_HEAD_REGS]) {
-  rows.with_slices([&](auto ns) {
-#pragma unroll
-    for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-      if (j * 64 < n) v[j] = rows.template get<decltype(ns)::value>(tok, col + min(j * 64 + lane, n - 1));
-  });
-}
-template <typename Put>
-__device__ __forceinline__ void fx_head_finish(CStage &st, int lane, FxHead &h, Put put) {
+// `xs`: MK_FX_MAX_HEAD_DIM floats of LDS of this wavefront
+template <int R, typename Put>
+__device__ __forceinline__ void fx_head_finish(CStage &st, int lane, FxHead<R> &h, float *xs, Put put) {
   const int D = st.head_dim, rot = (st.flags & MK_F_ROPE) ? st.rot_dims : 0, half = rot >> 1;
   float ss = 0.f;
-#pragma unroll
-  for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-    if (j * 64 < D) {
-      const int d = j * 64 + lane;
 #if MK_HAVE_HYB
-      h.x[j] += h.b[j];
-      if (j * 64 < rot) h.xp[j] += h.bp[j];
+#pragma unroll
+  for (int j = 0; j < R; j++) h.x[j] += h.b[j];
 #endif
-      if (j * 64 < rot && d < rot) h.x[j] = d < half ? h.x[j] * h.cs[j] - h.xp[j] * h.sn[j] : h.x[j] * h.cs[j] + h.xp[j] * h.sn[j];
+#pragma unroll
+  for (int j = 0; j < R; j++)
+    if (j * 64 < rot) xs[j * 64 + lane] = h.x[j];
+#pragma unroll
+  for (int j = 0; j < R; j++)
+    if (R == 2 || j * 64 < D) {
+      const int d = j * 64 + lane;
+      if (j * 64 < rot) {
+        const float xp = xs[d < rot ? (d < half ? d + half : d - half) : 0];
+        if (d < rot) h.x[j] = d < half ? h.x[j] * h.cs[j] - xp * h.sn[j] : h.x[j] * h.cs[j] + xp * h.sn[j];
+      }
       ss += d < D ? h.x[j] * h.x[j] : 0.f;
     }
   if (st.flags & MK_F_QK_NORM) {
     const float r = 1.f / sqrtf(wave_sum(ss) / (float)D + st.eps);
 #pragma unroll
-    for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-      if (j * 64 < D) h.x[j] *= r;
+    for (int j = 0; j < R; j++)
+      if (R == 2 || j * 64 < D) h.x[j] *= r;
   }
 #if MK_HAVE_DUAL
   if (st.flags & MK_F_ROW_NORM) {
 #pragma unroll
-    for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-      if (j * 64 < D) h.x[j] = (h.x[j] * h.r) * h.w[j];
+    for (int j = 0; j < R; j++)
+      if (R == 2 || j * 64 < D) h.x[j] = (h.x[j] * h.r) * h.w[j];
   }
 #endif
 #pragma unroll
-  for (int j = 0; j < MK_FX_HEAD_REGS; j++)
+  for (int j = 0; j < R; j++)
     if (j * 64 + lane < D) put(j * 64 + lane, h.x[j]);
 }
 
@@ -436,7 +468,7 @@ __device__ __forceinline__ int fx_value_col(CStage &st) {
 // row.  Queries go to the workspace, keys and values to their pages.  (When every request brings one token the attention
 // stage does this itself and the stage is skipped.)
 template <typename E>
-__device__ __forceinline__ void stage_fx_prep(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
+__device__ __forceinline__ void stage_fx_prep(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
   barrier_wait(c);
   constexpr int KW = FxType<E>::KW;
   const FxRows<E> rows = fx_rows<E>(st, c);
@@ -446,54 +478,51 @@ __device__ __forceinline__ void stage_fx_prep(CStage &st, Ctx &c, const MkRuntim
   const int per = H + 2 * nkv, total = M * per;
   E *kc = (E *)st.k_cache, *vc = (E *)st.v_cache;
   const int stride = c.G * MK_WAVES;
-  auto load = [&](int i, FxHead &h, int &page) {
-    const int t = i / per, s = i - t * per;
-    const int pos = __builtin_amdgcn_readfirstlane(c.sh_tok[t]);
-    page = s < H ? 0 : rt.kv_indices[__builtin_amdgcn_readfirstlane(c.sh_tok[3 * MK_MAX_TOKENS + t]) + pos / ps];
-    if (s < H + nkv) {
-      fx_head_load<E>(st, rows, t, s * D, pos, lane, h);
+  float *xs = (float *)smem + wave * MK_FX_MAX_HEAD_DIM;
+  fx_head_regs(D, DV, [&](auto regs) {
+    constexpr int R = decltype(regs)::value;
+    auto span = [&](int i, FxHead<R> &h, int &page) -> FxSpan {
+      const int t = i / per, s = i - t * per;
+      const int pos = __builtin_amdgcn_readfirstlane(c.sh_tok[t]);
+      page = s < H ? 0 : rt.kv_indices[__builtin_amdgcn_readfirstlane(c.sh_tok[3 * MK_MAX_TOKENS + t]) + pos / ps];
+      const bool head = s < H + nkv;
+      const FxSpan sp = {t, head ? s * D : fx_value_col(st) + (s - H - nkv) * DV, head ? D : DV};
+      fx_head_tables(st, rows, sp, head, pos, lane, h);
 #if MK_HAVE_DUAL
-      if (st.flags & MK_F_ROW_NORM) {
+      if (head && (st.flags & MK_F_ROW_NORM)) {
         const int c0 = s < H ? 0 : H * D, c1 = s < H ? H * D : (H + nkv) * D;
         fx_row_weights(st, s * D, lane, h);
         h.r = 1.f / sqrtf(wave_sum(fx_row_squares<E>((const E *)st.in + (size_t)t * st.ld_in, c0, c1, lane, 64)) / (float)(c1 - c0) + st.eps);
       }
 #endif
-    } else {
-      fx_value_load<E>(rows, t, fx_value_col(st) + (s - H - nkv) * DV, DV, lane, h.x);
-#if MK_HAVE_HYB
-      fx_bias_load(rows, fx_value_col(st) + (s - H - nkv) * DV, DV, 0, lane, h.b, h.bp);
-#endif
-    }
-  };
-  auto finish = [&](int i, FxHead &h, int page) {
-    const int t = i / per, s = i - t * per;
-    const int pp = __builtin_amdgcn_readfirstlane(c.sh_tok[t]) % ps;
-    if (s < H) {
-      E *q = (E *)st.q_ws + (size_t)t * st.ld_qws + (size_t)s * nkc * KW;
-      fx_head_finish(st, lane, h, [&](int d, float v) { fx_stc(q + d, fx_round<E>(v)); });
-      for (int d = D + lane; d < nkc * KW; d += 64) fx_stc(q + d, (E)0);
-    } else if (s < H + nkv) {
-      fx_head_finish(st, lane, h, [&](int d, float v) { fx_stc(kc + fx_k_at<E>(page, pp, ps, nkv, s - H, nkc, d), fx_round<E>(v)); });
-    } else {
-      const int g = s - H - nkv;
-#if MK_HAVE_HYB
+      return sp;
+    };
+    auto finish = [&](int i, FxHead<R> &h, int page) {
+      const int t = i / per, s = i - t * per;
+      const int pp = __builtin_amdgcn_readfirstlane(c.sh_tok[t]) % ps;
+      if (s < H) {
+        E *q = (E *)st.q_ws + (size_t)t * st.ld_qws + (size_t)s * nkc * KW;
+        fx_head_finish(st, lane, h, xs, [&](int d, float v) { fx_stc(q + d, fx_round<E>(v)); });
+        for (int d = D + lane; d < nkc * KW; d += 64) fx_stc(q + d, (E)0);
+      } else if (s < H + nkv) {
+        fx_head_finish(st, lane, h, xs, [&](int d, float v) { fx_stc(kc + fx_k_at<E>(page, pp, ps, nkv, s - H, nkc, d), fx_round<E>(v)); });
+      } else {
+        const int g = s - H - nkv;
 #pragma unroll
-      for (int j = 0; j < MK_FX_HEAD_REGS; j++) h.x[j] += h.b[j];
-#endif
-#pragma unroll
-      for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-        if (j * 64 + lane < DV) fx_stc(vc + fx_v_at<E>(page, pp, ps, nkv, g, nvb, j * 64 + lane), fx_round<E>(h.x[j]));
+        for (int j = 0; j < R; j++)
+          if (j * 64 + lane < DV) fx_stc(vc + fx_v_at<E>(page, pp, ps, nkv, g, nvb, j * 64 + lane), fx_round<E>(fx_value(h, j)));
+      }
+    };
+    for (int i = c.vid * MK_WAVES + wave; i < total; i += 2 * stride) {
+      FxHead<R> h0, h1;
+      int p0, p1;
+      const int i1 = i + stride < total ? i + stride : i;
+      const FxSpan s0 = span(i, h0, p0), s1 = span(i1, h1, p1);
+      fx_span_load2(rows, s0, s1, lane, h0, h1);
+      finish(i, h0, p0);
+      if (i1 != i) finish(i1, h1, p1);
     }
-  };
-  for (int i = c.vid * MK_WAVES + wave; i < total; i += 2 * stride) {
-    FxHead h0, h1;
-    int p0, p1 = 0;
-    load(i, h0, p0);
-    if (i + stride < total) load(i + stride, h1, p1);
-    finish(i, h0, p0);
-    if (i + stride < total) finish(i + stride, h1, p1);
-  }
+  });
   c.wrote_through = true;
 }
 
@@ -544,9 +573,8 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
   E *vn = kn + nkc * KW;                                       // new value, padded with zeros to nvb * 16
   float *part = (float *)(smem + (nkg * KC * 1024 + (nkc * KW + nvb * 16) * (int)sizeof(E) + 15) / 16 * 16);  // [4][16][PSTR]
   float *ml = part + MK_WAVES * 16 * PSTR;                     // [4][16] maxima, [4][16] sums
-  float *fin = ml + 128;                                       // [4][16] weights, [16] maxima, [16] sums
-  float *chk = fin + 96;                                       // [chunks][16] maxima, [chunks][16] sums -> weights
-  int *sflag = (int *)(chk + 2 * MK_ATTN_MAX_CHUNKS * 16);
+  float *fin = ml + 128;                                       // [4][16] weights
+  int *sflag = (int *)(fin + 96);
   int *spg = sflag + 4;                                        // page-table entries of the chunk
   // rows of the requests, in row tiles of 16
   int my_n, my_tiles;
@@ -683,44 +711,44 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
       }
       for (int i = D + tid; i < nkc * KW; i += MK_THREADS) kn[i] = (E)0;
       for (int i = DV + tid; i < nvb * 16; i += MK_THREADS) vn[i] = (E)0;
-      // rows 0 .. nrows - 1 are queries, row nrows (the chunk that owns the new position) is the new key; the last
-      // wavefront, whose tile has been in flight longest, takes row 0 and with it the first of the second round
-      const int n_rows = a.nrows + (newest ? 1 : 0), w_ = MK_WAVES - 1 - wave;
-      const bool v_row = newest && w_ == 1;
-      const int v_col = fx_value_col(st) + a.g * DV;
-      float vv[MK_FX_HEAD_REGS];
-      if (v_row) fx_value_load<E>(rows, a.t0, v_col, DV, lane, vv);
-#if MK_HAVE_HYB
-      float vb[MK_FX_HEAD_REGS], vbp[MK_FX_HEAD_REGS];
-      if (v_row) fx_bias_load(rows, v_col, DV, 0, lane, vb, vbp);
-#endif
-      auto load_row = [&](int r, FxHead &h) {
-        fx_head_load<E>(st, rows, a.t0, (r < a.nrows ? a.g * qpk + a.r0 + r : st.num_q_heads + a.g) * D, a.p, lane, h);
+      // rows 0 .. nrows - 1 are queries, the next two (the chunk that owns the new position) the new key and value.  The first
+      // wavefront takes some only where that saves the others a round: its tile was requested last, and loads arrive in order.
+      const int n_rows = a.nrows + (newest ? 2 : 0);
+      const int RW = (n_rows + 2 * MK_WAVES - 3) / (2 * MK_WAVES - 2) > (n_rows + 2 * MK_WAVES - 1) / (2 * MK_WAVES) ? MK_WAVES : MK_WAVES - 1;
+      float *xs = part + 16 + wave * MK_FX_MAX_HEAD_DIM;
+      fx_head_regs(D, DV, [&](auto regs) {
+        constexpr int R = decltype(regs)::value;
+        auto span = [&](int r, FxHead<R> &h) -> FxSpan {
+          const bool head = r <= a.nrows;
+          const FxSpan sp = {a.t0, head ? (r < a.nrows ? a.g * qpk + a.r0 + r : st.num_q_heads + a.g) * D : fx_value_col(st) + a.g * DV, head ? D : DV};
+          fx_head_tables(st, rows, sp, head, a.p, lane, h);
 #if MK_HAVE_DUAL
-        fx_row_weights(st, (r < a.nrows ? a.g * qpk + a.r0 + r : st.num_q_heads + a.g) * D, lane, h);
-        h.r = r < a.nrows ? rq : rk;
+          if (head) fx_row_weights(st, sp.col, lane, h);
+          h.r = r < a.nrows ? rq : rk;
 #endif
-      };
-      auto put_row = [&](int r, FxHead &h) {
-        if (r < a.nrows) fx_head_finish(st, lane, h, [&](int d, float v) { q[((d / KW) * 64 + ((d % KW) / EPC) * 16 + r) * EPC + d % EPC] = fx_round<E>(v); });
-        else fx_head_finish(st, lane, h, [&](int d, float v) { kn[d] = fx_round<E>(v); });
-      };
-      for (int r = w_; r < n_rows; r += 2 * MK_WAVES) {
-        FxHead h0, h1;
-        load_row(r, h0);
-        if (r + MK_WAVES < n_rows) load_row(r + MK_WAVES, h1);
-        put_row(r, h0);
-        if (r + MK_WAVES < n_rows) put_row(r + MK_WAVES, h1);
-      }
-      if (v_row) {
+          return sp;
+        };
+        auto put_row = [&](int r, FxHead<R> &h) {
+          if (r < a.nrows) {
+            fx_head_finish(st, lane, h, xs, [&](int d, float v) { q[((d / KW) * 64 + ((d % KW) / EPC) * 16 + r) * EPC + d % EPC] = fx_round<E>(v); });
+          } else if (r == a.nrows) {
+            fx_head_finish(st, lane, h, xs, [&](int d, float v) { kn[d] = fx_round<E>(v); });
+          } else {
 #pragma unroll
-        for (int j = 0; j < MK_FX_HEAD_REGS; j++)
-#if MK_HAVE_HYB
-          if (j * 64 + lane < DV) vn[j * 64 + lane] = fx_round<E>(vv[j] + vb[j]);
-#else
-          if (j * 64 + lane < DV) vn[j * 64 + lane] = fx_round<E>(vv[j]);
-#endif
-      }
+            for (int j = 0; j < R; j++)
+              if (j * 64 + lane < DV) vn[j * 64 + lane] = fx_round<E>(fx_value(h, j));
+          }
+        };
+        if (wave != 0 || RW == MK_WAVES)
+          for (int r = MK_WAVES - 1 - wave; r < n_rows; r += 2 * RW) {
+            FxHead<R> h0, h1;
+            const int r1 = r + RW < n_rows ? r + RW : r;
+            const FxSpan s0 = span(r, h0), s1 = span(r1, h1);
+            fx_span_load2(rows, s0, s1, lane, h0, h1);
+            put_row(r, h0);
+            if (r1 != r) put_row(r1, h1);
+          }
+      });
     } else {
       for (int i = tid; i < nkg * KC * 64; i += MK_THREADS) {
         const int s = i >> 6, r = i & 15, R = a.r0 + r;
@@ -956,36 +984,51 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
     }
     __syncthreads();
     if (!*sflag) continue;
+    // Every thread weighs the chunks of its query row itself: maxima, sums and partial results of up to sixteen chunks are one round trip
+    // (weights by way of LDS had made it two and three barriers).
     const float *pb = (const float *)rt.attn_part + (size_t)a.item * cmax * 16 * PST;
-    for (int i = tid; i < a.C * 16; i += MK_THREADS) {
-      chk[i] = ldc_f32(pb + (size_t)i * PST + VB * 16);
-      chk[MK_ATTN_MAX_CHUNKS * 16 + i] = ldc_f32(pb + (size_t)i * PST + VB * 16 + 1);
-    }
-    __syncthreads();
-    if (tid < 16) {
-      float M_ = MK_FX_NEG, L_ = 0.f;
-      for (int q = 0; q < a.C; q++) M_ = fmaxf(M_, chk[q * 16 + tid]);
-      for (int q = 0; q < a.C; q++) {
-        const float e = exp2f(chk[q * 16 + tid] - M_);
-        L_ += chk[MK_ATTN_MAX_CHUNKS * 16 + q * 16 + tid] * e;
-        chk[q * 16 + tid] = e;
-      }
-      fin[tid] = 1.f / (L_ + exp2f(sink_of(tid) - M_));
-    }
-    __syncthreads();
+    constexpr int CB = 16;
+    static_assert(MK_ATTN_MAX_CHUNKS <= 2 * CB, "at most two blocks of chunks");
     for (int i = tid; i < 16 * VB * 4; i += MK_THREADS) {
       const int r = i / (VB * 4), d = (i - r * (VB * 4)) * 4;
       if (r >= a.nrows || dv0 + d >= DV) continue;
+      float cm[CB], cl[CB];
+      f32x4 x[CB];
+      auto request = [&](int q0, bool data) {
+#pragma unroll
+        for (int q = 0; q < CB; q++)
+          if (q0 + q < a.C) {
+            const float *p = pb + ((size_t)(q0 + q) * 16 + r) * PST;
+            const unsigned long long u = ldc_u64(p + VB * 16);
+            cm[q] = __uint_as_float((uint32_t)u);
+            cl[q] = __uint_as_float((uint32_t)(u >> 32));
+            if (data) x[q] = fx_ldc_quad(p + d);
+          }
+      };
+      float M_ = MK_FX_NEG, L_ = 0.f;
       f32x4 o = {0.f, 0.f, 0.f, 0.f};
-      for (int q0 = 0; q0 < a.C; q0 += 8) {
-        f32x4 x[8];
+      auto largest = [&](int q0) {
 #pragma unroll
-        for (int q = 0; q < 8; q++) x[q] = fx_ldc_quad(pb + ((size_t)min(q0 + q, a.C - 1) * 16 + r) * PST + d);
-#pragma unroll
-        for (int q = 0; q < 8; q++)
-          if (q0 + q < a.C) o += x[q] * chk[(q0 + q) * 16 + r];
+        for (int q = 0; q < CB; q++)
+          if (q0 + q < a.C) M_ = fmaxf(M_, cm[q]);
+      };
+      if (a.C > CB) {
+        request(CB, false);
+        largest(CB);
       }
-      emit(r, d, o * fin[r]);
+      request(0, true);
+      largest(0);
+      for (int q0 = 0; q0 < a.C; q0 += CB) {
+        if (q0) request(q0, true);
+#pragma unroll
+        for (int q = 0; q < CB; q++)
+          if (q0 + q < a.C) {
+            const float e = exp2f(cm[q] - M_);
+            L_ += cl[q] * e;
+            o += x[q] * e;
+          }
+      }
+      emit(r, d, o * (1.f / (L_ + exp2f(sink_of(r) - M_))));
     }
   }
 }

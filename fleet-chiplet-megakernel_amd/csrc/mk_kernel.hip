@@ -4302,7 +4302,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
 #if MK_HAVE_FLEX
         case MK_OP_FX_EMBED: if constexpr (FX) stage_fx_embed<E>(st, c, rt, M); break;
         case MK_OP_FX_ADDNORM: if constexpr (FX) stage_fx_addnorm<E>(st, c, M, smem); break;
-        case MK_OP_FX_PREP: if constexpr (FX) stage_fx_prep<E>(st, c, rt, M); break;
+        case MK_OP_FX_PREP: if constexpr (FX) stage_fx_prep<E>(st, c, rt, M, smem); break;
         case MK_OP_FX_ATTN: if constexpr (FX) stage_fx_attn<E>(st, c, rt, M, MAXM == 1 || single, smem); break;
         case MK_OP_LINEAR_F32:
           if constexpr (F32) stage_fx_linear_f32(st, c, M, smem);

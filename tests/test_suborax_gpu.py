@@ -219,6 +219,24 @@ def test_attention_alone(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,D,DV,rot,n", [(7, 64, 64, 64, 2300), (8, 128, 128, 96, 1500), (13, 129, 40, 126, 700), (2, 512, 512, 510, 130)])
+def test_rows_and_chunks_of_one_request(H, D, DV, rot, n, dtype):
+    """One kv head: more than 16 chunks to combine; query rows that the first wavefront has to share or not, heads that need two, three or
+    eight registers a row, rotations that end inside one."""
+    from suborax_helpers import AttentionRig
+    rig = AttentionRig(H, 1, D, DV, rot, 1.0 / D ** 0.5, 12.0, True, torch.full((H,), 1.0), dtype=dtype, pages=n // 32 + 1)
+    rows, pages = _rows(rig, n, 21), list(range(n // 32, -1, -1))
+    cut = n - 6
+    for p0 in range(0, cut, 64):
+        last = rig.run([(0, p0, rows[p0:min(p0 + 64, cut)], pages)])[0]
+    want = rig.reference(rows)
+    torch.testing.assert_close(last, want[cut - len(last):cut], **_tol(dtype))
+    for p in range(cut, n):
+        torch.testing.assert_close(rig.run([(0, p, rows[p:p + 1], pages)])[0][0], want[p], msg=lambda m: f"query {p}: {m}", **_tol(dtype))
+    rig.close()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_far_keys_and_page_borders(dtype):
     """One key per query that stands out: the query at p is a multiple of the key at j (no rotation), so nearly all weight
     sits on j.  j runs over tile, page and chunk borders, the first positions and the newest ones; single tokens and portions."""
