@@ -3141,10 +3141,11 @@ int mk_compile(mk_graph *g) {
   for (auto &s : g->stages)
     if (s.op == MK_OP_ATTN) {
       // a work unit is (token, kv head, chunk) with chunks = clamp(G / (tokens * kv heads), 1, MK_ATTN_MAX_CHUNKS): never
-      // more than max(G, tokens * kv heads) units, each holding q/kv head partials
+      // more than max(G, tokens * kv heads) units, each holding q/kv head partials; units of several tokens hold 16 rows, and are
+      // split into chunks only where that makes at most G of them
       const size_t units = (size_t)std::max(g->G, rt.max_tokens * s.num_kv_heads);
       const int qpk = s.num_q_heads / s.num_kv_heads;
-      if ((rc = dev_alloc(g, &p, units * qpk * MK_ATTN_PSTRIDE * sizeof(float), false))) return rc;
+      if ((rc = dev_alloc(g, &p, std::max(units * qpk, (size_t)g->G * 16) * MK_ATTN_PSTRIDE * sizeof(float), false))) return rc;
       s.aux0 = p;
       s.aux1 = rt.attn_cnt + g->attn_cnt_n / 2;
     }

@@ -3395,50 +3395,132 @@ __device__ __forceinline__ void stage_moe_combine(CStage &st, Ctx &c, int M) {
   c.wrote_through = true;
 }
 
-// Per-head RMSNorm + rotate-half RoPE of one 128-wide head row by one wavefront (lane l owns elements
-// l and l+64, the two halves of a rotation pair).  The normalised value is rounded to bf16 before the
-// rotation, as in the reference (tasks/mi300/kv_cache_update_mi300.cuh:129-182).  Split in a load half and a
-// compute half so that a wavefront can have the loads of several rows in flight.
-__device__ __forceinline__ void head_row_load(const uint16_t *src, int lane, float &x0, float &x1) {
-  x0 = bf2f(ldc_u16(src + lane));
-  x1 = bf2f(ldc_u16(src + lane + 64));
-}
-// The same two elements when the producing linear left its K-slice partials unsummed: sum of the NS slices in slice
-// order, rounded to bf16 (what that linear would have stored).  `p` points at slice 0's element l of the row.
-template <int NS>
-__device__ __forceinline__ void head_row_load_slices(const float *p, size_t slice_stride, int lane, float &x0, float &x1) {
-  float a[NS], b[NS];
+// One 128-wide head row by one wavefront (lane l owns elements l and l + 64, the two halves of a rotation pair): query and key rows
+// get the per-head RMSNorm and the rotate-half RoPE, a value row is copied as it is.  The normalised value is rounded to bf16 before
+// the rotation, as in the reference (tasks/mi300/kv_cache_update_mi300.cuh:129-182).
+struct AttnRow {
+  int tok, off, pos;  // row and first column in the q/k/v tensor, position
+  int kind;           // 0 query, 1 key, 2 value
+  uint16_t *dst;      // LDS
+};
+// Where these rows come from: stored by the producing linear, or -- when it left its K-slice partials to this stage -- summed here, in
+// slice order, rounded to bf16 (what that linear would have stored).
+struct AttnSource {
+  uint16_t *in;
+  int ld, S;
+  const float *part;
+  size_t n, slice;
+  uint16_t qw[2], kw[2];  // this lane's norm weights
+};
+// Rows [0, n) by the workgroup, RF per wavefront in flight.  Bound by round trips: everything a row needs is requested before the first
+// value is waited for (the row, then its norm weights, then its rotation had made it three, and a branch around each row as many more).
+// own(tok): an unsummed row of this token is also stored where the linear would have.
+template <int RF, typename Row, typename Own>
+__device__ __forceinline__ void attn_rows(CStage &st, const AttnSource &src, int n, int lane, int wave, Row row, Own own) {
+  for (int i0 = MK_WAVES - 1 - wave; i0 < n; i0 += RF * MK_WAVES) {
+    AttnRow a[RF];
+    uint16_t cs[RF], sn[RF];
+    float x[RF][2];
 #pragma unroll
-  for (int q = 0; q < NS; q++) {
-    a[q] = ldc_f32(p + q * slice_stride + lane);
-    b[q] = ldc_f32(p + q * slice_stride + lane + 64);
-  }
-  float s0 = 0.f, s1 = 0.f;
+    for (int r = 0; r < RF; r++) a[r] = row(min(i0 + r * MK_WAVES, n - 1));
+    if (st.flags & MK_F_ROPE) {
 #pragma unroll
-  for (int q = 0; q < NS; q++) {
-    s0 += a[q];
-    s1 += b[q];
+      for (int r = 0; r < RF; r++) {
+        cs[r] = ((const uint16_t *)st.cos_tab + (size_t)a[r].pos * st.ld_cos)[lane];
+        sn[r] = ((const uint16_t *)st.sin_tab + (size_t)a[r].pos * st.ld_cos)[lane];
+      }
+    }
+    auto sum = [&](auto ns) {
+      constexpr int NS = decltype(ns)::value;
+      float q[RF][2][NS];
+#pragma unroll
+      for (int r = 0; r < RF; r++) {
+        const float *pp = src.part + (size_t)a[r].tok * src.n + a[r].off + lane;
+#pragma unroll
+        for (int b = 0; b < NS; b++) {
+          q[r][0][b] = ldc_f32(pp + b * src.slice);
+          q[r][1][b] = ldc_f32(pp + b * src.slice + 64);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RF; r++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          float v = 0.f;
+#pragma unroll
+          for (int b = 0; b < NS; b++) v += q[r][e][b];
+          x[r][e] = bfround(v);
+        }
+    };
+    if (src.S == 0) {
+      uint16_t q[RF][2];
+#pragma unroll
+      for (int r = 0; r < RF; r++) {
+        const uint16_t *pp = src.in + (size_t)a[r].tok * src.ld + a[r].off + lane;
+        q[r][0] = ldc_u16(pp);
+        q[r][1] = ldc_u16(pp + 64);
+      }
+#pragma unroll
+      for (int r = 0; r < RF; r++) {
+        x[r][0] = bf2f(q[r][0]);
+        x[r][1] = bf2f(q[r][1]);
+      }
+    } else if (src.S == 2) {
+      sum(std::integral_constant<int, 2>{});
+    } else if (src.S == 4) {
+      sum(std::integral_constant<int, 4>{});
+    } else {
+      sum(std::integral_constant<int, 8>{});
+    }
+#pragma unroll
+    for (int r = 0; r < RF; r++) {
+      if (i0 + r * MK_WAVES >= n) break;
+      float x0 = x[r][0], x1 = x[r][1];
+      if (src.S && own(a[r].tok)) {
+        uint16_t *d = src.in + (size_t)a[r].tok * src.ld + a[r].off;
+        d[lane] = (uint16_t)f2bf(x0);
+        d[lane + 64] = (uint16_t)f2bf(x1);
+      }
+      if (a[r].kind < 2) {
+        if (st.flags & MK_F_QK_NORM) {
+          const float ss = wave_sum(x0 * x0 + x1 * x1);
+          const float f = rsqrtf(ss * (1.f / 128.f) + st.eps);
+          x0 = bfround((x0 * f) * bf2f(a[r].kind ? src.kw[0] : src.qw[0]));
+          x1 = bfround((x1 * f) * bf2f(a[r].kind ? src.kw[1] : src.qw[1]));
+        }
+        if (st.flags & MK_F_ROPE) {
+          const float c_ = bf2f(cs[r]), s_ = bf2f(sn[r]);
+          const float y0 = x0 * c_ - x1 * s_;
+          const float y1 = x0 * s_ + x1 * c_;
+          x0 = y0;
+          x1 = y1;
+        }
+      }
+      a[r].dst[lane] = (uint16_t)f2bf(x0);
+      a[r].dst[lane + 64] = (uint16_t)f2bf(x1);
+    }
   }
-  x0 = bfround(s0);
-  x1 = bfround(s1);
 }
-__device__ __forceinline__ void head_row_finish(float x0, float x1, uint16_t *dst, const uint16_t *nw, const uint16_t *cos_row, const uint16_t *sin_row,
-                                                int flags, float eps, int lane) {
-  if (flags & MK_F_QK_NORM) {
-    const float ss = wave_sum(x0 * x0 + x1 * x1);
-    const float r = rsqrtf(ss * (1.f / 128.f) + eps);
-    x0 = bfround((x0 * r) * bf2f(nw[lane]));
-    x1 = bfround((x1 * r) * bf2f(nw[lane + 64]));
+// (before the barrier: the norm weights; after it: where the rows are)
+__device__ __forceinline__ AttnSource attn_source(CStage &st, int lane) {
+  AttnSource s;
+  if (st.flags & MK_F_QK_NORM) {
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      s.qw[e] = ((const uint16_t *)st.q_norm_w)[lane + 64 * e];
+      s.kw[e] = ((const uint16_t *)st.k_norm_w)[lane + 64 * e];
+    }
   }
-  if (flags & MK_F_ROPE) {
-    const float cs = bf2f(cos_row[lane]), sn = bf2f(sin_row[lane]);
-    const float y0 = x0 * cs - x1 * sn;
-    const float y1 = x0 * sn + x1 * cs;
-    x0 = y0;
-    x1 = y1;
-  }
-  dst[lane] = (uint16_t)f2bf(x0);
-  dst[lane + 64] = (uint16_t)f2bf(x1);
+  return s;
+}
+__device__ __forceinline__ void attn_source_ready(CStage &st, Ctx &c, AttnSource &s) {
+  s.in = (uint16_t *)st.in;
+  s.ld = st.ld_in;
+  s.S = c.defer_S;
+  s.part = c.defer_part;
+  s.n = (size_t)c.defer_n;
+  s.slice = (size_t)c.defer_rows * s.n;
+  c.defer_S = 0;
 }
 
 #ifndef MK_TUNE_ATTN_TILES
@@ -3467,7 +3549,7 @@ struct AttnUnit {
 // Reference tasks: kv_cache_update_impl (tasks/mi300/kv_cache_update_mi300.cuh:41-327),
 // paged_attention_minimal_decode (tasks/mi300/paged_attention_decode_minimal_mi300.cuh:100-371),
 // gang_attention_split_kv_kernel (tasks/mi300/gang_attention_mi300.cuh:49-153).
-template <int QPK, bool MF>
+template <int QPK>
 __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
   constexpr int D = 128;
   constexpr int NPRE = MK_TUNE_NPRE;          // positions per lane group requested ahead
@@ -3482,24 +3564,10 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
   int *sflag = (int *)(smem + 2048);
   uint16_t *knew = (uint16_t *)(smem + 4096);                             // [MK_MAX_NEW_PER_REQ][128]
   uint16_t *vnew = knew + MK_MAX_NEW_PER_REQ * D;                         // [MK_MAX_NEW_PER_REQ][128]
-  // MF (iterations of many tokens): the cached positions go through the matrix cores, one wavefront per 16-position
-  // tile, and leave four more partial results (one per wavefront) next to the sixteen lane groups'; each wavefront has
-  // two private 4 KB buffers for the V tiles it transposes through LDS.  The page list of the running unit aliases the
-  // partial-result area (used before the partials are written).
-  constexpr int NG = MF ? 20 : 16;
-  // A K or V tile in LDS: 16 rows of 256 bytes as four groups of four rows, one direct-to-LDS request per group (each
-  // lane 16 bytes: four whole rows, 1 KB contiguous in LDS), the groups GS bytes apart (+64: the transposed V reads of
-  // the four groups then fall into different banks).  With four q heads per kv head there is room to stage K this way
-  // as well (whole rows per request instead of 64 bytes of each of 16 rows); otherwise K goes to registers.
-  constexpr int GS = 1088, TS = 4 * GS;
-  constexpr bool KLDS = QPK == 4;
-  constexpr int SLOT = KLDS ? 2 * TS : TS;  // bytes per tile in flight
-  constexpr int PART_OFF = 4096 + 2 * MK_MAX_NEW_PER_REQ * D * 2, VBUF_OFF = PART_OFF + NG * QPK * 132 * 4;
+  constexpr int NG = 16;
+  constexpr int PART_OFF = 4096 + 2 * MK_MAX_NEW_PER_REQ * D * 2;
   float *part = (float *)(smem + PART_OFF);  // [NG][QPK][132]
-  int *spg = (int *)(smem + PART_OFF);
-  constexpr int RB = QPK == 4 ? MK_TUNE_ATTN_TILES : 2;  // (MF) tiles a wavefront keeps in flight, as LDS allows
-  static_assert(VBUF_OFF + (MF ? MK_WAVES * RB * SLOT : 0) <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
-  static_assert(MK_ATTN_MAX_REQ_PAGES * 4 <= NG * QPK * 132 * 4, "page list exceeds the area it aliases");
+  static_assert(PART_OFF + NG * QPK * 132 * 4 <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
   const int n_items = M * nkv;
   int cmax = c.G / n_items;
   cmax = cmax < 1 ? 1 : (cmax > MK_ATTN_MAX_CHUNKS ? MK_ATTN_MAX_CHUNKS : cmax);
@@ -3563,24 +3631,11 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
   };
   // the polling wavefront keeps its memory queue empty until the barrier is through (its loads would delay the poll
   // results behind them); its rows are requested right after and land while the q rows are being fetched
-  if (!MF && have0 && wave != 0) prefetch0();
+  if (have0 && wave != 0) prefetch0();
+  AttnSource src = attn_source(st, lane);
   barrier_wait(c);
-  if (!MF && have0 && wave == 0) prefetch0();
-  // the q/k/v rows: stored by the producing linear, or -- when it left its K-slice partials to this stage -- summed here
-  const int dS = c.defer_S;
-  c.defer_S = 0;
-  const float *dpart = c.defer_part;
-  const size_t dn = (size_t)c.defer_n, dslice = (size_t)c.defer_rows * dn;
-  auto fetch = [&](int tok, int off, float &y0, float &y1) {
-    if (dS == 0) {
-      head_row_load((const uint16_t *)st.in + (size_t)tok * st.ld_in + off, lane, y0, y1);
-    } else {
-      const float *pp = dpart + (size_t)tok * dn + off;
-      if (dS == 2) head_row_load_slices<2>(pp, dslice, lane, y0, y1);
-      else if (dS == 4) head_row_load_slices<4>(pp, dslice, lane, y0, y1);
-      else head_row_load_slices<8>(pp, dslice, lane, y0, y1);
-    }
-  };
+  if (have0 && wave == 0) prefetch0();
+  attn_source_ready(st, c, src);
 
   for (int uu = c.vid; uu < n_units; uu += c.G) {
     AttnUnit a;
@@ -3601,63 +3656,17 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
     }
     const int t = a.t, h = a.h, p = a.p, C = a.C;
     __syncthreads();  // LDS reuse across units
-    // (MF) this unit's page-table entries: requested here, stored to LDS after the row requests below are out -- an LDS
-    // store waits for its load, and loads return in order
-    const int pg_lo = a.start / ps;
-    const int npg = (MF && a.cend > a.start) ? (a.cend - 1) / ps - pg_lo + 1 : 0;
-    const int pg_first = tid < npg ? a.pages[pg_lo + tid] : 0;
-    // ---- phase A: prepare q heads and the new K/V rows of this chunk, two rows per wavefront in flight
-    const int n_rows = QPK + a.n_new;
-    for (int row0 = wave; row0 < n_rows; row0 += 2 * MK_WAVES) {
-      float x0[2], x1[2], v0[2], v1[2];
-      int tok[2], off[2];
-#pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const int row = row0 + r * MK_WAVES;
-        if (row < n_rows) {
-          const bool isq = row < QPK;
-          tok[r] = isq ? t : a.t0 + (a.new_lo + (row - QPK) - a.p0);
-          off[r] = h * (QPK + 2) * D + (isq ? row : QPK) * D;
-          fetch(tok[r], off[r], x0[r], x1[r]);
-          if (!isq) fetch(tok[r], off[r] + D, v0[r], v1[r]);  // (a V row is copied as it is)
-        }
-      }
-      if (MF && row0 == wave) {
-        if (tid < npg) spg[tid] = pg_first;
-        for (int i = tid + MK_THREADS; i < npg; i += MK_THREADS) spg[i] = a.pages[pg_lo + i];
-      }
-#pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const int row = row0 + r * MK_WAVES;
-        if (row < n_rows) {
-          const bool isq = row < QPK;
-          const int pos = isq ? p : a.new_lo + (row - QPK);
-          if (!isq) {
-            vnew[(row - QPK) * D + lane] = (uint16_t)f2bf(v0[r]);
-            vnew[(row - QPK) * D + lane + 64] = (uint16_t)f2bf(v1[r]);
-          }
-          if (dS && a.cidx == C - 1 && tok[r] == t) {
-            // the producing linear left these rows unsummed: the chunk that owns the token's newest position also
-            // stores the token's own q/k/v rows where that linear would have
-            uint16_t *dst = (uint16_t *)st.in + (size_t)t * st.ld_in + off[r];
-            dst[lane] = (uint16_t)f2bf(x0[r]);
-            dst[lane + 64] = (uint16_t)f2bf(x1[r]);
-            if (!isq) {
-              dst[D + lane] = (uint16_t)f2bf(v0[r]);
-              dst[D + lane + 64] = (uint16_t)f2bf(v1[r]);
-            }
-          }
-          head_row_finish(x0[r], x1[r], isq ? qs + row * D : knew + (row - QPK) * D, (const uint16_t *)(isq ? st.q_norm_w : st.k_norm_w),
-                          (const uint16_t *)st.cos_tab + (size_t)pos * st.ld_cos, (const uint16_t *)st.sin_tab + (size_t)pos * st.ld_cos, st.flags, st.eps,
-                          lane);
-        }
-      }
-    }
+    // ---- phase A: prepare q heads and the new K/V rows of this chunk
+    attn_rows<2>(st, src, QPK + 2 * a.n_new, lane, wave,
+                 [&](int i) -> AttnRow {
+                   const int j = i - QPK, kind = j < 0 ? 0 : j < a.n_new ? 1 : 2, jj = kind == 2 ? j - a.n_new : j, base = h * (QPK + 2) * D;
+                   return kind ? AttnRow{a.t0 + (a.new_lo + jj - a.p0), base + (QPK + kind - 1) * D, a.new_lo + jj, kind, (kind == 1 ? knew : vnew) + jj * D}
+                               : AttnRow{t, base + i * D, p, 0, qs + i * D};
+                 },
+                 [&](int tok) { return a.cidx == C - 1 && tok == t; });
     __syncthreads();
-    // the chunk that owns the newest position appends this token's K/V and publishes q (MF: after the tile loop, whose
-    // request counting must not see other vector-memory traffic)
-    auto append = [&]() {
-      if (a.cidx != C - 1) return;
+    // the chunk that owns the newest position appends this token's K/V and publishes q
+    if (a.cidx == C - 1) {
       const int j = p - a.new_lo;
       const size_t rowi = (size_t)a.pages[p / ps] * ps + (p % ps);
       uint32_t *kd = (uint32_t *)st.k_cache + (rowi * nkv + h) * (D / 2);
@@ -3668,8 +3677,7 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
         uint32_t *qd = (uint32_t *)st.q_ws + ((size_t)t * st.ld_qws + (size_t)h * QPK * D) / 2;
         for (int i = tid; i < QPK * D / 2; i += MK_THREADS) qd[i] = ((const uint32_t *)qs)[i];
       }
-    };
-    if (!MF) append();
+    }
     MK_MARK(c, first ? 0 : 2);
     // ---- phase B: online softmax over the chunk
     u32x4 qv[QPK];
@@ -3741,153 +3749,6 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
         }
       }
     };
-    if constexpr (MF) {
-      // ---- cached positions on the matrix cores.  Tile = 16 positions, one wavefront per tile.  Scores: A = the K tile
-      // (lane (i, g): row of position i; step s contracts dims 32 s + 8 g ..; read from the K tile in LDS, or -- eight q
-      // heads per kv head -- requested straight into registers, 64 bytes of each of 16 rows per request), B = q (lane
-      // (j, g): head j, same dims; heads past QPK are zero) -> lane (j, g) holds the scores of head j at
-      // positions 4 g .. 4 g + 3.  Those four weights, as bf16 (value and rounding remainder: two operands), are already
-      // the A operand of a 16x16x16 step over positions; its B operand -- four consecutive positions of one dim --
-      // is read out of the V tile that direct-to-LDS loads put into this wavefront's buffer.  The running maximum is
-      // kept per head for the whole wavefront (the products of a step are summed across its lanes, so they must share
-      // their reference), the running sum per lane.
-      typedef short s16x4 __attribute__((ext_vector_type(4)));
-      const int lr = lane & 15, lg = lane >> 4;
-      char *vb0 = smem + VBUF_OFF + wave * (RB * SLOT);
-      bf16x8 qb[4];
-#pragma unroll
-      for (int s_ = 0; s_ < 4; s_++) {
-        const u32x4 z = {0u, 0u, 0u, 0u};
-        qb[s_] = __builtin_bit_cast(bf16x8, lr < QPK ? *(const u32x4 *)(qs + lr * D + s_ * 32 + lg * 8) : z);
-      }
-      f32x4 o[8];
-#pragma unroll
-      for (int dt = 0; dt < 8; dt++) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-      float mrun = -INFINITY, lsum = 0.f;
-      const int nt = a.cend > a.start ? (a.cend - a.start + 15) >> 4 : 0;
-      auto row_base = [&](int pos) -> size_t {  // first 16-byte operand of the (position, head) row
-        const int pc = min(pos, a.cend - 1), pg = pc / ps;
-        return (((size_t)spg[pg - pg_lo] * ps + (pc - pg * ps)) * nkv + h) * (D / 8);
-      };
-      auto load_tile = [&](int tt, bf16x8 (&kk)[4], char *vbuf) {
-        const int p0 = a.start + min(tt, nt - 1) * 16;
-        if (!KLDS) {  // K to registers: lane (row, g), request s reads bytes 64 s + 16 g of its row
-          const size_t base = row_base(p0 + lr) + lg;
-#pragma unroll
-          for (int s_ = 0; s_ < 4; s_++) kk[s_] = __builtin_nontemporal_load((const bf16x8 *)(kc + base + s_ * 4));
-        }
-        // to LDS: request s brings rows 4 s .. 4 s + 3 whole (lane (row in group, 16-byte piece))
-        // (streaming requests -- the cache-policy bit the nontemporal loads of the other paths carry: a cached K/V row is
-        // read once per iteration and need not displace the activations the linears share through the L2)
-        constexpr int KV_NT = 2;
-        size_t gb[4];
-#pragma unroll
-        for (int s_ = 0; s_ < 4; s_++) gb[s_] = row_base(p0 + 4 * s_ + lg) + lr;
-        if (KLDS) {
-#pragma unroll
-          for (int s_ = 0; s_ < 4; s_++)
-            __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(kc + gb[s_]),
-                                             (__attribute__((address_space(3))) void *)(__attribute__((address_space(3))) char *)(vbuf + TS + s_ * GS), 16, 0, KV_NT);
-        }
-#pragma unroll
-        for (int s_ = 0; s_ < 4; s_++)
-          __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(vc + gb[s_]),
-                                           (__attribute__((address_space(3))) void *)(__attribute__((address_space(3))) char *)(vbuf + s_ * GS), 16, 0, KV_NT);
-      };
-      const int vlane = lg * GS + lr * 2;
-      const int klane = (lr >> 2) * GS + (lr & 3) * 256 + lg * 16;
-      auto compute_tile = [&](int t_, const bf16x8 (&kk)[4], const char *vbuf) {
-        f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s_ = 0; s_ < 4; s_++) {
-          const bf16x8 ko = KLDS ? __builtin_bit_cast(bf16x8, *(const u32x4 *)(vbuf + TS + klane + s_ * 64)) : kk[s_];
-          s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko, qb[s_], s4, 0, 0, 0);
-        }
-        const int pbase = a.start + t_ * 16 + lg * 4;
-        float sc[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) sc[r] = pbase + r < a.cend ? s4[r] * st.sm_scale_log2 : -INFINITY;
-        float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-        mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, mx))));
-        mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, mx))));
-        const float mn = fmaxf(mrun, mx);
-        const float alpha = __builtin_amdgcn_exp2f(mrun - mn);
-        float pw[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) pw[r] = __builtin_amdgcn_exp2f(sc[r] - mn);
-        lsum = lsum * alpha + ((pw[0] + pw[1]) + (pw[2] + pw[3]));
-        mrun = mn;
-        if (__ballot(lr < QPK && alpha != 1.f)) {  // (uniform) some head's maximum moved: rescale what has been summed
-          float ar[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) ar[r] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lg * 4 + r) << 2, __builtin_bit_cast(int, alpha)));
-#pragma unroll
-          for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[dt][r] *= ar[r];
-        }
-        float ph[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) ph[r] = bfround(pw[r]);
-        const unsigned h01 = pack2(ph[0], ph[1]), h23 = pack2(ph[2], ph[3]);
-        const unsigned l01 = pack2(pw[0] - ph[0], pw[1] - ph[1]), l23 = pack2(pw[2] - ph[2], pw[3] - ph[3]);
-        const s16x4 a_hi = __builtin_bit_cast(s16x4, (unsigned long long)h01 | ((unsigned long long)h23 << 32));
-        const s16x4 a_lo = __builtin_bit_cast(s16x4, (unsigned long long)l01 | ((unsigned long long)l23 << 32));
-        const char *vb = vbuf + vlane;
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++) {
-          const char *q_ = vb + dt * 32;
-          const unsigned v0 = *(const uint16_t *)(q_), v1 = *(const uint16_t *)(q_ + 256), v2 = *(const uint16_t *)(q_ + 512), v3 = *(const uint16_t *)(q_ + 768);
-          const s16x4 bv = __builtin_bit_cast(s16x4, (unsigned long long)(v0 | (v1 << 16)) | ((unsigned long long)(v2 | (v3 << 16)) << 32));
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_hi, bv, o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_lo, bv, o[dt], 0, 0, 0);
-        }
-      };
-      // RB tiles in flight per wavefront: every request is issued unconditionally (a tile index past the end re-reads the
-      // last tile; it is never computed), and the wait before a tile counts the 8 (RB - 1) requests of the tiles after it
-      int t_ = wave;
-      if (t_ < nt) {
-        bf16x8 kr[RB][4];
-#pragma unroll
-        for (int b_ = 0; b_ < RB - 1; b_++) load_tile(t_ + b_ * MK_WAVES, kr[b_], vb0 + b_ * SLOT);
-        bool more = true;
-        while (more) {
-#pragma unroll
-          for (int b_ = 0; b_ < RB; b_++) {
-            // slot (b_ + RB - 1) % RB was computed in the previous round: refill it with the tile RB - 1 ahead
-            load_tile(t_ + (RB - 1) * MK_WAVES, kr[(b_ + RB - 1) % RB], vb0 + ((b_ + RB - 1) % RB) * SLOT);
-            if (RB == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-            else if (RB == 3) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-            if (more) {
-              compute_tile(t_, kr[b_], vb0 + b_ * SLOT);
-              t_ += MK_WAVES;
-              more = t_ < nt;
-            }
-          }
-        }
-      }
-      MK_MARK(c, first ? 1 : 3);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the direct-to-LDS requests of the tile that was not computed)
-      append();
-      __syncthreads();  // every wavefront is done with the page list: the partial results may overwrite it
-      float lt = lsum;
-      lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, lt)));
-      lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, lt)));
-      const int gm = 16 + wave;
-      if (lg == 0 && lr < QPK) {
-        part[(gm * QPK + lr) * 132 + 128] = mrun;
-        part[(gm * QPK + lr) * 132 + 129] = lt;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int head = lg * 4 + r;
-        if (head < QPK) {
-#pragma unroll
-          for (int dt = 0; dt < 8; dt++) part[(gm * QPK + head) * 132 + dt * 16 + lr] = o[dt][r];
-        }
-      }
-    } else {
     int pos = a.start + gg;
     if (first) {
       if (pos < a.cend) process_block(pk, pv, pos);
@@ -3917,7 +3778,6 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
         pos += 16 * NPRE;
         if (pos >= a.cend) break;
       }
-    }
     }
     for (int j = gg; j < a.n_new; j += 16) process(((const u32x4 *)(knew + j * D))[j16], ((const u32x4 *)(vnew + j * D))[j16]);
     // ---- phase C: merge the 16 groups through LDS
@@ -4039,6 +3899,351 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
   // L2 until a later barrier of this iteration writes it back (the sampling stages and the scheduler step always do);
   // nothing reads them before the next iteration.
   c.wrote_through = true;
+}
+
+
+// The same for iterations of many tokens, on the matrix cores.  Work unit = (up to 16 / QPK consecutive tokens of one request, kv head,
+// KV chunk): their query rows are the 16 columns of a tile product, so a prompt's tokens share what is read of the cache.  One wavefront
+// per tile of 16 positions; the new positions of the iteration are tiles as well, out of LDS.
+//
+// Bound by the cache's way through L2 for long prompts and by round trips for short contexts.  A unit per token had read the cache once
+// for every token of a prompt and prepared its new key rows as often.  64 tokens of one prompt, 32 q / 8 kv heads, as a stage: behind 1216
+// cached positions 85 -> 31 us, behind 2432 127 -> 43; 64 streams of one token 33 -> 30.
+//
+// Tile: scores with A = K (lane (i, g): row of position i, dims 32 s + 8 g .. of step s) and B = q (lane (j, g): column j, same dims)
+// -> lane (j, g) holds column j at positions 4 g .. 4 g + 3.  Those four weights, as bf16 (value and rounding remainder: two operands),
+// are already the A operand of a 16x16x16 step over positions; its B operand -- four consecutive positions of one dim -- is read out of
+// the V tile in LDS.  The running maximum is kept per column for the whole wavefront, the running sum per lane.
+// K and V tiles are four groups of four rows of 256 bytes, one direct-to-LDS request per group (each lane 16 bytes: four whole rows), the
+// groups GS bytes apart (the transposed V reads of the four groups then fall into different banks).
+template <int QPK>
+__device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  constexpr int D = 128, NC = 16, TG = NC / QPK, RB = MK_TUNE_ATTN_TILES, PD = 132;
+  constexpr int GS = 1088, TS = 4 * GS, SLOT = 2 * TS, NEW_BYTES = MK_MAX_NEW_PER_REQ / 4 * GS;
+  constexpr int FLAG_OFF = NC * D * 2, KN_OFF = FLAG_OFF + 64, VN_OFF = KN_OFF + NEW_BYTES, PART_OFF = VN_OFF + NEW_BYTES, BUF_OFF = PART_OFF + MK_WAVES * NC * PD * 4;
+  static_assert(BUF_OFF + MK_WAVES * RB * SLOT <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
+  static_assert(MK_ATTN_MAX_REQ_PAGES * 4 <= MK_WAVES * NC * PD * 4, "page list exceeds the area it aliases");
+  static_assert(PART_OFF % 16 == 0 && BUF_OFF % 16 == 0 && KN_OFF % 16 == 0, "16-byte operands");
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int nkv = st.num_kv_heads, ps = rt.page_size;
+  uint16_t *qs = (uint16_t *)smem;                                 // [16][128]
+  int *sflag = (int *)(smem + FLAG_OFF);
+  char *knew = smem + KN_OFF, *vnew = smem + VN_OFF;               // new rows as tiles
+  float *part = (float *)(smem + PART_OFF);                        // [4][16][PD]: values, maximum, sum
+  int *spg = (int *)(smem + PART_OFF);                             // page list of the running unit (until the partials are written)
+  char *buf = smem + BUF_OFF + wave * (RB * SLOT);
+  const u32x4 *kc = (const u32x4 *)st.k_cache, *vc = (const u32x4 *)st.v_cache;
+  auto new_row = [&](char *base, int j) { return (uint16_t *)(base + (j >> 2) * GS + (j & 3) * 256); };
+  // groups of tokens: every TG-th token of a request begins one
+  const int my_first = lane < M ? c.sh_tok[2 * MK_MAX_TOKENS + lane] : 0;
+  const unsigned long long begins = __ballot(lane < M && (lane - my_first) % TG == 0);
+  const int groups = __popcll(begins), n_items = groups * nkv;
+  const int cmax = max(1, min(c.G / n_items, MK_ATTN_MAX_CHUNKS)), n_units = n_items * cmax;
+  struct Unit {
+    int item, cidx, C, t, n, h, p0, p, t0, tb, te, n_new;
+    const int *pages;
+  };
+  auto decode = [&](int u, Unit &a) -> bool {
+    a.item = u / cmax;
+    a.cidx = u - a.item * cmax;
+    const int g = a.item / nkv;
+    a.h = a.item - g * nkv;
+    const bool mine = ((begins >> lane) & 1) && __popcll(begins & ((1ull << lane) - 1)) == g;
+    a.t = (int)__ffsll(__ballot(mine)) - 1;
+    a.t0 = __builtin_amdgcn_readfirstlane(c.sh_tok[2 * MK_MAX_TOKENS + a.t]);
+    a.n = __popcll(__ballot(lane < M && lane >= a.t && lane < a.t + TG && my_first == a.t0));
+    a.p0 = __builtin_amdgcn_readfirstlane(c.sh_tok[a.t0]);
+    a.p = __builtin_amdgcn_readfirstlane(c.sh_tok[a.t]) + a.n - 1;  // newest position
+    const int nt = (a.p0 + 15) / 16, n_new = a.p + 1 - a.p0;        // cached tiles, new rows
+    // One cached tile per wavefront and a chunk of its own for the new rows while workgroups are plenty; else the last chunk, which
+    // prepares those rows, takes fewer tiles: a round of rows takes as long as about four tiles of every wavefront.
+    const int Cd = (nt + MK_WAVES - 1) / MK_WAVES + 1;
+    a.C = min(Cd, cmax);
+    if (a.cidx >= a.C) return false;
+    if (a.C == Cd) {
+      a.tb = a.cidx < a.C - 1 ? (int)((long long)nt * a.cidx / (a.C - 1)) : nt;
+      a.te = a.cidx < a.C - 1 ? (int)((long long)nt * (a.cidx + 1) / (a.C - 1)) : nt;
+    } else {
+      const int extra = 4 * MK_WAVES * ((a.n * QPK + 2 * n_new + 31) / 32 - 1);
+      const int total = nt + (a.C > 1 ? min(extra, (nt + a.C - 2) / (a.C - 1)) : 0);
+      a.tb = min(nt, (int)((long long)total * a.cidx / a.C));
+      a.te = a.cidx < a.C - 1 ? min(nt, (int)((long long)total * (a.cidx + 1) / a.C)) : nt;
+    }
+    a.n_new = a.cidx == a.C - 1 ? n_new : 0;
+    a.pages = rt.kv_indices + __builtin_amdgcn_readfirstlane(c.sh_tok[3 * MK_MAX_TOKENS + a.t]);
+    return true;
+  };
+  // (the norm weights and the first unit's page list are requested before the barrier is awaited)
+  AttnSource src = attn_source(st, lane);
+  Unit a0;
+  const bool have0 = c.vid < n_units && decode(c.vid, a0);
+  auto page_range = [&](const Unit &a, int &lo) -> int {
+    lo = a.tb * 16 / ps;
+    return a.te > a.tb ? (min(a.p0, a.te * 16) - 1) / ps - lo + 1 : 0;
+  };
+  int pg0 = 0;
+  if (have0) {
+    int lo;
+    if (tid < page_range(a0, lo)) pg0 = a0.pages[lo + tid];
+  }
+  barrier_wait(c);
+  attn_source_ready(st, c, src);
+
+  for (int uu = c.vid; uu < n_units; uu += c.G) {
+    Unit a;
+    const bool first = uu == c.vid;
+    int u = uu;
+    if (cmax == 1 && ((uu / c.G) & 1)) {  // every other round deals the units in reverse order (contexts differ)
+      const int r0 = (uu / c.G) * c.G, rn = min(c.G, n_units - r0);
+      u = r0 + rn - 1 - (uu - r0);
+    }
+    if (first) {
+      if (!have0) continue;
+      a = a0;
+    } else if (!decode(u, a)) {
+      continue;
+    }
+    const int n_cols = a.n * QPK, p_first = a.p + 1 - a.n, nt = a.te - a.tb, cend = min(a.p0, a.te * 16);
+    __syncthreads();  // LDS reuse across units
+    // ---- page list, then the first tiles, then the rows
+    int pg_lo;
+    const int npg = page_range(a, pg_lo);
+    if (first && tid < npg) spg[tid] = pg0;
+    for (int i = tid + (first ? MK_THREADS : 0); i < npg; i += MK_THREADS) spg[i] = a.pages[pg_lo + i];
+    for (int j = a.n_new * 16 + tid; j < (a.n_new + 15) / 16 * 256; j += MK_THREADS) ((u32x4 *)new_row(vnew, j >> 4))[j & 15] = (u32x4){0u, 0u, 0u, 0u};
+    __syncthreads();
+    auto row_base = [&](int pos) -> size_t {  // first 16-byte operand of the (position, head) row
+      const int pc = min(pos, cend - 1), pg = pc / ps;
+      return (((size_t)spg[pg - pg_lo] * ps + (pc - pg * ps)) * nkv + a.h) * (D / 8);
+    };
+    // request s brings rows 4 s .. 4 s + 3 whole (lane (row in group, 16-byte piece)); streaming requests: a cached row need not displace
+    // the activations the linears share through the L2.  A tile index past the end re-reads the last tile; it is never computed.
+    auto load_tile = [&](int tt, char *b) {
+      constexpr int KV_NT = 2;
+      const int q0 = (a.tb + min(tt, nt - 1)) * 16;
+      size_t gb[4];
+#pragma unroll
+      for (int s_ = 0; s_ < 4; s_++) gb[s_] = row_base(q0 + 4 * s_ + lg) + lr;
+#pragma unroll
+      for (int s_ = 0; s_ < 4; s_++)
+        __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(kc + gb[s_]),
+                                         (__attribute__((address_space(3))) void *)(__attribute__((address_space(3))) char *)(b + TS + s_ * GS), 16, 0, KV_NT);
+#pragma unroll
+      for (int s_ = 0; s_ < 4; s_++)
+        __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(vc + gb[s_]),
+                                         (__attribute__((address_space(3))) void *)(__attribute__((address_space(3))) char *)(b + s_ * GS), 16, 0, KV_NT);
+    };
+    if (wave < nt) {
+#pragma unroll
+      for (int b_ = 0; b_ < RB - 1; b_++) load_tile(wave + b_ * MK_WAVES, buf + b_ * SLOT);
+    }
+    auto row = [&](int i) -> AttnRow {
+      const int j = i - n_cols, kind = j < 0 ? 0 : j < a.n_new ? 1 : 2, jj = kind == 2 ? j - a.n_new : j, base = a.h * (QPK + 2) * D;
+      return kind ? AttnRow{a.t0 + jj, base + (QPK + kind - 1) * D, a.p0 + jj, kind, new_row(kind == 1 ? knew : vnew, jj)}
+                  : AttnRow{a.t + i / QPK, base + (i % QPK) * D, p_first + i / QPK, 0, qs + i * D};
+    };
+    auto own = [&](int tok) { return a.n_new > 0 && tok >= a.t; };
+    const int n_rows = n_cols + 2 * a.n_new;
+    if (n_rows > 4 * MK_WAVES) attn_rows<8>(st, src, n_rows, lane, wave, row, own);
+    else attn_rows<4>(st, src, n_rows, lane, wave, row, own);
+    __syncthreads();
+    // ---- tiles
+    bf16x8 qb[4];
+#pragma unroll
+    for (int s_ = 0; s_ < 4; s_++) {
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      qb[s_] = __builtin_bit_cast(bf16x8, lr < n_cols ? *(const u32x4 *)(qs + lr * D + s_ * 32 + lg * 8) : z);
+    }
+    f32x4 o[8];
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float mrun = -INFINITY, lsum = 0.f;
+    // positions [q0, q0 + 16) whose rows lie at kb / vb; this lane's column sees those up to `last` (at least one of them)
+    auto compute_tile = [&](int q0, int last, const char *kb, const char *vb) {
+      f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+      const char *kl = kb + (lr >> 2) * GS + (lr & 3) * 256 + lg * 16;
+#pragma unroll
+      for (int s_ = 0; s_ < 4; s_++) s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *(const u32x4 *)(kl + s_ * 64)), qb[s_], s4, 0, 0, 0);
+      float sc[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) sc[r] = q0 + lg * 4 + r <= last ? s4[r] * st.sm_scale_log2 : -INFINITY;
+      float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+      mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, mx))));
+      mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, mx))));
+      const float mn = fmaxf(mrun, mx);
+      const float alpha = __builtin_amdgcn_exp2f(mrun - mn);
+      float pw[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) pw[r] = __builtin_amdgcn_exp2f(sc[r] - mn);
+      lsum = lsum * alpha + ((pw[0] + pw[1]) + (pw[2] + pw[3]));
+      mrun = mn;
+      if (__ballot(lr < n_cols && alpha != 1.f)) {  // (uniform) some column's maximum moved: rescale what has been summed
+        float ar[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) ar[r] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lg * 4 + r) << 2, __builtin_bit_cast(int, alpha)));
+#pragma unroll
+        for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) o[dt][r] *= ar[r];
+      }
+      float ph[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) ph[r] = bfround(pw[r]);
+      const unsigned h01 = pack2(ph[0], ph[1]), h23 = pack2(ph[2], ph[3]);
+      const unsigned l01 = pack2(pw[0] - ph[0], pw[1] - ph[1]), l23 = pack2(pw[2] - ph[2], pw[3] - ph[3]);
+      const s16x4 a_hi = __builtin_bit_cast(s16x4, (unsigned long long)h01 | ((unsigned long long)h23 << 32));
+      const s16x4 a_lo = __builtin_bit_cast(s16x4, (unsigned long long)l01 | ((unsigned long long)l23 << 32));
+      const char *vl = vb + lg * GS + lr * 2;
+#pragma unroll
+      for (int dt = 0; dt < 8; dt++) {
+        const char *q_ = vl + dt * 32;
+        const unsigned v0 = *(const uint16_t *)(q_), v1 = *(const uint16_t *)(q_ + 256), v2 = *(const uint16_t *)(q_ + 512), v3 = *(const uint16_t *)(q_ + 768);
+        const s16x4 bv = __builtin_bit_cast(s16x4, (unsigned long long)(v0 | (v1 << 16)) | ((unsigned long long)(v2 | (v3 << 16)) << 32));
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_hi, bv, o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_lo, bv, o[dt], 0, 0, 0);
+      }
+    };
+    // cached tiles: RB in flight per wavefront; every request is issued unconditionally, and the wait before a tile counts the
+    // 8 (RB - 1) requests of the tiles after it
+    int t_ = wave;
+    if (t_ < nt) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows stored above are not counted below; the first tiles arrived with the rows)
+      bool more = true;
+      while (more) {
+#pragma unroll
+        for (int b_ = 0; b_ < RB; b_++) {
+          load_tile(t_ + (RB - 1) * MK_WAVES, buf + ((b_ + RB - 1) % RB) * SLOT);
+          static_assert(RB == 2, "the wait counts one tile's requests");
+          asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+          if (more) {
+            compute_tile((a.tb + t_) * 16, cend - 1, buf + b_ * SLOT + TS, buf + b_ * SLOT);
+            t_ += MK_WAVES;
+            more = t_ < nt;
+          }
+        }
+      }
+    }
+    // new tiles: all tokens of a group lie in the last of them (groups begin at multiples of TG in their request, TG divides 16)
+    const int p_col = p_first + min(lr, n_cols - 1) / QPK;
+    for (int k = wave; k * 16 < a.n_new; k += MK_WAVES) compute_tile(a.p0 + k * 16, p_col, knew + k * TS, vnew + k * TS);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the direct-to-LDS requests of the tile that was not computed)
+    // the chunk with the new rows appends the group's own K/V rows and publishes its queries
+    if (a.n_new) {
+      for (int i = tid; i < a.n * 64; i += MK_THREADS) {
+        const int pos = p_first + (i >> 6), e = i & 63;
+        const size_t at = (((size_t)a.pages[pos / ps] * ps + pos % ps) * nkv + a.h) * (D / 2) + e;
+        ((uint32_t *)st.k_cache)[at] = ((const uint32_t *)new_row(knew, pos - a.p0))[e];
+        ((uint32_t *)st.v_cache)[at] = ((const uint32_t *)new_row(vnew, pos - a.p0))[e];
+      }
+      if (st.q_ws)
+        for (int i = tid; i < n_cols * 64; i += MK_THREADS) {
+          const int col = i >> 6;
+          ((uint32_t *)st.q_ws)[((size_t)(a.t + col / QPK) * st.ld_qws + (size_t)(a.h * QPK + col % QPK) * D) / 2 + (i & 63)] = ((const uint32_t *)qs)[i];
+        }
+    }
+    __syncthreads();  // every wavefront is done with the page list: the partial results may overwrite it
+    // ---- wavefronts
+    float lt = lsum;
+    lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, lt)));
+    lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, lt)));
+    if (lg == 0) {
+      part[(wave * NC + lr) * PD + D] = mrun;
+      part[(wave * NC + lr) * PD + D + 1] = lt;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int dt = 0; dt < 8; dt++) part[(wave * NC + lg * 4 + r) * PD + dt * 16 + lr] = o[dt][r];
+    __syncthreads();
+    // (die-local or device-scope hand-over of chunks: see stage_attn)
+    const bool local = !rt.attn_part && c.even_xcds && (a.item * cmax) / c.quota == (a.item * cmax + a.C - 1) / c.quota;
+    float *part_base = rt.attn_part ? rt.attn_part : (float *)st.aux0;
+    const int col = tid >> 4, md = (tid & 15) * 8;  // this thread's column and dims
+    uint16_t *orow = (uint16_t *)st.out + (size_t)(a.t + col / QPK) * st.ld_out + (size_t)(a.h * QPK + col % QPK) * D + md;
+    auto emit = [&](const float (&v)[8], float l) {  // written through: the stage's barrier skips the L2 write-back
+#pragma unroll
+      for (int d = 0; d < 8; d += 2) __hip_atomic_store((uint32_t *)(orow + d), pack2(v[d] / l, v[d + 1] / l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (col < n_cols) {
+      float mx = -1e30f, ls = 0.f, os[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < MK_WAVES; w++) mx = fmaxf(mx, part[(w * NC + col) * PD + D]);
+#pragma unroll
+      for (int w = 0; w < MK_WAVES; w++) {
+        const float *pp = part + (w * NC + col) * PD;
+        const float wgt = __builtin_amdgcn_exp2f(pp[D] - mx);
+        ls += pp[D + 1] * wgt;
+#pragma unroll
+        for (int d = 0; d < 8; d++) os[d] += pp[md + d] * wgt;
+      }
+      if (a.C == 1) {
+        emit(os, ls);
+      } else {
+        // whole 128-byte lines (the maximum and sum fill a line of their own, 16 copies): see stage_attn
+        float *gp = part_base + ((size_t)u * NC + col) * MK_ATTN_PSTRIDE;
+#pragma unroll
+        for (int d = 0; d < 8; d += 4) *(f32x4 *)(gp + md + d) = (f32x4){os[d], os[d + 1], os[d + 2], os[d + 3]};
+        *(float2 *)(gp + D + 2 * (tid & 15)) = make_float2(mx, ls);
+      }
+    }
+    if (a.C == 1) continue;
+    // ---- chunks: the last to finish merges them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      int last;
+      if (local) {
+        unsigned *cnt = (unsigned *)st.aux1 + (size_t)a.item * 32;
+        last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP) == (unsigned)(a.C - 1);
+        if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      } else {
+        unsigned *cnt = &rt.attn_cnt[(size_t)a.item * 32];
+        last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.C - 1);
+        if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      *sflag = last;
+    }
+    __syncthreads();
+    if (!*sflag || col >= n_cols) continue;
+    const float *ip = part_base + ((size_t)a.item * cmax * NC + col) * MK_ATTN_PSTRIDE;
+    float mx = -1e30f, ls = 0.f, os[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto merge = [&](auto load8) {
+      constexpr int CB = 8;  // chunks in flight
+      for (int c0 = 0; c0 < a.C; c0 += CB) {
+        float2 ml[CB], ov[CB][4];
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+          if (c0 + j < a.C) {
+            const float *pp = ip + (size_t)(c0 + j) * NC * MK_ATTN_PSTRIDE;
+            ml[j] = load8(pp + D);
+#pragma unroll
+            for (int d = 0; d < 4; d++) ov[j][d] = load8(pp + md + 2 * d);
+          }
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+          if (c0 + j < a.C) {
+            const float mn = fmaxf(mx, ml[j].x);
+            const float sa = __builtin_amdgcn_exp2f(mx - mn), sb = __builtin_amdgcn_exp2f(ml[j].x - mn);
+            ls = ls * sa + ml[j].y * sb;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+              os[2 * d] = os[2 * d] * sa + ov[j][d].x * sb;
+              os[2 * d + 1] = os[2 * d + 1] * sa + ov[j][d].y * sb;
+            }
+            mx = mn;
+          }
+      }
+    };
+    if (local) merge([](const float *q) { return *(const float2 *)q; });
+    else
+      merge([](const float *q) {
+        const unsigned long long v = ldc_u64(q);
+        return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+      });
+    emit(os, ls);
+  }
+  c.wrote_through = true;  // (as in stage_attn)
 }
 
 // Greedy sampling, stage 1: every workgroup scans a contiguous slice of each token's logits and keeps
@@ -4391,18 +4596,18 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
           if constexpr (FX) {
             barrier_wait(c);
           } else if constexpr (MAXM == 1) {
-            if (st.num_q_heads == 4 * st.num_kv_heads) stage_attn<4, false>(st, c, rt, M, smem);
-            else if (st.num_q_heads == 8 * st.num_kv_heads) stage_attn<8, false>(st, c, rt, M, smem);
+            if (st.num_q_heads == 4 * st.num_kv_heads) stage_attn<4>(st, c, rt, M, smem);
+            else if (st.num_q_heads == 8 * st.num_kv_heads) stage_attn<8>(st, c, rt, M, smem);
             else barrier_wait(c);
           } else {
             // many (token, kv head) pairs per workgroup-chunk: cached positions on the matrix cores
             const bool mf = 2 * M * st.num_kv_heads >= c.G;
             if (st.num_q_heads == 4 * st.num_kv_heads) {
-              if (mf) stage_attn<4, true>(st, c, rt, M, smem);
-              else stage_attn<4, false>(st, c, rt, M, smem);
+              if (mf) stage_attn_tiles<4>(st, c, rt, M, smem);
+              else stage_attn<4>(st, c, rt, M, smem);
             } else if (st.num_q_heads == 8 * st.num_kv_heads) {
-              if (mf) stage_attn<8, true>(st, c, rt, M, smem);
-              else stage_attn<8, false>(st, c, rt, M, smem);
+              if (mf) stage_attn_tiles<8>(st, c, rt, M, smem);
+              else stage_attn<8>(st, c, rt, M, smem);
             } else {
               barrier_wait(c);
             }

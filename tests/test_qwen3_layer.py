@@ -111,6 +111,34 @@ def test_small_layer_prefill_chunks(L_cached, n_new):
     _check(res, cfg, L_cached, n_new)
 
 
+@pytest.mark.parametrize("nkv,L_cached,n_new", [(8, 0, 64), (8, 37, 33), (8, 1000, 17), (8, 2300, 64), (8, 15, 16), (8, 64, 4), (4, 0, 9), (4, 200, 64), (4, 15, 61), (4, 129, 3), (2, 70, 50)])
+def test_portions_in_units_of_several_tokens(nkv, L_cached, n_new):
+    """Attention units that take the tokens of a portion four (two) at a time: the last unit short or whole, new rows that fill their last tile
+    or not, no cached position, a cached tile cut short, one chunk and many."""
+    from helpers import flips
+    from oracle.qwen3_ref import Qwen3Config, attention_k, head_norm_rope_k
+    cfg = Qwen3Config(hidden_size=1024, num_q_heads=8 if nkv == 2 else 32, num_kv_heads=nkv, head_dim=128, intermediate_size=1536, num_layers=1)
+    res = _run_layer(cfg, L_cached, n_new, "fleet", seed=300 + L_cached + n_new)
+    nq, D = cfg.num_q_heads, 128
+    qkv = res["qkv_gpu"].view(n_new, nkv, nq // nkv + 2, D)
+    at = torch.arange(L_cached, L_cached + n_new)
+    page, row = torch.tensor(res["pages"])[at // res["page_size"]], at % res["page_size"]
+    k_new, v_new = res["k_after"][page, row], res["v_after"][page, row]
+    assert torch.equal(v_new.view(n_new, nkv, D), qkv[:, :, -1])
+    c, s_ = res["cos"][at][:, None, :], res["sin"][at][:, None, :]
+    for got, rows, w in ((res["qws_gpu"].view(n_new, nq, D), qkv[:, :, :-2].reshape(n_new, nq, D), "q_norm"), (k_new.view(n_new, nkv, D), qkv[:, :, -2], "k_norm")):
+        want = head_norm_rope_k(rows, res["lw"][w], c, s_).float()
+        # a normalised element may round the other way (one bf16 step of 2^-8, in both elements of a rotation pair), and so may the result
+        pair = torch.hypot(want[..., :64], want[..., 64:]).repeat(1, 1, 2)
+        assert bool(((got.float() - want).abs() <= 2.0 ** -8 * (2 ** 0.5 * pair + want.abs())).all()), w
+        assert (got.float() != want).float().mean() < 0.02, w
+    k = torch.cat([res["cache"].k[0, :L_cached], k_new.view(n_new, nkv, D)])
+    v = torch.cat([res["cache"].v[0, :L_cached], v_new.view(n_new, nkv, D)])
+    want = torch.stack([attention_k(res["qws_gpu"][t].view(nq, D), k[:L_cached + t + 1], v[:L_cached + t + 1]) for t in range(n_new)])
+    frac, u = flips(res["attn_gpu"].view(n_new, nq, D), want)
+    assert frac < 0.05 and u <= 1.0, f"attention: {frac:.4f} differ, max {u} ulp"
+
+
 def test_full_width_layer_prefill_chunk_mpk_mode():
     from oracle.qwen3_ref import Qwen3Config
     cfg = Qwen3Config(num_layers=1)
