@@ -137,7 +137,7 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
 // preceding linear's output, or its K-slice partials when that linear left its sum to this stage.  A workgroup per row.
 // Rows of up to 4096 values, four quads per thread.  Bound by the barrier and one round trip for the row: the slices of all quads are
 // requested before the first value is waited for (a branch around each quad had made a round trip per quad of it).
-// 4096 values from four slices, as a stage: 8.9 -> 6.7 us at 4 rows, 9.5 -> 7.1 at 64.
+// 4096 values from four slices, as a stage: 8.9 -> 6.7 us at 4 rows, 9.5 -> 7.1 at 64; now 3.6 and 4.2.
 __device__ __forceinline__ int fx_quad_at(const Ctx &c, int c0, int j, int n4) { return min(c0 + c.tid + j * MK_THREADS, n4 - 1); }
 // v = alpha * x + y of four quads of a row
 template <typename E>
@@ -149,9 +149,11 @@ __device__ __forceinline__ void fx_addnorm_sum(CStage &st, const Ctx &c, int dS,
       constexpr int Q = decltype(ns)::value;
       f32x4 q[4][Q];
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int b = 0; b < Q; b++) {
+        const auto rows = dev_rows(p + b * slice);
 #pragma unroll
-        for (int b = 0; b < Q; b++) q[j][b] = fx_ldc_quad(p + b * slice + 4 * fx_quad_at(c, c0, j, n4));
+        for (int j = 0; j < 4; j++) q[j][b] = __builtin_bit_cast(f32x4, ldc_16B(rows, 16 * fx_quad_at(c, c0, j, n4)));
+      }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         v[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -189,7 +191,7 @@ __device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char
   f32x4 x[4], v[4];
   auto load_x = [&](int t, int c0) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) x[j] = fx_ldc_quad(xr + (size_t)t * st.ld_res + 4 * fx_quad_at(c, c0, j, n4));
+    for (int j = 0; j < 4; j++) x[j] = __builtin_bit_cast(f32x4, ldc_16B(dev_rows(xr + (size_t)t * st.ld_res), 16 * fx_quad_at(c, c0, j, n4)));
   };
   auto squares = [&](int c0) {
     float ss = 0.f;
