@@ -90,6 +90,7 @@ typedef const __attribute__((address_space(4))) MkWeight CWeight;
 #define MK_HAVE_MIX 0
 #endif
 
+#define MK_NO_LISTS 0x7fffffff
 struct Ctx {
   int tid;   // threadIdx.x, made opaque for every stage that runs: see run_stage_program
   CStage *st;  // descriptor of the stage that runs (null before the first one)
@@ -109,7 +110,7 @@ struct Ctx {
   MkSync *sync;
   const int *sh_tok;  // LDS copy of this iteration's token metadata: [0] position, [1] batch slot, [2] first token of the request, [3] first page-table entry
   bool even_xcds;     // every die in use runs the same number of workgroups, so die index = vid / quota
-  int *sh_ticket;     // two LDS work counters, used alternately by consecutive executed stages; [2] = seq of the single-token
+  int *sh_ticket;     // two LDS work counters, used alternately by consecutive executed stages; [2] = seq (multi-token: ~seq) of the
                       // MoE stage that last filled the workgroup's expert list (kept outside the stages' scratch LDS)
   int seq;            // stages executed so far by this workgroup
   unsigned prof_n;    // entries this workgroup has written into the caller's profiler tensor
@@ -3111,7 +3112,7 @@ __device__ __forceinline__ void stage_moe_linear_m1(CStage &st, Ctx &c, char *sm
 // loop every unit waited for all outstanding loads).  The tile is written out at the end, one contiguous run of
 // rows per (token, slot).  A workgroup whose tile or staged rows do not fit runs a plain loop over the same units.
 template <int KL, int R, bool SILU>
-__device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M, char *smem) {
+__device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M, bool reuse, char *smem) {
   constexpr int NROW = SILU ? 2 : 1;
   constexpr int NARR = SILU ? 3 : 1;
   const int tid = c.tid, lane = tid & 63;
@@ -3127,6 +3128,7 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
   int *bnd = L->wtot[0];  // reused: the scans of the list building are done
   if (tid < 2) bnd[tid] = 0;
   __syncthreads();
+  if (tid == 0) c.sh_ticket[2] = ~c.seq;  // (everybody has looked at it)
   const long long total = (long long)NR * (L->pair_off[n_act] + RC * n_act);
   const long long tgt0 = total * c.vid / c.G, tgt1 = total * (c.vid + 1) / c.G;
   if (tid < n_act) {
@@ -3154,7 +3156,51 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
   // the decision below is per workgroup (uniform within it); either form covers exactly [u_begin, u_end)
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const u32x4 *W = (const u32x4 *)st.w.seg[0];
-  if ((size_t)n_pairs * k8 * 16 > (size_t)(MK_LDS_BYTES - MK_MOE_X_OFFSET) || (size_t)NARR * maxp * nu * 2 > (size_t)MK_MOE_OFFSET) {
+  const bool plain = (size_t)n_pairs * k8 * 16 > (size_t)(MK_LDS_BYTES - MK_MOE_X_OFFSET) || (size_t)NARR * maxp * nu * 2 > (size_t)MK_MOE_OFFSET;
+  int *ticket = c.sh_ticket + (c.seq & 1);
+  auto take = [&](int n) -> int {  // first of the next n units of this workgroup (may lie at or beyond u_end)
+    int t = 0;
+    if (lane == 0) t = __hip_atomic_fetch_add(ticket, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return __builtin_amdgcn_readfirstlane(t) + u_begin;
+  };
+  // Every row load is unconditional: a unit at or beyond the end of the range re-reads the range's last unit and is
+  // not reduced.  (With the loads under a branch every wait for one unit's rows drained the other units' loads too.)
+  auto load_unit = [&](int u_, u32x4 (&b)[NROW][KL]) {
+    const int u = min(u_, u_end - 1);
+    const int a = u / NR, j = u - a * NR;
+    const size_t e = (size_t)__builtin_amdgcn_readfirstlane(L->act_e[a]);
+#pragma unroll
+    for (int h = 0; h < NROW; h++) {
+      const u32x4 *p = W + (e * st.n + (size_t)(j + h * NR)) * k8;
+#pragma unroll
+      for (int kc = 0; kc < KL; kc++) b[h][kc] = ldg_stream(p + min(kc * 64 + lane, k8 - 1));  // lanes past the row re-read its last segment; their products are dropped below
+    }
+  };
+  // two groups of units in flight: while one is reduced the other one's rows are landing; tickets only grow, so the
+  // first group found beyond the range ends the loop
+  constexpr int QA = (R + 1) / 2, QB = R / 2;
+  u32x4 bufA[QA][NROW][KL], bufB[QB > 0 ? QB : 1][NROW][KL];
+  int gA = u_end, gB = u_end;
+  auto fill = [&]() {
+    gA = take(QA);
+#pragma unroll
+    for (int q = 0; q < QA; q++) load_unit(gA + q, bufA[q]);
+    if (QB > 0) {
+      gB = take(QB);
+#pragma unroll
+      for (int q = 0; q < QB; q++) load_unit(gB + q, bufB[q]);
+    }
+  };
+  // with the lists of the stage before, the first groups' rows are requested before the barrier is awaited (not the polling wavefront's:
+  // they would hold up the poll)
+  const bool early = !SILU && reuse && nu > 0 && !plain && __builtin_amdgcn_readfirstlane(tid >> 6) != 0;
+  if (early) fill();
+  if (!SILU && reuse) {
+    barrier_wait(c);
+    if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
+  }
+  if (plain) {
     // too many tokens on this workgroup's experts for the LDS windows: plain form over the same unit range
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint16_t *out = (uint16_t *)st.out, *out2 = (uint16_t *)st.out2;
@@ -3187,34 +3233,8 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
     }
     return;
   }
-  // stage the input rows of the (token, slot) pairs of this workgroup's experts
   u32x4 *xs4 = (u32x4 *)(smem + MK_MOE_X_OFFSET);
   uint16_t *so = (uint16_t *)smem;  // [array][pair of the expert][unit - u_begin]
-  for (int i = tid; i < n_pairs * k8; i += MK_THREADS) {
-    const int p = i / k8, o = i - p * k8;
-    const int ts = L->pair_ts[p_base + p], tok = ts & 255, slot = ts >> 8;
-    xs4[i] = ((const u32x4 *)((const uint16_t *)st.in + (size_t)tok * st.ld_in + (size_t)slot * st.ld_in_slot))[o];
-  }
-  __syncthreads();
-  int *ticket = c.sh_ticket + (c.seq & 1);
-  auto take = [&](int n) -> int {  // first of the next n units of this workgroup (may lie at or beyond u_end)
-    int t = 0;
-    if (lane == 0) t = __hip_atomic_fetch_add(ticket, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    return __builtin_amdgcn_readfirstlane(t) + u_begin;
-  };
-  // Every row load is unconditional: a unit at or beyond the end of the range re-reads the range's last unit and is
-  // not reduced.  (With the loads under a branch every wait for one unit's rows drained the other units' loads too.)
-  auto load_unit = [&](int u_, u32x4 (&b)[NROW][KL]) {
-    const int u = min(u_, u_end - 1);
-    const int a = u / NR, j = u - a * NR;
-    const size_t e = (size_t)__builtin_amdgcn_readfirstlane(L->act_e[a]);
-#pragma unroll
-    for (int h = 0; h < NROW; h++) {
-      const u32x4 *p = W + (e * st.n + (size_t)(j + h * NR)) * k8;
-#pragma unroll
-      for (int kc = 0; kc < KL; kc++) b[h][kc] = ldg_stream(p + min(kc * 64 + lane, k8 - 1));  // lanes past the row re-read its last segment; their products are dropped below
-    }
-  };
   auto reduce_unit = [&](const u32x4 (&b)[NROW][KL], int u) {
     const int a = u / NR;
     const int p0 = __builtin_amdgcn_readfirstlane(L->pair_off[a]), p1 = __builtin_amdgcn_readfirstlane(L->pair_off[a + 1]);
@@ -3291,19 +3311,15 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
       }
     }
   };
-  // two groups of units in flight: while one is reduced the other one's rows are landing; tickets only grow, so the
-  // first group found beyond the range ends the loop
-  constexpr int QA = (R + 1) / 2, QB = R / 2;
+  // stage the input rows of the (token, slot) pairs of this workgroup's experts
+  for (int i = tid; i < n_pairs * k8; i += MK_THREADS) {
+    const int p = i / k8, o = i - p * k8;
+    const int ts = L->pair_ts[p_base + p], tok = ts & 255, slot = ts >> 8;
+    xs4[i] = ((const u32x4 *)((const uint16_t *)st.in + (size_t)tok * st.ld_in + (size_t)slot * st.ld_in_slot))[o];
+  }
+  __syncthreads();
   if (nu > 0) {
-    u32x4 bufA[QA][NROW][KL], bufB[QB > 0 ? QB : 1][NROW][KL];
-    int gA = take(QA), gB = u_end;
-#pragma unroll
-    for (int q = 0; q < QA; q++) load_unit(gA + q, bufA[q]);
-    if (QB > 0) {
-      gB = take(QB);
-#pragma unroll
-      for (int q = 0; q < QB; q++) load_unit(gB + q, bufB[q]);
-    }
+    if (!early) fill();
     while (gA < u_end) {
       reduce_group(bufA, gA, std::integral_constant<int, QA>{});
       gA = take(QA);
@@ -3349,26 +3365,36 @@ __device__ __forceinline__ void stage_moe_linear(CStage &st, Ctx &c, int M, char
     }
   }
   if (M > 1) {
-    // common front: wait for the previous stage, one acquire (activation rows are read with cached loads), routing lists
+    // common front: wait for the previous stage, one acquire (activation rows are read with cached loads), routing lists.  Directly behind
+    // another expert linear over the same routing table (W2 behind W13) the lists are still in LDS: that stage starts its stream ahead of the
+    // barrier.  qwen3-30b-a3b, 16 tokens, W2: 61 -> 51 us.  (Rows of up to 1024 only: in the instances for longer ones, which have no such
+    // stage here, it moved the register allocation of the multi-token linears, a prompt of qwen3-8b 50.1 -> 50.7 ms.)
     MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
-    barrier_wait(c);
-    if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __syncthreads();
-    moe_build_lists(st, c, L, M, false);
-    if (c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)
+    bool reuse = !silu && st.k <= 1024 && __builtin_amdgcn_readfirstlane(c.sh_ticket[2]) == ~(c.seq - 1);
+    if (reuse) {
+      CStage &pv = (&st)[-1];
+      reuse = pv.op == MK_OP_MOE_LINEAR && pv.moe_routing == st.moe_routing && pv.num_experts == st.num_experts && pv.topk == st.topk && pv.ld_routing == st.ld_routing;
+    }
+    if (!reuse) {
+      barrier_wait(c);
+      if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      __syncthreads();
+      moe_build_lists(st, c, L, M, false);
+    }
+    if (!(reuse && (&st)[-1].moe_mask == st.moe_mask) && c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)
       const int n_act = L->n_act;
       for (int i = c.tid; i < st.num_experts; i += MK_THREADS) st.moe_mask[i] = i < n_act ? L->act_e[i] : -1;
       if (c.tid == 0) st.moe_mask[st.num_experts] = n_act;
     }
     if (st.k <= 1024) {
-      if (silu) stage_moe_linear_multi<2, 4, true>(st, c, M, smem);
-      else stage_moe_linear_multi<2, MK_TUNE_MOE_R2, false>(st, c, M, smem);
+      if (silu) stage_moe_linear_multi<2, 4, true>(st, c, M, false, smem);
+      else stage_moe_linear_multi<2, MK_TUNE_MOE_R2, false>(st, c, M, reuse, smem);
     } else if (st.k <= 2048) {
-      if (silu) stage_moe_linear_multi<4, MK_TUNE_MOE_R13, true>(st, c, M, smem);
-      else stage_moe_linear_multi<4, 4, false>(st, c, M, smem);
+      if (silu) stage_moe_linear_multi<4, MK_TUNE_MOE_R13, true>(st, c, M, false, smem);
+      else stage_moe_linear_multi<4, 4, false>(st, c, M, false, smem);
     } else {
-      if (silu) stage_moe_linear_multi<8, 1, true>(st, c, M, smem);
-      else stage_moe_linear_multi<8, 2, false>(st, c, M, smem);
+      if (silu) stage_moe_linear_multi<8, 1, true>(st, c, M, false, smem);
+      else stage_moe_linear_multi<8, 2, false>(st, c, M, false, smem);
     }
     return;
   }
@@ -4691,7 +4717,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   c.arrive_w0 = false;
   if (threadIdx.x == 0) {
     sh_ticket[0] = sh_ticket[1] = 0;
-    sh_ticket[2] = -2;
+    sh_ticket[2] = MK_NO_LISTS;
   }
   // ---- XCD discovery: rank of this workgroup inside its die, dies in use, workgroups per die
   if (threadIdx.x == 0) {
@@ -4766,6 +4792,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
     if (threadIdx.x == 0) {
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       sh_bcast[0] = ldc_i32(&rt.sched->num_tokens);
+      c.sh_ticket[2] = MK_NO_LISTS;  // (expert lists are this iteration's)
     }
     __syncthreads();
     const int Mrt = __builtin_amdgcn_readfirstlane(sh_bcast[0]);

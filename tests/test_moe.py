@@ -167,6 +167,46 @@ def test_moe_standalone_stages_and_user_routing():
     mpk.finalize()
 
 
+@pytest.mark.parametrize("E,topk,K,H,B", [(12, 3, 192, 256, 5), (40, 6, 1024, 320, 64), (4, 2, 1024, 512, 64), (12, 3, 1152, 256, 16)])
+def test_expert_linears_one_behind_the_other(E, topk, K, H, B):
+    """The second stage uses the routing table of the first (and writes a mask of its own), the third another table, the fourth that one again;
+    few and many tokens an expert (staged rows, plain form), rows of up to 1024 and longer ones, iterations of fewer tokens and of one."""
+    import mirage as mi
+    from oracle.qwen3_ref import linear_k
+    g = torch.Generator().manual_seed(E + K)
+    bf = torch.bfloat16
+    x = torch.randn(B, topk, K, generator=g).to(bf)
+    ws = [(torch.randn(E, H, K, generator=g) / K ** 0.5).to(bf) for _ in range(4)]
+    experts = [torch.stack([torch.randperm(E, generator=g)[:topk] for _ in range(B)]) for _ in range(2)]
+    routing = torch.zeros(2, E, B, dtype=torch.int32)
+    for q in range(2):
+        for tk in range(B):
+            for s in range(topk):
+                routing[q, experts[q][tk, s], tk] = s + 1
+    mpk = make_mpk(make_meta(B, 64, B, B, B), 64, B, B, B, 64, mode="onepass")
+    dev = lambda t, name: mpk.attach_input(t, name)
+    xs, rt = x.cuda(), [routing[q].cuda().contiguous() for q in range(2)]
+    masks, keep = [torch.zeros(E + 1, dtype=torch.int32, device="cuda") for _ in range(4)], [w.cuda() for w in ws]
+    xi, ri = dev(xs, "x"), [dev(r, f"r{q}") for q, r in enumerate(rt)]
+    ys = []
+    for i in range(4):
+        ys.append(mpk.new_tensor((B, topk, H), name=f"y{i}"))
+        mpk.moe_w2_linear_layer(input=xi, weight=dev(keep[i], f"w{i}"), moe_routing_indices=ri[i // 2], moe_mask=dev(masks[i], f"m{i}"), output=ys[i], grid_dim=(8, H // 64, 1), block_dim=(256, 1, 1))
+    mpk.compile()
+    for M in (B, 2, 1, B):
+        for m in masks:
+            m.zero_()
+        torch.cuda.synchronize()
+        mpk.run_once(list(range(M)), [0] * M)
+        for i in range(4):
+            e = experts[i // 2]
+            _close(f"stage {i}, {M} tokens", ys[i].to_torch()[:M].cpu(), torch.stack([torch.stack([linear_k(x[tk, s][None], ws[i][int(e[tk, s])])[0] for s in range(topk)]) for tk in range(M)]))
+            active = sorted(set(e[:M].flatten().tolist()))
+            m = masks[i].cpu()
+            assert int(m[E]) == len(active) and sorted(m[:len(active)].tolist()) == active
+    mpk.finalize()
+
+
 def _moe_cfg(layers=2, vocab=2048):
     from oracle.qwen3_ref import Qwen3Config
     return Qwen3Config(hidden_size=1024, num_q_heads=8, num_kv_heads=2, head_dim=128, intermediate_size=0, num_layers=layers, vocab_size=vocab,
