@@ -1011,6 +1011,10 @@ int lower_residual_prenorm(mk_graph *g, size_t &i) {
       pl.alpha = st.alpha;
       st.flags |= MK_F_ONLY_MULTI;
     }
+    // a plain linear in front whose whole output is the last summand may leave its split-K sum to this stage (which also stores it)
+    const Tensor *ly = y2 ? y2 : y;
+    if (ly && !sw && pl.op == MK_OP_LINEAR && !(pl.flags & (MK_F_SILU | MK_F_RES | MK_F_RELU2)) && pl.out == ly->ptr && pl.ld_out == (int)ly->strides[0] && pl.n == st.n && (pl.ld_out & 3) == 0)
+      pl.flags |= MK_F_DEFER_SUM;
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;

@@ -108,6 +108,35 @@ def test_gelu_gated_linear(dtype, rows, n, k):
     pk.finalize()
 
 
+@pytest.mark.parametrize("second", [False, True])
+@pytest.mark.parametrize("n,k", [(2048, 4096), (4096, 2048), (8192, 1024)])
+def test_sum_of_a_split_linear_in_front(n, k, second):
+    """A linear split over K (8, 4, 2 slices at these sizes) whose output is the last summand: the norm stage finishes the sum and stores it."""
+    g = torch.Generator().manual_seed(n + k)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    pk, _ = _graph(64, 64)
+    b16 = lambda t: t.to(torch.bfloat16).cuda()
+    t = dict(i=b16(rnd(64, k)), wl=b16(rnd(n, k) / k ** 0.5), x=rnd(64, n).cuda(), y=b16(rnd(64, n)), s1=(1 + 0.3 * rnd(n)).cuda(), s2=(1 + 0.3 * rnd(n)).cuda(), w=(1 + 0.3 * rnd(n)).cuda(),
+             lo=b16(torch.zeros(64, n)), nx=torch.zeros(64, n, device="cuda"), h=b16(torch.zeros(64, n)))
+    a = {q: pk.attach_input(v, q) for q, v in t.items()}
+    pk.linear_layer(a["i"], a["wl"], a["lo"], (1, 1, 1), (256, 1, 1))
+    kw = dict(input2=a["lo"], factor2=a["s2"]) if second else {}
+    pk.residual_prenorm_layer(a["y"] if second else a["lo"], a["x"], a["nx"], a["h"], weight=a["w"], width=n, eps=1e-4, factor=a["s1"], **kw)
+    pk.compile()
+    d = {q: v.double().cpu() for q, v in t.items()}
+    for M in (64, 17, 2, 1):
+        for q in ("lo", "nx", "h"):
+            t[q].zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        lo, nx, h = (t[q][:M].cpu().double() for q in ("lo", "nx", "h"))
+        torch.testing.assert_close(lo, (d["i"] @ d["wl"].T)[:M], **_tol(torch.bfloat16))
+        v = d["x"][:M] + d["s1"] * (d["y"][:M] if second else lo) + (d["s2"] * lo if second else 0)
+        torch.testing.assert_close(nx, v, rtol=1e-6, atol=2e-6)  # (two or three roundings of 2^-24 of values below 16)
+        torch.testing.assert_close(h, v / (v.pow(2).mean(-1, keepdim=True) + 1e-4).sqrt() * d["w"], rtol=2.0 ** -8, atol=1e-6)  # one rounding to bf16
+        assert not t["lo"][M:].any() and not t["nx"][M:].any()
+    pk.finalize()
+
+
 class JoinRig:
     """residual_prenorm with two summands, their factors and places, the convolution behind it and (fused) a linear."""
 
