@@ -904,6 +904,7 @@ int lower_flex_attention(mk_graph *g, size_t &i) {
   st.v_tiles = f32 ? 8 : (dv <= 64 ? 4 : 8);
   const int nkc = dk / KW, nkg = (nkc + st.k_tiles - 1) / st.k_tiles, nvs = (dv / 16 + st.v_tiles - 1) / st.v_tiles;
   const int64_t pages = ((int64_t)g->cfg.max_seq_length + ps - 1) / ps;
+  // (2 x MK_ATTN_MAX_CHUNKS x 16 words are spare: they keep the limit on the pages of a request where it was)
   const int64_t lds = (int64_t)nkg * st.k_tiles * 1024 + (int64_t)(dk + dv) * es + 16 + 4 * 16 * (st.v_tiles * 16 + 4) * 4 + (128 + 96 + 2 * MK_ATTN_MAX_CHUNKS * 16 + 4) * 4 + pages * 4;
   if (lds > MK_LDS_BYTES) return fail(MK_EUNSUPPORTED, "flex_attention: needs %lld bytes of LDS (head dim %d, %lld pages per request)", (long long)lds, D, (long long)pages);
   const size_t items = (size_t)B * ((H / G + 15) / 16) * G * nvs;
