@@ -327,6 +327,16 @@ int set_flex(mk_graph *g, int dtype, const char *task) {
   return MK_OK;
 }
 
+// The linear lowered last may leave its K-slice partials to the stage that is lowered next and reads `rows` first.  `res_too`: that stage
+// adds the linear's residual.  Partials are stored as whole tiles of 16 columns in rows of pl.n: a ragged last tile would reach into the
+// next row, so such a linear exchanges its slices itself.
+void leave_sum(mk_graph *g, const void *rows, int64_t ld, bool res_too = false) {
+  MkStage &pl = g->stages.back();
+  if (pl.op != MK_OP_LINEAR || (pl.flags & MK_F_SILU) || (!res_too && (pl.flags & MK_F_RES)) || pl.out != rows || pl.ld_out != ld || (pl.n & 15)) return;
+  pl.flags |= MK_F_DEFER_SUM;
+  g->stage_desc.back() += " sum=next";
+}
+
 // Lower one linear-type task (optionally preceded by a norm task whose output it consumes, optionally
 // followed by a silu_mul consuming its output) into stages.
 int lower_linear(mk_graph *g, size_t &i) {
@@ -451,8 +461,7 @@ int lower_linear(mk_graph *g, size_t &i) {
       MkStage &pl = g->stages.back();
       const bool rows_ok = (ns.k & 15) == 0 && ns.k / 8 <= 6 * MK_THREADS && (ns.ld_in & 7) == 0 && (ns.ld_out & 7) == 0 && ((uintptr_t)ns.in & 15) == 0;
       const bool res_ok = !(pl.flags & MK_F_RES) || ((pl.ld_res & 7) == 0 && ((uintptr_t)pl.res & 15) == 0);
-      if (pl.op == MK_OP_LINEAR && !(pl.flags & MK_F_SILU) && pl.out == ns.in && pl.ld_out == ns.ld_in && pl.n == ns.k && rows_ok && res_ok)
-        pl.flags |= MK_F_DEFER_SUM;
+      if (rows_ok && res_ok && pl.n == ns.k) leave_sum(g, ns.in, ns.ld_in, true);
     }
     g->stages.push_back(ns);
     g->stage_desc.push_back(fmt("NORM[multi-token only] %s -> %s k=%d", nx.name.c_str(), no.name.c_str(), st.k));
@@ -686,9 +695,7 @@ int lower_attention(mk_graph *g, size_t &i) {
   }
   if (!g->stages.empty()) {
     // a plain linear whose whole output is this stage's q/k/v rows may leave its split-K sum to this stage's row fetch
-    MkStage &pl = g->stages.back();
-    if (pl.op == MK_OP_LINEAR && !(pl.flags & (MK_F_SILU | MK_F_RES)) && pl.out == st.in && pl.ld_out == st.ld_in && pl.n == (nq + 2 * nkv) * D)
-      pl.flags |= MK_F_DEFER_SUM;
+    if (g->stages.back().n == (nq + 2 * nkv) * D) leave_sum(g, st.in, st.ld_in);
   }
   g->stages.push_back(st);
   g->stage_desc.push_back(fmt("ATTN %s -> %s q=%d kv=%d d=%d norm=%d rope=%d", tin.name.c_str(), to.name.c_str(), nq, nkv, D, !!(st.flags & MK_F_QK_NORM),
@@ -776,9 +783,8 @@ int lower_residual_rmsnorm(mk_graph *g, size_t &i) {
   st.ld_out2 = (int)xo.strides[0];
   if ((st.ld_in | st.ld_res | st.ld_out | st.ld_out2) & 3) return fail(MK_EINVAL, "residual_rmsnorm: row strides must be multiples of 4");
   if (!g->stages.empty()) {
-    MkStage &pl = g->stages.back();
-    if (pl.op == MK_OP_LINEAR && !(pl.flags & (MK_F_SILU | MK_F_RES)) && y && pl.out == st.in && pl.ld_out == st.ld_in && pl.n == st.n && width == n)
-      pl.flags |= MK_F_DEFER_SUM;
+    const MkStage &pl = g->stages.back();
+    if (y && pl.n == st.n && width == n) leave_sum(g, st.in, st.ld_in);
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;
@@ -911,8 +917,8 @@ int lower_flex_attention(mk_graph *g, size_t &i) {
   g->flex_items = std::max(g->flex_items, items);
   g->flex_part = std::max(g->flex_part, (size_t)g->G * 16 * (st.v_tiles * 16 + 32));
   if (!g->stages.empty()) {
-    MkStage &pl = g->stages.back();  // the q/k/v linear may leave its K-slice sum to this stage's row fetch
-    if (pl.op == MK_OP_LINEAR && !(pl.flags & (MK_F_SILU | MK_F_RES)) && pl.out == st.in && pl.ld_out == st.ld_in && pl.n >= cols && !(st.flags & MK_F_ROW_NORM)) pl.flags |= MK_F_DEFER_SUM;
+    // the q/k/v linear may leave its K-slice sum to this stage's row fetch
+    if (g->stages.back().n >= cols && !(st.flags & MK_F_ROW_NORM)) leave_sum(g, st.in, st.ld_in);
   }
   if (B > 1) {
     MkStage sp = st;
@@ -1014,8 +1020,7 @@ int lower_residual_prenorm(mk_graph *g, size_t &i) {
     }
     // a plain linear in front whose whole output is the last summand may leave its split-K sum to this stage (which also stores it)
     const Tensor *ly = y2 ? y2 : y;
-    if (ly && !sw && pl.op == MK_OP_LINEAR && !(pl.flags & (MK_F_SILU | MK_F_RES | MK_F_RELU2)) && pl.out == ly->ptr && pl.ld_out == (int)ly->strides[0] && pl.n == st.n && (pl.ld_out & 3) == 0)
-      pl.flags |= MK_F_DEFER_SUM;
+    if (ly && !sw && pl.n == st.n && (pl.ld_out & 3) == 0 && !(pl.flags & MK_F_RELU2)) leave_sum(g, ly->ptr, ly->strides[0]);
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;

@@ -118,6 +118,31 @@ def test_norm_folded_into_a_single_token_linear(width, n):
     pk.finalize()
 
 
+@pytest.mark.parametrize("n,k", [(2048, 4096), (2056, 4096), (4104, 2048)])
+def test_residual_norm_behind_a_split_linear(n, k):
+    """Whole tiles (the norm stage sums the slices) and a ragged last one (the linear does)."""
+    pk = _graph(64)
+    i, W = torch.randn(64, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") / k ** 0.5).bfloat16()
+    x, w = torch.randn(64, n, device="cuda"), torch.randn(n, device="cuda") * 0.2
+    y, xo, o = torch.zeros(64, n, device="cuda").bfloat16(), torch.zeros(64, n, device="cuda"), torch.zeros(64, n, device="cuda").bfloat16()
+    a = pk.attach_input
+    yy = a(y, "y")
+    pk.linear_layer(a(i, "i"), a(W, "W"), yy, (1, 1, 1), (256, 1, 1))
+    pk.residual_rmsnorm_layer(yy, a(x, "x"), a(w, "w"), a(xo, "xo"), a(o, "o"), alpha=1.6, eps=1e-6, weight_offset=1.0)
+    pk.compile()
+    for M in (64, 33, 5, 1):
+        for t in (y, xo, o):
+            t.zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        s = i[:M].double() @ W.double().T
+        v = 1.6 * x[:M].double() + s
+        f = (1.0 + w.double()) / (v.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt()
+        # a linear that sums its slices rounds to bf16 in front of the norm: half a step is up to 2^-8 of the value (the factor of the row hardly moves)
+        assert bool(((xo[:M].double() - v * f).abs() <= 2.0 ** -8 * (s * f).abs() + 1e-4 * (1.0 + v.abs())).all()), M
+        assert torch.equal(o[:M], xo[:M].bfloat16()) and not xo[M:].any(), M
+    pk.finalize()
+
+
 @pytest.mark.parametrize("k,n,silu", [(64, 33, False), (192, 500, False), (448, 130, True), (2048, 64, True)])
 def test_32_bit_linear(k, n, silu):
     import mirage as mi

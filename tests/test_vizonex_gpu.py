@@ -137,6 +137,11 @@ def test_sum_of_a_split_linear_in_front(n, k, second):
     pk.finalize()
 
 
+@pytest.mark.parametrize("second", [False, True])
+def test_sum_of_a_linear_with_a_ragged_last_tile_in_front(second):
+    test_sum_of_a_split_linear_in_front(2056, 4096, second)
+
+
 class JoinRig:
     """residual_prenorm with two summands, their factors and places, the convolution behind it and (fused) a linear."""
 
