@@ -318,6 +318,12 @@ float bits_f32(int bits) {
 bool rows_ok(const Tensor &t, int B, int64_t cols, int dtype) { return t.ndims == 2 && t.dims[0] >= B && t.dims[1] >= cols && t.dtype == dtype && !(t.strides[0] & 3); }
 bool vector_ok(const Tensor &t, int64_t n) { return t.dtype == MK_DT_F32 && (int64_t)t.elems() >= n; }
 
+// do the pieces of memory that hold rows [0, B) of n columns of two tensors of one type meet?
+bool rows_meet(const Tensor &a, const Tensor &b, int64_t B, int64_t n) {
+  const int64_t d = ((intptr_t)b.ptr - (intptr_t)a.ptr) / (int64_t)dtype_size(a.dtype);
+  return d < (B - 1) * a.strides[0] + n && -d < (B - 1) * b.strides[0] + n;
+}
+
 // a graph holds flex stages of one activation type, and none of the fixed-shape stages next to them (checked after lowering)
 int set_flex(mk_graph *g, int dtype, const char *task) {
   const int kind = dtype == MK_DT_F32 ? FLEX_F32 : FLEX_BF16;
@@ -1020,7 +1026,8 @@ int lower_residual_prenorm(mk_graph *g, size_t &i) {
     }
     // a plain linear in front whose whole output is the last summand may leave its split-K sum to this stage (which also stores it)
     const Tensor *ly = y2 ? y2 : y;
-    if (ly && !sw && pl.n == st.n && (pl.ld_out & 3) == 0 && !(pl.flags & MK_F_RELU2)) leave_sum(g, ly->ptr, ly->strides[0]);
+    // (not when the first summand reads those rows too, before they are there)
+    if (ly && !sw && pl.n == st.n && (pl.ld_out & 3) == 0 && !(pl.flags & MK_F_RELU2) && !(y2 && rows_meet(*y, *y2, B, n))) leave_sum(g, ly->ptr, ly->strides[0]);
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;

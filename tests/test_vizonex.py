@@ -288,3 +288,26 @@ def test_dual_tasks_check_their_operands():
     k.short_conv_layer(new(k, "x2", 8, 64), new(k, "w2", 4, 64, dt=mi.float32), new(k, "b", 64, dt=mi.float32), new(k, "t", 2, 3, 64), sl, new(k, "o2", 8, 64))
     with pytest.raises(Exception, match="cannot run in one graph"):
         k.describe_program()
+
+
+def test_a_sum_that_the_first_summand_reads_is_not_left_to_the_norm():
+    """The second summand may be a split linear's partials; its rows exist only behind the stage, so the first summand must not be among them:
+    neither the same tensor nor rows that overlap it."""
+    import mirage as mi
+    from helpers import make_meta, make_mpk
+    n = 2048
+
+    def leaves(first, second=4):
+        """rows of the two summands in one piece of memory (None: in another)"""
+        pk = make_mpk(make_meta(8, 64, 8, 8, 8, device="cpu"), 64, 8, 8, 8, 64, num_workers=256)
+        new = lambda name, *shape, dtype=mi.bfloat16: pk.new_tensor(shape, dtype=dtype, name=name)
+        row, vec = (lambda name: new(name, 8, n, dtype=mi.float32)), (lambda name: new(name, n, dtype=mi.float32))
+        memory = torch.zeros(16, n, dtype=torch.bfloat16)
+        y = pk.attach_input(memory[second:second + 8], "y")
+        y1 = new("y1", 8, n) if first is None else y if first == second else pk.attach_input(memory[first:first + 8], "y1")
+        pk.linear_layer(new("x", 8, 4096), new("w", n, 4096), y, (1, 1, 1), (256, 1, 1))
+        pk.residual_prenorm_layer(y1, row("r"), row("s"), new("h", 8, n), weight=vec("g"), factor=vec("a"), input2=y, factor2=vec("b"))
+        return "sum=next" in [l for l in pk.describe_program().splitlines() if " LINEAR" in l][0]
+
+    assert leaves(None) and leaves(0, 8) and leaves(8, 0)
+    assert not leaves(4) and not leaves(1) and not leaves(8)

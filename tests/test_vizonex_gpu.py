@@ -142,6 +142,28 @@ def test_sum_of_a_linear_with_a_ragged_last_tile_in_front(second):
     test_sum_of_a_split_linear_in_front(2056, 4096, second)
 
 
+@pytest.mark.parametrize("n,k", [(2048, 4096), (4096, 2048)])
+def test_sum_of_a_split_linear_that_is_both_summands(n, k):
+    g = torch.Generator().manual_seed(n + k)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    pk, _ = _graph(64, 64)
+    b16 = lambda t: t.to(torch.bfloat16).cuda()
+    t = dict(i=b16(rnd(64, k)), wl=b16(rnd(n, k) / k ** 0.5), x=rnd(64, n).cuda(), s1=(1 + 0.3 * rnd(n)).cuda(), s2=(1 + 0.3 * rnd(n)).cuda(), w=(1 + 0.3 * rnd(n)).cuda(),
+             lo=b16(torch.zeros(64, n)), nx=torch.zeros(64, n, device="cuda"), h=b16(torch.zeros(64, n)))
+    a = {q: pk.attach_input(v, q) for q, v in t.items()}
+    pk.linear_layer(a["i"], a["wl"], a["lo"], (1, 1, 1), (256, 1, 1))
+    pk.residual_prenorm_layer(a["lo"], a["x"], a["nx"], a["h"], weight=a["w"], width=n, eps=1e-4, factor=a["s1"], input2=a["lo"], factor2=a["s2"])
+    pk.compile()
+    d = {q: v.double().cpu() for q, v in t.items()}
+    for M in (64, 17, 1):
+        t["lo"].zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        lo, nx = (t[q][:M].cpu().double() for q in ("lo", "nx"))
+        torch.testing.assert_close(lo, (d["i"] @ d["wl"].T)[:M], **_tol(torch.bfloat16))
+        torch.testing.assert_close(nx, d["x"][:M] + (d["s1"] + d["s2"]) * lo, rtol=1e-6, atol=4e-6)  # (four roundings of 2^-24 of values below 16)
+    pk.finalize()
+
+
 class JoinRig:
     """residual_prenorm with two summands, their factors and places, the convolution behind it and (fused) a linear."""
 
