@@ -636,6 +636,7 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
     for (int i = tid; i < Ex * (MK_MAX_TOKENS / 8); i += MK_THREADS) ls->place[0][i] = 0u;
   }
   if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  if (!c.pending) __syncthreads();  // (an iteration's first stage has no barrier to wait for: everybody is done clearing)
   barrier_wait(c);
   // ---- which experts have which tokens
   if (rows_in) {

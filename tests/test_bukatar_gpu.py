@@ -385,6 +385,36 @@ def test_experts_long_reductions(dtype, rows, E, top, ff, shared, width):
     test_experts_alone(dtype, rows, E, top, ff, shared, width)
 
 
+def _expert_rig(dtype, E, top, n, k, ids, width=None):
+    """One expert linear over the caller's ids, the only stage of its graph: the caller's tensors and weights."""
+    from mirage.mpk.persistent_kernel import expert_tiles
+    g = torch.Generator().manual_seed(E + n)
+    w, x = (torch.randn(E, n, k, generator=g) / k ** 0.5).to(dtype), torch.randn(64, k, generator=g).to(dtype)
+    t = dict(x=x.cuda(), w=expert_tiles(w.cuda()), ids=torch.zeros(64, top, dtype=torch.int32, device="cuda"), o=torch.zeros(64, width or top * n, dtype=dtype, device="cuda"))
+    t["ids"][:len(ids)] = ids.to(torch.int32).cuda()
+    pk, _ = _graph(64, 64)
+    a = {q: pk.attach_input(v, q) for q, v in t.items()}
+    pk.expert_linear_layer(a["x"], a["w"], a["ids"], a["o"], E, top, n, k, n)
+    pk.compile()
+    return pk, t, x.double(), w.double()
+
+
+@BOTH
+@pytest.mark.parametrize("E,top,n,k", [(256, 8, 32, 64), (7, 3, 64, 192)])
+def test_experts_the_caller_chose_in_the_first_stage(dtype, E, top, n, k):
+    """No stage in front: the lists are filled behind nothing but the workgroup's own barrier."""
+    g = torch.Generator().manual_seed(E)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(64)])
+    pk, t, x, w = _expert_rig(dtype, E, top, n, k, ids)
+    for M in (64, 5, 2, 1, 33):
+        t["o"].zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        want = torch.einsum("tsnk,tk->tsn", w[ids[:M]], x[:M])
+        torch.testing.assert_close(t["o"][:M].cpu().double().view(M, top, n), want, **_tol(dtype))
+        assert not t["o"][M:].any()
+    pk.finalize()
+
+
 # ---------------------------------------------------------------- whole models
 @BOTH
 @pytest.mark.parametrize("name", ["even", "odd", "wide"])
