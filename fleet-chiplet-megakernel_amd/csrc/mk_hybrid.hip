@@ -675,9 +675,10 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
       }
     } else {
       for (int i = tid; i < M * topk; i += MK_THREADS) {
+        // (an expert that a token names twice -- the caller's ids may, and so may a routing over NaN -- has the place that came first: places
+        // put together would lie outside the token's row)
         const int t = i / topk, id = ldc_i32(st.ids + i);
-        atomicOr(&ls->tok[id], 1ull << t);
-        atomicOr(&ls->place[id][t >> 3], (unsigned)(i - t * topk) << ((t & 7) * 4));
+        if (!(atomicOr(&ls->tok[id], 1ull << t) >> t & 1)) atomicOr(&ls->place[id][t >> 3], (unsigned)(i - t * topk) << ((t & 7) * 4));
       }
     }
     __syncthreads();

@@ -415,6 +415,27 @@ def test_experts_the_caller_chose_in_the_first_stage(dtype, E, top, n, k):
     pk.finalize()
 
 
+@BOTH
+def test_an_expert_named_twice_stays_in_its_tokens_row(dtype):
+    """One of the places that name it gets the expert's output; nothing is written outside the token's places."""
+    E, top, n, k = 12, 6, 32, 64
+    ids = torch.tensor([[0, 0, 0, 0, 0, 0], [3, 1, 1, 4, 5, 6], [7, 8, 9, 2, 10, 2], [5, 4, 3, 2, 1, 0]]).repeat(16, 1)
+    pk, t, x, w = _expert_rig(dtype, E, top, n, k, ids, width=16 * n)
+    for M in (64, 3, 2, 1):
+        t["o"].fill_(7.0)
+        pk.run_once(list(range(M)), [0] * M)
+        o = t["o"].cpu().double().view(64, 16, n)
+        assert (o[:, top:] == 7).all() and (o[M:] == 7).all()
+        want = torch.einsum("tsnk,tk->tsn", w[ids[:M]], x[:M])
+        tol = _tol(dtype)
+        right = ((o[:M, :top] - want).abs() <= tol["atol"] + tol["rtol"] * want.abs()).all(-1)
+        for q in range(M):
+            for e in ids[q].unique():
+                places = (ids[q] == e).nonzero().flatten()
+                assert right[q, places].any() and all(right[q, p] or (o[q, p] == 7).all() for p in places.tolist()), (M, q, int(e))
+    pk.finalize()
+
+
 # ---------------------------------------------------------------- whole models
 @BOTH
 @pytest.mark.parametrize("name", ["even", "odd", "wide"])
