@@ -58,14 +58,15 @@ __device__ __forceinline__ void mx_summands(CStage &st, const E *y, const float 
   for (int j = 0; j < NS; j++) v[j] = fx_ldc_quad(y + 4 * at(j));
 }
 // ... of a linear that left its K-slice partials to the norm stage: summed in slice order, rounded as that linear would have and stored
-// where it would have.  All slices of four quads are requested at once.  The linear's own exchange of slices, by its last arriver, costs more:
+// where it would have.  All slices of a group of quads, up to sixteen requests, are under way at once.  The linear's own exchange of slices, by its last arriver, costs more:
 // 4096 x 16384 at 8 tokens 30.6 -> 28.3 us as a stage, the norm 7.9 -> 8.0; dodonex serving of 8 60.2 -> 59.7 ms, vizonex at 64 streams 84.7 -> 83.8.
 template <typename E, int NS, typename At>
 __device__ __forceinline__ void mx_deferred(const Ctx &c, int dS, E *row, int t, int n4, f32x4 (&v)[NS], At at) {
   const float *p = c.defer_part + (size_t)t * c.defer_n;
   const size_t slice = (size_t)c.defer_rows * c.defer_n;
   auto sum = [&](auto ns) {
-    constexpr int Q = decltype(ns)::value, JB = NS * Q <= 16 ? NS : 16 / Q;
+    constexpr int Q = decltype(ns)::value, JB = NS * Q <= 16 ? NS : NS % (16 / Q) == 0 ? 16 / Q : 12 / Q;  // quads requested together
+    static_assert(JB >= 1 && NS % JB == 0, "whole groups of quads");
 #pragma unroll
     for (int j0 = 0; j0 < NS; j0 += JB) {
       f32x4 q[JB][Q];
