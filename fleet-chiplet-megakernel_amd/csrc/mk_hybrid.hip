@@ -218,7 +218,7 @@ __device__ __forceinline__ void stage_hy_scan_t(CStage &st, Ctx &c, const MkRunt
       if (!real(a, h)) continue;
 #pragma unroll
       for (int i = 0; i < Q; i++)
-        if (on[i]) mx_stc_quad(state_of(a, h) + at[i], S[h][i]);
+        if (on[i]) fx_stc_quad(state_of(a, h) + at[i], S[h][i]);
     }
     if (keep <= L) {
 #pragma unroll

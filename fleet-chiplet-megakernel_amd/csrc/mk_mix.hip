@@ -21,11 +21,6 @@ __device__ __forceinline__ float mx_sigmoid(float, float z) { return 1.f / (1.f 
 __device__ __forceinline__ float mx_tanh(uint16_t, float z) { return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.8853900817779268f * z)); }
 __device__ __forceinline__ float mx_tanh(float, float z) { return tanhf(z); }
 
-// A quad of 32-bit values written through to memory in one store (the same visibility as stc_f32).
-__device__ __forceinline__ void mx_stc_quad(float *p, f32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"((const MK_GLOBAL void *)(unsigned long long)p), "v"(v) : "memory");
-}
-
 // Values of a norm stage's summand: this thread's NS quads of row `y`, at(j) the index of quad j.  Hybrid kernels: with `places` the sum of
 // st.slots rows of the token, st.ld_slot apart, weighted by `w`; the quads of SQ rows are requested at once.  (A bias is added by the caller, who has
 // it in advance.)
@@ -1292,7 +1287,7 @@ __device__ __forceinline__ void stage_mx_latent_attn_t(CStage &st, Ctx &c, const
           float *o = (float *)rt.attn_part + ((size_t)u * 16 * RT + r) * PST;
 #pragma unroll
           for (int j = 0; j < VBW; j++)
-            if (wave + MK_WAVES * j < nvb) mx_stc_quad(o + (wave + MK_WAVES * j) * 16 + lg * 4, acc[q][j]);
+            if (wave + MK_WAVES * j < nvb) fx_stc_quad(o + (wave + MK_WAVES * j) * 16 + lg * 4, acc[q][j]);
           if (wave == 0 && lg == 0) {
             stc_f32(o + Rp, m[q]);
             stc_f32(o + Rp + 1, Lr);
@@ -1429,7 +1424,7 @@ __device__ __forceinline__ void mx_delta_store(const f32x4 (&S)[NC][NI], float *
   for (int j = 0; j < NC; j++)
 #pragma unroll
     for (int i = 0; i < NI; i++)
-      if (col + j < Dp && i * 64 + lr * 4 < Dp) mx_stc_quad(state + (size_t)(col + j) * Dp + i * 64 + lr * 4, S[j][i]);
+      if (col + j < Dp && i * 64 + lr * 4 < Dp) fx_stc_quad(state + (size_t)(col + j) * Dp + i * 64 + lr * 4, S[j][i]);
 }
 template <int NI> struct MxDeltaVec {
   f32x4 r[NI], k[NI], u[NI], au[NI], w[NI];

@@ -610,3 +610,12 @@ int main() {
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", inc, str(src), "-o", str(exe)], check=True)
     res = subprocess.run([str(exe)], capture_output=True, text=True)
     assert res.returncode == 0 and res.stdout.strip() == "0", res.stdout
+
+
+def test_wide_stores_in_assembly_wait_for_their_registers():
+    """The instruction behind a store of more than eight bytes must not write the registers it still reads; the compiler does not look into
+    assembly for that, so the wait state belongs to the store's own text."""
+    csrc = os.path.join(ROOT, "fleet-chiplet-megakernel_amd", "csrc")
+    text = "".join(open(os.path.join(csrc, f)).read() for f in sorted(os.listdir(csrc)) if f.endswith((".hip", ".h", ".cpp")))
+    stores = re.findall(r'"[^"]*_store_dwordx[34][^"]*"', text)
+    assert stores and all("s_nop" in s for s in stores), stores
