@@ -3944,9 +3944,9 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 // cached positions 85 -> 31 us, behind 2432 127 -> 43; 64 streams of one token 33 -> 30.
 //
 // Tile: scores with A = K (lane (i, g): row of position i, dims 32 s + 8 g .. of step s) and B = q (lane (j, g): column j, same dims)
-// -> lane (j, g) holds column j at positions 4 g .. 4 g + 3.  Those four weights, as bf16 (value and rounding remainder: two operands),
-// are already the A operand of a 16x16x16 step over positions; its B operand -- four consecutive positions of one dim -- is read out of
-// the V tile in LDS.  The running maximum is kept per column for the whole wavefront, the running sum per lane.
+// -> lane (j, g) holds column j at positions 4 g .. 4 g + 3.  Those four weights are already the A operand of a 16x16x16 step over
+// positions, in bf16 terms: cached positions as value and rounding remainder (two operands, 16 bits of a weight), new ones, of which there
+// are few tiles, with all of their 24 bits (three).  The B operand -- four consecutive positions of one dim -- is read out of the V tile in LDS.  The running maximum is kept per column for the whole wavefront, the running sum per lane.
 // K and V tiles are four groups of four rows of 256 bytes, one direct-to-LDS request per group (each lane 16 bytes: four whole rows), the
 // groups GS bytes apart (the transposed V reads of the four groups then fall into different banks).
 template <int QPK>
@@ -4095,7 +4095,8 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     for (int dt = 0; dt < 8; dt++) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float mrun = -INFINITY, lsum = 0.f;
     // positions [q0, q0 + 16) whose rows lie at kb / vb; this lane's column sees those up to `last` (at least one of them)
-    auto compute_tile = [&](int q0, int last, const char *kb, const char *vb) {
+    auto compute_tile = [&](int q0, int last, const char *kb, const char *vb, auto fresh) {
+      constexpr bool NEW = decltype(fresh)::value;
       f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
       const char *kl = kb + (lr >> 2) * GS + (lr & 3) * 256 + lg * 16;
 #pragma unroll
@@ -4122,21 +4123,26 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
 #pragma unroll
           for (int r = 0; r < 4; r++) o[dt][r] *= ar[r];
       }
-      float ph[4];
+      constexpr int NP = NEW ? 3 : 2;
+      s16x4 wt[NP];
 #pragma unroll
-      for (int r = 0; r < 4; r++) ph[r] = bfround(pw[r]);
-      const unsigned h01 = pack2(ph[0], ph[1]), h23 = pack2(ph[2], ph[3]);
-      const unsigned l01 = pack2(pw[0] - ph[0], pw[1] - ph[1]), l23 = pack2(pw[2] - ph[2], pw[3] - ph[3]);
-      const s16x4 a_hi = __builtin_bit_cast(s16x4, (unsigned long long)h01 | ((unsigned long long)h23 << 32));
-      const s16x4 a_lo = __builtin_bit_cast(s16x4, (unsigned long long)l01 | ((unsigned long long)l23 << 32));
+      for (int q = 0; q < NP; q++) {
+        float ph[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          ph[r] = bfround(pw[r]);
+          pw[r] -= ph[r];  // (exact)
+        }
+        wt[q] = __builtin_bit_cast(s16x4, (unsigned long long)pack2(ph[0], ph[1]) | ((unsigned long long)pack2(ph[2], ph[3]) << 32));
+      }
       const char *vl = vb + lg * GS + lr * 2;
 #pragma unroll
       for (int dt = 0; dt < 8; dt++) {
         const char *q_ = vl + dt * 32;
         const unsigned v0 = *(const uint16_t *)(q_), v1 = *(const uint16_t *)(q_ + 256), v2 = *(const uint16_t *)(q_ + 512), v3 = *(const uint16_t *)(q_ + 768);
         const s16x4 bv = __builtin_bit_cast(s16x4, (unsigned long long)(v0 | (v1 << 16)) | ((unsigned long long)(v2 | (v3 << 16)) << 32));
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_hi, bv, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_lo, bv, o[dt], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NP; q++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wt[q], bv, o[dt], 0, 0, 0);
       }
     };
     // cached tiles: RB in flight per wavefront; every request is issued unconditionally, and the wait before a tile counts the
@@ -4152,7 +4158,7 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
           static_assert(RB == 2, "the wait counts one tile's requests");
           asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
           if (more) {
-            compute_tile((a.tb + t_) * 16, cend - 1, buf + b_ * SLOT + TS, buf + b_ * SLOT);
+            compute_tile((a.tb + t_) * 16, cend - 1, buf + b_ * SLOT + TS, buf + b_ * SLOT, std::false_type{});
             t_ += MK_WAVES;
             more = t_ < nt;
           }
@@ -4161,7 +4167,7 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     }
     // new tiles: all tokens of a group lie in the last of them (groups begin at multiples of TG in their request, TG divides 16)
     const int p_col = p_first + min(lr, n_cols - 1) / QPK;
-    for (int k = wave; k * 16 < a.n_new; k += MK_WAVES) compute_tile(a.p0 + k * 16, p_col, knew + k * TS, vnew + k * TS);
+    for (int k = wave; k * 16 < a.n_new; k += MK_WAVES) compute_tile(a.p0 + k * 16, p_col, knew + k * TS, vnew + k * TS, std::true_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the direct-to-LDS requests of the tile that was not computed)
     // the chunk with the new rows appends the group's own K/V rows and publishes its queries
     if (a.n_new) {

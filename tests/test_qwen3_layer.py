@@ -139,6 +139,29 @@ def test_portions_in_units_of_several_tokens(nkv, L_cached, n_new):
     assert frac < 0.05 and u <= 1.0, f"attention: {frac:.4f} differ, max {u} ulp"
 
 
+@pytest.mark.parametrize("nkv", [8, 4])
+def test_weights_of_new_positions_have_32_bits(nkv):
+    """Where values all but cancel, an output shows the precision of the softmax weights behind its own rounding."""
+    from oracle.qwen3_ref import Qwen3Config
+    n, nq, D = 64, 32, 128
+    cfg = Qwen3Config(hidden_size=1024, num_q_heads=nq, num_kv_heads=nkv, head_dim=D, intermediate_size=1536, num_layers=1)
+    worst = 0.0
+    for seed in range(4):
+        res = _run_layer(cfg, 0, n, "fleet", seed=900 + seed)
+        at = torch.arange(n)
+        page, row = torch.tensor(res["pages"])[at // res["page_size"]], at % res["page_size"]
+        head = torch.arange(nq) // (nq // nkv)
+        k, v = (res[t][page, row].view(n, nkv, D)[:, head].double() for t in ("k_after", "v_after"))
+        q = res["qws_gpu"].view(n, nq, D).double()
+        p = torch.softmax((torch.matmul(q.transpose(0, 1), k.permute(1, 2, 0)) / D ** 0.5).masked_fill(at[None, None] > at[None, :, None], -torch.inf), -1)
+        want = torch.matmul(p, v.transpose(0, 1)).transpose(0, 1)
+        scale = torch.matmul(p.pow(2), v.transpose(0, 1).pow(2)).sqrt().transpose(0, 1)
+        err = (res["attn_gpu"].view(n, nq, D).double() - want).abs() - 2.0 ** -8 * want.abs()  # (half a bf16 step)
+        worst = max(worst, float((err / scale).max()))
+    # a score is a 32-bit sum of 128 products of order one: its error, and with it a weight's, is a few times 2^-23; bf16 in two terms has 2^-18
+    assert worst < 2.0 ** -20, worst * 2.0 ** 20
+
+
 def test_full_width_layer_prefill_chunk_mpk_mode():
     from oracle.qwen3_ref import Qwen3Config
     cfg = Qwen3Config(num_layers=1)
