@@ -4123,6 +4123,36 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
 #pragma unroll
           for (int r = 0; r < 4; r++) o[dt][r] *= ar[r];
       }
+      const char *vl = vb + lg * GS + lr * 2;
+      if constexpr (NEW) {
+        // Positions that only some of the columns see have weight zero in the others, which a product over the tile takes for a value that
+        // is not finite too: such a tile is summed column by column.
+        unsigned top = 0;
+        if (a.n > 1 && q0 + 16 > p_first) {
+#pragma unroll
+          for (int dt = 0; dt < 8; dt++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) top |= (*(const uint16_t *)(vl + dt * 32 + e * 256) & 0x7f80u) + 0x80u;
+          }
+        }
+        if (__builtin_expect(__ballot(top & 0x8000u) != 0, 0)) {
+          for (int g = 0; g < 4; g++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const uint16_t *v = (const uint16_t *)(vb + g * GS + e * 256) + lr;
+#pragma unroll
+              for (int r = 0; r < 4; r++) {
+                const int col = lg * 4 + r;
+                const float w = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((g * 16 + col) << 2, __builtin_bit_cast(int, pw[e])));
+                const bool seen = q0 + g * 4 + e <= p_first + min(col, n_cols - 1) / QPK;
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) o[dt][r] = seen ? fmaf(w, bf2f(v[dt * 16]), o[dt][r]) : o[dt][r];
+              }
+            }
+          }
+          return;
+        }
+      }
       constexpr int NP = NEW ? 3 : 2;
       s16x4 wt[NP];
 #pragma unroll
@@ -4135,7 +4165,6 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
         }
         wt[q] = __builtin_bit_cast(s16x4, (unsigned long long)pack2(ph[0], ph[1]) | ((unsigned long long)pack2(ph[2], ph[3]) << 32));
       }
-      const char *vl = vb + lg * GS + lr * 2;
 #pragma unroll
       for (int dt = 0; dt < 8; dt++) {
         const char *q_ = vl + dt * 32;

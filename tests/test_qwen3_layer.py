@@ -8,7 +8,7 @@ from helpers import check_layer_stages as _check
 pytestmark = pytest.mark.gpu
 
 
-def _run_layer(cfg, L_cached, n_new, mode, seed=0, norm_std=0.02, mutate=None, batch_tokens=None, single_weight_copy=None):
+def _run_layer(cfg, L_cached, n_new, mode, seed=0, norm_std=0.02, mutate=None, batch_tokens=None, single_weight_copy=None, row=None):
     """One request with L_cached positions already in the KV cache and n_new new tokens in this pass."""
     from demo_qwen3 import Qwen3Decoder, Qwen3Shape
     from oracle.qwen3_ref import KVCache, Qwen3Oracle, make_layer_weights, rope_tables
@@ -17,6 +17,8 @@ def _run_layer(cfg, L_cached, n_new, mode, seed=0, norm_std=0.02, mutate=None, b
     if mutate is not None:
         mutate(lw)
     hidden = torch.randn(n_new, cfg.hidden_size, generator=g).to(torch.bfloat16)
+    if row is not None:
+        hidden[row[0]] = row[1]
     max_seq = L_cached + n_new + 8
     cache = KVCache(cfg, max_seq)
     cache.k[0, :L_cached] = torch.randn(L_cached, cfg.num_kv_heads, cfg.head_dim, generator=g).to(torch.bfloat16)
@@ -160,6 +162,19 @@ def test_weights_of_new_positions_have_32_bits(nkv):
         worst = max(worst, float((err / scale).max()))
     # a score is a 32-bit sum of 128 products of order one: its error, and with it a weight's, is a few times 2^-23; bf16 in two terms has 2^-18
     assert worst < 2.0 ** -20, worst * 2.0 ** 20
+
+
+@pytest.mark.parametrize("nkv", [8, 4])
+@pytest.mark.parametrize("L_cached,at", [(0, 1), (0, 39), (130, 62), (16, 35)])
+def test_a_token_that_is_not_finite_leaves_those_before_it_alone(nkv, L_cached, at):
+    """Its keys and values are NaN; tokens in front of it, of its own unit among them, come out as they do without it, those behind it do not."""
+    from oracle.qwen3_ref import Qwen3Config
+    cfg = Qwen3Config(hidden_size=1024, num_q_heads=32, num_kv_heads=nkv, head_dim=128, intermediate_size=1536, num_layers=1)
+    clean, res = (_run_layer(cfg, L_cached, 64, "fleet", seed=7, row=r) for r in (None, (at, float("nan"))))
+    a, b = (r["attn_gpu"].view(64, 32, 128).float() for r in (clean, res))
+    assert not a.isnan().any() and not b[:at].isnan().any() and b[at:].isnan().all()
+    # (tokens whose unit holds it are summed another way, in 32 bits: one bf16 step)
+    assert float(((b[:at] - a[:at]).abs() / a[:at].abs().clamp_min(1.0 / 16)).max()) <= 2.0 ** -7
 
 
 def test_full_width_layer_prefill_chunk_mpk_mode():
