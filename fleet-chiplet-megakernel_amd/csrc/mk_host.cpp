@@ -152,6 +152,13 @@ __global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, Launch
 }
 static_assert(sizeof(MkSched) % 4 == 0 && sizeof(MkSched) / 4 <= 192 && sizeof(MkSync) % 4 == 0, "copied word by word");
 
+// Launches report their own status: the thread's last error may be one that an earlier call of somebody else left.
+template <typename... P>
+static hipError_t launch_kernel(void (*kernel)(P...), unsigned grid, unsigned block, hipStream_t stream, P... params) {
+  void *args[] = {(void *)&params...};
+  return hipLaunchKernel((const void *)kernel, dim3(grid), dim3(block), args, 0, stream);
+}
+
 struct mk_graph {
   mk_config cfg;
   int num_cus = 0;
@@ -2718,8 +2725,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   g->launch_pending = true;
   g->launch_stream = stream;
   g->ms_due = true;
-  hipLaunchKernelGGL(mk_launch_done_kernel, dim3(1), dim3(256), 0, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status);
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status));
   return MK_OK;
 }
 
@@ -3059,8 +3065,7 @@ static int pack_weights(mk_graph *g, bool allocate) {
       g->packed_bytes += total * 16;
     }
     if (!st.wpack) continue;
-    hipLaunchKernelGGL(mk_pack_weights_kernel, dim3(2048), dim3(256), 0, 0, st.w, st.n, st.k, silu ? 1 : 0, st.silu_half, (u32x4 *)st.wpack, total);
-    HIP_TRY(hipGetLastError());
+    HIP_TRY(launch_kernel(mk_pack_weights_kernel, 2048, 256, 0, st.w, st.n, st.k, silu ? 1 : 0, st.silu_half, (u32x4 *)st.wpack, total));
   }
   HIP_TRY(hipDeviceSynchronize());
   return 0;
@@ -3326,8 +3331,7 @@ int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations) {
   rt.stage_prof = nullptr;  // per-stage timing is library-allocated scratch too: not recorded by this entry point
   rt.timing = nullptr;
   // the array keeps what the previous call left: barrier state and arrival counters must start at zero
-  hipLaunchKernelGGL(mk_fill_zero_kernel, dim3(16), dim3(256), 0, (hipStream_t)stream, (uint4 *)base, SS_CLEARED_END / 16);
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(launch_kernel(mk_fill_zero_kernel, 16, 256, (hipStream_t)stream, (uint4 *)base, (size_t)(SS_CLEARED_END / 16)));
   const int sched = g->cfg.mode == MK_MODE_OFFLINE ? MK_SCHED_OFFLINE : (g->cfg.mode == MK_MODE_ONLINE ? MK_SCHED_ONLINE : MK_SCHED_FROM_META);
   return do_launch(g, (hipStream_t)stream, sched == MK_SCHED_FROM_META ? 1 : max_iterations, sched, &rt);
 }

@@ -137,3 +137,41 @@ def test_attention_closed_forms(L_cached, n_new, width):
                 ulp, mabs = bf16_ulp_diff(attn[t, :, j], want.to(torch.bfloat16), floor=1.0 / 16)
                 assert ulp <= 1.0, f"token {t} q head {j}: mean of {L} V rows off by {ulp} ulp ({mabs})"
     assert res["stats"]["aborted"] == 0
+
+
+def _hip():
+    """The HIP runtime this process has loaded."""
+    import ctypes
+    paths = sorted({l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64.so" in l})
+    assert len(paths) == 1, paths
+    return ctypes.CDLL(paths[0])
+
+
+def _linear_graph(tokens=16, mode="onepass", n=256, k=512):
+    from helpers import make_meta, make_mpk
+    x, w, y = (torch.randn(s, device="cuda").bfloat16() for s in ((tokens, k), (n, k), (tokens, n)))
+    pk = make_mpk(make_meta(tokens, 64, tokens, tokens, tokens), 64, tokens, tokens, tokens, 64, mode=mode)
+    pk.linear_layer(pk.attach_input(x, "x"), pk.attach_input(w, "w"), pk.attach_input(y, "y"), (1, 1, 1), (256, 1, 1))
+    return pk, x, w, y
+
+
+def test_launches_report_their_own_status_only():
+    """An error that somebody's earlier call left in this thread is neither theirs nor a reason to fail."""
+    import ctypes
+    from mirage import _capi
+    hip, lib, stream = _hip(), _capi.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    pk, x, w, y = _linear_graph()
+    torch.cuda.synchronize()
+    try:
+        assert hip.hipSetDevice(1 << 20) != 0 and hip.hipPeekAtLastError() != 0
+        pk.compile()
+        pk.run_once(list(range(16)), [0] * 16)
+        pk.run_once(list(range(3)), [0] * 3)
+        for enqueue in (lib.mk_enqueue_steps, lib.mk_enqueue_steps_static):
+            _capi.check(enqueue(pk._handle, stream, 1))
+            _capi.check(lib.mk_wait(pk._handle, stream, None))
+    finally:
+        hip.hipGetLastError()
+    torch.testing.assert_close(y.double(), x.double() @ w.double().T, rtol=2.0 ** -7, atol=1e-3 * 512 ** 0.5)
+    assert pk.stats()["aborted"] == 0
+    pk.finalize()
