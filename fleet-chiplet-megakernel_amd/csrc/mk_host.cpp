@@ -2732,7 +2732,10 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
 int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   if (!g->launch_pending) return fail(MK_ESTATE, "no launch pending");
   HIP_TRY(hipStreamSynchronize(stream));
-  if (stream != g->launch_stream) HIP_TRY(hipStreamSynchronize(g->launch_stream));
+  if (stream != g->launch_stream) {  // (which may be gone by now)
+    HIP_TRY(hipSetDevice(g->cfg.device));
+    HIP_TRY(hipDeviceSynchronize());
+  }
   g->launch_pending = false;
   const LaunchStatus &hs = *g->h_status;
   int nx = 0;

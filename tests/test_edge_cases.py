@@ -175,3 +175,32 @@ def test_launches_report_their_own_status_only():
     torch.testing.assert_close(y.double(), x.double() @ w.double().T, rtol=2.0 ** -7, atol=1e-3 * 512 ** 0.5)
     assert pk.stats()["aborted"] == 0
     pk.finalize()
+
+
+def test_waiting_on_another_stream_than_the_launch():
+    """The launch's own stream is still at work, or has been destroyed since."""
+    import ctypes
+    from mirage import _capi
+    hip, lib, null = _hip(), _capi.load(), ctypes.c_void_p(0)
+    pk, x, w, y = _linear_graph()
+    pk.compile()
+    meta = pk.meta_tensors
+    meta["qo_indptr_buffer"].copy_(torch.arange(17, dtype=torch.int32))
+    meta["paged_kv_indptr_buffer"].copy_(torch.arange(17, dtype=torch.int32))
+    meta["paged_kv_indices_buffer"].copy_(torch.arange(16, dtype=torch.int32))
+    meta["paged_kv_last_page_len_buffer"].fill_(1)
+    want = x.double() @ w.double().T
+    for destroy in (False, True):
+        y.zero_()
+        torch.cuda.synchronize()
+        s = ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0  # (does not wait for the null stream, nor that for it)
+        _capi.check(lib.mk_enqueue_steps(pk._handle, s, 1))
+        if destroy:
+            assert hip.hipStreamSynchronize(s) == 0 and hip.hipStreamDestroy(s) == 0
+        _capi.check(lib.mk_wait(pk._handle, null, None))
+        torch.testing.assert_close(y.double(), want, rtol=2.0 ** -7, atol=1e-3 * 512 ** 0.5)
+        assert pk.stats()["aborted"] == 0 and pk.stats()["num_xcds"] > 0 and pk.stats()["last_launch_ms"] > 0
+        if not destroy:
+            assert hip.hipStreamDestroy(s) == 0
+    pk.finalize()
