@@ -177,18 +177,50 @@ def test_launches_report_their_own_status_only():
     pk.finalize()
 
 
-def test_waiting_on_another_stream_than_the_launch():
-    """The launch's own stream is still at work, or has been destroyed since."""
-    import ctypes
-    from mirage import _capi
-    hip, lib, null = _hip(), _capi.load(), ctypes.c_void_p(0)
-    pk, x, w, y = _linear_graph()
+def _sixteen_single_tokens(pk):
     pk.compile()
     meta = pk.meta_tensors
     meta["qo_indptr_buffer"].copy_(torch.arange(17, dtype=torch.int32))
     meta["paged_kv_indptr_buffer"].copy_(torch.arange(17, dtype=torch.int32))
     meta["paged_kv_indices_buffer"].copy_(torch.arange(16, dtype=torch.int32))
     meta["paged_kv_last_page_len_buffer"].fill_(1)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("entry", ["mk_enqueue_steps_static", "mk_enqueue_steps"])
+def test_a_captured_launch(entry):
+    """The first launch of a handle goes into a graph: its replays, among launches of their own, give what those give; statistics can be read."""
+    import ctypes
+    from mirage import _capi
+    lib = _capi.load()
+    pk, x, w, y = _linear_graph()
+    _sixteen_single_tokens(pk)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _capi.check(getattr(lib, entry)(pk._handle, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), 1))
+    _capi.check(lib.mk_wait(pk._handle, ctypes.c_void_p(0), None))
+    assert pk.stats()["aborted"] == 0
+    for i in range(4):
+        x.normal_()
+        got = []
+        for launch in (graph.replay, lambda: pk.run_steps(1)):
+            y.zero_()
+            launch()
+            torch.cuda.synchronize()
+            got.append(y.clone())
+        assert torch.equal(*got), i
+        torch.testing.assert_close(got[0].double(), x.double() @ w.double().T, rtol=2.0 ** -7, atol=1e-3 * 512 ** 0.5)
+    assert pk.stats()["aborted"] == 0 and pk.stats()["last_launch_ms"] > 0
+    pk.finalize()
+
+
+def test_waiting_on_another_stream_than_the_launch():
+    """The launch's own stream is still at work, or has been destroyed since."""
+    import ctypes
+    from mirage import _capi
+    hip, lib, null = _hip(), _capi.load(), ctypes.c_void_p(0)
+    pk, x, w, y = _linear_graph()
+    _sixteen_single_tokens(pk)
     want = x.double() @ w.double().T
     for destroy in (False, True):
         y.zero_()
