@@ -135,114 +135,96 @@ __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRunti
 // v = alpha * x + y;  out2 = v / sqrt(mean(v^2) + eps) * (w_offset + w) in 32 bits, out = the same rounded to E.  Rows are
 // st.n long with st.k of them real (the rest is zero in every operand).  x (st.res) is 32-bit, y (st.in, null: none) is the
 // preceding linear's output, or its K-slice partials when that linear left its sum to this stage.  A workgroup per row.
-// Rows of up to 4096 values, four quads per thread.  Bound by the barrier and one round trip for the row: the slices of all quads are
-// requested before the first value is waited for (a branch around each quad had made a round trip per quad of it).
-// 4096 values from four slices, as a stage: 8.9 -> 6.7 us at 4 rows, 9.5 -> 7.1 at 64; now 3.6 and 4.2.
+// Bound by the barrier and one round trip for the row: weights and residual are requested ahead of the barrier and all quads of a thread (four,
+// eight or twelve) before the first value is waited for, the slices of four quads at a time; a branch around each quad had made a round trip
+// per quad of it, and rows of more than 4096 values that waited in LDS for their factor a round trip per 4096.  As a stage, us, 4 / 64 rows:
+// 4096 values from four slices 8.9 -> 3.6 / 9.5 -> 4.2; of a 32-bit summand 8192 values 5.1 (by LDS 5.7) -> 3.5 / 5.6 (6.6) -> 4.3, 12,288 values
+// 6.1 (7.7) -> 4.2 / 8.0 (9.2) -> 5.6; of a bf16 one 8192 values 8.0 (7.1) -> 5.3 / 8.8 (8.0) -> 6.0.
 __device__ __forceinline__ int fx_quad_at(const Ctx &c, int c0, int j, int n4) { return min(c0 + c.tid + j * MK_THREADS, n4 - 1); }
-// v = alpha * x + y of four quads of a row
-template <typename E>
-__device__ __forceinline__ void fx_addnorm_sum(CStage &st, const Ctx &c, int dS, int t, int c0, int n4, const f32x4 (&x)[4], f32x4 (&v)[4]) {
-  if (dS) {
-    const float *p = c.defer_part + (size_t)t * c.defer_n;
-    const size_t slice = (size_t)c.defer_rows * c.defer_n;
-    auto sum_slices = [&](auto ns) {  // summed in slice order
-      constexpr int Q = decltype(ns)::value;
-      f32x4 q[4][Q];
+// slices of four quads of a row that the linear in front left unsummed, in slice order
+__device__ __forceinline__ void fx_addnorm_slices(const Ctx &c, int dS, int t, int c0, int n4, f32x4 *v) {
+  const float *p = c.defer_part + (size_t)t * c.defer_n;
+  const size_t slice = (size_t)c.defer_rows * c.defer_n;
+  auto sum = [&](auto ns) {
+    constexpr int Q = decltype(ns)::value;
+    f32x4 q[4][Q];
 #pragma unroll
-      for (int b = 0; b < Q; b++) {
-        const auto rows = dev_rows(p + b * slice);
+    for (int b = 0; b < Q; b++) {
+      const auto rows = dev_rows(p + b * slice);
 #pragma unroll
-        for (int j = 0; j < 4; j++) q[j][b] = __builtin_bit_cast(f32x4, ldc_16B(rows, 16 * fx_quad_at(c, c0, j, n4)));
-      }
+      for (int j = 0; j < 4; j++) q[j][b] = __builtin_bit_cast(f32x4, ldc_16B(rows, 16 * fx_quad_at(c, c0, j, n4)));
+    }
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        v[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 4; j++) {
+      v[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < Q; b++) v[j] += q[j][b];
-      }
-    };
-    if (dS == 2) sum_slices(std::integral_constant<int, 2>{});
-    else if (dS == 4) sum_slices(std::integral_constant<int, 4>{});
-    else sum_slices(std::integral_constant<int, 8>{});
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = st.in ? fx_ldc_quad((const E *)st.in + (size_t)t * st.ld_in + 4 * fx_quad_at(c, c0, j, n4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) v[j][e] = fmaf(st.alpha, x[j][e], v[j][e]);
+      for (int b = 0; b < Q; b++) v[j] += q[j][b];
+    }
+  };
+  if (dS == 2) sum(std::integral_constant<int, 2>{});
+  else if (dS == 4) sum(std::integral_constant<int, 4>{});
+  else sum(std::integral_constant<int, 8>{});
 }
-template <typename E>
-__device__ __forceinline__ void fx_addnorm_store(CStage &st, int t, int s, f32x4 v, f32x4 g, float r) {
-  f32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; e++) o[e] = (v[e] * r) * (st.w_offset + g[e]);
-  if (st.out2) fx_stc_quad((float *)st.out2 + (size_t)t * st.ld_out2 + 4 * s, o);
-  fx_stc_quad((E *)st.out + (size_t)t * st.ld_out + 4 * s, o);
-}
-template <typename E>
-__device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char *smem) {
+// NS quads per thread
+template <typename E, int NS>
+__device__ __forceinline__ void stage_fx_addnorm_t(CStage &st, Ctx &c, int M, char *smem) {
   const int tid = c.tid, n4 = st.n / 4;
   float *red = (float *)smem;
   const f32x4 *w4 = (const f32x4 *)st.norm_w;
   const float *xr = (const float *)st.res;
   const int t0 = c.even_xcds ? c.rank * c.nxcd + c.xi : c.vid;  // rows are dealt round-robin over the dies
-  f32x4 x[4], v[4];
-  auto load_x = [&](int t, int c0) {
+  f32x4 g[NS], x[NS], v[NS];
+  auto load_x = [&](int t) {
+    const auto row = dev_rows(xr + (size_t)t * st.ld_res);
 #pragma unroll
-    for (int j = 0; j < 4; j++) x[j] = __builtin_bit_cast(f32x4, ldc_16B(dev_rows(xr + (size_t)t * st.ld_res), 16 * fx_quad_at(c, c0, j, n4)));
+    for (int j = 0; j < NS; j++) x[j] = __builtin_bit_cast(f32x4, ldc_16B(row, 16 * fx_quad_at(c, 0, j, n4)));
   };
-  auto squares = [&](int c0) {
+#pragma unroll
+  for (int j = 0; j < NS; j++) g[j] = w4[fx_quad_at(c, 0, j, n4)];
+  // the residual row was written at least one barrier earlier than y: requested before the barrier is awaited (not by the
+  // wavefront that polls it)
+  const bool pre = (st.flags & MK_F_RES_EARLY) && t0 < M && tid >= 64;
+  if (pre) load_x(t0);
+  barrier_wait(c);
+  const int dS = c.defer_S;
+  c.defer_S = 0;
+  for (int t = t0; t < M; t += c.G) {
+    if (!(pre && t == t0)) load_x(t);
+    if (dS) {
+#pragma unroll
+      for (int j = 0; j < NS; j += 4) fx_addnorm_slices(c, dS, t, j * MK_THREADS, n4, v + j);
+    } else {
+#pragma unroll
+      for (int j = 0; j < NS; j++) v[j] = st.in ? fx_ldc_quad((const E *)st.in + (size_t)t * st.ld_in + 4 * fx_quad_at(c, 0, j, n4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NS; j++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) ss += c0 + tid + j * MK_THREADS < n4 ? v[j][e] * v[j][e] : 0.f;
-    return ss;
-  };
-  if (n4 <= 4 * MK_THREADS) {
-    f32x4 g[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) g[j] = w4[fx_quad_at(c, 0, j, n4)];
-    // the residual row was written at least one barrier earlier than y: requested before the barrier is awaited (not by the
-    // wavefront that polls it)
-    const bool pre = (st.flags & MK_F_RES_EARLY) && t0 < M && tid >= 64;
-    if (pre) load_x(t0, 0);
-    barrier_wait(c);
-    const int dS = c.defer_S;
-    c.defer_S = 0;
-    for (int t = t0; t < M; t += c.G) {
-      if (!(pre && t == t0)) load_x(t, 0);
-      fx_addnorm_sum<E>(st, c, dS, t, 0, n4, x, v);
-      const float r = 1.f / sqrtf(block_sum(squares(0), red) / (float)st.k + st.eps);
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        if (tid + j * MK_THREADS < n4) fx_addnorm_store<E>(st, t, tid + j * MK_THREADS, v[j], g[j], r);
-      __syncthreads();
-    }
-  } else {
-    // longer rows (up to 12,288 values) wait in LDS for their factor: twelve quads per thread cost every other stage of the kernel its registers
-    f32x4 *row = (f32x4 *)(smem + 1024);
-    barrier_wait(c);
-    const int dS = c.defer_S;
-    c.defer_S = 0;
-    for (int t = t0; t < M; t += c.G) {
-      float ss = 0.f;
-      for (int c0 = 0; c0 < n4; c0 += 4 * MK_THREADS) {
-        load_x(t, c0);
-        fx_addnorm_sum<E>(st, c, dS, t, c0, n4, x, v);
-        ss += squares(c0);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (c0 + tid + j * MK_THREADS < n4) row[c0 + tid + j * MK_THREADS] = v[j];
+      for (int e = 0; e < 4; e++) {
+        v[j][e] = fmaf(st.alpha, x[j][e], v[j][e]);
+        ss += tid + j * MK_THREADS < n4 ? v[j][e] * v[j][e] : 0.f;
       }
-      const float r = 1.f / sqrtf(block_sum(ss, red) / (float)st.k + st.eps);
-      for (int s = tid; s < n4; s += MK_THREADS) fx_addnorm_store<E>(st, t, s, row[s], w4[s], r);
-      __syncthreads();
-    }
+    const float r = 1.f / sqrtf(block_sum(ss, red) / (float)st.k + st.eps);
+#pragma unroll
+    for (int j = 0; j < NS; j++)
+      if (tid + j * MK_THREADS < n4) {
+        const int s = tid + j * MK_THREADS;
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = (v[j][e] * r) * (st.w_offset + g[j][e]);
+        if (st.out2) fx_stc_quad((float *)st.out2 + (size_t)t * st.ld_out2 + 4 * s, o);
+        fx_stc_quad((E *)st.out + (size_t)t * st.ld_out + 4 * s, o);
+      }
+    __syncthreads();
   }
   c.wrote_through = true;
+}
+template <typename E>
+__device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char *smem) {
+  if (st.n <= 4 * 4 * MK_THREADS) stage_fx_addnorm_t<E, 4>(st, c, M, smem);
+  else if (st.n <= 8 * 4 * MK_THREADS) stage_fx_addnorm_t<E, 8>(st, c, M, smem);
+  else stage_fx_addnorm_t<E, 12>(st, c, M, smem);
 }
 
 // ----------------------------------------------------------------------------- head rows

@@ -91,6 +91,13 @@ def test_residual_norm(dtype, width, ld, alpha, offset, with_y):
     pk.finalize()
 
 
+# the last row of four quads per thread, the first and the last of eight, the first and the longest of twelve
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4092, 4100, 8190, 8196, 12286])
+def test_residual_norm_of_long_rows(dtype, width):
+    test_residual_norm(dtype, width, -(-width // 4) * 4, 0.7, 1.0, True)
+
+
 @pytest.mark.parametrize("width,n", [(192, 80), (1024, 300), (2048, 512), (4096, 700)])
 def test_norm_folded_into_a_single_token_linear(width, n):
     """One token: the linear forms the norm itself (every size has its own code path); several tokens: two stages.  Same
@@ -118,7 +125,7 @@ def test_norm_folded_into_a_single_token_linear(width, n):
     pk.finalize()
 
 
-@pytest.mark.parametrize("n,k", [(2048, 4096), (2056, 4096), (4104, 2048)])
+@pytest.mark.parametrize("n,k", [(2048, 4096), (2056, 4096), (4104, 2048), (8192, 1024), (12288, 512)])
 def test_residual_norm_behind_a_split_linear(n, k):
     """Whole tiles (the norm stage sums the slices) and a ragged last one (the linear does)."""
     pk = _graph(64)
