@@ -385,18 +385,23 @@ def test_experts_long_reductions(dtype, rows, E, top, ff, shared, width):
     test_experts_alone(dtype, rows, E, top, ff, shared, width)
 
 
-def _expert_rig(dtype, E, top, n, k, ids, width=None):
+def _expert_rig(dtype, E, top, n, k, ids, width=None, shared=None):
     """One expert linear over the caller's ids, the only stage of its graph: the caller's tensors and weights."""
     from mirage.mpk.persistent_kernel import expert_tiles
     g = torch.Generator().manual_seed(E + n)
-    w, x = (torch.randn(E, n, k, generator=g) / k ** 0.5).to(dtype), torch.randn(64, k, generator=g).to(dtype)
-    t = dict(x=x.cuda(), w=expert_tiles(w.cuda()), ids=torch.zeros(64, top, dtype=torch.int32, device="cuda"), o=torch.zeros(64, width or top * n, dtype=dtype, device="cuda"))
+    ns, ks = shared or (0, 0)
+    place = max(n, ns)
+    w, x = (torch.randn(E, n, k, generator=g) / k ** 0.5).to(dtype), torch.randn(64, max(k, ks), generator=g).to(dtype)
+    t = dict(x=x.cuda(), w=expert_tiles(w.cuda()), ids=torch.zeros(64, top, dtype=torch.int32, device="cuda"), o=torch.zeros(64, width or (top + bool(ns)) * place, dtype=dtype, device="cuda"))
     t["ids"][:len(ids)] = ids.to(torch.int32).cuda()
+    if shared:
+        ws = (torch.randn(1, ns, ks, generator=g) / ks ** 0.5).to(dtype)
+        t["ws"] = expert_tiles(ws.cuda())
     pk, _ = _graph(64, 64)
     a = {q: pk.attach_input(v, q) for q, v in t.items()}
-    pk.expert_linear_layer(a["x"], a["w"], a["ids"], a["o"], E, top, n, k, n)
+    pk.expert_linear_layer(a["x"], a["w"], a["ids"], a["o"], E, top, n, k, place, **(dict(shared_weight=a["ws"], shared_n=ns, shared_k=ks) if shared else {}))
     pk.compile()
-    return pk, t, x.double(), w.double()
+    return (pk, t, x.double(), w.double()) + ((ws[0].double(),) if shared else ())
 
 
 @BOTH
@@ -433,6 +438,26 @@ def test_an_expert_named_twice_stays_in_its_tokens_row(dtype):
             for e in ids[q].unique():
                 places = (ids[q] == e).nonzero().flatten()
                 assert right[q, places].any() and all(right[q, p] or (o[q, p] == 7).all() for p in places.tolist()), (M, q, int(e))
+    pk.finalize()
+
+
+@BOTH
+@pytest.mark.parametrize("E,top,n,k,shared", [
+    # fewer units than workgroups, of both kinds and of either; more units, but of the shared expert fewer; more of the shared expert alone
+    (16, 2, 512, 1024, (1024, 1024)), (4, 1, 32, 64, (4096, 64)), (16, 8, 2048, 64, (512, 64)), (8, 2, 512, 128, (33000, 64))])
+def test_shares_of_the_shared_expert(dtype, E, top, n, k, shared):
+    g = torch.Generator().manual_seed(n)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(64)])
+    pk, t, x, w, ws = _expert_rig(dtype, E, top, n, k, ids, shared=shared)
+    place = max(n, shared[0])
+    for M in (1, 2, 3, 4, 5, 64):
+        t["o"].zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        o = t["o"][:M].cpu().double().view(M, top + 1, place)
+        for s in range(top):
+            torch.testing.assert_close(o[:, s, :n], torch.stack([w[int(ids[q, s])] @ x[q, :k] for q in range(M)]), **_tol(dtype))
+        torch.testing.assert_close(o[:, top, :shared[0]], x[:M, :shared[1]] @ ws.T, **_tol(dtype))
+        assert not t["o"][M:].any()
     pk.finalize()
 
 
