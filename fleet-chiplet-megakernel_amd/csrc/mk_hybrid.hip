@@ -435,25 +435,27 @@ template <typename E>
 __device__ __forceinline__ int hy_rows(int K) { return min(16, (HY_RED - HY_X) / (K * (int)sizeof(E))); }
 
 // What a workgroup walks: units [s0, s1) of the shared expert (gs groups of tokens, units_s each), then units [r0, r1) of the entries
-// (`units` each).
+// (`units` each).  2^ksl_s, 2^ksl wavefronts split the reduction of a pair of tiles of the one and the others.
 struct HyRange {
-  int s0, s1, r0, r1, gs, units_s, units;
+  int s0, s1, r0, r1, gs, units_s, units, ksl_s, ksl;
 };
 // The u-th unit of a range: D steps of the reduction are a block.
 struct HyUnit {
   const u32x4 *w0, *w1;  // this lane's operands of the two tiles
   int nks, kb, ke, nb;   // steps of the reduction, this wavefront's share of them, blocks it takes (alike for all wavefronts)
-  int i, pair, n;        // entry (negative: a group of the shared expert), pair of tiles (may lie behind the last one), outputs
+  int i, pair, n, ksl;   // entry (negative: a group of the shared expert), pair of tiles (may lie behind the last one), outputs, split
 };
 template <typename E, int D>
-__device__ __forceinline__ HyUnit hy_unit(CStage &st, const HyLists *ls, const HyRange &rg, int u, int ks, int wave, int lane) {
+__device__ __forceinline__ HyUnit hy_unit(CStage &st, const HyLists *ls, const HyRange &rg, int u, int wave, int lane) {
   HyUnit a;
-  const int ksl = ks == 4 ? 2 : ks - 1, ns = rg.s1 - rg.s0;  // (log2 of ks)
+  const int ns = rg.s1 - rg.s0;
   const bool shared = u < ns;
+  const int ksl = shared ? rg.ksl_s : rg.ksl, ks = 1 << ksl;
   const int v = shared ? rg.s0 + u : rg.r0 + u - ns, per = shared ? rg.units_s : rg.units, q = v / per;
   a.pair = ((v - q * per) << (2 - ksl)) + (wave >> ksl);
   a.i = shared ? q - rg.gs : q;
   a.n = shared ? st.n_shared : st.n;
+  a.ksl = ksl;
   a.nks = (shared ? st.k_shared : st.k) / FxType<E>::KW;
   const int kq = (a.nks + ks - 1) >> ksl, p = (a.n + 31) / 32;
   a.kb = min(a.nks, (wave & (ks - 1)) * kq);
@@ -466,17 +468,17 @@ __device__ __forceinline__ HyUnit hy_unit(CStage &st, const HyLists *ls, const H
 }
 constexpr int HY_FIRST = 8;  // steps of the ring that may have been requested in advance
 
-// Walk the units of `rg`.  ks wavefronts (4, 2 or 1) split the reduction of a pair of tiles.  w: the ring, its first steps requested if
+// Walk the units of `rg`.  w: the ring, its first steps requested if
 // `early`.  row_words: 16-byte words per row where all rows of a single token lie in LDS (row of place p at p * row_words; 0: one row).
 template <typename E, int D, bool XLDS>
-__device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const HyLists *ls, int M, const HyRange rg, int ks, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
+__device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const HyLists *ls, int M, const HyRange rg, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const bool glu = st.flags & MK_F_SILU;
   u32x4 *xl = (u32x4 *)(smem + HY_X);
   f32x4 *red = (f32x4 *)(smem + HY_RED);
   const int ns = rg.s1 - rg.s0, n_all = ns + rg.r1 - rg.r0;
-  HyUnit a = hy_unit<E, D>(st, ls, rg, 0, ks, wave, lane);
+  HyUnit a = hy_unit<E, D>(st, ls, rg, 0, wave, lane);
 #pragma unroll
   for (int j = 0; j < D; j++)
     if (j >= HY_FIRST || !early) {
@@ -486,7 +488,6 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
   int staged = 0x7fffffff, cnt = 1, tok = 0, place = 0;  // rows in LDS belong to this entry; token and place of column lane & 15
   const E *xr = nullptr;
   const u32x4 *xb = xl + lg;
-  const int ksl = ks == 4 ? 2 : ks - 1;  // log2
   const u32x4 zero = {0u, 0u, 0u, 0u};
   for (int u = 0; u < n_all; u++) {
     if (a.i != staged) {
@@ -545,7 +546,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
       }
     }
     const bool more = u + 1 < n_all;
-    const HyUnit nx = more ? hy_unit<E, D>(st, ls, rg, u + 1, ks, wave, lane) : a;
+    const HyUnit nx = more ? hy_unit<E, D>(st, ls, rg, u + 1, wave, lane) : a;
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     for (int blk = 0; blk < a.nb; blk++) {
       const bool last = blk + 1 == a.nb;
@@ -574,7 +575,8 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
 #pragma unroll
     for (int h = 0; h < 2; h++) rb[(wave * 2 + h) * 64 + lane] = acc[h];
     __syncthreads();
-    const f32x4 *rw = rb + (wave >> ksl << ksl) * 2 * 64 + lane;
+    const int ks = 1 << a.ksl;
+    const f32x4 *rw = rb + (wave >> a.ksl << a.ksl) * 2 * 64 + lane;
     auto total = [&](int h) {
       f32x4 v = rw[h * 64];
       for (int q = 1; q < ks; q++) v += rw[(2 * q + h) * 64];
@@ -600,16 +602,25 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Ex = st.num_experts, topk = st.topk;
-  // short reductions are split among fewer wavefronts, so that each of them has a ring's worth of steps
-  const int nks = st.k / KW, ks = nks >= 48 ? 4 : nks >= 24 ? 2 : 1, ppu = MK_WAVES / ks;  // pairs of tiles per unit
   HyLists *ls = (HyLists *)smem;
   const int fit = hy_rows<E>(st.k), fit_s = st.w_shared ? hy_rows<E>(st.k_shared) : 16;
   const bool xlds = fit >= 2 && fit_s >= 2;
   const int per = xlds ? fit : 16, per_s = xlds ? fit_s : 16;
   HyRange rg;
-  rg.units = ((st.n + 31) / 32 + ppu - 1) / ppu;
-  rg.units_s = st.w_shared ? ((st.n_shared + 31) / 32 + ppu - 1) / ppu : 0;
   rg.gs = st.w_shared ? (M + per_s - 1) / per_s : 0;
+  // A wavefront takes a whole reduction where that is not much longer than its ring, or half of it.  64 experts of 1024, 16 tokens, us, whole /
+  // halves / quarters: 512 values 16.4 / - / 22.5, 768: 19.6 / 22.1 / 22.9, 1024: 24.1 / 25.9 / 24.8, 1536: - / 33.1 / 34.9, 2048: - / 40.7 / 39.8.
+  // The shared expert goes by its own length (512 x 8192 beside 1024 x 1024, one token: 23.4 -> 15.6, eight workgroups had streamed it), and where
+  // there are not even as many pairs of tiles as workgroups, all four wavefronts share one.
+  const int pairs = (st.n + 31) / 32, pairs_s = st.w_shared ? (st.n_shared + 31) / 32 : 0;
+  const bool few = min(Ex, M * topk) * pairs + rg.gs * pairs_s <= c.G;
+  auto split = [&](int nks) { return few || nks >= 48 ? 2 : nks >= 24 ? 1 : 0; };
+  const int nks = st.k / KW;
+  rg.ksl = split(nks);
+  rg.ksl_s = split(st.k_shared / KW);
+  auto units = [&](int p, int ksl) { return (p + (MK_WAVES >> ksl) - 1) / (MK_WAVES >> ksl); };
+  rg.units = units(pairs, rg.ksl);
+  rg.units_s = units(pairs_s, rg.ksl_s);
   const int n_s = rg.gs * rg.units_s;
   auto share = [](int n, int v, int of) {  // n v / of, without the product
     const unsigned q = (unsigned)n / (unsigned)of;
@@ -643,7 +654,7 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   u32x4 w[2][12];
   const bool early = rg.s0 < rg.s1 && wave != 0;  // (wavefront 0 polls and routes)
   if (early) {
-    const HyUnit a = hy_unit<E, HY_FIRST>(st, ls, rg, 0, ks, wave, lane);
+    const HyUnit a = hy_unit<E, HY_FIRST>(st, ls, rg, 0, wave, lane);
 #pragma unroll
     for (int j = 0; j < HY_FIRST; j++) {
       w[0][j] = ldg_stream(a.w0 + (size_t)min(a.kb + j, a.nks - 1) * 64);
@@ -724,10 +735,10 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   }
   if (rg.s0 < rg.s1 || rg.r0 < rg.r1) {
     // a ring of 8 steps per tile, or of 12 where a wavefront's share of the reduction is then walked with fewer empty steps
-    const int kq = (nks + ks - 1) / ks;
-    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, c, ls, M, rg, ks, early, w, false, 0, smem);
-    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, c, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
-    else hy_expert_walk<E, 12, true>(st, c, ls, M, rg, ks, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    const int kq = (nks + (1 << rg.ksl) - 1) >> rg.ksl;
+    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, c, ls, M, rg, early, w, false, 0, smem);
+    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    else hy_expert_walk<E, 12, true>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
   }
   c.wrote_through = true;
 }
