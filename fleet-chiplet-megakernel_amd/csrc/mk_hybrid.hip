@@ -604,7 +604,12 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   const int Ex = st.num_experts, topk = st.topk;
   HyLists *ls = (HyLists *)smem;
   const int fit = hy_rows<E>(st.k), fit_s = st.w_shared ? hy_rows<E>(st.k_shared) : 16;
-  const bool xlds = fit >= 2 && fit_s >= 2;
+  // Rows in LDS for fewer tokens than an expert has make its weights pass again, which costs where the units fill the chip as it is: rows are
+  // read from memory then, 16 tokens at a time.  2048 x 16384 of 4 (4 rows fit), 33 / 64 tokens, us: before ranges 67 / 91, staged 112 / 193, from
+  // memory 46 / 80; 2048 x 8192 (8 rows) 43 / 52, 42 / 63, 26 / 43; a shared 512 x 8192 beside few units, 33 tokens: staged 21, from memory 35.
+  const int pairs = (st.n + 31) / 32, pairs_s = st.w_shared ? (st.n_shared + 31) / 32 : 0;
+  const bool again = (fit < 16 && M * topk > Ex * fit) || (fit_s < 16 && M > fit_s);
+  const bool xlds = fit >= 2 && fit_s >= 2 && !(again && min(Ex, M * topk) * pairs + (M + 15) / 16 * pairs_s >= c.G);
   const int per = xlds ? fit : 16, per_s = xlds ? fit_s : 16;
   HyRange rg;
   rg.gs = st.w_shared ? (M + per_s - 1) / per_s : 0;
@@ -612,7 +617,6 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   // halves / quarters: 512 values 16.4 / - / 22.5, 768: 19.6 / 22.1 / 22.9, 1024: 24.1 / 25.9 / 24.8, 1536: - / 33.1 / 34.9, 2048: - / 40.7 / 39.8.
   // The shared expert goes by its own length (512 x 8192 beside 1024 x 1024, one token: 23.4 -> 15.6, eight workgroups had streamed it), and where
   // there are not even as many pairs of tiles as workgroups, all four wavefronts share one.
-  const int pairs = (st.n + 31) / 32, pairs_s = st.w_shared ? (st.n_shared + 31) / 32 : 0;
   const bool few = min(Ex, M * topk) * pairs + rg.gs * pairs_s <= c.G;
   auto split = [&](int nks) { return few || nks >= 48 ? 2 : nks >= 24 ? 1 : 0; };
   const int nks = st.k / KW;

@@ -448,17 +448,28 @@ def test_an_expert_named_twice_stays_in_its_tokens_row(dtype):
 def test_shares_of_the_shared_expert(dtype, E, top, n, k, shared):
     g = torch.Generator().manual_seed(n)
     ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(64)])
-    pk, t, x, w, ws = _expert_rig(dtype, E, top, n, k, ids, shared=shared)
-    place = max(n, shared[0])
-    for M in (1, 2, 3, 4, 5, 64):
+    pk, t, x, w, *ws = _expert_rig(dtype, E, top, n, k, ids, shared=shared)
+    place = max(n, shared[0] if shared else 0)
+    for M in (1, 2, 3, 4, 5, 33, 64):
         t["o"].zero_()
         pk.run_once(list(range(M)), [0] * M)
-        o = t["o"][:M].cpu().double().view(M, top + 1, place)
+        o = t["o"][:M].cpu().double().view(M, top + bool(shared), place)
         for s in range(top):
             torch.testing.assert_close(o[:, s, :n], torch.stack([w[int(ids[q, s])] @ x[q, :k] for q in range(M)]), **_tol(dtype))
-        torch.testing.assert_close(o[:, top, :shared[0]], x[:M, :shared[1]] @ ws.T, **_tol(dtype))
+        if shared:
+            torch.testing.assert_close(o[:, top, :shared[0]], x[:M, :shared[1]] @ ws[0].T, **_tol(dtype))
         assert not t["o"][M:].any()
     pk.finalize()
+
+
+@BOTH
+@pytest.mark.parametrize("E,top,n,k,shared", [
+    # rows of which LDS holds few: units that fill the chip (rows from memory), units that do not (rows staged in groups)
+    (4, 1, 2080, 8192, None), (2, 1, 64, 8192, None), (3, 2, 2816, 5120, (96, 64)), (4, 1, 64, 64, (4128, 8192)),
+    # one unit per workgroup: shares of one step, of several blocks, of none, that end inside a block
+    (16, 2, 64, 64, None), (4, 2, 512, 4096, None), (5, 2, 96, 1568, (64, 1504)), (5, 1, 40, 96, (40, 32))])
+def test_rows_of_experts_from_memory(dtype, E, top, n, k, shared):
+    test_shares_of_the_shared_expert(dtype, E, top, n, k, shared)
 
 
 # ---------------------------------------------------------------- whole models
