@@ -468,9 +468,12 @@ __device__ __forceinline__ HyUnit hy_unit(CStage &st, const HyLists *ls, const H
 }
 constexpr int HY_FIRST = 8;  // steps of the ring that may have been requested in advance
 
-// Walk the units of `rg`.  w: the ring, its first steps requested if
-// `early`.  row_words: 16-byte words per row where all rows of a single token lie in LDS (row of place p at p * row_words; 0: one row).
-template <typename E, int D, bool XLDS>
+// Walk the units of `rg`.  w: the ring, its first steps requested if `early`.  row_words: 16-byte words per row where all rows of a single token
+// lie in LDS (row of place p at p * row_words; 0: one row).
+// XLDS: rows are staged in LDS.  ONCE: the range is one unit, so what would be staged is read once as well: its rows come straight from memory
+// beside the weights, and nothing is requested behind its last step.  us, before ranges -> staged -> ONCE: 64 x 64 of 16, 5 tokens 6.8 -> 8.4 ->
+// 7.1; 512 x 1024 of 16, 5 tokens 8.9 -> 9.1 -> 8.6; 512 x 2048 of 8, 64 tokens 14.1 -> 13.6 -> 11.1.
+template <typename E, int D, bool XLDS, bool ONCE>
 __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const HyLists *ls, int M, const HyRange rg, bool early, u32x4 (&w)[2][12], bool rows_in, int row_words, char *smem) {
   constexpr int EPC = FxType<E>::EPC, KW = FxType<E>::KW;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
@@ -481,7 +484,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
   HyUnit a = hy_unit<E, D>(st, ls, rg, 0, wave, lane);
 #pragma unroll
   for (int j = 0; j < D; j++)
-    if (j >= HY_FIRST || !early) {
+    if ((j >= HY_FIRST || !early) && (!ONCE || a.kb + j < a.ke)) {
       w[0][j] = ldg_stream(a.w0 + (size_t)min(a.kb + j, a.nks - 1) * 64);
       w[1][j] = ldg_stream(a.w1 + (size_t)min(a.kb + j, a.nks - 1) * 64);
     }
@@ -548,12 +551,14 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
     const bool more = u + 1 < n_all;
     const HyUnit nx = more ? hy_unit<E, D>(st, ls, rg, u + 1, wave, lane) : a;
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    for (int blk = 0; blk < a.nb; blk++) {
+    auto block = [&](int blk, auto refill) {
+      constexpr bool REFILL = decltype(refill)::value;
       const bool last = blk + 1 == a.nb;
       const int k0 = a.kb + blk * D;
       u32x4 b[D];
 #pragma unroll
       for (int j = 0; j < D; j++) {
+        if (ONCE && !REFILL && k0 + j >= a.ke) continue;
         const int s = min(k0 + j, a.nks - 1);
         if constexpr (XLDS) b[j] = xb[s * 4 * cnt];
         else b[j] = *(const u32x4 *)(xr + (size_t)s * KW);
@@ -564,12 +569,17 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
 #pragma unroll
       for (int j = 0; j < D; j++) {
         const bool real = k0 + j < a.ke;
+        if (ONCE && !REFILL && !real) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) acc[h] = fx_mma_k(E(), real ? w[h][j] : zero, b[j], acc[h]);
-        w[0][j] = ldg_stream(p0 + (size_t)min(kn + j, kl) * 64);
-        w[1][j] = ldg_stream(p1 + (size_t)min(kn + j, kl) * 64);
+        if constexpr (REFILL) {
+          w[0][j] = ldg_stream(p0 + (size_t)min(kn + j, kl) * 64);
+          w[1][j] = ldg_stream(p1 + (size_t)min(kn + j, kl) * 64);
+        }
       }
-    }
+    };
+    for (int blk = 0; blk < (ONCE ? a.nb - 1 : a.nb); blk++) block(blk, std::true_type{});
+    if constexpr (ONCE) block(a.nb - 1, std::false_type{});
     // ---- the wavefronts' sums
     f32x4 *rb = red + (u & 1) * (MK_WAVES * 2 * 64);
 #pragma unroll
@@ -740,9 +750,11 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
   if (rg.s0 < rg.s1 || rg.r0 < rg.r1) {
     // a ring of 8 steps per tile, or of 12 where a wavefront's share of the reduction is then walked with fewer empty steps
     const int kq = (nks + (1 << rg.ksl) - 1) >> rg.ksl;
-    if (!xlds && !rows_in) hy_expert_walk<E, 8, false>(st, c, ls, M, rg, early, w, false, 0, smem);
-    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
-    else hy_expert_walk<E, 12, true>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    const bool once = per == 16 && per_s == 16 && rg.s1 - rg.s0 + rg.r1 - rg.r0 == 1;
+    if (once && !rows_in) hy_expert_walk<E, 8, false, true>(st, c, ls, M, rg, early, w, false, 0, smem);
+    else if (!xlds && !rows_in) hy_expert_walk<E, 8, false, false>(st, c, ls, M, rg, early, w, false, 0, smem);
+    else if ((kq + 7) / 8 * 8 <= (kq + 11) / 12 * 12) hy_expert_walk<E, 8, true, false>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
+    else hy_expert_walk<E, 12, true, false>(st, c, ls, M, rg, early, w, rows_in, one_rows > 1 ? one_words : 0, smem);
   }
   c.wrote_through = true;
 }
