@@ -3556,9 +3556,6 @@ __device__ __forceinline__ void attn_source_ready(CStage &st, Ctx &c, AttnSource
   c.defer_S = 0;
 }
 
-#ifndef MK_TUNE_ATTN_TILES
-#define MK_TUNE_ATTN_TILES 2
-#endif
 #ifndef MK_TUNE_NPRE
 #define MK_TUNE_NPRE 4
 #endif
@@ -3941,7 +3938,8 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 //
 // Bound by the cache's way through L2 for long prompts and by round trips for short contexts.  A unit per token had read the cache once
 // for every token of a prompt and prepared its new key rows as often.  64 tokens of one prompt, 32 q / 8 kv heads, as a stage: behind 1216
-// cached positions 85 -> 31 us, behind 2432 127 -> 43; 64 streams of one token 33 -> 30.
+// cached positions 85 -> 31 us, behind 2432 127 -> 43; 64 streams of one token 33 -> 32.  (A portion at the very start of its prompt is as fast as
+// before or, with few kv heads, slower, its new rows being prepared by fewer workgroups: 64 tokens of 8 q / 2 kv heads 29 -> 32.)
 //
 // Tile: scores with A = K (lane (i, g): row of position i, dims 32 s + 8 g .. of step s) and B = q (lane (j, g): column j, same dims)
 // -> lane (j, g) holds column j at positions 4 g .. 4 g + 3.  Those four weights are already the A operand of a 16x16x16 step over
@@ -3952,7 +3950,7 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 template <int QPK>
 __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
-  constexpr int D = 128, NC = 16, TG = NC / QPK, RB = MK_TUNE_ATTN_TILES, PD = 132;
+  constexpr int D = 128, NC = 16, TG = NC / QPK, RB = 2, PD = 132;
   constexpr int GS = 1088, TS = 4 * GS, SLOT = 2 * TS, NEW_BYTES = MK_MAX_NEW_PER_REQ / 4 * GS;
   constexpr int FLAG_OFF = NC * D * 2, KN_OFF = FLAG_OFF + 64, VN_OFF = KN_OFF + NEW_BYTES, PART_OFF = VN_OFF + NEW_BYTES, BUF_OFF = PART_OFF + MK_WAVES * NC * PD * 4;
   static_assert(BUF_OFF + MK_WAVES * RB * SLOT <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
@@ -4565,9 +4563,9 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         if (nx.op == MK_OP_LINEAR && (nx.flags & MK_F_NORM) && nx.in == st.in && linear_small_ok(nx, c, M)) continue;
       }
       // Lane offsets that stages derive from the thread index would otherwise be computed once, ahead of all stages, and wait in scratch
-      // for the stage that wants them, which then starts with a chain of scratch loads.  Scratch per lane: 480 -> 0 bytes (fixed-shape
-      // stages), 640 -> 0 (flex), 1568 -> 0 (mix), 1648 -> 0 (hybrid), 2320 -> 624 (dual); vizonex-8b at 64 streams 95.5 -> 85.4 ms,
-      // bukatar-8b 57.0 -> 52.5, suborax-8b serving 135 -> 131.
+      // for the stage that wants them, which then starts with a chain of scratch loads.  Scratch per lane in the kernels of several tokens: 480 -> 0
+      // bytes (fixed-shape stages), 640 -> 80 (flex; declared, no instruction uses it), 1568 -> 0 (mix), 1648 -> 0 (hybrid), 2320 -> 608 (dual; 752
+      // by now, 498 registers spilled); vizonex-8b at 64 streams 95.5 -> 85.4 ms, bukatar-8b 57.0 -> 52.5, suborax-8b serving 135 -> 131.
       c.tid = threadIdx.x;
       asm volatile("" : "+v"(c.tid));
       __builtin_assume(c.tid >= 0 && c.tid < MK_THREADS);

@@ -183,14 +183,11 @@ class ServingSession:
             self._sampled.copy_(m.output_tokens.view(-1), non_blocking=True)
             pk.wait()
             return self._sampled.tolist()
-        if getattr(self, "_block", None) is not None:
-            self._block[:len(desc)].copy_(torch.tensor(desc, dtype=torch.int32))
-        else:
-            t = torch.tensor(desc, dtype=torch.int32)
-            for dst, lo, n in ((m.qo_indptr_buffer, 0, R + 1), (m.paged_kv_indptr_buffer, R + 1, R + 1), (m.paged_kv_last_page_len_buffer, 2 * R + 2, R),
-                               (self.state_slots, 3 * R + 2, R), (m.paged_kv_indices_buffer, 4 * R + 2, len(pages))):
-                if dst is not None:
-                    dst[:n].copy_(t[lo:lo + n])
+        t = torch.tensor(desc, dtype=torch.int32)
+        for dst, lo, n in ((m.qo_indptr_buffer, 0, R + 1), (m.paged_kv_indptr_buffer, R + 1, R + 1), (m.paged_kv_last_page_len_buffer, 2 * R + 2, R),
+                           (self.state_slots, 3 * R + 2, R), (m.paged_kv_indices_buffer, 4 * R + 2, len(pages))):
+            if dst is not None:
+                dst[:n].copy_(t[lo:lo + n])
         m.input_tokens.view(-1)[:len(ids)].copy_(torch.tensor(ids, dtype=torch.int64))
         m()
 

@@ -266,22 +266,30 @@ def test_state_slots_of_a_session():
     from mirage.mpk.serving import PagePool, ServingSession
 
     class Stub:
-        def __call__(self):
+        profiler_tensor = None
+
+        def enqueue_steps(self, n):
+            pass
+
+        def wait(self):
             pass
 
     s, R = ServingSession.__new__(ServingSession), 3
     s.page_size, s.max_rows, s.max_requests, s.rows_per_request, s.max_seq = 4, 8, R, 8, 64
     s.pool, s.slots, s.requests, s.mpk = PagePool(12), PagePool(R, "state slots"), {}, Stub()
-    s._block = torch.zeros(4 * R + 2 + 12, dtype=torch.int32)
-    s.mpk.input_tokens = torch.zeros(8, 1, dtype=torch.int64)
-    slots = lambda n: s._block[3 * R + 2:3 * R + 2 + n].tolist()
+    # as open() lays them out: ids, then the five index tensors
+    s._host, s._dev = (torch.zeros(2 * 8 + 4 * R + 2 + 12, dtype=torch.int32) for _ in range(2))
+    s.mpk.output_tokens, s.mpk.persistent_kernel, s._sampled = torch.zeros(8, 1, dtype=torch.int64), s.mpk, torch.zeros(8, dtype=torch.int64)
+    block = s._dev[2 * 8:]
+    slots = lambda n: block[3 * R + 2:3 * R + 2 + n].tolist()
     s._pass([("a", [1, 2]), ("b", [3])])
     a, b = slots(2)
     s._pass([("c", [1]), ("b", [4])])
     c, b2 = slots(2)
     assert b2 == b and {a, b, c} == {0, 1, 2}
     s._pass([("b", [5]), ("a", [6]), ("c", [7])])
-    assert slots(3) == [b, a, c] and s._block[4 * R + 2:].tolist()[:3] == s.requests["b"].pages + s.requests["a"].pages + s.requests["c"].pages
+    assert s._dev[:6].view(torch.int64).tolist() == [5, 6, 7]
+    assert slots(3) == [b, a, c] and block[4 * R + 2:].tolist()[:3] == s.requests["b"].pages + s.requests["a"].pages + s.requests["c"].pages
     with pytest.raises(RuntimeError, match="state slots"):
         s._pass([("d", [1])])
     assert "d" not in s.requests and len(s.slots) == 0
