@@ -342,10 +342,10 @@ int set_flex(mk_graph *g, int dtype, const char *task) {
 
 // The linear lowered last may leave its K-slice partials to the stage that is lowered next and reads `rows` first.  `res_too`: that stage
 // adds the linear's residual.  Partials are stored as whole tiles of 16 columns in rows of pl.n: a ragged last tile would reach into the
-// next row, so such a linear exchanges its slices itself.
+// next row, so such a linear exchanges its slices itself; so does one with an activation, which belongs behind the sum.
 void leave_sum(mk_graph *g, const void *rows, int64_t ld, bool res_too = false) {
   MkStage &pl = g->stages.back();
-  if (pl.op != MK_OP_LINEAR || (pl.flags & MK_F_SILU) || (!res_too && (pl.flags & MK_F_RES)) || pl.out != rows || pl.ld_out != ld || (pl.n & 15)) return;
+  if (pl.op != MK_OP_LINEAR || (pl.flags & (MK_F_SILU | MK_F_RELU2)) || (!res_too && (pl.flags & MK_F_RES)) || pl.out != rows || pl.ld_out != ld || (pl.n & 15)) return;
   pl.flags |= MK_F_DEFER_SUM;
   g->stage_desc.back() += " sum=next";
 }
@@ -1034,7 +1034,7 @@ int lower_residual_prenorm(mk_graph *g, size_t &i) {
     // a plain linear in front whose whole output is the last summand may leave its split-K sum to this stage (which also stores it)
     const Tensor *ly = y2 ? y2 : y;
     // (not when the first summand reads those rows too, before they are there)
-    if (ly && !sw && pl.n == st.n && (pl.ld_out & 3) == 0 && !(pl.flags & MK_F_RELU2) && !(y2 && rows_meet(*y, *y2, B, n))) leave_sum(g, ly->ptr, ly->strides[0]);
+    if (ly && !sw && pl.n == st.n && (pl.ld_out & 3) == 0 && !(y2 && rows_meet(*y, *y2, B, n))) leave_sum(g, ly->ptr, ly->strides[0]);
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;

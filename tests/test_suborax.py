@@ -270,18 +270,22 @@ def test_page_pool_and_step_packing():
 
 @pytest.mark.parametrize("front", ["residual_rmsnorm", "residual_prenorm", "flex_attention"])
 def test_which_linears_leave_their_sum_to_the_next_stage(front):
-    """A split linear leaves whole tiles of 16 columns in rows as long as its output: a ragged last tile would reach into the next row."""
+    """A split linear leaves whole tiles of 16 columns in rows as long as its output: a ragged last tile would reach into the next row.  Nor
+    does the stage behind know of an activation."""
     import mirage as mi
     from helpers import make_meta, make_mpk
     from mirage.mpk.persistent_kernel import flex_cache_dims
 
-    def leaves(heads):
+    def leaves(heads, squared=False):
         n = 8 * (heads + 2)
         pk = make_mpk(make_meta(8, 64, 8, 8, 8, device="cpu"), 64, 8, 8, 8, 64, num_workers=256)
         new = lambda name, *shape, dtype=mi.bfloat16: pk.new_tensor(shape, dtype=dtype, name=name)
         row, vec = (lambda name: new(name, 8, n, dtype=mi.float32)), (lambda name: new(name, n, dtype=mi.float32))
         y, h = new("y", 8, n), new("h", 8, n)
-        pk.linear_layer(new("x", 8, 4096), new("w", n, 4096), y, (1, 1, 1), (256, 1, 1))
+        z = new("z", 8, n) if squared else y
+        pk.linear_layer(new("x", 8, 4096), new("w", n, 4096), z, (1, 1, 1), (256, 1, 1))
+        if squared:
+            pk.relu_squared_layer(z, y)
         if front == "flex_attention":
             dk, dv = flex_cache_dims(8, 8)
             pk.flex_attention_layer(y, new("k", 8, 64, 1, dk), new("v", 8, 64, 1, dv), None, None, None, new("q", 8, heads * dk), h, heads, 1, 8, 8, 0, 1.0)
@@ -293,3 +297,4 @@ def test_which_linears_leave_their_sum_to_the_next_stage(front):
 
     assert leaves(254)
     assert not leaves(255)
+    assert not leaves(254, squared=True)

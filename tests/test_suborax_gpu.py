@@ -150,6 +150,31 @@ def test_residual_norm_behind_a_split_linear(n, k):
     pk.finalize()
 
 
+def test_residual_norm_behind_an_activation():
+    """max(x, 0)^2 belongs to the linear, split or not."""
+    import mirage as mi
+    n, k = 2048, 4096
+    pk = _graph(64)
+    i, W = torch.randn(64, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") / k ** 0.5).bfloat16()
+    x, w = torch.randn(64, n, device="cuda"), torch.randn(n, device="cuda") * 0.2
+    y, xo, o = torch.zeros(64, n, device="cuda").bfloat16(), torch.zeros(64, n, device="cuda"), torch.zeros(64, n, device="cuda").bfloat16()
+    a = pk.attach_input
+    yy, z = a(y, "y"), pk.new_tensor((64, n), dtype=mi.bfloat16, name="z")
+    pk.linear_layer(a(i, "i"), a(W, "W"), z, (1, 1, 1), (256, 1, 1))
+    pk.relu_squared_layer(z, yy)
+    pk.residual_rmsnorm_layer(yy, a(x, "x"), a(w, "w"), a(xo, "xo"), a(o, "o"), alpha=1.6, eps=1e-6, weight_offset=1.0)
+    pk.compile()
+    for M in (64, 5, 1):
+        xo.zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        s = (i[:M].double() @ W.double().T).clamp(min=0).pow(2)
+        v = 1.6 * x[:M].double() + s
+        f = (1.0 + w.double()) / (v.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt()
+        # half a bf16 step, up to 2^-8 of the squared value
+        assert bool(((xo[:M].double() - v * f).abs() <= 2.0 ** -8 * (s * f).abs() + 1e-4 * (1.0 + v.abs())).all()), M
+    pk.finalize()
+
+
 @pytest.mark.parametrize("k,n,silu", [(64, 33, False), (192, 500, False), (448, 130, True), (2048, 64, True)])
 def test_32_bit_linear(k, n, silu):
     import mirage as mi
