@@ -350,6 +350,17 @@ void leave_sum(mk_graph *g, const void *rows, int64_t ld, bool res_too = false) 
   g->stage_desc.back() += " sum=next";
 }
 
+// does a task behind task i read tensor `id` before another one writes it?  (Some stages sum slices without storing the rows.)
+bool read_later(const mk_graph *g, size_t i, int id) {
+  for (size_t j = i + 1; j < g->ltasks.size(); j++) {
+    const Task &t = g->ltasks[j];
+    const size_t n_in = t.ops.size() - (size_t)num_outputs(t);
+    if (std::find(t.ops.begin(), t.ops.begin() + n_in, id) != t.ops.begin() + n_in) return true;
+    if (std::find(t.ops.begin() + n_in, t.ops.end(), id) != t.ops.end()) return false;
+  }
+  return false;
+}
+
 // Lower one linear-type task (optionally preceded by a norm task whose output it consumes, optionally
 // followed by a silu_mul consuming its output) into stages.
 int lower_linear(mk_graph *g, size_t &i) {
@@ -797,7 +808,7 @@ int lower_residual_rmsnorm(mk_graph *g, size_t &i) {
   if ((st.ld_in | st.ld_res | st.ld_out | st.ld_out2) & 3) return fail(MK_EINVAL, "residual_rmsnorm: row strides must be multiples of 4");
   if (!g->stages.empty()) {
     const MkStage &pl = g->stages.back();
-    if (y && pl.n == st.n && width == n) leave_sum(g, st.in, st.ld_in);
+    if (y && pl.n == st.n && width == n && !read_later(g, i, t.ops[0])) leave_sum(g, st.in, st.ld_in);
     if (pl.out != st.res && pl.out2 != st.res && pl.norm_out != st.res) st.flags |= MK_F_RES_EARLY;
   }
   bool res, silu;
@@ -931,7 +942,7 @@ int lower_flex_attention(mk_graph *g, size_t &i) {
   g->flex_part = std::max(g->flex_part, (size_t)g->G * 16 * (st.v_tiles * 16 + 32));
   if (!g->stages.empty()) {
     // the q/k/v linear may leave its K-slice sum to this stage's row fetch
-    if (g->stages.back().n >= cols && !(st.flags & MK_F_ROW_NORM)) leave_sum(g, st.in, st.ld_in);
+    if (g->stages.back().n >= cols && !(st.flags & MK_F_ROW_NORM) && !read_later(g, i, t.ops[0])) leave_sum(g, st.in, st.ld_in);
   }
   if (B > 1) {
     MkStage sp = st;

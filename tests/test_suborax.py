@@ -276,7 +276,7 @@ def test_which_linears_leave_their_sum_to_the_next_stage(front):
     from helpers import make_meta, make_mpk
     from mirage.mpk.persistent_kernel import flex_cache_dims
 
-    def leaves(heads, squared=False):
+    def leaves(heads, squared=False, behind=None):
         n = 8 * (heads + 2)
         pk = make_mpk(make_meta(8, 64, 8, 8, 8, device="cpu"), 64, 8, 8, 8, 64, num_workers=256)
         new = lambda name, *shape, dtype=mi.bfloat16: pk.new_tensor(shape, dtype=dtype, name=name)
@@ -293,8 +293,14 @@ def test_which_linears_leave_their_sum_to_the_next_stage(front):
             pk.residual_rmsnorm_layer(y, row("r"), vec("g"), row("s"), h)
         else:
             pk.residual_prenorm_layer(y, row("r"), row("s"), h, weight=vec("g"))
+        if behind == "written":
+            pk.linear_layer(new("x2", 8, 4096), new("w2", n, 4096), y, (1, 1, 1), (256, 1, 1))
+        if behind:
+            pk.residual_rmsnorm_layer(y, row("r2"), vec("g2"), row("s2"), new("h2", 8, n))
         return "sum=next" in [l for l in pk.describe_program().splitlines() if " LINEAR" in l][0]
 
     assert leaves(254)
     assert not leaves(255)
     assert not leaves(254, squared=True)
+    # residual_prenorm stores the rows it sums; the others do not, so nobody else may want them
+    assert leaves(254, behind="read") == (front == "residual_prenorm") and leaves(254, behind="written")
