@@ -179,9 +179,10 @@ class ServingSession:
             if pk.profiler_tensor is not None:  # (the whole call also writes the trace)
                 m()
                 return None
-            pk.enqueue_steps(1)
+            stream = torch.cuda.current_stream(self._dev.device) if self._dev.is_cuda else None  # (the copies', whichever device is current)
+            pk.enqueue_steps(1, default_stream=stream)
             self._sampled.copy_(m.output_tokens.view(-1), non_blocking=True)
-            pk.wait()
+            pk.wait(default_stream=stream)
             return self._sampled.tolist()
         t = torch.tensor(desc, dtype=torch.int32)
         for dst, lo, n in ((m.qo_indptr_buffer, 0, R + 1), (m.paged_kv_indptr_buffer, R + 1, R + 1), (m.paged_kv_last_page_len_buffer, 2 * R + 2, R),

@@ -268,10 +268,10 @@ def test_state_slots_of_a_session():
     class Stub:
         profiler_tensor = None
 
-        def enqueue_steps(self, n):
+        def enqueue_steps(self, n, default_stream):
             pass
 
-        def wait(self):
+        def wait(self, default_stream):
             pass
 
     s, R = ServingSession.__new__(ServingSession), 3

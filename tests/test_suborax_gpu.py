@@ -371,6 +371,25 @@ def test_token_by_token_kernel():
         s.finalize()
 
 
+def test_steps_on_the_callers_streams():
+    """Every pass on another stream than the one before: copies and launch follow the caller's, results are the same."""
+    from suborax_helpers import CONFIGS, prompt, weights
+    cfg = CONFIGS["even"]
+    w, toks = weights(cfg), prompt(cfg, 40, seed=5)
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    got = []
+    for turns in (0, 1):
+        s, out = _session(cfg, w, torch.bfloat16), []
+        for k, (a, b) in enumerate([(0, 30), (30, 31), (31, 32), (32, 39), (39, 40)]):
+            with torch.cuda.stream(streams[k % 3 * turns]):
+                lg, greedy = s.step([("r", toks[a:b])], [list(range(b - a))])
+                torch.cuda.current_stream().synchronize()
+            out.append((lg.cpu(), greedy))
+        got.append(out)
+    for (a, x), (b, y) in zip(*got):
+        assert torch.equal(a, b) and x == y
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_mixed_batches_and_pages_used_again(dtype):
     """Unequal requests together, pausing and going on, ending and making room: the logits of every position are those of
