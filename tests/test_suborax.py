@@ -268,6 +268,37 @@ def test_page_pool_and_step_packing():
         s.pool.take(4)
 
 
+def test_ids_that_a_pass_takes():
+    """A pass of an opened session takes what torch makes ids of (tensors of one value among them) and lays it out for one copy."""
+    from mirage.mpk.serving import PagePool, ServingSession
+
+    class Stub:
+        profiler_tensor = None
+
+        def enqueue_steps(self, n, default_stream=None):
+            pass
+
+        def wait(self, default_stream=None):
+            pass
+
+    s = ServingSession.__new__(ServingSession)
+    s.page_size, s.max_rows, s.max_requests, s.rows_per_request, s.max_seq = 4, 8, 3, 8, 64
+    s.pool, s.requests, s.mpk = PagePool(6), {}, Stub()
+    s.mpk.persistent_kernel, s.mpk.output_tokens = Stub(), torch.arange(8)
+    s._dev = torch.zeros(2 * 8 + 4 * 3 + 2 + 6, dtype=torch.int32)
+    host = torch.empty(2 * 8 + len(s._dev), dtype=torch.int32)
+    s._sampled, s._host = host[:16].view(torch.int64), host[16:]
+    for toks in ([7, 8], torch.tensor([7, 8]), torch.tensor([[7], [8]]), [torch.tensor([7]), torch.tensor(8)], torch.tensor([7, 8]).numpy()):
+        s._dev.zero_()
+        assert s.step([("a", [1 << 40]), ("b", toks)])[1] == [0, 2]
+        assert s._dev[:16].view(torch.int64)[:3].tolist() == [1 << 40, 7, 8]
+        s.end("a")
+        s.end("b")
+    for toks in (["7"], [None]):
+        with pytest.raises((TypeError, ValueError)):
+            s.step([("c", toks)])
+
+
 @pytest.mark.parametrize("front", ["residual_rmsnorm", "residual_prenorm", "flex_attention"])
 def test_which_linears_leave_their_sum_to_the_next_stage(front):
     """A split linear leaves whole tiles of 16 columns in rows as long as its output: a ragged last tile would reach into the next row.  Nor
