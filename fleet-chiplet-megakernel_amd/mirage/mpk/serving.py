@@ -172,7 +172,8 @@ class ServingSession:
         desc = qo + [qo[-1]] * pad + kv + [kv[-1]] * pad + last + [0] * pad + slots + [0] * pad + pages
         if self._host is not None:
             n, host = 2 * self.max_rows, self._host.numpy()
-            host[:2 * len(ids)].view("int64")[:] = torch.tensor(ids, dtype=torch.int64).numpy()  # (whatever torch takes for ids, also tensors of one)
+            # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
+            host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
             host[n:n + len(desc)] = desc
             self._dev[:n + len(desc)].copy_(self._host[:n + len(desc)], non_blocking=True)
             pk = m.persistent_kernel
