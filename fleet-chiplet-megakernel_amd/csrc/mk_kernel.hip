@@ -4123,15 +4123,13 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
       }
       const char *vl = vb + lg * GS + lr * 2;
       if constexpr (NEW) {
-        // Positions that only some of the columns see have weight zero in the others, which a product over the tile takes for a value that
-        // is not finite too: such a tile is summed column by column.
+        // A tile with a value that is not finite is summed column by column, each weight in one piece: zero times infinity is no number,
+        // and zero is the weight of positions that only other columns see, and what is left behind the first term of many a weight.
         unsigned top = 0;
-        if (a.n > 1 && q0 + 16 > p_first) {
 #pragma unroll
-          for (int dt = 0; dt < 8; dt++) {
+        for (int dt = 0; dt < 8; dt++) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) top |= (*(const uint16_t *)(vl + dt * 32 + e * 256) & 0x7f80u) + 0x80u;
-          }
+          for (int e = 0; e < 4; e++) top |= (*(const uint16_t *)(vl + dt * 32 + e * 256) & 0x7f80u) + 0x80u;
         }
         if (__builtin_expect(__ballot(top & 0x8000u) != 0, 0)) {
           for (int g = 0; g < 4; g++) {

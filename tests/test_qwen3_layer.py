@@ -177,6 +177,28 @@ def test_a_token_that_is_not_finite_leaves_those_before_it_alone(nkv, L_cached, 
     assert float(((b[:at] - a[:at]).abs() / a[:at].abs().clamp_min(1.0 / 16)).max()) <= 2.0 ** -7
 
 
+@pytest.mark.parametrize("nkv", [8, 4])
+@pytest.mark.parametrize("L_cached,n,at", [(0, 61, 3), (40, 61, 60), (130, 64, 21)])
+def test_an_infinite_value_makes_infinite_outputs(nkv, L_cached, n, at):
+    """One value of one new position overflows: the outputs that see it are infinite (and not NaN), all others finite."""
+    from oracle.qwen3_ref import Qwen3Config
+    cfg = Qwen3Config(hidden_size=1024, num_q_heads=32, num_kv_heads=nkv, head_dim=128, intermediate_size=1536, num_layers=1)
+    dims = (5, 128 * (nkv - 1) + 77)
+
+    def mutate(lw):
+        for r in dims:  # an element of a normalised row is 32 at most, and about that in a row of one element: 1e39; others stay below 5: 1.5e38
+            lw["v_proj"][r, 9] = 3e37
+
+    row = torch.zeros(1024, dtype=torch.bfloat16)
+    row[9] = 1.0
+    res = _run_layer(cfg, L_cached, n, "fleet", seed=11, mutate=mutate, row=(at, row))
+    got = res["attn_gpu"].view(n, 32, 128).float()
+    want = torch.zeros(n, 32, 128, dtype=torch.bool)
+    for r in dims:
+        want[at:, r // 128 * (32 // nkv):(r // 128 + 1) * (32 // nkv), r % 128] = True
+    assert torch.equal(got == float("inf"), want) and bool(got[~want].isfinite().all())
+
+
 def test_full_width_layer_prefill_chunk_mpk_mode():
     from oracle.qwen3_ref import Qwen3Config
     cfg = Qwen3Config(num_layers=1)
