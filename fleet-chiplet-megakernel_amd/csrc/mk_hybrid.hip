@@ -570,8 +570,9 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
       for (int j = 0; j < D; j++) {
         const bool real = k0 + j < a.ke;
         if (ONCE && !REFILL && !real) continue;
+        const u32x4 x = real ? b[j] : zero;  // (both operands: steps behind the share hold values of others, which need not be finite)
 #pragma unroll
-        for (int h = 0; h < 2; h++) acc[h] = fx_mma_k(E(), real ? w[h][j] : zero, b[j], acc[h]);
+        for (int h = 0; h < 2; h++) acc[h] = fx_mma_k(E(), real ? w[h][j] : zero, x, acc[h]);
         if constexpr (REFILL) {
           w[0][j] = ldg_stream(p0 + (size_t)min(kn + j, kl) * 64);
           w[1][j] = ldg_stream(p1 + (size_t)min(kn + j, kl) * 64);

@@ -472,6 +472,28 @@ def test_rows_of_experts_from_memory(dtype, E, top, n, k, shared):
     test_shares_of_the_shared_expert(dtype, E, top, n, k, shared)
 
 
+# reductions whose shares end inside a block of steps, split among four wavefronts, two and none
+@BOTH
+@pytest.mark.parametrize("E,n,k", [(4, 64, 1568), (64, 512, 832), (64, 256, 416), (64, 512, 1600)])
+def test_infinite_values_in_front_of_experts(dtype, E, n, k):
+    """One infinite value in a row, anywhere in it: every output of the row is infinite, with the weight's sign, and of no other row."""
+    ids = (torch.arange(64)[:, None] + torch.arange(2) * (E // 2)) % E
+    pk, t, x, w = _expert_rig(dtype, E, 2, n, k, ids)
+    at = (torch.arange(64) * 97) % k  # spread over the row, its last values among them
+    at[::5] = k - 1
+    odd = torch.arange(64) % 3 != 2
+    t["x"][:64][odd.cuda(), at[odd].cuda()] = float("inf")
+    for M in (64, 5, 1):
+        t["o"].zero_()
+        pk.run_once(list(range(M)), [0] * M)
+        o = t["o"][:M].cpu().double().view(M, 2, n)
+        sign = torch.stack([w[ids[q], :, at[q]].sign() for q in range(M)])
+        assert torch.equal(o[odd[:M]], (sign * float("inf"))[odd[:M]]), M
+        rest = ~odd[:M]
+        torch.testing.assert_close(o[rest], torch.einsum("tsnk,tk->tsn", w[ids[:M]], x[:M])[rest], **_tol(dtype))
+    pk.finalize()
+
+
 # ---------------------------------------------------------------- whole models
 @BOTH
 @pytest.mark.parametrize("name", ["even", "odd", "wide"])
