@@ -637,7 +637,8 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
   };
   const bool early = single && have0 && wave != 0;  // (the polling wavefront keeps its memory queue empty)
   if (early) load_first(a0);
-  if (!single && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the prep stage's rows are read with cached loads
+  // (Keys and values are read with cached loads: a line that holds one of this iteration's positions is read by nobody between the cache
+  // invalidate that opens the iteration and the barrier behind the stage that writes them.)
   barrier_wait(c);
   c.wrote_through = true;
   FxRows<E> rows{};
@@ -1064,7 +1065,8 @@ __device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M,
   f32x4 *red = (f32x4 *)smem;  // [DB ? 2 : 1][waves][NH][MT][64]
   f32x4 *ops = red + (DB ? 2 : 1) * MK_WAVES * NH * MT * 64 + wave * 2 * NT * 128;  // [2][tile][8-row half][8 rows][8 words]
   struct Unit {
-    const f32x4 *row[NT][2];  // this lane's row of either half of a tile
+    const f32x4 *w[NH][2];  // this lane's weight row of either half of a tile
+    int x[MT][2];           // ... token row, in bytes
     int tile, m0;
   };
   auto unit = [&](int u) {
@@ -1076,9 +1078,9 @@ __device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M,
       const int o = min(a.tile * 16 + 8 * i + l8, n_out - 1);
       const int vr = SILU ? (o / half) * 2 * half + (o % half) : o;
 #pragma unroll
-      for (int h = 0; h < NH; h++) a.row[h][i] = (const f32x4 *)weight_row(st.w, vr + h * half, K / 4);
+      for (int h = 0; h < NH; h++) a.w[h][i] = (const f32x4 *)weight_row(st.w, vr + h * half, K / 4);
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) a.row[NH + mt][i] = (const f32x4 *)((const float *)st.in + (size_t)min(a.m0 + mt * 16 + 8 * i + l8, M - 1) * st.ld_in);
+      for (int mt = 0; mt < MT; mt++) a.x[mt][i] = min(a.m0 + mt * 16 + 8 * i + l8, M - 1) * st.ld_in * 4;
     }
     return a;
   };
@@ -1087,28 +1089,32 @@ __device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M,
   if (u0 < u1) a = unit(u0);
   const bool early = u0 < u1 && wave != 0;
   auto word = [&](int s) { return min(4 * s + c8, 4 * nks - 1); };  // this lane's 16-byte word of the step that begins at s (in units of 16 k)
-  auto request = [&](f32x4 (&r)[NT][2], const Unit &p, int s, int t0, int t1) {
+  const auto x_rows = dev_rows(st.in);
+  auto request_w = [&](f32x4 (&r)[NT][2], const Unit &p, int s) {
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-      if (t >= t0 && t < t1) {
+    for (int h = 0; h < NH; h++)
 #pragma unroll
-        for (int i = 0; i < 2; i++) r[t][i] = p.row[t][i][word(s)];
-      }
+      for (int i = 0; i < 2; i++) r[h][i] = p.w[h][i][word(s)];
+  };
+  auto request_x = [&](f32x4 (&r)[NT][2], const Unit &p, int s) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) r[NH + mt][i] = __builtin_bit_cast(f32x4, ldc_16B(x_rows, p.x[mt][i] + 16 * word(s)));
   };
   if (early) {
 #pragma unroll
-    for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, 0, NH);
+    for (int j = 0; j < D; j++) request_w(ring[j], a, kb + 2 * j);
   }
-  if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
   c.wrote_through = true;
   if (u0 >= u1) return;
   if (!early) {
 #pragma unroll
-    for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, 0, NH);
+    for (int j = 0; j < D; j++) request_w(ring[j], a, kb + 2 * j);
   }
 #pragma unroll
-  for (int j = 0; j < D; j++) request(ring[j], a, kb + 2 * j, NH, NT);
+  for (int j = 0; j < D; j++) request_x(ring[j], a, kb + 2 * j);
   f32x4 op[2][NT][2];  // operands of two steps, [tile][16 k]
   auto turn = [&](const f32x4 (&r)[NT][2], f32x4 (&o)[NT][2], int slot) {
     f32x4 *b = ops + slot * NT * 128;
@@ -1135,13 +1141,17 @@ __device__ __forceinline__ void stage_fx_linear_f32_t(CStage &st, Ctx &c, int M,
       const int k0 = kb + blk * 2 * D, kn = last ? kb : k0 + 2 * D, step = last && !more ? 0 : 2;  // (behind the range: one line again and again)
       Unit p;
 #pragma unroll
-      for (int t = 0; t < NT; t++)
+      for (int i = 0; i < 2; i++) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) p.row[t][i] = last ? nx.row[t][i] : a.row[t][i];
+        for (int h = 0; h < NH; h++) p.w[h][i] = last ? nx.w[h][i] : a.w[h][i];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) p.x[mt][i] = last ? nx.x[mt][i] : a.x[mt][i];
+      }
 #pragma unroll
       for (int j = 0; j < D; j++) {
         // operands of the step behind this one, whose place in the ring is then free (the one behind a block's last is its successor's first)
-        request(ring[j], p, kn + step * j, 0, NT);
+        request_w(ring[j], p, kn + step * j);
+        request_x(ring[j], p, kn + step * j);
         turn(ring[(j + 1) % D], op[(j + 1) & 1], (j + 1) & 1);
         const int s = k0 + 2 * j;
 #pragma unroll

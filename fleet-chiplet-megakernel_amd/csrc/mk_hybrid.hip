@@ -489,7 +489,8 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
       w[1][j] = ldg_stream(a.w1 + (size_t)min(a.kb + j, a.nks - 1) * 64);
     }
   int staged = 0x7fffffff, cnt = 1, tok = 0, place = 0;  // rows in LDS belong to this entry; token and place of column lane & 15
-  const E *xr = nullptr;
+  const auto x_rows = dev_rows(st.in);
+  int xr = 0;  // row of column lane & 15 in memory, in bytes
   const u32x4 *xb = xl + lg;
   const u32x4 zero = {0u, 0u, 0u, 0u};
   for (int u = 0; u < n_all; u++) {
@@ -516,7 +517,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
         auto place_of = [&](int t) { return shared ? st.topk : (int)(ls->place[e][t >> 3] >> ((t & 7) * 4) & 15u); };
         tok = token(min(lr, cnt - 1));
         place = place_of(tok);
-        xr = (const E *)st.in + (size_t)tok * st.ld_in + (size_t)place * st.ld_in_slot + lg * EPC;
+        xr = (tok * st.ld_in + place * st.ld_in_slot + lg * EPC) * (int)sizeof(E);
         xb = xl + lg * cnt + min(lr, cnt - 1);
         if constexpr (XLDS) {
           __syncthreads();  // (everybody is done with the rows of the entry before)
@@ -532,7 +533,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
               const bool in = q0 + z * MK_THREADS + tid < total;
               const int t = token(in ? r : 0), j = in ? 4 * b + (tid & 3) : 0;
               at[z] = in ? j * cnt + r : -1;
-              v[z] = *(const u32x4 *)((const E *)st.in + (size_t)t * st.ld_in + (size_t)place_of(t) * st.ld_in_slot + j * EPC);
+              v[z] = ldc_16B(x_rows, (t * st.ld_in + place_of(t) * st.ld_in_slot + j * EPC) * (int)sizeof(E));
               r += dr;
               b += db;
               if (r >= cnt) {
@@ -561,7 +562,7 @@ __device__ __forceinline__ void hy_expert_walk(CStage &st, const Ctx &c, const H
         if (ONCE && !REFILL && k0 + j >= a.ke) continue;
         const int s = min(k0 + j, a.nks - 1);
         if constexpr (XLDS) b[j] = xb[s * 4 * cnt];
-        else b[j] = *(const u32x4 *)(xr + (size_t)s * KW);
+        else b[j] = ldc_16B(x_rows, xr + s * KW * (int)sizeof(E));
       }
       // what the ring takes next: this unit's block or the first one of the unit behind (behind the range: one line again and again)
       const u32x4 *p0 = last ? nx.w0 : a.w0, *p1 = last ? nx.w1 : a.w1;
@@ -681,7 +682,6 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
     for (int i = tid; i < Ex; i += MK_THREADS) ls->tok[i] = 0ull;
     for (int i = tid; i < Ex * (MK_MAX_TOKENS / 8); i += MK_THREADS) ls->place[0][i] = 0u;
   }
-  if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   if (!c.pending) __syncthreads();  // (an iteration's first stage has no barrier to wait for: everybody is done clearing)
   barrier_wait(c);
   // ---- which experts have which tokens
@@ -699,9 +699,17 @@ __device__ __forceinline__ void stage_hy_experts(CStage &st, Ctx &c, int M, char
     } else {
       u32x4 *xl = (u32x4 *)(smem + HY_X);
       const int total = one_rows * one_words;
-      for (int q = tid - 64; q < total; q += MK_THREADS - 64) {
-        const int p = q / one_words, j = q - p * one_words;
-        xl[q] = *(const u32x4 *)((const E *)st.in + (size_t)p * st.ld_in_slot + min(j, (p == topk ? st.k_shared : one_rows == 1 ? one_words * EPC : st.k) / EPC - 1) * EPC);
+      const auto x_rows = dev_rows(st.in);
+      for (int q0 = tid - 64; q0 < total; q0 += 4 * (MK_THREADS - 64)) {
+        u32x4 v[4];
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+          const int q = min(q0 + z * (MK_THREADS - 64), total - 1), p = q / one_words, j = q - p * one_words;
+          v[z] = ldc_16B(x_rows, p * st.ld_in_slot * (int)sizeof(E) + 16 * min(j, (p == topk ? st.k_shared : one_rows == 1 ? one_words * EPC : st.k) / EPC - 1));
+        }
+#pragma unroll
+        for (int z = 0; z < 4; z++)
+          if (q0 + z * (MK_THREADS - 64) < total) xl[q0 + z * (MK_THREADS - 64)] = v[z];
       }
     }
     __syncthreads();

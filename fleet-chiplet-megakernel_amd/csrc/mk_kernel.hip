@@ -250,6 +250,10 @@ __device__ __forceinline__ u32x4 ldc_16B(const u32x4 *p) {
 // request carries half of the lines it touches: a row of 4096 summed from four slices, as a norm stage, 7.5 -> 5.4 us; 32-bit 6.0 -> 4.2).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_rows(const void *p) { return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 0xffffffffu, 0x00027000); }
 __device__ __forceinline__ u32x4 ldc_16B(__amdgpu_buffer_rsrc_t rows, int off) { return __builtin_amdgcn_raw_buffer_load_b128(rows, off, 0, 16 /* sc1 */); }
+// (They share what they bring through the die's L2 as ordinary loads do: 64 KB of rows into the LDS of every CU in 1.09 us either way, 512 KB in
+// 6.4; an acquire in front, which ordinary loads of another workgroup's rows need, takes another 1.8 us and what the L2 held for the next CU
+// with it.  So stages of several tokens read rows like this too: dodonex-8b 59.7 -> 57.1 ms, suborax-8b serving 122.2 -> 118.7, 64 streams of
+// qwen3-8b 286.2 -> 281.4.)
 // Stores that are written through to memory (device scope), for outputs of stages that skip the L2 write-back at
 // their barrier.
 __device__ __forceinline__ void stc_u16(uint16_t *p, uint16_t v) {
@@ -280,6 +284,21 @@ __device__ __forceinline__ void stc_bf16x4(uint16_t *row, int n0, int n_out, con
 #pragma unroll
     for (int i = 0; i < 4; i++)
       if (n0 + i < n_out) stc_u16(p + i, (uint16_t)f2bf(r[i]));
+  }
+}
+__device__ __forceinline__ uint16_t ldc_half(const uint16_t *p) { return __hip_atomic_load((const MK_GLOBAL uint16_t *)(unsigned long long)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// the same four as 32-bit values (columns behind the row's end: not read)
+__device__ __forceinline__ void ldc_bf16x4(const uint16_t *row, int n0, int n_out, float (&r)[4]) {
+  const uint16_t *p = row + n0;
+  if (n0 + 3 < n_out && (((unsigned long long)p) & 7) == 0) {
+    const unsigned long long u = ldc_u64(p);
+    r[0] = bf_lo((uint32_t)u);
+    r[1] = bf_hi((uint32_t)u);
+    r[2] = bf_lo((uint32_t)(u >> 32));
+    r[3] = bf_hi((uint32_t)(u >> 32));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = n0 + i < n_out ? bf2f(ldc_half(p + i)) : 0.f;
   }
 }
 __device__ __forceinline__ uint16_t ldc_u16(const uint16_t *p) {
@@ -1471,7 +1490,7 @@ __device__ __forceinline__ void stage_linear_small(CStage &st, Ctx &c, int M, ch
   auto load_group = [&](int o, u32x4 (&b)[Q][NROW][KL], uint16_t &r) {
 #pragma unroll
     for (int q = 0; q < Q; q++) load_unit(max(min(o + q, o_end - 1), 0), b[q]);
-    r = rbase[has_res ? max(min(o + ((lane / MB) & (Q - 1)), o_end - 1), 0) : 0];
+    r = ldc_half(rbase + (has_res ? max(min(o + ((lane / MB) & (Q - 1)), o_end - 1), 0) : 0));
   };
   u32x4 bufA[Q][NROW][KL], bufB[Q][NROW][KL];
   uint16_t rA = 0, rB = 0;
@@ -1483,8 +1502,6 @@ __device__ __forceinline__ void stage_linear_small(CStage &st, Ctx &c, int M, ch
     load_group(gB, bufB, rB);
   } else {
     if (c.pending && tid == 0) barrier_poll(c);
-    // the token rows come from other workgroups: one acquire, then ordinary loads that share them through the die's L2
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
   barrier_done(c);
@@ -1499,10 +1516,10 @@ __device__ __forceinline__ void stage_linear_small(CStage &st, Ctx &c, int M, ch
     // normalised rows, which are the norm task's output tensor.
     const u32x4 *nw4 = (const u32x4 *)st.norm_w;
     for (int m = wave; m < M; m += MK_WAVES) {
-      const u32x4 *xr = (const u32x4 *)(x + (size_t)m * ldx);
+      const auto xr = dev_rows(x + (size_t)m * ldx);
       u32x4 v[KL];
 #pragma unroll
-      for (int kc = 0; kc < KL; kc++) v[kc] = xr[kc * 64 + lane];
+      for (int kc = 0; kc < KL; kc++) v[kc] = ldc_16B(xr, (kc * 64 + lane) * 16);
       float ss = 0.f;
 #pragma unroll
       for (int kc = 0; kc < KL; kc++) {
@@ -1531,7 +1548,7 @@ __device__ __forceinline__ void stage_linear_small(CStage &st, Ctx &c, int M, ch
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
       const int ci = (i * MK_WAVES + wave) * 64 + lane, m = ci / K8, o = ci - m * K8;
-      if (m < M) xv[i] = ((const u32x4 *)(x + (size_t)m * ldx))[o];
+      if (m < M) xv[i] = ldc_16B(dev_rows(x), m * ldx * 2 + o * 16);
     }
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
@@ -1705,8 +1722,6 @@ template <int MT>
 __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, const MkRuntime &rt, int M, const TilePlan plan, char *smem) {
   barrier_wait(c);
   c.wrote_through = true;  // partial tiles and outputs are all written through: no L2 write-back at this stage's arrival
-  if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  __syncthreads();
   MK_MARK(c, 0);
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
@@ -1727,7 +1742,8 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
   int *sflag = (int *)(smem + 2 * MT * 2048);
   // token rows: wavefront w stages token tile w, every lane the same 32 contiguous bytes it would feed the matrix core
   // with, stored at its own lane slot of the operand block (consecutive 16-byte slots: no bank conflicts either way)
-  const uint16_t *xsrc = x + (size_t)min(min(wave, MT - 1) * 16 + lr, M - 1) * ldx + kbeg + lg * 16;
+  const auto xrows = dev_rows(x);
+  const int xsrc = (min(min(wave, MT - 1) * 16 + lr, M - 1) * ldx + kbeg + lg * 16) * 2;  // bytes
   const int xdst = min(wave, MT - 1) * 128 + lane;
   // first weight row of weight tile ti for this lane
   auto tile_row = [&](int ti) -> const uint16_t * {
@@ -1762,8 +1778,8 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
       }
     };
     auto x_load = [&](int step, u32x4 (&q)[2]) {
-      q[0] = *(const u32x4 *)(xsrc + (step << 6));
-      q[1] = *(const u32x4 *)(xsrc + (step << 6) + 8);
+      q[0] = ldc_16B(xrows, xsrc + (step << 7));
+      q[1] = ldc_16B(xrows, xsrc + (step << 7) + 16);
     };
     auto x_store = [&](int buf, const u32x4 (&q)[2]) {
       if (wave < MT) {
@@ -1889,14 +1905,14 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
         if (m < M) {
           uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
           const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
-          float rr[4];
+          float rr[4], res[4];
+          if (st.flags & MK_F_RES) ldc_bf16x4(rrow, otile * 16 + lg * 4, n_out, res);
 #pragma unroll
           for (int i = 0; i < 4; i++) {
-            const int n = otile * 16 + lg * 4 + i;
             float r;
             if (silu) r = TW >= 2 ? linear_glu(st, acc[(2 * u) % TW][mt][i], acc[(2 * u + 1) % TW][mt][i]) : 0.f;
             else r = acc[u][mt][i];
-            if ((st.flags & MK_F_RES) && n < n_out) r += bf2f(rrow[n]);
+            if (st.flags & MK_F_RES) r += res[i];
             rr[i] = linear_act(st, r);
           }
           stc_bf16x4(orow, otile * 16 + lg * 4, n_out, rr);
@@ -2046,8 +2062,8 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     for (int i = w; i < MT * NSP; i += nw) {
       const int step = i / MT, mt = i - step * MT, r0 = mt * 16 + (lane >> 3);
       __attribute__((address_space(3))) char *dst = (__attribute__((address_space(3))) char *)(buf + (size_t)i * 128);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0 + 8, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 16 /* sc1 */);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0 + 8, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 16);
     }
   };
 
@@ -2076,16 +2092,11 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
 #pragma unroll
       for (int j = 0; j < NBP; j++) w_load(wrow, j, a[j]);
     }
-    // Token rows come from other workgroups and are read with cached loads, so what this die's caches hold of them must
-    // go first.  The invalidate is issued BEFORE the barrier is awaited: nothing on this die reads the stage's input
-    // buffers between the stage that last consumed them (barriers ago) and this barrier, so no stale line can come
-    // back in between, and the invalidate's latency is off the path from the last arrival to the first row request.
     // The poll runs on the first row-staging wavefront, which has no weight loads in flight: loads return in order, so
     // on a streaming wavefront the poll's answer would wait behind the NB steps just requested -- two to four
     // microseconds for exactly the workgroups that enter last (those that did the norm stage's rows, or everybody after
     // an attention stage), which are the ones the stage then waits for.
     constexpr int POLL_TID = NSW * 64;
-    if (tid == POLL_TID) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     if (c.pending && tid == POLL_TID) barrier_poll(c);
     __syncthreads();
     barrier_done(c);
@@ -2172,12 +2183,12 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
           if (m < M) {
             uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
             const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
-            float rr[4];
+            float rr[4], res[4];
+            if (st.flags & MK_F_RES) ldc_bf16x4(rrow, otile * 16 + lg * 4, n_out, res);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-              const int n = otile * 16 + lg * 4 + i;
               float r = v[mt][i];
-              if ((st.flags & MK_F_RES) && n < n_out) r += bf2f(rrow[n]);
+              if (st.flags & MK_F_RES) r += res[i];
               rr[i] = linear_act(st, r);
             }
             stc_bf16x4(orow, otile * 16 + lg * 4, n_out, rr);
@@ -2315,10 +2326,6 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
 // on 256 workgroups) spend the registers on depth instead: <2, MK_TUNE_NBN>.
 template <int MT, int TG, int NB>
 __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, char *smem) {
-  // activations were produced by other workgroups: drop what this die's caches hold of them once, then use cached loads
-  // so the rows are shared through the die's L2.  (Issued before the barrier is awaited: nothing on this die reads
-  // the stage's input buffers between their previous consumer and this barrier.)
-  if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
   c.wrote_through = true;  // outputs are written through: no L2 write-back at this stage's arrival
   MK_MARK(c, 0);
@@ -2344,9 +2351,10 @@ __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, cha
   const bool packed = pipe && st.wpack != nullptr;
   const int wstep = packed ? 128 : 8, whalf = packed ? 64 : 1;  // 16-byte operands between steps / between the halves
   const int xhalf = packed ? 32 : 8;                           // elements between the halves of a token-row step
-  const uint16_t *xrow[MT];
+  const auto xrows = dev_rows(x);
+  int xrow[MT];  // bytes
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++) xrow[mt] = x + (size_t)min(mt * 16 + lr, M - 1) * ldx + (packed ? lg * 8 : lg * lgw);
+  for (int mt = 0; mt < MT; mt++) xrow[mt] = (min(mt * 16 + lr, M - 1) * ldx + (packed ? lg * 8 : lg * lgw)) * 2;
 
   for (int ot0 = t_begin; ot0 < t_end; ot0 += otg) {
     const int not_ = min(otg, t_end - ot0);       // output tiles in this sweep
@@ -2385,8 +2393,8 @@ __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, cha
           }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-          bb[mt][0] = *(const bf16x8 *)(xrow[mt] + k);
-          bb[mt][1] = *(const bf16x8 *)(xrow[mt] + k + xhalf);
+          bb[mt][0] = __builtin_bit_cast(bf16x8, ldc_16B(xrows, xrow[mt] + 2 * k));
+          bb[mt][1] = __builtin_bit_cast(bf16x8, ldc_16B(xrows, xrow[mt] + 2 * (k + xhalf)));
         }
       };
 #pragma unroll
@@ -2416,7 +2424,7 @@ __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, cha
         for (int t = 0; t < TG; t++)
           if (t < nt) a[t] = __builtin_nontemporal_load((const bf16x8 *)(wrow[t] + k));
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) b[mt] = *(const bf16x8 *)(xrow[mt] + k);
+        for (int mt = 0; mt < MT; mt++) b[mt] = __builtin_bit_cast(bf16x8, ldc_16B(xrows, xrow[mt] + 2 * k));
 #pragma unroll
         for (int t = 0; t < TG; t++)
           if (t < nt) {
@@ -2456,12 +2464,12 @@ __device__ __forceinline__ void stage_linear_mfma(CStage &st, Ctx &c, int M, cha
       if (m < M) {
         uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
         const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
-        float rr[4];
+        float rr[4], res[4];
+        if (st.flags & MK_F_RES) ldc_bf16x4(rrow, n0, n_out, res);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const int n = n0 + i;
           float r = silu ? linear_glu(st, v[i], v2[i]) : v[i];
-          if ((st.flags & MK_F_RES) && n < n_out) r += bf2f(rrow[n]);
+          if (st.flags & MK_F_RES) r += res[i];
           rr[i] = linear_act(st, r);
         }
         stc_bf16x4(orow, n0, n_out, rr);
@@ -2639,8 +2647,7 @@ __device__ __forceinline__ void moe_build_lists(CStage &st, const Ctx &c, MoeLds
     __syncthreads();
     return;
   }
-  // the expert's row of the routing table, all requested at once (the multi-token callers have done their acquire,
-  // but the table is tiny: device-scope loads keep this correct for any caller)
+  // the expert's row of the routing table, all requested at once
   int rv[MK_MAX_TOKENS];
   int cnt = 0;
   if (tid < E) {
@@ -3197,9 +3204,8 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
   if (early) fill();
   if (!SILU && reuse) {
     barrier_wait(c);
-    if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __syncthreads();
   }
+  const auto x_rows = dev_rows(st.in);
   if (plain) {
     // too many tokens on this workgroup's experts for the LDS windows: plain form over the same unit range
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3209,13 +3215,13 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
       const size_t e = (size_t)L->act_e[a];
       for (int p = L->pair_off[a]; p < L->pair_off[a + 1]; p++) {
         const int ts = L->pair_ts[p], tok = ts & 255, slot = ts >> 8;
-        const u32x4 *x = (const u32x4 *)((const uint16_t *)st.in + (size_t)tok * st.ld_in + (size_t)slot * st.ld_in_slot);
+        const int x = (tok * st.ld_in + slot * st.ld_in_slot) * 2;  // bytes
         float acc[NROW];
 #pragma unroll
         for (int h = 0; h < NROW; h++) {
           acc[h] = 0.f;
           const u32x4 *wr = W + (e * st.n + (size_t)(j + h * NR)) * k8;
-          for (int kc = lane; kc < k8; kc += 64) acc[h] = dot8(wr[kc], x[kc], acc[h]);
+          for (int kc = lane; kc < k8; kc += 64) acc[h] = dot8(wr[kc], ldc_16B(x_rows, x + kc * 16), acc[h]);
           acc[h] = wave_sum(acc[h]);
         }
         uint16_t *y = out + (size_t)tok * st.ld_out + (size_t)slot * st.ld_out_slot;
@@ -3312,10 +3318,17 @@ __device__ __forceinline__ void stage_moe_linear_multi(CStage &st, Ctx &c, int M
     }
   };
   // stage the input rows of the (token, slot) pairs of this workgroup's experts
-  for (int i = tid; i < n_pairs * k8; i += MK_THREADS) {
-    const int p = i / k8, o = i - p * k8;
-    const int ts = L->pair_ts[p_base + p], tok = ts & 255, slot = ts >> 8;
-    xs4[i] = ((const u32x4 *)((const uint16_t *)st.in + (size_t)tok * st.ld_in + (size_t)slot * st.ld_in_slot))[o];
+  for (int i0 = tid; i0 < n_pairs * k8; i0 += 4 * MK_THREADS) {
+    u32x4 v[4];
+#pragma unroll
+    for (int z = 0; z < 4; z++) {
+      const int i = min(i0 + z * MK_THREADS, n_pairs * k8 - 1), p = i / k8, o = i - p * k8;
+      const int ts = L->pair_ts[p_base + p], tok = ts & 255, slot = ts >> 8;
+      v[z] = ldc_16B(x_rows, (tok * st.ld_in + slot * st.ld_in_slot) * 2 + o * 16);
+    }
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+      if (i0 + z * MK_THREADS < n_pairs * k8) xs4[i0 + z * MK_THREADS] = v[z];
   }
   __syncthreads();
   if (nu > 0) {
@@ -3365,7 +3378,7 @@ __device__ __forceinline__ void stage_moe_linear(CStage &st, Ctx &c, int M, char
     }
   }
   if (M > 1) {
-    // common front: wait for the previous stage, one acquire (activation rows are read with cached loads), routing lists.  Directly behind
+    // common front: wait for the previous stage, routing lists.  Directly behind
     // another expert linear over the same routing table (W2 behind W13) the lists are still in LDS: that stage starts its stream ahead of the
     // barrier.  qwen3-30b-a3b, 16 tokens, W2: 61 -> 51 us.  (Rows of up to 1024 only: in the instances for longer ones, which have no such
     // stage here, it moved the register allocation of the multi-token linears, a prompt of qwen3-8b 50.1 -> 50.7 ms.)
@@ -3377,8 +3390,6 @@ __device__ __forceinline__ void stage_moe_linear(CStage &st, Ctx &c, int M, char
     }
     if (!reuse) {
       barrier_wait(c);
-      if (c.tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      __syncthreads();
       moe_build_lists(st, c, L, M, false);
     }
     if (!(reuse && (&st)[-1].moe_mask == st.moe_mask) && c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)

@@ -832,13 +832,13 @@ __device__ __forceinline__ void stage_mx_head_linear_t(CStage &st, Ctx &c, int M
   // weights do not depend on the previous stage: the first tile's are requested before its barrier completes
   const bool early = i0 < items && wave != 0;
   if (early) load_w(i0, kb);
-  if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   barrier_wait(c);
+  const auto x_rows = dev_rows(st.in);
   for (int i = i0; i < items; i += di) {
     const int tile = i / mts, mt0 = i - tile * mts, h = tile / nt, n0 = (tile - h * nt) * 16 + lg * 4;
-    const E *xr[MT];
+    int xr[MT];  // bytes
 #pragma unroll
-    for (int m = 0; m < MT; m++) xr[m] = (const E *)st.in + (size_t)min((mt0 + m) * 16 + lr, M - 1) * st.ld_in + (size_t)h * st.ld_in_slot + lg * EPC;
+    for (int m = 0; m < MT; m++) xr[m] = (min((mt0 + m) * 16 + lr, M - 1) * st.ld_in + h * st.ld_in_slot + lg * EPC) * (int)sizeof(E);
     f32x4 acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; m++) acc[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -848,7 +848,7 @@ __device__ __forceinline__ void stage_mx_head_linear_t(CStage &st, Ctx &c, int M
 #pragma unroll
       for (int j = 0; j < KB; j++)
 #pragma unroll
-        for (int m = 0; m < MT; m++) b[j][m] = *(const u32x4 *)(xr[m] + (size_t)min(k0 + j, nks - 1) * KW);
+        for (int m = 0; m < MT; m++) b[j][m] = ldc_16B(x_rows, xr[m] + min(k0 + j, nks - 1) * KW * (int)sizeof(E));
 #pragma unroll
       for (int j = 0; j < KB; j++) {
         const u32x4 w = k0 + j < ke ? a[j] : zero;
@@ -1060,7 +1060,8 @@ __device__ __forceinline__ void stage_mx_latent_attn_t(CStage &st, Ctx &c, const
   // the first tile is requested before the barrier is awaited when earlier iterations wrote all of it
   const bool early = have0 && wave != 0 && a0.tb < a0.te && (a0.tb + 1) * TPOS <= a0.p0;
   if (early) load_tile(a0.tb, rt.kv_indices[a0.pages + a0.tb * TPOS / ps]);
-  if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // rows of this iteration are read with cached loads
+  // (Latents are read with cached loads: a line that holds one of this iteration's positions is read by nobody between the cache invalidate
+  // that opens the iteration and the barrier behind the stage that writes them.)
   barrier_wait(c);
   const float sc1 = st.sm_scale * 1.4426950408889634f;
   for (int u = u0; u < n_units; u += c.G) {
