@@ -4641,7 +4641,13 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
             const TilePlan plan = linear_tiles_plan(st, c);
             const XresPlan xp = linear_xres_plan(st, c);
             if (xp.S >= 1 && (M > MK_TUNE_SMALL_MAX || packed_only)) {
-              if (M <= 32) {
+              // as many token tiles as the rows need: rows behind the last token are staged, multiplied and left to the next stage like the others
+              // (4 tokens with one tile instead of two, us: 6144 x 4096 11.7 -> 10.8, 4096 x 4096 9.8 -> 8.8, 4096 x 12288 19.8 -> 18.6; a third of
+              // 48 instead of 64 would be another pair of instances for fewer batches)
+              if (M <= 16) {
+                if (xp.tpu <= 4) stage_linear_mfma_xres<1, 2>(st, c, rt, M, xp, smem);
+                else stage_linear_mfma_xres<1, 3>(st, c, rt, M, xp, smem);
+              } else if (M <= 32) {
                 if (xp.tpu <= 4) stage_linear_mfma_xres<2, 2>(st, c, rt, M, xp, smem);
                 else stage_linear_mfma_xres<2, 3>(st, c, rt, M, xp, smem);
               } else {
