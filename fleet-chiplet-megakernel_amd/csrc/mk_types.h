@@ -278,6 +278,7 @@ enum MkSchedMode {
   MK_SCHED_OFFLINE = 1,      // on-GPU continuous batching over `tokens` (MODE_OFFLINE)
   MK_SCHED_FROM_META = 2,    // derived on the GPU from the qo / paged-kv meta tensors the host filled (MODE_ONLINE_NOTOKEN, MODE_ONEPASS)
   MK_SCHED_ONLINE = 3,       // one request, host-written tokens consumed num_new_tokens[0] at a time (MODE_ONLINE)
+  MK_SCHED_INGEST = 4,       // MK_SCHED_FROM_META, and nobody reads the logits or sampled tokens of the batch (mk_enqueue_ingest)
 };
 
 // Scheduler state that persists across launches (continuous batching, page ring).
@@ -287,13 +288,15 @@ struct MkSched {
   int bad_batch;          // host-described batch (MK_SCHED_FROM_META) that was rejected instead of run: 0 = fine, else the reason
 
   long long iterations;   // decode iterations executed so far (all launches)
-  long long pad2;
+  int inner;              // every row of the iteration lies in front of its prompt's last token (portions of several tokens only)
+  int pad2;
 };
 
 struct MkRuntime {
   int num_stages, max_tokens, max_requests, max_seq;
   int page_size, max_pages, total_requests, max_new_per_req;
-  int spec_len, pad_spec;  // speculative candidates a decoding request brings into an iteration beside its newest token (0: none)
+  int spec_len;  // speculative candidates a decoding request brings into an iteration beside its newest token (0: none)
+  int tail;      // first of the stages at the end that leave nothing for later iterations: only logits and sampled tokens need them
   long long eos_token_id;
   // meta tensors (persistent_kernel.py:2590-2600 order)
   int *step;

@@ -25,7 +25,7 @@ MK_MODES = {"offline": 0, "online": 1, "online_notoken": 2, "onepass": 3}
 EXPORTED_SYMBOLS = [
     "mk_graph_create", "mk_graph_destroy", "mk_tensor_attach", "mk_tensor_new", "mk_tensor_shuffle",
     "mk_tensor_num_dims", "mk_tensor_dim", "mk_tensor_ptr", "mk_add_task", "mk_generate_task_graph",
-    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_wait",
+    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_wait",
     "mk_run_once", "mk_repack_weights", "mk_tensor_releasable", "mk_set_profiler", "mk_get_stats", "mk_get_stage_profile", "mk_get_stage_marks", "mk_describe_program", "mk_last_error", "mk_version",
 ]
 
@@ -114,6 +114,7 @@ def load():
     lib.mk_launch_steps.argtypes = [vp, vp, ci, cip]
     lib.mk_enqueue_steps.argtypes = [vp, vp, ci]
     lib.mk_enqueue_steps_static.argtypes = [vp, vp, ci]
+    lib.mk_enqueue_ingest.argtypes = [vp, vp]
     lib.mk_wait.argtypes = [vp, vp, cip]
     i32p = ctypes.POINTER(ctypes.c_int32)
     lib.mk_run_once.argtypes = [vp, vp, ci, i32p, i32p, i32p]
@@ -220,6 +221,9 @@ class Graph:
     def enqueue_steps(self, stream, max_iterations, static=False):
         fn = self._lib.mk_enqueue_steps_static if static else self._lib.mk_enqueue_steps
         check(fn(self._h, ctypes.c_void_p(stream), int(max_iterations)))
+
+    def enqueue_ingest(self, stream):
+        check(self._lib.mk_enqueue_ingest(self._h, ctypes.c_void_p(stream)))
 
     def wait(self, stream) -> bool:
         fin = ctypes.c_int(0)

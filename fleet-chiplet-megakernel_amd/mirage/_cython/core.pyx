@@ -203,6 +203,9 @@ cdef class CyGraph:
         else:
             _check(mk.mk_enqueue_steps(self.g, s, max_iterations))
 
+    def enqueue_ingest(self, stream):
+        _check(mk.mk_enqueue_ingest(self.g, <void *><uintptr_t>(stream or 0)))
+
     def wait(self, stream) -> bool:
         cdef int rc, fin = 0
         cdef void *s = <void *><uintptr_t>(stream or 0)

@@ -60,6 +60,7 @@ cdef extern from "fleet_mk.h" nogil:
     int mk_launch_steps(mk_graph *g, void *stream, int max_iterations, int *finished_out)
     int mk_enqueue_steps(mk_graph *g, void *stream, int max_iterations)
     int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations)
+    int mk_enqueue_ingest(mk_graph *g, void *stream)
     int mk_wait(mk_graph *g, void *stream, int *finished_out)
     int mk_run_once(mk_graph *g, void *stream, int num_tokens, const int32_t *tok_slot, const int32_t *tok_pos, const int32_t *tok_first)
     int mk_repack_weights(mk_graph *g)

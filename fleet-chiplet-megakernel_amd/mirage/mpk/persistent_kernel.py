@@ -1077,6 +1077,10 @@ class PersistentKernel:
     def enqueue_steps(self, max_iterations: int, default_stream=None):
         self._g.enqueue_steps(self._stream_ptr(default_stream), int(max_iterations))
 
+    def enqueue_ingest(self, default_stream=None):
+        """enqueue_steps(1) over a batch that the host describes and whose logits and sampled tokens nobody reads."""
+        self._g.enqueue_ingest(self._stream_ptr(default_stream))
+
     def wait(self, default_stream=None) -> bool:
         return self._g.wait(self._stream_ptr(default_stream))
 

@@ -50,6 +50,7 @@ class ServingSession:
     # sampled tokens, so that a pass waits for the device once (a pageable copy in either direction costs 12 to 16 us, of which a pass had
     # three; one copy per wanted row of logits another 8 each: a decode step of 16 requests spent 280 us outside the launch, now 85)
     _host = _dev = _sampled = None
+    _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
     def __init__(self, mpk: MPK):
         if mpk.metadata.mode != "online_notoken":
@@ -118,6 +119,8 @@ class ServingSession:
                     room -= n
             if not batch:
                 break
+            # (portions in the middle of their prompts, of which no row is wanted)
+            self._unread = all(done[i] + n < len(entries[i][1]) and not any(done[i] <= p < done[i] + n for p in found[i]) for i, n in batch)
             sampled = self._pass([(entries[i][0], entries[i][1][done[i]:done[i] + n]) for i, n in batch])
             row, wanted = 0, []
             for i, n in batch:
@@ -146,7 +149,7 @@ class ServingSession:
         return torch.stack([r[k] for r, k in rows]), greedy
 
     def _pass(self, batch):
-        ps = self.page_size
+        ps, unread, self._unread = self.page_size, self._unread, False
         ids, qo, kv, last, slots, pages = [], [0], [0], [], [], []
         for rid, toks in batch:
             r = self.requests.get(rid)
@@ -181,6 +184,10 @@ class ServingSession:
                 m()
                 return None
             stream = torch.cuda.current_stream(self._dev.device) if self._dev.is_cuda else None  # (the copies', whichever device is current)
+            if unread:
+                pk.enqueue_ingest(default_stream=stream)
+                pk.wait(default_stream=stream)
+                return None
             pk.enqueue_steps(1, default_stream=stream)
             self._sampled.copy_(m.output_tokens.view(-1), non_blocking=True)
             pk.wait(default_stream=stream)
