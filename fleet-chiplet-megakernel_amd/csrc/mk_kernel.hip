@@ -3476,14 +3476,14 @@ struct AttnSource {
 // Rows [0, n) by the workgroup, RF per wavefront in flight.  Bound by round trips: everything a row needs is requested before the first
 // value is waited for (the row, then its norm weights, then its rotation had made it three, and a branch around each row as many more).
 // own(tok): an unsummed row of this token is also stored where the linear would have.
-template <int RF, typename Row, typename Own>
+template <int RF, int NW = MK_WAVES, typename Row, typename Own>
 __device__ __forceinline__ void attn_rows(CStage &st, const AttnSource &src, int n, int lane, int wave, Row row, Own own) {
-  for (int i0 = MK_WAVES - 1 - wave; i0 < n; i0 += RF * MK_WAVES) {
+  for (int i0 = NW - 1 - wave; i0 < n; i0 += RF * NW) {
     AttnRow a[RF];
     uint16_t cs[RF], sn[RF];
     float x[RF][2];
 #pragma unroll
-    for (int r = 0; r < RF; r++) a[r] = row(min(i0 + r * MK_WAVES, n - 1));
+    for (int r = 0; r < RF; r++) a[r] = row(min(i0 + r * NW, n - 1));
     if (st.flags & MK_F_ROPE) {
 #pragma unroll
       for (int r = 0; r < RF; r++) {
@@ -3535,7 +3535,7 @@ __device__ __forceinline__ void attn_rows(CStage &st, const AttnSource &src, int
     }
 #pragma unroll
     for (int r = 0; r < RF; r++) {
-      if (i0 + r * MK_WAVES >= n) break;
+      if (i0 + r * NW >= n) break;
       float x0 = x[r][0], x1 = x[r][1];
       if (src.S && own(a[r].tok)) {
         uint16_t *d = src.in + (size_t)a[r].tok * src.ld + a[r].off;
@@ -3960,6 +3960,23 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 }
 
 
+#define MK_ATTN_PAIR_PAGES 1024  // page-table entries of a request where a workgroup works on two units at a time
+#ifndef MK_TUNE_ATTN_SPREAD
+#define MK_TUNE_ATTN_SPREAD 384
+#endif
+// Whether a workgroup takes two units at a time (below): there are more of them than workgroups, and the longest context is not far above
+// the average, which two wavefronts walk in twice the time that four take.  64 requests, 32 q / 8 kv heads, as a stage, one unit after the
+// other -> two at a time, us: contexts of 320 32.0 -> 24.0; of 100 .. 700 (300 above the average) 35.0 -> 34.3; 63 of 20 and one of 300 22.8 ->
+// 19.9; of 100 .. 1480 (690 above) 49.2 -> 60.7; 63 of 20 and one of 900 33.6 -> 40.3.
+template <int QPK>
+__device__ __forceinline__ bool attn_in_pairs(CStage &st, const Ctx &c, const MkRuntime &rt, int M) {
+  const int lane = threadIdx.x & 63, first = lane < M ? c.sh_tok[2 * MK_MAX_TOKENS + lane] : 0;
+  if (__popcll(__ballot(lane < M && (lane - first) % (16 / QPK) == 0)) * st.num_kv_heads <= c.G || (rt.max_seq + rt.page_size - 1) / rt.page_size > MK_ATTN_PAIR_PAGES) return false;
+  const int pos = lane < M ? c.sh_tok[lane] : 0;
+  const float mean = wave_sum((float)pos) / (float)M;
+  return !__any((float)pos > mean + (float)MK_TUNE_ATTN_SPREAD);
+}
+
 // The same for iterations of many tokens, on the matrix cores.  Work unit = (up to 16 / QPK consecutive tokens of one request, kv head,
 // KV chunk): their query rows are the 16 columns of a tile product, so a prompt's tokens share what is read of the cache.  One wavefront
 // per tile of 16 positions; the new positions of the iteration are tiles as well, out of LDS.
@@ -3975,22 +3992,28 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 // are few tiles, with all of their 24 bits (three).  The B operand -- four consecutive positions of one dim -- is read out of the V tile in LDS.  The running maximum is kept per column for the whole wavefront, the running sum per lane.
 // K and V tiles are four groups of four rows of 256 bytes, one direct-to-LDS request per group (each lane 16 bytes: four whole rows), the
 // groups GS bytes apart (the transposed V reads of the four groups then fall into different banks).
-template <int QPK>
+template <int QPK, bool PAIR>
 __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   constexpr int D = 128, NC = 16, TG = NC / QPK, RB = 2, PD = 132;
+  constexpr int SUBS = PAIR ? 2 : 1, SW = MK_WAVES / SUBS, ST = SW * 64;  // units at a time, wavefronts and threads of one
   constexpr int GS = 1088, TS = 4 * GS, SLOT = 2 * TS, NEW_BYTES = MK_MAX_NEW_PER_REQ / 4 * GS;
-  constexpr int FLAG_OFF = NC * D * 2, KN_OFF = FLAG_OFF + 64, VN_OFF = KN_OFF + NEW_BYTES, PART_OFF = VN_OFF + NEW_BYTES, BUF_OFF = PART_OFF + MK_WAVES * NC * PD * 4;
+  // LDS: query rows, new rows and page list of every unit, then the tiles of every wavefront.  The wavefronts' partial results have an area
+  // of their own, which the page list shares, or, with two units, lie where the wavefront's tiles were.
+  constexpr int FLAG_OFF = SUBS * NC * D * 2, KN_OFF = FLAG_OFF + 64, PART_OFF = KN_OFF + SUBS * 2 * NEW_BYTES;
+  constexpr int BUF_OFF = PART_OFF + (PAIR ? SUBS * MK_ATTN_PAIR_PAGES * 4 : MK_WAVES * NC * PD * 4);
   static_assert(BUF_OFF + MK_WAVES * RB * SLOT <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
   static_assert(MK_ATTN_MAX_REQ_PAGES * 4 <= MK_WAVES * NC * PD * 4, "page list exceeds the area it aliases");
+  static_assert(NC * PD * 4 <= RB * SLOT, "partial results exceed the tiles they follow");
   static_assert(PART_OFF % 16 == 0 && BUF_OFF % 16 == 0 && KN_OFF % 16 == 0, "16-byte operands");
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int sub = wave / SW, sw = wave % SW, stid = tid % ST;  // which unit, wavefront and thread of it
   const int nkv = st.num_kv_heads, ps = rt.page_size;
-  uint16_t *qs = (uint16_t *)smem;                                 // [16][128]
+  uint16_t *qs = (uint16_t *)smem + sub * NC * D;                  // [16][128]
   int *sflag = (int *)(smem + FLAG_OFF);
-  char *knew = smem + KN_OFF, *vnew = smem + VN_OFF;               // new rows as tiles
-  float *part = (float *)(smem + PART_OFF);                        // [4][16][PD]: values, maximum, sum
-  int *spg = (int *)(smem + PART_OFF);                             // page list of the running unit (until the partials are written)
+  char *knew = smem + KN_OFF + sub * 2 * NEW_BYTES, *vnew = knew + NEW_BYTES;  // new rows as tiles
+  auto part_of = [&](int w) { return (float *)(smem + (PAIR ? BUF_OFF + (sub * SW + w) * (RB * SLOT) : PART_OFF + w * NC * PD * 4)); };  // [16][PD]: values, maximum, sum
+  int *spg = (int *)(smem + PART_OFF) + (PAIR ? sub * MK_ATTN_PAIR_PAGES : 0);  // page list of the running unit (until the partials are written)
   char *buf = smem + BUF_OFF + wave * (RB * SLOT);
   const u32x4 *kc = (const u32x4 *)st.k_cache, *vc = (const u32x4 *)st.v_cache;
   auto new_row = [&](char *base, int j) { return (uint16_t *)(base + (j >> 2) * GS + (j & 3) * 256); };
@@ -4051,27 +4074,28 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     }
     have = uu < n_units && decode(u_next, next);
     int lo;
-    if (have && tid < page_range(next, lo)) pg_next = next.pages[lo + tid];
+    if (have && stid < page_range(next, lo)) pg_next = next.pages[lo + stid];
   };
-  announce(c.vid);
+  announce(c.vid + sub * c.G);
   barrier_wait(c);
   attn_source_ready(st, c, src);
 
-  for (int uu = c.vid; uu < n_units; uu += c.G) {
-    if (!have) {
+  for (int uu = c.vid + sub * c.G; uu - sub * c.G < n_units; uu += SUBS * c.G) {
+    if (!PAIR && !have) {
       announce(uu + c.G);
       continue;
     }
-    const Unit a = next;
+    Unit a = next;
+    if (PAIR && !have) a.n = a.n_new = a.tb = a.te = 0;  // (the pair's other half has a unit: this one keeps the barriers)
     const int u = u_next;
     const int n_cols = a.n * QPK, p_first = a.p + 1 - a.n, nt = a.te - a.tb, cend = min(a.p0, a.te * 16);
     __syncthreads();  // LDS reuse across units
     // ---- page list, then the first tiles, then the rows
     int pg_lo;
     const int npg = page_range(a, pg_lo);
-    if (tid < npg) spg[tid] = pg_next;
-    for (int i = tid + MK_THREADS; i < npg; i += MK_THREADS) spg[i] = a.pages[pg_lo + i];
-    for (int j = a.n_new * 16 + tid; j < (a.n_new + 15) / 16 * 256; j += MK_THREADS) ((u32x4 *)new_row(vnew, j >> 4))[j & 15] = (u32x4){0u, 0u, 0u, 0u};
+    if (stid < npg) spg[stid] = pg_next;
+    for (int i = stid + ST; i < npg; i += ST) spg[i] = a.pages[pg_lo + i];
+    for (int j = a.n_new * 16 + stid; j < (a.n_new + 15) / 16 * 256; j += ST) ((u32x4 *)new_row(vnew, j >> 4))[j & 15] = (u32x4){0u, 0u, 0u, 0u};
     __syncthreads();
     auto row_base = [&](int pos) -> size_t {  // first 16-byte operand of the (position, head) row
       const int pc = min(pos, cend - 1), pg = pc / ps;
@@ -4094,11 +4118,11 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
         __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(vc + gb[s_]),
                                          (__attribute__((address_space(3))) void *)(__attribute__((address_space(3))) char *)(b + s_ * GS), 16, 0, KV_NT);
     };
-    if (wave < nt) {
+    if (sw < nt) {
 #pragma unroll
-      for (int b_ = 0; b_ < RB - 1; b_++) load_tile(wave + b_ * MK_WAVES, buf + b_ * SLOT);
+      for (int b_ = 0; b_ < RB - 1; b_++) load_tile(sw + b_ * SW, buf + b_ * SLOT);
     }
-    announce(uu + c.G);
+    announce(uu + SUBS * c.G);
     auto row = [&](int i) -> AttnRow {
       const int j = i - n_cols, kind = j < 0 ? 0 : j < a.n_new ? 1 : 2, jj = kind == 2 ? j - a.n_new : j, base = a.h * (QPK + 2) * D;
       return kind ? AttnRow{a.t0 + jj, base + (QPK + kind - 1) * D, a.p0 + jj, kind, new_row(kind == 1 ? knew : vnew, jj)}
@@ -4106,8 +4130,8 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     };
     auto own = [&](int tok) { return a.n_new > 0 && tok >= a.t; };
     const int n_rows = n_cols + 2 * a.n_new;
-    if (n_rows > 4 * MK_WAVES) attn_rows<8>(st, src, n_rows, lane, wave, row, own);
-    else attn_rows<4>(st, src, n_rows, lane, wave, row, own);
+    if (n_rows > 4 * SW) attn_rows<8, SW>(st, src, n_rows, lane, sw, row, own);
+    else attn_rows<4, SW>(st, src, n_rows, lane, sw, row, own);
     __syncthreads();
     // ---- tiles
     bf16x8 qb[4];
@@ -4200,19 +4224,19 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     };
     // cached tiles: RB in flight per wavefront; every request is issued unconditionally, and the wait before a tile counts the
     // 8 (RB - 1) requests of the tiles after it
-    int t_ = wave;
+    int t_ = sw;
     if (t_ < nt) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows stored above are not counted below; the first tiles arrived with the rows)
       bool more = true;
       while (more) {
 #pragma unroll
         for (int b_ = 0; b_ < RB; b_++) {
-          load_tile(t_ + (RB - 1) * MK_WAVES, buf + ((b_ + RB - 1) % RB) * SLOT);
+          load_tile(t_ + (RB - 1) * SW, buf + ((b_ + RB - 1) % RB) * SLOT);
           static_assert(RB == 2, "the wait counts one tile's requests");
           asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
           if (more) {
             compute_tile((a.tb + t_) * 16, cend - 1, buf + b_ * SLOT + TS, buf + b_ * SLOT, std::false_type{});
-            t_ += MK_WAVES;
+            t_ += SW;
             more = t_ < nt;
           }
         }
@@ -4220,57 +4244,74 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
     }
     // new tiles: all tokens of a group lie in the last of them (groups begin at multiples of TG in their request, TG divides 16)
     const int p_col = p_first + min(lr, n_cols - 1) / QPK;
-    for (int k = wave; k * 16 < a.n_new; k += MK_WAVES) compute_tile(a.p0 + k * 16, p_col, knew + k * TS, vnew + k * TS, std::true_type{});
+    for (int k = sw; k * 16 < a.n_new; k += SW) compute_tile(a.p0 + k * 16, p_col, knew + k * TS, vnew + k * TS, std::true_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the direct-to-LDS requests of the tile that was not computed)
     // the chunk with the new rows appends the group's own K/V rows and publishes its queries
     if (a.n_new) {
-      for (int i = tid; i < a.n * 64; i += MK_THREADS) {
+      for (int i = stid; i < a.n * 64; i += ST) {
         const int pos = p_first + (i >> 6), e = i & 63;
         const size_t at = (((size_t)a.pages[pos / ps] * ps + pos % ps) * nkv + a.h) * (D / 2) + e;
         ((uint32_t *)st.k_cache)[at] = ((const uint32_t *)new_row(knew, pos - a.p0))[e];
         ((uint32_t *)st.v_cache)[at] = ((const uint32_t *)new_row(vnew, pos - a.p0))[e];
       }
       if (st.q_ws)
-        for (int i = tid; i < n_cols * 64; i += MK_THREADS) {
+        for (int i = stid; i < n_cols * 64; i += ST) {
           const int col = i >> 6;
           ((uint32_t *)st.q_ws)[((size_t)(a.t + col / QPK) * st.ld_qws + (size_t)(a.h * QPK + col % QPK) * D) / 2 + (i & 63)] = ((const uint32_t *)qs)[i];
         }
     }
-    __syncthreads();  // every wavefront is done with the page list: the partial results may overwrite it
+    if (!PAIR) __syncthreads();  // every wavefront is done with the page list: the partial results may overwrite it
     // ---- wavefronts
     float lt = lsum;
     lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, lt)));
     lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, lt)));
+    float *part = part_of(sw);
     if (lg == 0) {
-      part[(wave * NC + lr) * PD + D] = mrun;
-      part[(wave * NC + lr) * PD + D + 1] = lt;
+      part[lr * PD + D] = mrun;
+      part[lr * PD + D + 1] = lt;
     }
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int dt = 0; dt < 8; dt++) part[(wave * NC + lg * 4 + r) * PD + dt * 16 + lr] = o[dt][r];
+      for (int dt = 0; dt < 8; dt++) part[(lg * 4 + r) * PD + dt * 16 + lr] = o[dt][r];
     __syncthreads();
     // (die-local or device-scope hand-over of chunks: see stage_attn)
     const bool local = !rt.attn_part && c.even_xcds && (a.item * cmax) / c.quota == (a.item * cmax + a.C - 1) / c.quota;
     float *part_base = rt.attn_part ? rt.attn_part : (float *)st.aux0;
-    const int col = tid >> 4, md = (tid & 15) * 8;  // this thread's column and dims
-    uint16_t *orow = (uint16_t *)st.out + (size_t)(a.t + col / QPK) * st.ld_out + (size_t)(a.h * QPK + col % QPK) * D + md;
+    const int md = (tid & 15) * 8;  // this thread's dims; its column: one of sixteen, or, with two units at a time, two of theirs
+    int col = stid >> 4;
     auto emit = [&](const float (&v)[8], float l) {  // written through: the stage's barrier skips the L2 write-back
+      uint16_t *orow = (uint16_t *)st.out + (size_t)(a.t + col / QPK) * st.ld_out + (size_t)(a.h * QPK + col % QPK) * D + md;
 #pragma unroll
       for (int d = 0; d < 8; d += 2) __hip_atomic_store((uint32_t *)(orow + d), pack2(v[d] / l, v[d + 1] / l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
-    if (col < n_cols) {
-      float mx = -1e30f, ls = 0.f, os[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto wavefronts = [&](float &mx, float &ls, float (&os)[8]) {  // the sum over the unit's wavefronts
+      mx = -1e30f;
+      ls = 0.f;
 #pragma unroll
-      for (int w = 0; w < MK_WAVES; w++) mx = fmaxf(mx, part[(w * NC + col) * PD + D]);
+      for (int d = 0; d < 8; d++) os[d] = 0.f;
 #pragma unroll
-      for (int w = 0; w < MK_WAVES; w++) {
-        const float *pp = part + (w * NC + col) * PD;
+      for (int w = 0; w < SW; w++) mx = fmaxf(mx, part_of(w)[col * PD + D]);
+#pragma unroll
+      for (int w = 0; w < SW; w++) {
+        const float *pp = part_of(w) + col * PD;
         const float wgt = __builtin_amdgcn_exp2f(pp[D] - mx);
         ls += pp[D + 1] * wgt;
 #pragma unroll
         for (int d = 0; d < 8; d++) os[d] += pp[md + d] * wgt;
       }
+    };
+    if constexpr (PAIR) {
+      for (; col < n_cols; col += ST / 16) {
+        float mx, ls, os[8];
+        wavefronts(mx, ls, os);
+        emit(os, ls);
+      }
+      continue;
+    }
+    if (col < n_cols) {
+      float mx, ls, os[8];
+      wavefronts(mx, ls, os);
       if (a.C == 1) {
         emit(os, ls);
       } else {
@@ -4703,10 +4744,12 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
             // many (token, kv head) pairs per workgroup-chunk: cached positions on the matrix cores
             const bool mf = 2 * M * st.num_kv_heads >= c.G;
             if (st.num_q_heads == 4 * st.num_kv_heads) {
-              if (mf) stage_attn_tiles<4>(st, c, rt, M, smem);
+              if (mf && attn_in_pairs<4>(st, c, rt, M)) stage_attn_tiles<4, true>(st, c, rt, M, smem);
+              else if (mf) stage_attn_tiles<4, false>(st, c, rt, M, smem);
               else stage_attn<4>(st, c, rt, M, smem);
             } else if (st.num_q_heads == 8 * st.num_kv_heads) {
-              if (mf) stage_attn_tiles<8>(st, c, rt, M, smem);
+              if (mf && attn_in_pairs<8>(st, c, rt, M)) stage_attn_tiles<8, true>(st, c, rt, M, smem);
+              else if (mf) stage_attn_tiles<8, false>(st, c, rt, M, smem);
               else stage_attn<8>(st, c, rt, M, smem);
             } else {
               barrier_wait(c);
