@@ -9,7 +9,7 @@
 //   * stage_fx_prep /   rotary positions on part of a head, heads divided by their root mean square, paged K/V append,
 //     stage_fx_attn     softcapped scores, softmax with an extra per-head logit in the denominator, split-KV on the matrix
 //                       cores for prompt portions and for single tokens alike;
-//   * stage_fx_linear_f32, stage_fx_argmax_f32  the 32-bit forms of the linear and of the sampling stage.
+//   * stage_fx_linear_f32  the 32-bit form of the linear.
 // The stages are instantiated for bf16 (E = uint16_t) and for 32-bit (E = float) activations, weights and caches; scores,
 // softmax, norms, angles and the residual stream are 32-bit in both.
 
@@ -1207,31 +1207,5 @@ __device__ __forceinline__ void stage_fx_linear_f32(CStage &st, Ctx &c, int M, c
     stage_fx_linear_f32_t<1, true>(st, c, M, smem);
   } else {
     stage_fx_linear_f32_t<1, false>(st, c, M, smem);
-  }
-}
-
-// Greedy sampling over 32-bit logits, stage 1 (stage 2 is stage_argmax_reduce): one wavefront per token.
-__device__ __forceinline__ void stage_fx_argmax_f32(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
-  barrier_wait(c);
-  const int n = st.n, per = (n + c.G - 1) / c.G, c0 = c.vid * per, c1 = min(n, c0 + per);
-  float *pv = rt.argmax_pv ? rt.argmax_pv : (float *)st.aux0;
-  int *pi = rt.argmax_pv ? rt.argmax_pi : (int *)st.aux1;
-  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
-  for (int t = wave; t < M; t += MK_WAVES) {
-    const float *row = (const float *)st.in + (size_t)t * st.ld_in;
-    float best = -INFINITY;
-    int bi = 0x7fffffff;
-    for (int i = c0 + lane; i < c1; i += 64) {
-      const float v = ldc_f32(row + i);
-      if (v > best) {
-        best = v;
-        bi = i;
-      }
-    }
-    wave_argmax(best, bi);
-    if (lane == 0) {
-      pv[t * c.G + c.vid] = best;
-      pi[t * c.G + c.vid] = bi;
-    }
   }
 }

@@ -1,5 +1,5 @@
 """Attention of many requests (a workgroup takes two units at a time where contexts are about equally long, four wavefronts take one
-otherwise) at the sizes where its split changes, against plain torch in 32 bits."""
+otherwise) and sampling, at the sizes where their splits change, against plain torch in 32 bits."""
 import pytest
 import torch
 
@@ -64,4 +64,36 @@ def test_attention_of_many_requests(R, kind, new, ps, nkv, qpk):
             bound = want.abs() * 2.0 ** -8 + float(V.abs().max()) * 2.0 ** -13
             assert bool(((got - want).abs() <= bound).all()), f"request {r} token {t}: off by {float((got - want).abs().max())}"
     assert bool((out[total:] == 0).all()) and pk.stats()["aborted"] == 0
+    pk.finalize()
+
+
+# (pieces of sixteen bytes, five of them a lane and turn: 163840 logits; rows that do not begin on sixteen bytes)
+@pytest.mark.parametrize("V", [1, 8, 1000, 1001, 4104, 163848, 200001])
+@pytest.mark.parametrize("B", [1, 17, 64])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sampling(B, V, dtype):
+    """The first of the largest values, wherever it lies; rows of the lowest values there are."""
+    meta = make_meta(B, 64, B, B, B)
+    pk = make_mpk(meta, 64, B, B, B, 64, mode="onepass")
+    logits = torch.randn(B, V, generator=torch.Generator().manual_seed(V + B)).to(dtype).cuda()
+    top = torch.finfo(dtype).max
+    at = [(i * V) // 7 + i for i in range(7)] + [0, V - 1]
+    want = []
+    for r in range(B):
+        if r == 1:
+            logits[r] = -top
+        elif V > 1:
+            a, b = min(at[r % 9], V - 1), min(at[(r + 4) % 9], V - 1)
+            logits[r, a] = logits[r, b] = top
+    if dtype == torch.float32:  # (32-bit sampling runs beside other 32-bit stages)
+        f32 = lambda name, *shape: pk.attach_input(torch.zeros(*shape, device="cuda"), name)
+        pk.embed_scaled_layer(pk.attach_input(meta["input_tokens"], "ids"), f32("table", 4, 64), f32("rows32", B, 64), f32("rows", B, 64), 1.0)
+    pk.argmax_layer(input=pk.attach_input(logits, "logits"), output=pk.attach_input(meta["output_tokens"], "out"), grid_dim=(1, 1, 1), block_dim=(128, 1, 1))
+    pk.compile()
+    for M in sorted({1, B // 2 + 1, B}):
+        meta["output_tokens"].fill_(-5)
+        torch.cuda.synchronize()
+        pk.run_once(list(range(M)), [0] * M)
+        want = [int((logits[r] == logits[r].max()).nonzero()[0]) for r in range(M)]
+        assert meta["output_tokens"].view(-1).tolist() == want + [-5] * (B - M)
     pk.finalize()
