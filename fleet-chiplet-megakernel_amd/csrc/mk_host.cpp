@@ -3070,19 +3070,22 @@ static int tail_stage(const mk_graph *g) {
   };
   int tail = n;
   while (tail > 0 && ends_here(g->stages[tail - 1])) tail--;
+  if (tail == n) return n;
   // tensors by the widest one that holds an address; the library's own scratch by the address itself
+  std::vector<std::pair<const char *, const char *>> spans;
+  for (const Tensor &t : g->tensors) {
+    if (!t.ptr || t.kind == T_SHUFFLED) continue;
+    size_t last = 0;
+    for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
+    spans.push_back({(const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype)});
+  }
   std::map<const void *, const void *> known;
   auto whole = [&](const void *p) {
     const auto it = known.find(p);
     if (it != known.end()) return it->second;
-    const char *q = (const char *)p, *best = q;
-    for (const Tensor &t : g->tensors) {
-      const char *b = (const char *)t.ptr;
-      if (!b || t.kind == T_SHUFFLED) continue;
-      size_t last = 0;
-      for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
-      if (q >= b && q < b + (last + 1) * dtype_size(t.dtype) && b < best) best = b;
-    }
+    const char *best = (const char *)p;
+    for (const auto &t : spans)
+      if (p >= t.first && p < t.second && t.first < best) best = t.first;
     return known[p] = (const void *)best;
   };
   auto written = [&](const MkStage &s, std::set<const void *> &to) {

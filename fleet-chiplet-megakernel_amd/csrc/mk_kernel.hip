@@ -4389,7 +4389,7 @@ __device__ __forceinline__ void stage_attn_tiles(CStage &st, Ctx &c, const MkRun
 //
 // Bound by round trips: a slice is a few hundred bytes.  Sixteen lanes take a token, sixteen bytes each, and every token's slice is requested
 // before the first is looked at; the results leave as whole lines, so that no cache is written back.  A wavefront per token with four tokens
-// in flight, a result at a time: 64 tokens of 32768 logits 16.0 -> 5.5 us, 4 tokens 8.0 -> 4.6, with the second stage 23 -> 10 and 14 -> 9.
+// in flight, a result at a time: 64 tokens of 32768 logits 16.3 -> 7.0 us, 4 tokens 8.4 -> 4.3, with the second stage 23 -> 11.5 and 12.3 -> 7.9.
 template <typename E, int MAXM>
 __device__ __forceinline__ void stage_argmax_partial(CStage &st, Ctx &c, const MkRuntime &rt, int M, char *smem) {
   constexpr int CH = 16 / sizeof(E);                          // logits of a piece of sixteen bytes

@@ -161,7 +161,8 @@ int mk_wait(mk_graph *g, void *stream, int *finished_out);
 /* mk_enqueue_steps in the modes whose batch the host describes (online_notoken / onepass; MK_EINVAL in the others), for a batch
  * whose logits and sampled tokens nobody reads, such as a portion in the middle of a prompt: caches and recurrent states come out as
  * mk_enqueue_steps leaves them, the stages behind the last one that writes them do not run, and the buffers they write keep older
- * values.  (With a profiler tensor attached everything runs.)  Pair with mk_wait. */
+ * values.  (With a profiler tensor attached, and in graphs of one token per
+ * iteration, everything runs.)  Pair with mk_wait. */
 int mk_enqueue_ingest(mk_graph *g, void *stream);
 /* mk_enqueue_steps for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc); it has no counterpart in the reference.  The call allocates and frees nothing, and every piece
