@@ -116,3 +116,34 @@ def test_rows_carried_from_one_iteration_to_the_next(carried):
     pk.wait()
     assert bool((acc != 0).any()) == carried
     pk.finalize()
+
+
+@pytest.mark.parametrize("B,R,total,portion,page_size,max_seq", [(64, 1, 2, 64, 16, 150), (64, 2, 3, 16, 4, 90), (64, 5, 9, 64, 16, 120), (40, 3, 6, 30, 8, 100), (64, 40, 50, 2, 8, 30)])
+def test_scheduler_of_portions(B, R, total, portion, page_size, max_seq):
+    """Long portions of one, two and many requests: the same batches, entry for entry, as the scheduler oracle's."""
+    import numpy as np
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    from oracle.sched_ref import SchedulerOracle
+    shape = Qwen3Shape(hidden_size=1024, num_q_heads=8, num_kv_heads=2, head_dim=128, intermediate_size=512, num_layers=1, vocab_size=512)
+    rng = np.random.default_rng(B + R + total)
+    prompts = [torch.from_numpy(rng.integers(0, shape.vocab_size, size=int(rng.integers(1, max_seq - 3)))) for _ in range(total)]
+    pages = R * ((max_seq + page_size - 1) // page_size)
+    dec = Qwen3Decoder(shape, random_weights(shape, seed=1), max_num_batched_tokens=B, max_num_batched_requests=R, max_seq_length=max_seq, page_size=page_size, max_num_pages=pages,
+                       total_requests=total, eos_token_id=0x7FFFFFFF, max_tokens_per_request=portion)
+    dec.load_prompts(prompts)
+    orc = SchedulerOracle([p.tolist() for p in prompts], R, B, pages, page_size, max_seq, max_new_per_req=portion)
+    out = None
+    while True:
+        n = orc.step(out)
+        fin = dec.mpk.run_steps(1)
+        if n == 0:
+            assert fin
+            break
+        assert not fin
+        nreq = int((orc["request_ids"] >= 0).sum())
+        for ours, theirs, m in (("step", "step", total), ("input_tokens", "input_tokens", n), ("qo_indptr_buffer", "qo_indptr", R + 1), ("paged_kv_indptr_buffer", "kv_indptr", R + 1),
+                                ("paged_kv_last_page_len_buffer", "kv_last_page_len", nreq), ("paged_kv_indices_buffer", "kv_indices", int(orc["kv_indptr"][R]))):
+            assert np.array_equal(dec.meta[ours].cpu().numpy().reshape(-1)[:m], orc[theirs].reshape(-1)[:m]), ours
+        out = dec.meta["output_tokens"].cpu().numpy().reshape(-1)
+    assert np.array_equal(dec.meta["tokens"].cpu().numpy(), orc["tokens"])
+    dec.mpk.finalize()
