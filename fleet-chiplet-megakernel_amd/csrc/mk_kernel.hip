@@ -4412,6 +4412,43 @@ __device__ __forceinline__ void stage_argmax_partial(CStage &st, Ctx &c, const M
   float *sv = (float *)smem;  // [MAXM] values, [MAXM] indices
   int *si = (int *)smem + MAXM;
   barrier_wait(c);
+  // One token only: a wavefront takes the slice, a dword a lane.  By sixteen lanes the kernel of one token was 15 us a pass slower with 151936
+  // logits (2.991 -> 2.976 ms a token, 36 layers; before that form 2.969); loads by the lanes of the token alone changed nothing (2.991).
+  if constexpr (MAXM == 1 && sizeof(E) == 2) {
+    const int per = ((n + c.G - 1) / c.G + 1) & ~1, c0 = c.vid * per, c1 = min(n, c0 + per), nd = (c1 - c0 + 1) / 2;
+    if (tid < 64) {
+      constexpr int NDW = 5;
+      uint32_t w[NDW];
+      float b1 = -INFINITY;
+      int i1 = 0x7fffffff;
+#pragma unroll
+      for (int j = 0; j < NDW; j++)
+        if (j * 64 + lane < nd) w[j] = ldc_u32((const uint16_t *)st.in + c0 + 2 * (j * 64 + lane));
+      auto consider = [&](uint32_t u, int i) {
+        const float v0 = bf_lo(u), v1 = bf_hi(u);
+        if (v0 > b1) {
+          b1 = v0;
+          i1 = i;
+        }
+        if (i + 1 < c1 && v1 > b1) {
+          b1 = v1;
+          i1 = i + 1;
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < NDW; j++)
+        if (j * 64 + lane < nd) consider(w[j], c0 + 2 * (j * 64 + lane));
+      for (int d = NDW * 64 + lane; d < nd; d += 64) consider(ldc_u32((const uint16_t *)st.in + c0 + 2 * d), c0 + 2 * d);
+      wave_argmax(b1, i1);
+      if (lane == 0) {
+        const int at = c.vid * rt.max_tokens;
+        stc_f32((rt.argmax_pv ? rt.argmax_pv : (float *)st.aux0) + at, b1);
+        __hip_atomic_store((rt.argmax_pv ? rt.argmax_pi : (int *)st.aux1) + at, i1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    c.wrote_through = true;
+    return;
+  }
   c.wrote_through = true;
   float best[RB];
   int bi[RB];
