@@ -198,6 +198,7 @@ struct mk_graph {
   std::vector<char> releasable;       // per tensor (single-weight-copy graphs, after mk_compile): the handle never reads it again
   bool single_copy = false;
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
+  int tail = 0;      // MkRuntime::tail
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
   int64_t row_major_bytes = 0;
@@ -214,8 +215,8 @@ namespace {
 
 int dev_alloc(mk_graph *g, void **out, size_t bytes, bool zero = true) {
   if (bytes == 0) bytes = 16;
-  if (g->host_only) {  // stand-in address: only its identity matters to the lowering
-    *out = malloc(16);
+  if (g->host_only) {  // stand-in: only its address and size matter to the lowering (never touched, so no memory stands behind it)
+    *out = malloc(bytes);
     if (!*out) return fail(MK_EINVAL, "out of host memory");
     g->host_allocs.push_back(*out);
     return MK_OK;
@@ -1912,6 +1913,61 @@ int lower_moe_combine(mk_graph *g, size_t &i, bool fused_single) {
   return MK_OK;
 }
 
+// First of the stages at the program's end that leave nothing behind but what this iteration's logits and sampled tokens are made of: behind
+// every stage that writes caches or recurrent states, and behind everything whose effects are not known to end with the iteration.  None
+// (num_stages) where an iteration could read, ahead of writing it, what such a stage of the iteration before has written.
+int tail_stage(const mk_graph *g) {
+  const int n = (int)g->stages.size();
+  if (g->spec_len > 0) return n;
+  auto ends_here = [](const MkStage &s) {
+    switch (s.op) {
+      case MK_OP_NORM: case MK_OP_LINEAR: case MK_OP_SILU_MUL: case MK_OP_ARGMAX_PARTIAL: case MK_OP_ARGMAX_REDUCE: case MK_OP_MOE_TOPK: case MK_OP_MOE_LINEAR:
+      case MK_OP_MOE_COMBINE: case MK_OP_FX_ADDNORM: case MK_OP_LINEAR_F32: case MK_OP_FX_ARGMAX_F32: case MK_OP_MX_PRENORM: case MK_OP_MX_HEAD_LINEAR:
+      case MK_OP_HY_ROUTE: case MK_OP_HY_EXPERTS: return !s.tail && !s.conv_w && !s.k_cache && !s.v_cache;
+      default: return false;
+    }
+  };
+  int tail = n;
+  while (tail > 0 && ends_here(g->stages[tail - 1])) tail--;
+  if (tail == n) return n;
+  // tensors by the widest one that holds an address; the library's own scratch by the address itself
+  std::vector<std::pair<const char *, const char *>> spans;
+  for (const Tensor &t : g->tensors) {
+    if (!t.ptr || t.kind == T_SHUFFLED) continue;
+    size_t last = 0;
+    for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
+    spans.push_back({(const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype)});
+  }
+  std::map<const void *, const void *> known;
+  auto whole = [&](const void *p) {
+    const auto it = known.find(p);
+    if (it != known.end()) return it->second;
+    const char *best = (const char *)p;
+    for (const auto &t : spans)
+      if (p >= t.first && p < t.second && t.first < best) best = t.first;
+    return known[p] = (const void *)best;
+  };
+  auto written = [&](const MkStage &s, std::set<const void *> &to) {
+    for (const void *p : {(const void *)s.out, (const void *)s.out2, (const void *)s.out3, (const void *)s.norm_out, (const void *)s.glu_out,
+                          (const void *)(s.op == MK_OP_HY_ROUTE || s.op == MK_OP_HY_EXPERTS ? s.ids : nullptr),
+                          (const void *)s.moe_topk_w, (const void *)s.moe_routing, (const void *)s.moe_mask})
+      if (p) to.insert(whole(p));
+  };
+  std::set<const void *> left, fresh;
+  for (int i = tail; i < n; i++) written(g->stages[i], left);
+  for (int i = 0; i < n; i++) {
+    const MkStage &s = g->stages[i];
+    for (const void *p : {s.in, s.in2, s.in3, s.res, s.y_in, s.y2, (const void *)s.slot_w, s.moe_logits, (const void *)s.moe_topk_w, (const void *)s.moe_routing,
+                          (const void *)s.moe_mask, (const void *)s.ids, s.w.seg[0], s.w.seg[1], s.w.seg[2], s.w_shared, s.norm_w, s.y_norm_w, s.q_norm_w, s.k_norm_w, (const void *)s.q_ws,
+                          (const void *)s.k_cache, (const void *)s.v_cache, s.cos_tab, s.sin_tab, s.sink, (const void *)s.aux0, (const void *)s.aux1, (const void *)s.in_bias,
+                          (const void *)s.a_tab, (const void *)s.d_tab, (const void *)s.temp, (const void *)s.y_scale, (const void *)s.y2_scale, s.conv_w, s.pos_tab,
+                          (const void *)s.choice_bias, (const void *)s.step_bias})
+      if (p && left.count(whole(p)) && !fresh.count(whole(p))) return n;
+    written(s, fresh);
+  }
+  return tail;
+}
+
 int lower(mk_graph *g) {
   g->stages.clear();
   g->stage_desc.clear();
@@ -2326,8 +2382,9 @@ int lower(mk_graph *g) {
       default: st.prof_event = 121; break;
     }
   }
+  g->tail = tail_stage(g);
   g->program_text.clear();
-  for (size_t s = 0; s < g->stage_desc.size(); s++) g->program_text += fmt("%3zu ", s) + g->stage_desc[s] + "\n";
+  for (size_t s = 0; s < g->stage_desc.size(); s++) g->program_text += fmt("%3zu ", s) + g->stage_desc[s] + ((int)s < g->tail ? "\n" : " unread=skip\n");
   return MK_OK;
 }
 
@@ -3054,61 +3111,6 @@ int mk_generate_task_graph(mk_graph *g, int num_gpus, int my_gpu_id, const char 
   return MK_OK;
 }
 
-// First of the stages at the program's end that leave nothing behind but what this iteration's logits and sampled tokens are made of: behind
-// every stage that writes caches or recurrent states, and behind everything whose effects are not known to end with the iteration.  None
-// (num_stages) where an iteration could read, ahead of writing it, what such a stage of the iteration before has written.
-static int tail_stage(const mk_graph *g) {
-  const int n = (int)g->stages.size();
-  if (g->spec_len > 0) return n;
-  auto ends_here = [](const MkStage &s) {
-    switch (s.op) {
-      case MK_OP_NORM: case MK_OP_LINEAR: case MK_OP_SILU_MUL: case MK_OP_ARGMAX_PARTIAL: case MK_OP_ARGMAX_REDUCE: case MK_OP_MOE_TOPK: case MK_OP_MOE_LINEAR:
-      case MK_OP_MOE_COMBINE: case MK_OP_FX_ADDNORM: case MK_OP_LINEAR_F32: case MK_OP_FX_ARGMAX_F32: case MK_OP_MX_PRENORM: case MK_OP_MX_HEAD_LINEAR:
-      case MK_OP_HY_ROUTE: case MK_OP_HY_EXPERTS: return !s.tail && !s.conv_w && !s.k_cache && !s.v_cache;
-      default: return false;
-    }
-  };
-  int tail = n;
-  while (tail > 0 && ends_here(g->stages[tail - 1])) tail--;
-  if (tail == n) return n;
-  // tensors by the widest one that holds an address; the library's own scratch by the address itself
-  std::vector<std::pair<const char *, const char *>> spans;
-  for (const Tensor &t : g->tensors) {
-    if (!t.ptr || t.kind == T_SHUFFLED) continue;
-    size_t last = 0;
-    for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
-    spans.push_back({(const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype)});
-  }
-  std::map<const void *, const void *> known;
-  auto whole = [&](const void *p) {
-    const auto it = known.find(p);
-    if (it != known.end()) return it->second;
-    const char *best = (const char *)p;
-    for (const auto &t : spans)
-      if (p >= t.first && p < t.second && t.first < best) best = t.first;
-    return known[p] = (const void *)best;
-  };
-  auto written = [&](const MkStage &s, std::set<const void *> &to) {
-    for (const void *p : {(const void *)s.out, (const void *)s.out2, (const void *)s.out3, (const void *)s.norm_out, (const void *)s.glu_out,
-                          (const void *)(s.op == MK_OP_HY_ROUTE || s.op == MK_OP_HY_EXPERTS ? s.ids : nullptr),
-                          (const void *)s.moe_topk_w, (const void *)s.moe_routing, (const void *)s.moe_mask})
-      if (p) to.insert(whole(p));
-  };
-  std::set<const void *> left, fresh;
-  for (int i = tail; i < n; i++) written(g->stages[i], left);
-  for (int i = 0; i < n; i++) {
-    const MkStage &s = g->stages[i];
-    for (const void *p : {s.in, s.in2, s.in3, s.res, s.y_in, s.y2, (const void *)s.slot_w, s.moe_logits, (const void *)s.moe_topk_w, (const void *)s.moe_routing,
-                          (const void *)s.moe_mask, (const void *)s.ids, s.w.seg[0], s.w.seg[1], s.w.seg[2], s.w_shared, s.norm_w, s.y_norm_w, s.q_norm_w, s.k_norm_w,
-                          (const void *)s.k_cache, (const void *)s.v_cache, s.cos_tab, s.sin_tab, s.sink, (const void *)s.aux0, (const void *)s.aux1, (const void *)s.in_bias,
-                          (const void *)s.a_tab, (const void *)s.d_tab, (const void *)s.temp, (const void *)s.y_scale, (const void *)s.y2_scale, s.conv_w, s.pos_tab,
-                          (const void *)s.choice_bias, (const void *)s.step_bias})
-      if (p && left.count(whole(p)) && !fresh.count(whole(p))) return n;
-    written(s, fresh);
-  }
-  return tail;
-}
-
 // Matrix-core copies of the linear weights (MkStage::wpack).  A graph that can run more than eight tokens per iteration
 // streams its weights through the matrix cores in 16-row tiles; read from a row-major matrix that is 64 bytes from each
 // of 16 rows per request, which HBM serves at about three quarters of the rate of one contiguous stream.  So every such
@@ -3176,7 +3178,7 @@ int mk_compile(mk_graph *g) {
   if (per_cu < 1 || g->G > per_cu * g->num_cus) return fail(MK_EINVAL, "grid of %d workgroups cannot be co-resident (%d per CU x %d CUs)", g->G, per_cu, g->num_cus);
   MkRuntime &rt = g->h_rt;
   rt.num_stages = (int)g->stages.size();
-  rt.tail = tail_stage(g);
+  rt.tail = g->tail;
   rt.max_tokens = c.max_num_batched_tokens;
   rt.max_requests = c.max_num_batched_requests;
   rt.max_seq = c.max_seq_length;

@@ -224,7 +224,8 @@ int mk_get_stage_marks(mk_graph *g, int workgroup, int64_t *ticks_out, int max_s
  * 1 + b + k * workgroups; low 32 bits tag = stage instance << 19 | b << 11 | task type << 2 | (0 begin / 1 end), high 32
  * bits = low word of the device time in ns.  The tensor is cleared here and by mk_init_requests; NULL stops recording. */
 int mk_set_profiler(mk_graph *g, void *device_u64, int64_t num_entries);
-/* Stage listing (one line per stage) for debugging and tests; owned by the handle. */
+/* Stage listing (one line per stage) for debugging and tests; owned by the handle.  Lines that end in "unread=skip": stages an iteration
+ * leaves out whose logits and sampled tokens nobody reads (mk_enqueue_ingest, portions inside prompts). */
 int mk_describe_program(mk_graph *g, const char **text_out);
 
 const char *mk_last_error(void);
