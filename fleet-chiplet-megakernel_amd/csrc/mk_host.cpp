@@ -1929,7 +1929,8 @@ int tail_stage(const mk_graph *g) {
   };
   int tail = n;
   while (tail > 0 && ends_here(g->stages[tail - 1])) tail--;
-  if (tail == n) return n;
+  if (tail > 0 && (g->stages[tail - 1].flags & MK_F_DEFER_SUM)) tail++;  // (its sum may be left to the stage behind it)
+  if (tail >= n) return n;
   // tensors by the widest one that holds an address; the library's own scratch by the address itself
   std::vector<std::pair<const char *, const char *>> spans;
   for (const Tensor &t : g->tensors) {

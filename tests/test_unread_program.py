@@ -46,3 +46,22 @@ def test_query_latents_written_for_the_next_iteration(carried):
     pk.latent_attention_layer(q, ql, cache, cos, sin, out, H, rank, rot, 64, 0, 1.0)
     _linear(pk, out, H * rank, ql if carried else other)
     assert _skipped(pk) == [False, False, not carried]
+
+
+def test_norm_that_finishes_the_sum_of_the_stage_in_front():
+    """The linear behind a convolution over time keeps the request's ring and runs in every iteration; the sum over its slices of K is
+    left to the norm behind it, which therefore runs as well."""
+    pk, n = _pk(), 64
+    x, xo, xp, g = (_attach(pk, k, *s, dtype=torch.float32)[0] for k, s in (("x", (B, n)), ("xo", (B, n)), ("xp", (B, n)), ("g", (n,))))
+    y, rows, conv, z, out, last = (_attach(pk, k, B, n)[0] for k in ("y", "rows", "conv", "z", "out", "last"))
+    taps, ring = _attach(pk, "taps", 4, n)[0], _attach(pk, "ring", R, 4, n)[0]
+    slots, _ = _attach(pk, "slots", R, dtype=torch.int32)
+    pk.residual_prenorm_layer(y, x, xo, rows, weight=g)
+    pk.ring_conv_layer(rows, taps, ring, slots, conv, identity=True)
+    _linear(pk, conv, n, z)
+    pk.residual_prenorm_layer(z, xo, xp, out, weight=g)
+    _linear(pk, out, n, last, "w2")
+    kinds = [line.split()[1] for line in pk.describe_program().splitlines()]
+    assert kinds == ["MX_PRENORM[multi-token", "DU_CONV[portions]", "LINEAR", "MX_PRENORM[multi-token", "LINEAR"]
+    assert "sum=next" in pk.describe_program().splitlines()[2]
+    assert _skipped(pk) == [False] * 4 + [True]
