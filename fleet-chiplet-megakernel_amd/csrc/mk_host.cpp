@@ -16,7 +16,6 @@
 #include <array>
 #include <map>
 #include <numeric>
-#include <set>
 #include <string>
 #include <vector>
 
@@ -171,6 +170,7 @@ struct mk_graph {
   bool host_only = false;  // created with device < 0: records, validates, lowers and emits the task graph, never launches
   std::vector<void *> allocs;
   std::vector<void *> host_allocs;
+  std::vector<std::pair<void *, size_t>> alloc_sizes;  // of both
   std::vector<MkStage> stages;
   std::vector<std::string> stage_desc;
   MkRuntime h_rt;
@@ -219,10 +219,12 @@ int dev_alloc(mk_graph *g, void **out, size_t bytes, bool zero = true) {
     *out = malloc(bytes);
     if (!*out) return fail(MK_EINVAL, "out of host memory");
     g->host_allocs.push_back(*out);
+    g->alloc_sizes.push_back({*out, bytes});
     return MK_OK;
   }
   HIP_TRY(hipMalloc(out, bytes));
   g->allocs.push_back(*out);
+  g->alloc_sizes.push_back({*out, bytes});
   if (zero) HIP_TRY(hipMemset(*out, 0, bytes));
   return MK_OK;
 }
@@ -1913,11 +1915,234 @@ int lower_moe_combine(mk_graph *g, size_t &i, bool fused_single) {
   return MK_OK;
 }
 
+// Rows of an iteration's tokens that a stage reads or writes: token t's are `width` bytes from p + t * stride on (stride 0: one piece for all).
+struct RowSpan {
+  const char *p;
+  int64_t width, stride;
+};
+// What a stage does with memory that other stages write.  `reads` and `elsewhere` (operands of which only the address is known here) hold all it
+// reads; `writes` what is new behind it in every iteration, whichever of its forms ran, if the rows in `routing` are this iteration's, `zeros` the
+// padding of such rows, `handed` what is new for the stage directly behind alone, and `touches` what it may write besides.
+struct StageRows {
+  std::vector<RowSpan> reads, writes, zeros, handed, touches, routing;
+  std::vector<const void *> elsewhere;
+};
+StageRows rows_of(const mk_graph *g, size_t i) {
+  const std::vector<MkStage> &stages = g->stages;
+  const MkStage &s = stages[i];
+  StageRows r;
+  const int es = g->flex == FLEX_F32 ? 4 : 2, B = g->cfg.max_num_batched_tokens;
+  auto piece = [](std::vector<RowSpan> &to, const void *p, int64_t n, int64_t size, int64_t ld) {
+    if (p) to.push_back({(const char *)p, n * size, ld * size});
+  };
+  auto pieces = [&](std::vector<RowSpan> &to, const void *p, int count, int64_t apart, int64_t n, int64_t size, int64_t ld) {
+    for (int q = 0; p && q < (apart ? count : 1); q++) piece(to, (const char *)p + q * apart * size, n, size, ld);
+  };
+  auto padded = [&](void *p, int64_t size, int64_t ld) {  // rows of s.n values of which s.k are real, the rest is zero
+    piece(r.writes, p, s.k, size, ld);
+    if (p && s.n > s.k) piece(r.zeros, (const char *)p + s.k * size, s.n - s.k, size, ld);
+  };
+  auto whole = [](std::vector<RowSpan> &to, const void *p, int64_t n) {
+    if (p) to.push_back({(const char *)p, n * 4, 0});
+  };
+  // operands that the cases below describe are taken out of what is read elsewhere
+  const void *in = s.in, *res = s.res, *y_in = s.y_in, *y2 = s.y2, *slot_w = s.slot_w, *logits = s.moe_logits, *topk_w = s.moe_topk_w, *routing = s.moe_routing, *ids = s.ids, *aux0 = s.aux0, *aux1 = s.aux1,
+             *q_ws = s.q_ws, *w_shared = s.w_shared, *norm_out = nullptr;
+  auto took = [](const void *&p) {
+    const void *was = p;
+    p = nullptr;
+    return was;
+  };
+  const bool grouped = s.flags & MK_F_GROUPS, glu = s.flags & MK_F_SILU;
+  const int shared = s.w_shared ? 1 : 0;
+  switch (s.op) {
+    case MK_OP_EMBED:
+    case MK_OP_FX_EMBED:
+      piece(r.writes, s.out, s.k, es, s.ld_out);
+      piece(r.writes, s.out2, s.k, 4, s.ld_out2);
+      break;
+    case MK_OP_NORM:
+      piece(r.reads, took(in), s.k, 2, s.ld_in);
+      piece(r.writes, s.out, s.k, 2, s.ld_out);
+      break;
+    case MK_OP_FX_ADDNORM:
+      piece(r.reads, took(in), s.n, es, s.ld_in);
+      piece(r.reads, took(res), s.n, 4, s.ld_res);
+      padded(s.out, es, s.ld_out);
+      padded(s.out2, 4, s.ld_out2);
+      break;
+    case MK_OP_MX_PRENORM:
+      pieces(r.reads, took(in), s.slots && !s.y2 ? s.slots : 1, s.ld_slot, s.n, es, s.ld_in);
+      pieces(r.reads, took(y2), s.slots ? s.slots : 1, s.ld_slot, s.n, es, s.ld_y2);
+      if (s.slots) piece(r.reads, took(slot_w), s.slots, 4, s.ld_slot_w);
+      piece(r.reads, took(res), s.n, 4, s.ld_res);
+      padded(s.out, es, s.ld_out);
+      padded(s.out2, 4, s.ld_out2);
+      piece(r.touches, s.out3, s.n, es, s.ld_out3);
+      break;
+    case MK_OP_LINEAR:
+    case MK_OP_LINEAR_F32: {
+      const int n_out = glu ? s.n / 2 : s.n;
+      piece(r.reads, took(in), s.k, es, s.ld_in);
+      if (s.flags & (MK_F_ADDNORM | MK_F_PRENORM)) {  // (a single token's norm: the operands are those of the norm stage in front, which is asked about them)
+        for (const void **q : {&y_in, &y2, &slot_w, &res}) took(*q);
+      } else if (s.flags & MK_F_JOIN) {
+        piece(r.reads, took(res), s.n, 4, s.ld_res);
+      } else if (s.flags & MK_F_RES) {
+        piece(r.reads, took(res), n_out, 2, s.ld_res);
+      }
+      // (where this stage does not write these, the norm stage in front or behind does, padding included)
+      const int real = s.flags & (MK_F_ADDNORM | MK_F_PRENORM) ? s.k_real : s.flags & MK_F_NORM ? s.k : s.n;
+      piece(r.touches, s.norm_out, real, es, s.ld_norm);
+      piece(r.touches, s.out2, real, 4, s.ld_out2);
+      piece(r.touches, s.out3, real, es, s.ld_out3);
+      if (s.flags & MK_F_NORM) piece(r.reads, s.norm_out, s.k, es, s.ld_norm);
+      // (some stages sum the slices of the linear in front without storing the rows)
+      const int behind = (s.flags & MK_F_DEFER_SUM) && i + 1 < stages.size() ? stages[i + 1].op : MK_OP_NORM;
+      piece(behind == MK_OP_NORM || behind == MK_OP_MX_PRENORM ? r.writes : r.handed, s.out, n_out, es, s.ld_out);
+      break;
+    }
+    case MK_OP_SILU_MUL: {
+      const int rows = s.topk ? s.topk : 1;
+      pieces(r.reads, took(in), rows, s.ld_in, 2 * s.n, 2, (int64_t)rows * s.ld_in);
+      pieces(r.writes, s.out, rows, s.ld_out, s.n, 2, (int64_t)rows * s.ld_out);
+      break;
+    }
+    case MK_OP_ATTN:
+      piece(r.reads, took(in), (int64_t)(s.num_q_heads + 2 * s.num_kv_heads) * s.head_dim, 2, s.ld_in);
+      took(q_ws);  // (written)
+      piece(r.writes, s.out, (int64_t)s.num_q_heads * s.head_dim, 2, s.ld_out);
+      break;
+    case MK_OP_ARGMAX_PARTIAL:
+    case MK_OP_FX_ARGMAX_F32:
+      piece(r.reads, took(in), s.n, s.op == MK_OP_FX_ARGMAX_F32 ? 4 : 2, s.ld_in);
+      whole(r.writes, took(aux0), (int64_t)B * g->G);
+      whole(r.writes, took(aux1), (int64_t)B * g->G);
+      break;
+    case MK_OP_ARGMAX_REDUCE:
+      whole(r.reads, took(aux0), (int64_t)B * g->G);
+      whole(r.reads, took(aux1), (int64_t)B * g->G);
+      piece(r.writes, s.out, 1, 8, 1);
+      break;
+    case MK_OP_MOE_TOPK:
+      piece(r.reads, took(logits), s.num_experts, 2, s.ld_logits);
+      piece(r.writes, took(topk_w), s.topk, 4, s.ld_topk_w);
+      whole(r.writes, took(routing), (int64_t)s.num_experts * s.ld_routing);
+      break;
+    case MK_OP_MOE_LINEAR: {
+      pieces(r.reads, took(in), s.topk, s.ld_in_slot, s.k, 2, s.ld_in);
+      whole(r.routing, took(routing), (int64_t)s.num_experts * s.ld_routing);
+      if (s.flags & MK_F_MOE_INLINE_TOPK) {  // (what a single token's routing writes, the router in front does for others)
+        piece(r.reads, took(logits), s.num_experts, 2, s.ld_logits);
+        piece(r.touches, took(topk_w), s.topk, 4, s.ld_topk_w);
+        r.touches.push_back(r.routing[0]);
+      } else if (s.flags & MK_F_MOE_COMBINE) {
+        piece(r.reads, took(topk_w), s.topk, 4, s.ld_topk_w);
+      }
+      if (s.flags & MK_F_MOE_COMBINE) {
+        piece(r.reads, took(res), s.n, 2, s.ld_res);
+        piece(r.touches, s.out2, s.n, 2, s.ld_out2);
+      }
+      whole(r.touches, s.moe_mask, s.num_experts + 1);
+      pieces(glu ? r.touches : r.writes, s.out, s.topk, s.ld_out_slot, s.n, 2, s.ld_out);
+      if (glu) pieces(r.writes, s.out2, s.topk, s.ld_out2_slot, s.n / 2, 2, s.ld_out2);
+      break;
+    }
+    case MK_OP_MOE_COMBINE:
+      pieces(r.reads, took(in), s.topk, s.ld_in_slot, s.n, 2, s.ld_in);
+      piece(r.reads, took(topk_w), s.topk, 4, s.ld_topk_w);
+      piece(r.reads, took(res), s.n, 2, s.ld_res);
+      piece(r.writes, s.out, s.n, 2, s.ld_out);
+      break;
+    case MK_OP_MX_HEAD_LINEAR:
+      pieces(r.reads, took(in), s.groups, s.ld_in_slot, s.k, es, s.ld_in);
+      if (s.flags & MK_F_OUT32) piece(r.writes, s.out2, s.n, 4, s.ld_out2);
+      else pieces(r.writes, s.out, s.groups, s.ld_out_slot, s.n, es, s.ld_out);
+      break;
+    case MK_OP_HY_ROUTE:
+      piece(r.reads, took(logits), s.num_experts + (grouped ? 0 : shared), 4, s.ld_logits);
+      took(w_shared);  // (only its presence counts)
+      piece(r.writes, took(ids), s.topk, 4, s.topk);
+      piece(r.writes, took(slot_w), s.topk + shared, 4, s.ld_slot_w);
+      break;
+    case MK_OP_HY_EXPERTS: {
+      pieces(r.reads, in, s.topk, s.ld_in_slot, s.k, es, s.ld_in);
+      if (shared) piece(r.reads, (const char *)in + (int64_t)s.topk * s.ld_in_slot * es, s.k_shared, es, s.ld_in);
+      took(in);
+      piece(r.routing, took(ids), s.topk, 4, s.topk);
+      if (s.flags & MK_F_MOE_INLINE_TOPK) {
+        piece(r.reads, took(logits), s.num_experts + (grouped ? 0 : shared), 4, s.ld_logits);
+        piece(r.touches, took(slot_w), s.topk + shared, 4, s.ld_slot_w);
+        r.touches.push_back(r.routing[0]);
+      }
+      pieces(r.writes, s.out, s.topk, s.ld_out_slot, glu ? s.n / 2 : s.n, es, s.ld_out);
+      if (shared) piece(r.writes, (const char *)s.out + (int64_t)s.topk * s.ld_out_slot * es, glu ? s.n_shared / 2 : s.n_shared, es, s.ld_out);
+      break;
+    }
+    case MK_OP_DU_CONV:
+      piece(r.reads, (const char *)in + (int64_t)s.cols[0] * es, s.n, es, s.ld_in);
+      if (s.step_bias) piece(r.reads, (const char *)in + (int64_t)s.cols[1] * es, s.num_q_heads, es, s.ld_in);
+      took(in);
+      piece(r.writes, s.out, s.n, es, s.ld_out);  // (or the norm in front does)
+      break;
+    case MK_OP_COPY:
+      piece(r.reads, took(in), s.n, 2, s.ld_in);
+      piece(r.writes, s.out, s.n, 2, s.ld_out);
+      break;
+    default:  // (stages that read rows of their own outputs are among these)
+      norm_out = s.norm_out;
+      for (const void *p : {(const void *)s.out, (const void *)s.out2, (const void *)s.out3})
+        if (p) r.elsewhere.push_back(p);
+      break;
+  }
+  r.reads.insert(r.reads.end(), r.routing.begin(), r.routing.end());
+  for (const void *p : {in, res, y_in, y2, slot_w, logits, topk_w, routing, ids, aux0, aux1, q_ws, w_shared, norm_out, s.in2, s.in3, s.w.seg[0], s.w.seg[1], s.w.seg[2], s.norm_w, s.y_norm_w, s.q_norm_w, s.k_norm_w,
+                        (const void *)s.k_cache, (const void *)s.v_cache, s.cos_tab, s.sin_tab, s.sink, (const void *)s.in_bias, (const void *)s.a_tab, (const void *)s.d_tab, (const void *)s.tail,
+                        (const void *)s.temp, (const void *)s.y_scale, (const void *)s.y2_scale, s.conv_w, s.pos_tab, (const void *)s.choice_bias, (const void *)s.step_bias})
+    if (p) r.elsewhere.push_back(p);
+  return r;
+}
+
+// Pieces of memory, joined where they overlap or, with `beside`, lie next to each other.
+struct Extents {
+  bool beside = false;
+  std::map<const char *, const char *> at;  // begin -> end
+  void add(const char *lo, const char *hi) {
+    if (lo >= hi) return;
+    auto it = at.upper_bound(lo);
+    if (it != at.begin() && std::prev(it)->second >= lo + !beside) it = std::prev(it);
+    while (it != at.end() && it->first + !beside <= hi) {
+      lo = std::min(lo, it->first);
+      hi = std::max(hi, it->second);
+      it = at.erase(it);
+    }
+    at[lo] = hi;
+  }
+  bool holds(const char *lo, const char *hi) const {
+    auto it = at.upper_bound(lo);
+    return it != at.begin() && std::prev(it)->second >= hi;
+  }
+};
+
+const char *end_of(const RowSpan &s, int B) { return s.p + (B - 1) * s.stride + s.width; }
+// The pieces of token 0's part of `a` that meet some token's part of `b`, widened to all of it where the rows lie differently.
+std::vector<std::pair<const char *, const char *>> common(const RowSpan &a, const RowSpan &b, int B) {
+  if (a.p >= end_of(b, B) || b.p >= end_of(a, B)) return {};
+  if (a.stride != b.stride || a.stride < a.width || b.stride < b.width || a.width <= 0 || b.width <= 0) return {{a.p, a.p + a.width}};
+  std::vector<std::pair<const char *, const char *>> out;
+  const int64_t d = b.p - a.p, first = (d >= 0 ? d : d - a.stride + 1) / a.stride;  // b begins in a's row `first`
+  for (int64_t j = first; j <= first + 1 && std::abs(j) < B; j++) {  // (its tail may reach into the row behind)
+    const char *lo = std::max(a.p, b.p - j * a.stride), *hi = std::min(a.p + a.width, b.p - j * a.stride + b.width);
+    if (lo < hi) out.push_back({lo, hi});
+  }
+  return out;
+}
+
 // First of the stages at the program's end that leave nothing behind but what this iteration's logits and sampled tokens are made of: behind
 // every stage that writes caches or recurrent states, and behind everything whose effects are not known to end with the iteration.  None
-// (num_stages) where an iteration could read, ahead of writing it, what such a stage of the iteration before has written.
+// (num_stages) where an iteration could read something that such a stage writes before the same part of every token's row is written again.
 int tail_stage(const mk_graph *g) {
-  const int n = (int)g->stages.size();
+  const int n = (int)g->stages.size(), B = g->cfg.max_num_batched_tokens;
   if (g->spec_len > 0) return n;
   auto ends_here = [](const MkStage &s) {
     switch (s.op) {
@@ -1931,40 +2156,64 @@ int tail_stage(const mk_graph *g) {
   while (tail > 0 && ends_here(g->stages[tail - 1])) tail--;
   if (tail > 0 && (g->stages[tail - 1].flags & MK_F_DEFER_SUM)) tail++;  // (its sum may be left to the stage behind it)
   if (tail >= n) return n;
-  // tensors by the widest one that holds an address; the library's own scratch by the address itself
-  std::vector<std::pair<const char *, const char *>> spans;
+  std::vector<StageRows> rows;
+  for (int i = 0; i < n; i++) rows.push_back(rows_of(g, i));
+  std::vector<RowSpan> left;
+  for (int i = tail; i < n; i++) {
+    for (const auto *v : {&rows[i].writes, &rows[i].handed, &rows[i].touches}) left.insert(left.end(), v->begin(), v->end());
+    // padding holds zeros before and after, unless some stage uses those columns for something else
+    for (const RowSpan &z : rows[i].zeros)
+      if (std::any_of(rows.begin(), rows.end(), [&](const StageRows &r) {
+            auto meets = [&](const RowSpan &w) { return !common(z, w, B).empty(); };
+            return std::any_of(r.writes.begin(), r.writes.end(), meets) || std::any_of(r.handed.begin(), r.handed.end(), meets) || std::any_of(r.touches.begin(), r.touches.end(), meets);
+          }))
+        left.push_back(z);
+  }
+  // an operand of which only the address is known may reach as far as the tensors that hold it
+  Extents held;
   for (const Tensor &t : g->tensors) {
     if (!t.ptr || t.kind == T_SHUFFLED) continue;
     size_t last = 0;
     for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
-    spans.push_back({(const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype)});
+    held.add((const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype));
   }
-  std::map<const void *, const void *> known;
-  auto whole = [&](const void *p) {
-    const auto it = known.find(p);
-    if (it != known.end()) return it->second;
-    const char *best = (const char *)p;
-    for (const auto &t : spans)
-      if (p >= t.first && p < t.second && t.first < best) best = t.first;
-    return known[p] = (const void *)best;
+  for (const auto &a : g->alloc_sizes) held.add((const char *)a.first, (const char *)a.first + a.second);
+  std::map<const void *, bool> asked;
+  auto left_elsewhere = [&](const void *p) {
+    const auto known = asked.find(p);
+    if (known != asked.end()) return known->second;
+    const char *lo = (const char *)p, *hi = lo + 1;
+    auto it = held.at.upper_bound(lo);
+    if (it != held.at.begin() && std::prev(it)->second > lo) {
+      it = std::prev(it);
+      lo = it->first;
+      hi = it->second;
+    }
+    return asked[p] = std::any_of(left.begin(), left.end(), [&](const RowSpan &s) { return s.p < hi && lo < end_of(s, B); });
   };
-  auto written = [&](const MkStage &s, std::set<const void *> &to) {
-    for (const void *p : {(const void *)s.out, (const void *)s.out2, (const void *)s.out3, (const void *)s.norm_out, (const void *)s.glu_out,
-                          (const void *)(s.op == MK_OP_HY_ROUTE || s.op == MK_OP_HY_EXPERTS ? s.ids : nullptr),
-                          (const void *)s.moe_topk_w, (const void *)s.moe_routing, (const void *)s.moe_mask})
-      if (p) to.insert(whole(p));
+  const mk_config &c = g->cfg;
+  for (const void *p : {(const void *)c.step, (const void *)c.tokens, (const void *)c.num_new_tokens, (const void *)c.prompt_lengths, (const void *)g->state_ids})  // (the scheduler's)
+    if (p && left_elsewhere(p)) return n;
+  std::map<int64_t, Extents> fresh;  // token 0's part of what the iteration has written so far, by the distance of the rows
+  auto holds = [&](int64_t stride, const char *lo, const char *hi) {
+    const auto f = fresh.find(stride);
+    return f != fresh.end() && f->second.holds(lo, hi);
   };
-  std::set<const void *> left, fresh;
-  for (int i = tail; i < n; i++) written(g->stages[i], left);
   for (int i = 0; i < n; i++) {
-    const MkStage &s = g->stages[i];
-    for (const void *p : {s.in, s.in2, s.in3, s.res, s.y_in, s.y2, (const void *)s.slot_w, s.moe_logits, (const void *)s.moe_topk_w, (const void *)s.moe_routing,
-                          (const void *)s.moe_mask, (const void *)s.ids, s.w.seg[0], s.w.seg[1], s.w.seg[2], s.w_shared, s.norm_w, s.y_norm_w, s.q_norm_w, s.k_norm_w, (const void *)s.q_ws,
-                          (const void *)s.k_cache, (const void *)s.v_cache, s.cos_tab, s.sin_tab, s.sink, (const void *)s.aux0, (const void *)s.aux1, (const void *)s.in_bias,
-                          (const void *)s.a_tab, (const void *)s.d_tab, (const void *)s.temp, (const void *)s.y_scale, (const void *)s.y2_scale, s.conv_w, s.pos_tab,
-                          (const void *)s.choice_bias, (const void *)s.step_bias})
-      if (p && left.count(whole(p)) && !fresh.count(whole(p))) return n;
-    written(s, fresh);
+    const StageRows &r = rows[i];
+    auto handed = [&](const RowSpan &s) {
+      return i > 0 && std::any_of(rows[i - 1].handed.begin(), rows[i - 1].handed.end(), [&](const RowSpan &h) { return h.p == s.p && h.stride == s.stride && h.width >= s.width; });
+    };
+    if (std::any_of(r.elsewhere.begin(), r.elsewhere.end(), left_elsewhere)) return n;
+    for (const RowSpan &s : r.reads) {
+      if (handed(s)) continue;
+      for (const RowSpan &l : left)
+        for (const auto &q : common(s, l, B))
+          if (!holds(s.stride, q.first, q.second)) return n;
+    }
+    if (std::all_of(r.routing.begin(), r.routing.end(), [&](const RowSpan &s) { return holds(s.stride, s.p, s.p + s.width); }))
+      for (const auto *v : {&r.writes, &r.zeros})
+        for (const RowSpan &s : *v) fresh.try_emplace(s.stride, Extents{true, {}}).first->second.add(s.p, s.p + s.width);
   }
   return tail;
 }

@@ -15,9 +15,19 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("lengths", [(150,), (65, 130, 3)])
 def test_session(family, dtype, lengths):
     """Prompts in portions of which only the last rows are wanted, against the same passes with every row wanted."""
+    _session(family, "even", dtype, lengths)
+
+
+# (the last layer of these routes tokens to experts)
+@pytest.mark.parametrize("family,dtype", [("bukatar", torch.bfloat16), ("bukatar", torch.float32), ("vizonex", torch.bfloat16), ("vizonex", torch.float32)])
+def test_session_of_a_model_that_ends_with_experts(family, dtype):
+    _session(family, "odd", dtype, (65, 130, 3))
+
+
+def _session(family, kind, dtype, lengths):
     from mirage.mpk import MirageModelConfig, ServingSession
     h = importlib.import_module(family + "_helpers")
-    cfg = h.CONFIGS["even"]
+    cfg = h.CONFIGS[kind]
     w = {k: v.cuda() for k, v in h.weights(cfg).items()}
     outs = []
     for every in (False, True):
