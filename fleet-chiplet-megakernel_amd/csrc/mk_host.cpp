@@ -199,6 +199,7 @@ struct mk_graph {
   bool single_copy = false;
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
   int tail = 0;      // MkRuntime::tail
+  int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
   int64_t row_major_bytes = 0;
@@ -3042,6 +3043,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
   HIP_TRY(hipEventRecord(g->ev1, stream));
   g->launch_pending = true;
+  g->last_stages = run_scheduler == MK_SCHED_INGEST && !rt->profiler && rt->max_tokens > 1 ? rt->tail : rt->num_stages;
   g->launch_stream = stream;
   g->ms_due = true;
   HIP_TRY(launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status));
@@ -3752,7 +3754,7 @@ static int copy_stage_ticks(mk_graph *g, int workgroup, int first, int64_t *tick
   std::vector<long long> buf((size_t)MK_PROF_TICKS * recs);
   HIP_TRY(hipMemcpy(buf.data(), g->h_rt.stage_prof + (size_t)MK_PROF_TICKS * workgroup * recs, sizeof(long long) * buf.size(), hipMemcpyDeviceToHost));
   for (int s = 0; s < n; s++)
-    for (int k = 0; k < 4; k++) ticks_out[4 * s + k] = buf[(size_t)MK_PROF_TICKS * s + first + k];
+    for (int k = 0; k < 4; k++) ticks_out[4 * s + k] = s >= g->last_stages && s < recs - 1 ? 0 : buf[(size_t)MK_PROF_TICKS * s + first + k];  // (left out: an older iteration's)
   return n;
 }
 

@@ -1121,7 +1121,7 @@ class PersistentKernel:
     def stage_profile(self, workgroup: int = 0, raw: bool = False, marks: bool = False):
         """Per-stage timing of the last iteration on one virtual workgroup: list of (description, entered,
         barrier_satisfied, work_done, arrived) in microseconds relative to that workgroup's first stage (raw=True:
-        100 MHz ticks, comparable across workgroups; 0 = stage skipped).  The last entry, "SCHEDULER", times the scheduler
+        100 MHz ticks, comparable across workgroups; 0 = stage never run, or left out by enqueue_ingest).  The last entry, "SCHEDULER", times the scheduler
         step that opened the iteration: (previous iteration complete, batch prepared [workgroup 0], batch published, 0).
         marks=True returns the four in-stage marks of a library built with -DMK_TRACE instead."""
         n = self.stats()["num_stages"] + 1

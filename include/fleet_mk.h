@@ -208,7 +208,8 @@ typedef struct mk_stats {
 } mk_stats;
 int mk_get_stats(mk_graph *g, mk_stats *out);
 /* Device-side stage timing of the LAST decode iteration, as seen by virtual workgroup `workgroup`: for each stage four
- * 100 MHz wall-clock ticks {entered, previous stage's barrier satisfied, work done, arrival posted}.  Returns the number
+ * 100 MHz wall-clock ticks {entered, previous stage's barrier satisfied, work done, arrival posted}, zeros for the stages that
+ * mk_enqueue_ingest left out.  Returns the number
  * of stages written (<= max_stages).  One record more than there are stages may be asked for: the last one times the
  * scheduler step of that iteration {previous iteration complete, batch prepared (workgroup 0 only), batch published to
  * this workgroup, 0}.  Counterpart of the reference's MPK_ENABLE_EVENT_TIMING ring

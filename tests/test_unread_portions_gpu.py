@@ -107,6 +107,28 @@ def test_what_an_unread_batch_leaves():
     off.mpk.finalize()
 
 
+def test_stage_times_of_an_unread_batch():
+    """Stages that were left out show no times, those that ran show this batch's."""
+    from oracle.qwen3_ref import make_model_weights
+    cfg = _cfg()
+    on = _decoder(cfg, make_model_weights(cfg, seed=48), max_num_batched_tokens=8, max_num_batched_requests=1, max_seq_length=16, page_size=16, kernel_mode="online_notoken")
+    _described(on.meta, 8)
+    on.mpk()
+    before = on.mpk.stage_profile(raw=True)
+    ran = [line[3] > 0 for line in before]
+    on.mpk.enqueue_ingest()
+    on.mpk.wait()
+    for old, new, r in zip(before, on.mpk.stage_profile(raw=True), ran):
+        if old[0].endswith("unread=skip"):
+            assert tuple(new[1:]) == (0, 0, 0, 0)
+        elif r:
+            assert new[3] > old[3]
+    assert any(line[0].endswith("unread=skip") for line in before)
+    on.mpk()
+    assert [line[3] > 0 for line in on.mpk.stage_profile(raw=True)] == ran
+    on.mpk.finalize()
+
+
 @pytest.mark.parametrize("carried", [False, True])
 def test_rows_carried_from_one_iteration_to_the_next(carried):
     """A stage at the end whose output an iteration reads before it is written again runs in every iteration."""
