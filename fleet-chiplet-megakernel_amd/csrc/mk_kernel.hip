@@ -2730,24 +2730,28 @@ __device__ __forceinline__ void moe_build_lists(CStage &st, const Ctx &c, MoeLds
   __syncthreads();
 }
 
-// Per-expert linear of one token, whichever the sizes: y[slot, :] = W[e(slot)] x(slot), one weight row (or one
-// [gate ; up] row pair) per wavefront step.
+// Per-expert linear over the active experts: y[t, slot, :] = W[e(t,slot)] x(t, slot), one weight row (or one
+// [gate ; up] row pair) per wavefront step, each row read once and applied to every token routed to its expert.
 // Work units (active expert, row) are dealt out in contiguous runs per wavefront; the rows of the next R units are
 // in flight in registers while a unit is reduced.  Optional epilogues: SwiGLU (gate and up rounded to bf16 first, as
-// the separate activation task of the reference sees them) and the weighted sum over the
+// the separate activation task of the reference sees them) and, for a single token, the weighted sum over the
 // slots plus residual, accumulated in slot order in fp32 from the bf16-rounded expert outputs.
 // KL = 16-byte row segments per lane (K <= 512 KL).
 // Reference tasks: moe_linear_kernel_mi300 (tasks/mi300/moe_linear_mi300.cuh:53-295), silu_mul_task_impl,
 // mul_sum_add_mi300_task_impl (tasks/mi300/moe_mul_sum_add_mi300.cuh:31-55).
 template <int KL, int R, bool SILU>
-__device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, char *smem) {
+__device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, int M, char *smem) {
   constexpr int NROW = SILU ? 2 : 1;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   MoeLds *L = (MoeLds *)(smem + MK_MOE_OFFSET);
   const int k8 = st.k / 8;
-  const bool combine = !SILU && (st.flags & MK_F_MOE_COMBINE);
-  const bool inline_topk = st.flags & MK_F_MOE_INLINE_TOPK;
+  const bool combine = !SILU && (st.flags & MK_F_MOE_COMBINE) && M == 1;
+  const bool inline_topk = (st.flags & MK_F_MOE_INLINE_TOPK) && M == 1;
   barrier_wait(c);
+  if (M > 1) {  // activation rows are read with cached loads below: drop stale lines of this CU's L1 first
+    if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
+  }
   if (inline_topk) {
     if (wave == 0) {
       int sel[4];
@@ -2769,15 +2773,15 @@ __device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, char *sme
   } else if (combine && tid < st.topk) {
     L->w[tid] = ldc_f32(st.moe_topk_w + tid);
   }
-  moe_build_lists(st, c, L, 1, inline_topk);
+  moe_build_lists(st, c, L, M, inline_topk);
   const int n_act = L->n_act;
   if (c.vid == 0 && st.moe_mask) {  // publish the active-expert list (its order is unspecified in the reference)
     for (int i = tid; i < st.num_experts; i += MK_THREADS) st.moe_mask[i] = i < n_act ? L->act_e[i] : -1;
     if (tid == 0) st.moe_mask[st.num_experts] = n_act;
   }
-  // stage the input row(s) in LDS (one row, or one row per slot) where they fit
+  // single token: stage the input row(s) in LDS (one row, or one row per slot)
   const int nslot_in = st.ld_in_slot ? st.topk : 1;
-  const bool x_lds = (size_t)nslot_in * st.k * 2 <= (size_t)MK_RED_OFFSET;
+  const bool x_lds = M == 1 && (size_t)nslot_in * st.k * 2 <= (size_t)MK_RED_OFFSET;
   u32x4 *xs4 = (u32x4 *)smem;
   if (x_lds) {
     for (int i = tid; i < nslot_in * k8; i += MK_THREADS) {
@@ -2839,27 +2843,28 @@ __device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, char *sme
         const int p0 = L->pair_off[a], p1 = L->act_e[a] >= 0 ? L->pair_off[a + 1] : p0;
         if (combine && a == 0) comb = bf2f(ldc_u16((const uint16_t *)st.res + j));
         for (int p = p0; p < p1; p++) {
-          const int slot = L->pair_ts[p] >> 8;
-          const u32x4 *x = x_lds ? xs4 + (st.ld_in_slot ? slot * k8 : 0) : (const u32x4 *)((const uint16_t *)st.in + (size_t)slot * st.ld_in_slot);
+          const int ts = L->pair_ts[p], tok = ts & 255, slot = ts >> 8;
+          const u32x4 *x = x_lds ? xs4 + (st.ld_in_slot ? slot * k8 : 0)
+                                 : (const u32x4 *)((const uint16_t *)st.in + (size_t)tok * st.ld_in + (size_t)slot * st.ld_in_slot);
           float acc[NROW];
 #pragma unroll
           for (int h = 0; h < NROW; h++) acc[h] = 0.f;
 #pragma unroll
           for (int kc = 0; kc < KL; kc++) {
             u32x4 xv = zero;
-            if (kc * 64 + lane < k8) xv = x_lds ? x[kc * 64 + lane] : ldc_16B(x + kc * 64 + lane);
+            if (kc * 64 + lane < k8) xv = (x_lds || M > 1) ? x[kc * 64 + lane] : ldc_16B(x + kc * 64 + lane);
 #pragma unroll
             for (int h = 0; h < NROW; h++) acc[h] = dot8(buf[jj][h][kc], xv, acc[h]);
           }
 #pragma unroll
           for (int h = 0; h < NROW; h++) acc[h] = wave_sum(acc[h]);
-          uint16_t *y = out + (size_t)slot * st.ld_out_slot;
+          uint16_t *y = out + (size_t)tok * st.ld_out + (size_t)slot * st.ld_out_slot;
           if (SILU) {
             const uint32_t g = f2bf(acc[0]), up = f2bf(acc[NROW - 1]);
             if (lane == 0) {
               y[j] = (uint16_t)g;
               y[j + NR] = (uint16_t)up;
-              out2[(size_t)slot * st.ld_out2_slot + j] = (uint16_t)f2bf(silu_mul(bf2f((uint16_t)g), bf2f((uint16_t)up)));
+              out2[(size_t)tok * st.ld_out2 + (size_t)slot * st.ld_out2_slot + j] = (uint16_t)f2bf(silu_mul(bf2f((uint16_t)g), bf2f((uint16_t)up)));
             }
           } else {
             const uint32_t v = f2bf(acc[0]);
@@ -3439,14 +3444,14 @@ __device__ __forceinline__ void stage_moe_linear(CStage &st, Ctx &c, int M, char
     return;
   }
   if (st.k <= 1024) {
-    if (silu) stage_moe_linear_t<2, 4, true>(st, c, smem);
-    else stage_moe_linear_t<2, 6, false>(st, c, smem);
+    if (silu) stage_moe_linear_t<2, 4, true>(st, c, M, smem);
+    else stage_moe_linear_t<2, 6, false>(st, c, M, smem);
   } else if (st.k <= 2048) {
-    if (silu) stage_moe_linear_t<4, 3, true>(st, c, smem);
-    else stage_moe_linear_t<4, 4, false>(st, c, smem);
+    if (silu) stage_moe_linear_t<4, 3, true>(st, c, M, smem);
+    else stage_moe_linear_t<4, 4, false>(st, c, M, smem);
   } else {
-    if (silu) stage_moe_linear_t<8, 1, true>(st, c, smem);
-    else stage_moe_linear_t<8, 2, false>(st, c, smem);
+    if (silu) stage_moe_linear_t<8, 1, true>(st, c, M, smem);
+    else stage_moe_linear_t<8, 2, false>(st, c, M, smem);
   }
 }
 
