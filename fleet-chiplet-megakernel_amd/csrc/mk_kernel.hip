@@ -3975,20 +3975,25 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 
 
 #define MK_ATTN_PAIR_PAGES 1024  // page-table entries of a request where a workgroup works on two units at a time
-#ifndef MK_TUNE_ATTN_SPREAD
-#define MK_TUNE_ATTN_SPREAD 384
-#endif
-// Whether a workgroup takes two units at a time (below): there are more of them than workgroups, and the longest context is not far above
-// the average, which two wavefronts walk in twice the time that four take.  64 requests, 32 q / 8 kv heads, as a stage, one unit after the
-// other -> two at a time, us: contexts of 320 32.0 -> 24.0; of 100 .. 700 (300 above the average) 35.0 -> 34.3; 63 of 20 and one of 300 22.8 ->
-// 19.9; of 100 .. 1480 (690 above) 49.2 -> 60.7; 63 of 20 and one of 900 33.6 -> 40.3.
-template <int QPK>
-__device__ __forceinline__ bool attn_in_pairs(CStage &st, const Ctx &c, const MkRuntime &rt, int M) {
+// Whether a workgroup takes two units at a time (below).  One after the other, its units take as many turns as the workgroup has; two at a time
+// half of them, rounded up, which last as long as the longer of the two and walk a context with two wavefronts instead of four.  So pairs save
+// what a turn costs besides its positions (420 positions' worth, 320 with eight queries a head, of which two wavefronts prepare twice as many)
+// and lose 0.95 of every position that the second unit does not have as well, and half a turn where the number of turns is odd.  The longest turn of
+// pairs is taken to be the longest context's, the others average ones; a workgroup that takes one after the other has at least the average
+// of all, or the longest context and the shortest ones.
+// As a stage of 64 requests, us, one after the other -> two at a time.  Two turns (8 kv heads, 4 queries): contexts of 320 29.5 -> 21.8, 1000 54.5 ->
+// 48.4, 1480 73.5 -> 66.8; of 1000 .. 1480 66.2 -> 63.9, 100 .. 700 34.4 -> 34.4, 100 .. 850 36.6 -> 40.1, 1000 .. 1700 69.3 -> 70.9; 63 of 20 and one
+// of 390 25.3 -> 23.7, of 900 33.6 -> 40.3.  Three turns (12 kv heads): 320 43.9 -> 39.1, 510 53.4 -> 53.3, 700 65.5 -> 67.3, 1000 83.5 -> 90.5, 100 .. 700
+// 50.3 -> 53.1; with 8 queries 320 45.8 -> 44.8, 450 55.2 -> 56.8.  Four (16): 320 56.4 -> 40.9, 1480 149.5 -> 136.4, 100 .. 850 70.4 -> 65.5, 100 .. 1480
+// 94.3 -> 95.3.  Five (20): 700 108.6 -> 102.4, 1000 136.9 -> 137.9, 1480 185.7 -> 190.0.  (By the longest context's distance from the average, 384,
+// three turns of 1000 and 1480 positions had become 10 % and 12 % slower than one unit after the other, two turns of 100 .. 850 9 %.)
+__device__ __forceinline__ bool attn_in_pairs(CStage &st, const Ctx &c, const MkRuntime &rt, int M, int qpk) {
   const int lane = threadIdx.x & 63, first = lane < M ? c.sh_tok[2 * MK_MAX_TOKENS + lane] : 0;
-  if (__popcll(__ballot(lane < M && (lane - first) % (16 / QPK) == 0)) * st.num_kv_heads <= c.G || (rt.max_seq + rt.page_size - 1) / rt.page_size > MK_ATTN_PAIR_PAGES) return false;
-  const int pos = lane < M ? c.sh_tok[lane] : 0;
-  const float mean = wave_sum((float)pos) / (float)M;
-  return !__any((float)pos > mean + (float)MK_TUNE_ATTN_SPREAD);
+  const int units = __popcll(__ballot(lane < M && ((lane - first) & (16 / qpk - 1)) == 0)) * st.num_kv_heads, turns = (units + c.G - 1) / c.G, pairs = (turns + 1) / 2;
+  if (turns < 2 || (rt.max_seq + rt.page_size - 1) / rt.page_size > MK_ATTN_PAIR_PAGES) return false;
+  const float pos = lane < M ? (float)c.sh_tok[lane] : 0.f;
+  const float mean = wave_sum(pos) / (float)M, most = wave_max(pos), least = -wave_max(lane < M ? -pos : -most);
+  return 1.95f * (most + (float)(pairs - 1) * mean) <= (qpk == 4 ? 420.f : 320.f) * (float)(turns - pairs) + fmaxf((float)turns * mean, most + (float)(turns - 1) * least);
 }
 
 // The same for iterations of many tokens, on the matrix cores.  Work unit = (up to 16 / QPK consecutive tokens of one request, kv head,
@@ -4832,13 +4837,14 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
             else barrier_wait(c);
           } else {
             // many (token, kv head) pairs per workgroup-chunk: cached positions on the matrix cores
-            const bool mf = 2 * M * st.num_kv_heads >= c.G;
-            if (st.num_q_heads == 4 * st.num_kv_heads) {
-              if (mf && attn_in_pairs<4>(st, c, rt, M)) stage_attn_tiles<4, true>(st, c, rt, M, smem);
+            const bool mf = 2 * M * st.num_kv_heads >= c.G, four = st.num_q_heads == 4 * st.num_kv_heads, eight = st.num_q_heads == 8 * st.num_kv_heads;
+            const bool pairs = mf && (four || eight) && attn_in_pairs(st, c, rt, M, four ? 4 : 8);
+            if (four) {
+              if (pairs) stage_attn_tiles<4, true>(st, c, rt, M, smem);
               else if (mf) stage_attn_tiles<4, false>(st, c, rt, M, smem);
               else stage_attn<4>(st, c, rt, M, smem);
-            } else if (st.num_q_heads == 8 * st.num_kv_heads) {
-              if (mf && attn_in_pairs<8>(st, c, rt, M)) stage_attn_tiles<8, true>(st, c, rt, M, smem);
+            } else if (eight) {
+              if (pairs) stage_attn_tiles<8, true>(st, c, rt, M, smem);
               else if (mf) stage_attn_tiles<8, false>(st, c, rt, M, smem);
               else stage_attn<8>(st, c, rt, M, smem);
             } else {

@@ -23,15 +23,28 @@ def _lens(kind, R):
                                                    (64, "one long", 1, 64, 8, 4), (40, "near", 2, 16, 8, 4), (64, "520", 1, 2048, 5, 8)])
 def test_attention_of_many_requests(R, kind, new, ps, nkv, qpk):
     """`new`: rows of the first requests, as many as 64 rows allow."""
+    _check(_lens(kind, R), new, ps, nkv, qpk, 7 * R + len(kind))
+
+
+# (requests of 1024 pages fill a unit's page list when two are taken at a time, of 1025 are taken one at a time; two, three and five turns of a
+# workgroup, of which the longest contexts just allow two units at a time or just do not, on either side of the line that the rule draws)
+@pytest.mark.parametrize("lens,ps,nkv,qpk,max_seq", [([1024] * 64, 1, 5, 8, 1024), ([1024] * 64, 1, 5, 8, 1025), ([1024] + [1000] * 63, 1, 8, 4, 1024),
+                                                     ([20] * 63 + [430], 16, 8, 4, 1024), ([20] * 63 + [500], 16, 8, 4, 1024), ([455] * 64, 16, 12, 4, 1024), ([480] * 64, 16, 12, 4, 1024),
+                                                     ([345] * 64, 16, 12, 8, 1024), ([370] * 64, 16, 12, 8, 1024), ([980] * 64, 16, 20, 4, 1024), ([1000] * 64, 16, 20, 4, 1024)])
+def test_attention_at_the_limits_of_two_units_at_a_time(lens, ps, nkv, qpk, max_seq):
+    _check(lens, 1, ps, nkv, qpk, sum(lens), max_seq)
+
+
+def _check(lens, new, ps, nkv, qpk, seed, max_seq=None):
     import mirage as mi
-    cached = [n - 1 for n in _lens(kind, R)]
+    R, cached = len(lens), [n - 1 for n in lens]
     rows = [new if i < (64 - R) // max(1, new - 1) and new > 1 else 1 for i in range(R)]
     total, longest = sum(rows), max(c + n for c, n in zip(cached, rows))
     need = [-(-(c + n) // ps) for c, n in zip(cached, rows)]
-    pages, max_seq = sum(need), -(-(longest + 1) // ps) * ps
+    pages, max_seq = sum(need), max_seq or -(-(longest + 1) // ps) * ps
     meta = make_meta(R, max_seq, 64, R, pages)
     pk = make_mpk(meta, max_seq, 64, R, pages, ps, mode="onepass")
-    g = torch.Generator().manual_seed(7 * R + len(kind))
+    g = torch.Generator().manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).cuda()
     qkv, kc, vc, out = rnd(64, nkv * (qpk + 2) * D), rnd(pages, ps, nkv, D), rnd(pages, ps, nkv, D), torch.zeros(64, nkv * qpk * D, dtype=torch.bfloat16, device="cuda")
     k0, v0 = kc.clone(), vc.clone()
