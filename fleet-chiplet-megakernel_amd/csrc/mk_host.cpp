@@ -2594,6 +2594,23 @@ int lower(mk_graph *g) {
     const bool not_dual = (op >= MK_OP_MX_LATENT_PREP && op <= MK_OP_MX_DELTA_OUT && op != MK_OP_MX_HEAD_LINEAR) || (op >= MK_OP_HY_CONV && op <= MK_OP_HY_SCAN);
     if (!ok || (g->dual && not_dual)) return fail(MK_EUNSUPPORTED, "stage %zu (%s) cannot run in one graph with the others", s, g->stage_desc[s].c_str());
   }
+  // stages of several tokens that reach their input rows by 32-bit offsets from the first one
+  for (size_t s = 0; s < g->stages.size() && B > 1; s++) {
+    const MkStage &st = g->stages[s];
+    int64_t cols = 0, es = g->flex == FLEX_F32 ? 4 : 2;
+    switch (st.op) {
+      case MK_OP_LINEAR: case MK_OP_LINEAR_F32: cols = st.k; break;
+      case MK_OP_MOE_LINEAR: case MK_OP_HY_EXPERTS: cols = (int64_t)st.topk * st.ld_in_slot + std::max(st.k, st.k_shared); break;
+      case MK_OP_MX_HEAD_LINEAR: case MK_OP_HY_STEP: case MK_OP_MX_DECAY: cols = (int64_t)(st.groups - 1) * st.ld_in_slot + st.k; break;
+      case MK_OP_ARGMAX_PARTIAL: case MK_OP_FX_ARGMAX_F32:
+        cols = st.n;
+        es = st.op == MK_OP_ARGMAX_PARTIAL ? 2 : 4;
+        break;
+      default: continue;
+    }
+    const int64_t span = ((B - 1) * (int64_t)std::max(st.ld_in, (st.flags & MK_F_NORM) ? st.ld_norm : 0) + cols) * es;
+    if (span > 0xffffffffll) return fail(MK_EUNSUPPORTED, "stage %zu (%s): its input rows span %lld bytes (at most 4 GiB)", s, g->stage_desc[s].c_str(), (long long)span);
+  }
   for (auto &st : g->stages) {  // the task type a stage is shown as in a profiler trace (runtime_header.h:91-188)
     switch (st.op) {
       case MK_OP_EMBED: st.prof_event = 101; break;
