@@ -637,8 +637,9 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
   };
   const bool early = single && have0 && wave != 0;  // (the polling wavefront keeps its memory queue empty)
   if (early) load_first(a0);
-  // (Keys and values are read with cached loads: a line that holds one of this iteration's positions is read by nobody between the cache
-  // invalidate that opens the iteration and the barrier behind the stage that writes them.)
+  // (Keys and values are read with cached loads.  Where some request brings several tokens, nothing of this layer's cache is requested before the
+  // barrier behind the stage that writes the new positions.  Where every request brings one, tiles are requested early, and a line with the
+  // new position may be cached as it was before: that position always comes from LDS, and the next iteration opens with an invalidate.)
   barrier_wait(c);
   c.wrote_through = true;
   FxRows<E> rows{};

@@ -3968,8 +3968,8 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
     }
   }
   // The attention outputs went through to memory.  The appended K/V rows and the published q rows stay in this die's
-  // L2 until a later barrier of this iteration writes it back (the sampling stages and the scheduler step always do);
-  // nothing reads them before the next iteration.
+  // L2 until something writes it back: the barrier behind the scheduler step that opens the next iteration, or the end of the launch.  (No
+  // later stage of this iteration needs to.)  Nothing reads them before the next iteration.
   c.wrote_through = true;
 }
 
@@ -4414,8 +4414,10 @@ __device__ __forceinline__ void stage_argmax_partial(CStage &st, Ctx &c, const M
   float *sv = (float *)smem;  // [MAXM] values, [MAXM] indices
   int *si = (int *)smem + MAXM;
   barrier_wait(c);
-  // One token only: a wavefront takes the slice, a dword a lane.  By sixteen lanes the kernel of one token was 15 us a pass slower with 151936
-  // logits (2.991 -> 2.976 ms a token, 36 layers; before that form 2.969); loads by the lanes of the token alone changed nothing (2.991).
+  // One token only: a wavefront takes the slice, a dword a lane.  By sixteen lanes the fixed-shape kernel of one token was 15 us a pass slower with
+  // 151936 logits (2.991 -> 2.976 ms a token, 36 layers; before that form 2.969), more than the stage takes: it moves the register allocation of the
+  // linears.  The kernels of the other stage sets do not care: 64 tokens with 32768 logits, by sixteen lanes / by a wavefront, suborax-8b 43.73 / 43.68 ms,
+  // dodonex-8b 47.96 / 47.91, bukatar-8b 33.56 / 33.50, vizonex-8b 33.34 / 33.41 (qwen3-8b 41.86 / 41.78).
   if constexpr (MAXM == 1 && sizeof(E) == 2) {
     const int per = ((n + c.G - 1) / c.G + 1) & ~1, c0 = c.vid * per, c1 = min(n, c0 + per), nd = (c1 - c0 + 1) / 2;
     if (tid < 64) {
@@ -5018,8 +5020,9 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       pr[2] = (long long)wall_clock64();
     }
     // An iteration that only brings prompts forward ends with the last stage that writes caches or recurrent states: the logits and sampled
-    // tokens of rows in front of a prompt's last token are read by nobody.  The last iteration of a launch is run whole, so that every buffer
-    // the caller can look at holds what it always did, and so is every one that a profiler tensor is to show; where requests bring one token
+    // tokens of rows in front of a prompt's last token are read by nobody.  The last iteration of a launch is run whole, so that the caller finds
+    // its tokens' rows in every buffer (rows behind its last token hold those of an older iteration that was run whole and had as many), and so
+    // is every one that a profiler tensor is to show; where requests bring one token
     // at a time, prompts are walked as decoding walks them, all stages included.  (A prompt of 2501 tokens of qwen3-8b, 8 layers, vocabulary
     // 32768: 46.7 -> 41.1 ms; prompts of four requests of suborax-8b 1175 -> 994 us a pass, 32-bit 868 -> 676.)
     int n_stages = rt.num_stages;

@@ -148,6 +148,8 @@ int mk_compile(mk_graph *g);
 int mk_init_requests(mk_graph *g);
 /* Replaces launch_persistent_kernel (persistent_kernel.cuh:2260-2329): one cooperative launch that runs until all
  * requests are finished (offline / online modes) or over the one batch the host described (online_notoken / onepass).
+ * Row buffers hold the rows of the last iteration's tokens; what lies behind them is of older iterations, not always of the last that
+ * had as many tokens (iterations that only bring prompts forward end behind the last cache or state).
  * Blocks until the kernel has drained, like the reference. `stream` is a hipStream_t (may be 0). */
 int mk_launch(mk_graph *g, void *stream);
 /* Same kernel, but returns after at most `max_iterations` decode iterations; scheduler state persists in HBM so the
