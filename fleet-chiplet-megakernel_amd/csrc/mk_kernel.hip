@@ -2732,7 +2732,7 @@ __device__ __forceinline__ void moe_build_lists(CStage &st, const Ctx &c, MoeLds
 
 // Per-expert linear over the active experts of one token, whatever the sizes: y[slot, :] = W[e(slot)] x(slot), one weight row (or one
 // [gate ; up] row pair) per wavefront step.  (M is 1.  Written without it and without the token index, the register allocation of the multi-token
-// linears in the same kernel moved: a prompt of qwen3-8b 39.7 -> 39.8 ms, with the rule of attn_in_pairs 40.0 to 40.4 instead of 39.8.)
+// linears in the same kernel moved: a prompt of qwen3-8b 39.7 -> 39.8 ms, with the rule of attn_in_pairs up to 40.4.)
 // Work units (active expert, row) are dealt out in contiguous runs per wavefront; the rows of the next R units are
 // in flight in registers while a unit is reduced.  Optional epilogues: SwiGLU (gate and up rounded to bf16 first, as
 // the separate activation task of the reference sees them) and the weighted sum over the
@@ -3979,21 +3979,24 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
 // half of them, rounded up, which last as long as the longer of the two and walk a context with two wavefronts instead of four.  So pairs save
 // what a turn costs besides its positions (420 positions' worth, 320 with eight queries a head, of which two wavefronts prepare twice as many)
 // and lose 0.95 of every position that the second unit does not have as well, and half a turn where the number of turns is odd.  The longest turn of
-// pairs is taken to be the longest context's, the others average ones; a workgroup that takes one after the other has at least the average
-// of all, or the longest context and the shortest ones.
+// pairs is taken to be the longest context's, the others average ones; a workgroup that takes one after the other is taken to walk average
+// contexts, or the longest one, whichever is more.  (With the shortest contexts beside the longest, or with the sum in one place for both query
+// counts, the rule is no better and the linears of the same kernel get other registers: 3 to 25 tokens of qwen3-8b 0.6 to 0.9 % slower.)
 // As a stage of 64 requests, us, one after the other -> two at a time.  Two turns (8 kv heads, 4 queries): contexts of 320 29.5 -> 21.8, 1000 54.5 ->
 // 48.4, 1480 73.5 -> 66.8; of 1000 .. 1480 66.2 -> 63.9, 100 .. 700 34.4 -> 34.4, 100 .. 850 36.6 -> 40.1, 1000 .. 1700 69.3 -> 70.9; 63 of 20 and one
 // of 390 25.3 -> 23.7, of 900 33.6 -> 40.3.  Three turns (12 kv heads): 320 43.9 -> 39.1, 510 53.4 -> 53.3, 700 65.5 -> 67.3, 1000 83.5 -> 90.5, 100 .. 700
 // 50.3 -> 53.1; with 8 queries 320 45.8 -> 44.8, 450 55.2 -> 56.8.  Four (16): 320 56.4 -> 40.9, 1480 149.5 -> 136.4, 100 .. 850 70.4 -> 65.5, 100 .. 1480
 // 94.3 -> 95.3.  Five (20): 700 108.6 -> 102.4, 1000 136.9 -> 137.9, 1480 185.7 -> 190.0.  (By the longest context's distance from the average, 384,
 // three turns of 1000 and 1480 positions had become 10 % and 12 % slower than one unit after the other, two turns of 100 .. 850 9 %.)
-__device__ __forceinline__ bool attn_in_pairs(CStage &st, const Ctx &c, const MkRuntime &rt, int M, int qpk) {
+template <int QPK>
+__device__ __forceinline__ bool attn_in_pairs(CStage &st, const Ctx &c, const MkRuntime &rt, int M) {
   const int lane = threadIdx.x & 63, first = lane < M ? c.sh_tok[2 * MK_MAX_TOKENS + lane] : 0;
-  const int units = __popcll(__ballot(lane < M && ((lane - first) & (16 / qpk - 1)) == 0)) * st.num_kv_heads, turns = (units + c.G - 1) / c.G, pairs = (turns + 1) / 2;
+  const int units = __popcll(__ballot(lane < M && (lane - first) % (16 / QPK) == 0)) * st.num_kv_heads, turns = (units + c.G - 1) / c.G, pairs = (turns + 1) / 2;
   if (turns < 2 || (rt.max_seq + rt.page_size - 1) / rt.page_size > MK_ATTN_PAIR_PAGES) return false;
-  const float pos = lane < M ? (float)c.sh_tok[lane] : 0.f;
-  const float mean = wave_sum(pos) / (float)M, most = wave_max(pos), least = -wave_max(lane < M ? -pos : -most);
-  return 1.95f * (most + (float)(pairs - 1) * mean) <= (qpk == 4 ? 420.f : 320.f) * (float)(turns - pairs) + fmaxf((float)turns * mean, most + (float)(turns - 1) * least);
+  const int pos = lane < M ? c.sh_tok[lane] : 0;
+  const float mean = wave_sum((float)pos) / (float)M;
+  const float save = (QPK == 4 ? 420.f : 320.f) * (float)(turns - pairs) - 1.95f * (float)(pairs - 1) * mean;
+  return !__any((float)pos > fmaxf((save + (float)turns * mean) * (1.f / 1.95f), save * (1.f / 0.95f)));
 }
 
 // The same for iterations of many tokens, on the matrix cores.  Work unit = (up to 16 / QPK consecutive tokens of one request, kv head,
@@ -4839,14 +4842,13 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
             else barrier_wait(c);
           } else {
             // many (token, kv head) pairs per workgroup-chunk: cached positions on the matrix cores
-            const bool mf = 2 * M * st.num_kv_heads >= c.G, four = st.num_q_heads == 4 * st.num_kv_heads, eight = st.num_q_heads == 8 * st.num_kv_heads;
-            const bool pairs = mf && (four || eight) && attn_in_pairs(st, c, rt, M, four ? 4 : 8);
-            if (four) {
-              if (pairs) stage_attn_tiles<4, true>(st, c, rt, M, smem);
+            const bool mf = 2 * M * st.num_kv_heads >= c.G;
+            if (st.num_q_heads == 4 * st.num_kv_heads) {
+              if (mf && attn_in_pairs<4>(st, c, rt, M)) stage_attn_tiles<4, true>(st, c, rt, M, smem);
               else if (mf) stage_attn_tiles<4, false>(st, c, rt, M, smem);
               else stage_attn<4>(st, c, rt, M, smem);
-            } else if (eight) {
-              if (pairs) stage_attn_tiles<8, true>(st, c, rt, M, smem);
+            } else if (st.num_q_heads == 8 * st.num_kv_heads) {
+              if (mf && attn_in_pairs<8>(st, c, rt, M)) stage_attn_tiles<8, true>(st, c, rt, M, smem);
               else if (mf) stage_attn_tiles<8, false>(st, c, rt, M, smem);
               else stage_attn<8>(st, c, rt, M, smem);
             } else {
