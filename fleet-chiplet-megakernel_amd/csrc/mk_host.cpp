@@ -137,15 +137,20 @@ size_t dtype_size(int dt) {
 struct LaunchStatus {
   unsigned xcd_count[MK_MAX_XCD];
   unsigned abort_flag, abort_where;
+  long long t_begin, t_end;
   MkSched sched;
 };
-// Runs behind every launch: one workgroup puts the outcome in pinned host memory and leaves the barrier state zeroed for the next launch.
-// (Bound by the launch; a memset in front and two pageable copies behind cost 12 + 2 x 13 us per launch on MI355X, this adds about 1.)
-__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out) {
+// Runs behind every launch: one workgroup puts the outcome (and, for mk_enqueue_batch, the sampled tokens) in pinned host memory and leaves
+// the barrier state zeroed for the next launch.
+// (Bound by the launch; a memset in front and two pageable copies behind cost 12 + 2 x 13 us per launch on MI355X, this adds about 1.5.)
+__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out, const long long *tokens, int num_tokens, long long *host_tokens) {
   const unsigned t = threadIdx.x;
-  if (t < MK_MAX_XCD) out->xcd_count[t] = sync->xcd_count[t];
+  for (int i = (int)t; i < num_tokens; i += (int)blockDim.x) host_tokens[i] = tokens[i];
+  if (t < MK_MAX_XCD) out->xcd_count[t] = sync->xcd_count[t][0];
   if (t == 32) out->abort_flag = sync->abort_flag;
   if (t == 33) out->abort_where = sync->abort_where;
+  if (t == 34) out->t_begin = sync->t_begin;
+  if (t == 35) out->t_end = sync->t_end;
   if (t >= 64 && t < 64 + sizeof(MkSched) / 4) ((unsigned *)&out->sched)[t - 64] = ((const unsigned *)sched)[t - 64];
   __syncthreads();
   for (unsigned i = t; i < sizeof(MkSync) / 4; i += blockDim.x) ((unsigned *)sync)[i] = 0u;
@@ -181,11 +186,14 @@ struct mk_graph {
   long long *d_timing = nullptr;
   int timing_cap = 0;
   std::string json, program_text;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // batches in host memory (mk_set_host_batch): as the device sees them, and how many words fit
+  const int *batch_src = nullptr;
+  int *batch_dst = nullptr;
+  long long *batch_tokens = nullptr;
+  int64_t batch_cap = 0;
   bool launch_pending = false;
   LaunchStatus *h_status = nullptr;  // pinned host memory: what the last launch left (mk_launch_done_kernel)
   hipStream_t launch_stream = nullptr;
-  bool ms_due = false;               // last_ms has not been read from the events yet
   int max_kv_heads = 1, max_qpk = 1;  // over the attention stages
   double last_ms = 0.0;
   int last_nxcd = 0, last_aborted = 0;
@@ -3049,21 +3057,19 @@ static const void *kernel_of(const mk_graph *g) {
   return k;
 }
 
-int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler, const MkRuntime *rt = nullptr) {
+int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler, const MkRuntime *rt = nullptr, long long *host_tokens = nullptr) {
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending: call mk_wait first");
   HIP_TRY(hipSetDevice(g->cfg.device));
   if (!rt) rt = &g->h_rt;
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
-  HIP_TRY(hipEventRecord(g->ev0, stream));
   HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
-  HIP_TRY(hipEventRecord(g->ev1, stream));
   g->launch_pending = true;
   g->last_stages = run_scheduler == MK_SCHED_INGEST && !rt->profiler && rt->max_tokens > 1 ? rt->tail : rt->num_stages;
   g->launch_stream = stream;
-  g->ms_due = true;
-  HIP_TRY(launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status));
+  HIP_TRY(launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status, (const long long *)rt->output_tokens,
+                        host_tokens ? rt->max_tokens : 0, host_tokens));
   return MK_OK;
 }
 
@@ -3080,6 +3086,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   for (int i = 0; i < MK_MAX_XCD; i++) nx += hs.xcd_count[i] > 0;
   g->last_nxcd = nx;
   g->last_aborted = hs.abort_flag != 0;
+  if (!hs.abort_flag) g->last_ms = (hs.t_end - hs.t_begin) * 1e-5;
   const MkSched &sc = hs.sched;
   if (finished_out) *finished_out = sc.finished;
   if (hs.abort_flag) {
@@ -3220,8 +3227,6 @@ int mk_graph_destroy(mk_graph *g) {
   for (void *p : g->allocs) (void)hipFree(p);
   for (void *p : g->host_allocs) free(p);
   if (g->h_status) (void)hipHostFree(g->h_status);
-  if (g->ev0) (void)hipEventDestroy(g->ev0);
-  if (g->ev1) (void)hipEventDestroy(g->ev1);
   delete g;
   return MK_OK;
 }
@@ -3581,8 +3586,6 @@ int mk_compile(mk_graph *g) {
   if ((rc = dev_alloc(g, &p, sizeof(MkRuntime)))) return rc;
   g->d_rt = (MkRuntime *)p;
   if ((rc = upload_runtime(g))) return rc;
-  HIP_TRY(hipEventCreate(&g->ev0));
-  HIP_TRY(hipEventCreate(&g->ev1));
   HIP_TRY(hipHostMalloc((void **)&g->h_status, sizeof(LaunchStatus)));
   memset(g->h_status, 0, sizeof(LaunchStatus));
   if ((rc = resolve_scratch(g->cfg.device))) return rc;  // set-up is where the static launch scratch's address is looked up
@@ -3651,6 +3654,46 @@ int mk_enqueue_ingest(mk_graph *g, void *stream) {
   if (!g) return fail(MK_EINVAL, "null argument");
   if (g->cfg.mode == MK_MODE_OFFLINE || g->cfg.mode == MK_MODE_ONLINE) return fail(MK_EINVAL, "mk_enqueue_ingest runs a batch that the host describes (online_notoken / onepass)");
   return do_launch(g, (hipStream_t)stream, 1, MK_SCHED_INGEST);
+}
+
+// Address of [p, p + bytes) as the graph's device sees it: pinned host memory, or device memory.  Null: it is neither from end to end.
+static void *device_view(const void *p, size_t bytes, hipMemoryType type) {
+  hipPointerAttribute_t a, b;
+  const bool ok = hipPointerGetAttributes(&a, p) == hipSuccess && hipPointerGetAttributes(&b, (const char *)p + bytes - 1) == hipSuccess;
+  if (!ok) (void)hipGetLastError();
+  if (!ok || a.type != type || b.type != type || !a.devicePointer || (char *)b.devicePointer - (char *)a.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
+  return a.devicePointer;
+}
+
+int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens) {
+  if (!g) return fail(MK_EINVAL, "null argument");
+  if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
+  if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending");
+  if (g->cfg.mode == MK_MODE_OFFLINE || g->cfg.mode == MK_MODE_ONLINE) return fail(MK_EINVAL, "the host describes batches in the modes online_notoken and onepass");
+  g->batch_cap = 0;
+  if (!host_words) return MK_OK;
+  if (!device_words || words < 1 || words > (1ll << 28)) return fail(MK_EINVAL, "a batch in host memory needs device memory of as many words");
+  if (((uintptr_t)host_words | (uintptr_t)device_words) & 3) return fail(MK_EINVAL, "words of a batch lie on four bytes");
+  HIP_TRY(hipSetDevice(g->cfg.device));
+  const size_t token_bytes = sizeof(int64_t) * (size_t)g->h_rt.max_tokens;
+  g->batch_src = (const int *)device_view(host_words, 4 * (size_t)words, hipMemoryTypeHost);
+  g->batch_dst = (int *)device_view(device_words, 4 * (size_t)words, hipMemoryTypeDevice);
+  g->batch_tokens = host_tokens ? (long long *)device_view(host_tokens, token_bytes, hipMemoryTypeHost) : nullptr;
+  if (!g->batch_src || !g->batch_dst || (host_tokens && (!g->batch_tokens || (uintptr_t)host_tokens & 7)))
+    return fail(MK_EINVAL, "batch words and sampled tokens are in pinned host memory, the words' place in device memory");
+  g->batch_cap = words;
+  return MK_OK;
+}
+
+int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest) {
+  if (!g) return fail(MK_EINVAL, "null argument");
+  if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
+  if (words < 1 || words > g->batch_cap) return fail(MK_EINVAL, "batch of %lld words, mk_set_host_batch named %lld", (long long)words, (long long)g->batch_cap);
+  MkRuntime rt = g->h_rt;
+  rt.batch_src = g->batch_src;
+  rt.batch_dst = g->batch_dst;
+  rt.batch_words = words;
+  return do_launch(g, (hipStream_t)stream, 1, ingest ? MK_SCHED_INGEST : MK_SCHED_FROM_META, &rt, ingest ? nullptr : g->batch_tokens);
 }
 
 int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations) {
@@ -3744,13 +3787,6 @@ int mk_get_stats(mk_graph *g, mk_stats *out) {
   out->weight_bytes = g->weight_bytes;
   out->packed_weight_bytes = g->packed_bytes;
   out->row_major_weight_bytes = g->row_major_bytes;
-  if (g->ms_due && !g->launch_pending) {
-    // (a launch that went into a caller's graph has no time of its own)
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, g->ev0, g->ev1) == hipSuccess) g->last_ms = ms;
-    else (void)hipGetLastError();
-    g->ms_due = false;
-  }
   out->last_launch_ms = g->last_ms;
   if (g->compiled && !g->launch_pending) {
     MkSched sc;

@@ -721,7 +721,8 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // rows [qo_indptr[i], qo_indptr[i+1]) and its sequence, new tokens included, is (pages - 1) * page_size + last_page_len
 // long, so its rows sit at the last positions of that sequence.  Derives the per-row slot / position / first-row arrays
 // on the device (no host round trip, so a serving loop can enqueue launches back to back).  Runs on one thread.
-// Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).
+// Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).  Reads and
+// writes at device scope: mk_fetch_batch may have written the tensors a moment ago, and nobody releases behind the step.
 __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt, int lane) {
   const int R = rt.max_requests, B = rt.max_tokens;
   // A batch the stages cannot run as described is not run at all: truncating a request's rows would leave the rest with
@@ -729,7 +730,8 @@ __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt,
   // bad, of the first slot that cannot run: 1 = rows outside [0, max tokens), overlapping, or with gaps; 2 = more rows for one
   // request than max_tokens_per_request; 3 = a sequence shorter than its new rows, longer than max_seq_length, or without pages.
   const int i = min(lane, R - 1);  // (at most 64 slots)
-  const int q0 = rt.qo_indptr[i], q1 = rt.qo_indptr[i + 1], pages = rt.kv_indptr[i + 1] - rt.kv_indptr[i], last = rt.kv_last_page_len[i];
+  const int q0 = ldc_i32(rt.qo_indptr + i), q1 = ldc_i32(rt.qo_indptr + i + 1), pages = ldc_i32(rt.kv_indptr + i + 1) - ldc_i32(rt.kv_indptr + i),
+            last = ldc_i32(rt.kv_last_page_len + i);
   const int n = lane < R ? q1 - q0 : 0;  // (<= 0: an unused slot; hosts that fill only the first entries leave zeros behind them)
   const int len = (int)((long long)(pages - 1) * rt.page_size) + last;
   const bool inside = n > 0 && q0 >= 0 && n <= B && q0 <= B - n;
@@ -751,19 +753,44 @@ __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt,
   const unsigned long long covered = (unsigned long long)(unsigned)wave_bcast((int)lo, 63) | ((unsigned long long)(unsigned)wave_bcast((int)hi, 63) << 32);
   int ntok = covered ? 64 - __clzll((long long)covered) : 0;
   if (covered != (ntok >= 64 ? ~0ull : ((1ull << ntok) - 1ull)) && !bad) bad = 1;
-  if (!bad) {
-    for (int j = 0; j < n; j++) {
-      rt.tok_slot[q0 + j] = i;
-      rt.tok_pos[q0 + j] = len - n + j;
-      rt.tok_first[q0 + j] = q0;
+  if (bad) ntok = 0;
+  // a lane per row (by the lanes of the slots, row after row, 64 rows of one request took 16 us)
+  int slot = 0, first = 0, pos = 0;
+  for (unsigned long long live = ntok ? __ballot(n > 0) : 0ull; live; live &= live - 1) {
+    const int s = (int)__ffsll(live) - 1, f = wave_bcast(q0, s);
+    if (lane >= f && lane < wave_bcast(q1, s)) {
+      slot = s;
+      first = f;
+      pos = wave_bcast(len, s) - wave_bcast(q1, s) + lane;
     }
   }
-  if (bad) ntok = 0;
+  if (lane < ntok) {
+    stc_i32(rt.tok_slot + lane, slot);
+    stc_i32(rt.tok_pos + lane, pos);
+    stc_i32(rt.tok_first + lane, first);
+  }
   if (lane == 0) {
-    rt.sched->bad_batch = bad;
-    rt.sched->num_tokens = ntok;
+    stc_i32(&rt.sched->bad_batch, bad);
+    stc_i32(&rt.sched->num_tokens, ntok);
   }
   return ntok;
+}
+
+// The words of a batch in pinned host memory go where the stages read them, by one workgroup, each word read once.  Bound by one round trip
+// over the bus, which overlaps nothing: 2 us for up to 2048 words.  (As a copy on the stream in front of the launch it cost 12: a cooperative
+// launch sits on a queue of its own and waits for the copy's signal.  Words behind the end read again as the first ones, as elsewhere here, made it
+// 18 to 40: lines that the host has just written are slow to fetch, every time.)
+__device__ __attribute__((noinline)) void mk_fetch_batch(const int *src, int *dst, long long words) {
+  for (long long i = threadIdx.x; i < words; i += 8 * MK_THREADS) {
+    int v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (i + k * MK_THREADS < words) v[k] = __hip_atomic_load(src + i + k * MK_THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (i + k * MK_THREADS < words) stc_i32(dst + i + k * MK_THREADS, v[k]);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // The reference's MODE_ONLINE step (persistent_kernel.cuh:538-568): one request (slot 0, request 0) whose tokens the
@@ -4927,29 +4954,35 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
     sh_ticket[0] = sh_ticket[1] = 0;
     sh_ticket[2] = MK_NO_LISTS;
   }
-  // ---- XCD discovery: rank of this workgroup inside its die, dies in use, workgroups per die
+  // ---- XCD discovery: rank of this workgroup inside its die, dies in use, workgroups per die.  The dies' counters are all there is: they are
+  // final once they add up to the grid.  (One counter for the whole grid beside them, awaited with acquiring loads: 8.0 us instead of 4.6 in a launch of
+  // nothing else.)
   if (threadIdx.x == 0) {
     MkSync *s = rt.sync;
-    const unsigned rank = __hip_atomic_fetch_add(&s->xcd_count[c.xcd], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_fetch_add(&s->init_ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned spins = 0;
-    while (__hip_atomic_load(&s->init_ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < (unsigned)c.G && spin_ok(s, spins, 0xFFFF0000u))
+    if (blockIdx.x == 0) s->t_begin = (long long)wall_clock64();
+    const unsigned rank = __hip_atomic_fetch_add(&s->xcd_count[c.xcd][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned n[MK_MAX_XCD], spins = 0;
+    while (true) {
+      unsigned sum = 0;
+      for (int i = 0; i < MK_MAX_XCD; i++) sum += n[i] = __hip_atomic_load(&s->xcd_count[i][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (sum >= (unsigned)c.G || !spin_ok(s, spins, 0xFFFF0000u)) break;
       __builtin_amdgcn_s_sleep(1);
-    int nx = 0, before = 0, xi = 0;
+    }
+    int nx = 0, before = 0, xi = 0, mine = 0;
     for (int i = 0; i < MK_MAX_XCD; i++) {
-      const unsigned n = __hip_atomic_load(&s->xcd_count[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      nx += n > 0;
+      nx += n[i] > 0;
       if (i < c.xcd) {
-        before += (int)n;
-        xi += n > 0;
+        before += (int)n[i];
+        xi += n[i] > 0;
       }
+      if (i == c.xcd) mine = (int)n[i];
+      sh_quota[i] = (int)n[i];
     }
     sh_quota[8] = xi;
     sh_quota[9] = (int)rank;
-    for (int i = 0; i < 8; i++) sh_quota[i] = (int)__hip_atomic_load(&s->xcd_count[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     sh_bcast[0] = before + (int)rank;
     sh_bcast[1] = nx;
-    sh_bcast[2] = (int)__hip_atomic_load(&s->xcd_count[c.xcd], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sh_bcast[2] = mine;
     sh_bcast[3] = (int)__hip_atomic_load(&s->abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
@@ -4981,6 +5014,13 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       int ntok_w = 0;
       const bool from_meta = run_scheduler == MK_SCHED_FROM_META || run_scheduler == MK_SCHED_INGEST;
       if (c.vid == 0 && threadIdx.x < 64 && wave_sched) ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x);
+      if (from_meta) {
+        if (c.vid == 0 && rt.batch_words) {
+          mk_fetch_batch(rt.batch_src, rt.batch_dst, rt.batch_words);
+          __syncthreads();
+        }
+        c.wrote_through = true;  // (nothing else was written in this launch)
+      }
       if (c.vid == 0 && threadIdx.x < 64 && from_meta) ntok_w = mk_batch_from_meta(*rtp, threadIdx.x);
       if (c.vid == 0 && threadIdx.x == 0) {
         int ntok;
@@ -5037,7 +5077,10 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   }
   barrier_wait(c);  // drain: nobody leaves while another workgroup may still poll
   if (rt.profiler && threadIdx.x == 0) rt.profiler_count[c.vid] = c.prof_n;
-  if (c.vid == 0 && threadIdx.x == 0 && rt.timing) rt.timing[0] = (long long)wall_clock64();
+  if (c.vid == 0 && threadIdx.x == 0) {
+    rt.sync->t_end = (long long)wall_clock64();
+    if (rt.timing) rt.timing[0] = rt.sync->t_end;
+  }
 }
 
 // build.py compiles this file once per -DMK_KERNEL_*, so that the kernels compile side by side and a build may leave out

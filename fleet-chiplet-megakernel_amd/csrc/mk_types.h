@@ -254,17 +254,12 @@ MK_HOST_DEVICE inline MkLatentLds mk_latent_lds(int es, int rt, int nkc, int sub
 // Hierarchical barrier state.  One 128-byte line per counter so that XCD-local
 // counters stay in that XCD's L2.
 struct MkSync {
-  unsigned global_ctr;
-  unsigned pad0[31];
   unsigned local_ctr[MK_MAX_XCD][32];
-  unsigned local_flag[MK_MAX_XCD][32];
-  unsigned xcd_count[MK_MAX_XCD];
-  unsigned pad1[32 - MK_MAX_XCD];
-  unsigned init_ctr;
-  unsigned pad2[31];
+  unsigned xcd_count[MK_MAX_XCD][32];  // workgroups of this launch on each die
   unsigned abort_flag;
   unsigned abort_where;
-  unsigned pad3[30];
+  unsigned pad[30];
+  long long t_begin, t_end;  // 100 MHz ticks: the first workgroup's entry, everybody through
 };
 
 // Barrier completion test.  Arrival counters and their targets (quota x epoch) are 32-bit and only ever grow during a
@@ -309,6 +304,10 @@ struct MkRuntime {
   int *kv_indptr;
   int *kv_indices;
   int *kv_last_page_len;
+  // a batch that the launch fetches itself (mk_enqueue_batch): pinned host memory, where it goes, 32-bit words of it (0: the tensors hold it already)
+  const int *batch_src;
+  int *batch_dst;
+  long long batch_words;
   // library-owned scheduler memory
   int *request_ids;   // [max_requests] request id per batch slot, -1 = free
   int *state_ids;     // [max_requests] recurrent-state slot per batch slot, a permutation (null: the graph has no recurrence)

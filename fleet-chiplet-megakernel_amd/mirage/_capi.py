@@ -25,7 +25,7 @@ MK_MODES = {"offline": 0, "online": 1, "online_notoken": 2, "onepass": 3}
 EXPORTED_SYMBOLS = [
     "mk_graph_create", "mk_graph_destroy", "mk_tensor_attach", "mk_tensor_new", "mk_tensor_shuffle",
     "mk_tensor_num_dims", "mk_tensor_dim", "mk_tensor_ptr", "mk_add_task", "mk_generate_task_graph",
-    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_wait",
+    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_set_host_batch", "mk_enqueue_batch", "mk_wait",
     "mk_run_once", "mk_repack_weights", "mk_tensor_releasable", "mk_set_profiler", "mk_get_stats", "mk_get_stage_profile", "mk_get_stage_marks", "mk_describe_program", "mk_last_error", "mk_version",
 ]
 
@@ -115,6 +115,8 @@ def load():
     lib.mk_enqueue_steps.argtypes = [vp, vp, ci]
     lib.mk_enqueue_steps_static.argtypes = [vp, vp, ci]
     lib.mk_enqueue_ingest.argtypes = [vp, vp]
+    lib.mk_set_host_batch.argtypes = [vp, vp, vp, ctypes.c_int64, vp]
+    lib.mk_enqueue_batch.argtypes = [vp, vp, ctypes.c_int64, ci]
     lib.mk_wait.argtypes = [vp, vp, cip]
     i32p = ctypes.POINTER(ctypes.c_int32)
     lib.mk_run_once.argtypes = [vp, vp, ci, i32p, i32p, i32p]
@@ -224,6 +226,12 @@ class Graph:
 
     def enqueue_ingest(self, stream):
         check(self._lib.mk_enqueue_ingest(self._h, ctypes.c_void_p(stream)))
+
+    def set_host_batch(self, host_words, device_words, words, host_tokens):
+        check(self._lib.mk_set_host_batch(self._h, host_words, device_words, int(words), host_tokens))
+
+    def enqueue_batch(self, stream, words, ingest):
+        check(self._lib.mk_enqueue_batch(self._h, ctypes.c_void_p(stream), int(words), int(ingest)))
 
     def wait(self, stream) -> bool:
         fin = ctypes.c_int(0)

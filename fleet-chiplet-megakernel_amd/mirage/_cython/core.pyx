@@ -206,6 +206,13 @@ cdef class CyGraph:
     def enqueue_ingest(self, stream):
         _check(mk.mk_enqueue_ingest(self.g, <void *><uintptr_t>(stream or 0)))
 
+    def set_host_batch(self, host_words, device_words, words, host_tokens):
+        _check(mk.mk_set_host_batch(self.g, <const int32_t *><uintptr_t>(host_words or 0), <int32_t *><uintptr_t>(device_words or 0), <int64_t>words,
+                                    <int64_t *><uintptr_t>(host_tokens or 0)))
+
+    def enqueue_batch(self, stream, words, ingest):
+        _check(mk.mk_enqueue_batch(self.g, <void *><uintptr_t>(stream or 0), <int64_t>words, 1 if ingest else 0))
+
     def wait(self, stream) -> bool:
         cdef int rc, fin = 0
         cdef void *s = <void *><uintptr_t>(stream or 0)

@@ -61,6 +61,8 @@ cdef extern from "fleet_mk.h" nogil:
     int mk_enqueue_steps(mk_graph *g, void *stream, int max_iterations)
     int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations)
     int mk_enqueue_ingest(mk_graph *g, void *stream)
+    int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens)
+    int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest)
     int mk_wait(mk_graph *g, void *stream, int *finished_out)
     int mk_run_once(mk_graph *g, void *stream, int num_tokens, const int32_t *tok_slot, const int32_t *tok_pos, const int32_t *tok_first)
     int mk_repack_weights(mk_graph *g)

@@ -1077,9 +1077,25 @@ class PersistentKernel:
     def enqueue_steps(self, max_iterations: int, default_stream=None):
         self._g.enqueue_steps(self._stream_ptr(default_stream), int(max_iterations))
 
-    def enqueue_ingest(self, default_stream=None):
-        """enqueue_steps(1) over a batch that the host describes and whose logits and sampled tokens nobody reads."""
-        self._g.enqueue_ingest(self._stream_ptr(default_stream))
+    def enqueue_ingest(self, default_stream=None, host_words: int = 0):
+        """enqueue_steps(1) over a batch that the host describes and whose logits and sampled tokens nobody reads; with `host_words`
+        over the batch in that many words of what attach_host_batch named."""
+        if host_words:
+            self._g.enqueue_batch(self._stream_ptr(default_stream), host_words, True)
+        else:
+            self._g.enqueue_ingest(self._stream_ptr(default_stream))
+
+    def attach_host_batch(self, host_words, device_words, host_tokens=None):
+        """Batches that a launch fetches from pinned memory by itself: `host_words` (int32, pinned) is laid out as `device_words`, of which the
+        meta tensors are slices.  enqueue_batch(n) runs the batch in the first n words and leaves the sampled tokens in `host_tokens` (int64,
+        pinned).  The tensors are kept as long as this object."""
+        assert host_words.is_pinned() and host_words.dtype == device_words.dtype == torch.int32 and host_words.is_contiguous() and device_words.is_contiguous()
+        assert host_tokens is None or (host_tokens.is_pinned() and host_tokens.dtype == torch.int64 and host_tokens.is_contiguous() and len(host_tokens) >= self.max_num_batched_tokens)
+        self._g.set_host_batch(host_words.data_ptr(), device_words.data_ptr(), min(len(host_words), len(device_words)), host_tokens.data_ptr() if host_tokens is not None else None)
+        self._host_batch = host_words, device_words, host_tokens
+
+    def enqueue_batch(self, host_words: int, default_stream=None):
+        self._g.enqueue_batch(self._stream_ptr(default_stream), host_words, False)
 
     def wait(self, default_stream=None) -> bool:
         return self._g.wait(self._stream_ptr(default_stream))

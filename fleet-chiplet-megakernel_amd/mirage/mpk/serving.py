@@ -46,10 +46,12 @@ class _Request:
 class ServingSession:
     # models with recurrent layers: the tensor that names every batch slot's state slot, and the pool of state slots
     state_slots = slots = None
-    # sessions opened here: a pass's ids and description in pinned memory, the device tensor they are copied to, and a pinned place for the
-    # sampled tokens, so that a pass waits for the device once (a pageable copy in either direction costs 12 to 16 us, of which a pass had
-    # three; one copy per wanted row of logits another 8 each: a decode step of 16 requests spent 280 us outside the launch, now 85)
+    # sessions opened here: a pass's ids and description in pinned memory, the device tensor they go to, and a pinned place for the sampled
+    # tokens.  The launch fetches and leaves them itself (_fetched), so that nothing but the launch is on the stream and a pass waits for the
+    # device once
     _host = _dev = _sampled = None
+    _fetched = False
+    _view = None  # of the logits
     _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
     def __init__(self, mpk: MPK):
@@ -88,12 +90,16 @@ class ServingSession:
         session = ServingSession(mpk)
         host = torch.empty(2 * max_rows + len(dev), dtype=torch.int32, pin_memory=True)
         session._sampled, session._host, session._dev = host[:2 * max_rows].view(torch.int64), host[2 * max_rows:], dev
+        mpk.persistent_kernel.attach_host_batch(session._host, dev, session._sampled)
+        session._fetched = True
         return session
 
     # ------------------------------------------------------------------ steps
     def logits(self) -> torch.Tensor:
         """Logits of the rows of the last pass (a view of the library's tensor)."""
-        return self.mpk.model_builder.logits.to_torch()
+        if self._view is None:  # (making one takes 5 us)
+            self._view = self.mpk.model_builder.logits.to_torch()
+        return self._view
 
     def step(self, entries: Sequence[Tuple[object, Sequence[int]]], want: Sequence[Sequence[int]] = None):
         """Run `entries` = (request, its next tokens) as one batch.  Returns (logits, next tokens): float32 rows for the
@@ -178,12 +184,20 @@ class ServingSession:
             # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
             host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
             host[n:n + len(desc)] = desc
-            self._dev[:n + len(desc)].copy_(self._host[:n + len(desc)], non_blocking=True)
             pk = m.persistent_kernel
+            if self._fetched and pk.profiler_tensor is None:
+                stream = torch.cuda.current_stream(self._dev.device)  # (the logits' copies', whichever device is current)
+                if unread:
+                    pk.enqueue_ingest(default_stream=stream, host_words=n + len(desc))
+                else:
+                    pk.enqueue_batch(n + len(desc), default_stream=stream)
+                pk.wait(default_stream=stream)
+                return None if unread else self._sampled.tolist()
+            self._dev[:n + len(desc)].copy_(self._host[:n + len(desc)], non_blocking=True)
             if pk.profiler_tensor is not None:  # (the whole call also writes the trace)
                 m()
                 return None
-            stream = torch.cuda.current_stream(self._dev.device) if self._dev.is_cuda else None  # (the copies', whichever device is current)
+            stream = torch.cuda.current_stream(self._dev.device) if self._dev.is_cuda else None
             if unread:
                 pk.enqueue_ingest(default_stream=stream)
                 pk.wait(default_stream=stream)

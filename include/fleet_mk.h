@@ -166,6 +166,14 @@ int mk_wait(mk_graph *g, void *stream, int *finished_out);
  * values.  (With a profiler tensor attached, and in graphs of one token per
  * iteration, everything runs.)  Pair with mk_wait. */
 int mk_enqueue_ingest(mk_graph *g, void *stream);
+/* Batches that a launch fetches by itself, in the same modes: `host_words` (pinned host memory) has the ids and the index tensors of a
+ * batch laid out as `device_words` has them, where the graph's tensors point; both hold `words` 32-bit words.  mk_enqueue_batch is
+ * mk_enqueue_steps (or, with `ingest`, mk_enqueue_ingest) over the batch in the first `words` of them, and, without `ingest`, leaves the
+ * sampled tokens in `host_tokens` (pinned, max_num_batched_tokens values; may be NULL).  The launch reads the words and writes the
+ * tokens until mk_wait has returned; the memory belongs to the caller and must live until the handle is destroyed or another place is named.
+ * host_words == NULL forgets it.  MK_EINVAL for memory of another kind. */
+int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens);
+int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
 /* mk_enqueue_steps for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc); it has no counterpart in the reference.  The call allocates and frees nothing, and every piece
  * of scratch its launch uses -- barrier counters, K-split partial tiles and counters, attention split-KV partials and
@@ -203,7 +211,7 @@ typedef struct mk_stats {
   int aborted;             /* watchdog fired in the last launch */
   int64_t iterations;      /* decode iterations executed since mk_init_requests */
   int64_t weight_bytes;    /* bytes of weight matrices streamed by one iteration */
-  double last_launch_ms;   /* HIP-event time of the last launch's kernel, on the stream it ran on */
+  double last_launch_ms;   /* device time of the last launch that mk_wait has seen, from its first workgroup's entry to its last stage's end */
   int64_t packed_weight_bytes; /* device memory the handle holds for matrix-core copies of the weights (0: none) */
   int64_t row_major_weight_bytes; /* bytes of attached linear weights the handle still reads in place (0 with
                                      MK_CFG_SINGLE_WEIGHT_COPY: every linear weight lives in its tile copy only) */
