@@ -81,11 +81,11 @@ template <typename E>
 __device__ __forceinline__ void stage_fx_embed(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
   barrier_wait(c);
   const int k = st.k;
-  for (int t = c.vid; t < M; t += c.G) {
+  for (int t = row_item(c, c.vid); t < M; t += c.G) {
     long long id;
     if (st.flags & MK_F_EMBED_FROM_TOKENS) {
-      const int req = ldc_i32(&rt.request_ids[ldc_i32(&rt.tok_slot[t])]);
-      id = (long long)ldc_u64(&rt.tokens[(long long)req * rt.max_seq + ldc_i32(&rt.tok_pos[t])]);
+      const int req = ldc_i32(&rt.request_ids[c.sh_tok[MK_MAX_TOKENS + t]]);
+      id = (long long)ldc_u64(&rt.tokens[(long long)req * rt.max_seq + c.sh_tok[t]]);
     } else {
       id = (long long)ldc_u64((const long long *)st.in + t);
     }
@@ -172,7 +172,7 @@ __device__ __forceinline__ void stage_fx_addnorm_t(CStage &st, Ctx &c, int M, ch
   float *red = (float *)smem;
   const f32x4 *w4 = (const f32x4 *)st.norm_w;
   const float *xr = (const float *)st.res;
-  const int t0 = c.even_xcds ? c.rank * c.nxcd + c.xi : c.vid;  // rows are dealt round-robin over the dies
+  const int t0 = row_item(c);
   f32x4 g[NS], x[NS], v[NS];
   auto load_x = [&](int t) {
     const auto row = dev_rows(xr + (size_t)t * st.ld_res);

@@ -31,6 +31,21 @@ extern "C" __global__ void mk_pack_weights_kernel(const MkWeight w, int n, int k
 MK_DECLARE_KERNEL(mk_persistent_kernel);
 MK_DECLARE_KERNEL(mk_persistent_kernel_m1);
 #endif
+#ifdef MK_HAVE_KERNEL_DENSE_PAIR
+MK_DECLARE_KERNEL(mk_persistent_kernel_pair);
+#endif
+#ifdef MK_HAVE_KERNEL_FLEX_PAIR
+MK_DECLARE_KERNEL(mk_persistent_kernel_flex_pair);
+#endif
+#ifdef MK_HAVE_KERNEL_MIX_PAIR
+MK_DECLARE_KERNEL(mk_persistent_kernel_mix_pair);
+#endif
+#ifdef MK_HAVE_KERNEL_HYB_PAIR
+MK_DECLARE_KERNEL(mk_persistent_kernel_hyb_pair);
+#endif
+#ifdef MK_HAVE_KERNEL_DUAL_PAIR
+MK_DECLARE_KERNEL(mk_persistent_kernel_dual_pair);
+#endif
 #ifdef MK_HAVE_KERNEL_FLEX
 MK_DECLARE_KERNEL(mk_persistent_kernel_flex);
 #endif
@@ -179,6 +194,7 @@ struct mk_graph {
   std::vector<MkStage> stages;
   std::vector<std::string> stage_desc;
   MkRuntime h_rt;
+  std::vector<unsigned> pair_prog;  // MkRuntime::pair_prog
   MkRuntime *d_rt = nullptr;
   MkStage *d_stages = nullptr;
   MkSync *d_sync = nullptr;
@@ -2227,6 +2243,134 @@ int tail_stage(const mk_graph *g) {
   return tail;
 }
 
+// Two portions inside prompts as one iteration (MkPairEntry): linears that run for both portions at once, and between two of them the stages of
+// the first portion, then those of the second, as two iterations would run them.  What a cache or a state gets from the first portion is
+// written back and read anew in between; stages that only take rows to rows follow each other without a barrier where there is one of them.
+// Empty: the graph does not run portions that way.
+std::vector<unsigned> pair_program(const mk_graph *g) {
+  std::vector<unsigned> prog;
+  const mk_config &c = g->cfg;
+  const char *pack = getenv("FLEET_MK_PACK_WEIGHTS");
+  const int n = g->tail;
+  if (!(c.flags & MK_CFG_PAIR_PORTIONS) || n >= (int)g->stages.size() || n > MK_PAIR_STAGE || g->flex == FLEX_F32 || g->spec_len > 0 || c.mode == MK_MODE_ONLINE || (pack && atoi(pack) == 0)) return prog;
+  if (c.max_num_batched_tokens <= 32 || c.max_num_batched_tokens > MK_MAX_TOKENS || c.max_tokens_per_request <= 8) return prog;
+  auto keeps_nothing = [&](const MkStage &s) { return !s.k_cache && !s.v_cache && !s.tail && !s.conv_w; };
+  auto row_wise = [&](const MkStage &s) {
+    return keeps_nothing(s) && (s.op == MK_OP_NORM || s.op == MK_OP_FX_ADDNORM || s.op == MK_OP_MX_PRENORM || s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED);
+  };
+  auto passes = [&](const MkStage &s) {  // (leaves nothing for another iteration)
+    switch (s.op) {
+      case MK_OP_NORM: case MK_OP_FX_ADDNORM: case MK_OP_MX_PRENORM: case MK_OP_EMBED: case MK_OP_FX_EMBED: case MK_OP_LINEAR: case MK_OP_SILU_MUL: case MK_OP_MOE_TOPK: case MK_OP_MOE_LINEAR:
+      case MK_OP_MOE_COMBINE: case MK_OP_MX_HEAD_LINEAR: case MK_OP_HY_ROUTE: case MK_OP_HY_EXPERTS: case MK_OP_COPY: return keeps_nothing(s);
+      default: return false;
+    }
+  };
+  std::vector<char> both(n, 0);
+  for (int i = 0; i < n; i++) {
+    MkStage s = g->stages[i];
+    both[i] = s.op == MK_OP_LINEAR && keeps_nothing(s) && (s.k & 63) == 0 && mk_xres_plan(s, g->G).S >= 1;
+  }
+  // a sum left to the stage behind stays in the buffer that other split linears use, until the second portion has read it too
+  for (int i = n - 1; i >= 0; i--) {
+    if (!both[i] || !(g->stages[i].flags & MK_F_DEFER_SUM)) continue;
+    for (int j = i + 1; j < n && !both[j]; j++)
+      if (g->stages[j].op == MK_OP_LINEAR) both[i] = 0;
+  }
+  if (std::count(both.begin(), both.end(), 1) == 0) return prog;
+  for (int i = 0; i < n;) {
+    if (both[i]) {
+      prog.push_back(i++ | MK_PAIR_BOTH);
+      continue;
+    }
+    int j = i;
+    bool carries = false;
+    for (; j < n && !both[j]; j++) carries = carries || !passes(g->stages[j]);
+    if (j == i + 1 && row_wise(g->stages[i])) {
+      prog.push_back(i | MK_PAIR_ON);
+    } else {
+      for (int q = i; q < j; q++) prog.push_back(q | (carries ? MK_PAIR_RELEASE : 0));
+      if (carries) prog.push_back(MK_PAIR_ACQUIRE);
+    }
+    for (int q = i; q < j; q++) prog.push_back(q | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
+    i = j;
+  }
+  return prog;
+}
+
+// The stages as they run for the second portion: over rows of its own, in copies of the memory that stages write rows to.  False: some stage
+// could not be told apart from the first portion's, and portions run one by one.
+int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
+  const mk_config &c = g->cfg;
+  *ok = false;
+  Extents held, rows;  // tensors and allocations; those among them that stages write rows to
+  for (const Tensor &t : g->tensors) {
+    if (!t.ptr || t.kind == T_SHUFFLED) continue;
+    size_t last = 0;
+    for (int d = 0; d < t.ndims; d++) last += (size_t)(t.dims[d] - 1) * (size_t)t.strides[d];
+    held.add((const char *)t.ptr, (const char *)t.ptr + (last + 1) * dtype_size(t.dtype));
+  }
+  for (const auto &a : g->alloc_sizes) held.add((const char *)a.first, (const char *)a.first + a.second);
+  auto find = [](const Extents &e, const void *p) {
+    auto it = e.at.upper_bound((const char *)p);
+    return it != e.at.begin() && std::prev(it)->second > (const char *)p ? std::prev(it) : e.at.end();
+  };
+  out.assign(g->stages.begin(), g->stages.end());
+  for (int i = 0; i < g->tail; i++) {
+    const MkStage &s = g->stages[i];
+    const bool routed = s.op == MK_OP_HY_ROUTE || s.op == MK_OP_HY_EXPERTS;
+    for (const void *p : {(const void *)s.out, (const void *)s.out2, (const void *)s.out3, (const void *)s.norm_out, (const void *)s.q_ws, (const void *)s.glu_out, (const void *)s.moe_topk_w,
+                          (const void *)s.moe_routing, (const void *)s.moe_mask, (const void *)(routed ? s.ids : nullptr), (const void *)(routed ? s.slot_w : nullptr)}) {
+      if (!p) continue;
+      const auto it = find(held, p);
+      if (it == held.at.end()) return MK_OK;
+      rows.add(it->first, it->second);
+    }
+  }
+  auto own = [&](const void *p) { return p && find(rows, p) != rows.at.end(); };
+  for (const void *p : {(const void *)c.step, (const void *)c.tokens, (const void *)c.input_tokens, (const void *)c.num_new_tokens, (const void *)c.prompt_lengths, (const void *)c.qo_indptr,
+                        (const void *)c.paged_kv_indptr, (const void *)c.paged_kv_indices, (const void *)c.paged_kv_last_page_len, (const void *)g->state_ids})
+    if (own(p)) return MK_OK;
+  for (int i = 0; i < g->tail; i++) {
+    const MkStage &s = g->stages[i];
+    for (const void *p : {(const void *)s.k_cache, (const void *)s.v_cache, (const void *)s.tail, s.w.seg[0], s.w.seg[1], s.w.seg[2], s.norm_w, s.y_norm_w, s.q_norm_w, s.k_norm_w, s.cos_tab, s.sin_tab, s.sink,
+                          (const void *)s.in_bias, (const void *)s.a_tab, (const void *)s.d_tab, (const void *)s.temp, (const void *)s.y_scale, (const void *)s.y2_scale, s.conv_w, s.pos_tab,
+                          (const void *)s.choice_bias, (const void *)s.step_bias, s.op == MK_OP_HY_ROUTE ? nullptr : s.w_shared /* (there only its presence counts) */, (const void *)s.aux0,
+                          (const void *)s.aux1, s.wpack})
+      if (own(p)) return MK_OK;
+    // (ids that are not the iteration's tokens would be the first portion's)
+    if ((s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) && !(s.flags & MK_F_EMBED_FROM_TOKENS) && s.in != (const void *)c.input_tokens) return MK_OK;
+    if ((s.flags & MK_F_GELU_TABLE) && s.aux0 != (const void *)c.input_tokens) return MK_OK;
+  }
+  size_t total = sizeof(int64_t) * MK_MAX_TOKENS;  // (the ids in front)
+  for (const auto &e : rows.at) total += (e.second - e.first + 255) / 256 * 256;
+  void *block;
+  const int rc = dev_alloc(g, &block, total, false);
+  if (rc) return rc;
+  void *ids = block;
+  g->h_rt.ids2 = (long long *)ids;
+  std::map<const char *, char *> copy;
+  char *to = (char *)block + sizeof(int64_t) * MK_MAX_TOKENS;
+  for (const auto &e : rows.at) {
+    HIP_TRY(hipMemcpyAsync(to, e.first, e.second - e.first, hipMemcpyDeviceToDevice, nullptr));  // (padding that stages leave as it is)
+    copy[e.first] = to;
+    to += (e.second - e.first + 255) / 256 * 256;
+  }
+  HIP_TRY(hipStreamSynchronize(nullptr));
+  auto moved = [&](auto &p) {
+    const auto it = p ? find(rows, p) : rows.at.end();
+    if (it != rows.at.end()) p = (std::remove_reference_t<decltype(p)>)(void *)(copy[it->first] + ((const char *)p - it->first));
+  };
+  for (int i = 0; i < g->tail; i++) {
+    MkStage &s = out[i];
+    moved(s.in); moved(s.out); moved(s.res); moved(s.norm_out); moved(s.q_ws); moved(s.moe_logits); moved(s.moe_topk_w); moved(s.moe_routing); moved(s.moe_mask);
+    moved(s.out2); moved(s.y_in); moved(s.in2); moved(s.glu_out); moved(s.slot_w); moved(s.ids); moved(s.in3); moved(s.y2); moved(s.out3);
+    if (s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) s.in = ids;
+    if (s.flags & MK_F_GELU_TABLE) s.aux0 = ids;
+  }
+  *ok = true;
+  return MK_OK;
+}
+
 int lower(mk_graph *g) {
   g->stages.clear();
   g->stage_desc.clear();
@@ -2659,6 +2803,7 @@ int lower(mk_graph *g) {
     }
   }
   g->tail = tail_stage(g);
+  g->pair_prog = pair_program(g);
   g->program_text.clear();
   for (size_t s = 0; s < g->stage_desc.size(); s++) g->program_text += fmt("%3zu ", s) + g->stage_desc[s] + ((int)s < g->tail ? "\n" : " unread=skip\n");
   return MK_OK;
@@ -3004,6 +3149,26 @@ int upload_runtime(mk_graph *g) {
 // `rt` is the runtime block the kernel receives by value; its barrier state is zero (from its allocation, or the launch before)
 // graphs with flex stages (mk_flex.hip) have kernels of their own; graphs that never run more than one token per iteration
 // use the instantiation for exactly that.  Null: not in this build of the library.
+static const void *pair_kernel_of(const mk_graph *g) {
+  const void *k = nullptr;
+  if (g->flex == FLEX_F32) return k;
+#ifdef MK_HAVE_KERNEL_DENSE_PAIR
+  if (g->flex == FLEX_NONE) k = (const void *)mk_persistent_kernel_pair;
+#endif
+#ifdef MK_HAVE_KERNEL_DUAL_PAIR
+  if (g->flex != FLEX_NONE && g->dual) k = (const void *)mk_persistent_kernel_dual_pair;
+#endif
+#ifdef MK_HAVE_KERNEL_HYB_PAIR
+  if (g->flex != FLEX_NONE && !g->dual && g->hyb) k = (const void *)mk_persistent_kernel_hyb_pair;
+#endif
+#ifdef MK_HAVE_KERNEL_MIX_PAIR
+  if (g->flex != FLEX_NONE && !g->dual && !g->hyb && g->mix) k = (const void *)mk_persistent_kernel_mix_pair;
+#endif
+#ifdef MK_HAVE_KERNEL_FLEX_PAIR
+  if (g->flex != FLEX_NONE && !g->dual && !g->hyb && !g->mix) k = (const void *)mk_persistent_kernel_flex_pair;
+#endif
+  return k;
+}
 static const void *kernel_of(const mk_graph *g) {
   const bool m1 = g->cfg.max_num_batched_tokens == 1;
   const void *k = nullptr;
@@ -3064,7 +3229,9 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   if (!rt) rt = &g->h_rt;
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
-  HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
+  // (one portion an iteration: the kernel without the linears for two, whose registers are its own)
+  const bool pairs = rt->pair_n > 0 && (run_scheduler == MK_SCHED_OFFLINE || rt->batch2 > 0) && !rt->profiler;
+  HIP_TRY(hipLaunchCooperativeKernel(pairs ? pair_kernel_of(g) : kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
   g->launch_pending = true;
   g->last_stages = run_scheduler == MK_SCHED_INGEST && !rt->profiler && rt->max_tokens > 1 ? rt->tail : rt->num_stages;
   g->launch_stream = stream;
@@ -3098,8 +3265,8 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   }
   if (sc.bad_batch) {
     static const char *why[] = {"", "rows outside [0, max_num_batched_tokens), overlapping, or with gaps", "more rows for one request than max_tokens_per_request",
-                                "a sequence shorter than its new rows, longer than max_seq_length, or without pages"};
-    return fail(MK_EINVAL, "the batch described in qo_indptr / paged_kv_* was rejected and nothing was run: %s", why[sc.bad_batch > 0 && sc.bad_batch <= 3 ? sc.bad_batch : 1]);
+                                "a sequence shorter than its new rows, longer than max_seq_length, or without pages", "fewer than three rows beside another portion"};
+    return fail(MK_EINVAL, "the batch described in qo_indptr / paged_kv_* was rejected and nothing was run: %s", why[sc.bad_batch > 0 && sc.bad_batch <= 4 ? sc.bad_batch : 1]);
   }
   return MK_OK;
 }
@@ -3450,6 +3617,12 @@ int mk_compile(mk_graph *g) {
   int per_cu = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_of(g), MK_THREADS, MK_LDS_BYTES));
   if (per_cu < 1 || g->G > per_cu * g->num_cus) return fail(MK_EINVAL, "grid of %d workgroups cannot be co-resident (%d per CU x %d CUs)", g->G, per_cu, g->num_cus);
+  const void *pairs = g->pair_prog.empty() ? nullptr : pair_kernel_of(g);
+  if (pairs) {
+    HIP_TRY(hipFuncSetAttribute(pairs, hipFuncAttributeMaxDynamicSharedMemorySize, MK_LDS_BYTES));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pairs, MK_THREADS, MK_LDS_BYTES));
+    if (per_cu < 1 || g->G > per_cu * g->num_cus) pairs = nullptr;
+  }
   MkRuntime &rt = g->h_rt;
   rt.num_stages = (int)g->stages.size();
   rt.tail = g->tail;
@@ -3478,11 +3651,11 @@ int mk_compile(mk_graph *g) {
   rt.request_ids = (int *)p;
   if ((rc = dev_alloc(g, &p, sizeof(int) * rt.max_pages))) return rc;
   rt.page_queue = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * rt.max_tokens))) return rc;
+  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;  // (a second portion's behind the first one's)
   rt.tok_slot = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * rt.max_tokens))) return rc;
+  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;
   rt.tok_pos = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * rt.max_tokens))) return rc;
+  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;
   rt.tok_first = (int *)p;
   if ((rc = dev_alloc(g, &p, sizeof(MkSched)))) return rc;
   rt.sched = g->d_sched = (MkSched *)p;
@@ -3573,6 +3746,20 @@ int mk_compile(mk_graph *g) {
   rt.splitk_part = p;
   if ((rc = dev_alloc(g, &p, (size_t)g->G * 32 * sizeof(unsigned)))) return rc;
   rt.splitk_cnt = (unsigned *)p;
+  if (pairs) {
+    std::vector<MkStage> second;
+    bool ok;
+    if ((rc = second_stages(g, second, &ok))) return rc;
+    if (ok) {
+      if ((rc = dev_alloc(g, &p, sizeof(MkStage) * second.size(), false))) return rc;
+      HIP_TRY(hipMemcpy(p, second.data(), sizeof(MkStage) * second.size(), hipMemcpyHostToDevice));
+      rt.stages2 = (const MkStage *)p;
+      if ((rc = dev_alloc(g, &p, sizeof(unsigned) * g->pair_prog.size(), false))) return rc;
+      HIP_TRY(hipMemcpy(p, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
+      rt.pair_prog = (const unsigned *)p;
+      rt.pair_n = (int)g->pair_prog.size();
+    }
+  }
   g->timing_cap = 8192;
   if ((rc = dev_alloc(g, &p, sizeof(long long) * (g->timing_cap + 2)))) return rc;
   rt.timing = g->d_timing = (long long *)p;
@@ -3696,6 +3883,21 @@ int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest) {
   return do_launch(g, (hipStream_t)stream, 1, ingest ? MK_SCHED_INGEST : MK_SCHED_FROM_META, &rt, ingest ? nullptr : g->batch_tokens);
 }
 
+int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2) {
+  if (!g) return fail(MK_EINVAL, "null argument");
+  if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
+  if (!g->h_rt.pair_n || g->h_rt.profiler) return fail(MK_EUNSUPPORTED, "this graph runs portions of prompts one by one");
+  if (words < 1 || words2 < 1 || second < words || second + words2 > g->batch_cap || (second & 1))
+    return fail(MK_EINVAL, "batches of %lld words and of %lld from word %lld on, mk_set_host_batch named %lld", (long long)words, (long long)words2, (long long)second, (long long)g->batch_cap);
+  MkRuntime rt = g->h_rt;
+  rt.batch_src = g->batch_src;
+  rt.batch_dst = g->batch_dst;
+  rt.batch_words = words;
+  rt.batch2 = (int)second;
+  rt.batch_words2 = words2;
+  return do_launch(g, (hipStream_t)stream, 1, MK_SCHED_INGEST, &rt);
+}
+
 int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations) {
   if (!g) return fail(MK_EINVAL, "null argument");
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
@@ -3788,6 +3990,7 @@ int mk_get_stats(mk_graph *g, mk_stats *out) {
   out->packed_weight_bytes = g->packed_bytes;
   out->row_major_weight_bytes = g->row_major_bytes;
   out->last_launch_ms = g->last_ms;
+  out->paired_portions = g->h_rt.pair_n > 0;
   if (g->compiled && !g->launch_pending) {
     MkSched sc;
     HIP_TRY(hipMemcpy(&sc, g->d_sched, sizeof(sc), hipMemcpyDeviceToHost));

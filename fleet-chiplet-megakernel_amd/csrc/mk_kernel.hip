@@ -74,20 +74,27 @@ typedef const __attribute__((address_space(4))) MkWeight CWeight;
 #define MK_TUNE_R24 2
 #endif
 
-#if defined(MK_KERNEL_DUAL) || defined(MK_KERNEL_DUAL_M1) || defined(MK_KERNEL_DUAL_F32)
+#if defined(MK_KERNEL_DUAL) || defined(MK_KERNEL_DUAL_PAIR) || defined(MK_KERNEL_DUAL_M1) || defined(MK_KERNEL_DUAL_F32)
 #define MK_HAVE_DUAL 1  // ... the dual stages (mk_dual.hip) beside flex, mix and hybrid ones, without latent attention, delta rule and selective scan
 #else
 #define MK_HAVE_DUAL 0
 #endif
-#if defined(MK_KERNEL_HYB) || defined(MK_KERNEL_HYB_M1) || defined(MK_KERNEL_HYB_F32) || MK_HAVE_DUAL
+#if defined(MK_KERNEL_HYB) || defined(MK_KERNEL_HYB_PAIR) || defined(MK_KERNEL_HYB_M1) || defined(MK_KERNEL_HYB_F32) || MK_HAVE_DUAL
 #define MK_HAVE_HYB 1
 #else
 #define MK_HAVE_HYB 0
 #endif
-#if defined(MK_KERNEL_MIX) || defined(MK_KERNEL_MIX_M1) || defined(MK_KERNEL_MIX_F32) || MK_HAVE_HYB
+#if defined(MK_KERNEL_MIX) || defined(MK_KERNEL_MIX_PAIR) || defined(MK_KERNEL_MIX_M1) || defined(MK_KERNEL_MIX_F32) || MK_HAVE_HYB
 #define MK_HAVE_MIX 1  // this translation unit holds a kernel with the mix stages (mk_mix.hip) beside the flex ones
 #else
 #define MK_HAVE_MIX 0
+#endif
+
+// kernels that run two portions inside prompts as one iteration, beside everything else
+#if defined(MK_KERNEL_DENSE_PAIR) || defined(MK_KERNEL_FLEX_PAIR) || defined(MK_KERNEL_MIX_PAIR) || defined(MK_KERNEL_HYB_PAIR) || defined(MK_KERNEL_DUAL_PAIR)
+#define MK_PAIR 1
+#else
+#define MK_PAIR 0
 #endif
 
 #define MK_NO_LISTS 0x7fffffff
@@ -125,6 +132,10 @@ struct Ctx {
   const float *defer_part;  // [slice][row][n] fp32
   const void *defer_res;  // residual rows of that linear (null: none)
   int defer_ld_res;
+#if MK_PAIR
+  const void *defer_res2;  // of the second portion
+  int rows_dealt;          // rows of the first portion that the running stage has dealt already
+#endif
 #if MK_HAVE_MIX
   bool mx_split;  // the latent attention (delta rule) that just ran left some request in chunks (its heads in slices)
 #endif
@@ -318,7 +329,7 @@ __device__ __forceinline__ uint16_t ldc_u16(const uint16_t *p) {
 }
 
 // ----------------------------------------------------------------------------- grid barrier
-// Stage barrier with one arrival counter per XCD (each in its own 128-byte line, so a die's arrivals meet in that
+// Stage barrier with one arrival counter per XCD (each in 256 bytes of its own, so a die's arrivals meet in that
 // die's L2 and only completed lines travel between dies).  Replaces the reference's per-event two-level counters
 // (persistent_kernel.cuh:1214-1284).
 __device__ __forceinline__ bool spin_ok(MkSync *s, unsigned &spins, unsigned where) {
@@ -335,7 +346,7 @@ __device__ __forceinline__ bool spin_ok(MkSync *s, unsigned &spins, unsigned whe
 }
 
 // arrive: this workgroup's outputs of the current stage are complete: write them back (agent-scope release) and
-// count the arrival in the counter of this workgroup's XCD (one 128-byte line per die, so the 32 arrivals of a die meet
+// count the arrival in the counter of this workgroup's XCD (one line per die, so the 32 arrivals of a die meet
 // in that die's L2).  Nothing is returned, so nobody waits on the atomic.
 __device__ __forceinline__ void barrier_arrive(Ctx &c) {
   MkSync *s = c.sync;
@@ -561,7 +572,11 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 }
 __device__ __forceinline__ int wave_bcast(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
 
-__device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRuntime &rt, int *lds, int lane) {
+// `half` 1: the portion that runs beside the one just prepared, in the same iteration (MK_PAIR_NEXT in the result of the step that prepared that).
+#define MK_PAIR_NEXT (1 << 16)
+__device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRuntime &rt, int *lds, int lane, int half) {
+  const int second = MK_PAIR ? half * MK_MAX_TOKENS : 0;
+  long long *const ids = second ? rt.ids2 : rt.input_tokens;
   MkSched *sc = rt.sched;
   const int R = rt.max_requests, B = rt.max_tokens, PS = rt.page_size, NP = rt.max_pages;
   int *snap = lds, *freed = lds + NP;
@@ -645,10 +660,10 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
     for (int b = 64; b; b >>= 1)
       if (__any(n >= most + b)) most += b;
     auto write = [&](int row, int first, int rq, int pos, int slot_) {
-      rt.input_tokens[row] = rt.tokens[(long long)rq * rt.max_seq + pos];
-      rt.tok_slot[row] = slot_;
-      rt.tok_pos[row] = pos;
-      rt.tok_first[row] = first;
+      ids[row] = rt.tokens[(long long)rq * rt.max_seq + pos];
+      rt.tok_slot[row + second] = slot_;
+      rt.tok_pos[row + second] = pos;
+      rt.tok_first[row + second] = first;
     };
     unsigned long long several = __ballot(n > 1);
     const bool shared = __popcll(several) < most;
@@ -666,6 +681,7 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
   int taken = wave_bcast(fresh_incl, 63);
   int nreq = nrun;
   bool inner = rt.max_new_per_req > 1 && !__any(n > 0 && (st + n >= plen || st + n + 1 >= rt.max_seq));
+  bool pairs = false;  // the next portion could run in the same iteration: nothing hangs on this one's samples, it is full, and lies inside prompts
   // 4. admit new requests while there is room: lane k looks at request next_request_id + k
   {
     const int next = sc->next_request_id;
@@ -692,6 +708,13 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
       for (int j = 0; j < cneed; j++) rt.kv_indices[page0 + j] = ring_page(a0 + j);
     }
     rows(cn, ntok + cw_incl - cwish, cand, 0, nreq + lane);
+    if (MK_PAIR && !half && rt.pair_n) {
+      const int w1 = alive ? min(plen - st - n, rt.max_new_per_req) : 0, i1 = wave_incl_scan(w1, lane), s1 = wave_bcast(i1, 63);
+      const int w2 = admit ? min(cplen - cn, rt.max_new_per_req) : 0, i2 = s1 + wave_incl_scan(w2, lane);
+      const int n1 = min(i1, B) - min(i1 - w1, B), n2 = min(i2, B) - min(i2 - w2, B);
+      const bool ends = (n1 > 0 && (st + n + n1 >= plen || st + n + n1 + 1 >= rt.max_seq)) || (n2 > 0 && (cn + n2 >= cplen || cn + n2 + 1 >= rt.max_seq));
+      pairs = inner && wave_bcast(i2, 63) >= B && !__any(ends);
+    }
     const int cn_incl = wave_incl_scan(cn, lane);
     ntok += wave_bcast(cn_incl, 63);
     npage += wave_bcast(cneed_incl, 63);
@@ -708,11 +731,16 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
   if (lane == 0) {
     sc->page_queue_head = head0 + taken;
     sc->page_queue_tail = tail0 + n_freed;
-    sc->num_tokens = ntok;
+    if (second) {
+      sc->num_tokens2 = ntok;
+    } else {
+      sc->num_tokens = ntok;
+      sc->num_tokens2 = 0;
+      sc->inner = inner;
+    }
     sc->num_reqs = nreq;
-    sc->inner = inner;
   }
-  return ntok;
+  return pairs && 2 * ntok > B ? ntok | MK_PAIR_NEXT : ntok;
 }
 
 // Batch description for a launch whose batch the HOST prepared (the reference's MODE_ONLINE_NOTOKEN, one pass per launch,
@@ -723,15 +751,17 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // on the device (no host round trip, so a serving loop can enqueue launches back to back).  Runs on one thread.
 // Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).  Reads and
 // writes at device scope: mk_fetch_batch may have written the tensors a moment ago, and nobody releases behind the step.
-__device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt, int lane) {
-  const int R = rt.max_requests, B = rt.max_tokens;
+// `off`: words to the description, of the portion that runs beside the first one in the same iteration (0: the first one's); what is looked up by
+// slot lies there as well.
+__device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt, int lane, int off, bool pair) {
+  const int R = rt.max_requests, B = rt.max_tokens, second = MK_PAIR && off ? MK_MAX_TOKENS : 0;
   // A batch the stages cannot run as described is not run at all: truncating a request's rows would leave the rest with
   // the slot / position an earlier launch gave them, and they would append K/V rows to some other request's cache.
   // bad, of the first slot that cannot run: 1 = rows outside [0, max tokens), overlapping, or with gaps; 2 = more rows for one
   // request than max_tokens_per_request; 3 = a sequence shorter than its new rows, longer than max_seq_length, or without pages.
   const int i = min(lane, R - 1);  // (at most 64 slots)
-  const int q0 = ldc_i32(rt.qo_indptr + i), q1 = ldc_i32(rt.qo_indptr + i + 1), pages = ldc_i32(rt.kv_indptr + i + 1) - ldc_i32(rt.kv_indptr + i),
-            last = ldc_i32(rt.kv_last_page_len + i);
+  const int q0 = ldc_i32(rt.qo_indptr + off + i), q1 = ldc_i32(rt.qo_indptr + off + i + 1), pages = ldc_i32(rt.kv_indptr + off + i + 1) - ldc_i32(rt.kv_indptr + off + i),
+            last = ldc_i32(rt.kv_last_page_len + off + i);
   const int n = lane < R ? q1 - q0 : 0;  // (<= 0: an unused slot; hosts that fill only the first entries leave zeros behind them)
   const int len = (int)((long long)(pages - 1) * rt.page_size) + last;
   const bool inside = n > 0 && q0 >= 0 && n <= B && q0 <= B - n;
@@ -753,6 +783,7 @@ __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt,
   const unsigned long long covered = (unsigned long long)(unsigned)wave_bcast((int)lo, 63) | ((unsigned long long)(unsigned)wave_bcast((int)hi, 63) << 32);
   int ntok = covered ? 64 - __clzll((long long)covered) : 0;
   if (covered != (ntok >= 64 ? ~0ull : ((1ull << ntok) - 1ull)) && !bad) bad = 1;
+  if (pair && ntok < 3 && !bad) bad = 4;
   if (bad) ntok = 0;
   // a lane per row (by the lanes of the slots, row after row, 64 rows of one request took 16 us)
   int slot = 0, first = 0, pos = 0;
@@ -765,13 +796,20 @@ __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt,
     }
   }
   if (lane < ntok) {
-    stc_i32(rt.tok_slot + lane, slot);
-    stc_i32(rt.tok_pos + lane, pos);
-    stc_i32(rt.tok_first + lane, first);
+    stc_i32(rt.tok_slot + second + lane, off + slot);
+    stc_i32(rt.tok_pos + second + lane, pos);
+    stc_i32(rt.tok_first + second + lane, first);
+    if (second) stc_u64(rt.ids2 + lane, ldc_u64((const int *)rt.input_tokens + off + 2 * lane));
   }
   if (lane == 0) {
-    stc_i32(&rt.sched->bad_batch, bad);
-    stc_i32(&rt.sched->num_tokens, ntok);
+    if (!second) {
+      stc_i32(&rt.sched->bad_batch, bad);
+      stc_i32(&rt.sched->num_tokens, ntok);
+    } else if (bad) {  // (then the first one does not run either)
+      stc_i32(&rt.sched->bad_batch, bad);
+      stc_i32(&rt.sched->num_tokens, 0);
+    }
+    stc_i32(&rt.sched->num_tokens2, second ? ntok : 0);
   }
   return ntok;
 }
@@ -864,15 +902,26 @@ __device__ __forceinline__ const u32x4 *weight_row(CWeight &w, int r, int k8) {
 // Every stage function posts barrier_wait(c) itself, after any work that does not depend on the previous
 // stage (weight prefetch), and the main loop posts barrier_arrive(c) when the function returns.
 
+// The row a workgroup takes first where rows are dealt round-robin over the dies (and then every G-th).  A second portion's rows, in a stage that has
+// just dealt the first one's, go to the workgroups behind those.
+__device__ __forceinline__ int row_item(const Ctx &c, int t) {
+#if MK_PAIR
+  return t >= c.rows_dealt ? t - c.rows_dealt : t - c.rows_dealt + c.G;
+#else
+  return t;
+#endif
+}
+__device__ __forceinline__ int row_item(const Ctx &c) { return row_item(c, c.even_xcds ? c.rank * c.nxcd + c.xi : c.vid); }
+
 // Gather embedding rows.  Reference task: tasks/ampere/embedding.cuh:42-72.
 __device__ __forceinline__ void stage_embed(CStage &st, Ctx &c, const MkRuntime &rt, int M) {
   barrier_wait(c);
   const int k8 = st.k / 8;
-  for (int t = c.vid; t < M; t += c.G) {
+  for (int t = row_item(c, c.vid); t < M; t += c.G) {
     long long id;
     if (st.flags & MK_F_EMBED_FROM_TOKENS) {
-      const int req = ldc_i32(&rt.request_ids[ldc_i32(&rt.tok_slot[t])]);
-      id = (long long)ldc_u64(&rt.tokens[(long long)req * rt.max_seq + ldc_i32(&rt.tok_pos[t])]);
+      const int req = ldc_i32(&rt.request_ids[c.sh_tok[MK_MAX_TOKENS + t]]);
+      id = (long long)ldc_u64(&rt.tokens[(long long)req * rt.max_seq + c.sh_tok[t]]);
     } else {
       id = (long long)ldc_u64((const long long *)st.in + t);
     }
@@ -916,7 +965,7 @@ __device__ __forceinline__ void stage_norm_rows(CStage &st, Ctx &c, int M, char 
   const int dS = c.defer_S;
   c.defer_S = 0;
   // rows are dealt round-robin over the dies, so a handful of rows does not funnel through one die's memory path
-  const int t0 = c.even_xcds ? c.rank * c.nxcd + c.xi : c.vid;
+  const int t0 = row_item(c);
   for (int t = t0; t < M; t += c.G) {
     const u32x4 *x = (const u32x4 *)((const uint16_t *)st.in + (size_t)t * st.ld_in);
     u32x4 *y = (u32x4 *)((uint16_t *)st.out + (size_t)t * st.ld_out);
@@ -2010,55 +2059,18 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
 // in slice order), or leave the sum to a norm stage that follows.  Used for the QKV, o, gate/up and down projections at
 // 9..64 tokens.  SwiGLU stages number their weight tiles gate, up, gate, up ...; with three tiles per wavefront the
 // middle pair straddles the two streaming wavefronts and is joined through LDS in the epilogue.
-#define MK_XRES_STEPS 8  // steps per pass
 #ifndef MK_TUNE_XRES_PRE
 #define MK_TUNE_XRES_PRE 6  // ring steps requested before the previous stage's barrier is awaited
 #endif
-struct XresPlan {
-  int S;       // K slices per tile range (0: this form cannot run the stage)
-  int R;       // tile ranges a workgroup walks one after another (1 unless S is 1)
-  int groups;  // tile ranges
-  int wt;      // weight tiles of the stage
-  int tpu;     // most tiles a range holds (decides tiles per wavefront and prefetch depth for every workgroup alike)
-};
-__device__ __forceinline__ XresPlan linear_xres_plan(CStage &st, const Ctx &c) {
-  XresPlan p;
-  p.S = 0;
-  p.groups = 0;
-  p.tpu = 0;
-  const bool silu = st.flags & MK_F_SILU;
-  const int n_out = silu ? st.n / 2 : st.n, unit = silu ? 2 : 1;
-  p.wt = ((n_out + 15) / 16) * unit;
-  for (int S = 1; S <= 8; S *= 2) {
-    if (c.G % S || st.k % (S * 64 * MK_XRES_STEPS)) break;
-    const int gs = c.G / S;
-    int tpu = (p.wt + gs - 1) / gs;  // tiles per range
-    tpu = (tpu + unit - 1) / unit * unit;
-    if (tpu < 4) continue;           // too few tiles to occupy two streaming wavefronts: split K further
-    p.S = S;
-    p.R = 1;
-    if (tpu > 6) {
-      // more than three tiles each: several ranges of equal size, one after another, whose rows are staged anew (an eighth of the weights'
-      // bytes at 64 tokens).  The form for any shape, whose wavefronts read the rows in operand order at every step, took 66.6 / 56.7 us
-      // for 32768 x 4096 at 64 tokens / the last 5 of a prompt; this takes 55.1 / 45.6.
-      const int nun = p.wt / unit;
-      p.R = (nun * unit + 6 * c.G - 1) / (6 * c.G);
-      while ((nun + c.G * p.R - 1) / (c.G * p.R) * unit > 6) p.R++;
-      p.tpu = (nun + c.G * p.R - 1) / (c.G * p.R) * unit;
-      p.groups = min(nun, c.G * p.R);
-      return p;
-    }
-    p.tpu = tpu;
-    p.groups = (p.wt / unit + tpu / unit - 1) / (tpu / unit);
-    return p;
-  }
-  return p;
-}
+__device__ __forceinline__ XresPlan linear_xres_plan(CStage &st, const Ctx &c) { return mk_xres_plan(st, c.G); }
 
+// MT token tiles.  Eight: those of two portions (MK_PAIR_BOTH), four tiles each: M rows of this stage and M2 of `st2`, which differs in where its rows lie.
+// Passes are then half as long, and so is the ring.
 template <int MT, int TW>
-__device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const MkRuntime &rt, int M, const XresPlan plan, char *smem) {
+__device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const MkRuntime &rt, int M, const XresPlan plan, char *smem, CStage &st2, int M2) {
   c.wrote_through = true;  // partial tiles and outputs are all written through: no L2 write-back at this stage's arrival
-  constexpr int NSP = MK_XRES_STEPS;
+  constexpr bool BOTH = MT == 8;
+  constexpr int NSP = BOTH ? MK_XRES_STEPS / 2 : MK_XRES_STEPS;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const bool silu = st.flags & MK_F_SILU;
@@ -2076,6 +2088,7 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   const int kslice = K / S, kbeg = sl * kslice, nsteps = kslice >> 6, npass = nsteps / NSP;
   const uint16_t *x = (st.flags & MK_F_NORM) ? (const uint16_t *)st.norm_out : (const uint16_t *)st.in;
   const int ldx = (st.flags & MK_F_NORM) ? st.ld_norm : st.ld_in;
+  const uint16_t *x2 = !BOTH ? x : (st.flags & MK_F_NORM) ? (const uint16_t *)st2.norm_out : (const uint16_t *)st2.in;
   u32x4 *xl = (u32x4 *)smem;  // two buffers of [step of the pass][token tile][16 rows][8] 16-byte words
   constexpr int XBUF = NSP * MT * 128;  // 16-byte operands per buffer
   int *sflag = (int *)(smem + 2 * XBUF * 16);
@@ -2090,6 +2103,9 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     c.defer_part = (const float *)rt.splitk_part;
     c.defer_res = (st.flags & MK_F_RES) ? st.res : nullptr;
     c.defer_ld_res = st.ld_res;
+#if MK_PAIR
+    c.defer_res2 = (st.flags & MK_F_RES) ? st2.res : nullptr;
+#endif
   }
   // this lane's first operand of weight tile ti, and the distance (in 16-byte operands) between steps and between the two
   // halves of a step: the re-laid copy streams contiguously, the row-major original reads 64 bytes of each of 16 rows
@@ -2116,17 +2132,18 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   // (64 tokens, operand order -> lines, us: 24576 x 4096 41.9 -> 39.6, 4096 x 12288 28.9 -> 27.0, 6144 x 4096 17.3 -> 16.7.)
   auto stage_pass = [&](int pass, int par, int w, int nw) {
     const uint16_t *base = x + kbeg + pass * (NSP * 64) + ((lane & 7) ^ (lane >> 3)) * 8;
+    const uint16_t *base2 = BOTH ? x2 + kbeg + pass * (NSP * 64) + ((lane & 7) ^ (lane >> 3)) * 8 : base;
     u32x4 *buf = xl + (par & 1) * XBUF;
     for (int i = w; i < MT * NSP; i += nw) {
-      const int step = i / MT, mt = i - step * MT, r0 = mt * 16 + (lane >> 3);
+      const int step = i / MT, mt = i - step * MT, r0 = (BOTH ? mt & 3 : mt) * 16 + (lane >> 3), last = (BOTH && mt >= 4 ? M2 : M) - 1;
       __attribute__((address_space(3))) char *dst = (__attribute__((address_space(3))) char *)(buf + (size_t)i * 128);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 16 /* sc1 */);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0 + 8, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 16);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)((BOTH && mt >= 4 ? base2 : base) + (size_t)min(r0, last) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 16 /* sc1 */);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)((BOTH && mt >= 4 ? base2 : base) + (size_t)min(r0 + 8, last) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 16);
     }
   };
 
   {
-    constexpr int NB = 8, NSW = 2;    // ring depth in steps; streaming wavefronts
+    constexpr int NB = NSP, NSW = 2;  // ring depth in steps; streaming wavefronts
     const bool loader = wave >= NSW;  // stages token rows, holds no tiles
     int tw0 = tb + wave * TW;         // a streaming wavefront's first tile
     // (between two ranges of a workgroup the ring stays full, so a wavefront without a tile in one of them reads the last one along)
@@ -2145,7 +2162,7 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     // weights do not depend on the previous stage: the first NBP steps are requested before its barrier is awaited, the
     // rest of the ring right after the first pass's token rows (what a CU has in flight sits in front of the barrier
     // poll and of the row requests)
-    constexpr int NBP = MK_TUNE_XRES_PRE < NB ? MK_TUNE_XRES_PRE : NB;
+    constexpr int NBP = BOTH ? 3 : MK_TUNE_XRES_PRE < NB ? MK_TUNE_XRES_PRE : NB;
     if (streams) {
 #pragma unroll
       for (int j = 0; j < NBP; j++) w_load(wrow, j, a[j]);
@@ -2237,10 +2254,10 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
       auto store_tile = [&](int otile, const f32x4 (&v)[MT]) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-          const int m = mt * 16 + lr;
-          if (m < M) {
-            uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
-            const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
+          const int m = (BOTH ? mt & 3 : mt) * 16 + lr;
+          if (m < (BOTH && mt >= 4 ? M2 : M)) {
+            uint16_t *orow = (uint16_t *)(BOTH && mt >= 4 ? st2.out : st.out) + (size_t)m * st.ld_out;
+            const uint16_t *rrow = (const uint16_t *)(BOTH && mt >= 4 ? st2.res : st.res) + (size_t)m * st.ld_res;
             float rr[4], res[4];
             if (st.flags & MK_F_RES) ldc_bf16x4(rrow, otile * 16 + lg * 4, n_out, res);
 #pragma unroll
@@ -2321,12 +2338,15 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     }
     // ---- combine the S slices: partial tiles through the write-through buffer, summed by the last workgroup to arrive
     if (S > 1) {
+      // [workgroup][wavefront][tile][token tile][lane], 64 KB a workgroup: four wavefronts (two hold tiles) of four by four tiles, or two of four by eight
+      auto part_at = [&](int wg, int ti, int mt) { return (BOTH ? (((size_t)wg * 2 + wave) * 4 + ti) * 8 + mt : (((size_t)wg * 4 + wave) * 4 + ti) * 4 + mt) * 64 + lane; };
+      constexpr int QS = BOTH ? 2 : 4;  // slices requested at once
       if (has_tile) {
 #pragma unroll
         for (int t = 0; t < TW; t++)
 #pragma unroll
           for (int mt = 0; mt < MT; mt++)
-            stc_16B(part + ((((size_t)c.vid * 4 + wave) * 4 + t) * 4 + mt) * 64 + lane, __builtin_bit_cast(u32x4, acc[t][mt]));
+            stc_16B(part + part_at(c.vid, t, mt), __builtin_bit_cast(u32x4, acc[t][mt]));
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -2345,18 +2365,18 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
       for (int t = 0; t < TW; t++)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) acc[t][mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-      for (int q0 = 0; has_tile && q0 < S; q0 += 4) {  // four slices of both tiles requested at once; summed in slice order
-        u32x4 pv[4][TW][MT];
+      for (int q0 = 0; has_tile && q0 < S; q0 += QS) {  // summed in slice order
+        u32x4 pv[QS][TW][MT];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < QS; q++)
           if (q0 + q < S) {
 #pragma unroll
             for (int t = 0; t < TW; t++)
 #pragma unroll
-              for (int mt = 0; mt < MT; mt++) pv[q][t][mt] = ldc_16B(part + ((((size_t)(g * S + q0 + q) * 4 + wave) * 4 + t) * 4 + mt) * 64 + lane);
+              for (int mt = 0; mt < MT; mt++) pv[q][t][mt] = ldc_16B(part + part_at(g * S + q0 + q, t, mt));
           }
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < QS; q++)
           if (q0 + q < S) {
 #pragma unroll
             for (int t = 0; t < TW; t++)
@@ -4711,7 +4731,7 @@ __device__ __attribute__((noinline)) void mk_verify_greedy(int stage, const MkRu
   }
 }
 
-#if defined(MK_KERNEL_FLEX) || defined(MK_KERNEL_FLEX_M1) || defined(MK_KERNEL_FLEX_F32) || MK_HAVE_MIX
+#if defined(MK_KERNEL_FLEX) || defined(MK_KERNEL_FLEX_PAIR) || defined(MK_KERNEL_FLEX_M1) || defined(MK_KERNEL_FLEX_F32) || MK_HAVE_MIX
 #include "mk_flex.hip"
 #if MK_HAVE_MIX
 #include "mk_mix.hip"
@@ -4728,17 +4748,51 @@ __device__ __attribute__((noinline)) void mk_verify_greedy(int stage, const MkRu
 #endif
 
 // The stage set of an instantiation: the fixed-shape stages (E = void), or the flex stages for E-typed activations.
+// M2: rows of a second portion inside prompts (MK_PAIR; 0: none).  A prompt's iterations are bound by streaming the weights, 64 rows at a time; two
+// portions as one iteration stream them once: see MkPairEntry.  Prompts of 2501 tokens of qwen3-8b, 8 layers: 40.0 -> 32.5 ms; of four requests of
+// up to 1501 tokens of suborax-8b, with 24 steps behind them: 97.0 -> 83.3.
 template <int MAXM, typename E>
-__device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkRuntime *rtp, Ctx &c, const int M, const int n_stages, char *smem) {
+__device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkRuntime *rtp, Ctx &c, const int M1, const int M2, const int n_stages, char *smem) {
     constexpr bool FX = !std::is_void<E>::value;
     constexpr bool F32 = std::is_same<E, float>::value;
+    int M = M1;
     bool single = M == 1;  // every request of the iteration brings one token
-    if constexpr (FX && MAXM > 1) {
-      const int lane = threadIdx.x & 63;
-      single = __all(lane >= M || c.sh_tok[2 * MK_MAX_TOKENS + lane] == lane);
-    }
+    auto one_each = [&]() {
+      if constexpr (FX && MAXM > 1) {
+        const int lane = threadIdx.x & 63;
+        single = __all(lane >= M || c.sh_tok[2 * MK_MAX_TOKENS + lane] == lane);
+      }
+    };
+    one_each();
+#if MK_PAIR
+    const bool pair = M2 > 0;
+    const int *const tok1 = c.sh_tok;
+    int sum_S = 0;  // what the last linear for both portions left to the stage behind it
+    bool all_through = true;
+    for (int e = 0; e < (pair ? rt.pair_n : n_stages) && !c.dead; e++) {
+      const unsigned ent = pair ? ((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e] : (unsigned)e;
+      const int s = (int)(ent & MK_PAIR_STAGE);
+      if (ent & MK_PAIR_ACQUIRE) {
+        barrier_wait(c);
+        if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        __syncthreads();
+        continue;
+      }
+      if (pair && ((ent & MK_PAIR_SECOND) != 0) != (c.sh_tok != tok1)) {
+        c.sh_tok = ent & MK_PAIR_SECOND ? tok1 + 4 * MK_MAX_TOKENS : tok1;
+        M = ent & MK_PAIR_SECOND ? M2 : M1;
+        one_each();
+      }
+      if (ent & MK_PAIR_AGAIN) {
+        c.defer_S = sum_S;
+        c.defer_part = (const float *)rt.splitk_part + (size_t)MK_MAX_TOKENS * c.defer_n;
+        c.defer_res = c.defer_res2;
+      }
+      CStage &st = ((CStage *)(unsigned long long)(ent & MK_PAIR_SECOND ? rt.stages2 : rt.stages))[s];
+#else
     for (int s = 0; s < (MAXM == 1 ? rt.num_stages : n_stages) && !c.dead; s++) {
       CStage &st = ((CStage *)(unsigned long long)rt.stages)[s];
+#endif
       const int op = st.op, flags = st.flags;
       // (a handle that holds only the matrix-core copies of its weights runs every linear in a matrix-core form, which
       // reads normalised rows from the NORM stage's output: that stage then runs for one and two tokens as well)
@@ -4753,7 +4807,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
 #endif
       if ((flags & MK_F_ONLY_MULTI) && op == MK_OP_NORM && s + 1 < rt.num_stages && !packed_only) {
         // the few-token linear normalises its rows itself
-        CStage &nx = ((CStage *)(unsigned long long)rt.stages)[s + 1];
+        CStage &nx = (&st)[1];
         if (nx.op == MK_OP_LINEAR && (nx.flags & MK_F_NORM) && nx.in == st.in && linear_small_ok(nx, c, M)) continue;
       }
       // Lane offsets that stages derive from the thread index would otherwise be computed once, ahead of all stages, and wait in scratch
@@ -4804,6 +4858,15 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         case MK_OP_NORM: if constexpr (!FX) stage_norm(st, c, M, smem); break;
         case MK_OP_LINEAR:
           if constexpr (F32) barrier_wait(c);
+#if MK_PAIR
+          else if (ent & MK_PAIR_BOTH) {
+            const XresPlan xp = linear_xres_plan(st, c);
+            CStage &st2 = ((CStage *)(unsigned long long)rt.stages2)[s];
+            if (xp.tpu <= 4) stage_linear_mfma_xres<8, 2>(st, c, rt, M1, xp, smem, st2, M2);
+            else stage_linear_mfma_xres<8, 3>(st, c, rt, M1, xp, smem, st2, M2);
+            sum_S = c.defer_S;
+          }
+#endif
           else if constexpr (MAXM == 1) stage_linear_m1<true, FX>(st, c, smem);
           else if (M == 1 && !(packed_only && st.wpack)) stage_linear_m1<false, FX>(st, c, smem);
           else if (linear_small_ok(st, c, M) && !(packed_only && st.wpack)) {
@@ -4820,14 +4883,14 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
               // (4 tokens with one tile instead of two, us: 6144 x 4096 11.7 -> 10.8, 4096 x 4096 9.8 -> 8.8, 4096 x 12288 19.8 -> 18.6; a third of
               // 48 instead of 64 would be another pair of instances for fewer batches)
               if (M <= 16) {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<1, 2>(st, c, rt, M, xp, smem);
-                else stage_linear_mfma_xres<1, 3>(st, c, rt, M, xp, smem);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<1, 2>(st, c, rt, M, xp, smem, st, 0);
+                else stage_linear_mfma_xres<1, 3>(st, c, rt, M, xp, smem, st, 0);
               } else if (M <= 32) {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<2, 2>(st, c, rt, M, xp, smem);
-                else stage_linear_mfma_xres<2, 3>(st, c, rt, M, xp, smem);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<2, 2>(st, c, rt, M, xp, smem, st, 0);
+                else stage_linear_mfma_xres<2, 3>(st, c, rt, M, xp, smem, st, 0);
               } else {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<4, 2>(st, c, rt, M, xp, smem);
-                else stage_linear_mfma_xres<4, 3>(st, c, rt, M, xp, smem);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<4, 2>(st, c, rt, M, xp, smem, st, 0);
+                else stage_linear_mfma_xres<4, 3>(st, c, rt, M, xp, smem, st, 0);
               }
             } else if (plan.S >= 1 && !(packed_only && st.wpack)) {  // (this form reads the row-major weights)
               if (M <= 16) stage_linear_mfma_tiles<1>(st, c, rt, M, plan, smem);
@@ -4891,6 +4954,20 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         default: barrier_wait(c); break;
       }
       const long long t_out = (long long)wall_clock64();
+#if MK_PAIR
+      c.rows_dealt = 0;
+      if (ent & MK_PAIR_ON) {  // (as between two stages, but nobody waits for anybody)
+        all_through = c.wrote_through;
+        c.wrote_through = false;
+        c.rows_dealt = M1;
+        c.seq++;
+        if (threadIdx.x == 0) c.sh_ticket[c.seq & 1] = 0;
+        __syncthreads();
+        continue;
+      }
+      c.wrote_through = c.wrote_through && all_through && !(ent & MK_PAIR_RELEASE);
+      all_through = true;
+#endif
       barrier_arrive(c);
       if (threadIdx.x == 0 && rt.profiler) {
         // begin = this stage's inputs were complete (the previous stage's barrier seen), end = its outputs were posted
@@ -4926,7 +5003,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int sh_bcast[4];
   __shared__ int sh_quota[10];
-  __shared__ int sh_tok[4][MK_MAX_TOKENS];
+  __shared__ int sh_tok[MK_PAIR ? 8 : 4][MK_MAX_TOKENS];
   __shared__ int sh_ticket[3];
   // rt arrives by value in the kernel-argument segment (scalar loads); rtp is the same structure in device memory
   // for the one non-inlined function that takes its address (the scheduler step)
@@ -4948,6 +5025,11 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   c.prof_n = 0;
   c.st = nullptr;
   c.defer_S = 0;
+#if MK_PAIR
+  c.rows_dealt = 0;
+  c.defer_n = 0;
+  c.defer_res2 = nullptr;
+#endif
   c.wrote_through = false;
   c.arrive_w0 = false;
   if (threadIdx.x == 0) {
@@ -5003,7 +5085,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
     if (c.vid == 0 && threadIdx.x == 0) rt.profiler[0] = (unsigned long long)(unsigned)c.G | (1ull << 32);
   }
 
-  for (int it = 0; it < max_iters && !c.dead; it++) {
+  for (int it = 0, more = 1; it < max_iters && !c.dead; it += more) {
     // ---- scheduler step on one thread of virtual workgroup 0, published through the barrier
     long long t_sched0 = 0, t_sched1 = 0;
     if (run_scheduler) {
@@ -5013,23 +5095,46 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && (rt.max_requests > 2 || MAXM > 1 && rt.max_new_per_req > 8) && rt.spec_len == 0;
       int ntok_w = 0;
       const bool from_meta = run_scheduler == MK_SCHED_FROM_META || run_scheduler == MK_SCHED_INGEST;
-      if (c.vid == 0 && threadIdx.x < 64 && wave_sched) ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x);
+      bool second = false;
+      if (c.vid == 0 && threadIdx.x < 64 && wave_sched) {
+        ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, 0);
+#if MK_PAIR
+        second = __builtin_amdgcn_readfirstlane(ntok_w & MK_PAIR_NEXT) && it + 2 < max_iters && !rt.profiler;  // (the launch's last iteration runs alone)
+        ntok_w &= MK_PAIR_NEXT - 1;
+        if (second) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+          mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, 1);
+        }
+#endif
+      }
       if (from_meta) {
         if (c.vid == 0 && rt.batch_words) {
           mk_fetch_batch(rt.batch_src, rt.batch_dst, rt.batch_words);
+#if MK_PAIR
+          if (rt.batch2) mk_fetch_batch(rt.batch_src + rt.batch2, rt.batch_dst + rt.batch2, rt.batch_words2);
+#endif
           __syncthreads();
         }
         c.wrote_through = true;  // (nothing else was written in this launch)
       }
-      if (c.vid == 0 && threadIdx.x < 64 && from_meta) ntok_w = mk_batch_from_meta(*rtp, threadIdx.x);
+      if (c.vid == 0 && threadIdx.x < 64 && from_meta) {
+        ntok_w = mk_batch_from_meta(*rtp, threadIdx.x, 0, MK_PAIR && rt.batch2);
+#if MK_PAIR
+        second = rt.batch2 && ntok_w > 0;  // (rtp is the graph's; what belongs to this launch is in rt)
+        if (second && mk_batch_from_meta(*rtp, threadIdx.x, rt.batch2, true) == 0) ntok_w = 0;
+#endif
+      }
       if (c.vid == 0 && threadIdx.x == 0) {
         int ntok;
         if (wave_sched || from_meta) ntok = ntok_w;
         else if (run_scheduler == MK_SCHED_OFFLINE) ntok = mk_prepare_next_batch(*rtp, (int *)smem);
         else ntok = mk_online_next_batch(*rtp);
         if (ntok == 0) rt.sched->finished = 1;
-        else rt.sched->iterations++;
-        if (rt.timing && rt.sched->iterations <= rt.timing_cap) rt.timing[rt.sched->iterations] = (long long)wall_clock64();
+        else rt.sched->iterations += second ? 2 : 1;
+        for (int q = second ? 1 : 0; q >= 0; q--)
+          if (rt.timing && rt.sched->iterations - q <= rt.timing_cap) rt.timing[rt.sched->iterations - q] = (long long)wall_clock64();
         t_sched1 = (long long)wall_clock64();
       }
       barrier_arrive(c);
@@ -5041,6 +5146,9 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       sh_bcast[0] = ldc_i32(&rt.sched->num_tokens);
       if constexpr (MAXM > 1) sh_bcast[1] = ldc_i32(&rt.sched->inner);
+#if MK_PAIR
+      sh_bcast[2] = run_scheduler ? ldc_i32(&rt.sched->num_tokens2) : 0;
+#endif
       c.sh_ticket[2] = MK_NO_LISTS;  // (expert lists are this iteration's)
     }
     __syncthreads();
@@ -5054,6 +5162,18 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       sh_tok[2][t] = ldc_i32(&rt.tok_first[t]);
       sh_tok[3][t] = ldc_i32(&rt.kv_indptr[slot]);
     }
+    int M2 = 0;
+#if MK_PAIR
+    M2 = M > 0 ? __builtin_amdgcn_readfirstlane(sh_bcast[2]) : 0;
+    more = M2 > 0 ? 2 : 1;
+    if (const int t = (int)threadIdx.x - MK_MAX_TOKENS; t >= 0 && t < M2) {
+      const int slot = ldc_i32(&rt.tok_slot[MK_MAX_TOKENS + t]);  // (what is looked up by it, page tables among it, lies batch2 words behind)
+      sh_tok[4][t] = ldc_i32(&rt.tok_pos[MK_MAX_TOKENS + t]);
+      sh_tok[5][t] = slot;
+      sh_tok[6][t] = ldc_i32(&rt.tok_first[MK_MAX_TOKENS + t]);
+      sh_tok[7][t] = rt.batch2 + ldc_i32(&rt.kv_indptr[slot]);
+    }
+#endif
     __syncthreads();
     if (threadIdx.x == 0 && rt.stage_prof && run_scheduler) {
       long long *pr = rt.stage_prof + MK_PROF_TICKS * ((size_t)c.vid * (rt.num_stages + 1) + rt.num_stages);
@@ -5073,7 +5193,10 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       if (!rt.profiler && (run_scheduler == MK_SCHED_INGEST || (run_scheduler == MK_SCHED_OFFLINE && inner && it + 1 < max_iters))) n_stages = rt.tail;
     }
     if (M == 0 || c.dead) break;
-    run_stage_program<MAXM, E>(rt, rtp, c, MAXM == 1 ? 1 : M, n_stages, smem);
+    run_stage_program<MAXM, E>(rt, rtp, c, MAXM == 1 ? 1 : M, M2, n_stages, smem);
+#if MK_PAIR
+    c.sh_tok = &sh_tok[0][0];
+#endif
   }
   barrier_wait(c);  // drain: nobody leaves while another workgroup may still poll
   if (rt.profiler && threadIdx.x == 0) rt.profiler_count[c.vid] = c.prof_n;
@@ -5095,6 +5218,25 @@ extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void mk_persistent_kernel
 extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void mk_persistent_kernel_m1(MK_KERNEL_ARGS) {
   mk_kernel_body<1, void>(rt, rtp, max_iters, run_scheduler);
 }
+#endif
+// graphs whose portions inside prompts run two at a time: everything the kernel of several tokens has, and the linears for both portions.  (Kernels of
+// their own, so that the others keep their registers.)
+#define MK_PAIR_KERNEL(name, E) \
+  extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void name(MK_KERNEL_ARGS) { mk_kernel_body<MK_MAX_TOKENS, E>(rt, rtp, max_iters, run_scheduler); }
+#ifdef MK_KERNEL_DENSE_PAIR
+MK_PAIR_KERNEL(mk_persistent_kernel_pair, void)
+#endif
+#ifdef MK_KERNEL_FLEX_PAIR
+MK_PAIR_KERNEL(mk_persistent_kernel_flex_pair, uint16_t)
+#endif
+#ifdef MK_KERNEL_MIX_PAIR
+MK_PAIR_KERNEL(mk_persistent_kernel_mix_pair, uint16_t)
+#endif
+#ifdef MK_KERNEL_HYB_PAIR
+MK_PAIR_KERNEL(mk_persistent_kernel_hyb_pair, uint16_t)
+#endif
+#ifdef MK_KERNEL_DUAL_PAIR
+MK_PAIR_KERNEL(mk_persistent_kernel_dual_pair, uint16_t)
 #endif
 #ifdef MK_KERNEL_FLEX  // graphs with flex stages (mk_flex.hip), 16-bit activations
 extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void mk_persistent_kernel_flex(MK_KERNEL_ARGS) {

@@ -130,7 +130,7 @@ __device__ __forceinline__ void stage_mx_prenorm_t(CStage &st, Ctx &c, int M, bo
   const int ng = st.norm_groups, gl = ng ? st.k / ng : st.k;
   const f32x4 *w4 = (const f32x4 *)st.norm_w, *yw4 = (const f32x4 *)st.y_norm_w;
   const float *xr = (const float *)st.res;
-  const int t0 = mx_spread(c);
+  const int t0 = row_item(c);
   f32x4 g[NS], x[NS];
   auto at = [&](int j) { return min(tid + j * MK_THREADS, n4 - 1); };
   auto load_x = [&](int t) {

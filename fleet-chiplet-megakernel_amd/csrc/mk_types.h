@@ -236,6 +236,50 @@ struct MkStage {
 };
 static_assert(sizeof(MkStage) % 64 == 0, "a descriptor is whole scalar-cache lines");
 
+#define MK_XRES_STEPS 8  // steps of 64 in a pass of the matrix-core linears with staged rows
+struct XresPlan {
+  int S;       // K slices per tile range (0: this form cannot run the stage)
+  int R;       // tile ranges a workgroup walks one after another (1 unless S is 1)
+  int groups;  // tile ranges
+  int wt;      // weight tiles of the stage
+  int tpu;     // most tiles a range holds (decides tiles per wavefront and prefetch depth for every workgroup alike)
+};
+// How a linear runs in the matrix-core form with staged rows (stage_linear_mfma_xres): tiles and slices go by the stage and the workgroups alone.
+template <typename Stage>
+MK_HOST_DEVICE inline XresPlan mk_xres_plan(Stage &st, int G) {
+  XresPlan p;
+  p.S = 0;
+  p.groups = 0;
+  p.tpu = 0;
+  const bool silu = st.flags & MK_F_SILU;
+  const int n_out = silu ? st.n / 2 : st.n, unit = silu ? 2 : 1;
+  p.wt = ((n_out + 15) / 16) * unit;
+  for (int S = 1; S <= 8; S *= 2) {
+    if (G % S || st.k % (S * 64 * MK_XRES_STEPS)) break;
+    const int gs = G / S;
+    int tpu = (p.wt + gs - 1) / gs;  // tiles per range
+    tpu = (tpu + unit - 1) / unit * unit;
+    if (tpu < 4) continue;           // too few tiles to occupy two streaming wavefronts: split K further
+    p.S = S;
+    p.R = 1;
+    if (tpu > 6) {
+      // more than three tiles each: several ranges of equal size, one after another, whose rows are staged anew (an eighth of the weights'
+      // bytes at 64 tokens).  The form for any shape, whose wavefronts read the rows in operand order at every step, took 66.6 / 56.7 us
+      // for 32768 x 4096 at 64 tokens / the last 5 of a prompt; this takes 55.1 / 45.6.
+      const int nun = p.wt / unit;
+      p.R = (nun * unit + 6 * G - 1) / (6 * G);
+      while ((nun + G * p.R - 1) / (G * p.R) * unit > 6) p.R++;
+      p.tpu = (nun + G * p.R - 1) / (G * p.R) * unit;
+      p.groups = nun < G * p.R ? nun : G * p.R;
+      return p;
+    }
+    p.tpu = tpu;
+    p.groups = (p.wt / unit + tpu / unit - 1) / (tpu / unit);
+    return p;
+  }
+  return p;
+}
+
 // LDS map of MX_LATENT_ATTN, in bytes: query operands, one tile of cached rows, weights of the tile's positions, row statistics,
 // page-table entries.  RT: 16-row query tiles per unit; nkc: operand rows of a cached latent; sub: 16-position sub-tiles of a tile.
 struct MkLatentLds {
@@ -251,10 +295,10 @@ MK_HOST_DEVICE inline MkLatentLds mk_latent_lds(int es, int rt, int nkc, int sub
   return l;
 }
 
-// Hierarchical barrier state.  One 128-byte line per counter so that XCD-local
-// counters stay in that XCD's L2.
+// Hierarchical barrier state.  256 bytes per counter: all workgroups poll all of them, and neighbours 128 bytes apart, two in 256 aligned ones,
+// took a decode step of 64 streams of qwen3-8b 0.7 % longer (257.5 -> 255.5 ms).
 struct MkSync {
-  unsigned local_ctr[MK_MAX_XCD][32];
+  unsigned local_ctr[MK_MAX_XCD][64];
   unsigned xcd_count[MK_MAX_XCD][32];  // workgroups of this launch on each die
   unsigned abort_flag;
   unsigned abort_where;
@@ -284,7 +328,19 @@ struct MkSched {
 
   long long iterations;   // decode iterations executed so far (all launches)
   int inner;              // every row of the iteration lies in front of its prompt's last token (portions of several tokens only)
-  int pad2;
+  int num_tokens2;        // rows of the portion that runs in the same iteration (0: none)
+};
+
+// What an iteration of two portions runs, one after another: a stage's index with these bits.  Linears that stream their weights through the matrix
+// cores run for both portions at once (MK_PAIR_BOTH); the stages between two of them run for the first portion and then for the second one.
+enum MkPairEntry {
+  MK_PAIR_STAGE = 0xffff,
+  MK_PAIR_SECOND = 1 << 16,   // for the second portion
+  MK_PAIR_BOTH = 1 << 17,
+  MK_PAIR_ON = 1 << 18,       // the second portion's run of this stage follows without a barrier
+  MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written for the second portion to read: write back behind the stage ...
+  MK_PAIR_ACQUIRE = 1 << 20,  // ... and, no stage, drop what the caches of the dies hold
+  MK_PAIR_AGAIN = 1 << 21,    // the linear in front may have left its sum to this stage
 };
 
 struct MkRuntime {
@@ -308,6 +364,14 @@ struct MkRuntime {
   const int *batch_src;
   int *batch_dst;
   long long batch_words;
+  // two portions inside prompts as one iteration (null / 0: not in this graph).  stages2: the stages as they run for the second portion, over rows of
+  // its own; pair_prog: [pair_n] what runs, see MkPairEntry; ids2: the second portion's tokens; its rows' slots, positions and first rows lie
+  // MK_MAX_TOKENS behind the first one's.  batch2 (mk_enqueue_batches): words from the first portion's description to the second one's, which has batch_words2
+  const MkStage *stages2;
+  const unsigned *pair_prog;
+  long long *ids2;
+  long long batch_words2;
+  int pair_n, batch2;
   // library-owned scheduler memory
   int *request_ids;   // [max_requests] request id per batch slot, -1 = free
   int *state_ids;     // [max_requests] recurrent-state slot per batch slot, a permutation (null: the graph has no recurrence)

@@ -19,13 +19,14 @@ MK_EABORT = -4
 MK_EUNSUPPORTED = -5
 
 MK_CFG_SINGLE_WEIGHT_COPY = 1
+MK_CFG_PAIR_PORTIONS = 2
 MK_MODES = {"offline": 0, "online": 1, "online_notoken": 2, "onepass": 3}
 
 # symbols include/fleet_mk.h declares; tests check that the library exports every one
 EXPORTED_SYMBOLS = [
     "mk_graph_create", "mk_graph_destroy", "mk_tensor_attach", "mk_tensor_new", "mk_tensor_shuffle",
     "mk_tensor_num_dims", "mk_tensor_dim", "mk_tensor_ptr", "mk_add_task", "mk_generate_task_graph",
-    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_set_host_batch", "mk_enqueue_batch", "mk_wait",
+    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_set_host_batch", "mk_enqueue_batch", "mk_enqueue_batches", "mk_wait",
     "mk_run_once", "mk_repack_weights", "mk_tensor_releasable", "mk_set_profiler", "mk_get_stats", "mk_get_stage_profile", "mk_get_stage_marks", "mk_describe_program", "mk_last_error", "mk_version",
 ]
 
@@ -71,6 +72,7 @@ class MkStats(ctypes.Structure):
         ("last_launch_ms", ctypes.c_double),
         ("packed_weight_bytes", ctypes.c_int64),
         ("row_major_weight_bytes", ctypes.c_int64),
+        ("paired_portions", ctypes.c_int),
     ]
 
 
@@ -117,6 +119,7 @@ def load():
     lib.mk_enqueue_ingest.argtypes = [vp, vp]
     lib.mk_set_host_batch.argtypes = [vp, vp, vp, ctypes.c_int64, vp]
     lib.mk_enqueue_batch.argtypes = [vp, vp, ctypes.c_int64, ci]
+    lib.mk_enqueue_batches.argtypes = [vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
     lib.mk_wait.argtypes = [vp, vp, cip]
     i32p = ctypes.POINTER(ctypes.c_int32)
     lib.mk_run_once.argtypes = [vp, vp, ci, i32p, i32p, i32p]
@@ -232,6 +235,9 @@ class Graph:
 
     def enqueue_batch(self, stream, words, ingest):
         check(self._lib.mk_enqueue_batch(self._h, ctypes.c_void_p(stream), int(words), int(ingest)))
+
+    def enqueue_batches(self, stream, words, second, words2):
+        check(self._lib.mk_enqueue_batches(self._h, ctypes.c_void_p(stream), int(words), int(second), int(words2)))
 
     def wait(self, stream) -> bool:
         fin = ctypes.c_int(0)

@@ -213,6 +213,9 @@ cdef class CyGraph:
     def enqueue_batch(self, stream, words, ingest):
         _check(mk.mk_enqueue_batch(self.g, <void *><uintptr_t>(stream or 0), <int64_t>words, 1 if ingest else 0))
 
+    def enqueue_batches(self, stream, words, second, words2):
+        _check(mk.mk_enqueue_batches(self.g, <void *><uintptr_t>(stream or 0), <int64_t>words, <int64_t>second, <int64_t>words2))
+
     def wait(self, stream) -> bool:
         cdef int rc, fin = 0
         cdef void *s = <void *><uintptr_t>(stream or 0)
@@ -244,7 +247,7 @@ cdef class CyGraph:
         return {"num_workgroups": st.num_workgroups, "num_stages": st.num_stages, "num_tasks": st.num_tasks, "num_events": st.num_events,
                 "num_xcds": st.num_xcds, "aborted": st.aborted, "iterations": st.iterations, "weight_bytes": st.weight_bytes,
                 "last_launch_ms": st.last_launch_ms, "packed_weight_bytes": st.packed_weight_bytes,
-                "row_major_weight_bytes": st.row_major_weight_bytes}
+                "row_major_weight_bytes": st.row_major_weight_bytes, "paired_portions": st.paired_portions}
 
     def stage_ticks(self, int workgroup, int max_stages, marks=False) -> list:
         cdef int64_t *buf = <int64_t *>malloc(sizeof(int64_t) * 4 * (max_stages if max_stages > 0 else 1))

@@ -54,6 +54,7 @@ class PersistentKernel:
         max_tokens_per_request: int = None,
         single_weight_copy: bool = None,
         binding: str = None,
+        pair_portions: bool = False,
     ):
         """Arguments as the reference constructor (persistent_kernel.py:368-387).  `max_tokens_per_request` is the
         reference's compile-time MPK_MAX_TOKENS_PER_REQUEST (prompt tokens one request ingests per iteration; 8 on AMD,
@@ -61,6 +62,8 @@ class PersistentKernel:
         `single_weight_copy` (no counterpart in the reference; None takes FLEET_MK_SINGLE_WEIGHT_COPY, else False): a graph
         with max_num_batched_tokens >= 2 then keeps every linear weight ONCE, in the matrix-core tile layout compile()
         makes; `release_row_major_weights()` afterwards drops the attached tensors nothing reads any more.
+        `pair_portions`: the caller's word that no stage reads rows its iteration has not written, token ids apart; two portions inside prompts may then
+        run as one iteration (fleet_mk.h, MK_CFG_PAIR_PORTIONS).
         `binding`: "ctypes" or "cython" -- which binding of the C ABI carries the calls (None: FLEET_MK_BINDING, else ctypes)."""
         self.__finalized__ = False
         self._is_compiled = False
@@ -141,7 +144,7 @@ class PersistentKernel:
             total_num_requests=self.total_num_requests,
             device=-1 if self.host_only else (device.index if device.index is not None else torch.cuda.current_device()),
             eos_token_id=int(eos_token_id), rms_eps=1e-6, mode=_capi.MK_MODES[mode], max_tokens_per_request=self.max_tokens_per_request,
-            flags=_capi.MK_CFG_SINGLE_WEIGHT_COPY if self.single_weight_copy else 0,
+            flags=(_capi.MK_CFG_SINGLE_WEIGHT_COPY if self.single_weight_copy else 0) | (_capi.MK_CFG_PAIR_PORTIONS if pair_portions else 0),
             step=mt["step"].data_ptr(), tokens=mt["tokens"].data_ptr(), input_tokens=mt["input_tokens"].data_ptr(),
             output_tokens=mt["output_tokens"].data_ptr(), num_new_tokens=mt["num_new_tokens"].data_ptr(),
             prompt_lengths=mt["prompt_lengths"].data_ptr(), qo_indptr=mt["qo_indptr_buffer"].data_ptr(),
@@ -1093,6 +1096,10 @@ class PersistentKernel:
         assert host_tokens is None or (host_tokens.is_pinned() and host_tokens.dtype == torch.int64 and host_tokens.is_contiguous() and len(host_tokens) >= self.max_num_batched_tokens)
         self._g.set_host_batch(host_words.data_ptr(), device_words.data_ptr(), min(len(host_words), len(device_words)), host_tokens.data_ptr() if host_tokens is not None else None)
         self._host_batch = host_words, device_words, host_tokens
+
+    def enqueue_batches(self, host_words: int, second: int, second_words: int, default_stream=None):
+        """Two batches whose logits and sampled tokens nobody reads, as one launch; the second is described from word `second` on."""
+        self._g.enqueue_batches(self._stream_ptr(default_stream), host_words, second, second_words)
 
     def enqueue_batch(self, host_words: int, default_stream=None):
         self._g.enqueue_batch(self._stream_ptr(default_stream), host_words, False)

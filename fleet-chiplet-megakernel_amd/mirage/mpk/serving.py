@@ -51,6 +51,8 @@ class ServingSession:
     # device once
     _host = _dev = _sampled = None
     _fetched = False
+    # two passes of which no row is wanted may be one launch (enqueue_batches): word the second one's description begins at, 0: not in this graph
+    _second = 0
     _view = None  # of the logits
     _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
@@ -76,10 +78,13 @@ class ServingSession:
         with a cache of `max_tokens` positions."""
         pages = max(1, max_tokens // page_size)
         max_seq = max_seq_length or pages * page_size
-        # the batch description of a pass travels in one copy: the five index tensors are slices of one buffer
+        # the batch description of a pass travels in one piece: the five index tensors are slices of one buffer, behind which there is room for a
+        # second description
         R = max_requests
-        dev = torch.zeros(2 * max_rows + 4 * R + 2 + pages, dtype=torch.int32, device=device)
-        ids, block = dev[:2 * max_rows].view(torch.int64).view(max_rows, 1), dev[2 * max_rows:]
+        words = 2 * max_rows + 4 * R + 2 + pages
+        second = (words + 1) // 2 * 2
+        dev = torch.zeros(second + words, dtype=torch.int32, device=device)
+        ids, block = dev[:2 * max_rows].view(torch.int64).view(max_rows, 1), dev[2 * max_rows:words]
         qo, kv, last, slots, idx = block.split([R + 1, R + 1, R, R, pages])
         meta = MPKMetadata(mode="online_notoken", max_seq_length=max(2, max_seq), max_num_batched_requests=R, max_num_batched_tokens=max_rows, max_num_pages=pages,
                            page_size=page_size, device=device, weight_from_model=model_path is not None, model_path=model_path, model_name=model_name,
@@ -92,6 +97,7 @@ class ServingSession:
         session._sampled, session._host, session._dev = host[:2 * max_rows].view(torch.int64), host[2 * max_rows:], dev
         mpk.persistent_kernel.attach_host_batch(session._host, dev, session._sampled)
         session._fetched = True
+        session._second = second if mpk.persistent_kernel.stats()["paired_portions"] else 0
         return session
 
     # ------------------------------------------------------------------ steps
@@ -116,18 +122,37 @@ class ServingSession:
         done = [0] * len(entries)
         # single tokens first, so that they share their pass with the head of the longer portions
         order = sorted(range(len(entries)), key=lambda i: len(entries[i][1]))
-        while True:
+
+        def next_batch(done):
             batch, room = [], self.max_rows
             for i in order:
                 n = min(len(entries[i][1]) - done[i], self.rows_per_request, room)
                 if n > 0 and len(batch) < self.max_requests:
                     batch.append((i, n))
                     room -= n
+            # (portions in the middle of their prompts, of which no row is wanted)
+            return batch, all(done[i] + n < len(entries[i][1]) and not any(done[i] <= p < done[i] + n for p in found[i]) for i, n in batch)
+
+        def tokens(batch, done):
+            return [(entries[i][0], entries[i][1][done[i]:done[i] + n]) for i, n in batch]
+
+        while True:
+            batch, unread = next_batch(done)
             if not batch:
                 break
-            # (portions in the middle of their prompts, of which no row is wanted)
-            self._unread = all(done[i] + n < len(entries[i][1]) and not any(done[i] <= p < done[i] + n for p in found[i]) for i, n in batch)
-            sampled = self._pass([(entries[i][0], entries[i][1][done[i]:done[i] + n]) for i, n in batch])
+            if unread and self._second and self._fetched and self.mpk.persistent_kernel.profiler_tensor is None:
+                then = list(done)
+                for i, n in batch:
+                    then[i] += n
+                batch2, unread2 = next_batch(then)
+                if batch2 and unread2 and all(2 * sum(n for _, n in b) > self.max_rows for b in (batch, batch2)):
+                    self._two_passes(tokens(batch, done), tokens(batch2, then))
+                    done = then
+                    for i, n in batch2:
+                        done[i] += n
+                    continue
+            self._unread = unread
+            sampled = self._pass(tokens(batch, done))
             row, wanted = 0, []
             for i, n in batch:
                 lo, hi = done[i], done[i] + n
@@ -154,8 +179,9 @@ class ServingSession:
             return run, greedy
         return torch.stack([r[k] for r, k in rows]), greedy
 
-    def _pass(self, batch):
-        ps, unread, self._unread = self.page_size, self._unread, False
+    def _describe(self, batch):
+        """The requests of a pass have its rows from now on: their ids, and the five index tensors one behind the other."""
+        ps = self.page_size
         ids, qo, kv, last, slots, pages = [], [0], [0], [], [], []
         for rid, toks in batch:
             r = self.requests.get(rid)
@@ -176,24 +202,46 @@ class ServingSession:
             kv.append(len(pages))
             last.append(r.length - (len(r.pages) - 1) * ps)
             slots.append(max(r.slot, 0))
+        pad = self.max_requests - len(batch)
+        return ids, qo + [qo[-1]] * pad + kv + [kv[-1]] * pad + last + [0] * pad + slots + [0] * pad + pages, len(pages)
+
+    def _put(self, at, ids, desc):
+        """A description in pinned memory, from word `at` on; its length."""
+        n, host = 2 * self.max_rows, self._host.numpy()[at:]
+        # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
+        host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
+        host[n:n + len(desc)] = desc
+        return n + len(desc)
+
+    def _two_passes(self, batch, batch2):
+        """Two passes of which nobody reads logits or sampled tokens, as one launch."""
+        pk, stream = self.mpk.persistent_kernel, torch.cuda.current_stream(self._dev.device)
+        words = self._put(0, *self._describe(batch)[:2])
+        try:
+            words2 = self._put(self._second, *self._describe(batch2)[:2])
+        except Exception:  # (out of pages, or not ids: the first pass has happened all the same)
+            pk.enqueue_ingest(default_stream=stream, host_words=words)
+            pk.wait(default_stream=stream)
+            raise
+        pk.enqueue_batches(words, self._second, words2, default_stream=stream)
+        pk.wait(default_stream=stream)
+
+    def _pass(self, batch):
+        unread, self._unread = self._unread, False
+        ids, desc, num_pages = self._describe(batch)
         R, m = self.max_requests, self.mpk
-        pad = R - len(batch)
-        desc = qo + [qo[-1]] * pad + kv + [kv[-1]] * pad + last + [0] * pad + slots + [0] * pad + pages
         if self._host is not None:
-            n, host = 2 * self.max_rows, self._host.numpy()
-            # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
-            host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
-            host[n:n + len(desc)] = desc
+            words = self._put(0, ids, desc)
             pk = m.persistent_kernel
             if self._fetched and pk.profiler_tensor is None:
                 stream = torch.cuda.current_stream(self._dev.device)  # (the logits' copies', whichever device is current)
                 if unread:
-                    pk.enqueue_ingest(default_stream=stream, host_words=n + len(desc))
+                    pk.enqueue_ingest(default_stream=stream, host_words=words)
                 else:
-                    pk.enqueue_batch(n + len(desc), default_stream=stream)
+                    pk.enqueue_batch(words, default_stream=stream)
                 pk.wait(default_stream=stream)
                 return None if unread else self._sampled.tolist()
-            self._dev[:n + len(desc)].copy_(self._host[:n + len(desc)], non_blocking=True)
+            self._dev[:words].copy_(self._host[:words], non_blocking=True)
             if pk.profiler_tensor is not None:  # (the whole call also writes the trace)
                 m()
                 return None
@@ -208,7 +256,7 @@ class ServingSession:
             return self._sampled.tolist()
         t = torch.tensor(desc, dtype=torch.int32)
         for dst, lo, n in ((m.qo_indptr_buffer, 0, R + 1), (m.paged_kv_indptr_buffer, R + 1, R + 1), (m.paged_kv_last_page_len_buffer, 2 * R + 2, R),
-                           (self.state_slots, 3 * R + 2, R), (m.paged_kv_indices_buffer, 4 * R + 2, len(pages))):
+                           (self.state_slots, 3 * R + 2, R), (m.paged_kv_indices_buffer, 4 * R + 2, num_pages)):
             if dst is not None:
                 dst[:n].copy_(t[lo:lo + n])
         m.input_tokens.view(-1)[:len(ids)].copy_(torch.tensor(ids, dtype=torch.int64))

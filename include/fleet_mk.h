@@ -61,8 +61,12 @@ enum mk_mode { MK_MODE_OFFLINE = 0, MK_MODE_ONLINE = 1, MK_MODE_ONLINE_NOTOKEN =
  *      iterations).  With this flag the tile copy is the ONLY one the handle reads after mk_compile: iterations of one and
  *      two tokens run the matrix-core forms as well (a single-token iteration then costs about what a four-token one
  *      does), and every tensor for which mk_tensor_releasable() returns 1 may be freed by the caller.  mk_compile fails
- *      with MK_EUNSUPPORTED if a linear weight cannot be tiled (reduction length not a multiple of 256). */
-enum mk_config_flags { MK_CFG_SINGLE_WEIGHT_COPY = 1 };
+ *      with MK_EUNSUPPORTED if a linear weight cannot be tiled (reduction length not a multiple of 256).
+ *  MK_CFG_PAIR_PORTIONS  the caller's word that no stage reads rows which the iteration it runs in has not written (token ids, caches and recurrent
+ *      states apart): two portions inside prompts, which are iterations of their own otherwise, may then run as one that streams the weights
+ *      once, the second over copies of the row buffers.  Results are the same bit by bit; iterations are counted, limited and timed as
+ *      before, and the last one of a launch runs alone. */
+enum mk_config_flags { MK_CFG_SINGLE_WEIGHT_COPY = 1, MK_CFG_PAIR_PORTIONS = 2 };
 
 /* Constructor arguments of PersistentKernel (persistent_kernel.py:368-387) plus the
  * ten meta tensors in the order the reference hands them to init_func
@@ -174,6 +178,10 @@ int mk_enqueue_ingest(mk_graph *g, void *stream);
  * host_words == NULL forgets it.  MK_EINVAL for memory of another kind. */
 int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens);
 int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
+/* Two such batches as one launch, of which nobody reads logits or sampled tokens (mk_enqueue_ingest): the second, whose rows may continue the
+ * first one's requests, is described in `words2` words from word `second` (even) on, laid out like the first.  For graphs whose portions
+ * run in pairs (mk_stats.paired_portions; MK_EUNSUPPORTED otherwise); each brings at least three rows. */
+int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2);
 /* mk_enqueue_steps for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc); it has no counterpart in the reference.  The call allocates and frees nothing, and every piece
  * of scratch its launch uses -- barrier counters, K-split partial tiles and counters, attention split-KV partials and
@@ -215,6 +223,7 @@ typedef struct mk_stats {
   int64_t packed_weight_bytes; /* device memory the handle holds for matrix-core copies of the weights (0: none) */
   int64_t row_major_weight_bytes; /* bytes of attached linear weights the handle still reads in place (0 with
                                      MK_CFG_SINGLE_WEIGHT_COPY: every linear weight lives in its tile copy only) */
+  int paired_portions;     /* 1: two portions inside prompts run as one iteration (MK_CFG_PAIR_PORTIONS) */
 } mk_stats;
 int mk_get_stats(mk_graph *g, mk_stats *out);
 /* Device-side stage timing of the LAST decode iteration, as seen by virtual workgroup `workgroup`: for each stage four

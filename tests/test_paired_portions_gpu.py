@@ -1,0 +1,104 @@
+"""Two portions inside prompts as one iteration (MK_CFG_PAIR_PORTIONS): the same logits, tokens, caches, states and scheduler tensors, bit by
+bit, as portions one by one."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# linears that run for both portions at once: split in slices and left to the stage behind or summed by the last to arrive, whole, in ranges of
+# four to six tiles; and such that do not (reductions that are no multiple of 512 slices)
+SHAPES = {
+    "wide": dict(hidden_size=4096, num_q_heads=32, num_kv_heads=8, intermediate_size=1536),
+    "mixed": dict(hidden_size=2048, num_q_heads=24, num_kv_heads=6, intermediate_size=6144),
+    "long": dict(hidden_size=2048, num_q_heads=16, num_kv_heads=2, intermediate_size=12288),
+    "experts": dict(hidden_size=2048, num_q_heads=32, num_kv_heads=4, intermediate_size=0, num_experts=16, num_experts_per_tok=4, moe_intermediate_size=768),
+}
+
+
+@pytest.mark.parametrize("name,lengths,B,portion,steps", [
+    ("wide", (64 * 4 + 7,), 64, 64, 100), ("wide", (64 * 5,), 64, 64, 3), ("wide", (129, 200, 65), 64, 64, 100), ("wide", (150, 90, 33), 64, 20, 7), ("mixed", (64 * 3 + 1,), 64, 64, 100),
+    ("mixed", (180, 75), 40, 40, 100), ("long", (64 * 4 + 63,), 64, 64, 2), ("experts", (64 * 4 + 30,), 64, 64, 100), ("wide", (64, 65), 33, 33, 100)])
+def test_offline(name, lengths, B, portion, steps):
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES[name])
+    g = torch.Generator().manual_seed(5)
+    prompts = [torch.randint(0, 512, (n,), generator=g) for n in lengths]
+    w, max_seq, outs = random_weights(shape, seed=2), max(lengths) + 6, []
+    for pairs in (True, False):
+        dec = Qwen3Decoder(shape, w, max_num_batched_tokens=B, max_num_batched_requests=len(lengths), max_seq_length=max_seq, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=portion,
+                           pair_portions=pairs)
+        assert dec.mpk.stats()["paired_portions"] == pairs
+        dec.load_prompts(prompts)
+        out, fin = [], False
+        while not fin:
+            fin = dec.mpk.run_steps(steps)
+            # (rows behind the last iteration's tokens are of older ones)
+            out += [dec.logits().clone(), torch.tensor(dec.mpk.stats()["iterations"])] + [v.clone() for k, v in dec.meta.items() if k != "input_tokens"]
+        out += [dec.k_cache.clone(), dec.v_cache.clone()]
+        outs.append([t.cpu() for t in out])
+        dec.mpk.finalize()
+    assert len(outs[0]) == len(outs[1]) and all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+def _model(family):
+    import generate
+    make, sizes = generate.SHAPES[family + "-2k"]
+    torch.manual_seed(7)
+    return generate.random_model(make(**sizes, layers={"suborax": 2, "dodonex": 4, "bukatar": 4, "vizonex": 4}[family], vocab=1000, **({"positions": 512} if family == "vizonex" else {})))[0]
+
+
+@pytest.mark.parametrize("family", ["suborax", "dodonex", "bukatar", "vizonex"])
+def test_session(family):
+    """Prompts of several requests, some of which begin or end inside a pair, then steps of one token each."""
+    from mirage.mpk import ServingSession
+    model = _model(family)
+    g = torch.Generator().manual_seed(9)
+    prompts = [torch.randint(0, 1000, (n,), generator=g).tolist() for n in (300, 215, 170)]
+    outs = []
+    for pairs in (True, False):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=1536, max_requests=3, max_seq_length=512)
+        assert s._second > 0
+        s._second, calls = s._second if pairs else 0, []
+        run = s.mpk.persistent_kernel.enqueue_batches
+        s.mpk.persistent_kernel.enqueue_batches = lambda *a, **k: (calls.append(1), run(*a, **k))
+        out = [s.step(list(enumerate(prompts)), [[len(p) - 1] for p in prompts])]
+        out += [s.step([(r, [3 + i]) for r in range(3)], [[0]] * 3) for i in range(2)]
+        out.append(s.step([(0, prompts[1][:190])], [[189]]))
+        assert len(calls) >= 3 if pairs else not calls
+        outs.append([(lg.cpu(), greedy) for lg, greedy in out])
+        s.finalize()
+    for (a, ga), (b, gb) in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a, b) and ga == gb
+
+
+def test_descriptions_that_do_not_fit():
+    from mirage import _capi
+    from mirage.mpk import ServingSession
+    s = ServingSession.open(model_config=_model("suborax"), max_tokens=512, max_requests=2, max_seq_length=256)
+    pk, at, n = s.mpk.persistent_kernel, s._second, len(s._dev)
+    for bad in ((0, at, 4), (at + 1, at, 4), (4, at, 0), (4, at, n - at + 1), (4, at + 1, 4)):
+        with pytest.raises(_capi.MkError, match="mk_set_host_batch named"):
+            pk.enqueue_batches(*bad)
+    cache = [c.clone() for c in s.mpk.model_builder.k_cache]
+    for rows in ((64, 2), (2, 64)):  # too few rows beside another portion: nothing runs
+        words = s._put(0, *s._describe([("a", list(range(rows[0])))])[:2])
+        words2 = s._put(at, *s._describe([("b", list(range(rows[1])))])[:2])
+        pk.enqueue_batches(words, at, words2)
+        with pytest.raises(_capi.MkError, match="fewer than three rows"):
+            pk.wait()
+        s.end("a")
+        s.end("b")
+    assert all(torch.equal(a, b) for a, b in zip(cache, s.mpk.model_builder.k_cache))
+    s.finalize()
+
+
+def test_graphs_that_run_portions_one_by_one():
+    from mirage import _capi
+    from suborax_helpers import CONFIGS, weights
+    from mirage.mpk import MirageModelConfig, ServingSession
+    cfg = CONFIGS[sorted(CONFIGS)[0]]
+    s = ServingSession.open(model_config=MirageModelConfig(architecture=cfg, state_dict={k: v.cuda() for k, v in weights(cfg).items()}), max_tokens=512, max_requests=2, max_seq_length=256)
+    assert s._second == 0 and s.mpk.persistent_kernel.stats()["paired_portions"] == 0  # (linears of this size do not stream through the matrix cores)
+    with pytest.raises(_capi.MkError, match="one by one"):
+        s.mpk.persistent_kernel.enqueue_batches(4, 8, 4)
+    s.finalize()
