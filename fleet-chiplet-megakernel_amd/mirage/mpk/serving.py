@@ -123,10 +123,15 @@ class ServingSession:
         # single tokens first, so that they share their pass with the head of the longer portions
         order = sorted(range(len(entries)), key=lambda i: len(entries[i][1]))
 
+        # places in front of the first one whose logits are wanted (the last one's greedy token always is): as long as they fill passes, passes
+        # are made of them alone, which are run without what only logits need, two at a time where the graph can
+        inner = [min([len(e[1]) - 1, *f]) for e, f in zip(entries, found)]
+
         def next_batch(done):
             batch, room = [], self.max_rows
+            ends = inner if sum(max(0, h - d) for h, d in zip(inner, done)) >= room else [len(e[1]) for e in entries]
             for i in order:
-                n = min(len(entries[i][1]) - done[i], self.rows_per_request, room)
+                n = min(ends[i] - done[i], self.rows_per_request, room)
                 if n > 0 and len(batch) < self.max_requests:
                     batch.append((i, n))
                     room -= n
