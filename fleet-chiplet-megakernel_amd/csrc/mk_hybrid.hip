@@ -306,16 +306,9 @@ __device__ __forceinline__ void hy_route_groups(CStage &st, const float *z, int 
   w = 0.f;
   id = 0;
   for (int k = 0; k < st.topk; k++) {
-    float bv = p[0];
-    int be = lane;
-#pragma unroll
-    for (int q = 1; q < 4; q++)
-      if (p[q] > bv) {
-        bv = p[q];
-        be = q * 64 + lane;
-      }
-    wave_argmax(bv, be);
-    be = __builtin_amdgcn_readfirstlane(be);
+    float bv;
+    int be;
+    wave_pick(p, k, bv, be);
     const float sv = lane_f32(be < 64 ? s[0] : be < 128 ? s[1] : be < 192 ? s[2] : s[3], be & 63);
     if (lane == k) {
       w = sv * st.choice_scale;
@@ -357,15 +350,9 @@ __device__ __forceinline__ void hy_route_wave(CStage &st, const float *z, int la
   w = 0.f;
   id = 0;
   for (int s = 0; s < st.topk; s++) {
-    float bv = p[0];
-    int be = lane;
-#pragma unroll
-    for (int q = 1; q < 4; q++)
-      if (p[q] > bv) {
-        bv = p[q];
-        be = q * 64 + lane;
-      }
-    wave_argmax(bv, be);
+    float bv;
+    int be;
+    wave_pick(p, s, bv, be);
     tot += bv;
     if (lane == s) {
       w = bv;

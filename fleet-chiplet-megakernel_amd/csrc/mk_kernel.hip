@@ -2636,10 +2636,26 @@ __device__ __forceinline__ void wave_argmax(float &bv, int &be) {
   be = re;
 }
 
+// The largest of a wavefront's 256 values (value q of lane l has index 64 q + l) and its index, the lower one of equal values; in every lane.  Bound by
+// the chain of dependent instructions: a maximum without indices and one comparison per value are 40 of them, pairs of value and index carried
+// through the reduction were 100 (eight of 128 experts of each of 16 tokens, as a stage: 6.5 -> 4.9 us).  `none`: the index where no value equals the maximum (all of them NaN).
+__device__ __forceinline__ void wave_pick(const float (&p)[4], int none, float &bv, int &be) {
+  bv = wave_max(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])));
+  be = none;
+#pragma unroll
+  for (int q = 3; q >= 0; q--) {
+    const unsigned long long has = __ballot(p[q] == bv);
+    if (has) be = q * 64 + (int)__ffsll(has) - 1;
+  }
+}
+
 // Route one token with one wavefront: fp32 softmax over all experts, `topk` rounds of arg-max (equal probabilities
 // go to the lower expert id), weights renormalised by the sum of the selected probabilities.  Lane l owns experts
 // l, l+64, ...: sel[j] becomes 1 + slot for a selected expert l + 64 j, 0 otherwise; lane s < topk returns the weight
 // and expert of slot s.  Reference task: tasks/mi300/moe_topk_softmax_mi300.cuh:100-213.
+// PICK: by wave_pick.  Not inside the single-token expert linear: that stage became 1.1 us shorter, but W2 behind it, whose registers are allotted
+// together with it, 1.8 longer (a step of qwen3-30b-a3b, 8 layers, 64 times: 30.15 -> 30.7 ms).
+template <bool PICK>
 __device__ __forceinline__ void moe_route_wave(const uint16_t *logits, int E, int topk, int lane, int sel[4], float &w_slot, int &e_slot) {
   float p[4];
   float mx = -3.0e38f;
@@ -2666,13 +2682,17 @@ __device__ __forceinline__ void moe_route_wave(const uint16_t *logits, int E, in
   for (int s = 0; s < topk; s++) {
     float bv = p[0];
     int be = lane;
+    if constexpr (PICK) {
+      wave_pick(p, s, bv, be);
+    } else {
 #pragma unroll
-    for (int j = 1; j < 4; j++)
-      if (p[j] > bv) {
-        bv = p[j];
-        be = j * 64 + lane;
-      }
-    wave_argmax(bv, be);
+      for (int j = 1; j < 4; j++)
+        if (p[j] > bv) {
+          bv = p[j];
+          be = j * 64 + lane;
+        }
+      wave_argmax(bv, be);
+    }
     tot += bv;
     if (lane == s) {
       w_slot = bv;
@@ -2698,7 +2718,7 @@ __device__ __forceinline__ void stage_moe_topk(CStage &st, Ctx &c, int M) {
     int sel[4];
     float w;
     int e;
-    moe_route_wave((const uint16_t *)st.moe_logits + (size_t)t * st.ld_logits, E, st.topk, lane, sel, w, e);
+    moe_route_wave<true>((const uint16_t *)st.moe_logits + (size_t)t * st.ld_logits, E, st.topk, lane, sel, w, e);
     if (lane < st.topk) __hip_atomic_store(st.moe_topk_w + (size_t)t * st.ld_topk_w + lane, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int j = 0; j < 4; j++)
@@ -2801,7 +2821,7 @@ __device__ __forceinline__ void stage_moe_linear_t(CStage &st, Ctx &c, int M, ch
       int sel[4];
       float w;
       int e;
-      moe_route_wave((const uint16_t *)st.moe_logits, st.num_experts, st.topk, lane, sel, w, e);
+      moe_route_wave<false>((const uint16_t *)st.moe_logits, st.num_experts, st.topk, lane, sel, w, e);
 #pragma unroll
       for (int j = 0; j < 4; j++)
         if (j * 64 + lane < st.num_experts) {
@@ -3036,7 +3056,7 @@ __device__ __forceinline__ void stage_moe_linear_m1(CStage &st, Ctx &c, char *sm
       int sel[4];
       float w;
       int e;
-      moe_route_wave((const uint16_t *)st.moe_logits, E, topk, lane, sel, w, e);
+      moe_route_wave<false>((const uint16_t *)st.moe_logits, E, topk, lane, sel, w, e);
       if (lane < topk) {
         L->act_e[lane] = e;
         L->w[lane] = w;
@@ -3776,7 +3796,7 @@ __device__ __forceinline__ void stage_attn(CStage &st, Ctx &c, const MkRuntime &
     const int t = a.t, h = a.h, p = a.p, C = a.C;
     __syncthreads();  // LDS reuse across units
     // ---- phase A: prepare q heads and the new K/V rows of this chunk
-    attn_rows<2>(st, src, QPK + 2 * a.n_new, lane, wave,
+    attn_rows<QPK == 8 ? 3 : 2>(st, src, QPK + 2 * a.n_new, lane, wave,  // (the rows of one new position in one round trip)
                  [&](int i) -> AttnRow {
                    const int j = i - QPK, kind = j < 0 ? 0 : j < a.n_new ? 1 : 2, jj = kind == 2 ? j - a.n_new : j, base = h * (QPK + 2) * D;
                    return kind ? AttnRow{a.t0 + (a.new_lo + jj - a.p0), base + (QPK + kind - 1) * D, a.new_lo + jj, kind, (kind == 1 ? knew : vnew) + jj * D}
