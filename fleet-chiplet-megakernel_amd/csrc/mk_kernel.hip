@@ -753,7 +753,7 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // writes at device scope: mk_fetch_batch may have written the tensors a moment ago, and nobody releases behind the step.
 // `off`: words to the description, of the portion that runs beside the first one in the same iteration (0: the first one's); what is looked up by
 // slot lies there as well.
-__device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt, int lane, int off, bool pair) {
+__device__ __forceinline__ int mk_batch_from_meta(const MkRuntime &rt, int lane, int off, bool pair) {
   const int R = rt.max_requests, B = rt.max_tokens, second = MK_PAIR && off ? MK_MAX_TOKENS : 0;
   // A batch the stages cannot run as described is not run at all: truncating a request's rows would leave the rest with
   // the slot / position an earlier launch gave them, and they would append K/V rows to some other request's cache.
@@ -814,21 +814,38 @@ __device__ __attribute__((noinline)) int mk_batch_from_meta(const MkRuntime &rt,
   return ntok;
 }
 
-// The words of a batch in pinned host memory go where the stages read them, by one workgroup, each word read once.  Bound by one round trip
-// over the bus, which overlaps nothing: 2 us for up to 2048 words.  (As a copy on the stream in front of the launch it cost 12: a cooperative
+// The words of a batch in pinned host memory go where the stages read them, by one wavefront, each word read once.  Bound by one round trip
+// over the bus, 2 us for up to 2048 words.  (As a copy on the stream in front of the launch it cost 12: a cooperative
 // launch sits on a queue of its own and waits for the copy's signal.  Words behind the end read again as the first ones, as elsewhere here, made it
 // 18 to 40: lines that the host has just written are slow to fetch, every time.)
-__device__ __attribute__((noinline)) void mk_fetch_batch(const int *src, int *dst, long long words) {
-  for (long long i = threadIdx.x; i < words; i += 8 * MK_THREADS) {
-    int v[8];
+__device__ __forceinline__ void mk_fetch_batch(const int *src, int *dst, long long words, int lane) {
+  for (long long i = lane; i < words; i += 32 * 64) {
+    int v[32];
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (i + k * MK_THREADS < words) v[k] = __hip_atomic_load(src + i + k * MK_THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (int k = 0; k < 32; k++)
+      if (i + k * 64 < words) v[k] = __hip_atomic_load(src + i + k * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (i + k * MK_THREADS < words) stc_i32(dst + i + k * MK_THREADS, v[k]);
+    for (int k = 0; k < 32; k++)
+      if (i + k * 64 < words) stc_i32(dst + i + k * 64, v[k]);
   }
+}
+
+// The scheduler's step of a launch whose batch the host describes, by one wavefront of the first workgroup, beside the handshake that opens the
+// launch: behind it, on the first virtual workgroup, its 5.6 us came on top (13 passes of suborax-small FIG1).
+__device__ __attribute__((noinline)) void mk_open_batch(const MkRuntime &rt, int lane, const int *src, int *dst, long long words, int second, long long words2) {
+  if (words) mk_fetch_batch(src, dst, words, lane);
+  if (MK_PAIR && second) mk_fetch_batch(src + second, dst + second, words2, lane);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int ntok = mk_batch_from_meta(rt, lane, 0, MK_PAIR && second);
+  const bool pair = MK_PAIR && second && ntok > 0;
+  if (pair && mk_batch_from_meta(rt, lane, second, true) == 0) ntok = 0;
+  if (lane == 0) {
+    MkSched *sc = rt.sched;
+    if (ntok == 0) sc->finished = 1;
+    else sc->iterations += pair ? 2 : 1;
+    for (int q = pair ? 1 : 0; q >= 0; q--)
+      if (rt.timing && sc->iterations - q <= rt.timing_cap) rt.timing[sc->iterations - q] = (long long)wall_clock64();
+  }
 }
 
 // The reference's MODE_ONLINE step (persistent_kernel.cuh:538-568): one request (slot 0, request 0) whose tokens the
@@ -5059,6 +5076,11 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   // ---- XCD discovery: rank of this workgroup inside its die, dies in use, workgroups per die.  The dies' counters are all there is: they are
   // final once they add up to the grid.  (One counter for the whole grid beside them, awaited with acquiring loads: 8.0 us instead of 4.6 in a launch of
   // nothing else.)
+  const bool from_meta = run_scheduler == MK_SCHED_FROM_META || run_scheduler == MK_SCHED_INGEST;
+  if (from_meta && blockIdx.x == 0 && __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 1) {
+    // (rtp is the graph's; what belongs to this launch is in rt)
+    mk_open_batch(*rtp, threadIdx.x & 63, rt.batch_src, rt.batch_dst, rt.batch_words, MK_PAIR ? rt.batch2 : 0, MK_PAIR ? rt.batch_words2 : 0);
+  }
   if (threadIdx.x == 0) {
     MkSync *s = rt.sync;
     if (blockIdx.x == 0) s->t_begin = (long long)wall_clock64();
@@ -5114,7 +5136,6 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       // a handful of slots and short portions: one thread walks them; else a wavefront, one lane per slot
       const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && (rt.max_requests > 2 || MAXM > 1 && rt.max_new_per_req > 8) && rt.spec_len == 0;
       int ntok_w = 0;
-      const bool from_meta = run_scheduler == MK_SCHED_FROM_META || run_scheduler == MK_SCHED_INGEST;
       bool second = false;
       if (c.vid == 0 && threadIdx.x < 64 && wave_sched) {
         ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, 0);
@@ -5129,26 +5150,10 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
         }
 #endif
       }
-      if (from_meta) {
-        if (c.vid == 0 && rt.batch_words) {
-          mk_fetch_batch(rt.batch_src, rt.batch_dst, rt.batch_words);
-#if MK_PAIR
-          if (rt.batch2) mk_fetch_batch(rt.batch_src + rt.batch2, rt.batch_dst + rt.batch2, rt.batch_words2);
-#endif
-          __syncthreads();
-        }
-        c.wrote_through = true;  // (nothing else was written in this launch)
-      }
-      if (c.vid == 0 && threadIdx.x < 64 && from_meta) {
-        ntok_w = mk_batch_from_meta(*rtp, threadIdx.x, 0, MK_PAIR && rt.batch2);
-#if MK_PAIR
-        second = rt.batch2 && ntok_w > 0;  // (rtp is the graph's; what belongs to this launch is in rt)
-        if (second && mk_batch_from_meta(*rtp, threadIdx.x, rt.batch2, true) == 0) ntok_w = 0;
-#endif
-      }
-      if (c.vid == 0 && threadIdx.x == 0) {
+      if (from_meta) c.wrote_through = true;  // (nothing else was written in this launch)
+      if (c.vid == 0 && threadIdx.x == 0 && !from_meta) {
         int ntok;
-        if (wave_sched || from_meta) ntok = ntok_w;
+        if (wave_sched) ntok = ntok_w;
         else if (run_scheduler == MK_SCHED_OFFLINE) ntok = mk_prepare_next_batch(*rtp, (int *)smem);
         else ntok = mk_online_next_batch(*rtp);
         if (ntok == 0) rt.sched->finished = 1;
@@ -5157,6 +5162,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
           if (rt.timing && rt.sched->iterations - q <= rt.timing_cap) rt.timing[rt.sched->iterations - q] = (long long)wall_clock64();
         t_sched1 = (long long)wall_clock64();
       }
+      if (from_meta && c.vid == 0 && threadIdx.x == 0) t_sched1 = t_sched0;  // (prepared by now, or awaited below)
       barrier_arrive(c);
     }
     barrier_wait(c);
