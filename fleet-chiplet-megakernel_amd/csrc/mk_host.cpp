@@ -170,6 +170,11 @@ __global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, Launch
   __syncthreads();
   for (unsigned i = t; i < sizeof(MkSync) / 4; i += blockDim.x) ((unsigned *)sync)[i] = 0u;
 }
+// Between the two kernels of one launch: the barrier's counters begin anew, the launch's time and a watchdog's verdict stay.
+__global__ void mk_launch_resume_kernel(MkSync *sync) {
+  for (unsigned i = threadIdx.x; i < sizeof(sync->local_ctr) / 4; i += blockDim.x) ((unsigned *)sync->local_ctr)[i] = 0u;
+  for (unsigned i = threadIdx.x; i < sizeof(sync->xcd_count) / 4; i += blockDim.x) ((unsigned *)sync->xcd_count)[i] = 0u;
+}
 static_assert(sizeof(MkSched) % 4 == 0 && sizeof(MkSched) / 4 <= 192 && sizeof(MkSync) % 4 == 0, "copied word by word");
 
 // Launches report their own status: the thread's last error may be one that an earlier call of somebody else left.
@@ -223,6 +228,7 @@ struct mk_graph {
   bool single_copy = false;
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
   int tail = 0;      // MkRuntime::tail
+  bool inside_prompts = true;  // the last launch ended inside prompts, or none has been since the requests began
   int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
@@ -3229,9 +3235,17 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   if (!rt) rt = &g->h_rt;
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
-  // (one portion an iteration: the kernel without the linears for two, whose registers are its own)
-  const bool pairs = rt->pair_n > 0 && (run_scheduler == MK_SCHED_OFFLINE || rt->batch2 > 0) && !rt->profiler;
-  HIP_TRY(hipLaunchCooperativeKernel(pairs ? pair_kernel_of(g) : kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
+  // Two portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions and the other kernel
+  // goes on; the launch begins with it unless the last one ended outside prompts (25 to 45 us of launch and handshake for nothing, and only speed is
+  // lost where the guess is wrong).
+  const bool both = rt->batch2 > 0;
+  const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && max_iters > 2 && g->inside_prompts;
+  if (first || both) HIP_TRY(hipLaunchCooperativeKernel(pair_kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
+  if (first) {
+    HIP_TRY(launch_kernel(mk_launch_resume_kernel, 1, 256, stream, rt->sync));
+    run_scheduler = MK_SCHED_RESUME;
+  }
+  if (!both) HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
   g->launch_pending = true;
   g->last_stages = run_scheduler == MK_SCHED_INGEST && !rt->profiler && rt->max_tokens > 1 ? rt->tail : rt->num_stages;
   g->launch_stream = stream;
@@ -3255,6 +3269,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   g->last_aborted = hs.abort_flag != 0;
   if (!hs.abort_flag) g->last_ms = (hs.t_end - hs.t_begin) * 1e-5;
   const MkSched &sc = hs.sched;
+  g->inside_prompts = sc.inner != 0;
   if (finished_out) *finished_out = sc.finished;
   if (hs.abort_flag) {
     // workgroups that unwound mid-stage may have left the split-K and split-KV arrival counters mid-count (their last
@@ -3803,6 +3818,7 @@ int mk_init_requests(mk_graph *g) {
   sc.page_queue_head = 0;
   sc.page_queue_tail = rt.max_pages;
   HIP_TRY(hipMemcpy(g->d_sched, &sc, sizeof(sc), hipMemcpyHostToDevice));
+  g->inside_prompts = true;
   HIP_TRY(hipMemset(rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
   HIP_TRY(hipMemset(rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));
   HIP_TRY(hipMemset(rt.profiler_count, 0, sizeof(unsigned) * (size_t)g->G));

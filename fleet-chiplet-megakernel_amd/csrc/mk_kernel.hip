@@ -4802,12 +4802,11 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
     };
     one_each();
 #if MK_PAIR
-    const bool pair = M2 > 0;
     const int *const tok1 = c.sh_tok;
     int sum_S = 0;  // what the last linear for both portions left to the stage behind it
     bool all_through = true;
-    for (int e = 0; e < (pair ? rt.pair_n : n_stages) && !c.dead; e++) {
-      const unsigned ent = pair ? ((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e] : (unsigned)e;
+    for (int e = 0; e < rt.pair_n && !c.dead; e++) {
+      const unsigned ent = ((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e];
       const int s = (int)(ent & MK_PAIR_STAGE);
       if (ent & MK_PAIR_ACQUIRE) {
         barrier_wait(c);
@@ -4815,7 +4814,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         __syncthreads();
         continue;
       }
-      if (pair && ((ent & MK_PAIR_SECOND) != 0) != (c.sh_tok != tok1)) {
+      if (((ent & MK_PAIR_SECOND) != 0) != (c.sh_tok != tok1)) {
         c.sh_tok = ent & MK_PAIR_SECOND ? tok1 + 4 * MK_MAX_TOKENS : tok1;
         M = ent & MK_PAIR_SECOND ? M2 : M1;
         one_each();
@@ -4905,12 +4904,15 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
           }
 #endif
           else if constexpr (MAXM == 1) stage_linear_m1<true, FX>(st, c, smem);
+#if !MK_PAIR  // (portions in pairs have three rows or more)
           else if (M == 1 && !(packed_only && st.wpack)) stage_linear_m1<false, FX>(st, c, smem);
           else if (linear_small_ok(st, c, M) && !(packed_only && st.wpack)) {
             if (M <= 2) stage_linear_small_dispatch<2>(st, c, M, smem);
             else if (M <= 4) stage_linear_small_dispatch<4>(st, c, M, smem);
             else stage_linear_small_dispatch<8>(st, c, M, smem);
-          } else {
+          }
+#endif
+          else {
             const int wt = (((flags & MK_F_SILU) ? st.n / 2 : st.n) + 15) / 16;  // output tiles of the stage
             const bool narrow = ((wt + c.G - 1) / c.G) * ((flags & MK_F_SILU) ? 2 : 1) <= 2;
             const TilePlan plan = linear_tiles_plan(st, c);
@@ -5083,7 +5085,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   }
   if (threadIdx.x == 0) {
     MkSync *s = rt.sync;
-    if (blockIdx.x == 0) s->t_begin = (long long)wall_clock64();
+    if (blockIdx.x == 0 && run_scheduler != MK_SCHED_RESUME) s->t_begin = (long long)wall_clock64();
     const unsigned rank = __hip_atomic_fetch_add(&s->xcd_count[c.xcd][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned n[MK_MAX_XCD], spins = 0;
     while (true) {
@@ -5127,14 +5129,23 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
     if (c.vid == 0 && threadIdx.x == 0) rt.profiler[0] = (unsigned long long)(unsigned)c.G | (1ull << 32);
   }
 
-  for (int it = 0, more = 1; it < max_iters && !c.dead; it += more) {
+  int it0 = 0;
+  bool prepared = false;  // the iteration is scheduled already
+  if constexpr (MAXM > 1 && !MK_PAIR) {
+    prepared = run_scheduler == MK_SCHED_RESUME;
+    if (prepared) {
+      run_scheduler = MK_SCHED_OFFLINE;
+      it0 = __builtin_amdgcn_readfirstlane(ldc_i32(&rt.sched->resume_it));
+    }
+  }
+  for (int it = it0, more = 1; it < max_iters && !c.dead; it += more) {
     // ---- scheduler step on one thread of virtual workgroup 0, published through the barrier
     long long t_sched0 = 0, t_sched1 = 0;
     if (run_scheduler) {
       barrier_wait(c);  // the previous iteration's sampled tokens are complete
       t_sched0 = (long long)wall_clock64();
       // a handful of slots and short portions: one thread walks them; else a wavefront, one lane per slot
-      const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && (rt.max_requests > 2 || MAXM > 1 && rt.max_new_per_req > 8) && rt.spec_len == 0;
+      const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && !prepared && (rt.max_requests > 2 || MAXM > 1 && rt.max_new_per_req > 8) && rt.spec_len == 0;
       int ntok_w = 0;
       bool second = false;
       if (c.vid == 0 && threadIdx.x < 64 && wave_sched) {
@@ -5151,18 +5162,20 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
 #endif
       }
       if (from_meta) c.wrote_through = true;  // (nothing else was written in this launch)
-      if (c.vid == 0 && threadIdx.x == 0 && !from_meta) {
+      if (c.vid == 0 && threadIdx.x == 0 && !from_meta && !prepared) {
         int ntok;
         if (wave_sched) ntok = ntok_w;
         else if (run_scheduler == MK_SCHED_OFFLINE) ntok = mk_prepare_next_batch(*rtp, (int *)smem);
         else ntok = mk_online_next_batch(*rtp);
         if (ntok == 0) rt.sched->finished = 1;
         else rt.sched->iterations += second ? 2 : 1;
+        if (MK_PAIR) rt.sched->resume_it = ntok == 0 ? max_iters : it;
         for (int q = second ? 1 : 0; q >= 0; q--)
           if (rt.timing && rt.sched->iterations - q <= rt.timing_cap) rt.timing[rt.sched->iterations - q] = (long long)wall_clock64();
         t_sched1 = (long long)wall_clock64();
       }
-      if (from_meta && c.vid == 0 && threadIdx.x == 0) t_sched1 = t_sched0;  // (prepared by now, or awaited below)
+      if ((from_meta || prepared) && c.vid == 0 && threadIdx.x == 0) t_sched1 = t_sched0;  // (scheduled by now, or awaited below)
+      prepared = false;
       barrier_arrive(c);
     }
     barrier_wait(c);
@@ -5219,6 +5232,9 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       if (!rt.profiler && (run_scheduler == MK_SCHED_INGEST || (run_scheduler == MK_SCHED_OFFLINE && inner && it + 1 < max_iters))) n_stages = rt.tail;
     }
     if (M == 0 || c.dead) break;
+#if MK_PAIR
+    if (M2 == 0) break;  // (the iteration is left to the kernel behind this one)
+#endif
     run_stage_program<MAXM, E>(rt, rtp, c, MAXM == 1 ? 1 : M, M2, n_stages, smem);
 #if MK_PAIR
     c.sh_tok = &sh_tok[0][0];
@@ -5245,8 +5261,10 @@ extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void mk_persistent_kernel
   mk_kernel_body<1, void>(rt, rtp, max_iters, run_scheduler);
 }
 #endif
-// graphs whose portions inside prompts run two at a time: everything the kernel of several tokens has, and the linears for both portions.  (Kernels of
-// their own, so that the others keep their registers.)
+// Iterations of two portions inside prompts, and nothing else: a launch of the offline scheduler that begins inside prompts runs this kernel up to its
+// first iteration that is none, which the kernel of several tokens goes on from (MK_SCHED_RESUME).  Two kernels, as registers are allotted to
+// all stages of one together: decode steps that ran here too were up to 3.7 % longer (qwen3-8b, 8 layers, rows for portions of 64, 24 requests
+// 883 -> 915 us, 8 requests 807 -> 826), and with the pairs as a function beside the other stages both were slower (690 -> 1010, prompts 32.3 -> 36.0 ms).
 #define MK_PAIR_KERNEL(name, E) \
   extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void name(MK_KERNEL_ARGS) { mk_kernel_body<MK_MAX_TOKENS, E>(rt, rtp, max_iters, run_scheduler); }
 #ifdef MK_KERNEL_DENSE_PAIR

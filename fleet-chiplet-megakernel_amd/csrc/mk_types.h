@@ -317,6 +317,7 @@ enum MkSchedMode {
   MK_SCHED_OFFLINE = 1,      // on-GPU continuous batching over `tokens` (MODE_OFFLINE)
   MK_SCHED_FROM_META = 2,    // derived on the GPU from the qo / paged-kv meta tensors the host filled (MODE_ONLINE_NOTOKEN, MODE_ONEPASS)
   MK_SCHED_ONLINE = 3,       // one request, host-written tokens consumed num_new_tokens[0] at a time (MODE_ONLINE)
+  MK_SCHED_RESUME = 5,       // MK_SCHED_OFFLINE from iteration MkSched::resume_it on, which has been scheduled: the launch began with pairs of portions
   MK_SCHED_INGEST = 4,       // MK_SCHED_FROM_META, and nobody reads the logits or sampled tokens of the batch (mk_enqueue_ingest)
 };
 
@@ -329,6 +330,7 @@ struct MkSched {
   long long iterations;   // decode iterations executed so far (all launches)
   int inner;              // every row of the iteration lies in front of its prompt's last token (portions of several tokens only)
   int num_tokens2;        // rows of the portion that runs in the same iteration (0: none)
+  int resume_it, unused;  // the launch's first iteration that the pair kernel left to the other one
 };
 
 // What an iteration of two portions runs, one after another: a stage's index with these bits.  Linears that stream their weights through the matrix
