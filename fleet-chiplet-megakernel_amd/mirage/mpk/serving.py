@@ -54,6 +54,9 @@ class ServingSession:
     # two passes of which no row is wanted may be one launch (enqueue_batches): word the second one's description begins at, 0: not in this graph
     _second = 0
     _view = None  # of the logits
+    # 32-bit linears add in an order that depends on how many rows a pass has, and results are the same bit by bit whichever rows are wanted: there
+    # the rows that nobody reads stay where they are (16.9 ms for three prompts and their steps of a 2048-wide model, 15.7 with them in front)
+    _unread_first = True
     _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
     def __init__(self, mpk: MPK):
@@ -68,6 +71,7 @@ class ServingSession:
         self.state_slots = getattr(mpk.model_builder, "state_slots", None)
         if self.state_slots is not None:
             self.slots = PagePool(self.max_requests, "state slots")
+        self._unread_first = mpk.metadata.dtype != torch.float32
         self.requests: Dict[object, _Request] = {}
         mpk._ensure_compiled()
 
@@ -129,7 +133,7 @@ class ServingSession:
 
         def next_batch(done):
             batch, room = [], self.max_rows
-            ends = inner if sum(max(0, h - d) for h, d in zip(inner, done)) >= room else [len(e[1]) for e in entries]
+            ends = inner if self._unread_first and sum(max(0, h - d) for h, d in zip(inner, done)) >= room else [len(e[1]) for e in entries]
             for i in order:
                 n = min(ends[i] - done[i], self.rows_per_request, room)
                 if n > 0 and len(batch) < self.max_requests:

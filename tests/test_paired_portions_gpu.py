@@ -19,14 +19,24 @@ SHAPES = {
     ("wide", (64 * 4 + 7,), 64, 64, 100), ("wide", (64 * 5,), 64, 64, 3), ("wide", (129, 200, 65), 64, 64, 100), ("wide", (150, 90, 33), 64, 20, 7), ("mixed", (64 * 3 + 1,), 64, 64, 100),
     ("mixed", (180, 75), 40, 40, 100), ("long", (64 * 4 + 63,), 64, 64, 2), ("experts", (64 * 4 + 30,), 64, 64, 100), ("wide", (64, 65), 33, 33, 100)])
 def test_offline(name, lengths, B, portion, steps):
+    _offline(name, lengths, B, portion, steps, len(lengths))
+
+
+@pytest.mark.parametrize("R,steps", [(1, 100), (1, 3), (1, 5), (2, 100)])
+def test_requests_that_wait(R, steps):
+    """Prompts that begin when others have been answered: behind the first iteration that is not of two portions, and where a launch begins."""
+    _offline("wide", (200, 150, 300), 64, 64, steps, R)
+
+
+def _offline(name, lengths, B, portion, steps, R):
     from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
     shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES[name])
     g = torch.Generator().manual_seed(5)
     prompts = [torch.randint(0, 512, (n,), generator=g) for n in lengths]
     w, max_seq, outs = random_weights(shape, seed=2), max(lengths) + 6, []
     for pairs in (True, False):
-        dec = Qwen3Decoder(shape, w, max_num_batched_tokens=B, max_num_batched_requests=len(lengths), max_seq_length=max_seq, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=portion,
-                           pair_portions=pairs)
+        dec = Qwen3Decoder(shape, w, max_num_batched_tokens=B, max_num_batched_requests=R, max_seq_length=max_seq, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=portion,
+                           pair_portions=pairs, total_requests=len(lengths))
         assert dec.mpk.stats()["paired_portions"] == pairs
         dec.load_prompts(prompts)
         out, fin = [], False
