@@ -55,7 +55,7 @@ class ServingSession:
     _second = 0
     _view = None  # of the logits
     # 32-bit linears add in an order that depends on how many rows a pass has, and results are the same bit by bit whichever rows are wanted: there
-    # the rows that nobody reads stay where they are (16.9 ms for three prompts and their steps of a 2048-wide model, 15.7 with them in front)
+    # the rows that nobody reads stay where they are (16.2 ms for three prompts and their steps of a 2048-wide model, 15.7 with them in front)
     _unread_first = True
     _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
