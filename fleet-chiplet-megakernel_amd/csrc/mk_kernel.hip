@@ -923,7 +923,7 @@ __device__ __forceinline__ const u32x4 *weight_row(CWeight &w, int r, int k8) {
 // just dealt the first one's, go to the workgroups behind those.
 __device__ __forceinline__ int row_item(const Ctx &c, int t) {
 #if MK_PAIR
-  return t >= c.rows_dealt ? t - c.rows_dealt : t - c.rows_dealt + c.G;
+  return mk_first_row(t, c.rows_dealt, c.G);
 #else
   return t;
 #endif

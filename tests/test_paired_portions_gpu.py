@@ -11,6 +11,7 @@ SHAPES = {
     "wide": dict(hidden_size=4096, num_q_heads=32, num_kv_heads=8, intermediate_size=1536),
     "mixed": dict(hidden_size=2048, num_q_heads=24, num_kv_heads=6, intermediate_size=6144),
     "long": dict(hidden_size=2048, num_q_heads=16, num_kv_heads=2, intermediate_size=12288),
+    "narrow": dict(hidden_size=1024, num_q_heads=32, num_kv_heads=4, intermediate_size=6144),
     "experts": dict(hidden_size=2048, num_q_heads=32, num_kv_heads=4, intermediate_size=0, num_experts=16, num_experts_per_tok=4, moe_intermediate_size=768),
 }
 
@@ -28,7 +29,13 @@ def test_requests_that_wait(R, steps):
     _offline("wide", (200, 150, 300), 64, 64, steps, R)
 
 
-def _offline(name, lengths, B, portion, steps, R):
+@pytest.mark.parametrize("workgroups,name,B", [(32, "wide", 64), (48, "wide", 64), (32, "mixed", 40), (48, "narrow", 64)])
+def test_grids_smaller_than_a_portion(workgroups, name, B):
+    """Rows of the second portion start again at the first workgroup; "narrow": where a linear left its sum to them."""
+    _offline(name, (B * 4 + 7, 70), B, B, 100, 2, num_workers=workgroups)
+
+
+def _offline(name, lengths, B, portion, steps, R, **kw):
     from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
     shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES[name])
     g = torch.Generator().manual_seed(5)
@@ -36,7 +43,7 @@ def _offline(name, lengths, B, portion, steps, R):
     w, max_seq, outs = random_weights(shape, seed=2), max(lengths) + 6, []
     for pairs in (True, False):
         dec = Qwen3Decoder(shape, w, max_num_batched_tokens=B, max_num_batched_requests=R, max_seq_length=max_seq, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=portion,
-                           pair_portions=pairs, total_requests=len(lengths))
+                           pair_portions=pairs, total_requests=len(lengths), **kw)
         assert dec.mpk.stats()["paired_portions"] == pairs
         dec.load_prompts(prompts)
         out, fin = [], False
