@@ -21,6 +21,7 @@
 
 #include "../../include/fleet_mk.h"
 #include "mk_types.h"
+#include "mk_launch.h"
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -228,6 +229,7 @@ struct mk_graph {
   bool single_copy = false;
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
   int tail = 0;      // MkRuntime::tail
+  bool requests_lost = false;  // a call failed behind the kernel that scheduled an iteration (mk_enqueue_parts): until the requests begin anew
   bool inside_prompts = true;  // the last launch ended inside prompts, or none has been since the requests began
   int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
@@ -3231,6 +3233,7 @@ static const void *kernel_of(const mk_graph *g) {
 int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler, const MkRuntime *rt = nullptr, long long *host_tokens = nullptr) {
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending: call mk_wait first");
+  if (g->requests_lost) return fail(MK_ESTATE, "a launch failed half-way and left its requests inside an iteration: call mk_init_requests first");
   HIP_TRY(hipSetDevice(g->cfg.device));
   if (!rt) rt = &g->h_rt;
   const MkRuntime *rtp = g->d_rt;
@@ -3240,17 +3243,39 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   // lost where the guess is wrong).
   const bool both = rt->batch2 > 0;
   const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && max_iters > 2 && g->inside_prompts;
-  if (first || both) HIP_TRY(hipLaunchCooperativeKernel(pair_kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
-  if (first) {
-    HIP_TRY(launch_kernel(mk_launch_resume_kernel, 1, 256, stream, rt->sync));
-    run_scheduler = MK_SCHED_RESUME;
-  }
-  if (!both) HIP_TRY(hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream));
+  const char *what = "";
+  auto enqueue = [&](MkLaunchPart part) -> int {
+    switch (part) {
+      case MK_PART_PAIRS:
+        what = "kernel of two portions";
+        return hipLaunchCooperativeKernel(pair_kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream);
+      case MK_PART_RESUME:
+        what = "hand-over";
+        run_scheduler = MK_SCHED_RESUME;
+        return launch_kernel(mk_launch_resume_kernel, 1, 256, stream, rt->sync);
+      case MK_PART_MAIN:
+        what = "kernel";
+        return hipLaunchCooperativeKernel(kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream);
+      default:
+        what = "end of the launch";
+        return launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status, (const long long *)rt->output_tokens,
+                             host_tokens ? rt->max_tokens : 0, host_tokens);
+    }
+  };
+  auto undo = [&](bool lost) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(stream, &capture);
+    if (capture != hipStreamCaptureStatusNone) return;  // (nothing runs; what the capture holds is its owner's to drop)
+    (void)hipStreamSynchronize(stream);
+    (void)hipMemset(rt->sync, 0, sizeof(MkSync));
+    (void)hipGetLastError();
+    g->requests_lost = lost;
+  };
+  const int err = mk_enqueue_parts(first, both, enqueue, undo);
+  if (err) return fail(MK_EHIP, "launch: %s: %s", what, hipGetErrorString((hipError_t)err));
   g->launch_pending = true;
   g->last_stages = run_scheduler == MK_SCHED_INGEST && !rt->profiler && rt->max_tokens > 1 ? rt->tail : rt->num_stages;
   g->launch_stream = stream;
-  HIP_TRY(launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status, (const long long *)rt->output_tokens,
-                        host_tokens ? rt->max_tokens : 0, host_tokens));
   return MK_OK;
 }
 
@@ -3819,6 +3844,7 @@ int mk_init_requests(mk_graph *g) {
   sc.page_queue_tail = rt.max_pages;
   HIP_TRY(hipMemcpy(g->d_sched, &sc, sizeof(sc), hipMemcpyHostToDevice));
   g->inside_prompts = true;
+  g->requests_lost = false;
   HIP_TRY(hipMemset(rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
   HIP_TRY(hipMemset(rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));
   HIP_TRY(hipMemset(rt.profiler_count, 0, sizeof(unsigned) * (size_t)g->G));
