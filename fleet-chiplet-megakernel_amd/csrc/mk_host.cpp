@@ -2262,6 +2262,8 @@ std::vector<unsigned> pair_program(const mk_graph *g) {
   const int n = g->tail;
   if (!(c.flags & MK_CFG_PAIR_PORTIONS) || n >= (int)g->stages.size() || n > MK_PAIR_STAGE || g->flex == FLEX_F32 || g->spec_len > 0 || c.mode == MK_MODE_ONLINE || (pack && atoi(pack) == 0)) return prog;
   if (c.max_num_batched_tokens <= 32 || c.max_num_batched_tokens > MK_MAX_TOKENS || c.max_tokens_per_request <= 8) return prog;
+  if (c.mode != MK_MODE_OFFLINE && std::any_of(g->stages.begin(), g->stages.end(), [](const MkStage &s) { return (s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) && (s.flags & MK_F_EMBED_FROM_TOKENS); }))
+    return prog;  // (the rows of requests that the host does not describe)
   auto keeps_nothing = [&](const MkStage &s) { return !s.k_cache && !s.v_cache && !s.tail && !s.conv_w; };
   auto row_wise = [&](const MkStage &s) {
     return keeps_nothing(s) && (s.op == MK_OP_NORM || s.op == MK_OP_FX_ADDNORM || s.op == MK_OP_MX_PRENORM || s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED);
@@ -3931,6 +3933,13 @@ int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second,
   if (!g->h_rt.pair_n || g->h_rt.profiler) return fail(MK_EUNSUPPORTED, "this graph runs portions of prompts one by one");
   if (words < 1 || words2 < 1 || second < words || second + words2 > g->batch_cap || (second & 1))
     return fail(MK_EINVAL, "batches of %lld words and of %lld from word %lld on, mk_set_host_batch named %lld", (long long)words, (long long)words2, (long long)second, (long long)g->batch_cap);
+  // the second description is read `second` words behind every tensor of the first one: all of that is in the named words
+  auto named = [&](const void *p, size_t bytes) { return !p || ((const char *)p >= (const char *)g->batch_dst && (const char *)p + 4 * second + bytes <= (const char *)(g->batch_dst + g->batch_cap)); };
+  const mk_config &c = g->cfg;
+  const size_t R = (size_t)c.max_num_batched_requests;
+  if (!named(c.input_tokens, 8 * (size_t)c.max_num_batched_tokens) || !named(c.qo_indptr, 4 * (R + 1)) || !named(c.paged_kv_indptr, 4 * (R + 1)) || !named(c.paged_kv_last_page_len, 4 * R) ||
+      !named(c.paged_kv_indices, 4 * (size_t)c.max_num_pages) || !named(g->state_ids, 4 * R))
+    return fail(MK_EINVAL, "two batches in one launch need the ids and all index tensors, and as much again from word %lld on, in the device words that mk_set_host_batch named", (long long)second);
   MkRuntime rt = g->h_rt;
   rt.batch_src = g->batch_src;
   rt.batch_dst = g->batch_dst;

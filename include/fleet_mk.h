@@ -180,7 +180,8 @@ int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_wo
 int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
 /* Two such batches as one launch, of which nobody reads logits or sampled tokens (mk_enqueue_ingest): the second, whose rows may continue the
  * first one's requests, is described in `words2` words from word `second` (even) on, laid out like the first.  For graphs whose portions
- * run in pairs (mk_stats.paired_portions; MK_EUNSUPPORTED otherwise); each brings at least three rows. */
+ * run in pairs (mk_stats.paired_portions; MK_EUNSUPPORTED otherwise); each brings at least three rows.  All index tensors of the graph, and as many
+ * words again from word `second` on, lie in the device words named (MK_EINVAL). */
 int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2);
 /* mk_enqueue_steps for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc); it has no counterpart in the reference.  The call allocates and frees nothing, and every piece

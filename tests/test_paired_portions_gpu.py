@@ -109,6 +109,27 @@ def test_descriptions_that_do_not_fit():
     s.finalize()
 
 
+def test_words_that_do_not_hold_both_descriptions():
+    """The second description is read behind the graph's own tensors: launches where that lies outside the named words are refused."""
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    from mirage import _capi
+    from mirage.mpk import ServingSession
+    shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES["wide"])
+    dec = Qwen3Decoder(shape, random_weights(shape, seed=2), max_num_batched_tokens=64, max_num_batched_requests=2, max_seq_length=200, page_size=16, max_tokens_per_request=64,
+                       kernel_mode="online_notoken")
+    assert dec.mpk.stats()["paired_portions"]
+    dec.mpk.attach_host_batch(torch.zeros(4096, dtype=torch.int32, pin_memory=True), torch.zeros(4096, dtype=torch.int32, device="cuda"))  # (its tensors lie elsewhere)
+    with pytest.raises(_capi.MkError, match="the ids and all index tensors"):
+        dec.mpk.enqueue_batches(4, 2048, 4)
+    dec.mpk.finalize()
+    s = ServingSession.open(model_config=_model("suborax"), max_tokens=512, max_requests=2, max_seq_length=256)
+    pk, at, n = s.mpk.persistent_kernel, s._second, len(s._dev)
+    pk._g.set_host_batch(s._host.data_ptr(), s._dev.data_ptr(), n - 1, s._sampled.data_ptr())
+    with pytest.raises(_capi.MkError, match="the ids and all index tensors"):
+        pk.enqueue_batches(4, at, 4)
+    s.finalize()
+
+
 def test_graphs_that_run_portions_one_by_one():
     from mirage import _capi
     from suborax_helpers import CONFIGS, weights
