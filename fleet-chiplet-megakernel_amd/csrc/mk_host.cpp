@@ -3887,11 +3887,12 @@ int mk_enqueue_ingest(mk_graph *g, void *stream) {
   return do_launch(g, (hipStream_t)stream, 1, MK_SCHED_INGEST);
 }
 
-// Address of [p, p + bytes) as the graph's device sees it: pinned host memory, or device memory.  Null: it is neither from end to end.
-static void *device_view(const void *p, size_t bytes, hipMemoryType type) {
+// Address of [p, p + bytes) as `device` sees it: pinned host memory, or that device's own.  Null: it is neither from end to end.
+static void *device_view(const void *p, size_t bytes, hipMemoryType type, int device) {
   hipPointerAttribute_t a, b;
   const bool ok = hipPointerGetAttributes(&a, p) == hipSuccess && hipPointerGetAttributes(&b, (const char *)p + bytes - 1) == hipSuccess;
   if (!ok) (void)hipGetLastError();
+  if (ok && type == hipMemoryTypeDevice && (a.device != device || b.device != device)) return nullptr;
   if (!ok || a.type != type || b.type != type || !a.devicePointer || (char *)b.devicePointer - (char *)a.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
   return a.devicePointer;
 }
@@ -3907,11 +3908,11 @@ int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_wo
   if (((uintptr_t)host_words | (uintptr_t)device_words) & 3) return fail(MK_EINVAL, "words of a batch lie on four bytes");
   HIP_TRY(hipSetDevice(g->cfg.device));
   const size_t token_bytes = sizeof(int64_t) * (size_t)g->h_rt.max_tokens;
-  g->batch_src = (const int *)device_view(host_words, 4 * (size_t)words, hipMemoryTypeHost);
-  g->batch_dst = (int *)device_view(device_words, 4 * (size_t)words, hipMemoryTypeDevice);
-  g->batch_tokens = host_tokens ? (long long *)device_view(host_tokens, token_bytes, hipMemoryTypeHost) : nullptr;
+  g->batch_src = (const int *)device_view(host_words, 4 * (size_t)words, hipMemoryTypeHost, g->cfg.device);
+  g->batch_dst = (int *)device_view(device_words, 4 * (size_t)words, hipMemoryTypeDevice, g->cfg.device);
+  g->batch_tokens = host_tokens ? (long long *)device_view(host_tokens, token_bytes, hipMemoryTypeHost, g->cfg.device) : nullptr;
   if (!g->batch_src || !g->batch_dst || (host_tokens && (!g->batch_tokens || (uintptr_t)host_tokens & 7)))
-    return fail(MK_EINVAL, "batch words and sampled tokens are in pinned host memory, the words' place in device memory");
+    return fail(MK_EINVAL, "batch words and sampled tokens are in pinned host memory, the words' place in the graph's device's memory");
   g->batch_cap = words;
   return MK_OK;
 }
