@@ -9,7 +9,9 @@ own ms_per_step, context range and roofline); --batch N runs one batch size only
 
 roofline: the dominant (only) kernel is mk_persistent_kernel; its algorithmic bytes per launch are
 K x (all bf16 weight matrices once + the K/V rows of every cached position of every request), divided by the launch
-duration measured with HIP events on the launch stream, against the 8 TB/s HBM peak.
+duration by the device's own clock (mk_stats.last_launch_ms: from the kernel's start to its end; lines of before that
+clock were timed by HIP events on the launch's stream, which held the launch itself too, 10 to 20 us), against the 8 TB/s
+HBM peak.
 cpu_baseline: the CPU oracle's torch-order decode (the reference's PyTorch path restated) of the whole model timed on the
 host cores: an 80-token prompt, then a window of 8 decode steps (a few layers + LM head extrapolated when the host has
 too little memory for the 16 GB of weights); a reported baseline, not a target.

@@ -3294,7 +3294,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   for (int i = 0; i < MK_MAX_XCD; i++) nx += hs.xcd_count[i] > 0;
   g->last_nxcd = nx;
   g->last_aborted = hs.abort_flag != 0;
-  if (!hs.abort_flag) g->last_ms = (hs.t_end - hs.t_begin) * 1e-5;
+  g->last_ms = hs.abort_flag ? 0.0 : (hs.t_end - hs.t_begin) * 1e-5;
   const MkSched &sc = hs.sched;
   g->inside_prompts = sc.inner != 0;
   if (finished_out) *finished_out = sc.finished;

@@ -312,7 +312,7 @@ struct MkSync {
   unsigned abort_flag;
   unsigned abort_where;
   unsigned pad[30];
-  long long t_begin, t_end;  // 100 MHz ticks: the first workgroup's entry, everybody through
+  long long t_begin, t_end;  // 100 MHz ticks: when workgroup 0 of the launch's first kernel began, and when everybody was through
 };
 
 // Barrier completion test.  Arrival counters and their targets (quota x epoch) are 32-bit and only ever grow during a

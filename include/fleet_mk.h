@@ -220,7 +220,9 @@ typedef struct mk_stats {
   int aborted;             /* watchdog fired in the last launch */
   int64_t iterations;      /* decode iterations executed since mk_init_requests */
   int64_t weight_bytes;    /* bytes of weight matrices streamed by one iteration */
-  double last_launch_ms;   /* device time of the last launch that mk_wait has seen, from its first workgroup's entry to its last stage's end */
+  double last_launch_ms;   /* device time of the last launch that mk_wait has seen, from when workgroup 0 of its first kernel begins to the end of its
+                              last stage (by the device's clock: without what lies in front of the kernel and behind it on the stream); 0 if it
+                              was aborted */
   int64_t packed_weight_bytes; /* device memory the handle holds for matrix-core copies of the weights (0: none) */
   int64_t row_major_weight_bytes; /* bytes of attached linear weights the handle still reads in place (0 with
                                      MK_CFG_SINGLE_WEIGHT_COPY: every linear weight lives in its tile copy only) */
