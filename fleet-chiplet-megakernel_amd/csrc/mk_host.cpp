@@ -2308,7 +2308,7 @@ std::vector<unsigned> pair_program(const mk_graph *g) {
 }
 
 // The stages as they run for the second portion: over rows of its own, in copies of the memory that stages write rows to.  False: some stage
-// could not be told apart from the first portion's, and portions run one by one.
+// could not be told apart from the first portion's, or the copies do not fit the memory, and portions run one by one.
 int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
   const mk_config &c = g->cfg;
   *ok = false;
@@ -2354,8 +2354,10 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
   size_t total = sizeof(int64_t) * MK_MAX_TOKENS;  // (the ids in front)
   for (const auto &e : rows.at) total += (e.second - e.first + 255) / 256 * 256;
   void *block;
-  const int rc = dev_alloc(g, &block, total, false);
-  if (rc) return rc;
+  if (dev_alloc(g, &block, total, false) != MK_OK) {
+    (void)hipGetLastError();
+    return MK_OK;
+  }
   void *ids = block;
   g->h_rt.ids2 = (long long *)ids;
   std::map<const char *, char *> copy;
@@ -3788,20 +3790,6 @@ int mk_compile(mk_graph *g) {
   rt.splitk_part = p;
   if ((rc = dev_alloc(g, &p, (size_t)g->G * 32 * sizeof(unsigned)))) return rc;
   rt.splitk_cnt = (unsigned *)p;
-  if (pairs) {
-    std::vector<MkStage> second;
-    bool ok;
-    if ((rc = second_stages(g, second, &ok))) return rc;
-    if (ok) {
-      if ((rc = dev_alloc(g, &p, sizeof(MkStage) * second.size(), false))) return rc;
-      HIP_TRY(hipMemcpy(p, second.data(), sizeof(MkStage) * second.size(), hipMemcpyHostToDevice));
-      rt.stages2 = (const MkStage *)p;
-      if ((rc = dev_alloc(g, &p, sizeof(unsigned) * g->pair_prog.size(), false))) return rc;
-      HIP_TRY(hipMemcpy(p, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
-      rt.pair_prog = (const unsigned *)p;
-      rt.pair_n = (int)g->pair_prog.size();
-    }
-  }
   g->timing_cap = 8192;
   if ((rc = dev_alloc(g, &p, sizeof(long long) * (g->timing_cap + 2)))) return rc;
   rt.timing = g->d_timing = (long long *)p;
@@ -3814,6 +3802,23 @@ int mk_compile(mk_graph *g) {
   rt.profiler_cap = g->profiler_cap;
   if ((rc = dev_alloc(g, &p, sizeof(MkRuntime)))) return rc;
   g->d_rt = (MkRuntime *)p;
+  if (pairs) {  // (behind all other memory that the graph needs: where this does not fit, portions run one by one)
+    std::vector<MkStage> second;
+    bool ok;
+    if ((rc = second_stages(g, second, &ok))) return rc;
+    if (ok) {
+      const size_t bytes = sizeof(MkStage) * second.size();
+      if (dev_alloc(g, &p, bytes + sizeof(unsigned) * g->pair_prog.size(), false) == MK_OK) {
+        HIP_TRY(hipMemcpy(p, second.data(), bytes, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy((char *)p + bytes, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
+        rt.stages2 = (const MkStage *)p;
+        rt.pair_prog = (const unsigned *)((char *)p + bytes);
+        rt.pair_n = (int)g->pair_prog.size();
+      } else {
+        (void)hipGetLastError();
+      }
+    }
+  }
   if ((rc = upload_runtime(g))) return rc;
   HIP_TRY(hipHostMalloc((void **)&g->h_status, sizeof(LaunchStatus)));
   memset(g->h_status, 0, sizeof(LaunchStatus));
