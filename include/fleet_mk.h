@@ -173,7 +173,7 @@ int mk_enqueue_ingest(mk_graph *g, void *stream);
 /* Batches that a launch fetches by itself, in the same modes: `host_words` (pinned host memory) has the ids and the index tensors of a
  * batch laid out as `device_words` has them, where the graph's tensors point; both hold `words` 32-bit words.  mk_enqueue_batch is
  * mk_enqueue_steps (or, with `ingest`, mk_enqueue_ingest) over the batch in the first `words` of them, and, without `ingest`, leaves the
- * sampled tokens in `host_tokens` (pinned, max_num_batched_tokens values; may be NULL).  The launch reads the words and writes the
+ * sampled tokens in `host_tokens` (pinned, max_num_batched_tokens values; may be NULL).  The launch reads the words (or, where they are many, a copy in front of it on the stream does) and writes the
  * tokens until mk_wait has returned; the memory belongs to the caller and must live until the handle is destroyed or another place is named.
  * host_words == NULL forgets it.  MK_EINVAL for memory of another kind. */
 int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens);

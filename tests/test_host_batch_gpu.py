@@ -55,6 +55,24 @@ def test_every_word_arrives_and_none_behind():
     s.finalize()
 
 
+@pytest.mark.parametrize("ingest", [False, True])
+def test_descriptions_that_are_copied(ingest):
+    """Long descriptions reach the device by a copy in front of the launch: the same words, on both sides of that line."""
+    cfg, s = _session(max_tokens=32 * 7000, max_requests=2, page_size=32, max_seq_length=64)
+    pk, n0 = s.mpk.persistent_kernel, 2 * s.max_rows + 4 * 2 + 2 + 1
+    want, _ = s.step([("a", [5])], [[0]])
+    g = torch.Generator().manual_seed(4)
+    for words in (7167, 7168, 7169, 14000):
+        s._host[n0:] = torch.randint(0, 1 << 30, s._host[n0:].shape, generator=g, dtype=torch.int32)
+        s._dev.fill_(-7)
+        s.logits().zero_()
+        (pk.enqueue_ingest(host_words=words) if ingest else pk.enqueue_batch(words))
+        pk.wait()
+        assert torch.equal(s._dev[:words].cpu(), s._host[:words]) and (s._dev[words:] == -7).all()
+        assert torch.equal(s.logits()[:1].float(), want) != ingest
+    s.finalize()
+
+
 def test_memory_of_another_kind_is_refused():
     cfg, s = _session(max_tokens=256, max_requests=2, max_seq_length=64)
     pk, host, dev, tokens = s.mpk.persistent_kernel, s._host, s._dev, s._sampled

@@ -88,6 +88,24 @@ def test_session(family):
         assert torch.isfinite(a).all() and torch.equal(a, b) and ga == gb
 
 
+def test_descriptions_that_are_copied():
+    """Both descriptions in front of the launch, where they are long (mk_set_host_batch's words by a copy), against fetched ones."""
+    from mirage.mpk import ServingSession
+    model, outs = _model("suborax"), []
+    toks = torch.randint(0, 1000, (300,), generator=torch.Generator().manual_seed(9)).tolist()
+    for whole in (False, True):
+        s = ServingSession.open(model_config=model, max_tokens=64 * 4000, max_requests=2, max_seq_length=512)
+        put, calls = s._put, []
+        if whole:
+            s._put = lambda at, ids, desc: put(at, ids, desc + [0] * (s._second - 2 * s.max_rows - len(desc)))
+        run = s.mpk.persistent_kernel.enqueue_batches
+        s.mpk.persistent_kernel.enqueue_batches = lambda *a, **k: (calls.append(a), run(*a, **k))
+        outs.append(s.step([("a", toks)], [[299]]))
+        assert len(calls) == 2 and all((a[0] + a[2] > 8000) == whole for a in calls)
+        s.finalize()
+    assert torch.equal(outs[0][0], outs[1][0]) and outs[0][1] == outs[1][1]
+
+
 def test_descriptions_that_do_not_fit():
     from mirage import _capi
     from mirage.mpk import ServingSession
