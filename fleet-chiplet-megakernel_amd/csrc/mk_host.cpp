@@ -154,13 +154,40 @@ struct LaunchStatus {
   unsigned xcd_count[MK_MAX_XCD];
   unsigned abort_flag, abort_where;
   long long t_begin, t_end;
+  int pair_ahead;  // the next launch of the offline scheduler begins with two portions in one iteration, by what its requests have left (mk_pair_ahead)
   MkSched sched;
 };
+// By the first wavefront of a workgroup.  Bound by three dependent round trips, 2 to 3 us.
+__device__ int launch_pair_ahead(const MkRuntime *rt) {
+  __shared__ int st[64], plen[64];
+  const int t = threadIdx.x, running = rt->sched->num_reqs, next = rt->sched->next_request_id;
+  const int n = min(rt->max_requests, running + rt->total_requests - next);
+  if (t < n) {
+    const bool has = t < running;
+    const int req = has ? rt->request_ids[t] : next + t - running;
+    st[t] = has ? rt->step[req] + rt->qo_indptr[t + 1] - rt->qo_indptr[t] : 0;  // (with the rows of the iteration that just ran)
+    plen[t] = rt->prompt_lengths[req];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return t == 0 && mk_pair_ahead(st, plen, running, n, rt->max_tokens, rt->max_new_per_req, rt->max_seq);
+}
+// When requests begin.  Prompts that are not there yet (lengths of zero) may be of any length.
+__global__ void mk_pair_ahead_kernel(const MkRuntime *rt, LaunchStatus *out) {
+  const int ahead = launch_pair_ahead(rt);
+  if (threadIdx.x == 0) out->pair_ahead = ahead || rt->prompt_lengths[0] <= 0;
+}
 // Runs behind every launch: one workgroup puts the outcome (and, for mk_enqueue_batch, the sampled tokens) in pinned host memory and leaves
 // the barrier state zeroed for the next launch.
 // (Bound by the launch; a memset in front and two pageable copies behind cost 12 + 2 x 13 us per launch on MI355X, this adds about 1.5.)
-__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out, const long long *tokens, int num_tokens, long long *host_tokens) {
+// `offline`: the graph's runtime, if its scheduler's launches may begin with two portions in one iteration.
+__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out, const long long *tokens, int num_tokens, long long *host_tokens, const MkRuntime *offline) {
   const unsigned t = threadIdx.x;
+  if (t < 64) {
+    const int ahead = offline && sched->inner && sched->num_reqs > 0 ? launch_pair_ahead(offline) : 0;
+    if (t == 0) out->pair_ahead = ahead;
+  }
   for (int i = (int)t; i < num_tokens; i += (int)blockDim.x) host_tokens[i] = tokens[i];
   if (t < MK_MAX_XCD) out->xcd_count[t] = sync->xcd_count[t][0];
   if (t == 32) out->abort_flag = sync->abort_flag;
@@ -230,7 +257,7 @@ struct mk_graph {
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
   int tail = 0;      // MkRuntime::tail
   bool requests_lost = false;  // a call failed behind the kernel that scheduled an iteration (mk_enqueue_parts): until the requests begin anew
-  bool inside_prompts = true;  // the last launch ended inside prompts, or none has been since the requests began
+  bool pair_ahead = true;    // LaunchStatus::pair_ahead of the last launch, or of the requests when they began
   int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
@@ -3243,10 +3270,10 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
   // Two portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions and the other kernel
-  // goes on; the launch begins with it unless the last one ended outside prompts (25 to 45 us of launch and handshake for nothing, and only speed is
-  // lost where the guess is wrong).
+  // goes on; a launch begins with it where the requests' prompts, as they were when the last one ended or the requests began, say that its first two
+  // portions fit (for nothing it is 25 to 45 us of launch and handshake; only speed is lost where prompts were changed since).
   const bool both = rt->batch2 > 0;
-  const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && max_iters > 2 && g->inside_prompts;
+  const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && max_iters > 2 && g->pair_ahead;
   const char *what = "";
   auto enqueue = [&](MkLaunchPart part) -> int {
     switch (part) {
@@ -3263,7 +3290,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
       default:
         what = "end of the launch";
         return launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status, (const long long *)rt->output_tokens,
-                             host_tokens ? rt->max_tokens : 0, host_tokens);
+                             host_tokens ? rt->max_tokens : 0, host_tokens, g->cfg.mode == MK_MODE_OFFLINE && rt->pair_n > 0 ? rtp : (const MkRuntime *)nullptr);
     }
   };
   auto undo = [&](bool lost) {
@@ -3298,7 +3325,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   g->last_aborted = hs.abort_flag != 0;
   g->last_ms = hs.abort_flag ? 0.0 : (hs.t_end - hs.t_begin) * 1e-5;
   const MkSched &sc = hs.sched;
-  g->inside_prompts = sc.inner != 0;
+  g->pair_ahead = hs.pair_ahead != 0;
   if (finished_out) *finished_out = sc.finished;
   if (hs.abort_flag) {
     // workgroups that unwound mid-stage may have left the split-K and split-KV arrival counters mid-count (their last
@@ -3850,8 +3877,12 @@ int mk_init_requests(mk_graph *g) {
   sc.page_queue_head = 0;
   sc.page_queue_tail = rt.max_pages;
   HIP_TRY(hipMemcpy(g->d_sched, &sc, sizeof(sc), hipMemcpyHostToDevice));
-  g->inside_prompts = true;
   g->requests_lost = false;
+  if (rt.pair_n > 0 && g->cfg.mode == MK_MODE_OFFLINE) {
+    HIP_TRY(launch_kernel(mk_pair_ahead_kernel, 1, 64, nullptr, (const MkRuntime *)g->d_rt, g->h_status));
+    HIP_TRY(hipStreamSynchronize(nullptr));
+    g->pair_ahead = g->h_status->pair_ahead != 0;
+  }
   HIP_TRY(hipMemset(rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
   HIP_TRY(hipMemset(rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));
   HIP_TRY(hipMemset(rt.profiler_count, 0, sizeof(unsigned) * (size_t)g->G));
