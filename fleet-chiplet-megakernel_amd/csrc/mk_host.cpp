@@ -2302,6 +2302,9 @@ std::vector<unsigned> pair_program(const mk_graph *g) {
       default: return false;
     }
   };
+  auto left_out = [&](const MkStage &s) {  // (by iterations in which nobody has several rows, or nothing was split)
+    return s.op == MK_OP_FX_PREP || s.op == MK_OP_DU_CONV || s.op == MK_OP_MX_LATENT_MERGE || s.op == MK_OP_MX_DELTA_OUT;
+  };
   std::vector<char> both(n, 0);
   for (int i = 0; i < n; i++) {
     MkStage s = g->stages[i];
@@ -2325,7 +2328,12 @@ std::vector<unsigned> pair_program(const mk_graph *g) {
     if (j == i + 1 && row_wise(g->stages[i])) {
       prog.push_back(i | MK_PAIR_ON);
     } else {
-      for (int q = i; q < j; q++) prog.push_back(q | (carries ? MK_PAIR_RELEASE : 0));
+      // One write-back of the caches is enough, behind the last of these stages that no iteration leaves out, or behind later ones that may write.
+      // (Each is 2 to 4 us.  Behind every stage, pairs were slower than their portions one by one where few linears run for both, us a pair: dodonex-2k
+      // + 53, vizonex-8b + 50, vizonex-2k + 63, bukatar-2k + 37; now - 7, - 15, - 14, - 21, and suborax-8b - 174 -> - 184, dodonex-8b - 37 -> - 93.)
+      int last = j - 1;
+      while (last >= i && left_out(g->stages[last])) last--;
+      for (int q = i; q < j; q++) prog.push_back(q | (carries && (q == last || (q > last && !passes(g->stages[q]))) ? MK_PAIR_RELEASE : 0));
       if (carries) prog.push_back(MK_PAIR_ACQUIRE);
     }
     for (int q = i; q < j; q++) prog.push_back(q | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));

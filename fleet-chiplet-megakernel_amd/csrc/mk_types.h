@@ -349,7 +349,7 @@ enum MkPairEntry {
   MK_PAIR_SECOND = 1 << 16,   // for the second portion
   MK_PAIR_BOTH = 1 << 17,
   MK_PAIR_ON = 1 << 18,       // the second portion's run of this stage follows without a barrier
-  MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written for the second portion to read: write back behind the stage ...
+  MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written, here or by the stages in front, for the second portion to read: write back ...
   MK_PAIR_ACQUIRE = 1 << 20,  // ... and, no stage, drop what the caches of the dies hold
   MK_PAIR_AGAIN = 1 << 21,    // the linear in front may have left its sum to this stage
 };

@@ -64,6 +64,72 @@ def _model(family):
     return generate.random_model(make(**sizes, layers={"suborax": 2, "dodonex": 4, "bukatar": 4, "vizonex": 4}[family], vocab=1000, **({"positions": 512} if family == "vizonex" else {})))[0]
 
 
+def _kept(builder):
+    """What the iterations of a layer-list model leave for later ones: caches, states and rings, and the batch slots' state slots."""
+    for name in ("k_cache", "v_cache", "latent_cache", "state", "tail", "canon", "state_slots"):
+        held = getattr(builder, name, None)
+        for t in held.values() if isinstance(held, dict) else held if isinstance(held, list) else [] if held is None else [held]:
+            yield t
+
+
+@pytest.mark.parametrize("family", ["suborax", "dodonex", "bukatar", "vizonex"])
+@pytest.mark.parametrize("lengths,R,portion,steps", [((64 * 4 + 7, 64 * 3), 1, 64, 100), ((200, 150, 33), 3, 30, 5), ((90,) * 40, 34, 64, 100)])
+def test_offline_families(family, lengths, R, portion, steps):
+    """The scheduler's pairs in the other kernels, and what goes on behind them: states that move between slots, scans, rings, experts; a batch
+    of more requests than a portion has rows for."""
+    import generate
+    model = _model(family)
+    g = torch.Generator().manual_seed(6)
+    prompts = [torch.randint(0, 1000, (n,), generator=g) for n in lengths]
+    max_seq, outs = max(lengths) + 6, []
+    for pairs in (True, False):
+        gen = generate.Generator(max_seq, model_config=model, batch=R, max_num_batched_tokens=64, max_tokens_per_request=portion, page_size=64, total_requests=len(lengths), eos_token_id=-1,
+                                 pair_portions=pairs)
+        assert gen.mpk.stats()["paired_portions"] == pairs
+        gen.load_prompts(prompts)
+        out, fin = [], False
+        while not fin:
+            fin = gen.mpk.run_steps(steps)
+            out += [gen.logits().clone(), torch.tensor(gen.mpk.stats()["iterations"])] + [v.clone() for k, v in gen.meta.items() if k != "input_tokens"]
+        kept = [t.clone() for t in _kept(gen.model.model_builder)]
+        out += kept
+        outs.append([t.cpu() for t in out])
+        gen.finalize()
+    assert kept and len(outs[0]) == len(outs[1]) and all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("entry", ["mk_enqueue_steps", "mk_enqueue_steps_static"])
+def test_in_a_callers_graph(entry):
+    """A captured launch that begins with pairs, replayed over prompts of other lengths (without any pair as well), the program's own work in between."""
+    import ctypes
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    from mirage import _capi
+    lib = _capi.load()
+    shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES["wide"])
+    w, gen = random_weights(shape, seed=2), torch.Generator().manual_seed(8)
+    decs = [Qwen3Decoder(shape, w, max_num_batched_tokens=64, max_num_batched_requests=2, max_seq_length=400, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=64, pair_portions=p)
+            for p in (True, False)]
+    draw = lambda lengths: [torch.randint(0, 512, (n,), generator=gen) for n in lengths]
+    decs[0].load_prompts(draw((300, 200)))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _capi.check(getattr(lib, entry)(decs[0].mpk._handle, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), 9))
+    _capi.check(lib.mk_wait(decs[0].mpk._handle, ctypes.c_void_p(0), None))
+    for lengths in ((300, 200), (20, 7), (390, 64), (129, 100)):
+        prompts, outs = draw(lengths), []
+        for dec in decs:
+            dec.k_cache.zero_()
+            dec.v_cache.zero_()
+            dec.load_prompts(prompts)
+            graph.replay() if dec is decs[0] else dec.mpk.run_steps(9)
+            torch.cuda.synchronize()
+            outs.append([t.clone() for t in (dec.logits()[:2], dec.meta["step"], dec.meta["tokens"], dec.k_cache, dec.v_cache)])
+            assert dec.mpk.stats()["aborted"] == 0 and dec.mpk.stats()["iterations"] == 9
+        assert all(torch.equal(a, b) for a, b in zip(*outs)), lengths
+    for dec in decs:
+        dec.mpk.finalize()
+
+
 @pytest.mark.parametrize("family", ["suborax", "dodonex", "bukatar", "vizonex"])
 def test_session(family):
     """Prompts of several requests, some of which begin or end inside a pair, then steps of one token each."""
