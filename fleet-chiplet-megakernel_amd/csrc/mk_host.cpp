@@ -154,11 +154,11 @@ struct LaunchStatus {
   unsigned xcd_count[MK_MAX_XCD];
   unsigned abort_flag, abort_where;
   long long t_begin, t_end;
-  int pair_ahead;  // the next launch of the offline scheduler begins with two portions in one iteration, by what its requests have left (mk_pair_ahead)
+  int pairs_ahead;  // the next launch of the offline scheduler begins with pairs of portions that pay for a kernel of their own (mk_pairs_ahead)
   MkSched sched;
 };
 // By the first wavefront of a workgroup.  Bound by three dependent round trips, 2 to 3 us.
-__device__ int launch_pair_ahead(const MkRuntime *rt) {
+__device__ int launch_pairs_ahead(const MkRuntime *rt, int need) {
   __shared__ int st[64], plen[64];
   const int t = threadIdx.x, running = rt->sched->num_reqs, next = rt->sched->next_request_id;
   const int n = min(rt->max_requests, running + rt->total_requests - next);
@@ -171,22 +171,22 @@ __device__ int launch_pair_ahead(const MkRuntime *rt) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  return t == 0 && mk_pair_ahead(st, plen, running, n, rt->max_tokens, rt->max_new_per_req, rt->max_seq);
+  return t == 0 && mk_pairs_ahead(st, plen, running, n, rt->max_tokens, rt->max_new_per_req, rt->max_seq, need);
 }
 // When requests begin.  Prompts that are not there yet (lengths of zero) may be of any length.
-__global__ void mk_pair_ahead_kernel(const MkRuntime *rt, LaunchStatus *out) {
-  const int ahead = launch_pair_ahead(rt);
-  if (threadIdx.x == 0) out->pair_ahead = ahead || rt->prompt_lengths[0] <= 0;
+__global__ void mk_pairs_ahead_kernel(const MkRuntime *rt, int need, LaunchStatus *out) {
+  const int ahead = launch_pairs_ahead(rt, need);
+  if (threadIdx.x == 0) out->pairs_ahead = ahead || rt->prompt_lengths[0] <= 0;
 }
 // Runs behind every launch: one workgroup puts the outcome (and, for mk_enqueue_batch, the sampled tokens) in pinned host memory and leaves
 // the barrier state zeroed for the next launch.
 // (Bound by the launch; a memset in front and two pageable copies behind cost 12 + 2 x 13 us per launch on MI355X, this adds about 1.5.)
-// `offline`: the graph's runtime, if its scheduler's launches may begin with two portions in one iteration.
-__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out, const long long *tokens, int num_tokens, long long *host_tokens, const MkRuntime *offline) {
+// `offline`: the graph's runtime, if its scheduler's launches may begin with `need` pairs of portions.
+__global__ void mk_launch_done_kernel(MkSync *sync, const MkSched *sched, LaunchStatus *out, const long long *tokens, int num_tokens, long long *host_tokens, const MkRuntime *offline, int need) {
   const unsigned t = threadIdx.x;
   if (t < 64) {
-    const int ahead = offline && sched->inner && sched->num_reqs > 0 ? launch_pair_ahead(offline) : 0;
-    if (t == 0) out->pair_ahead = ahead;
+    const int ahead = offline && sched->inner && sched->num_reqs > 0 ? launch_pairs_ahead(offline, need) : 0;
+    if (t == 0) out->pairs_ahead = ahead;
   }
   for (int i = (int)t; i < num_tokens; i += (int)blockDim.x) host_tokens[i] = tokens[i];
   if (t < MK_MAX_XCD) out->xcd_count[t] = sync->xcd_count[t][0];
@@ -257,7 +257,8 @@ struct mk_graph {
   int spec_len = 0;  // guesses per decoding request (set by a find_ngram_global task)
   int tail = 0;      // MkRuntime::tail
   bool requests_lost = false;  // a call failed behind the kernel that scheduled an iteration (mk_enqueue_parts): until the requests begin anew
-  bool pair_ahead = true;    // LaunchStatus::pair_ahead of the last launch, or of the requests when they began
+  bool pairs_ahead = true;   // LaunchStatus::pairs_ahead of the last launch, or of the requests when they began
+  int pairs_worth = 1;       // pairs of portions that pay for a kernel of their own (pair_program)
   int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
@@ -2282,7 +2283,13 @@ int tail_stage(const mk_graph *g) {
 // the first portion, then those of the second, as two iterations would run them.  What a cache or a state gets from the first portion is
 // written back and read anew in between; stages that only take rows to rows follow each other without a barrier where there is one of them.
 // Empty: the graph does not run portions that way.
-std::vector<unsigned> pair_program(const mk_graph *g) {
+//
+// *worth: pairs at the beginning of an offline launch that pay for the kernel they run in, which is 42 us of launch and handshake.  A pair gains, against its
+// portions one by one, about 8 us for every linear that runs for both and 0.05 us for every megabyte of their weights, and loses 7.5 where one portion
+// hands over to the other; expert linears of many tokens are 6 us faster in that kernel.  By that rule / measured, us a pair (25 portions of one
+// prompt, four layers): qwen3-8b 134 / 174, its width with 1536 columns 69 / 74, 2048 wide with 6144 columns and 2 / 6 kv heads 2 / 4 and 11 / 12, qwen3-30b-a3b
+// 90 / 96, suborax-8b 134 / 188, -2k 64 / 55, dodonex-8b 61 / 97, -2k 17 / 10, bukatar-8b 103 / 132, -2k 25 / 25, vizonex-8b 39 / 18, -2k 9 / 17.
+std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
   std::vector<unsigned> prog;
   const mk_config &c = g->cfg;
   const char *pack = getenv("FLEET_MK_PACK_WEIGHTS");
@@ -2339,6 +2346,15 @@ std::vector<unsigned> pair_program(const mk_graph *g) {
     for (int q = i; q < j; q++) prog.push_back(q | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
     i = j;
   }
+  double gain = 0;
+  for (const unsigned e : prog) {
+    const MkStage &s = g->stages[e & MK_PAIR_STAGE];
+    if (e & MK_PAIR_ACQUIRE) gain -= 7.5;
+    else if (e & MK_PAIR_BOTH) gain += 8 + 0.05e-6 * 2 * s.n * s.k;
+    else if (s.op == MK_OP_MOE_LINEAR) gain += 6;
+  }
+  *worth = gain > 0 ? (int)std::min(1e6, std::ceil(42 / gain)) : 1 << 20;
+  if (const char *given = getenv("FLEET_MK_PAIRS_WORTH")) *worth = std::max(1, atoi(given));
   return prog;
 }
 
@@ -2850,7 +2866,7 @@ int lower(mk_graph *g) {
     }
   }
   g->tail = tail_stage(g);
-  g->pair_prog = pair_program(g);
+  g->pair_prog = pair_program(g, &g->pairs_worth);
   g->program_text.clear();
   for (size_t s = 0; s < g->stage_desc.size(); s++) g->program_text += fmt("%3zu ", s) + g->stage_desc[s] + ((int)s < g->tail ? "\n" : " unread=skip\n");
   return MK_OK;
@@ -3278,10 +3294,10 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
   // Two portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions and the other kernel
-  // goes on; a launch begins with it where the requests' prompts, as they were when the last one ended or the requests began, say that its first two
-  // portions fit (for nothing it is 25 to 45 us of launch and handshake; only speed is lost where prompts were changed since).
+  // goes on; a launch begins with it where the requests' prompts, as they were when the last one ended or the requests began, say that enough pairs come
+  // first to pay for it (only speed is lost where prompts were changed since).
   const bool both = rt->batch2 > 0;
-  const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && max_iters > 2 && g->pair_ahead;
+  const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && g->pairs_ahead && (max_iters - 1) / 2 >= g->pairs_worth;
   const char *what = "";
   auto enqueue = [&](MkLaunchPart part) -> int {
     switch (part) {
@@ -3298,7 +3314,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
       default:
         what = "end of the launch";
         return launch_kernel(mk_launch_done_kernel, 1, 256, stream, rt->sync, (const MkSched *)g->d_sched, g->h_status, (const long long *)rt->output_tokens,
-                             host_tokens ? rt->max_tokens : 0, host_tokens, g->cfg.mode == MK_MODE_OFFLINE && rt->pair_n > 0 ? rtp : (const MkRuntime *)nullptr);
+                             host_tokens ? rt->max_tokens : 0, host_tokens, g->cfg.mode == MK_MODE_OFFLINE && rt->pair_n > 0 ? rtp : (const MkRuntime *)nullptr, g->pairs_worth);
     }
   };
   auto undo = [&](bool lost) {
@@ -3333,7 +3349,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
   g->last_aborted = hs.abort_flag != 0;
   g->last_ms = hs.abort_flag ? 0.0 : (hs.t_end - hs.t_begin) * 1e-5;
   const MkSched &sc = hs.sched;
-  g->pair_ahead = hs.pair_ahead != 0;
+  g->pairs_ahead = hs.pairs_ahead != 0;
   if (finished_out) *finished_out = sc.finished;
   if (hs.abort_flag) {
     // workgroups that unwound mid-stage may have left the split-K and split-KV arrival counters mid-count (their last
@@ -3887,9 +3903,9 @@ int mk_init_requests(mk_graph *g) {
   HIP_TRY(hipMemcpy(g->d_sched, &sc, sizeof(sc), hipMemcpyHostToDevice));
   g->requests_lost = false;
   if (rt.pair_n > 0 && g->cfg.mode == MK_MODE_OFFLINE) {
-    HIP_TRY(launch_kernel(mk_pair_ahead_kernel, 1, 64, nullptr, (const MkRuntime *)g->d_rt, g->h_status));
+    HIP_TRY(launch_kernel(mk_pairs_ahead_kernel, 1, 64, nullptr, (const MkRuntime *)g->d_rt, g->pairs_worth, g->h_status));
     HIP_TRY(hipStreamSynchronize(nullptr));
-    g->pair_ahead = g->h_status->pair_ahead != 0;
+    g->pairs_ahead = g->h_status->pairs_ahead != 0;
   }
   HIP_TRY(hipMemset(rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
   HIP_TRY(hipMemset(rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));

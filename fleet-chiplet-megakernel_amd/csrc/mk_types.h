@@ -354,29 +354,31 @@ enum MkPairEntry {
   MK_PAIR_AGAIN = 1 << 21,    // the linear in front may have left its sum to this stage
 };
 
-// Whether the next two iterations of the offline scheduler could run as one: the rule of its step (MK_PAIR_NEXT), for entries that have consumed st[i]
-// of plen[i] prompt tokens -- the first `running` have batch slots, those behind them wait, and no more than there are slots for are given.  B: rows of
-// an iteration, most: of one request in it.  st is overwritten.
-MK_HOST_DEVICE inline bool mk_pair_ahead(int *st, const int *plen, int running, int n, int B, int most, int max_seq) {
-  int rows = 0;
-  for (int i = 0; i < n; i++) {
-    if (i >= running && rows >= B) {
-      n = i;  // (not admitted yet)
-      break;
+// Whether the next iterations of the offline scheduler run as `need` pairs of portions: by the rule of its step (MK_PAIR_NEXT), for entries that have
+// consumed st[i] of plen[i] prompt tokens -- the first `running` have batch slots, those behind them wait, and no more than there are slots for are
+// given.  B: rows of an iteration, most: of one request in it.  st is overwritten.
+MK_HOST_DEVICE inline bool mk_pairs_ahead(int *st, const int *plen, int running, int n, int B, int most, int max_seq, int need) {
+  for (int pair = 0; pair < need; pair++) {
+    int rows = 0;
+    for (int i = 0; i < n && rows < B; i++) {
+      const bool waits = i >= running;
+      const int left = plen[i] - st[i], wish = left > 0 ? (left < most ? left : most) : (waits ? 0 : 1), take = wish < B - rows ? wish : B - rows;
+      if (st[i] + take >= plen[i] || st[i] + take + 1 >= max_seq) return false;
+      if (waits) running = i + 1;
+      st[i] += take;
+      rows += take;
     }
-    const int left = plen[i] - st[i], wish = left > 0 ? (left < most ? left : most) : (i < running ? 1 : 0), take = wish < B - rows ? wish : B - rows;
-    if ((take > 0 || i >= running) && (st[i] + take >= plen[i] || st[i] + take + 1 >= max_seq)) return false;
-    st[i] += take;
-    rows += take;
+    if (most <= 1 || 2 * rows <= B) return false;
+    rows = 0;
+    for (int i = 0; i < running && rows < B; i++) {
+      const int left = plen[i] - st[i], wish = left < most ? left : most, take = wish < B - rows ? wish : B - rows;
+      if (st[i] + take >= plen[i] || st[i] + take + 1 >= max_seq) return false;
+      st[i] += take;
+      rows += take;
+    }
+    if (rows < B) return false;
   }
-  if (most <= 1 || 2 * rows <= B) return false;
-  rows = 0;
-  for (int i = 0; i < n && rows < B; i++) {
-    const int left = plen[i] - st[i], wish = left < most ? left : most, take = wish < B - rows ? wish : B - rows;
-    if (st[i] + take >= plen[i] || st[i] + take + 1 >= max_seq) return false;
-    rows += take;
-  }
-  return rows >= B;
+  return true;
 }
 
 struct MkRuntime {

@@ -65,7 +65,9 @@ enum mk_mode { MK_MODE_OFFLINE = 0, MK_MODE_ONLINE = 1, MK_MODE_ONLINE_NOTOKEN =
  *  MK_CFG_PAIR_PORTIONS  the caller's word that no stage reads rows which the iteration it runs in has not written (token ids, caches and recurrent
  *      states apart): two portions inside prompts, which are iterations of their own otherwise, may then run as one that streams the weights
  *      once, the second over copies of the row buffers.  Results are the same bit by bit; iterations are counted, limited and timed as
- *      before, and the last one of a launch runs alone. */
+ *      before, and the last one of a launch runs alone.  Offline launches begin with such pairs where enough of them come first to pay for the
+ *      kernel they run in, by the prompt lengths at mk_init_requests (load them before) or what the last launch left; the environment
+ *      variable FLEET_MK_PAIRS_WORTH (read by mk_compile) names another number of pairs. */
 enum mk_config_flags { MK_CFG_SINGLE_WEIGHT_COPY = 1, MK_CFG_PAIR_PORTIONS = 2 };
 
 /* Constructor arguments of PersistentKernel (persistent_kernel.py:368-387) plus the
@@ -173,9 +175,9 @@ int mk_enqueue_ingest(mk_graph *g, void *stream);
 /* Batches that a launch fetches by itself, in the same modes: `host_words` (pinned host memory) has the ids and the index tensors of a
  * batch laid out as `device_words` has them, where the graph's tensors point; both hold `words` 32-bit words.  mk_enqueue_batch is
  * mk_enqueue_steps (or, with `ingest`, mk_enqueue_ingest) over the batch in the first `words` of them, and, without `ingest`, leaves the
- * sampled tokens in `host_tokens` (pinned, max_num_batched_tokens values; may be NULL).  The launch reads the words (or, where they are many, a copy in front of it on the stream does) and writes the
- * tokens until mk_wait has returned; the memory belongs to the caller and must live until the handle is destroyed or another place is named.
- * host_words == NULL forgets it.  MK_EINVAL for memory of another kind. */
+ * sampled tokens in `host_tokens` (pinned, max_num_batched_tokens values; may be NULL).  The launch reads the words (where they are many, a copy
+ * in front of it on the stream does) and writes the tokens until mk_wait has returned; the memory belongs to the caller and must live until
+ * the handle is destroyed or another place is named.  host_words == NULL forgets it.  MK_EINVAL for memory of another kind. */
 int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens);
 int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
 /* Two such batches as one launch, of which nobody reads logits or sampled tokens (mk_enqueue_ingest): the second, whose rows may continue the

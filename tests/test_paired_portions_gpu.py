@@ -5,6 +5,13 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def _any_pair(monkeypatch):
+    """Offline launches begin with pairs where there is one, however little these small models gain by it."""
+    monkeypatch.setenv("FLEET_MK_PAIRS_WORTH", "1")
+
+
 # linears that run for both portions at once: split in slices and left to the stage behind or summed by the last to arrive, whole, in ranges of
 # four to six tiles; and such that do not (reductions that are no multiple of 512 slices)
 SHAPES = {

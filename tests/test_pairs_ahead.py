@@ -1,4 +1,4 @@
-"""Whether a launch of the offline scheduler begins with two portions in one iteration (mk_pair_ahead), against the batches that the scheduler oracle forms."""
+"""Whether a launch of the offline scheduler begins with a given number of pairs of portions (mk_pairs_ahead), against the batches that the scheduler oracle forms."""
 import os
 import random
 import subprocess
@@ -9,12 +9,12 @@ SOURCE = r'''
 #include "mk_types.h"
 #include <stdio.h>
 int main() {
-  int running, n, B, most, max_seq;
-  while (scanf("%d %d %d %d %d", &running, &n, &B, &most, &max_seq) == 5) {
+  int running, n, B, most, max_seq, need;
+  while (scanf("%d %d %d %d %d %d", &running, &n, &B, &most, &max_seq, &need) == 6) {
     int st[64], plen[64];
     for (int i = 0; i < n; i++)
       if (scanf("%d %d", st + i, plen + i) != 2) return 1;
-    printf("%d", mk_pair_ahead(st, plen, running, n, B, most, max_seq));
+    printf("%d", mk_pairs_ahead(st, plen, running, n, B, most, max_seq, need));
   }
 }
 '''
@@ -37,8 +37,8 @@ def test_as_the_scheduler(tmp_path, seed):
     asked, want = [], []
     for _ in range(60):
         B, R, total = rng.choice([33, 40, 64]), rng.choice([1, 2, 3, rng.randint(1, 12)]), rng.randint(1, 8)
-        most, max_seq = rng.choice([9, 20, B, 64]), rng.randint(100, 420)
-        plens = [rng.randint(1, min(max_seq - 3, rng.choice([20, 90, 400]))) for _ in range(total)]
+        most, max_seq = rng.choice([9, 20, B, 64]), rng.randint(100, 620)
+        plens = [rng.randint(1, min(max_seq - 3, rng.choice([20, 90, 600]))) for _ in range(total)]
         its = _iterations(plens, R, B, most, max_seq)
         inside = lambda it: all(at + n < plens[r] and at + n + 1 < max_seq for r, at, n in it if n > 0)
         for i in range(len(its)):
@@ -47,10 +47,12 @@ def test_as_the_scheduler(tmp_path, seed):
             live = [(at + n, plens[r]) for r, at, n in its[i - 1]] if i else []
             first = max((r for it in its[:i] for r, _, _ in it), default=-1) + 1
             live_n, waiting = len(live), [(0, p) for p in plens[first:]][:max(0, R - len(live))]
-            asked.append(" ".join(map(str, (live_n, live_n + len(waiting), B, most, max_seq, *(x for e in live + waiting for x in e)))))
-            pair = its[i:i + 2]
-            want.append(len(pair) == 2 and all(map(inside, pair)) and [r for r, _, _ in pair[0]] == [r for r, _, _ in pair[1]]
-                        and 2 * sum(n for _, _, n in pair[0]) > B and sum(n for _, _, n in pair[1]) == B)
+            def pair(two):
+                return (len(two) == 2 and all(map(inside, two)) and [r for r, _, _ in two[0]] == [r for r, _, _ in two[1]]
+                        and 2 * sum(n for _, _, n in two[0]) > B and sum(n for _, _, n in two[1]) == B)
+            need = rng.choice([1, 1, 2, 3])
+            asked.append(" ".join(map(str, (live_n, live_n + len(waiting), B, most, max_seq, need, *(x for e in live + waiting for x in e)))))
+            want.append(all(pair(its[i + 2 * k:i + 2 * k + 2]) for k in range(need)))
     src = tmp_path / "ahead.cpp"
     src.write_text(SOURCE)
     exe = tmp_path / "ahead"
