@@ -54,8 +54,9 @@ class ServingSession:
     # two passes of which no row is wanted may be one launch (enqueue_batches): word the second one's description begins at, 0: not in this graph
     _second = 0
     _view = None  # of the logits
-    # 32-bit linears add in an order that depends on how many rows a pass has, and results are the same bit by bit whichever rows are wanted: there
-    # the rows that nobody reads stay where they are (16.2 ms for three prompts and their steps of a 2048-wide model, 15.7 with them in front)
+    # rows that nobody reads go into passes of their own, in front (see step).  Which rows share a pass decides in which order attention, experts and linears
+    # of few rows add, so that 16-bit results depend, in rounding, on the rows that are wanted; 32-bit sessions keep the rows in order, and their results
+    # are the same bit by bit whichever are wanted (16.2 ms for three prompts and their steps of a 2048-wide model, 15.7 with those rows in front)
     _unread_first = True
     _unread = False  # nobody reads the logits or the sampled tokens of the pass that runs
 
@@ -113,7 +114,11 @@ class ServingSession:
 
     def step(self, entries: Sequence[Tuple[object, Sequence[int]]], want: Sequence[Sequence[int]] = None):
         """Run `entries` = (request, its next tokens) as one batch.  Returns (logits, next tokens): float32 rows for the
-        wanted places (want[i] indexes entries[i]'s tokens) in order, or None, and the greedy token after each entry."""
+        wanted places (want[i] indexes entries[i]'s tokens) in order, or None, and the greedy token after each entry.
+
+        Tokens that do not fit one pass are spread over several, and how depends on `want`: in a 16-bit session the same tokens with other places
+        wanted give logits, caches and so perhaps greedy tokens that differ as two orders of the same sums do (relative 5e-3 measured, each as far from
+        64-bit results as the other); the same call gives the same bits.  A 32-bit session's results do not depend on `want`."""
         if len({rid for rid, _ in entries}) != len(entries):
             raise ValueError("a request may appear once in a step")
         want = want if want is not None else [[] for _ in entries]
@@ -124,23 +129,33 @@ class ServingSession:
         found = [dict.fromkeys(w) for w in want]  # place -> (logits of a run of rows, row of the run)
         greedy = [None] * len(entries)
         done = [0] * len(entries)
-        # single tokens first, so that they share their pass with the head of the longer portions
+        # shorter portions first, so that single tokens share their pass with the head of the longer ones
         order = sorted(range(len(entries)), key=lambda i: len(entries[i][1]))
 
         # places in front of the first one whose logits are wanted (the last one's greedy token always is): as long as they fill passes, passes
-        # are made of them alone, which are run without what only logits need, two at a time where the graph can
-        inner = [min([len(e[1]) - 1, *f]) for e, f in zip(entries, found)]
+        # are made of them alone, which are run without what only logits need, two at a time where the graph can.  A pass holds at most
+        # max_requests requests: where more have tokens left, or those there are cannot fill it, such passes would come on top of the others
+        # (64 entries of 3 tokens at 16 requests and 64 rows: seven passes instead of four)
+        whole = [len(e[1]) for e in entries]
+        inner = [min([n - 1, *f]) for n, f in zip(whole, found)]
 
-        def next_batch(done):
+        def fill(ends, done):
             batch, room = [], self.max_rows
-            ends = inner if self._unread_first and sum(max(0, h - d) for h, d in zip(inner, done)) >= room else [len(e[1]) for e in entries]
             for i in order:
                 n = min(ends[i] - done[i], self.rows_per_request, room)
                 if n > 0 and len(batch) < self.max_requests:
                     batch.append((i, n))
                     room -= n
+            return batch, room
+
+        def next_batch(done):
+            batch, room = [], 1
+            if self._unread_first and sum(max(0, h - d) for h, d in zip(inner, done)) >= self.max_rows and sum(d < n for n, d in zip(whole, done)) <= self.max_requests:
+                batch, room = fill(inner, done)
+            if room:
+                batch, _ = fill(whole, done)
             # (portions in the middle of their prompts, of which no row is wanted)
-            return batch, all(done[i] + n < len(entries[i][1]) and not any(done[i] <= p < done[i] + n for p in found[i]) for i, n in batch)
+            return batch, all(done[i] + n < whole[i] and not any(done[i] <= p < done[i] + n for p in found[i]) for i, n in batch)
 
         def tokens(batch, done):
             return [(entries[i][0], entries[i][1][done[i]:done[i] + n]) for i, n in batch]

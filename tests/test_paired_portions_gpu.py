@@ -161,6 +161,29 @@ def test_session(family):
         assert torch.isfinite(a).all() and torch.equal(a, b) and ga == gb
 
 
+@pytest.mark.parametrize("family", ["suborax", "bukatar"])
+def test_wanted_rows_and_rounding(family):
+    """Which rows are wanted decides which rows share a pass, and with that the order of sums: 16-bit logits differ by rounding at most.  (Sessions of these
+    families are 0.003 to 0.013 from 64-bit results, in 2-norms; two of them differ by no more than both together, 0.026.)"""
+    from mirage.mpk import ServingSession
+    model = _model(family)
+    g = torch.Generator().manual_seed(9)
+    prompts = [torch.randint(0, 1000, (n,), generator=g).tolist() for n in (300, 215, 170)]
+    last = []
+    for want in ([[len(p) - 1] for p in prompts], [list(range(len(p))) for p in prompts], [[0, len(p) - 1] for p in prompts]):
+        outs = []
+        for _ in range(2):
+            s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=1536, max_requests=3, max_seq_length=512)
+            out, _ = s.step(list(enumerate(prompts)), want)
+            ends = torch.tensor([len(w) for w in want]).cumsum(0) - 1
+            outs.append(out[ends.cuda()].double().cpu())
+            s.finalize()
+        assert torch.equal(*outs)
+        last.append(outs[0])
+    for other in last[1:]:
+        assert (other - last[0]).norm() / last[0].norm() < 0.026
+
+
 def test_descriptions_that_are_copied():
     """Both descriptions in front of the launch, where they are long (mk_set_host_batch's words by a copy), against fetched ones."""
     from mirage.mpk import ServingSession
