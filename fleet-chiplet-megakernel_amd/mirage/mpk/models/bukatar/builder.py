@@ -230,6 +230,7 @@ def random_state_dict(cfg: BukatarConfig, seed: int = 0, device="cuda", std: flo
 
 @register_model_builder("Bukatar")
 class BukatarBuilder(LayerListBuilder):
+    pair_portions = True
 
     def __init__(self, mpk: PersistentKernel, weights: Optional[dict] = None):
         super().__init__(mpk, weights)

@@ -178,6 +178,7 @@ def random_state_dict(cfg: DodonexConfig, seed: int = 0, device="cuda", std: flo
 @register_model_builder("Dodonex")
 class DodonexBuilder(GraphBuilder):
     owns_kv_cache = True
+    pair_portions = True
     dtypes = (torch.bfloat16, torch.float32)
 
     def __init__(self, mpk: PersistentKernel, weights: Optional[dict] = None):

@@ -44,6 +44,8 @@ class GraphBuilder(abc.ABC):
     default_eos_token_id = None  # used when neither the caller nor the checkpoint names one
     max_positions = None         # most positions of a sequence where the model itself bounds them
     dtypes = (torch.bfloat16,)   # activation / weight types the model can be built in
+    pair_portions = False        # True: no stage of this class's graphs reads rows its iteration has not written, token ids apart (see PersistentKernel);
+                                 # not inherited, as a subclass may add stages that do
 
     def __init__(self, mpk, weights: Optional[Dict[str, Any]] = None):
         self.mpk = mpk

@@ -108,6 +108,7 @@ def _pad64(n: int) -> int:
 @register_model_builder("Suborax")
 class SuboraxBuilder(GraphBuilder):
     owns_kv_cache = True
+    pair_portions = True
     dtypes = (torch.bfloat16, torch.float32)
 
     def __init__(self, mpk: PersistentKernel, weights: Optional[dict] = None):

@@ -195,6 +195,8 @@ def random_state_dict(cfg: VizonexConfig, seed: int = 0, device="cuda", std: flo
 
 @register_model_builder("Vizonex")
 class VizonexBuilder(LayerListBuilder):
+    pair_portions = True
+
     def __init__(self, mpk: PersistentKernel, weights: Optional[dict] = None):
         super().__init__(mpk, weights)
         self.k_cache, self.v_cache, self.state, self.tail, self.canon, self.state_slots = {}, {}, {}, {}, {}, None

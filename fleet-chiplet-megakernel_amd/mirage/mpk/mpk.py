@@ -72,7 +72,7 @@ class MPKMetadata:
     eos_token_id: Optional[int] = None
     max_tokens_per_request: Optional[int] = None
     single_weight_copy: Optional[bool] = None  # keep every linear weight once, in tile order (see PersistentKernel)
-    pair_portions: bool = True  # two portions inside prompts may run as one iteration (the builders' programs carry no rows from one to the next)
+    pair_portions: bool = True  # two portions inside prompts may run as one iteration, where the model's builder says so (GraphBuilder.pair_portions)
     dtype: torch.dtype = torch.bfloat16  # activations, weights and caches; the builder refuses what its model cannot run in
 
     def check_valid(self):
@@ -180,7 +180,7 @@ class MPK:
                 **({} if meta.state_slots_buffer is None else {"state_slots_buffer": meta.state_slots_buffer})},
             profiler_tensor=self.profiler_tensor, trace_name=meta.trace_name, spec_decode_config=meta.spec_decode_config,
             use_cutlass_kernel=False, eos_token_id=next(e for e in (meta.eos_token_id, builder_cls.default_eos_token_id, -1) if e is not None),
-            max_tokens_per_request=meta.max_tokens_per_request, single_weight_copy=meta.single_weight_copy, pair_portions=meta.pair_portions)
+            max_tokens_per_request=meta.max_tokens_per_request, single_weight_copy=meta.single_weight_copy, pair_portions=meta.pair_portions and bool(vars(builder_cls).get("pair_portions")))
         self.is_built = self.task_graph_generated = self.is_compiled = False
 
     def compensate_meta_tensors(self):

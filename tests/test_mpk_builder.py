@@ -294,3 +294,22 @@ def test_mpk_online_notoken_returns_normalised_hidden_state():
     cos = torch.nn.functional.cosine_similarity(h.flatten(), h64.flatten(), dim=0)
     assert float(cos) > 0.9999
     mpk.finalize()
+
+
+def test_whose_portions_run_in_pairs(monkeypatch):
+    """The shipped builders' graphs carry no rows from one iteration to the next and say so; what a caller registers says it itself or runs portions one by one."""
+    from mirage.mpk import MPK, mpk as module
+    from mirage.mpk.model_registry import _MODEL_BUILDERS, get_builder
+    from oracle.qwen3_ref import make_model_weights
+    made, cfg = [], _cfg()
+    real = module.PersistentKernel
+    monkeypatch.setattr(module, "PersistentKernel", lambda **kw: (made.append(kw["pair_portions"]), real(**kw))[1])
+    own = type("Own", (get_builder("Qwen3"),), {})
+    for name, cls, asked, want in (("Qwen3", get_builder("Qwen3"), True, True), ("Qwen3", get_builder("Qwen3"), False, False), ("Own", own, True, False),
+                                   ("Own", type("Word", (own,), {"pair_portions": True}), True, True)):
+        monkeypatch.setitem(_MODEL_BUILDERS, name, cls)
+        md = _metadata(cfg, make_model_weights(cfg, seed=61), "cpu", num_workers=256)
+        md.model_name, md.pair_portions = name, asked
+        MPK(md)
+        assert made[-1] is want, (name, asked)
+    assert all(vars(get_builder(n)).get("pair_portions") for n in ("Qwen3", "Suborax", "Dodonex", "Bukatar", "Vizonex"))
