@@ -108,9 +108,10 @@ class ServingSession:
     # ------------------------------------------------------------------ steps
     def logits(self) -> torch.Tensor:
         """Logits of the rows of the last pass (a view of the library's tensor)."""
-        if self._view is None:  # (making one takes 5 us)
-            self._view = self.mpk.model_builder.logits.to_torch()
-        return self._view
+        if self._view is None or self.mpk.persistent_kernel.__finalized__:  # (making one takes 5 us; of a finalized kernel's memory there is none to be had)
+            with torch.inference_mode(False):
+                self._view = self.mpk.model_builder.logits.to_torch()
+        return self._view.detach()  # (the caller's own: what it does to its shape stays with it)
 
     def step(self, entries: Sequence[Tuple[object, Sequence[int]]], want: Sequence[Sequence[int]] = None):
         """Run `entries` = (request, its next tokens) as one batch.  Returns (logits, next tokens): float32 rows for the

@@ -73,6 +73,24 @@ def test_descriptions_that_are_copied(ingest):
     s.finalize()
 
 
+def test_views_of_the_logits():
+    """A view per call, whatever mode the first one was asked for in and whatever became of an earlier one; none behind finalize()."""
+    cfg, s = _session(max_tokens=256, max_requests=2, max_seq_length=64)
+    with torch.inference_mode():
+        s.step([("a", [5])], [[0]])
+        s.logits()
+    view = s.logits()
+    assert not view.is_inference() and view.data_ptr() == s.logits().data_ptr()
+    shape = view.shape
+    view.unsqueeze_(0).requires_grad_()
+    assert s.logits().shape == shape and not s.logits().requires_grad
+    lg, _ = s.step([("a", [6])], [[0]])
+    assert torch.equal(lg, s.logits()[:1].float())
+    s.finalize()
+    with pytest.raises(RuntimeError):
+        s.logits()
+
+
 def test_memory_of_another_kind_is_refused():
     cfg, s = _session(max_tokens=256, max_requests=2, max_seq_length=64)
     pk, host, dev, tokens = s.mpk.persistent_kernel, s._host, s._dev, s._sampled
