@@ -90,7 +90,7 @@ typedef const __attribute__((address_space(4))) MkWeight CWeight;
 #define MK_HAVE_MIX 0
 #endif
 
-// kernels that run two portions inside prompts as one iteration, beside everything else
+// kernels that run iterations of two portions inside prompts, and nothing else
 #if defined(MK_KERNEL_DENSE_PAIR) || defined(MK_KERNEL_FLEX_PAIR) || defined(MK_KERNEL_MIX_PAIR) || defined(MK_KERNEL_HYB_PAIR) || defined(MK_KERNEL_DUAL_PAIR)
 #define MK_PAIR 1
 #else
@@ -748,7 +748,7 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // paged_kv_indices and paged_kv_last_page_len the way the reference's attention tasks read them -- request slot i owns
 // rows [qo_indptr[i], qo_indptr[i+1]) and its sequence, new tokens included, is (pages - 1) * page_size + last_page_len
 // long, so its rows sit at the last positions of that sequence.  Derives the per-row slot / position / first-row arrays
-// on the device (no host round trip, so a serving loop can enqueue launches back to back).  Runs on one thread.
+// on the device (no host round trip, so a serving loop can enqueue launches back to back).
 // Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).  Reads and
 // writes at device scope: mk_fetch_batch may have written the tensors a moment ago, and nobody releases behind the step.
 // `off`: words to the description, of the portion that runs beside the first one in the same iteration (0: the first one's); what is looked up by

@@ -304,8 +304,8 @@ MK_HOST_DEVICE inline MkLatentLds mk_latent_lds(int es, int rt, int nkc, int sub
   return l;
 }
 
-// Hierarchical barrier state.  256 bytes per counter: all workgroups poll all of them, and neighbours 128 bytes apart, two in 256 aligned ones,
-// took a decode step of 64 streams of qwen3-8b 0.7 % longer (257.5 -> 255.5 ms).
+// Hierarchical barrier state.  256 bytes per arrival counter: all workgroups poll all of them, and with neighbours 128 bytes apart, two in 256
+// aligned ones, a decode step of 64 streams of qwen3-8b took 0.7 % longer (257.5 -> 255.5 ms).  (The dies' workgroups are counted once a launch: a line each.)
 struct MkSync {
   unsigned local_ctr[MK_MAX_XCD][64];
   unsigned xcd_count[MK_MAX_XCD][32];  // workgroups of this launch on each die
@@ -414,9 +414,10 @@ struct MkRuntime {
   int *request_ids;   // [max_requests] request id per batch slot, -1 = free
   int *state_ids;     // [max_requests] recurrent-state slot per batch slot, a permutation (null: the graph has no recurrence)
   int *page_queue;    // [max_pages] ring of free page ids
-  int *tok_slot;      // [max_tokens] batch slot of each token of this iteration
-  int *tok_pos;       // [max_tokens] absolute position of each token
-  int *tok_first;     // [max_tokens] index of the first token of the same request in this iteration
+  // (two of each, MK_MAX_TOKENS apart: the second portion's rows lie behind the first one's, however many those are)
+  int *tok_slot;      // [2][MK_MAX_TOKENS] batch slot of each token of this iteration
+  int *tok_pos;       // [2][MK_MAX_TOKENS] absolute position of each token
+  int *tok_first;     // [2][MK_MAX_TOKENS] index of the first token of the same request in this iteration (of its portion)
   MkSched *sched;
   const MkStage *stages;
   MkSync *sync;
@@ -426,7 +427,8 @@ struct MkRuntime {
   float *argmax_pv;     // non-null: the sampling stages' per-workgroup partials live here ([workgroups][max_tokens] values / indices)
   int *argmax_pi;       // instead of in the buffers their descriptors name
   unsigned *attn_cnt;   // [max_tokens * num_kv_heads][32]: one 128-byte line per counter
-  void *splitk_part;    // [workgroups][4 wavefronts][4 weight tiles][4 token tiles][64 lanes] f32x4: K-slice partials of the split-K linear
+  void *splitk_part;    // 64 KB a workgroup, f32x4 K-slice partials of the split-K linear: [4 wavefronts][4 weight tiles][4 token tiles][64 lanes], for two
+                        // portions [2 wavefronts][4 weight tiles][8 token tiles][64 lanes]; or, left to the stage behind, [slice][16, 32, 64 or 128 rows][n]
   unsigned *splitk_cnt; // [workgroups][32]: arrival counter per split-K group (one 128-byte line each)
   long long *timing;    // [1 + timing_cap] wall-clock ticks (100 MHz) at the start of each iteration; [0] = kernel end
   int timing_cap;
