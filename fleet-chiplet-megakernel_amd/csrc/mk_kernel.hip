@@ -134,7 +134,7 @@ struct Ctx {
   int defer_ld_res;
 #if MK_PAIR
   const void *defer_res2;  // of the second portion
-  int rows_dealt;          // rows of the first portion that the running stage has dealt already
+  int rows_ahead;          // where the running stage has dealt the first portion's rows already: mk_rows_ahead of them
 #endif
 #if MK_HAVE_MIX
   bool mx_split;  // the latent attention (delta rule) that just ran left some request in chunks (its heads in slices)
@@ -923,7 +923,7 @@ __device__ __forceinline__ const u32x4 *weight_row(CWeight &w, int r, int k8) {
 // just dealt the first one's, go to the workgroups behind those.
 __device__ __forceinline__ int row_item(const Ctx &c, int t) {
 #if MK_PAIR
-  return mk_first_row(t, c.rows_dealt, c.G);
+  return mk_first_row(t, c.rows_ahead, c.G);
 #else
   return t;
 #endif
@@ -4994,11 +4994,11 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       }
       const long long t_out = (long long)wall_clock64();
 #if MK_PAIR
-      c.rows_dealt = 0;
+      c.rows_ahead = 0;
       if (ent & MK_PAIR_ON) {  // (as between two stages, but nobody waits for anybody)
         all_through = c.wrote_through;
         c.wrote_through = false;
-        c.rows_dealt = M1;
+        c.rows_ahead = mk_rows_ahead(M1, c.G);
         c.seq++;
         if (threadIdx.x == 0) c.sh_ticket[c.seq & 1] = 0;
         __syncthreads();
@@ -5065,7 +5065,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   c.st = nullptr;
   c.defer_S = 0;
 #if MK_PAIR
-  c.rows_dealt = 0;
+  c.rows_ahead = 0;
   c.defer_n = 0;
   c.defer_res2 = nullptr;
 #endif

@@ -280,14 +280,13 @@ MK_HOST_DEVICE inline XresPlan mk_xres_plan(Stage &st, int G) {
   return p;
 }
 
-// The first row of the workgroup that comes `at`-th of G in the order rows are dealt in (it takes every G-th one from there), where `dealt` rows of
-// another portion have been dealt just before: the rows go on from the workgroup behind the last of those, round and round (grids may be smaller than
-// a portion).
-MK_HOST_DEVICE inline int mk_first_row(int at, int dealt, int G) {
-  int t = at - dealt;
-  while (t < 0) t += G;
-  return t;
+// Rows are dealt to G workgroups in turn.  Where those of another portion have been dealt just before, they go on with the workgroup behind the last of
+// them: `ahead` workgroups further (grids may be smaller than a portion), and the first row of the workgroup that comes `at`-th is what mk_first_row says.
+MK_HOST_DEVICE inline int mk_rows_ahead(int dealt, int G) {
+  while (dealt >= G) dealt -= G;
+  return dealt;
 }
+MK_HOST_DEVICE inline int mk_first_row(int at, int ahead, int G) { return at >= ahead ? at - ahead : at - ahead + G; }
 
 // LDS map of MX_LATENT_ATTN, in bytes: query operands, one tile of cached rows, weights of the tile's positions, row statistics,
 // page-table entries.  RT: 16-row query tiles per unit; nkc: operand rows of a cached latent; sub: 16-position sub-tiles of a tile.

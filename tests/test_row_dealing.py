@@ -1,4 +1,4 @@
-"""Rows of a second portion are dealt to the workgroups behind those that took the first one's (mk_first_row, the same function as in the kernels)."""
+"""Rows of a second portion are dealt to the workgroups behind those that took the first one's (mk_rows_ahead and mk_first_row, the same functions as in the kernels)."""
 import os
 import subprocess
 
@@ -15,7 +15,7 @@ int main() {
       for (int M2 = 1; M2 <= MK_MAX_TOKENS; M2++) {
         int times[MK_MAX_TOKENS] = {}, behind = -1;
         for (int at = 0; at < G; at++) {
-          const int t0 = mk_first_row(at, M1, G);
+          const int t0 = mk_first_row(at, mk_rows_ahead(M1, G), G);
           if (t0 < 0 || t0 >= G) bad++;
           else if (t0 == 0) behind = at;
           for (int t = t0; t < M2; t += G) {
