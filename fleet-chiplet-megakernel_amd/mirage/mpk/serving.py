@@ -138,7 +138,8 @@ class ServingSession:
         # max_requests requests: where more have tokens left, or those there are cannot fill it, such passes would come on top of the others
         # (64 entries of 3 tokens at 16 requests and 64 rows: seven passes instead of four)
         whole = [len(e[1]) for e in entries]
-        inner = [min([n - 1, *f]) for n, f in zip(whole, found)]
+        ahead = self._unread_first and sum(whole) > self.max_rows
+        inner = [min([n - 1, *f]) for n, f in zip(whole, found)] if ahead else whole
 
         def fill(ends, done):
             batch, room = [], self.max_rows
@@ -151,7 +152,7 @@ class ServingSession:
 
         def next_batch(done):
             batch, room = [], 1
-            if self._unread_first and sum(max(0, h - d) for h, d in zip(inner, done)) >= self.max_rows and sum(d < n for n, d in zip(whole, done)) <= self.max_requests:
+            if ahead and sum(max(0, h - d) for h, d in zip(inner, done)) >= self.max_rows and sum(d < n for n, d in zip(whole, done)) <= self.max_requests:
                 batch, room = fill(inner, done)
             if room:
                 batch, _ = fill(whole, done)
