@@ -3323,6 +3323,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
     if (capture != hipStreamCaptureStatusNone) return;  // (nothing runs; what the capture holds is its owner's to drop)
     (void)hipStreamSynchronize(stream);
     (void)hipMemset(rt->sync, 0, sizeof(MkSync));
+    (void)hipStreamSynchronize(nullptr);  // (the next launch may be on a stream that does not wait for this one)
     (void)hipGetLastError();
     g->requests_lost = lost;
   };
