@@ -551,6 +551,14 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
   const int nkc = (D + KW - 1) / KW, nkg = (nkc + KC - 1) / KC, nvb = (DV + 15) / 16, nvs = (nvb + VB - 1) / VB;
   const int ps = rt.page_size;
   const u32x4 *kc = (const u32x4 *)st.k_cache, *vc = (const u32x4 *)st.v_cache;
+#if MK_PAIR
+  // (portions follow each other without a barrier: each has scratch of its own)
+  float *const part_base = rt.group_attn_part + (size_t)c.portion * rt.group_attn;
+  unsigned *const cnt_base = rt.group_attn_cnt + (size_t)c.portion * rt.group_cnt * 32;
+#else
+  float *const part_base = (float *)rt.attn_part;
+  unsigned *const cnt_base = rt.attn_cnt;
+#endif
   // LDS
   u32x4 *qs = (u32x4 *)smem;                                   // [nkg * KC][64] query operands
   E *kn = (E *)(smem + nkg * KC * 1024);                       // new key, padded with zeros to nkc * KW
@@ -936,7 +944,7 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
 #pragma unroll
         for (int w = 0; w < MK_WAVES; w++) fin[w * 16 + tid] *= inv;
       } else {
-        float *pb = (float *)rt.attn_part + ((size_t)u * 16 + tid) * PST + VB * 16;
+        float *pb = part_base + ((size_t)u * 16 + tid) * PST + VB * 16;
         stc_f32(pb, M_);
         stc_f32(pb + 1, L_);
       }
@@ -956,14 +964,14 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
 #pragma unroll
       for (int w = 0; w < MK_WAVES; w++) o += *(const f32x4 *)(part + (w * 16 + r) * PSTR + d) * fin[w * 16 + r];
       if (a.C == 1) emit(r, d, o);
-      else stc_16B((u32x4 *)((float *)rt.attn_part + ((size_t)u * 16 + r) * PST + d), __builtin_bit_cast(u32x4, o));
+      else stc_16B((u32x4 *)(part_base + ((size_t)u * 16 + r) * PST + d), __builtin_bit_cast(u32x4, o));
     }
     if (a.C == 1) continue;
     // ---- chunks: the last workgroup to arrive combines them
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-      unsigned *cnt = rt.attn_cnt + (size_t)a.item * 32;
+      unsigned *cnt = cnt_base + (size_t)a.item * 32;
       const int last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.C - 1);
       if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       *sflag = last;
@@ -972,7 +980,7 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
     if (!*sflag) continue;
     // Every thread weighs the chunks of its query row itself: maxima, sums and partial results of up to sixteen chunks are one round trip
     // (weights by way of LDS had made it two and three barriers).
-    const float *pb = (const float *)rt.attn_part + (size_t)a.item * cmax * 16 * PST;
+    const float *pb = part_base + (size_t)a.item * cmax * 16 * PST;
     constexpr int CB = 16;
     static_assert(MK_ATTN_MAX_CHUNKS <= 2 * CB, "at most two blocks of chunks");
     for (int i = tid; i < 16 * VB * 4; i += MK_THREADS) {

@@ -239,7 +239,9 @@ struct mk_graph {
   const int *batch_host = nullptr, *batch_src = nullptr;
   int *batch_dst = nullptr;
   long long *batch_tokens = nullptr;
-  int64_t batch_cap = 0;
+  int64_t batch_cap = 0, batch_more = 0;   // ... and how many go on behind them (mk_set_more_batches)
+  struct Held { int64_t at, words; };
+  std::vector<Held> held;                  // descriptions that the next mk_enqueue_held runs together
   bool launch_pending = false;
   LaunchStatus *h_status = nullptr;  // pinned host memory: what the last launch left (mk_launch_done_kernel)
   hipStream_t launch_stream = nullptr;
@@ -259,6 +261,7 @@ struct mk_graph {
   bool requests_lost = false;  // a call failed behind the kernel that scheduled an iteration (mk_enqueue_parts): until the requests begin anew
   bool pairs_ahead = true;   // LaunchStatus::pairs_ahead of the last launch, or of the requests when they began
   int pairs_worth = 1;       // pairs of portions that pay for a kernel of their own (pair_program)
+  size_t group_cnt_bytes = 0;  // of MkRuntime::group_attn_cnt
   int last_stages = 0;  // stages that the last iteration's batch was to run through (tail, or all)
   void *profiler_ptr = nullptr;  // the caller's profiler tensor (mk_set_profiler)
   long long profiler_cap = 0;
@@ -2279,9 +2282,10 @@ int tail_stage(const mk_graph *g) {
   return tail;
 }
 
-// Two portions inside prompts as one iteration (MkPairEntry): linears that run for both portions at once, and between two of them the stages of
-// the first portion, then those of the second, as two iterations would run them.  What a cache or a state gets from the first portion is
-// written back and read anew in between; stages that only take rows to rows follow each other without a barrier where there is one of them.
+// Several portions inside prompts as one iteration (MkPairEntry): linears that run for all portions at once, and between two of them the stages of
+// the first portion, then those of the second, and so on, as iterations of their own would run them.  What a cache or a state gets from a portion is
+// written back and read anew in front of the next one; stages that only take rows to rows run for one portion after the other without a barrier, and so do
+// stages that put keys and values into pages and, behind them all, the attention over those pages, which looks at no position behind a row's own.
 // Empty: the graph does not run portions that way.
 //
 // *worth: pairs at the beginning of an offline launch that pay for the kernel they run in, which is 42 us of launch and handshake.  A pair gains, against its
@@ -2317,9 +2321,10 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
     MkStage s = g->stages[i];
     both[i] = s.op == MK_OP_LINEAR && keeps_nothing(s) && (s.k & 63) == 0 && mk_xres_plan(s, g->G).S >= 1;
   }
-  // a sum left to the stage behind stays in the buffer that other split linears use, until the second portion has read it too
+  // what says where a sum is that was left to the stage behind says so of the last linear that left one, and is kept until all portions have read it: by a
+  // stage that runs for all of them at once, or with no other linear in between
   for (int i = n - 1; i >= 0; i--) {
-    if (!both[i] || !(g->stages[i].flags & MK_F_DEFER_SUM)) continue;
+    if (!both[i] || !(g->stages[i].flags & MK_F_DEFER_SUM) || (i + 1 < n && row_wise(g->stages[i + 1]))) continue;
     for (int j = i + 1; j < n && !both[j]; j++)
       if (g->stages[j].op == MK_OP_LINEAR) both[i] = 0;
   }
@@ -2330,27 +2335,55 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
       continue;
     }
     int j = i;
-    bool carries = false;
-    for (; j < n && !both[j]; j++) carries = carries || !passes(g->stages[j]);
-    if (j == i + 1 && row_wise(g->stages[i])) {
-      prog.push_back(i | MK_PAIR_ON);
-    } else {
+    while (j < n && !both[j]) j++;
+    // a run [q0, q1) for one portion after the other; the first stage of all may find a sum that the linear in front has left
+    auto in_turn = [&](int q0, int q1, bool on) {
+      bool carries = false;
+      for (int q = q0; q < q1; q++) carries = carries || !(on || passes(g->stages[q]));
       // One write-back of the caches is enough, behind the last of these stages that no iteration leaves out, or behind later ones that may write.
       // (Each is 2 to 4 us.  Behind every stage, pairs were slower than their portions one by one where few linears run for both, us a pair: dodonex-2k
       // + 53, vizonex-8b + 50, vizonex-2k + 63, bukatar-2k + 37; now - 7, - 15, - 14, - 21, and suborax-8b - 174 -> - 184, dodonex-8b - 37 -> - 93.)
-      int last = j - 1;
-      while (last >= i && left_out(g->stages[last])) last--;
-      for (int q = i; q < j; q++) prog.push_back(q | (carries && (q == last || (q > last && !passes(g->stages[q]))) ? MK_PAIR_RELEASE : 0));
+      int last = q1 - 1;
+      while (last >= q0 && left_out(g->stages[last])) last--;
+      auto entry = [&](int q) { return q | (on ? MK_PAIR_ON : 0) | (carries && (q == last || (q > last && !passes(g->stages[q]))) ? MK_PAIR_RELEASE : 0); };
+      for (int q = q0; q < q1; q++) prog.push_back(entry(q));
+      const size_t again = prog.size();
       if (carries) prog.push_back(MK_PAIR_ACQUIRE);
+      for (int q = q0; q < q1; q++) prog.push_back(entry(q) | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
+      prog.back() |= MK_PAIR_LOOP | (unsigned)(prog.size() - 1 - again) << MK_PAIR_BACK_SHIFT;
+    };
+    auto prepared = [&](int q) {  // attention over pages, all of whose new rows the stage in front has put there
+      const MkStage &s = g->stages[q];
+      return s.op == MK_OP_FX_ATTN && q > i && g->stages[q - 1].op == MK_OP_FX_PREP && g->stages[q - 1].k_cache == s.k_cache && g->stages[q - 1].v_cache == s.v_cache;
+    };
+    // (not a stage that may find a sum which a stage of the same run has left)
+    auto first = [&](int q) { return q == i || !(g->stages[q - 1].flags & MK_F_DEFER_SUM); };
+    auto attends = [&](int q) {  // attention that may run for all portions at once
+      const MkStage &s = g->stages[q];
+      return s.op == MK_OP_ATTN && first(q) && (s.num_q_heads == 4 * s.num_kv_heads || s.num_q_heads == 8 * s.num_kv_heads);
+    };
+    auto alone = [&](int q) { return first(q) && (row_wise(g->stages[q]) || prepared(q) || (q + 1 < j && prepared(q + 1))); };
+    for (int q = i; q < j;) {
+      int e = q + 1;
+      if (attends(q)) {
+        const size_t at = prog.size();
+        prog.push_back(q | MK_PAIR_BOTH);
+        in_turn(q, e, false);
+        prog[at] |= (unsigned)(prog.size() - at - 1) << MK_PAIR_BACK_SHIFT;
+      } else {
+        if (!alone(q))
+          while (e < j && !alone(e) && !attends(e)) e++;
+        in_turn(q, e, alone(q));
+      }
+      q = e;
     }
-    for (int q = i; q < j; q++) prog.push_back(q | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
     i = j;
   }
   double gain = 0;
   for (const unsigned e : prog) {
     const MkStage &s = g->stages[e & MK_PAIR_STAGE];
     if (e & MK_PAIR_ACQUIRE) gain -= 7.5;
-    else if (e & MK_PAIR_BOTH) gain += 8 + 0.05e-6 * 2 * s.n * s.k;
+    else if ((e & MK_PAIR_BOTH) && s.op == MK_OP_LINEAR) gain += 8 + 0.05e-6 * 2 * s.n * s.k;
     else if (s.op == MK_OP_MOE_LINEAR) gain += 6;
   }
   *worth = gain > 0 ? (int)std::min(1e6, std::ceil(42 / gain)) : 1 << 20;
@@ -2358,11 +2391,12 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
   return prog;
 }
 
-// The stages as they run for the second portion: over rows of its own, in copies of the memory that stages write rows to.  False: some stage
-// could not be told apart from the first portion's, or the copies do not fit the memory, and portions run one by one.
-int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
+// The stages as they run for the second portion and those behind it: over rows of their own, in copies of the memory that stages write rows to.  *portions:
+// as many run together at most, fewer where memory is short; 1: some stage could not be told apart from the first portion's, or not even one copy fits, and
+// portions run one by one.
+int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions) {
   const mk_config &c = g->cfg;
-  *ok = false;
+  *portions = 1;
   Extents held, rows;  // tensors and allocations; those among them that stages write rows to
   for (const Tensor &t : g->tensors) {
     if (!t.ptr || t.kind == T_SHUFFLED) continue;
@@ -2375,7 +2409,6 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
     auto it = e.at.upper_bound((const char *)p);
     return it != e.at.begin() && std::prev(it)->second > (const char *)p ? std::prev(it) : e.at.end();
   };
-  out.assign(g->stages.begin(), g->stages.end());
   for (int i = 0; i < g->tail; i++) {
     const MkStage &s = g->stages[i];
     const bool routed = s.op == MK_OP_HY_ROUTE || s.op == MK_OP_HY_EXPERTS;
@@ -2402,35 +2435,42 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, bool *ok) {
     if ((s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) && !(s.flags & MK_F_EMBED_FROM_TOKENS) && s.in != (const void *)c.input_tokens) return MK_OK;
     if ((s.flags & MK_F_GELU_TABLE) && s.aux0 != (const void *)c.input_tokens) return MK_OK;
   }
-  size_t total = sizeof(int64_t) * MK_MAX_TOKENS;  // (the ids in front)
-  for (const auto &e : rows.at) total += (e.second - e.first + 255) / 256 * 256;
-  void *block;
-  if (dev_alloc(g, &block, total, false) != MK_OK) {
+  size_t bytes = 0;
+  for (const auto &e : rows.at) bytes += (e.second - e.first + 255) / 256 * 256;
+  int P = MK_GROUP;
+  void *block = nullptr;
+  for (; P > 1; P /= 2) {  // (the ids in front)
+    if (dev_alloc(g, &block, (size_t)(P - 1) * (sizeof(int64_t) * MK_MAX_TOKENS + bytes), false) == MK_OK) break;
     (void)hipGetLastError();
-    return MK_OK;
   }
-  void *ids = block;
+  if (P < 2) return MK_OK;
+  int64_t *ids = (int64_t *)block;
   g->h_rt.ids2 = (long long *)ids;
-  std::map<const char *, char *> copy;
-  char *to = (char *)block + sizeof(int64_t) * MK_MAX_TOKENS;
-  for (const auto &e : rows.at) {
-    HIP_TRY(hipMemcpyAsync(to, e.first, e.second - e.first, hipMemcpyDeviceToDevice, nullptr));  // (padding that stages leave as it is)
-    copy[e.first] = to;
-    to += (e.second - e.first + 255) / 256 * 256;
+  char *to = (char *)(ids + (size_t)(P - 1) * MK_MAX_TOKENS);
+  out.clear();
+  for (int p = 1; p < P; p++, ids += MK_MAX_TOKENS) {
+    std::map<const char *, char *> copy;
+    for (const auto &e : rows.at) {
+      HIP_TRY(hipMemcpyAsync(to, e.first, e.second - e.first, hipMemcpyDeviceToDevice, nullptr));  // (padding that stages leave as it is)
+      copy[e.first] = to;
+      to += (e.second - e.first + 255) / 256 * 256;
+    }
+    auto moved = [&](auto &p) {
+      const auto it = p ? find(rows, p) : rows.at.end();
+      if (it != rows.at.end()) p = (std::remove_reference_t<decltype(p)>)(void *)(copy[it->first] + ((const char *)p - it->first));
+    };
+    const size_t first = out.size();
+    out.insert(out.end(), g->stages.begin(), g->stages.end());
+    for (int i = 0; i < g->tail; i++) {
+      MkStage &s = out[first + i];
+      moved(s.in); moved(s.out); moved(s.res); moved(s.norm_out); moved(s.q_ws); moved(s.moe_logits); moved(s.moe_topk_w); moved(s.moe_routing); moved(s.moe_mask);
+      moved(s.out2); moved(s.y_in); moved(s.in2); moved(s.glu_out); moved(s.slot_w); moved(s.ids); moved(s.in3); moved(s.y2); moved(s.out3);
+      if (s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) s.in = ids;
+      if (s.flags & MK_F_GELU_TABLE) s.aux0 = ids;
+    }
   }
   HIP_TRY(hipStreamSynchronize(nullptr));
-  auto moved = [&](auto &p) {
-    const auto it = p ? find(rows, p) : rows.at.end();
-    if (it != rows.at.end()) p = (std::remove_reference_t<decltype(p)>)(void *)(copy[it->first] + ((const char *)p - it->first));
-  };
-  for (int i = 0; i < g->tail; i++) {
-    MkStage &s = out[i];
-    moved(s.in); moved(s.out); moved(s.res); moved(s.norm_out); moved(s.q_ws); moved(s.moe_logits); moved(s.moe_topk_w); moved(s.moe_routing); moved(s.moe_mask);
-    moved(s.out2); moved(s.y_in); moved(s.in2); moved(s.glu_out); moved(s.slot_w); moved(s.ids); moved(s.in3); moved(s.y2); moved(s.out3);
-    if (s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) s.in = ids;
-    if (s.flags & MK_F_GELU_TABLE) s.aux0 = ids;
-  }
-  *ok = true;
+  *portions = P;
   return MK_OK;
 }
 
@@ -3296,7 +3336,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   // Two portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions and the other kernel
   // goes on; a launch begins with it where the requests' prompts, as they were when the last one ended or the requests began, say that enough pairs come
   // first to pay for it (only speed is lost where prompts were changed since).
-  const bool both = rt->batch2 > 0;
+  const bool both = rt->batch_n > 0;
   const bool first = run_scheduler == MK_SCHED_OFFLINE && rt->pair_n > 0 && !rt->profiler && g->pairs_ahead && (max_iters - 1) / 2 >= g->pairs_worth;
   const char *what = "";
   auto enqueue = [&](MkLaunchPart part) -> int {
@@ -3357,6 +3397,7 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
     // arriver resets them); the next launch on this handle must not inherit that
     HIP_TRY(hipMemset(g->h_rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
     HIP_TRY(hipMemset(g->h_rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));
+    if (g->group_cnt_bytes) HIP_TRY(hipMemset(g->h_rt.group_attn_cnt, 0, g->group_cnt_bytes));
     return fail(MK_EABORT, "kernel watchdog fired (barrier epoch %u): a workgroup waited longer than the spin limit", hs.abort_where);
   }
   if (sc.bad_batch) {
@@ -3747,11 +3788,11 @@ int mk_compile(mk_graph *g) {
   rt.request_ids = (int *)p;
   if ((rc = dev_alloc(g, &p, sizeof(int) * rt.max_pages))) return rc;
   rt.page_queue = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;  // (a second portion's behind the first one's)
+  if ((rc = dev_alloc(g, &p, sizeof(int) * MK_GROUP * MK_MAX_TOKENS))) return rc;  // (those of portions that run beside the first one behind its own)
   rt.tok_slot = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;
+  if ((rc = dev_alloc(g, &p, sizeof(int) * MK_GROUP * MK_MAX_TOKENS))) return rc;
   rt.tok_pos = (int *)p;
-  if ((rc = dev_alloc(g, &p, sizeof(int) * 2 * MK_MAX_TOKENS))) return rc;
+  if ((rc = dev_alloc(g, &p, sizeof(int) * MK_GROUP * MK_MAX_TOKENS))) return rc;
   rt.tok_first = (int *)p;
   if ((rc = dev_alloc(g, &p, sizeof(MkSched)))) return rc;
   rt.sched = g->d_sched = (MkSched *)p;
@@ -3856,19 +3897,42 @@ int mk_compile(mk_graph *g) {
   g->d_rt = (MkRuntime *)p;
   if (pairs) {  // (behind all other memory that the graph needs: where this does not fit, portions run one by one)
     std::vector<MkStage> second;
-    bool ok;
-    if ((rc = second_stages(g, second, &ok))) return rc;
-    if (ok) {
-      const size_t bytes = sizeof(MkStage) * second.size();
-      if (dev_alloc(g, &p, bytes + sizeof(unsigned) * g->pair_prog.size(), false) == MK_OK) {
-        HIP_TRY(hipMemcpy(p, second.data(), bytes, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy((char *)p + bytes, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
-        rt.stages2 = (const MkStage *)p;
-        rt.pair_prog = (const unsigned *)((char *)p + bytes);
-        rt.pair_n = (int)g->pair_prog.size();
-      } else {
-        (void)hipGetLastError();
+    int portions;
+    if ((rc = second_stages(g, second, &portions))) return rc;
+    while (portions > 1) {
+      const size_t bytes = sizeof(MkStage) * (portions - 1) * g->stages.size(), prog = align256(sizeof(unsigned) * g->pair_prog.size());
+      size_t part = 0;  // floats of partial sums
+      int heads = 0;    // of queries prepared ahead of the attention
+      for (const unsigned e : g->pair_prog) {
+        if (!(e & MK_PAIR_BOTH)) continue;
+        MkStage &s = g->stages[e & MK_PAIR_STAGE];
+        if (s.op == MK_OP_ATTN) heads = std::max(heads, s.num_q_heads);
+        if (s.op != MK_OP_LINEAR) continue;
+        const XresPlan plan = mk_xres_plan(s, g->G);
+        if (plan.S > 1) part = std::max(part, (size_t)plan.S * portions * MK_MAX_TOKENS * std::max(plan.wt * 16, s.n));
       }
+      const size_t attn = align256(g->flex_part * sizeof(float)), items = g->flex_items;
+      const size_t at_prog = align256(bytes), at_part = at_prog + prog, at_attn = at_part + align256(part * sizeof(float)), at_q = at_attn + portions * attn, at_cnt = at_q + align256((size_t)portions * MK_MAX_TOKENS * heads * 256),
+                   cnt = portions * items * 32 * sizeof(unsigned);
+      if (dev_alloc(g, &p, at_cnt + cnt, false) != MK_OK) {
+        (void)hipGetLastError();
+        portions /= 2;
+        continue;
+      }
+      HIP_TRY(hipMemcpy(p, second.data(), bytes, hipMemcpyHostToDevice));
+      HIP_TRY(hipMemcpy((char *)p + at_prog, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
+      rt.stages2 = (const MkStage *)p;
+      rt.pair_prog = (const unsigned *)((char *)p + at_prog);
+      rt.group_part = (float *)((char *)p + at_part);
+      rt.group_q = (uint16_t *)((char *)p + at_q);
+      rt.group_attn_part = (float *)((char *)p + at_attn);
+      rt.group_attn = (long long)(attn / sizeof(float));
+      rt.group_attn_cnt = (unsigned *)((char *)p + at_cnt);
+      rt.group_cnt = (long long)items;
+      g->group_cnt_bytes = cnt;
+      rt.pair_n = (int)g->pair_prog.size();
+      rt.group = portions;
+      break;
     }
   }
   if ((rc = upload_runtime(g))) return rc;
@@ -3910,6 +3974,7 @@ int mk_init_requests(mk_graph *g) {
   }
   HIP_TRY(hipMemset(rt.attn_cnt, 0, sizeof(unsigned) * g->attn_cnt_n));
   HIP_TRY(hipMemset(rt.splitk_cnt, 0, sizeof(unsigned) * 32 * (size_t)g->G));
+  if (g->group_cnt_bytes) HIP_TRY(hipMemset(rt.group_attn_cnt, 0, g->group_cnt_bytes));
   HIP_TRY(hipMemset(rt.profiler_count, 0, sizeof(unsigned) * (size_t)g->G));
   if (rt.profiler) HIP_TRY(hipMemset(rt.profiler, 0, sizeof(unsigned long long) * (size_t)rt.profiler_cap));
   return MK_OK;
@@ -3963,7 +4028,8 @@ int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_wo
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending");
   if (g->cfg.mode == MK_MODE_OFFLINE || g->cfg.mode == MK_MODE_ONLINE) return fail(MK_EINVAL, "the host describes batches in the modes online_notoken and onepass");
-  g->batch_cap = 0;
+  g->batch_cap = g->batch_more = 0;
+  g->held.clear();
   if (!host_words) return MK_OK;
   if (!device_words || words < 1 || words > (1ll << 28)) return fail(MK_EINVAL, "a batch in host memory needs device memory of as many words");
   if (((uintptr_t)host_words | (uintptr_t)device_words) & 3) return fail(MK_EINVAL, "words of a batch lie on four bytes");
@@ -3983,19 +4049,10 @@ int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_wo
 // and what the copy costs hardly grows with them.  A pass, fetched / copied, us: 139 words 123.4 / 135.8, 4096 126.7 / 134.7, 6144 129.1 / 131.0, 7168
 // 131.0 / 131.1, 8192 132.0 / 131.3, 12288 137.2 / 132.2, 65536 206.6 / 140.1.
 #define MK_FETCH_WORDS 7168
-static int bring_batch(mk_graph *g, hipStream_t stream, MkRuntime &rt, int64_t words, int64_t second, int64_t words2) {
-  rt.batch_src = g->batch_src;
-  rt.batch_dst = g->batch_dst;
-  rt.batch2 = (int)second;
-  if (words + words2 <= MK_FETCH_WORDS) {
-    rt.batch_words = words;
-    rt.batch_words2 = words2;
-    return MK_OK;
-  }
+static int copy_batch(mk_graph *g, hipStream_t stream, int64_t at, int64_t words) {
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending: call mk_wait first");  // (and may still read the words there)
   HIP_TRY(hipSetDevice(g->cfg.device));
-  HIP_TRY(hipMemcpyAsync(g->batch_dst, g->batch_host, 4 * (size_t)words, hipMemcpyHostToDevice, stream));
-  if (second) HIP_TRY(hipMemcpyAsync(g->batch_dst + second, g->batch_host + second, 4 * (size_t)words2, hipMemcpyHostToDevice, stream));
+  HIP_TRY(hipMemcpyAsync(g->batch_dst + at, g->batch_host + at, 4 * (size_t)words, hipMemcpyHostToDevice, stream));
   return MK_OK;
 }
 
@@ -4004,26 +4061,82 @@ int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest) {
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (words < 1 || words > g->batch_cap) return fail(MK_EINVAL, "batch of %lld words, mk_set_host_batch named %lld", (long long)words, (long long)g->batch_cap);
   MkRuntime rt = g->h_rt;
-  if (const int rc = bring_batch(g, (hipStream_t)stream, rt, words, 0, 0)) return rc;
+  rt.batch_src = g->batch_src;
+  rt.batch_dst = g->batch_dst;
+  if (words <= MK_FETCH_WORDS) rt.batch_words = words;
+  else if (const int rc = copy_batch(g, (hipStream_t)stream, 0, words)) return rc;
   return do_launch(g, (hipStream_t)stream, 1, ingest ? MK_SCHED_INGEST : MK_SCHED_FROM_META, &rt, ingest ? nullptr : g->batch_tokens);
 }
 
-int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2) {
+// Two descriptions, from word `at` and `at + second` on.
+static int check_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2) {
   if (!g) return fail(MK_EINVAL, "null argument");
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (!g->h_rt.pair_n || g->h_rt.profiler) return fail(MK_EUNSUPPORTED, "this graph runs portions of prompts one by one");
-  if (words < 1 || words2 < 1 || second < words || second + words2 > g->batch_cap || (second & 1))
-    return fail(MK_EINVAL, "batches of %lld words and of %lld from word %lld on, mk_set_host_batch named %lld", (long long)words, (long long)words2, (long long)second, (long long)g->batch_cap);
-  // the second description is read `second` words behind every tensor of the first one: all of that is in the named words
-  auto named = [&](const void *p, size_t bytes) { return !p || ((const char *)p >= (const char *)g->batch_dst && (const char *)p + 4 * second + bytes <= (const char *)(g->batch_dst + g->batch_cap)); };
+  const int64_t cap = g->batch_cap + (at ? g->batch_more : 0);
+  if (words < 1 || words2 < 1 || second < words || at < 0 || at + second + words2 > cap || ((second | at) & 1))
+    return fail(MK_EINVAL, "batches of %lld words from word %lld and of %lld from word %lld on, mk_set_host_batch named %lld", (long long)words, (long long)at, (long long)words2,
+                (long long)(at + second), (long long)cap);
+  // the descriptions are read `at` and `at + second` words behind every tensor of the graph: all of that is in the named words
+  auto named = [&](const void *p, size_t bytes) { return !p || ((const char *)p >= (const char *)g->batch_dst && (const char *)p + 4 * (at + second) + bytes <= (const char *)(g->batch_dst + cap)); };
   const mk_config &c = g->cfg;
   const size_t R = (size_t)c.max_num_batched_requests;
   if (!named(c.input_tokens, 8 * (size_t)c.max_num_batched_tokens) || !named(c.qo_indptr, 4 * (R + 1)) || !named(c.paged_kv_indptr, 4 * (R + 1)) || !named(c.paged_kv_last_page_len, 4 * R) ||
       !named(c.paged_kv_indices, 4 * (size_t)c.max_num_pages) || !named(g->state_ids, 4 * R))
-    return fail(MK_EINVAL, "two batches in one launch need the ids and all index tensors, and as much again from word %lld on, in the device words that mk_set_host_batch named", (long long)second);
+    return fail(MK_EINVAL, "several batches in one launch need the ids and all index tensors, and as much again from word %lld on, in the device words that mk_set_host_batch named", (long long)(at + second));
+  return MK_OK;
+}
+static int launch_batches(mk_graph *g, hipStream_t stream, const mk_graph::Held *b, int n) {
   MkRuntime rt = g->h_rt;
-  if (const int rc = bring_batch(g, (hipStream_t)stream, rt, words, second, words2)) return rc;
-  return do_launch(g, (hipStream_t)stream, 1, MK_SCHED_INGEST, &rt);
+  rt.batch_src = g->batch_src;
+  rt.batch_dst = g->batch_dst;
+  rt.batch_n = n;
+  int64_t most = 0;
+  for (int p = 0; p < n; p += 2) most = std::max(most, b[p].words + b[p + 1].words);
+  for (int p = 0; p < n; p++) {
+    rt.batch_at[p] = (int)b[p].at;
+    rt.batch_len[p] = most <= MK_FETCH_WORDS ? (int)b[p].words : 0;
+    if (most > MK_FETCH_WORDS)
+      if (const int rc = copy_batch(g, stream, b[p].at, b[p].words)) return rc;
+  }
+  return do_launch(g, stream, 1, MK_SCHED_INGEST, &rt);
+}
+
+int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2) {
+  if (const int rc = check_batches(g, 0, words, second, words2)) return rc;
+  const mk_graph::Held b[2] = {{0, words}, {second, words2}};
+  return launch_batches(g, (hipStream_t)stream, b, 2);
+}
+
+int mk_set_more_batches(mk_graph *g, int64_t words) {
+  if (!g) return fail(MK_EINVAL, "null argument");
+  if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending");
+  if (!g->batch_cap || words < 0 || g->batch_cap + words > (1ll << 28)) return fail(MK_EINVAL, "%lld words behind those that mk_set_host_batch named (%lld)", (long long)words, (long long)g->batch_cap);
+  HIP_TRY(hipSetDevice(g->cfg.device));
+  const size_t bytes = 4 * (size_t)(g->batch_cap + words);
+  if (device_view(g->batch_host, bytes, hipMemoryTypeHost, g->cfg.device) != (void *)g->batch_src || device_view(g->batch_dst, bytes, hipMemoryTypeDevice, g->cfg.device) != (void *)g->batch_dst)
+    return fail(MK_EINVAL, "batch words are in pinned host memory, their place in the graph's device's memory, all in one piece");
+  g->batch_more = words;
+  g->held.clear();
+  return MK_OK;
+}
+
+int mk_hold_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2) {
+  if (const int rc = check_batches(g, at, words, second, words2)) return rc;
+  if (g->held.empty() != (at == 0)) return fail(MK_EINVAL, "the first batches are described from word 0 on, others behind them");
+  if ((int)g->held.size() + 2 > g->h_rt.group) return fail(MK_EINVAL, "this graph runs %d batches together at most (mk_stats.portions_together)", g->h_rt.group);
+  g->held.push_back({at, words});
+  g->held.push_back({at + second, words2});
+  return MK_OK;
+}
+
+int mk_enqueue_held(mk_graph *g, void *stream) {
+  if (!g) return fail(MK_EINVAL, "null argument");
+  if (g->held.empty()) return fail(MK_ESTATE, "no batches are held: call mk_hold_batches first");
+  if (g->h_rt.profiler) return fail(MK_EUNSUPPORTED, "this graph runs portions of prompts one by one");
+  std::vector<mk_graph::Held> b;
+  b.swap(g->held);
+  return launch_batches(g, (hipStream_t)stream, b.data(), (int)b.size());
 }
 
 int mk_enqueue_steps_static(mk_graph *g, void *stream, int max_iterations) {
@@ -4119,6 +4232,7 @@ int mk_get_stats(mk_graph *g, mk_stats *out) {
   out->row_major_weight_bytes = g->row_major_bytes;
   out->last_launch_ms = g->last_ms;
   out->paired_portions = g->h_rt.pair_n > 0;
+  out->portions_together = g->h_rt.pair_n > 0 ? g->h_rt.group : 1;
   if (g->compiled && !g->launch_pending) {
     MkSched sc;
     HIP_TRY(hipMemcpy(&sc, g->d_sched, sizeof(sc), hipMemcpyDeviceToHost));

@@ -133,8 +133,9 @@ struct Ctx {
   const void *defer_res;  // residual rows of that linear (null: none)
   int defer_ld_res;
 #if MK_PAIR
-  const void *defer_res2;  // of the second portion
-  int rows_ahead;          // where the running stage has dealt the first portion's rows already: mk_rows_ahead of them
+  int defer_stage;         // the linear itself (its residual rows are each portion's own)
+  int rows_ahead;          // where the running stage has dealt rows of portions in front already: mk_rows_ahead of them
+  int portion;             // that the running stage runs for
 #endif
 #if MK_HAVE_MIX
   bool mx_split;  // the latent attention (delta rule) that just ran left some request in chunks (its heads in slices)
@@ -572,11 +573,11 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 }
 __device__ __forceinline__ int wave_bcast(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
 
-// `half` 1: the portion that runs beside the one just prepared, in the same iteration (MK_PAIR_NEXT in the result of the step that prepared that).
+// `portion` > 0: one that runs beside those just prepared, in the same iteration (MK_PAIR_NEXT in the result of the step that prepared the last of them).
 #define MK_PAIR_NEXT (1 << 16)
-__device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRuntime &rt, int *lds, int lane, int half) {
-  const int second = MK_PAIR ? half * MK_MAX_TOKENS : 0;
-  long long *const ids = second ? rt.ids2 : rt.input_tokens;
+__device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRuntime &rt, int *lds, int lane, int portion) {
+  const int second = MK_PAIR ? portion * MK_MAX_TOKENS : 0;
+  long long *const ids = second ? rt.ids2 + second - MK_MAX_TOKENS : rt.input_tokens;
   MkSched *sc = rt.sched;
   const int R = rt.max_requests, B = rt.max_tokens, PS = rt.page_size, NP = rt.max_pages;
   int *snap = lds, *freed = lds + NP;
@@ -708,7 +709,7 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
       for (int j = 0; j < cneed; j++) rt.kv_indices[page0 + j] = ring_page(a0 + j);
     }
     rows(cn, ntok + cw_incl - cwish, cand, 0, nreq + lane);
-    if (MK_PAIR && !half && rt.pair_n) {
+    if (MK_PAIR && rt.pair_n) {
       const int w1 = alive ? min(plen - st - n, rt.max_new_per_req) : 0, i1 = wave_incl_scan(w1, lane), s1 = wave_bcast(i1, 63);
       const int w2 = admit ? min(cplen - cn, rt.max_new_per_req) : 0, i2 = s1 + wave_incl_scan(w2, lane);
       const int n1 = min(i1, B) - min(i1 - w1, B), n2 = min(i2, B) - min(i2 - w2, B);
@@ -731,11 +732,9 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
   if (lane == 0) {
     sc->page_queue_head = head0 + taken;
     sc->page_queue_tail = tail0 + n_freed;
-    if (second) {
-      sc->num_tokens2 = ntok;
-    } else {
+    if (MK_PAIR) sc->group[portion] = ntok;
+    if (!second) {
       sc->num_tokens = ntok;
-      sc->num_tokens2 = 0;
       sc->inner = inner;
     }
     sc->num_reqs = nreq;
@@ -751,10 +750,10 @@ __device__ __attribute__((noinline)) int mk_prepare_next_batch_wave(const MkRunt
 // on the device (no host round trip, so a serving loop can enqueue launches back to back).
 // Runs on a wavefront, a lane per batch slot, so that the slots' loads overlap (one thread took one to two microseconds per slot).  Reads and
 // writes at device scope: mk_fetch_batch may have written the tensors a moment ago, and nobody releases behind the step.
-// `off`: words to the description, of the portion that runs beside the first one in the same iteration (0: the first one's); what is looked up by
-// slot lies there as well.
-__device__ __forceinline__ int mk_batch_from_meta(const MkRuntime &rt, int lane, int off, bool pair) {
-  const int R = rt.max_requests, B = rt.max_tokens, second = MK_PAIR && off ? MK_MAX_TOKENS : 0;
+// `off`: words to the description of a portion that runs beside the first one in the same iteration (0: the first one's); what is looked up by
+// slot lies there as well.  `several`: there are such portions, this one being the `portion`-th.
+__device__ __forceinline__ int mk_batch_from_meta(const MkRuntime &rt, int lane, int off, bool several, int portion) {
+  const int R = rt.max_requests, B = rt.max_tokens, second = MK_PAIR ? portion * MK_MAX_TOKENS : 0;
   // A batch the stages cannot run as described is not run at all: truncating a request's rows would leave the rest with
   // the slot / position an earlier launch gave them, and they would append K/V rows to some other request's cache.
   // bad, of the first slot that cannot run: 1 = rows outside [0, max tokens), overlapping, or with gaps; 2 = more rows for one
@@ -783,7 +782,7 @@ __device__ __forceinline__ int mk_batch_from_meta(const MkRuntime &rt, int lane,
   const unsigned long long covered = (unsigned long long)(unsigned)wave_bcast((int)lo, 63) | ((unsigned long long)(unsigned)wave_bcast((int)hi, 63) << 32);
   int ntok = covered ? 64 - __clzll((long long)covered) : 0;
   if (covered != (ntok >= 64 ? ~0ull : ((1ull << ntok) - 1ull)) && !bad) bad = 1;
-  if (pair && ntok < 3 && !bad) bad = 4;
+  if (several && ntok < 3 && !bad) bad = 4;
   if (bad) ntok = 0;
   // a lane per row (by the lanes of the slots, row after row, 64 rows of one request took 16 us)
   int slot = 0, first = 0, pos = 0;
@@ -799,17 +798,16 @@ __device__ __forceinline__ int mk_batch_from_meta(const MkRuntime &rt, int lane,
     stc_i32(rt.tok_slot + second + lane, off + slot);
     stc_i32(rt.tok_pos + second + lane, pos);
     stc_i32(rt.tok_first + second + lane, first);
-    if (second) stc_u64(rt.ids2 + lane, ldc_u64((const int *)rt.input_tokens + off + 2 * lane));
+    if (second) stc_u64(rt.ids2 + second - MK_MAX_TOKENS + lane, ldc_u64((const int *)rt.input_tokens + off + 2 * lane));
   }
+  const bool single = !__any(n > 1);
   if (lane == 0) {
-    if (!second) {
+    if (several) {  // (where one is bad, none of them runs: mk_kernel_body)
+      stc_i32(&rt.sched->group[portion], bad ? -bad : single ? ntok | MK_GROUP_SINGLE : ntok);
+    } else {
       stc_i32(&rt.sched->bad_batch, bad);
       stc_i32(&rt.sched->num_tokens, ntok);
-    } else if (bad) {  // (then the first one does not run either)
-      stc_i32(&rt.sched->bad_batch, bad);
-      stc_i32(&rt.sched->num_tokens, 0);
     }
-    stc_i32(&rt.sched->num_tokens2, second ? ntok : 0);
   }
   return ntok;
 }
@@ -831,22 +829,28 @@ __device__ __forceinline__ void mk_fetch_batch(const int *src, int *dst, long lo
 }
 
 // The scheduler's step of a launch whose batch the host describes, by one wavefront of the first workgroup, beside the handshake that opens the
-// launch: behind it, on the first virtual workgroup, its 5.6 us came on top (13 passes of suborax-small FIG1).
-__device__ __attribute__((noinline)) void mk_open_batch(const MkRuntime &rt, int lane, const int *src, int *dst, long long words, int second, long long words2) {
+// launch: behind it, on the first virtual workgroup, its 5.6 us came on top (13 passes of suborax-small 2005 -> 1980 us).
+__device__ __attribute__((noinline)) void mk_open_batch(const MkRuntime &rt, int lane, const int *src, int *dst, long long words) {
   if (words) mk_fetch_batch(src, dst, words, lane);
-  if (MK_PAIR && second) mk_fetch_batch(src + second, dst + second, words2, lane);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  int ntok = mk_batch_from_meta(rt, lane, 0, MK_PAIR && second);
-  const bool pair = MK_PAIR && second && ntok > 0;
-  if (pair && mk_batch_from_meta(rt, lane, second, true) == 0) ntok = 0;
+  const int ntok = mk_batch_from_meta(rt, lane, 0, false, 0);
   if (lane == 0) {
     MkSched *sc = rt.sched;
     if (ntok == 0) sc->finished = 1;
-    else sc->iterations += pair ? 2 : 1;
-    for (int q = pair ? 1 : 0; q >= 0; q--)
-      if (rt.timing && sc->iterations - q <= rt.timing_cap) rt.timing[sc->iterations - q] = (long long)wall_clock64();
+    else sc->iterations += 1;
+    if (rt.timing && sc->iterations <= rt.timing_cap) rt.timing[sc->iterations] = (long long)wall_clock64();
   }
 }
+#if MK_PAIR
+// The same for one portion of several, each by a workgroup of its own (one after the other, a portion takes 4 to 6 us); what the launch makes of them
+// all is for mk_kernel_body.
+__device__ __attribute__((noinline)) void mk_open_portion(const MkRuntime &rt, int lane, const int *src, int *dst, int words, int off, int portion, int portions) {
+  if (words) mk_fetch_batch(src + off, dst + off, words, lane);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  mk_batch_from_meta(rt, lane, off, true, portion);
+  if (lane == 0 && portion == portions - 1 && portions < MK_GROUP) stc_i32(&rt.sched->group[portions], 0);
+}
+#endif
 
 // The reference's MODE_ONLINE step (persistent_kernel.cuh:538-568): one request (slot 0, request 0) whose tokens the
 // host has written into tokens[0, :]; every pass consumes num_new_tokens[0] of them starting at step[0].  After a pass
@@ -1066,9 +1070,10 @@ __device__ __forceinline__ void stage_norm_rows(CStage &st, Ctx &c, int M, char 
   }
   c.wrote_through = true;
 }
+__device__ __forceinline__ bool norm_by_rows(CStage &st) { return (st.k & 7) == 0 && st.k / 8 <= 6 * MK_THREADS && (st.ld_in & 7) == 0 && (st.ld_out & 7) == 0; }
 __device__ __forceinline__ void stage_norm(CStage &st, Ctx &c, int M, char *smem) {
   const int k8 = st.k / 8;
-  if ((st.k & 7) == 0 && k8 <= 6 * MK_THREADS && (st.ld_in & 7) == 0 && (st.ld_out & 7) == 0) {
+  if (norm_by_rows(st)) {
     if (k8 <= MK_THREADS) stage_norm_rows<1>(st, c, M, smem);
     else if (k8 <= 2 * MK_THREADS) stage_norm_rows<2>(st, c, M, smem);
     else stage_norm_rows<6>(st, c, M, smem);
@@ -2081,13 +2086,11 @@ __device__ __forceinline__ void stage_linear_mfma_tiles(CStage &st, Ctx &c, cons
 #endif
 __device__ __forceinline__ XresPlan linear_xres_plan(CStage &st, const Ctx &c) { return mk_xres_plan(st, c.G); }
 
-// MT token tiles.  Eight: those of two portions (MK_PAIR_BOTH), four tiles each: M rows of this stage and M2 of `st2`, which differs in where its rows lie.
-// Passes are then half as long, and so is the ring.
+// MT token tiles.
 template <int MT, int TW>
-__device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const MkRuntime &rt, int M, const XresPlan plan, char *smem, CStage &st2, int M2) {
+__device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const MkRuntime &rt, int M, const XresPlan plan, char *smem) {
   c.wrote_through = true;  // partial tiles and outputs are all written through: no L2 write-back at this stage's arrival
-  constexpr bool BOTH = MT == 8;
-  constexpr int NSP = BOTH ? MK_XRES_STEPS / 2 : MK_XRES_STEPS;
+  constexpr int NSP = MK_XRES_STEPS;
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const bool silu = st.flags & MK_F_SILU;
@@ -2105,7 +2108,6 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   const int kslice = K / S, kbeg = sl * kslice, nsteps = kslice >> 6, npass = nsteps / NSP;
   const uint16_t *x = (st.flags & MK_F_NORM) ? (const uint16_t *)st.norm_out : (const uint16_t *)st.in;
   const int ldx = (st.flags & MK_F_NORM) ? st.ld_norm : st.ld_in;
-  const uint16_t *x2 = !BOTH ? x : (st.flags & MK_F_NORM) ? (const uint16_t *)st2.norm_out : (const uint16_t *)st2.in;
   u32x4 *xl = (u32x4 *)smem;  // two buffers of [step of the pass][token tile][16 rows][8] 16-byte words
   constexpr int XBUF = NSP * MT * 128;  // 16-byte operands per buffer
   int *sflag = (int *)(smem + 2 * XBUF * 16);
@@ -2120,9 +2122,6 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     c.defer_part = (const float *)rt.splitk_part;
     c.defer_res = (st.flags & MK_F_RES) ? st.res : nullptr;
     c.defer_ld_res = st.ld_res;
-#if MK_PAIR
-    c.defer_res2 = (st.flags & MK_F_RES) ? st2.res : nullptr;
-#endif
   }
   // this lane's first operand of weight tile ti, and the distance (in 16-byte operands) between steps and between the two
   // halves of a step: the re-laid copy streams contiguously, the row-major original reads 64 bytes of each of 16 rows
@@ -2149,13 +2148,12 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   // (64 tokens, operand order -> lines, us: 24576 x 4096 41.9 -> 39.6, 4096 x 12288 28.9 -> 27.0, 6144 x 4096 17.3 -> 16.7.)
   auto stage_pass = [&](int pass, int par, int w, int nw) {
     const uint16_t *base = x + kbeg + pass * (NSP * 64) + ((lane & 7) ^ (lane >> 3)) * 8;
-    const uint16_t *base2 = BOTH ? x2 + kbeg + pass * (NSP * 64) + ((lane & 7) ^ (lane >> 3)) * 8 : base;
     u32x4 *buf = xl + (par & 1) * XBUF;
     for (int i = w; i < MT * NSP; i += nw) {
-      const int step = i / MT, mt = i - step * MT, r0 = (BOTH ? mt & 3 : mt) * 16 + (lane >> 3), last = (BOTH && mt >= 4 ? M2 : M) - 1;
+      const int step = i / MT, mt = i - step * MT, r0 = mt * 16 + (lane >> 3);
       __attribute__((address_space(3))) char *dst = (__attribute__((address_space(3))) char *)(buf + (size_t)i * 128);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)((BOTH && mt >= 4 ? base2 : base) + (size_t)min(r0, last) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 16 /* sc1 */);
-      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)((BOTH && mt >= 4 ? base2 : base) + (size_t)min(r0 + 8, last) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 16);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)dst, 16, 0, 16 /* sc1 */);
+      __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)(unsigned long long)(base + (size_t)min(r0 + 8, M - 1) * ldx + (step << 6)), (__attribute__((address_space(3))) void *)(dst + 1024), 16, 0, 16);
     }
   };
 
@@ -2179,7 +2177,7 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     // weights do not depend on the previous stage: the first NBP steps are requested before its barrier is awaited, the
     // rest of the ring right after the first pass's token rows (what a CU has in flight sits in front of the barrier
     // poll and of the row requests)
-    constexpr int NBP = BOTH ? 3 : MK_TUNE_XRES_PRE < NB ? MK_TUNE_XRES_PRE : NB;
+    constexpr int NBP = MK_TUNE_XRES_PRE < NB ? MK_TUNE_XRES_PRE : NB;
     if (streams) {
 #pragma unroll
       for (int j = 0; j < NBP; j++) w_load(wrow, j, a[j]);
@@ -2271,10 +2269,10 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
       auto store_tile = [&](int otile, const f32x4 (&v)[MT]) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-          const int m = (BOTH ? mt & 3 : mt) * 16 + lr;
-          if (m < (BOTH && mt >= 4 ? M2 : M)) {
-            uint16_t *orow = (uint16_t *)(BOTH && mt >= 4 ? st2.out : st.out) + (size_t)m * st.ld_out;
-            const uint16_t *rrow = (const uint16_t *)(BOTH && mt >= 4 ? st2.res : st.res) + (size_t)m * st.ld_res;
+          const int m = mt * 16 + lr;
+          if (m < M) {
+            uint16_t *orow = (uint16_t *)st.out + (size_t)m * st.ld_out;
+            const uint16_t *rrow = (const uint16_t *)st.res + (size_t)m * st.ld_res;
             float rr[4], res[4];
             if (st.flags & MK_F_RES) ldc_bf16x4(rrow, otile * 16 + lg * 4, n_out, res);
 #pragma unroll
@@ -2355,9 +2353,8 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
     }
     // ---- combine the S slices: partial tiles through the write-through buffer, summed by the last workgroup to arrive
     if (S > 1) {
-      // [workgroup][wavefront][tile][token tile][lane], 64 KB a workgroup: four wavefronts (two hold tiles) of four by four tiles, or two of four by eight
-      auto part_at = [&](int wg, int ti, int mt) { return (BOTH ? (((size_t)wg * 2 + wave) * 4 + ti) * 8 + mt : (((size_t)wg * 4 + wave) * 4 + ti) * 4 + mt) * 64 + lane; };
-      constexpr int QS = BOTH ? 2 : 4;  // slices requested at once
+      auto part_at = [&](int wg, int ti, int mt) { return ((((size_t)wg * 4 + wave) * 4 + ti) * 4 + mt) * 64 + lane; };
+      constexpr int QS = 4;  // slices requested at once
       if (has_tile) {
 #pragma unroll
         for (int t = 0; t < TW; t++)
@@ -4768,6 +4765,9 @@ __device__ __attribute__((noinline)) void mk_verify_greedy(int stage, const MkRu
   }
 }
 
+#if MK_PAIR
+#include "mk_group.hip"
+#endif
 #if defined(MK_KERNEL_FLEX) || defined(MK_KERNEL_FLEX_PAIR) || defined(MK_KERNEL_FLEX_M1) || defined(MK_KERNEL_FLEX_F32) || MK_HAVE_MIX
 #include "mk_flex.hip"
 #if MK_HAVE_MIX
@@ -4785,11 +4785,11 @@ __device__ __attribute__((noinline)) void mk_verify_greedy(int stage, const MkRu
 #endif
 
 // The stage set of an instantiation: the fixed-shape stages (E = void), or the flex stages for E-typed activations.
-// M2: rows of a second portion inside prompts (MK_PAIR; 0: none).  A prompt's iterations are bound by streaming the weights, 64 rows at a time; two
-// portions as one iteration stream them once: see MkPairEntry.  Prompts of 2501 tokens of qwen3-8b, 8 layers: 40.0 -> 32.5 ms; of four requests of
-// up to 1501 tokens of suborax-8b, with 24 steps behind them: 97.0 -> 83.3.
+// Several portions inside prompts as one iteration (MK_PAIR): see MkPairEntry.  M1: rows of the first one; sh_rows: of all, in LDS; tok: the tokens of the
+// first one and, behind them, of the one that runs beside it (c.sh_tok); any_single: in some portion every request brings one row.
 template <int MAXM, typename E>
-__device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkRuntime *rtp, Ctx &c, const int M1, const int M2, const int n_stages, char *smem) {
+__device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkRuntime *rtp, Ctx &c, const int M1, const int portions, const bool any_single, const int *sh_rows, int *tok,
+                                                  const int n_stages, char *smem) {
     constexpr bool FX = !std::is_void<E>::value;
     constexpr bool F32 = std::is_same<E, float>::value;
     int M = M1;
@@ -4802,11 +4802,11 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
     };
     one_each();
 #if MK_PAIR
-    const int *const tok1 = c.sh_tok;
-    int sum_S = 0;  // what the last linear for both portions left to the stage behind it
+    int sum_S = 0, prep_S = 0;  // what the last linear for all portions left to the stage behind it; what was left to the last stage that prepares rows
     bool all_through = true;
+    int again = 1, held = 1, shown = 0;  // the portion that entries for the second one and those behind it run for; whose tokens lie behind the first one's; c.sh_tok's
     for (int e = 0; e < rt.pair_n && !c.dead; e++) {
-      const unsigned ent = ((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e];
+      const unsigned ent = (unsigned)__builtin_amdgcn_readfirstlane((int)((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e]);
       const int s = (int)(ent & MK_PAIR_STAGE);
       if (ent & MK_PAIR_ACQUIRE) {
         barrier_wait(c);
@@ -4814,17 +4814,50 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         __syncthreads();
         continue;
       }
-      if (((ent & MK_PAIR_SECOND) != 0) != (c.sh_tok != tok1)) {
-        c.sh_tok = ent & MK_PAIR_SECOND ? tok1 + 4 * MK_MAX_TOKENS : tok1;
-        M = ent & MK_PAIR_SECOND ? M2 : M1;
+      const int portion = ent & MK_PAIR_SECOND ? again : 0;
+      const bool behind = again + 1 < portions;  // another portion comes behind this one
+      const bool on = (ent & MK_PAIR_ON) && (!(ent & MK_PAIR_SECOND) || behind), release = (ent & MK_PAIR_RELEASE) && (!(ent & MK_PAIR_SECOND) || behind);
+      auto turn = [&]() {  // where the last entry of a portion has run: on to the next portion's
+        if (ent & MK_PAIR_LOOP) {
+          if (behind) {
+            again++;
+            e -= 1 + (int)(ent >> MK_PAIR_BACK_SHIFT);
+          } else {
+            again = 1;
+          }
+        }
+      };
+      // (the last portion's run of a stage that nobody has waited behind yet posts the arrival for all of them; not before everybody has arrived in front: the
+      // barrier counts arrivals, not workgroups)
+#define MK_LEAVE_OUT { if ((ent & MK_PAIR_ON) && !on) { barrier_wait(c); c.rows_ahead = 0; c.wrote_through = all_through; all_through = true; barrier_arrive(c); } turn(); continue; }
+      // Norms look at no tokens; and a workgroup that none of a portion's rows are dealt to need not look at the stage: 512 rows of 4096 values from four slices
+      // 35 -> 20 us.
+      const int dealt = mk_portion_stages(rt, 0)[s].op;
+      const bool rows_only = dealt == MK_OP_NORM || dealt == MK_OP_FX_ADDNORM;
+      c.portion = portion;
+      M = __builtin_amdgcn_readfirstlane(sh_rows[portion]);
+      if (rows_only && (ent & MK_PAIR_ON) && row_item(c) >= M && (dealt != MK_OP_NORM || norm_by_rows(mk_portion_stages(rt, 0)[s]))) {
+        c.defer_S = 0;
+        if (on) c.rows_ahead = mk_rows_ahead(c.rows_ahead + M, c.G);
+        MK_LEAVE_OUT;
+      }
+      if (!rows_only && portion != shown) {
+        if (portion && portion != held) {
+          mk_portion_rows(rt, tok + 4 * MK_MAX_TOKENS, (int)threadIdx.x, M, portion);
+          held = portion;
+          __syncthreads();
+        }
+        c.sh_tok = portion ? tok + 4 * MK_MAX_TOKENS : tok;
+        shown = portion;
         one_each();
       }
       if (ent & MK_PAIR_AGAIN) {
         c.defer_S = sum_S;
-        c.defer_part = (const float *)rt.splitk_part + (size_t)MK_MAX_TOKENS * c.defer_n;
-        c.defer_res = c.defer_res2;
+        c.defer_part = rt.group_part + (size_t)portion * MK_MAX_TOKENS * c.defer_n;
+        CStage &sum = mk_portion_stages(rt, portion)[c.defer_stage];
+        c.defer_res = sum.flags & MK_F_RES ? sum.res : nullptr;
       }
-      CStage &st = ((CStage *)(unsigned long long)(ent & MK_PAIR_SECOND ? rt.stages2 : rt.stages))[s];
+      CStage &st = mk_portion_stages(rt, portion)[s];
 #else
     for (int s = 0; s < (MAXM == 1 ? rt.num_stages : n_stages) && !c.dead; s++) {
       CStage &st = ((CStage *)(unsigned long long)rt.stages)[s];
@@ -4832,19 +4865,29 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       const int op = st.op, flags = st.flags;
       // (a handle that holds only the matrix-core copies of its weights runs every linear in a matrix-core form, which
       // reads normalised rows from the NORM stage's output: that stage then runs for one and two tokens as well)
+#if MK_PAIR
+      // (a portion whose rows nobody prepares leaves its sum to the attention, which comes behind other portions' preparation)
+      if (FX && op == MK_OP_FX_PREP) prep_S = c.defer_S;
+      if (FX && op == MK_OP_FX_ATTN && (ent & MK_PAIR_ON) && single) {
+        c.defer_S = prep_S;
+        c.defer_part = rt.group_part + (size_t)portion * MK_MAX_TOKENS * c.defer_n;
+      }
+#else
+#define MK_LEAVE_OUT continue
+#endif
       const bool packed_only = MAXM > 1 && rt.packed_only;
-      if ((flags & MK_F_ONLY_MULTI) && M == 1 && !(packed_only && (op == MK_OP_NORM || (FX && (op == MK_OP_FX_ADDNORM || op == MK_OP_MX_PRENORM))))) continue;
-      if (FX && op == MK_OP_FX_PREP && single) continue;
+      if ((flags & MK_F_ONLY_MULTI) && M == 1 && !(packed_only && (op == MK_OP_NORM || (FX && (op == MK_OP_FX_ADDNORM || op == MK_OP_MX_PRENORM))))) MK_LEAVE_OUT;
+      if (FX && op == MK_OP_FX_PREP && single) MK_LEAVE_OUT;
 #if MK_HAVE_DUAL
-      if (op == MK_OP_DU_CONV && (flags & MK_F_PORTIONS) && (MAXM == 1 || single)) continue;
+      if (op == MK_OP_DU_CONV && (flags & MK_F_PORTIONS) && (MAXM == 1 || single)) MK_LEAVE_OUT;
 #endif
 #if MK_HAVE_MIX
-      if ((op == MK_OP_MX_LATENT_MERGE || op == MK_OP_MX_DELTA_OUT) && !c.mx_split) continue;
+      if ((op == MK_OP_MX_LATENT_MERGE || op == MK_OP_MX_DELTA_OUT) && !c.mx_split) MK_LEAVE_OUT;
 #endif
       if ((flags & MK_F_ONLY_MULTI) && op == MK_OP_NORM && s + 1 < rt.num_stages && !packed_only) {
         // the few-token linear normalises its rows itself
         CStage &nx = (&st)[1];
-        if (nx.op == MK_OP_LINEAR && (nx.flags & MK_F_NORM) && nx.in == st.in && linear_small_ok(nx, c, M)) continue;
+        if (nx.op == MK_OP_LINEAR && (nx.flags & MK_F_NORM) && nx.in == st.in && linear_small_ok(nx, c, M)) MK_LEAVE_OUT;
       }
       // Lane offsets that stages derive from the thread index would otherwise be computed once, ahead of all stages, and wait in scratch
       // for the stage that wants them, which then starts with a chain of scratch loads.  Scratch per lane in the kernels of several tokens: 480 -> 0
@@ -4853,6 +4896,18 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       c.tid = threadIdx.x;
       asm volatile("" : "+v"(c.tid));
       __builtin_assume(c.tid >= 0 && c.tid < MK_THREADS);
+#if MK_PAIR
+      GroupTasks tasks;
+      if constexpr (!FX) {
+        if (op == MK_OP_ATTN && (ent & MK_PAIR_BOTH)) {
+          if (!(st.num_q_heads == 4 * st.num_kv_heads   ? attn_group_tasks<4>(st, c, rt, portions, sh_rows, tasks)
+                : st.num_q_heads == 8 * st.num_kv_heads ? attn_group_tasks<8>(st, c, rt, portions, sh_rows, tasks)
+                                                        : false))
+            continue;  // (portion by portion: the entries that follow)
+          e += (int)(ent >> MK_PAIR_BACK_SHIFT);
+        }
+      }
+#endif
       c.st = &st;
       const long long t_in = (long long)wall_clock64();
       switch (op) {
@@ -4896,10 +4951,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
           if constexpr (F32) barrier_wait(c);
 #if MK_PAIR
           else if (ent & MK_PAIR_BOTH) {
-            const XresPlan xp = linear_xres_plan(st, c);
-            CStage &st2 = ((CStage *)(unsigned long long)rt.stages2)[s];
-            if (xp.tpu <= 4) stage_linear_mfma_xres<8, 2>(st, c, rt, M1, xp, smem, st2, M2);
-            else stage_linear_mfma_xres<8, 3>(st, c, rt, M1, xp, smem, st2, M2);
+            stage_linear_group(st, c, rt, s, portions, sh_rows, smem);
             sum_S = c.defer_S;
           }
 #endif
@@ -4922,14 +4974,14 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
               // (4 tokens with one tile instead of two, us: 6144 x 4096 11.7 -> 10.8, 4096 x 4096 9.8 -> 8.8, 4096 x 12288 19.8 -> 18.6; a third of
               // 48 instead of 64 would be another pair of instances for fewer batches)
               if (M <= 16) {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<1, 2>(st, c, rt, M, xp, smem, st, 0);
-                else stage_linear_mfma_xres<1, 3>(st, c, rt, M, xp, smem, st, 0);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<1, 2>(st, c, rt, M, xp, smem);
+                else stage_linear_mfma_xres<1, 3>(st, c, rt, M, xp, smem);
               } else if (M <= 32) {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<2, 2>(st, c, rt, M, xp, smem, st, 0);
-                else stage_linear_mfma_xres<2, 3>(st, c, rt, M, xp, smem, st, 0);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<2, 2>(st, c, rt, M, xp, smem);
+                else stage_linear_mfma_xres<2, 3>(st, c, rt, M, xp, smem);
               } else {
-                if (xp.tpu <= 4) stage_linear_mfma_xres<4, 2>(st, c, rt, M, xp, smem, st, 0);
-                else stage_linear_mfma_xres<4, 3>(st, c, rt, M, xp, smem, st, 0);
+                if (xp.tpu <= 4) stage_linear_mfma_xres<4, 2>(st, c, rt, M, xp, smem);
+                else stage_linear_mfma_xres<4, 3>(st, c, rt, M, xp, smem);
               }
             } else if (plan.S >= 1 && !(packed_only && st.wpack)) {  // (this form reads the row-major weights)
               if (M <= 16) stage_linear_mfma_tiles<1>(st, c, rt, M, plan, smem);
@@ -4965,6 +5017,11 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         case MK_OP_ATTN:
           if constexpr (FX) {
             barrier_wait(c);
+#if MK_PAIR
+          } else if (ent & MK_PAIR_BOTH) {
+            if (st.num_q_heads == 4 * st.num_kv_heads) stage_attn_group<4>(c, rt, s, portions, sh_rows, tasks, smem);
+            else stage_attn_group<8>(c, rt, s, portions, sh_rows, tasks, smem);
+#endif
           } else if constexpr (MAXM == 1) {
             if (st.num_q_heads == 4 * st.num_kv_heads) stage_attn<4>(st, c, rt, M, smem);
             else if (st.num_q_heads == 8 * st.num_kv_heads) stage_attn<8>(st, c, rt, M, smem);
@@ -4994,18 +5051,27 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       }
       const long long t_out = (long long)wall_clock64();
 #if MK_PAIR
-      c.rows_ahead = 0;
-      if (ent & MK_PAIR_ON) {  // (as between two stages, but nobody waits for anybody)
-        all_through = c.wrote_through;
+      if (on) {  // (as between two stages, but nobody waits for anybody)
+        all_through = all_through && c.wrote_through;
         c.wrote_through = false;
-        c.rows_ahead = mk_rows_ahead(M1, c.G);
-        c.seq++;
-        if (threadIdx.x == 0) c.sh_ticket[c.seq & 1] = 0;
-        __syncthreads();
+        c.rows_ahead = mk_rows_ahead(c.rows_ahead + M, c.G);
+        if (FX && op == MK_OP_FX_ATTN && any_single) {  // (which appends the rows of such portions itself)
+          barrier_arrive(c);
+          barrier_wait(c);
+          if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+          __syncthreads();
+        } else {
+          c.seq++;
+          if (threadIdx.x == 0) c.sh_ticket[c.seq & 1] = 0;
+          __syncthreads();
+        }
+        turn();
         continue;
       }
-      c.wrote_through = c.wrote_through && all_through && !(ent & MK_PAIR_RELEASE);
+      c.rows_ahead = 0;
+      c.wrote_through = c.wrote_through && all_through && !release;
       all_through = true;
+      turn();
 #endif
       barrier_arrive(c);
       if (threadIdx.x == 0 && rt.profiler) {
@@ -5044,6 +5110,9 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   __shared__ int sh_quota[10];
   __shared__ int sh_tok[MK_PAIR ? 8 : 4][MK_MAX_TOKENS];
   __shared__ int sh_ticket[3];
+#if MK_PAIR
+  __shared__ int sh_rows[MK_GROUP];
+#endif
   // rt arrives by value in the kernel-argument segment (scalar loads); rtp is the same structure in device memory
   // for the one non-inlined function that takes its address (the scheduler step)
   Ctx c;
@@ -5067,7 +5136,8 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
 #if MK_PAIR
   c.rows_ahead = 0;
   c.defer_n = 0;
-  c.defer_res2 = nullptr;
+  c.defer_stage = 0;
+  c.portion = 0;
 #endif
   c.wrote_through = false;
   c.arrive_w0 = false;
@@ -5079,10 +5149,15 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   // final once they add up to the grid.  (One counter for the whole grid beside them, awaited with acquiring loads: 8.0 us instead of 4.6 in a launch of
   // nothing else.)
   const bool from_meta = run_scheduler == MK_SCHED_FROM_META || run_scheduler == MK_SCHED_INGEST;
+#if MK_PAIR
+  if (from_meta && __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 1)
+    for (int p = blockIdx.x; p < rt.batch_n; p += c.G) mk_open_portion(*rtp, threadIdx.x & 63, rt.batch_src, rt.batch_dst, rt.batch_len[p], rt.batch_at[p], p, rt.batch_n);
+#else
   if (from_meta && blockIdx.x == 0 && __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 1) {
     // (rtp is the graph's; what belongs to this launch is in rt)
-    mk_open_batch(*rtp, threadIdx.x & 63, rt.batch_src, rt.batch_dst, rt.batch_words, MK_PAIR ? rt.batch2 : 0, MK_PAIR ? rt.batch_words2 : 0);
+    mk_open_batch(*rtp, threadIdx.x & 63, rt.batch_src, rt.batch_dst, rt.batch_words);
   }
+#endif
   if (threadIdx.x == 0) {
     MkSync *s = rt.sync;
     if (blockIdx.x == 0 && run_scheduler != MK_SCHED_RESUME) s->t_begin = (long long)wall_clock64();
@@ -5146,19 +5221,19 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       t_sched0 = (long long)wall_clock64();
       // a handful of slots and short portions: one thread walks them; else a wavefront, one lane per slot
       const bool wave_sched = run_scheduler == MK_SCHED_OFFLINE && !prepared && (rt.max_requests > 2 || MAXM > 1 && rt.max_new_per_req > 8) && rt.spec_len == 0;
-      int ntok_w = 0;
-      bool second = false;
+      int ntok_w = 0, portions = 1;
       if (c.vid == 0 && threadIdx.x < 64 && wave_sched) {
         ntok_w = mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, 0);
 #if MK_PAIR
-        second = __builtin_amdgcn_readfirstlane(ntok_w & MK_PAIR_NEXT) && it + 2 < max_iters && !rt.profiler;  // (the launch's last iteration runs alone)
+        bool next = __builtin_amdgcn_readfirstlane(ntok_w & MK_PAIR_NEXT);
         ntok_w &= MK_PAIR_NEXT - 1;
-        if (second) {
+        for (; next && portions < rt.group && it + portions + 1 < max_iters && !rt.profiler; portions++) {  // (the launch's last iteration runs alone)
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-          mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, 1);
+          next = __builtin_amdgcn_readfirstlane(mk_prepare_next_batch_wave(*rtp, (int *)smem, threadIdx.x, portions) & MK_PAIR_NEXT);
         }
+        if (threadIdx.x == 0 && portions < MK_GROUP) rt.sched->group[portions] = 0;
 #endif
       }
       if (from_meta) c.wrote_through = true;  // (nothing else was written in this launch)
@@ -5168,9 +5243,9 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
         else if (run_scheduler == MK_SCHED_OFFLINE) ntok = mk_prepare_next_batch(*rtp, (int *)smem);
         else ntok = mk_online_next_batch(*rtp);
         if (ntok == 0) rt.sched->finished = 1;
-        else rt.sched->iterations += second ? 2 : 1;
+        else rt.sched->iterations += portions;
         if (MK_PAIR) rt.sched->resume_it = ntok == 0 ? max_iters : it;
-        for (int q = second ? 1 : 0; q >= 0; q--)
+        for (int q = portions - 1; q >= 0; q--)
           if (rt.timing && rt.sched->iterations - q <= rt.timing_cap) rt.timing[rt.sched->iterations - q] = (long long)wall_clock64();
         t_sched1 = (long long)wall_clock64();
       }
@@ -5186,7 +5261,26 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       sh_bcast[0] = ldc_i32(&rt.sched->num_tokens);
       if constexpr (MAXM > 1) sh_bcast[1] = ldc_i32(&rt.sched->inner);
 #if MK_PAIR
-      sh_bcast[2] = run_scheduler ? ldc_i32(&rt.sched->num_tokens2) : 0;
+      int rows[MK_GROUP], n = 0, single = 0, bad = 0;
+#pragma unroll
+      for (int p = 0; p < MK_GROUP; p++) rows[p] = ldc_i32(&rt.sched->group[p]);
+#pragma unroll
+      for (int p = 0; p < MK_GROUP; p++) {
+        if (n == p && rows[p] != 0 && p < rt.group) n = p + 1;
+        sh_rows[p] = rows[p] & (MK_GROUP_SINGLE - 1);
+        if (n == p + 1 && rows[p] < 0 && !bad) bad = -rows[p];
+        if (n == p + 1 && rows[p] & MK_GROUP_SINGLE) single = 1;
+      }
+      if (from_meta) sh_bcast[0] = bad ? 0 : sh_rows[0];
+      sh_bcast[1] = n | (single << 8);
+      if (from_meta && c.vid == 0) {
+        MkSched *sc = rt.sched;
+        sc->bad_batch = bad;
+        if (bad) sc->finished = 1;
+        else sc->iterations += n;
+        for (int q = n - 1; q >= 0 && !bad; q--)
+          if (rt.timing && sc->iterations - q <= rt.timing_cap) rt.timing[sc->iterations - q] = c.t_wait;
+      }
 #endif
       c.sh_ticket[2] = MK_NO_LISTS;  // (expert lists are this iteration's)
     }
@@ -5201,17 +5295,11 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
       sh_tok[2][t] = ldc_i32(&rt.tok_first[t]);
       sh_tok[3][t] = ldc_i32(&rt.kv_indptr[slot]);
     }
-    int M2 = 0;
+    int portions = 1;
 #if MK_PAIR
-    M2 = M > 0 ? __builtin_amdgcn_readfirstlane(sh_bcast[2]) : 0;
-    more = M2 > 0 ? 2 : 1;
-    if (const int t = (int)threadIdx.x - MK_MAX_TOKENS; t >= 0 && t < M2) {
-      const int slot = ldc_i32(&rt.tok_slot[MK_MAX_TOKENS + t]);  // (what is looked up by it, page tables among it, lies batch2 words behind)
-      sh_tok[4][t] = ldc_i32(&rt.tok_pos[MK_MAX_TOKENS + t]);
-      sh_tok[5][t] = slot;
-      sh_tok[6][t] = ldc_i32(&rt.tok_first[MK_MAX_TOKENS + t]);
-      sh_tok[7][t] = rt.batch2 + ldc_i32(&rt.kv_indptr[slot]);
-    }
+    portions = M > 0 ? __builtin_amdgcn_readfirstlane(sh_bcast[1] & 255) : 0;
+    more = max(portions, 1);
+    if (portions > 1) mk_portion_rows(rt, sh_tok[4], (int)threadIdx.x - MK_MAX_TOKENS, sh_rows[1], 1);
 #endif
     __syncthreads();
     if (threadIdx.x == 0 && rt.stage_prof && run_scheduler) {
@@ -5228,16 +5316,17 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
     // 32768: 46.7 -> 41.1 ms; prompts of four requests of suborax-8b 1175 -> 994 us a pass, 32-bit 868 -> 676.)
     int n_stages = rt.num_stages;
     if constexpr (MAXM > 1) {
-      const bool inner = __builtin_amdgcn_readfirstlane(sh_bcast[1]) != 0;
+      const bool inner = MK_PAIR || __builtin_amdgcn_readfirstlane(sh_bcast[1]) != 0;
       if (!rt.profiler && (run_scheduler == MK_SCHED_INGEST || (run_scheduler == MK_SCHED_OFFLINE && inner && it + 1 < max_iters))) n_stages = rt.tail;
     }
     if (M == 0 || c.dead) break;
 #if MK_PAIR
-    if (M2 == 0) break;  // (the iteration is left to the kernel behind this one)
-#endif
-    run_stage_program<MAXM, E>(rt, rtp, c, MAXM == 1 ? 1 : M, M2, n_stages, smem);
-#if MK_PAIR
+    if (portions < 2) break;  // (the iteration is left to the kernel behind this one)
+    run_stage_program<MAXM, E>(rt, rtp, c, M, portions, (sh_bcast[1] >> 8) != 0, sh_rows, &sh_tok[0][0], n_stages, smem);
     c.sh_tok = &sh_tok[0][0];
+    c.portion = 0;
+#else
+    run_stage_program<MAXM, E>(rt, rtp, c, MAXM == 1 ? 1 : M, portions, false, nullptr, nullptr, n_stages, smem);
 #endif
   }
   barrier_wait(c);  // drain: nobody leaves while another workgroup may still poll

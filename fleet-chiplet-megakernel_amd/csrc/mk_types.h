@@ -21,6 +21,7 @@
 #define MK_MAX_XCD 16
 #define MK_MAX_SEGS 3         // a shuffled weight has at most 3 sources (q,k,v)
 #define MK_MAX_TOKENS 64      // max tokens per iteration supported by the kernels
+#define MK_GROUP 8            // portions of prompts that may run as one iteration, MK_MAX_TOKENS rows each at most
 #define MK_ATTN_MAX_CHUNKS 32 // split-KV fan-out limit per (token, kv head)
 #define MK_ATTN_PSTRIDE 160   // floats per (work unit, q head) split-KV partial: 128 values + one 128-byte line of (max, sum)
 #define MK_MAX_NEW_PER_REQ 64 // most prompt tokens one request may ingest per iteration (the attention stage keeps their K/V rows in LDS); the
@@ -280,6 +281,33 @@ MK_HOST_DEVICE inline XresPlan mk_xres_plan(Stage &st, int G) {
   return p;
 }
 
+// The same linear over the rows of several portions (stage_linear_group): a task is (four wavefronts of `tw` weight tiles, K slice, two portions), and
+// a workgroup takes tasks [v tasks / G, (v + 1) tasks / G).  Slices are those of one portion alone, so that sums are the same.  Few large tasks take few
+// bytes of rows and weights per product, many small ones fill the chip: a step of 64 along K takes 256 tw clocks of the matrix cores, or 3.2 for each of
+// the 64 tw + 128 lines of 128 bytes that a workgroup fetches for it (40 bytes a clock), whichever is longer.
+struct GroupPlan {
+  int S, wt, tw, nb, mb, tasks;
+};
+template <typename Stage>
+MK_HOST_DEVICE inline GroupPlan mk_group_plan(Stage &st, int G, int portions) {
+  const XresPlan x = mk_xres_plan(st, G);
+  GroupPlan p;
+  p.S = x.S;
+  p.wt = x.wt;
+  p.mb = (portions + 1) / 2;
+  p.tw = p.nb = p.tasks = 0;
+  int best = 0;
+  for (int tw = 2; tw <= 4 && p.S; tw++) {
+    const int nb = (p.wt + 4 * tw - 1) / (4 * tw), tasks = nb * p.mb * p.S, core = 256 * tw, path = (64 * tw + 128) * 16 / 5, cost = (tasks + G - 1) / G * (core > path ? core : path);
+    if (p.tw && cost >= best) continue;
+    best = cost;
+    p.tw = tw;
+    p.nb = nb;
+    p.tasks = tasks;
+  }
+  return p;
+}
+
 // Rows are dealt to G workgroups in turn.  Where those of another portion have been dealt just before, they go on with the workgroup behind the last of
 // them: `ahead` workgroups further (grids may be smaller than a portion), and the first row of the workgroup that comes `at`-th is what mk_first_row says.
 MK_HOST_DEVICE inline int mk_rows_ahead(int dealt, int G) {
@@ -337,20 +365,24 @@ struct MkSched {
 
   long long iterations;   // decode iterations executed so far (all launches)
   int inner;              // every row of the iteration lies in front of its prompt's last token (portions of several tokens only)
-  int num_tokens2;        // rows of the portion that runs in the same iteration (0: none)
-  int resume_it, unused;  // the launch's first iteration that the pair kernel left to the other one
+  int resume_it;          // the launch's first iteration that the pair kernel left to the other one
+  int group[MK_GROUP];    // rows of the portions that run in this iteration, up to the first 0 (iterations of several only); MK_GROUP_SINGLE: every
+                          // request of the portion brings one row; negative: the description was rejected, for this reason
 };
+#define MK_GROUP_SINGLE 0x10000
 
-// What an iteration of two portions runs, one after another: a stage's index with these bits.  Linears that stream their weights through the matrix
-// cores run for both portions at once (MK_PAIR_BOTH); the stages between two of them run for the first portion and then for the second one.
+// What an iteration of several portions runs, one after another: a stage's index with these bits.  Linears that stream their weights through the matrix
+// cores run for all portions at once (MK_PAIR_BOTH); the stages between two of them run for the first portion, then for the second one, and so on.
 enum MkPairEntry {
   MK_PAIR_STAGE = 0xffff,
-  MK_PAIR_SECOND = 1 << 16,   // for the second portion
-  MK_PAIR_BOTH = 1 << 17,
-  MK_PAIR_ON = 1 << 18,       // the second portion's run of this stage follows without a barrier
-  MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written, here or by the stages in front, for the second portion to read: write back ...
+  MK_PAIR_SECOND = 1 << 16,   // for the second portion, and each one behind it
+  MK_PAIR_BOTH = 1 << 17,     // for all at once; attention (MK_OP_ATTN): where the portions allow it, and the `back` entries behind it, for one after the other, are skipped
+  MK_PAIR_ON = 1 << 18,       // the next portion's run of this stage follows without a barrier
+  MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written, here or by the stages in front, for the next portion to read: write back ...
   MK_PAIR_ACQUIRE = 1 << 20,  // ... and, no stage, drop what the caches of the dies hold
   MK_PAIR_AGAIN = 1 << 21,    // the linear in front may have left its sum to this stage
+  MK_PAIR_LOOP = 1 << 22,     // the last entry of a portion: the next one's run `back` entries in front
+  MK_PAIR_BACK_SHIFT = 23,    // (nine bits)
 };
 
 // Whether the next iterations of the offline scheduler run as `need` pairs of portions: by the rule of its step (MK_PAIR_NEXT), for entries that have
@@ -401,22 +433,28 @@ struct MkRuntime {
   const int *batch_src;
   int *batch_dst;
   long long batch_words;
-  // two portions inside prompts as one iteration (null / 0: not in this graph).  stages2: the stages as they run for the second portion, over rows of
-  // its own; pair_prog: [pair_n] what runs, see MkPairEntry; ids2: the second portion's tokens; its rows' slots, positions and first rows lie
-  // MK_MAX_TOKENS behind the first one's.  batch2 (mk_enqueue_batches): words from the first portion's description to the second one's, which has batch_words2
+  // several portions inside prompts as one iteration (null / 0: not in this graph).  group: as many at most; stages2: the stages as they run for the
+  // second portion, over rows of its own, then for the third, [group - 1][num_stages]; pair_prog: [pair_n] what runs, see MkPairEntry; ids2: their tokens,
+  // [group - 1][MK_MAX_TOKENS]; their rows' slots, positions and first rows lie MK_MAX_TOKENS behind those of the portion in front.
+  // batch_n (mk_enqueue_batches): portions that the host describes, each batch_at words behind the first one and of batch_len words (0: there already)
   const MkStage *stages2;
   const unsigned *pair_prog;
   long long *ids2;
-  long long batch_words2;
-  int pair_n, batch2;
+  int pair_n, group;
+  int batch_n, batch_at[MK_GROUP], batch_len[MK_GROUP];
+  // scratch of such iterations: K-slice partials of the linears, [slice][portion][MK_MAX_TOKENS][n]; chunk partials and arrival counters of the flex attention, group_attn values and group_cnt counters for every portion
+  float *group_part, *group_attn_part;
+  unsigned *group_attn_cnt;
+  uint16_t *group_q;    // prepared queries of the 128-wide attention, [portion][MK_MAX_TOKENS][heads][128]
+  long long group_attn, group_cnt;
   // library-owned scheduler memory
   int *request_ids;   // [max_requests] request id per batch slot, -1 = free
   int *state_ids;     // [max_requests] recurrent-state slot per batch slot, a permutation (null: the graph has no recurrence)
   int *page_queue;    // [max_pages] ring of free page ids
-  // (two of each, MK_MAX_TOKENS apart: the second portion's rows lie behind the first one's, however many those are)
-  int *tok_slot;      // [2][MK_MAX_TOKENS] batch slot of each token of this iteration
-  int *tok_pos;       // [2][MK_MAX_TOKENS] absolute position of each token
-  int *tok_first;     // [2][MK_MAX_TOKENS] index of the first token of the same request in this iteration (of its portion)
+  // (one of each for every portion, MK_MAX_TOKENS apart)
+  int *tok_slot;      // [MK_GROUP][MK_MAX_TOKENS] batch slot of each token of this iteration
+  int *tok_pos;       // [MK_GROUP][MK_MAX_TOKENS] absolute position of each token
+  int *tok_first;     // [MK_GROUP][MK_MAX_TOKENS] index of the first token of the same request in this iteration (of its portion)
   MkSched *sched;
   const MkStage *stages;
   MkSync *sync;
@@ -426,8 +464,8 @@ struct MkRuntime {
   float *argmax_pv;     // non-null: the sampling stages' per-workgroup partials live here ([workgroups][max_tokens] values / indices)
   int *argmax_pi;       // instead of in the buffers their descriptors name
   unsigned *attn_cnt;   // [max_tokens * num_kv_heads][32]: one 128-byte line per counter
-  void *splitk_part;    // 64 KB a workgroup, f32x4 K-slice partials of the split-K linear: [4 wavefronts][4 weight tiles][4 token tiles][64 lanes], for two
-                        // portions [2 wavefronts][4 weight tiles][8 token tiles][64 lanes]; or, left to the stage behind, [slice][16, 32, 64 or 128 rows][n]
+  void *splitk_part;    // 64 KB a workgroup, f32x4 K-slice partials of the split-K linear: [4 wavefronts][4 weight tiles][4 token tiles][64 lanes];
+                        // or, left to the stage behind, [slice][16, 32 or 64 rows][n]
   unsigned *splitk_cnt; // [workgroups][32]: arrival counter per split-K group (one 128-byte line each)
   long long *timing;    // [1 + timing_cap] wall-clock ticks (100 MHz) at the start of each iteration; [0] = kernel end
   int timing_cap;

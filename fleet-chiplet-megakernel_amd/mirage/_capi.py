@@ -26,7 +26,8 @@ MK_MODES = {"offline": 0, "online": 1, "online_notoken": 2, "onepass": 3}
 EXPORTED_SYMBOLS = [
     "mk_graph_create", "mk_graph_destroy", "mk_tensor_attach", "mk_tensor_new", "mk_tensor_shuffle",
     "mk_tensor_num_dims", "mk_tensor_dim", "mk_tensor_ptr", "mk_add_task", "mk_generate_task_graph",
-    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_set_host_batch", "mk_enqueue_batch", "mk_enqueue_batches", "mk_wait",
+    "mk_compile", "mk_init_requests", "mk_launch", "mk_launch_steps", "mk_enqueue_steps", "mk_enqueue_steps_static", "mk_enqueue_ingest", "mk_set_host_batch", "mk_enqueue_batch", "mk_enqueue_batches", "mk_set_more_batches",
+    "mk_hold_batches", "mk_enqueue_held", "mk_wait",
     "mk_run_once", "mk_repack_weights", "mk_tensor_releasable", "mk_set_profiler", "mk_get_stats", "mk_get_stage_profile", "mk_get_stage_marks", "mk_describe_program", "mk_last_error", "mk_version",
 ]
 
@@ -73,6 +74,7 @@ class MkStats(ctypes.Structure):
         ("packed_weight_bytes", ctypes.c_int64),
         ("row_major_weight_bytes", ctypes.c_int64),
         ("paired_portions", ctypes.c_int),
+        ("portions_together", ctypes.c_int),
     ]
 
 
@@ -120,6 +122,9 @@ def load():
     lib.mk_set_host_batch.argtypes = [vp, vp, vp, ctypes.c_int64, vp]
     lib.mk_enqueue_batch.argtypes = [vp, vp, ctypes.c_int64, ci]
     lib.mk_enqueue_batches.argtypes = [vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+    lib.mk_set_more_batches.argtypes = [vp, ctypes.c_int64]
+    lib.mk_hold_batches.argtypes = [vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+    lib.mk_enqueue_held.argtypes = [vp, vp]
     lib.mk_wait.argtypes = [vp, vp, cip]
     i32p = ctypes.POINTER(ctypes.c_int32)
     lib.mk_run_once.argtypes = [vp, vp, ci, i32p, i32p, i32p]
@@ -238,6 +243,15 @@ class Graph:
 
     def enqueue_batches(self, stream, words, second, words2):
         check(self._lib.mk_enqueue_batches(self._h, ctypes.c_void_p(stream), int(words), int(second), int(words2)))
+
+    def set_more_batches(self, words):
+        check(self._lib.mk_set_more_batches(self._h, int(words)))
+
+    def hold_batches(self, at, words, second, words2):
+        check(self._lib.mk_hold_batches(self._h, int(at), int(words), int(second), int(words2)))
+
+    def enqueue_held(self, stream):
+        check(self._lib.mk_enqueue_held(self._h, ctypes.c_void_p(stream)))
 
     def wait(self, stream) -> bool:
         fin = ctypes.c_int(0)

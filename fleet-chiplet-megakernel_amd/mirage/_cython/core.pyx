@@ -216,6 +216,15 @@ cdef class CyGraph:
     def enqueue_batches(self, stream, words, second, words2):
         _check(mk.mk_enqueue_batches(self.g, <void *><uintptr_t>(stream or 0), <int64_t>words, <int64_t>second, <int64_t>words2))
 
+    def set_more_batches(self, words):
+        _check(mk.mk_set_more_batches(self.g, <int64_t>words))
+
+    def hold_batches(self, at, words, second, words2):
+        _check(mk.mk_hold_batches(self.g, <int64_t>at, <int64_t>words, <int64_t>second, <int64_t>words2))
+
+    def enqueue_held(self, stream):
+        _check(mk.mk_enqueue_held(self.g, <void *><uintptr_t>(stream or 0)))
+
     def wait(self, stream) -> bool:
         cdef int rc, fin = 0
         cdef void *s = <void *><uintptr_t>(stream or 0)
@@ -247,7 +256,8 @@ cdef class CyGraph:
         return {"num_workgroups": st.num_workgroups, "num_stages": st.num_stages, "num_tasks": st.num_tasks, "num_events": st.num_events,
                 "num_xcds": st.num_xcds, "aborted": st.aborted, "iterations": st.iterations, "weight_bytes": st.weight_bytes,
                 "last_launch_ms": st.last_launch_ms, "packed_weight_bytes": st.packed_weight_bytes,
-                "row_major_weight_bytes": st.row_major_weight_bytes, "paired_portions": st.paired_portions}
+                "row_major_weight_bytes": st.row_major_weight_bytes, "paired_portions": st.paired_portions,
+                "portions_together": st.portions_together}
 
     def stage_ticks(self, int workgroup, int max_stages, marks=False) -> list:
         cdef int64_t *buf = <int64_t *>malloc(sizeof(int64_t) * 4 * (max_stages if max_stages > 0 else 1))

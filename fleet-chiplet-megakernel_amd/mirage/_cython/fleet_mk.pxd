@@ -44,6 +44,7 @@ cdef extern from "fleet_mk.h" nogil:
         int64_t packed_weight_bytes
         int64_t row_major_weight_bytes
         int paired_portions
+        int portions_together
 
     int mk_graph_create(const mk_config *cfg, mk_graph **out)
     int mk_graph_destroy(mk_graph *g)
@@ -65,6 +66,9 @@ cdef extern from "fleet_mk.h" nogil:
     int mk_set_host_batch(mk_graph *g, const int32_t *host_words, int32_t *device_words, int64_t words, int64_t *host_tokens)
     int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest)
     int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2)
+    int mk_set_more_batches(mk_graph *g, int64_t words)
+    int mk_hold_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2)
+    int mk_enqueue_held(mk_graph *g, void *stream)
     int mk_wait(mk_graph *g, void *stream, int *finished_out)
     int mk_run_once(mk_graph *g, void *stream, int num_tokens, const int32_t *tok_slot, const int32_t *tok_pos, const int32_t *tok_first)
     int mk_repack_weights(mk_graph *g)

@@ -1097,9 +1097,20 @@ class PersistentKernel:
         self._g.set_host_batch(host_words.data_ptr(), device_words.data_ptr(), min(len(host_words), len(device_words)), host_tokens.data_ptr() if host_tokens is not None else None)
         self._host_batch = host_words, device_words, host_tokens
 
-    def enqueue_batches(self, host_words: int, second: int, second_words: int, default_stream=None):
-        """Two batches whose logits and sampled tokens nobody reads, as one launch; the second is described from word `second` on."""
-        self._g.enqueue_batches(self._stream_ptr(default_stream), host_words, second, second_words)
+    def attach_more_batches(self, words: int):
+        """What attach_host_batch named goes on for `words` more words, in both places (of tensors that the caller keeps)."""
+        self._g.set_more_batches(words)
+
+    def enqueue_batches(self, host_words: int, second: int, second_words: int, default_stream=None, at: int = 0, hold: bool = False):
+        """Two batches whose logits and sampled tokens nobody reads, as one launch; the second is described from word `second` on.  hold: they wait for the
+        next such call and run in its launch, in front of its batches (stats()["portions_together"] of them at most); the descriptions of each call are
+        then in words of their own, from word `at` on."""
+        if hold or at:
+            self._g.hold_batches(at, host_words, second, second_words)
+            if not hold:
+                self._g.enqueue_held(self._stream_ptr(default_stream))
+        else:
+            self._g.enqueue_batches(self._stream_ptr(default_stream), host_words, second, second_words)
 
     def enqueue_batch(self, host_words: int, default_stream=None):
         self._g.enqueue_batch(self._stream_ptr(default_stream), host_words, False)

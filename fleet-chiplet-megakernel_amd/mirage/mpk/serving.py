@@ -17,6 +17,9 @@ import torch
 from .mpk import MPK, MPKMetadata
 
 
+MAX_TOGETHER = 8  # passes of which no row is wanted that may be one launch (as many as the kernels run together)
+
+
 class PagePool:
     """Free list of cache pages (or state slots).  What is given back is handed out again first."""
 
@@ -51,8 +54,12 @@ class ServingSession:
     # device once
     _host = _dev = _sampled = None
     _fetched = False
-    # two passes of which no row is wanted may be one launch (enqueue_batches): word the second one's description begins at, 0: not in this graph
+    # two passes of which no row is wanted may be one launch (enqueue_batches): word the second one's description begins at, 0: not in this graph.  Or
+    # more of them, _together at most, each two with descriptions _apart words behind those of the two in front (in _words: _host is where those begin)
     _second = 0
+    _together = 2
+    _apart = 0
+    _words = _every = None
     _view = None  # of the logits
     # rows that nobody reads go into passes of their own, in front (see step).  Which rows share a pass decides in which order attention, experts and linears
     # of few rows add, so that 16-bit results depend, in rounding, on the rows that are wanted; 32-bit sessions keep the rows in order, and their results
@@ -88,7 +95,9 @@ class ServingSession:
         R = max_requests
         words = 2 * max_rows + 4 * R + 2 + pages
         second = (words + 1) // 2 * 2
-        dev = torch.zeros(second + words, dtype=torch.int32, device=device)
+        apart = second + second
+        every = torch.zeros(MAX_TOGETHER // 2 * apart, dtype=torch.int32, device=device)
+        dev = every[:second + words]
         ids, block = dev[:2 * max_rows].view(torch.int64).view(max_rows, 1), dev[2 * max_rows:words]
         qo, kv, last, slots, idx = block.split([R + 1, R + 1, R, R, pages])
         meta = MPKMetadata(mode="online_notoken", max_seq_length=max(2, max_seq), max_num_batched_requests=R, max_num_batched_tokens=max_rows, max_num_pages=pages,
@@ -98,11 +107,15 @@ class ServingSession:
         mpk = MPK(meta)
         mpk.build()
         session = ServingSession(mpk)
-        host = torch.empty(2 * max_rows + len(dev), dtype=torch.int32, pin_memory=True)
-        session._sampled, session._host, session._dev = host[:2 * max_rows].view(torch.int64), host[2 * max_rows:], dev
+        host = torch.empty(2 * max_rows + len(every), dtype=torch.int32, pin_memory=True)
+        session._sampled, session._words = host[:2 * max_rows].view(torch.int64), host[2 * max_rows:]
+        session._host, session._dev = session._words[:len(dev)], dev
         mpk.persistent_kernel.attach_host_batch(session._host, dev, session._sampled)
         session._fetched = True
-        session._second = second if mpk.persistent_kernel.stats()["paired_portions"] else 0
+        stats = mpk.persistent_kernel.stats()
+        if stats["paired_portions"]:
+            session._second, session._apart, session._together, session._every = second, apart, min(MAX_TOGETHER, stats["portions_together"]), every
+            mpk.persistent_kernel.attach_more_batches(len(every) - len(dev))
         return session
 
     # ------------------------------------------------------------------ steps
@@ -167,16 +180,21 @@ class ServingSession:
             if not batch:
                 break
             if unread and self._second and self._fetched and self.mpk.persistent_kernel.profiler_tensor is None:
-                then = list(done)
-                for i, n in batch:
-                    then[i] += n
-                batch2, unread2 = next_batch(then)
-                if batch2 and unread2 and all(2 * sum(n for _, n in b) > self.max_rows for b in (batch, batch2)):
-                    self._two_passes(tokens(batch, done), tokens(batch2, then))
-                    done = then
-                    for i, n in batch2:
-                        done[i] += n
+                # (as many neighbours as run together, two by two)
+                ahead_of, then, passes = [], list(done), []
+                while batch and unread and 2 * sum(n for _, n in batch) > self.max_rows and len(passes) < self._together:
+                    passes.append(tokens(batch, then))
+                    then = list(then)
+                    for i, n in batch:
+                        then[i] += n
+                    ahead_of.append(then)
+                    batch, unread = next_batch(then)
+                pairs = len(passes) // 2
+                if pairs:
+                    self._passes(passes[:2 * pairs])
+                    done = ahead_of[2 * pairs - 1]
                     continue
+                batch, unread = next_batch(done)
             self._unread = unread
             sampled = self._pass(tokens(batch, done))
             row, wanted = 0, []
@@ -233,24 +251,29 @@ class ServingSession:
 
     def _put(self, at, ids, desc):
         """A description in pinned memory, from word `at` on; its length."""
-        n, host = 2 * self.max_rows, self._host.numpy()[at:]
+        n, host = 2 * self.max_rows, self._words.numpy()[at:]
         # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
         host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
         host[n:n + len(desc)] = desc
         return n + len(desc)
 
-    def _two_passes(self, batch, batch2):
-        """Two passes of which nobody reads logits or sampled tokens, as one launch."""
-        pk, stream = self.mpk.persistent_kernel, torch.cuda.current_stream(self._dev.device)
-        words = self._put(0, *self._describe(batch)[:2])
+    def _passes(self, batches):
+        """Passes of which nobody reads logits or sampled tokens, an even number of them, as one launch."""
+        pk, stream, words = self.mpk.persistent_kernel, torch.cuda.current_stream(self._dev.device), []
         try:
-            words2 = self._put(self._second, *self._describe(batch2)[:2])
-        except Exception:  # (out of pages, or not ids: the first pass has happened all the same)
-            pk.enqueue_ingest(default_stream=stream, host_words=words)
-            pk.wait(default_stream=stream)
-            raise
-        pk.enqueue_batches(words, self._second, words2, default_stream=stream)
-        pk.wait(default_stream=stream)
+            for i, batch in enumerate(batches):
+                words.append(self._put(i // 2 * self._apart + i % 2 * self._second, *self._describe(batch)[:2]))
+        finally:  # (out of pages, or not ids: the passes in front have happened all the same)
+            pairs = len(words) // 2
+            for p in range(pairs):
+                pk.enqueue_batches(words[2 * p], self._second, words[2 * p + 1], default_stream=stream, at=p * self._apart, hold=p + 1 < pairs)
+            if pairs:
+                pk.wait(default_stream=stream)
+            if len(words) % 2:
+                if pairs:  # (described behind the others: once more, where a pass by itself is)
+                    self._words[:words[-1]].copy_(self._words[pairs * self._apart:pairs * self._apart + words[-1]])
+                pk.enqueue_ingest(default_stream=stream, host_words=words[-1])
+                pk.wait(default_stream=stream)
 
     def _pass(self, batch):
         unread, self._unread = self._unread, False

@@ -63,8 +63,8 @@ enum mk_mode { MK_MODE_OFFLINE = 0, MK_MODE_ONLINE = 1, MK_MODE_ONLINE_NOTOKEN =
  *      does), and every tensor for which mk_tensor_releasable() returns 1 may be freed by the caller.  mk_compile fails
  *      with MK_EUNSUPPORTED if a linear weight cannot be tiled (reduction length not a multiple of 256).
  *  MK_CFG_PAIR_PORTIONS  the caller's word that no stage reads rows which the iteration it runs in has not written (token ids, caches and recurrent
- *      states apart): two portions inside prompts, which are iterations of their own otherwise, may then run as one that streams the weights
- *      once, the second over copies of the row buffers.  Results are the same bit by bit; iterations are counted, limited and timed as
+ *      states apart): up to eight portions inside prompts, which are iterations of their own otherwise, may then run as one that streams the weights
+ *      once, all but the first over copies of the row buffers.  Results are the same bit by bit; iterations are counted, limited and timed as
  *      before, and the last one of a launch runs alone.  Offline launches begin with such pairs where enough of them come first to pay for the
  *      kernel they run in, by the prompt lengths at mk_init_requests (load them before) or what the last launch left; the environment
  *      variable FLEET_MK_PAIRS_WORTH (read by mk_compile) names another number of pairs. */
@@ -185,6 +185,12 @@ int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
  * run in pairs (mk_stats.paired_portions; MK_EUNSUPPORTED otherwise); each brings at least three rows.  All index tensors of the graph, and as many
  * words again from word `second` on, lie in the device words named (MK_EINVAL). */
 int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2);
+/* More than two such batches as one launch, mk_stats.portions_together at most.  mk_set_more_batches: both places that mk_set_host_batch named go on for
+ * `words` more words.  mk_hold_batches: two batches, described from word `at` (even) and from word `at + second` on, run with the next mk_enqueue_held,
+ * behind those held so far; the first ones' `at` is 0.  mk_enqueue_held launches them and holds none from then on (neither does naming other words). */
+int mk_set_more_batches(mk_graph *g, int64_t words);
+int mk_hold_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2);
+int mk_enqueue_held(mk_graph *g, void *stream);
 /* mk_enqueue_steps for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc); it has no counterpart in the reference.  The call allocates and frees nothing, and every piece
  * of scratch its launch uses -- barrier counters, K-split partial tiles and counters, attention split-KV partials and
@@ -228,7 +234,8 @@ typedef struct mk_stats {
   int64_t packed_weight_bytes; /* device memory the handle holds for matrix-core copies of the weights (0: none) */
   int64_t row_major_weight_bytes; /* bytes of attached linear weights the handle still reads in place (0 with
                                      MK_CFG_SINGLE_WEIGHT_COPY: every linear weight lives in its tile copy only) */
-  int paired_portions;     /* 1: two portions inside prompts run as one iteration (MK_CFG_PAIR_PORTIONS) */
+  int paired_portions;     /* 1: several portions inside prompts run as one iteration (MK_CFG_PAIR_PORTIONS) */
+  int portions_together;   /* as many at most (1: one by one) */
 } mk_stats;
 int mk_get_stats(mk_graph *g, mk_stats *out);
 /* Device-side stage timing of the LAST decode iteration, as seen by virtual workgroup `workgroup`: for each stage four

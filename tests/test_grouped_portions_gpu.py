@@ -1,0 +1,149 @@
+"""More than two portions inside prompts as one iteration: the same results, bit by bit, as portions one by one, where tasks of the linears and of the attention
+end within a portion, a pair or a tile."""
+import pytest
+import torch
+
+from test_paired_portions_gpu import SHAPES, _any_pair, _kept, _model, _offline  # noqa: F401  (_any_pair: a fixture)
+
+pytestmark = pytest.mark.gpu
+
+# queries per kv head of four and eight; chunks of two, four and eight; rows of an output that are no multiple of a task's
+SHAPES.update({
+    "eight": dict(hidden_size=2048, num_q_heads=64, num_kv_heads=8, intermediate_size=6144),
+    "odd": dict(hidden_size=4096, num_q_heads=24, num_kv_heads=6, intermediate_size=5120),
+})
+
+
+@pytest.mark.parametrize("name,lengths,B,portion,R", [
+    ("wide", (64 * 9 + 5,), 64, 64, 1), ("wide", (64 * 16 + 1,), 64, 64, 1), ("eight", (64 * 7 + 40,), 64, 64, 1), ("long", (64 * 6 + 9,), 64, 64, 1), ("narrow", (64 * 5 + 33,), 64, 64, 1),
+    ("odd", (64 * 8 + 17,), 64, 64, 1), ("wide", (300, 290, 280, 270), 64, 20, 4), ("wide", (90,) * 12, 64, 9, 12), ("mixed", (50 * 7 + 3, 50 * 5), 50, 50, 2), ("experts", (64 * 8 + 30,), 64, 64, 1),
+    ("wide", (33 * 7 + 2,), 33, 33, 1)])
+def test_offline(name, lengths, B, portion, R):
+    _offline(name, lengths, B, portion, 1000, R)
+
+
+@pytest.mark.parametrize("steps", [4, 6, 9])
+def test_launches_that_end_inside(steps):
+    """The last iteration of a launch runs alone, whatever could run beside it."""
+    _offline("wide", (64 * 12 + 3,), 64, 64, steps, 1)
+
+
+def test_pages_that_hold_no_whole_tile():
+    """Pages of four and of twenty-four positions: tiles of sixteen reach into others, and no page is a power of two."""
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    shape = Qwen3Shape(head_dim=128, num_layers=2, vocab_size=512, **SHAPES["wide"])
+    w, prompt = random_weights(shape, seed=2), torch.randint(0, 512, (64 * 6 + 11,), generator=torch.Generator().manual_seed(5))
+    for page in (4, 24):
+        outs = []
+        for pairs in (True, False):
+            dec = Qwen3Decoder(shape, w, max_num_batched_tokens=64, max_num_batched_requests=1, max_seq_length=400, page_size=page, eos_token_id=0x7FFFFFFF, max_tokens_per_request=64, pair_portions=pairs)
+            dec.load_prompts([prompt])
+            dec.mpk.run_steps(7)
+            outs.append([t.clone().cpu() for t in (dec.logits()[:11], dec.k_cache, dec.v_cache)])
+            dec.mpk.finalize()
+        assert all(torch.equal(a, b) for a, b in zip(*outs)), page
+
+
+def test_values_that_are_not_finite():
+    """An infinity in a row of values reaches the positions that see it and no others, in whichever portion they are."""
+    from demo_qwen3 import Qwen3Decoder, Qwen3Shape, random_weights
+    shape = Qwen3Shape(head_dim=128, num_layers=1, vocab_size=512, **SHAPES["wide"])
+    w, prompt = random_weights(shape, seed=2), torch.randint(0, 511, (64 * 4 + 9,), generator=torch.Generator().manual_seed(5))
+    w["embed"][511] = float("inf")
+    prompt[150] = 511
+    outs = []
+    for pairs in (True, False):
+        dec = Qwen3Decoder(shape, w, max_num_batched_tokens=64, max_num_batched_requests=1, max_seq_length=280, page_size=16, eos_token_id=0x7FFFFFFF, max_tokens_per_request=64, pair_portions=pairs)
+        dec.load_prompts([prompt])
+        dec.mpk.run_steps(5)
+        outs.append([t.clone().cpu().view(torch.int16) for t in (dec.k_cache, dec.v_cache)])
+        dec.mpk.finalize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("family", ["suborax", "dodonex", "bukatar", "vizonex"])
+def test_session(family):
+    """As many passes in a launch as run together, prompts of one token among them, and portions in which every request brings one row."""
+    from mirage.mpk import ServingSession
+    model, g = _model(family), torch.Generator().manual_seed(9)
+    lengths = (70, 1, 2, 3) + (2,) * 40 + (500, 330)
+    prompts = [torch.randint(0, 1000, (n,), generator=g).tolist() for n in lengths]
+    outs = []
+    for together in (8, 4, 0):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 64, max_requests=48, max_seq_length=512)
+        s._second, s._together, held = s._second if together else 0, together, []
+        run = s.mpk.persistent_kernel.enqueue_batches
+        s.mpk.persistent_kernel.enqueue_batches = lambda *a, **k: (held.append(k["hold"]), run(*a, **k))
+        out = [s.step(list(enumerate(prompts)), [[n - 1] for n in lengths])]
+        out += [s.step([(r, [3 + i]) for r in range(len(lengths))], [[0]] * len(lengths)) for i in range(2)]
+        assert any(held) if together == 8 else True
+        outs.append([(lg.cpu(), greedy) for lg, greedy in out])
+        s.finalize()
+    for other in outs[:2]:
+        for (a, ga), (b, gb) in zip(other, outs[2]):
+            assert torch.isfinite(a).all() and torch.equal(a, b) and ga == gb
+
+
+def test_portions_of_single_rows():
+    """Portions in which every request brings one row append keys and values in the attention itself, beside portions whose rows are prepared ahead of it."""
+    from mirage.mpk import ServingSession
+    model, outs = _model("suborax"), []
+    for grouped in (True, False):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 64, max_requests=40, max_seq_length=512)
+        passes = [[(r, [r + 1]) for r in range(40)], [(0, list(range(50)))], [(r, [r + 7]) for r in range(40)], [(1, list(range(30))), (2, list(range(30)))]]
+        if grouped:
+            s._passes(passes)
+        else:
+            for p in passes:
+                s._unread = True
+                s._pass(p)
+        outs.append([c.clone().cpu() for c in s.mpk.model_builder.k_cache + s.mpk.model_builder.v_cache] + [s.step([(0, [5]), (1, [6]), (3, [7])], [[0]] * 3)[0].cpu()])
+        s.finalize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_batches_that_do_not_fit():
+    from mirage import _capi
+    from mirage.mpk import ServingSession
+    s = ServingSession.open(model_config=_model("suborax"), max_tokens=1024, max_requests=2, max_seq_length=512)
+    pk, at, apart = s.mpk.persistent_kernel, s._second, s._apart
+    assert s._together == pk.stats()["portions_together"] == 8
+    with pytest.raises(_capi.MkError, match="from word 0 on"):
+        pk.enqueue_batches(4, at, 4, at=apart, hold=True)
+    with pytest.raises(_capi.MkError, match="no batches are held"):
+        pk._g.enqueue_held(pk._stream_ptr(None))
+    words = [s._put(i // 2 * apart + i % 2 * at, *s._describe([("a", list(range(64)))])[:2]) for i in range(8)]
+    for p in range(4):
+        pk.enqueue_batches(words[2 * p], at, words[2 * p + 1], at=p * apart, hold=True)
+    with pytest.raises(_capi.MkError, match="8 batches together"):
+        pk.enqueue_batches(4, at, 4, at=apart, hold=True)
+    with pytest.raises(_capi.MkError, match="mk_set_host_batch named"):
+        pk.enqueue_batches(4, at, 4, at=4 * apart, hold=True)
+    pk._g.enqueue_held(pk._stream_ptr(None))
+    pk.wait()
+    assert pk.stats()["iterations"] == 8
+    cache = [c.clone() for c in s.mpk.model_builder.k_cache]
+    for rows in ((64, 64, 64, 2), (2, 64, 64, 64), (64, 64, 2, 64)):  # (one too small: nothing runs)
+        s.end("b")
+        words = [s._put(i // 2 * apart + i % 2 * at, *s._describe([("b", list(range(n)))])[:2]) for i, n in enumerate(rows)]
+        pk.enqueue_batches(words[0], at, words[1], hold=True)
+        pk.enqueue_batches(words[2], at, words[3], at=apart)
+        with pytest.raises(_capi.MkError, match="fewer than three rows"):
+            pk.wait()
+    assert all(torch.equal(a, b) for a, b in zip(cache, s.mpk.model_builder.k_cache))
+    s.finalize()
+
+
+def test_out_of_pages_behind_some_passes():
+    """What has been described runs, then the error comes; what the requests have in the cache is what ran."""
+    from mirage.mpk import ServingSession
+    model, outs = _model("suborax"), []
+    for grouped in (True, False):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 7, max_requests=2, max_seq_length=448)
+        if not grouped:
+            s._second = 0
+        with pytest.raises(RuntimeError, match="out of cache pages"):
+            s.step([(r, [i % 900 for i in range(300)]) for r in "ab"])
+        outs.append([c.clone().cpu() for c in s.mpk.model_builder.k_cache] + [torch.tensor([r.length for r in s.requests.values()])])
+        s.finalize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
