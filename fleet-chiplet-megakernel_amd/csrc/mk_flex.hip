@@ -227,6 +227,76 @@ __device__ __forceinline__ void stage_fx_addnorm(CStage &st, Ctx &c, int M, char
   else stage_fx_addnorm_t<E, 12>(st, c, M, smem);
 }
 
+#if MK_PAIR
+// The rows of several portions, two of them in flight: see norm_group_rows.
+template <typename E, int NS>
+__device__ __forceinline__ void fx_addnorm_group(Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, char *smem) {
+  CStage &st = mk_portion_stages(rt, 0)[s];
+  const int tid = c.tid, n4 = st.n / 4;
+  float *red = (float *)smem;
+  const f32x4 *w4 = (const f32x4 *)st.norm_w;
+  f32x4 g[NS];
+#pragma unroll
+  for (int j = 0; j < NS; j++) g[j] = w4[fx_quad_at(c, 0, j, n4)];
+  barrier_wait(c);
+  const int dS = c.defer_S, total = group_rows(portions, sh_rows);
+  c.defer_S = 0;
+  for (int i = row_item(c); i < total; i += 2 * c.G) {
+    GroupRow r[2];
+    f32x4 x[2][NS], v[2][NS];
+#pragma unroll
+    for (int z = 0; z < 2; z++) {
+      r[z] = group_row(i + z * c.G, portions, sh_rows);
+      CStage &sp = mk_portion_stages(rt, r[z].portion)[s];
+      const auto row = dev_rows((const float *)sp.res + (size_t)r[z].row * st.ld_res);
+#pragma unroll
+      for (int j = 0; j < NS; j++) x[z][j] = __builtin_bit_cast(f32x4, ldc_16B(row, 16 * fx_quad_at(c, 0, j, n4)));
+      if (dS) {
+#pragma unroll
+        for (int j = 0; j < NS; j += 4) fx_addnorm_slices(c, dS, r[z].portion * MK_MAX_TOKENS + r[z].row, j * MK_THREADS, n4, v[z] + j);
+      } else {
+#pragma unroll
+        for (int j = 0; j < NS; j++) v[z][j] = sp.in ? fx_ldc_quad((const E *)sp.in + (size_t)r[z].row * st.ld_in + 4 * fx_quad_at(c, 0, j, n4)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    float ss[2] = {0.f, 0.f};
+#pragma unroll
+    for (int z = 0; z < 2; z++)
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[z][j][e] = fmaf(st.alpha, x[z][j][e], v[z][j][e]);
+          ss[z] += tid + j * MK_THREADS < n4 ? v[z][j][e] * v[z][j][e] : 0.f;
+        }
+    block_sums(ss, red);
+#pragma unroll
+    for (int z = 0; z < 2; z++) {
+      const float f = 1.f / sqrtf(ss[z] / (float)st.k + st.eps);
+      CStage &sp = mk_portion_stages(rt, r[z].portion)[s];
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+        if (r[z].valid && tid + j * MK_THREADS < n4) {
+          const int q = tid + j * MK_THREADS;
+          f32x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; e++) o[e] = (v[z][j][e] * f) * (st.w_offset + g[j][e]);
+          if (sp.out2) fx_stc_quad((float *)sp.out2 + (size_t)r[z].row * st.ld_out2 + 4 * q, o);
+          fx_stc_quad((E *)sp.out + (size_t)r[z].row * st.ld_out + 4 * q, o);
+        }
+    }
+    __syncthreads();
+  }
+  c.wrote_through = true;
+}
+template <typename E>
+__device__ __forceinline__ void stage_fx_addnorm_group(CStage &st, Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, char *smem) {
+  if (st.n <= 4 * 4 * MK_THREADS) fx_addnorm_group<E, 4>(c, rt, s, portions, sh_rows, smem);
+  else if (st.n <= 8 * 4 * MK_THREADS) fx_addnorm_group<E, 8>(c, rt, s, portions, sh_rows, smem);
+  else fx_addnorm_group<E, 12>(c, rt, s, portions, sh_rows, smem);
+}
+#endif
+
 // ----------------------------------------------------------------------------- head rows
 // Where the q/k/v rows of an attention stage come from: the linear's output, or its unsummed K-slice partials.
 template <typename E> struct FxRows {

@@ -15,6 +15,35 @@ __device__ __forceinline__ void mk_portion_rows(const MkRuntime &rt, int *tok, i
   tok[3 * MK_MAX_TOKENS + t] = (rt.batch_n ? rt.batch_at[portion] : 0) + ldc_i32(&rt.kv_indptr[slot]);
 }
 
+// Positions and first page-table entries of all portions' tokens (first rows as well, if somewhere), MK_MAX_TOKENS a portion, in LDS.
+__device__ __forceinline__ void group_tokens(const MkRuntime &rt, int portions, const int *sh_rows, int *pos, int *pages, int *first = nullptr) {
+  constexpr int N = MK_GROUP * MK_MAX_TOKENS / MK_THREADS;
+  int x[N], slot[N], f[N];
+  auto there = [&](int j) {
+    const int i = threadIdx.x + j * MK_THREADS;
+    return i < portions * MK_MAX_TOKENS && (i & (MK_MAX_TOKENS - 1)) < sh_rows[i / MK_MAX_TOKENS];
+  };
+  // (each of the three together: one token behind the other is four trips to memory instead of two)
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int i = there(j) ? threadIdx.x + j * MK_THREADS : 0;
+    x[j] = ldc_i32(&rt.tok_pos[i]);
+    slot[j] = ldc_i32(&rt.tok_slot[i]);
+    f[j] = first ? ldc_i32(&rt.tok_first[i]) : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < N; j++) slot[j] = ldc_i32(&rt.kv_indptr[slot[j]]);
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int i = threadIdx.x + j * MK_THREADS;
+    if (!there(j)) continue;
+    pos[i] = x[j];
+    pages[i] = (rt.batch_n ? rt.batch_at[i / MK_MAX_TOKENS] : 0) + slot[j];
+    if (first) first[i] = f[j];
+  }
+  __syncthreads();
+}
+
 // 16 bytes of every lane, `off` bytes behind a uniform address, straight to LDS: lane l's land at byte `lds` + 16 l.  In assembly, as the compiler waits for all
 // such requests of its own in front of every read of LDS, whichever buffer that reads: the ring of weights ran dry at every pass.  Whoever requests rows
 // waits for them by count.
@@ -239,21 +268,210 @@ __device__ __forceinline__ void stage_linear_group(CStage &st, Ctx &c, const MkR
   c.wrote_through = true;
 }
 
+// ---- norms of several portions' rows (MK_PAIR_BOTH on a NORM or FX_ADDNORM stage)
+//
+// The rows of all portions, one portion's behind the other's, are dealt round the dies as one portion's are; a workgroup has two in flight, whose sums over it
+// are taken together.  Bound by the barrier and by round trips: 512 rows of 4096 values from four slices, portion by portion, a row at a time, 20 us, now 13.
+struct GroupRow {
+  int portion, row;
+  bool valid;
+};
+// Row i of all (the last one, not valid, where there are fewer).
+__device__ __forceinline__ GroupRow group_row(int i, int portions, const int *sh_rows) {
+  int p = 0;
+  while (p + 1 < portions) {
+    const int M = __builtin_amdgcn_readfirstlane(sh_rows[p]);
+    if (i < M) break;
+    i -= M;
+    p++;
+  }
+  const int last = __builtin_amdgcn_readfirstlane(sh_rows[p]) - 1;
+  return {p, min(i, last), i <= last};
+}
+__device__ __forceinline__ int group_rows(int portions, const int *sh_rows) {
+  int n = 0;
+  for (int p = 0; p < portions; p++) n += __builtin_amdgcn_readfirstlane(sh_rows[p]);
+  return n;
+}
+// Sums over the workgroup of one value a thread, of two rows (see block_sum).
+__device__ __forceinline__ void block_sums(float (&v)[2], float *red) {
+  v[0] = wave_sum(v[0]);
+  v[1] = wave_sum(v[1]);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = v[0];
+    red[4 + (threadIdx.x >> 6)] = v[1];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int z = 0; z < 2; z++) v[z] = red[4 * z] + red[4 * z + 1] + red[4 * z + 2] + red[4 * z + 3];
+}
+// Residual rows of the linear that left its sum, of a portion.
+__device__ __forceinline__ const void *group_residual(const Ctx &c, const MkRuntime &rt, int portion) {
+  CStage &sum = mk_portion_stages(rt, portion)[c.defer_stage];
+  return sum.flags & MK_F_RES ? sum.res : nullptr;
+}
+template <int NS>
+__device__ __forceinline__ void norm_group_rows(Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, char *smem) {
+  CStage &st = mk_portion_stages(rt, 0)[s];
+  const int tid = c.tid, k8 = st.k / 8;
+  float *red = (float *)smem;
+  const u32x4 *w4 = (const u32x4 *)st.norm_w;
+  auto at = [&](int j) { return min(tid + j * MK_THREADS, k8 - 1); };
+  auto on = [&](int j) { return NS <= 2 || j * MK_THREADS < k8; };
+  u32x4 g[NS];
+#pragma unroll
+  for (int j = 0; j < NS; j++)
+    if (on(j)) g[j] = w4[at(j)];
+  barrier_wait(c);
+  const int dS = c.defer_S, total = group_rows(portions, sh_rows);
+  c.defer_S = 0;
+  auto rows = [&](auto ns) {
+    constexpr int Q = decltype(ns)::value, JB = Q && NS * Q <= 8 ? NS : 1;  // segments requested together
+    for (int i = row_item(c); i < total; i += 2 * c.G) {
+      GroupRow r[2];
+      const u32x4 *x[2], *res[2];
+      u32x4 v[2][NS];
+#pragma unroll
+      for (int z = 0; z < 2; z++) {
+        r[z] = group_row(i + z * c.G, portions, sh_rows);
+        x[z] = (const u32x4 *)((const uint16_t *)mk_portion_stages(rt, r[z].portion)[s].in + (size_t)r[z].row * st.ld_in);
+        res[z] = Q ? (const u32x4 *)group_residual(c, rt, r[z].portion) : nullptr;
+        if (res[z]) res[z] = (const u32x4 *)((const uint16_t *)res[z] + (size_t)r[z].row * c.defer_ld_res);
+      }
+      if constexpr (Q == 0) {
+#pragma unroll
+        for (int z = 0; z < 2; z++)
+#pragma unroll
+          for (int j = 0; j < NS; j++)
+            if (on(j)) v[z][j] = ldc_16B(x[z] + at(j));
+      } else {  // (the rows are still K-slice partials: see stage_norm_rows)
+#pragma unroll
+        for (int j0 = 0; j0 < NS; j0 += JB) {
+          if (!on(j0)) continue;
+          u32x4 pv[2][JB][Q][2], rv[2][JB];
+#pragma unroll
+          for (int z = 0; z < 2; z++) {
+            __amdgpu_buffer_rsrc_t part[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) part[q] = dev_rows(c.defer_part + ((size_t)q * c.defer_rows + r[z].portion * MK_MAX_TOKENS + r[z].row) * st.k);
+#pragma unroll
+            for (int j = 0; j < JB; j++) {
+              const int seg = at(j0 + j);
+              rv[z][j] = ldc_16B(res[z] ? res[z] + seg : (const u32x4 *)c.defer_part);
+#pragma unroll
+              for (int q = 0; q < Q; q++) {
+                pv[z][j][q][0] = ldc_16B(part[q], seg * 32);
+                pv[z][j][q][1] = ldc_16B(part[q], seg * 32 + 16);
+              }
+            }
+          }
+#pragma unroll
+          for (int z = 0; z < 2; z++)
+#pragma unroll
+            for (int j = 0; j < JB; j++) {
+              float a[8];
+#pragma unroll
+              for (int e = 0; e < 8; e++) a[e] = 0.f;
+#pragma unroll
+              for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                  a[e] += __uint_as_float(pv[z][j][q][0][e]);
+                  a[4 + e] += __uint_as_float(pv[z][j][q][1][e]);
+                }
+              if (res[z]) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                  a[2 * e] += bf_lo(rv[z][j][e]);
+                  a[2 * e + 1] += bf_hi(rv[z][j][e]);
+                }
+              }
+#pragma unroll
+              for (int e = 0; e < 4; e++) v[z][j0 + j][e] = pack2(a[2 * e], a[2 * e + 1]);
+            }
+        }
+#pragma unroll
+        for (int z = 0; z < 2; z++)
+#pragma unroll
+          for (int j = 0; j < NS; j++)
+            if (r[z].valid && tid + j * MK_THREADS < k8) stc_16B((u32x4 *)x[z] + tid + j * MK_THREADS, v[z][j]);
+      }
+      float ss[2] = {0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < 2; z++)
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+          if (!on(j)) continue;
+          const bool ok = tid + j * MK_THREADS < k8;
+#pragma unroll
+          for (int e = 0; e < 4; e++) ss[z] += ok ? bf_lo(v[z][j][e]) * bf_lo(v[z][j][e]) + bf_hi(v[z][j][e]) * bf_hi(v[z][j][e]) : 0.f;
+        }
+      block_sums(ss, red);
+#pragma unroll
+      for (int z = 0; z < 2; z++) {
+        const float f = rsqrtf(ss[z] / (float)st.k + st.eps);
+        u32x4 *y = (u32x4 *)((uint16_t *)mk_portion_stages(rt, r[z].portion)[s].out + (size_t)r[z].row * st.ld_out);
+#pragma unroll
+        for (int j = 0; j < NS; j++)
+          if (r[z].valid && tid + j * MK_THREADS < k8) {
+            u32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = pack2((bf_lo(v[z][j][e]) * f) * bf_lo(g[j][e]), (bf_hi(v[z][j][e]) * f) * bf_hi(g[j][e]));
+            stc_16B(y + tid + j * MK_THREADS, o);
+          }
+      }
+      __syncthreads();
+    }
+  };
+  if (dS == 0) rows(std::integral_constant<int, 0>{});
+  else if (dS == 2) rows(std::integral_constant<int, 2>{});
+  else if (dS == 4) rows(std::integral_constant<int, 4>{});
+  else rows(std::integral_constant<int, 8>{});
+  c.wrote_through = true;
+}
+__device__ __forceinline__ void stage_norm_group(CStage &st, Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, char *smem) {
+  if (st.k / 8 <= MK_THREADS) norm_group_rows<1>(c, rt, s, portions, sh_rows, smem);
+  else if (st.k / 8 <= 2 * MK_THREADS) norm_group_rows<2>(c, rt, s, portions, sh_rows, smem);
+  else norm_group_rows<6>(c, rt, s, portions, sh_rows, smem);
+}
+
 // ---- attention of several portions (MK_PAIR_BOTH on an ATTN stage), 128-wide heads
 //
 // First every portion's rows are prepared (q/k norm, rotation; keys and values into their pages, queries into a scratch), then, behind a barrier, all
 // portions' tokens are attended at once, everything out of the pages.  Portions one after the other, each with a barrier, a write-back and an invalidate in
-// between, prepared a portion's key and value rows in every unit of sixteen query rows: 512 tokens behind 1540 of 32 q / 8 kv heads 377 us as a stage, now 150.
+// between, prepared a portion's key and value rows in every unit of sixteen query rows: 512 tokens behind 1540 of 32 q / 8 kv heads 377 us as a stage, now 128.
 //
 // A task is up to two units of stage_attn_tiles, neighbouring token groups of one request and kv head: a cached tile, once in LDS, is scored against all
 // their queries, and its values, read back transposed, are packed once.  Sums are made as that stage makes them: a unit's chunks are as many and end where
 // they would for its portion alone, tile t of a chunk belongs to partial sum (t - first) mod 4, and those are merged in their order; as the chunks of the
 // units begin at tiles of their own, a wavefront takes the tiles w, w + 4, ... of the request and tells each unit's sum which one it is in the end.
-// (Four units a task: their queries and sums leave no registers for the tile, 180 us.)  Bound by one wavefront's chain through a tile: operands out of LDS,
-// scores, weights, products.
+// (Four units a task: their queries and sums leave no registers for the tile, 180 us.)  Bound by what a wavefront issues for a tile of sixteen positions and two units, about 1 us: scores,
+// 16 exponentials, 64 sums scaled, weights in two terms, products.  (512 tokens alone, us behind 0 / 512 / 1536 / 3072 positions: 72 / 104 / 162 / 231 with the sums
+// among the accumulation registers, scaled only where a maximum moved, and heads of a kv group on all dies; 62 / 80 / 114 / 168 with what add_products says, now 63 / 79 / 112 / 161.)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void lds_request(const void *p, unsigned lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off sc1" ::"v"((const MK_GLOBAL void *)(unsigned long long)p), "s"(lds) : "memory", "m0");
 }
+// o[dt] += values of 16 dims by weights of 16 columns, for the eight tiles of dims of a head: lane l holds column l & 15, dims 16 dt + 4 (l >> 4) .. + 3.  In
+// assembly, which keeps the sums among the vector registers: the compiler puts what matrix instructions write among the others in a kernel of this size, and
+// every tile scales all of them, which is two more instructions a value there (64 of them: 0.3 us a tile).  It knows nothing of how long these instructions
+// write, so the last of them is waited for.
+#define MK_PV(i, w) "v_mfma_f32_16x16x16_bf16 %" #i ", %[v" #i "], %[" #w "], %" #i "\n\t"
+#define MK_PV8(w) MK_PV(0, w) MK_PV(1, w) MK_PV(2, w) MK_PV(3, w) MK_PV(4, w) MK_PV(5, w) MK_PV(6, w) MK_PV(7, w)
+#define MK_PV_SUMS "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]), "+v"(o[6]), "+v"(o[7])
+#define MK_PV_VALUES [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [v4] "v"(v[4]), [v5] "v"(v[5]), [v6] "v"(v[6]), [v7] "v"(v[7])
+__device__ __forceinline__ void add_products(f32x4 (&o)[8], const s16x4 (&v)[8], s16x4 w) {
+  asm volatile("s_nop 3\n\t" MK_PV8(w) "s_nop 11" : MK_PV_SUMS : MK_PV_VALUES, [w] "v"(w));
+}
+__device__ __forceinline__ void add_products(f32x4 (&o)[8], const s16x4 (&v)[8], const s16x4 (&w)[2]) {
+  asm volatile("s_nop 3\n\t" MK_PV8(w0) MK_PV8(w1) "s_nop 11" : MK_PV_SUMS : MK_PV_VALUES, [w0] "v"(w[0]), [w1] "v"(w[1]));
+}
+#undef MK_PV
+#undef MK_PV8
+#undef MK_PV_SUMS
+#undef MK_PV_VALUES
 // Maximum over a column's four lanes, l & 15 + 16 i.
 __device__ __forceinline__ float lanes_max(float v) {
   const unsigned u = __float_as_uint(v);
@@ -299,23 +517,24 @@ __device__ __forceinline__ bool attn_group_tasks(CStage &st, const Ctx &c, const
 }
 template <int QPK>
 __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, const GroupTasks &g, char *smem) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  constexpr int D = 128, TG = 16 / QPK, NU = 2, RB = 3, PD = 132, GS = 1088, TS = 4 * GS, SLOT = 2 * TS;
-  constexpr int PART_OFF = MK_WAVES * RB * SLOT, PAGE_OFF = PART_OFF + MK_WAVES * SLOT;  // tiles of every wavefront; new tiles, and partial sums; page list
-  static_assert(PAGE_OFF + MK_ATTN_PAIR_PAGES * 4 <= MK_LDS_BYTES && MK_WAVES * 16 * PD * 4 <= MK_WAVES * SLOT, "attention scratch exceeds the LDS window");
+  constexpr int D = 128, TG = 16 / QPK, NU = 2, RB = 3, PD = 132, GS = 1056, TS = 4 * GS, SLOT = 2 * TS;
+  // LDS: tiles of every wavefront, and the second unit's partial sums; new tiles, and the first unit's; page lists of this task and the next; the tokens' positions,
+  // first rows and first page-table entries
+  constexpr int PART_OFF = MK_WAVES * RB * SLOT, PAGE_OFF = PART_OFF + MK_WAVES * SLOT, ROWS_OFF = PAGE_OFF + 2 * MK_ATTN_PAIR_PAGES * 4, ROWS = MK_GROUP * MK_MAX_TOKENS;
+  static_assert(ROWS_OFF + 3 * ROWS * 4 <= MK_LDS_BYTES && 16 * PD * 4 <= SLOT && NU == 2, "attention scratch exceeds the LDS window");
   static_assert(MK_MAX_TOKENS == 16 * MK_WAVES, "a new tile for every wavefront");
   const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   CStage &st = mk_portion_stages(rt, 0)[s];
   const int nkv = st.num_kv_heads, H = st.num_q_heads, ps = rt.page_size;
   const unsigned lds = (unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)smem;
-  auto base_of = [&](int p) { return rt.batch_n ? rt.batch_at[p] : 0; };
+  int *tab = (int *)(smem + ROWS_OFF);
+  group_tokens(rt, portions, sh_rows, tab, tab + 2 * ROWS, tab + ROWS);
   // ---- rows: a wavefront stays with one portion, whose tokens are a lane each; eight head rows in flight
   {
     const int W = c.vid * MK_WAVES + wave, n_waves = c.G * MK_WAVES, p = W % portions, at = W / portions, step = (n_waves - p + portions - 1) / portions;
     const int M = __builtin_amdgcn_readfirstlane(sh_rows[p]), per = H + 2 * nkv, n = M * per;
     CStage &sp = mk_portion_stages(rt, p)[s];
-    const int row = p * MK_MAX_TOKENS + min(lane, M - 1), pos = ldc_i32(&rt.tok_pos[row]), slot = ldc_i32(&rt.tok_slot[row]);
-    const int page = rt.kv_indices[base_of(p) + ldc_i32(&rt.kv_indptr[slot]) + pos / ps];
+    const int row = p * MK_MAX_TOKENS + min(lane, M - 1), pos = tab[row], page = rt.kv_indices[tab[2 * ROWS + row] + pos / ps];
     const size_t line = ((size_t)page * ps + pos % ps) * nkv;  // of the token's keys and values
     uint16_t w[2][2];
     if (st.flags & MK_F_QK_NORM) {
@@ -331,128 +550,169 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
     const size_t slice = (size_t)c.defer_rows * c.defer_n;
     const int ld_part = c.defer_n;
     c.defer_S = 0;
-    constexpr int RF = 8;
-    for (int i0 = at; i0 < n; i0 += RF * step) {
-      int tok[RF], head[RF];
-      uint16_t cs[RF], sn[RF];
-      float x[RF][2];
-#pragma unroll
-      for (int r = 0; r < RF; r++) {
+    // (the heads of a kv head and, behind them, its key and value lie together)
+    auto column = [&](int hd) { return hd < H ? (hd / QPK) * (QPK + 2) * D + hd % QPK * D : ((hd - H) % nkv) * (QPK + 2) * D + (QPK + (hd - H) / nkv) * D; };
+    // RF rows at a time, while the next RF are on their way: 24 of them a wavefront are all requested before the first is stored (a load that is waited for
+    // behind a store waits for the store as well; eight at a time, one after the other, took 21 us)
+    auto rows = [&](auto ns) {
+      constexpr int NS = decltype(ns)::value, NQ = NS ? NS : 1, RF = NS > 4 ? 4 : 12;
+      struct Rows {
+        float q[RF][2][NQ];
+        uint16_t cs[RF], sn[RF];
+      } r0, r1;
+      auto row_at = [&](int i0, int r, int &tok, int &head) {
         const int i = min(i0 + r * step, n - 1);
-        tok[r] = i / per;
-        head[r] = i - tok[r] * per;
-        if (st.flags & MK_F_ROPE) {
-          const size_t o = (size_t)__builtin_amdgcn_readlane(pos, tok[r]) * st.ld_cos;
-          cs[r] = ((const uint16_t *)st.cos_tab + o)[lane];
-          sn[r] = ((const uint16_t *)st.sin_tab + o)[lane];
-        }
-      }
-      // (the heads of a kv head and, behind them, its key and value lie together)
-      auto column = [&](int hd) { return hd < H ? (hd / QPK) * (QPK + 2) * D + hd % QPK * D : ((hd - H) % nkv) * (QPK + 2) * D + (QPK + (hd - H) / nkv) * D; };
-      auto sum = [&](auto ns) {
-        constexpr int NS = decltype(ns)::value;
-        float q[RF][2][NS];
-#pragma unroll
-        for (int r = 0; r < RF; r++) {
-          const float *pp = part + (size_t)tok[r] * ld_part + column(head[r]) + lane;
-#pragma unroll
-          for (int b = 0; b < NS; b++) {
-            q[r][0][b] = ldc_f32(pp + b * slice);
-            q[r][1][b] = ldc_f32(pp + b * slice + 64);
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < RF; r++)
-#pragma unroll
-          for (int e = 0; e < 2; e++) {
-            float v = 0.f;
-#pragma unroll
-            for (int b = 0; b < NS; b++) v += q[r][e][b];
-            x[r][e] = bfround(v);
-          }
+        tok = i / per;
+        head = i - tok * per;
       };
-      if (S == 0) {
-        uint16_t q[RF][2];
+      auto request = [&](int i0, Rows &w) {
 #pragma unroll
         for (int r = 0; r < RF; r++) {
-          const uint16_t *pp = (const uint16_t *)sp.in + (size_t)tok[r] * sp.ld_in + column(head[r]) + lane;
-          q[r][0] = ldc_u16(pp);
-          q[r][1] = ldc_u16(pp + 64);
-        }
+          int tok, head;
+          row_at(i0, r, tok, head);
+          if constexpr (NS == 0) {
+            const uint16_t *pp = (const uint16_t *)sp.in + (size_t)tok * sp.ld_in + column(head) + lane;
+            w.q[r][0][0] = bf2f(ldc_u16(pp));
+            w.q[r][1][0] = bf2f(ldc_u16(pp + 64));
+          } else {
+            const float *pp = part + (size_t)tok * ld_part + column(head) + lane;
 #pragma unroll
-        for (int r = 0; r < RF; r++) {
-          x[r][0] = bf2f(q[r][0]);
-          x[r][1] = bf2f(q[r][1]);
-        }
-      } else if (S == 2) {
-        sum(std::integral_constant<int, 2>{});
-      } else if (S == 4) {
-        sum(std::integral_constant<int, 4>{});
-      } else {
-        sum(std::integral_constant<int, 8>{});
-      }
-#pragma unroll
-      for (int r = 0; r < RF; r++) {
-        if (i0 + r * step >= n) break;
-        float x0 = x[r][0], x1 = x[r][1];
-        const int kind = head[r] < H ? 0 : 1 + (head[r] - H) / nkv, h = (head[r] - H) % nkv;
-        if (S) {  // (what the linear would have stored)
-          uint16_t *d = (uint16_t *)sp.in + (size_t)tok[r] * sp.ld_in + column(head[r]);
-          d[lane] = (uint16_t)f2bf(x0);
-          d[lane + 64] = (uint16_t)f2bf(x1);
-        }
-        if (kind < 2) {
-          if (st.flags & MK_F_QK_NORM) {
-            const float ss = wave_sum(x0 * x0 + x1 * x1);
-            const float f = rsqrtf(ss * (1.f / 128.f) + st.eps);
-            x0 = bfround((x0 * f) * bf2f(kind ? w[1][0] : w[0][0]));
-            x1 = bfround((x1 * f) * bf2f(kind ? w[1][1] : w[0][1]));
+            for (int b = 0; b < NS; b++) {
+              w.q[r][0][b] = ldc_f32(pp + b * slice);
+              w.q[r][1][b] = ldc_f32(pp + b * slice + 64);
+            }
           }
+          const size_t o = st.flags & MK_F_ROPE ? (size_t)__builtin_amdgcn_readlane(pos, tok) * st.ld_cos : 0;
           if (st.flags & MK_F_ROPE) {
-            const float c_ = bf2f(cs[r]), s_ = bf2f(sn[r]);
-            const float y0 = x0 * c_ - x1 * s_;
-            const float y1 = x0 * s_ + x1 * c_;
-            x0 = y0;
-            x1 = y1;
+            w.cs[r] = ((const uint16_t *)st.cos_tab + o)[lane];
+            w.sn[r] = ((const uint16_t *)st.sin_tab + o)[lane];
           }
         }
-        const size_t at_line = ((size_t)(unsigned)__builtin_amdgcn_readlane((int)line, tok[r]) | (size_t)(unsigned)__builtin_amdgcn_readlane((int)(line >> 32), tok[r]) << 32) + h;
-        uint16_t *d = kind == 0 ? rt.group_q + ((size_t)(p * MK_MAX_TOKENS + tok[r]) * H + head[r]) * D : (uint16_t *)(kind == 1 ? st.k_cache : st.v_cache) + at_line * D;
-        stc_u16(d + lane, (uint16_t)f2bf(x0));
-        stc_u16(d + lane + 64, (uint16_t)f2bf(x1));
-        if (kind == 0 && sp.q_ws) {
-          uint16_t *q = (uint16_t *)sp.q_ws + (size_t)tok[r] * sp.ld_qws + (size_t)head[r] * D;
-          q[lane] = (uint16_t)f2bf(x0);
-          q[lane + 64] = (uint16_t)f2bf(x1);
+      };
+      auto finish = [&](int i0, const Rows &in) {
+#pragma unroll
+        for (int r = 0; r < RF; r++) {
+          if (i0 + r * step >= n) break;
+          int tok, head;
+          row_at(i0, r, tok, head);
+          float x0 = in.q[r][0][0], x1 = in.q[r][1][0];
+          const int kind = head < H ? 0 : 1 + (head - H) / nkv, h = (head - H) % nkv;
+          if constexpr (NS > 0) {
+            x0 = x1 = 0.f;
+#pragma unroll
+            for (int b = 0; b < NS; b++) {
+              x0 += in.q[r][0][b];
+              x1 += in.q[r][1][b];
+            }
+            x0 = bfround(x0);
+            x1 = bfround(x1);
+            uint16_t *d = (uint16_t *)sp.in + (size_t)tok * sp.ld_in + column(head);  // (what the linear would have stored)
+            d[lane] = (uint16_t)f2bf(x0);
+            d[lane + 64] = (uint16_t)f2bf(x1);
+          }
+          if (kind < 2) {
+            if (st.flags & MK_F_QK_NORM) {
+              const float ss = wave_sum(x0 * x0 + x1 * x1);
+              const float f = rsqrtf(ss * (1.f / 128.f) + st.eps);
+              x0 = bfround((x0 * f) * bf2f(kind ? w[1][0] : w[0][0]));
+              x1 = bfround((x1 * f) * bf2f(kind ? w[1][1] : w[0][1]));
+            }
+            if (st.flags & MK_F_ROPE) {
+              const float c_ = bf2f(in.cs[r]), s_ = bf2f(in.sn[r]);
+              const float y0 = x0 * c_ - x1 * s_;
+              const float y1 = x0 * s_ + x1 * c_;
+              x0 = y0;
+              x1 = y1;
+            }
+          }
+          const size_t at_line = ((size_t)(unsigned)__builtin_amdgcn_readlane((int)line, tok) | (size_t)(unsigned)__builtin_amdgcn_readlane((int)(line >> 32), tok) << 32) + h;
+          uint16_t *d = kind == 0 ? rt.group_q + ((size_t)(p * MK_MAX_TOKENS + tok) * H + head) * D : (uint16_t *)(kind == 1 ? st.k_cache : st.v_cache) + at_line * D;
+          stc_u16(d + lane, (uint16_t)f2bf(x0));
+          stc_u16(d + lane + 64, (uint16_t)f2bf(x1));
+          if (kind == 0 && sp.q_ws) {
+            uint16_t *q = (uint16_t *)sp.q_ws + (size_t)tok * sp.ld_qws + (size_t)head * D;
+            q[lane] = (uint16_t)f2bf(x0);
+            q[lane + 64] = (uint16_t)f2bf(x1);
+          }
         }
+      };
+      if (at < n) request(at, r0);
+      for (int i0 = at; i0 < n; i0 += 2 * RF * step) {
+        if (i0 + RF * step < n) request(i0 + RF * step, r1);
+        __builtin_amdgcn_sched_barrier(0);
+        finish(i0, r0);
+        if (i0 + 2 * RF * step < n) request(i0 + 2 * RF * step, r0);
+        __builtin_amdgcn_sched_barrier(0);
+        finish(i0 + RF * step, r1);
       }
-    }
+    };
+    if (S == 0) rows(std::integral_constant<int, 0>{});
+    else if (S == 2) rows(std::integral_constant<int, 2>{});
+    else if (S == 4) rows(std::integral_constant<int, 4>{});
+    else rows(std::integral_constant<int, 8>{});
   }
   c.wrote_through = true;  // (what else was written nobody reads before the next iteration)
   barrier_arrive(c);
   // ---- tasks
   const int n_tasks = g.quads * nkv;
   if (c.vid >= n_tasks) barrier_wait(c);
-  for (int u = c.vid; u < n_tasks; u += c.G) {
-    int k = u % g.quads, p = 0;
-    const int h = u / g.quads;  // (kv head outermost: its tasks sit on neighbouring workgroups, on one die where there are eight heads)
+  // The kv heads of the same tokens are neighbours, on one die: rows of one head lie two kilobytes apart, so that a die that reads no other's uses two of the
+  // sixteen channels of its cache.  Every other round takes the tasks from the end, as contexts grow.
+  struct Task {
+    int h, p, t, t0, t_end, p0, n_units, new_all;  // kv head, portion, first row; first and last row of the request there, its first position; units of the portion
+    const int *pages;
+  };
+  auto decode = [&](int u, Task &a) {
+    const int round = u / c.G, r0 = round * c.G, rn = min(c.G, n_tasks - r0), turned = round & 1 ? r0 + rn - 1 - (u - r0) : u;
+    int k = turned / nkv;
+    a.h = turned - k * nkv;
+    a.p = 0;
     unsigned long long begins = g.tasks[0];
-    int n_units = __popcll(g.units[0]);
+    a.n_units = __popcll(g.units[0]);
 #pragma unroll
     for (int q = 0; q + 1 < MK_GROUP; q++)
-      if (p == q && k >= __popcll(g.tasks[q])) {
+      if (a.p == q && k >= __popcll(g.tasks[q])) {
         k -= __popcll(g.tasks[q]);
-        p = q + 1;
+        a.p = q + 1;
         begins = g.tasks[q + 1];
-        n_units = __popcll(g.units[q + 1]);
+        a.n_units = __popcll(g.units[q + 1]);
       }
     const bool mine = ((begins >> lane) & 1) && __popcll(begins & ((1ull << lane) - 1)) == k;
-    const int t = (int)__ffsll(__ballot(mine)) - 1, M = __builtin_amdgcn_readfirstlane(sh_rows[p]);
-    const int row = p * MK_MAX_TOKENS + min(lane, M - 1), my_first = ldc_i32(&rt.tok_first[row]), my_pos = ldc_i32(&rt.tok_pos[row]), my_slot = ldc_i32(&rt.tok_slot[row]);
-    const int t0 = __builtin_amdgcn_readlane(my_first, t), p0 = __builtin_amdgcn_readlane(my_pos, t0), t_end = t0 + __popcll(__ballot(lane < M && my_first == t0));
-    const int *pages = rt.kv_indices + base_of(p) + __builtin_amdgcn_readfirstlane(ldc_i32(&rt.kv_indptr[__builtin_amdgcn_readlane(my_slot, t)]));
+    a.t = (int)__ffsll(__ballot(mine)) - 1;
+    const int M = __builtin_amdgcn_readfirstlane(sh_rows[a.p]), *rows = tab + a.p * MK_MAX_TOKENS, my_first = rows[ROWS + min(lane, M - 1)];
+    a.t0 = __builtin_amdgcn_readlane(my_first, a.t);
+    a.p0 = __builtin_amdgcn_readfirstlane(rows[a.t0]);
+    a.t_end = a.t0 + __popcll(__ballot(lane < M && my_first == a.t0));
+    a.new_all = min(a.t + g.per_task * TG, a.t_end) - a.t0;
+    a.pages = rt.kv_indices + __builtin_amdgcn_readfirstlane(rows[2 * ROWS + a.t]);
+  };
+  // page lists: a task's is requested while the one in front ends
+  constexpr int PG = MK_ATTN_PAIR_PAGES / MK_THREADS;
+  int pg_next[PG];
+  auto request_pages = [&](const Task &a) {
+#pragma unroll
+    for (int i = 0; i < PG; i++)
+      if (tid + i * MK_THREADS <= (a.p0 + a.new_all - 1) / ps) pg_next[i] = a.pages[tid + i * MK_THREADS];
+  };
+  auto put_pages = [&](const Task &a, int *to) {
+#pragma unroll
+    for (int i = 0; i < PG; i++)
+      if (tid + i * MK_THREADS <= (a.p0 + a.new_all - 1) / ps) to[tid + i * MK_THREADS] = pg_next[i];
+  };
+  Task next;
+  if (c.vid < n_tasks) {
+    decode(c.vid, next);
+    request_pages(next);
+    put_pages(next, (int *)(smem + PAGE_OFF));
+    barrier_wait(c);  // every row is where it belongs
+  }
+  for (int u = c.vid, turn = 0; u < n_tasks; u += c.G, turn ^= 1) {
+    const Task a = next;
+    const bool goes_on = u + c.G < n_tasks;
+    if (goes_on) decode(u + c.G, next);
+    const int h = a.h, p = a.p, t = a.t, t0 = a.t0, p0 = a.p0, t_end = a.t_end, new_all = a.new_all;
     CStage &sp = mk_portion_stages(rt, p)[s];
-    const int cmax = max(1, min(c.G / (n_units * nkv), MK_ATTN_MAX_CHUNKS)), nt = (p0 + 15) / 16, Cd = (nt + MK_WAVES - 1) / MK_WAVES + 1, C = min(Cd, cmax);
+    const int cmax = max(1, min(c.G / (a.n_units * nkv), MK_ATTN_MAX_CHUNKS)), nt = (p0 + 15) / 16, Cd = (nt + MK_WAVES - 1) / MK_WAVES + 1, C = min(Cd, cmax);
     int n_u[NU], new_u[NU];  // tokens of a unit, positions it sees that are new in its portion
 #pragma unroll
     for (int e = 0; e < NU; e++) {
@@ -460,33 +720,31 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
       n_u[e] = e < g.per_task ? max(0, min(TG, t_end - first)) : 0;
       new_u[e] = n_u[e] ? first + n_u[e] - t0 : 0;
     }
-    const int new_all = min(t + g.per_task * TG, t_end) - t0;
     // first tile of chunk `i` of unit `e` (see stage_attn_tiles)
     auto bound = [&](int e, int i) -> int {
       if (i >= C) return nt;
-      if (C == Cd) return i < C - 1 ? (int)((long long)nt * i / (C - 1)) : nt;
+      if (C == Cd) return i < C - 1 ? nt * i / (C - 1) : nt;
       const int extra = 4 * MK_WAVES * ((n_u[e] * QPK + 2 * new_u[e] + 31) / 32 - 1), total = nt + (C > 1 ? min(extra, (nt + C - 2) / (C - 1)) : 0);
-      return min(nt, (int)((long long)total * i / C));
+      return min(nt, total * i / C);
     };
-    int *spg = (int *)(smem + PAGE_OFF);
-    lds_barrier();  // (LDS of the task in front)
-    for (int i = tid; i <= (p0 + new_all - 1) / ps; i += MK_THREADS) spg[i] = pages[i];
-    if (c.pending) barrier_wait(c);  // every row is where it belongs
-    __syncthreads();
+    const int *spg = (const int *)(smem + PAGE_OFF) + turn * MK_ATTN_PAIR_PAGES;
+    __syncthreads();  // (the page list; LDS of the task in front)
     const char *kc = (const char *)st.k_cache, *vc = (const char *)st.v_cache;
     const float scale = st.sm_scale_log2;
     // positions [q0, q0 + 16), none behind `last` (read again instead), as a tile at LDS byte b: values, then keys, each four groups of four rows.  Where pages are
     // powers of two and hold whole tiles, a whole tile of the cache is one address and its lanes' distances (new tiles begin anywhere).
     const int shift = 31 - __builtin_clz(ps);
     const bool plain = ps >= 16 && (ps & (ps - 1)) == 0;
+    // (piece c of key row r lies at c ^ 4 (r & 3): the four rows of a group would meet in the same banks)
     unsigned apart[4];
+    const unsigned kflip = (lr ^ (lg * 4)) * 16 - lr * 16;
 #pragma unroll
     for (int r = 0; r < 4; r++) apart[r] = (unsigned)((4 * r + lg) * nkv) * (2 * D) + lr * 16;
     auto load_rows = [&](int q0, int last, unsigned b) {
       if (plain && (q0 & 15) == 0 && q0 + 15 <= last) {
         const size_t at = (((size_t)__builtin_amdgcn_readfirstlane(spg[q0 >> shift]) * ps + (q0 & (ps - 1))) * nkv + h) * (2 * D);
 #pragma unroll
-        for (int r = 0; r < 4; r++) lds_request(kc + at, apart[r], b + TS + r * GS);
+        for (int r = 0; r < 4; r++) lds_request(kc + at, apart[r] + kflip, b + TS + r * GS);
 #pragma unroll
         for (int r = 0; r < 4; r++) lds_request(vc + at, apart[r], b + r * GS);
       } else {
@@ -497,7 +755,7 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
           at[r] = (((size_t)spg[pg] * ps + (pc - pg * ps)) * nkv + h) * (2 * D) + lr * 16;
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++) lds_request(kc + at[r], b + TS + r * GS);
+        for (int r = 0; r < 4; r++) lds_request(kc + at[r] + (int)kflip, b + TS + r * GS);
 #pragma unroll
         for (int r = 0; r < 4; r++) lds_request(vc + at[r], b + r * GS);
       }
@@ -543,7 +801,7 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
       // scores of units [0, N) with the keys kf of positions [q0, q0 + 16), those up to `last` (the lane's own) seen: weights in pw, the units' maxima and sums, and
       // what has been summed, brought up to them.  (All units together: one's chain of dependent instructions, the maximum over the wavefront among them, is
       // longer than what it issues.)
-      auto weigh = [&](auto first_c, auto count_c, const bf16x8 (&kf)[4], int q0, int last, float (&pw)[NU][4]) {
+      auto weigh = [&](auto first_c, auto count_c, const bf16x8 (&kf)[4], int q0, int last, float (&pw)[NU][4], auto meanwhile) {
         constexpr int E0 = decltype(first_c)::value, E1 = E0 + decltype(count_c)::value;
         f32x4 s4[NU];
         float mx[NU], alpha[NU];
@@ -553,6 +811,7 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
         for (int r = 0; r < 4; r++)
 #pragma unroll
           for (int e = E0; e < E1; e++) s4[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[r], qb[e][r], s4[e], 0, 0, 0);
+        meanwhile();
 #pragma unroll
         for (int e = E0; e < E1; e++) {
 #pragma unroll
@@ -564,7 +823,6 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
         }
 #pragma unroll
         for (int e = E0; e < E1; e++) mx[e] = lanes_max(mx[e]);
-        bool moved = false;
 #pragma unroll
         for (int e = E0; e < E1; e++) {
           const float mn = fmaxf(mrun[e], mx[e]);
@@ -573,20 +831,14 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
           for (int r = 0; r < 4; r++) pw[e][r] = __builtin_amdgcn_exp2f(pw[e][r] - mn);
           lsum[e] = lsum[e] * alpha[e] + ((pw[e][0] + pw[e][1]) + (pw[e][2] + pw[e][3]));
           mrun[e] = mn;
-          moved = moved || alpha[e] != 1.f;
         }
-        if (__ballot(moved)) {  // (uniform) some column's maximum moved: rescale what has been summed
+        // (always: among 32 columns some maximum moves at most tiles of a context of a few thousand positions)
 #pragma unroll
-          for (int e = E0; e < E1; e++) {
-            float ar[4];
+        for (int e = E0; e < E1; e++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) ar[r] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lg * 4 + r) << 2, __builtin_bit_cast(int, alpha[e])));
+          for (int dt = 0; dt < 8; dt++)
 #pragma unroll
-            for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-              for (int r = 0; r < 4; r++) o[e][dt][r] *= ar[r];
-          }
-        }
+            for (int r = 0; r < 4; r++) o[e][dt][r] *= alpha[e];
       };
       auto terms = [&](float (&pw)[4], auto &wt) {  // bf16 terms of the weights
 #pragma unroll
@@ -603,9 +855,16 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
       auto keys = [&](const char *b, bf16x8 (&kf)[4]) {
         const char *kl = b + TS + (lr >> 2) * GS + (lr & 3) * 256 + lg * 16;
 #pragma unroll
-        for (int r = 0; r < 4; r++) kf[r] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(kl + r * 64));
+        for (int r = 0; r < 4; r++) kf[r] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(kl + (r ^ (lr & 3)) * 64));
       };
-      auto pack4 = [](unsigned v0, unsigned v1, unsigned v2, unsigned v3) { return __builtin_bit_cast(s16x4, (unsigned long long)(v0 | (v1 << 16)) | ((unsigned long long)(v2 | (v3 << 16)) << 32)); };
+      // a lane's values, four positions of a dim: four rows of sixteen dims, read as eight bytes a lane, come back transposed
+      auto values_of = [&](const char *b, s16x4 (&v)[8]) {
+        typedef __attribute__((address_space(3))) s16x4 *Lds;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < 8; dt++) v[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(b + lg * GS + (lr >> 2) * 256 + (lr & 3) * 8 + dt * 32));
+        __builtin_amdgcn_sched_barrier(0);
+      };
       auto each = [&](auto f) {
         f(std::integral_constant<int, 0>{});
         f(std::integral_constant<int, 1>{});
@@ -615,67 +874,51 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
       const int t_last = hi - 1 - ((hi - 1 - wave) & (MK_WAVES - 1));
       const bool some = t_ < hi;
       auto load_tile = [&](int tt, int b) { load_rows(min(tt, t_last) * 16, p0 - 1, buf + b * SLOT); };
+      if (ci > 0) lds_barrier();  // (partial sums of the chunk in front have been read)
       if (some) {
 #pragma unroll
         for (int b = 0; b < RB - 1; b++) load_tile(t_ + b * MK_WAVES, b);
       }
       const bool with_new = ci == C - 1;
       if (with_new) {
-        lds_barrier();  // (partial sums of the chunk in front have been read)
         if (wave * 16 < new_all) load_rows(p0 + wave * 16, p0 + new_all - 1, lds + PART_OFF + wave * SLOT);
       }
-      bool more = some;
-      while (more) {
+      auto tile = [&](int b) {  // the one in buffer b
+        load_tile(t_ + (RB - 1) * MK_WAVES, (b + RB - 1) % RB);
+        static_assert(RB == 3, "the wait counts two tiles' requests");
+        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        const char *vb = smem + wave * (RB * SLOT) + b * SLOT;
+        bf16x8 kf[4];
+        keys(vb, kf);
+        s16x4 v[8];
+        auto values = [&]() { values_of(vb, v); };  // (requested behind the score products, all at once: the compiler would wait one by one)
+        auto units = [&](auto first_c, auto count_c) {
+          constexpr int E0 = decltype(first_c)::value, E1 = E0 + decltype(count_c)::value;
+          float pw[NU][4];
+          weigh(first_c, count_c, kf, t_ * 16, p0 - 1, pw, values);
+          s16x4 wt[NU][2];
 #pragma unroll
-        for (int b = 0; b < RB; b++) {
-          load_tile(t_ + (RB - 1) * MK_WAVES, (b + RB - 1) % RB);
-          static_assert(RB == 3, "the wait counts two tiles' requests");
-          asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-          if (more) {
-            const char *vb = smem + wave * (RB * SLOT) + b * SLOT;
-            bf16x8 kf[4];
-            keys(vb, kf);
-            unsigned v[8][4];
-            const char *vl = vb + lg * GS + lr * 2;
+          for (int e = E0; e < E1; e++) terms(pw[e], wt[e]);
 #pragma unroll
-            for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-              for (int r = 0; r < 4; r++) v[dt][r] = *(const uint16_t *)(vl + dt * 32 + r * 256);
-            __builtin_amdgcn_sched_barrier(0);  // (all of them in flight; else the compiler reads and waits value by value)
-            s16x4 bv[8];
-            auto pack_values = [&]() {
-#pragma unroll
-              for (int dt = 0; dt < 8; dt++) bv[dt] = pack4(v[dt][0], v[dt][1], v[dt][2], v[dt][3]);
-            };
-            auto units = [&](auto first_c, auto count_c) {
-              constexpr int E0 = decltype(first_c)::value, E1 = E0 + decltype(count_c)::value;
-              float pw[NU][4];
-              weigh(first_c, count_c, kf, t_ * 16, p0 - 1, pw);
-              pack_values();
-              s16x4 wt[NU][2];
-#pragma unroll
-              for (int e = E0; e < E1; e++) terms(pw[e], wt[e]);
-#pragma unroll
-              for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-                for (int q = 0; q < 2; q++)
-#pragma unroll
-                  for (int e = E0; e < E1; e++) o[e][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wt[e][q], bv[dt], o[e][dt], 0, 0, 0);
-            };
-            using std::integral_constant;
-            if (t_ >= all_b && t_ < all_e && n_u[NU - 1]) {
-              units(integral_constant<int, 0>{}, integral_constant<int, NU>{});
-            } else {
-              each([&](auto unit) {
-                constexpr int e = decltype(unit)::value;
-                if (t_ >= tb[e] && t_ < te[e]) units(unit, integral_constant<int, 1>{});
-              });
-            }
-            t_ += MK_WAVES;
-            more = t_ < hi;
-          }
+          for (int e = E0; e < E1; e++) add_products(o[e], v, wt[e]);
+        };
+        using std::integral_constant;
+        if (t_ >= all_b && t_ < all_e && n_u[NU - 1]) {
+          units(integral_constant<int, 0>{}, integral_constant<int, NU>{});
+        } else {
+          each([&](auto unit) {
+            constexpr int e = decltype(unit)::value;
+            if (t_ >= tb[e] && t_ < te[e]) units(unit, integral_constant<int, 1>{});
+          });
         }
+        t_ += MK_WAVES;
+      };
+      while (t_ + (RB - 1) * MK_WAVES < hi) {
+#pragma unroll
+        for (int b = 0; b < RB; b++) tile(b);
       }
+      if (t_ < hi) tile(0);
+      if (t_ < hi) tile(1);
       // ---- new tiles: one of them, at most, belongs to a wavefront's partial sum of a unit
       if (with_new) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -685,38 +928,38 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
           const int sw = (wave - tb[e]) & (MK_WAVES - 1);
           if (sw * 16 >= new_u[e]) return;
           const int q0 = p0 + sw * 16, newest = p0 + new_u[e] - 1, p_first = newest + 1 - n_u[e], n_cols = n_u[e] * QPK;
-          const char *vb = smem + PART_OFF + sw * SLOT, *vl = vb + lg * GS + lr * 2;
+          const char *vb = smem + PART_OFF + sw * SLOT;
           bf16x8 kf[4];
           keys(vb, kf);
           float pws[NU][4];
-          weigh(unit, std::integral_constant<int, 1>{}, kf, q0, p_first + min(lr, n_cols - 1) / QPK, pws);
+          s16x4 bv[8];
+          weigh(unit, std::integral_constant<int, 1>{}, kf, q0, p_first + min(lr, n_cols - 1) / QPK, pws, [&]() { values_of(vb, bv); });
           auto &pw = pws[e];
           // (rows behind the unit's newest position count as zeros)
-          s16x4 bv[8];
           unsigned top = 0;
+          const int there = min(max(newest + 1 - q0 - lg * 4, 0), 4);  // of the lane's four
+          const unsigned there0 = there >= 2 ? 0xffffffffu : there ? 0xffffu : 0u, there1 = there >= 4 ? 0xffffffffu : there == 3 ? 0xffffu : 0u;
 #pragma unroll
           for (int dt = 0; dt < 8; dt++) {
-            unsigned v[4];
+            u32x2 v = __builtin_bit_cast(u32x2, bv[dt]);
+            v[0] &= there0;
+            v[1] &= there1;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-              v[r] = q0 + lg * 4 + r <= newest ? *(const uint16_t *)(vl + dt * 32 + r * 256) : 0u;
-              top |= (v[r] & 0x7f80u) + 0x80u;
-            }
-            bv[dt] = pack4(v[0], v[1], v[2], v[3]);
+            for (int r = 0; r < 2; r++) top |= ((v[r] & 0x7f80u) + 0x80u) | (((v[r] >> 16) & 0x7f80u) + 0x80u);
+            bv[dt] = __builtin_bit_cast(s16x4, v);
           }
           if (__builtin_expect(__ballot(top & 0x8000u) != 0, 0)) {  // values that are not finite: column by column, see stage_attn_tiles
+            const bool none = lr >= n_cols;
             for (int g4 = 0; g4 < 4; g4++) {
 #pragma unroll
               for (int r4 = 0; r4 < 4; r4++) {
-                const uint16_t *v = (const uint16_t *)(vb + g4 * GS + r4 * 256) + lr;
+                const uint16_t *v = (const uint16_t *)(vb + g4 * GS + r4 * 256) + lg * 4;
+                const float wgt = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((g4 * 16 + lr) << 2, __builtin_bit_cast(int, pw[r4])));
+                const bool seen = q0 + g4 * 4 + r4 <= p_first + (none ? n_cols - 1 : lr) / QPK;
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                  const int col = lg * 4 + r;
-                  const float wgt = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((g4 * 16 + col) << 2, __builtin_bit_cast(int, pw[r4])));
-                  const bool seen = q0 + g4 * 4 + r4 <= p_first + min(col, n_cols - 1) / QPK;
+                for (int dt = 0; dt < 8; dt++)
 #pragma unroll
-                  for (int dt = 0; dt < 8; dt++) o[e][dt][r] = seen ? fmaf(wgt, bf2f(v[dt * 16]), o[e][dt][r]) : o[e][dt][r];
-                }
+                  for (int r = 0; r < 4; r++) o[e][dt][r] = seen ? fmaf(wgt, bf2f(v[dt * 16 + r]), o[e][dt][r]) : o[e][dt][r];
               }
             }
             return;
@@ -724,39 +967,40 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
           s16x4 wt[3];
           terms(pw, wt);
 #pragma unroll
-          for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-            for (int q = 0; q < 3; q++) o[e][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wt[q], bv[dt], o[e][dt], 0, 0, 0);
+          for (int q = 0; q < 3; q++) add_products(o[e], bv, wt[q]);
         });
       }
-      // ---- a unit's four partial sums, in their order, then its chunks
-      float *parts = (float *)(smem + PART_OFF);
+      // ---- a unit's four partial sums, in their order, then its chunks.  (What the tiles requested behind the end bring has landed before sums take their place.)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (with_new && goes_on) request_pages(next);
+      lds_barrier();
+      auto part_of = [&](int e, int w) { return (float *)(smem + (e ? 0 : PART_OFF) + w * SLOT); };
       each([&](auto unit) {
         constexpr int e = decltype(unit)::value;
         if (!n_u[e]) return;
-        const int sw = (wave - tb[e]) & (MK_WAVES - 1);
         float lt = lsum[e];
         lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 16) << 2, __builtin_bit_cast(int, lt)));
         lt += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, lt)));
-        lds_barrier();
-        float *part = parts + sw * 16 * PD;
+        float *part = part_of(e, (wave - tb[e]) & (MK_WAVES - 1));
         if (lg == 0) {
           part[lr * PD + D] = mrun[e];
           part[lr * PD + D + 1] = lt;
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-          for (int dt = 0; dt < 8; dt++) part[(lg * 4 + r) * PD + dt * 16 + lr] = o[e][dt][r];
-        lds_barrier();
+        for (int dt = 0; dt < 8; dt++) *(f32x4 *)(part + lr * PD + dt * 16 + lg * 4) = o[e][dt];
+      });
+      lds_barrier();
+      each([&](auto unit) {
+        constexpr int e = decltype(unit)::value;
+        if (!n_u[e]) return;
         float mx = -1e30f, ls = 0.f, os[8];
 #pragma unroll
         for (int d = 0; d < 8; d++) os[d] = 0.f;
 #pragma unroll
-        for (int w = 0; w < MK_WAVES; w++) mx = fmaxf(mx, parts[(w * 16 + mcol) * PD + D]);
+        for (int w = 0; w < MK_WAVES; w++) mx = fmaxf(mx, part_of(e, w)[mcol * PD + D]);
 #pragma unroll
         for (int w = 0; w < MK_WAVES; w++) {
-          const float *pp = parts + (w * 16 + mcol) * PD;
+          const float *pp = part_of(e, w) + mcol * PD;
           const float wgt = __builtin_amdgcn_exp2f(pp[D] - mx);
           ls += pp[D + 1] * wgt;
 #pragma unroll
@@ -776,6 +1020,7 @@ __device__ __forceinline__ void stage_attn_group(Ctx &c, const MkRuntime &rt, in
         }
       });
     }
+    if (goes_on) put_pages(next, (int *)(smem + PAGE_OFF) + (turn ^ 1) * MK_ATTN_PAIR_PAGES);
 #pragma unroll
     for (int e = 0; e < NU; e++)
       if (mcol < n_u[e] * QPK) {

@@ -2358,6 +2358,7 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
     };
     // (not a stage that may find a sum which a stage of the same run has left)
     auto first = [&](int q) { return q == i || !(g->stages[q - 1].flags & MK_F_DEFER_SUM); };
+    auto normed = [&](const MkStage &s) { return row_wise(s) && ((s.op == MK_OP_NORM && mk_norm_by_rows(s)) || s.op == MK_OP_FX_ADDNORM); };
     auto attends = [&](int q) {  // attention that may run for all portions at once
       const MkStage &s = g->stages[q];
       return s.op == MK_OP_ATTN && first(q) && (s.num_q_heads == 4 * s.num_kv_heads || s.num_q_heads == 8 * s.num_kv_heads);
@@ -2365,14 +2366,16 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
     auto alone = [&](int q) { return first(q) && (row_wise(g->stages[q]) || prepared(q) || (q + 1 < j && prepared(q + 1))); };
     for (int q = i; q < j;) {
       int e = q + 1;
-      if (attends(q)) {
+      if (first(q) && normed(g->stages[q])) {
+        prog.push_back(q | MK_PAIR_BOTH);
+      } else if (attends(q)) {
         const size_t at = prog.size();
         prog.push_back(q | MK_PAIR_BOTH);
         in_turn(q, e, false);
         prog[at] |= (unsigned)(prog.size() - at - 1) << MK_PAIR_BACK_SHIFT;
       } else {
         if (!alone(q))
-          while (e < j && !alone(e) && !attends(e)) e++;
+          while (e < j && !alone(e) && !attends(e) && !(first(e) && normed(g->stages[e]))) e++;
         in_turn(q, e, alone(q));
       }
       q = e;

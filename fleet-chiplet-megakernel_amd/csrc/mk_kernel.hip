@@ -1070,10 +1070,9 @@ __device__ __forceinline__ void stage_norm_rows(CStage &st, Ctx &c, int M, char 
   }
   c.wrote_through = true;
 }
-__device__ __forceinline__ bool norm_by_rows(CStage &st) { return (st.k & 7) == 0 && st.k / 8 <= 6 * MK_THREADS && (st.ld_in & 7) == 0 && (st.ld_out & 7) == 0; }
 __device__ __forceinline__ void stage_norm(CStage &st, Ctx &c, int M, char *smem) {
   const int k8 = st.k / 8;
-  if (norm_by_rows(st)) {
+  if (mk_norm_by_rows(st)) {
     if (k8 <= MK_THREADS) stage_norm_rows<1>(st, c, M, smem);
     else if (k8 <= 2 * MK_THREADS) stage_norm_rows<2>(st, c, M, smem);
     else stage_norm_rows<6>(st, c, M, smem);
@@ -4830,18 +4829,17 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       // (the last portion's run of a stage that nobody has waited behind yet posts the arrival for all of them; not before everybody has arrived in front: the
       // barrier counts arrivals, not workgroups)
 #define MK_LEAVE_OUT { if ((ent & MK_PAIR_ON) && !on) { barrier_wait(c); c.rows_ahead = 0; c.wrote_through = all_through; all_through = true; barrier_arrive(c); } turn(); continue; }
-      // Norms look at no tokens; and a workgroup that none of a portion's rows are dealt to need not look at the stage: 512 rows of 4096 values from four slices
-      // 35 -> 20 us.
-      const int dealt = mk_portion_stages(rt, 0)[s].op;
-      const bool rows_only = dealt == MK_OP_NORM || dealt == MK_OP_FX_ADDNORM;
       c.portion = portion;
       M = __builtin_amdgcn_readfirstlane(sh_rows[portion]);
-      if (rows_only && (ent & MK_PAIR_ON) && row_item(c) >= M && (dealt != MK_OP_NORM || norm_by_rows(mk_portion_stages(rt, 0)[s]))) {
+#if MK_HAVE_MIX
+      // (a workgroup that none of a portion's rows are dealt to need not look at the stage; rows without a summand may be dealt in parts)
+      if ((ent & MK_PAIR_ON) && mk_portion_stages(rt, 0)[s].op == MK_OP_MX_PRENORM && mk_portion_stages(rt, 0)[s].in && row_item(c) >= M) {
         c.defer_S = 0;
         if (on) c.rows_ahead = mk_rows_ahead(c.rows_ahead + M, c.G);
         MK_LEAVE_OUT;
       }
-      if (!rows_only && portion != shown) {
+#endif
+      if (portion != shown) {
         if (portion && portion != held) {
           mk_portion_rows(rt, tok + 4 * MK_MAX_TOKENS, (int)threadIdx.x, M, portion);
           held = portion;
@@ -4913,7 +4911,15 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       switch (op) {
 #if MK_HAVE_FLEX
         case MK_OP_FX_EMBED: if constexpr (FX) stage_fx_embed<E>(st, c, rt, M); break;
-        case MK_OP_FX_ADDNORM: if constexpr (FX) stage_fx_addnorm<E>(st, c, M, smem); break;
+        case MK_OP_FX_ADDNORM:
+#if MK_PAIR
+          if (ent & MK_PAIR_BOTH) {
+            if constexpr (FX) stage_fx_addnorm_group<E>(st, c, rt, s, portions, sh_rows, smem);
+            break;
+          }
+#endif
+          if constexpr (FX) stage_fx_addnorm<E>(st, c, M, smem);
+          break;
         case MK_OP_FX_PREP: if constexpr (FX) stage_fx_prep<E>(st, c, rt, M, smem); break;
         case MK_OP_FX_ATTN: if constexpr (FX) stage_fx_attn<E>(st, c, rt, M, MAXM == 1 || single, smem); break;
         case MK_OP_LINEAR_F32:
@@ -4946,7 +4952,15 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
         case MK_OP_HY_EXPERTS: stage_hy_experts<E, MAXM>(st, c, M, smem); break;
 #endif
         case MK_OP_EMBED: if constexpr (!FX) stage_embed(st, c, rt, M); break;
-        case MK_OP_NORM: if constexpr (!FX) stage_norm(st, c, M, smem); break;
+        case MK_OP_NORM:
+#if MK_PAIR
+          if (ent & MK_PAIR_BOTH) {
+            if constexpr (!FX) stage_norm_group(st, c, rt, s, portions, sh_rows, smem);
+            break;
+          }
+#endif
+          if constexpr (!FX) stage_norm(st, c, M, smem);
+          break;
         case MK_OP_LINEAR:
           if constexpr (F32) barrier_wait(c);
 #if MK_PAIR

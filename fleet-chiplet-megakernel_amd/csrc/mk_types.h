@@ -308,6 +308,10 @@ MK_HOST_DEVICE inline GroupPlan mk_group_plan(Stage &st, int G, int portions) {
   return p;
 }
 
+// NORM stages whose rows a workgroup takes in pieces of sixteen bytes, at most six a thread (others go value by value).
+template <typename Stage>
+MK_HOST_DEVICE inline bool mk_norm_by_rows(Stage &st) { return (st.k & 7) == 0 && st.k / 8 <= 6 * MK_THREADS && (st.ld_in & 7) == 0 && (st.ld_out & 7) == 0; }
+
 // Rows are dealt to G workgroups in turn.  Where those of another portion have been dealt just before, they go on with the workgroup behind the last of
 // them: `ahead` workgroups further (grids may be smaller than a portion), and the first row of the workgroup that comes `at`-th is what mk_first_row says.
 MK_HOST_DEVICE inline int mk_rows_ahead(int dealt, int G) {
@@ -376,7 +380,7 @@ struct MkSched {
 enum MkPairEntry {
   MK_PAIR_STAGE = 0xffff,
   MK_PAIR_SECOND = 1 << 16,   // for the second portion, and each one behind it
-  MK_PAIR_BOTH = 1 << 17,     // for all at once; attention (MK_OP_ATTN): where the portions allow it, and the `back` entries behind it, for one after the other, are skipped
+  MK_PAIR_BOTH = 1 << 17,     // for all at once; 128-wide attention (MK_OP_ATTN): where the portions allow it, and the `back` entries behind it, for one after the other, are skipped
   MK_PAIR_ON = 1 << 18,       // the next portion's run of this stage follows without a barrier
   MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written, here or by the stages in front, for the next portion to read: write back ...
   MK_PAIR_ACQUIRE = 1 << 20,  // ... and, no stage, drop what the caches of the dies hold
