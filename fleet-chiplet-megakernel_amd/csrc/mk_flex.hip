@@ -400,6 +400,30 @@ __device__ __forceinline__ float fx_row_squares(const E *row, int c0, int c1, in
 struct FxSpan {
   int tok, col, n;
 };
+#if MK_PAIR
+template <typename E, int R, int N>
+__device__ __forceinline__ void fx_span_loads(const FxRows<E> &rows, const FxSpan (&s)[N], int lane, FxHead<R> (&h)[N]) {
+  rows.with_slices([&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    int most = 0;
+#pragma unroll
+    for (int z = 0; z < N; z++) most = max(most, s[z].n);
+#pragma unroll
+    for (int j = 0; j < R; j += 2)
+      if (R == 2 || j * 64 < most) {
+        float q[N][2][NS ? NS : 1];
+#pragma unroll
+        for (int z = 0; z < N; z++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) rows.template request<NS>(s[z].tok, s[z].col + min((j + i) * 64 + lane, s[z].n - 1), q[z][i]);
+#pragma unroll
+        for (int z = 0; z < N; z++)
+#pragma unroll
+          for (int i = 0; i < 2; i++) h[z].x[j + i] = rows.template value<NS>(q[z][i]);
+      }
+  });
+}
+#endif
 template <typename E, int R>
 __device__ __forceinline__ void fx_span_load2(const FxRows<E> &rows, const FxSpan &s0, const FxSpan &s1, int lane, FxHead<R> &h0, FxHead<R> &h1) {
   rows.with_slices([&](auto ns) {
@@ -579,6 +603,67 @@ __device__ __forceinline__ void stage_fx_prep(CStage &st, Ctx &c, const MkRuntim
   });
   c.wrote_through = true;
 }
+
+#if MK_PAIR
+// The rows of several portions, none of which leaves its rows to the attention: a wavefront stays with one portion, whose tokens are a lane each, and has as
+// many rows in flight as registers allow (two at a time, portion by portion: six portions of 64 rows of 32 q / 8 kv heads of 128, from four slices, 30 us, now 19).
+template <typename E>
+__device__ __forceinline__ void stage_fx_prep_group(Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, char *smem) {
+  constexpr int KW = FxType<E>::KW;
+  const int lane = c.tid & 63, wave = __builtin_amdgcn_readfirstlane(c.tid >> 6), W = c.vid * MK_WAVES + wave, n_waves = c.G * MK_WAVES;
+  const int p = W % portions, first = W / portions, step = (n_waves - p + portions - 1) / portions, M = __builtin_amdgcn_readfirstlane(sh_rows[p]);
+  CStage &st = mk_portion_stages(rt, p)[s];
+  const int H = st.num_q_heads, nkv = st.num_kv_heads, D = st.head_dim, DV = st.v_dim;
+  const int nkc = (D + KW - 1) / KW, nvb = (DV + 15) / 16, ps = rt.page_size, per = H + 2 * nkv, total = M * per;
+  const int row = p * MK_MAX_TOKENS + min(lane, M - 1), my_pos = ldc_i32(&rt.tok_pos[row]);
+  const int my_page = rt.kv_indices[(rt.batch_n ? rt.batch_at[p] : 0) + ldc_i32(&rt.kv_indptr[ldc_i32(&rt.tok_slot[row])]) + my_pos / ps];
+  E *kc = (E *)st.k_cache, *vc = (E *)st.v_cache;
+  float *xs = (float *)smem + wave * MK_FX_MAX_HEAD_DIM;
+  barrier_wait(c);
+  FxRows<E> rows = fx_rows<E>(st, c);
+  if (rows.S) rows.part += (size_t)p * MK_MAX_TOKENS * rows.ldp;
+  fx_head_regs(D, DV, [&](auto regs) {
+    constexpr int R = decltype(regs)::value, N = R == 2 ? 6 : 2;
+    for (int i0 = first; i0 < total; i0 += N * step) {
+      FxHead<R> h[N];
+      FxSpan sp[N];
+#pragma unroll
+      for (int z = 0; z < N; z++) {
+        const int i = min(i0 + z * step, total - 1), t = i / per, q = i - t * per;
+        const bool head = q < H + nkv;
+        sp[z] = {t, head ? q * D : fx_value_col(st) + (q - H - nkv) * DV, head ? D : DV};
+        fx_head_tables(st, rows, sp[z], head, __builtin_amdgcn_readlane(my_pos, t), lane, h[z]);
+#if MK_HAVE_DUAL
+        if (head && (st.flags & MK_F_ROW_NORM)) {
+          const int c0 = q < H ? 0 : H * D, c1 = q < H ? H * D : (H + nkv) * D;
+          fx_row_weights(st, q * D, lane, h[z]);
+          h[z].r = 1.f / sqrtf(wave_sum(fx_row_squares<E>((const E *)st.in + (size_t)t * st.ld_in, c0, c1, lane, 64)) / (float)(c1 - c0) + st.eps);
+        }
+#endif
+      }
+      fx_span_loads<E, R, N>(rows, sp, lane, h);
+#pragma unroll
+      for (int z = 0; z < N; z++) {
+        const int i = i0 + z * step, t = sp[z].tok, q = i - t * per;
+        if (i >= total) break;
+        const int page = __builtin_amdgcn_readlane(my_page, t), pp = __builtin_amdgcn_readlane(my_pos, t) % ps;
+        if (q < H) {
+          E *to = (E *)st.q_ws + (size_t)t * st.ld_qws + (size_t)q * nkc * KW;
+          fx_head_finish(st, lane, h[z], xs, [&](int d, float v) { fx_stc(to + d, fx_round<E>(v)); });
+          for (int d = D + lane; d < nkc * KW; d += 64) fx_stc(to + d, (E)0);
+        } else if (q < H + nkv) {
+          fx_head_finish(st, lane, h[z], xs, [&](int d, float v) { fx_stc(kc + fx_k_at<E>(page, pp, ps, nkv, q - H, nkc, d), fx_round<E>(v)); });
+        } else {
+#pragma unroll
+          for (int j = 0; j < R; j++)
+            if (j * 64 + lane < DV) fx_stc(vc + fx_v_at<E>(page, pp, ps, nkv, q - H - nkv, nvb, j * 64 + lane), fx_round<E>(fx_value(h[z], j)));
+        }
+      }
+    }
+  });
+  c.wrote_through = true;
+}
+#endif
 
 // ----------------------------------------------------------------------------- attention
 __device__ __forceinline__ f32x4 fx_mma_k(uint16_t, u32x4 a, u32x4 b, f32x4 acc) {
@@ -870,21 +955,28 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
       if (kg + 1 < nkg) return;
       float sc[SUB][4];
       float tm = MK_FX_NEG;
+      auto each = [&](auto f) {
+#pragma unroll
+        for (int u_ = 0; u_ < SUB; u_++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) f(sc[u_][i], S[u_][i] * sc_row);
+      };
+      // (one branch for all values: with one at every value they follow each other)
+      if (cap > 0.f) {
+        if constexpr (sizeof(E) == 2) {
+          each([&](float &s, float x) { s = __builtin_amdgcn_exp2f(x * (2.f * LOG2E)); });
+          each([&](float &s, float x) { s = (cap * LOG2E) * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + s)); });
+        } else {
+          each([&](float &s, float x) { s = (cap * LOG2E) * tanhf(x); });
+        }
+      } else {
+        each([&](float &s, float x) { s = x * LOG2E; });
+      }
 #pragma unroll
       for (int u_ = 0; u_ < SUB; u_++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float s = S[u_][i] * sc_row;
-          if (cap > 0.f) {
-            if constexpr (sizeof(E) == 2) {
-              const float e = __builtin_amdgcn_exp2f(s * (2.f * LOG2E));
-              s = (cap * LOG2E) * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e));
-            } else {
-              s = (cap * LOG2E) * tanhf(s);
-            }
-          } else {
-            s *= LOG2E;
-          }
+          float s = sc[u_][i];
           const int at = tile * TP + u_ * 16 + lg * 4 + i;
           bool seen = at <= plim;
           if (MK_HAVE_HYB) seen = seen && (win == 0 || plim - at < win || at < keep);
@@ -1096,6 +1188,457 @@ __device__ __forceinline__ void stage_fx_attn_t(CStage &st, Ctx &c, const MkRunt
     }
   }
 }
+#if MK_PAIR
+// Four tiles of dims' sums, first with the rounded weights, then with their remainders.  In assembly, as in add_products.
+__device__ __forceinline__ void fx_add_products(f32x4 &o0, f32x4 &o1, f32x4 &o2, f32x4 &o3, u32x4 v0, u32x4 v1, u32x4 v2, u32x4 v3, u32x4 hi, u32x4 lo) {
+#define MK_PV(o, w) "v_mfma_f32_16x16x32_bf16 %" #o ", %[v" #o "], %[" #w "], %" #o "\n\t"
+  asm volatile("s_nop 3\n\t" MK_PV(0, hi) MK_PV(1, hi) MK_PV(2, hi) MK_PV(3, hi) MK_PV(0, lo) MK_PV(1, lo) MK_PV(2, lo) MK_PV(3, lo) "s_nop 11"
+               : "+v"(o0), "+v"(o1), "+v"(o2), "+v"(o3)
+               : [v0] "v"(v0), [v1] "v"(v1), [v2] "v"(v2), [v3] "v"(v3), [hi] "v"(hi), [lo] "v"(lo));
+#undef MK_PV
+}
+// Attention of several portions whose rows the prep stage has written (MK_PAIR_BOTH on a FX_ATTN stage).
+//
+// Bound by round trips, hand-overs and chains of dependent instructions: a unit of stage_fx_attn_t waits for its page entries, its queries and its first tile,
+// for each tile's maximum, then for the other chunks' workgroups and what those have stored.  Here a task is two units, neighbouring row tiles of a
+// request, whose chains cover each other over the same tiles, with all of their chunks, whose partial results stay in LDS (those behind CHUNKS in memory
+// that only this workgroup reads); pages and queries of the next task are requested while one runs, and the first tile of the next chunk or task before
+// sums are merged.  (Units whose chunks end at different tiles follow each other; few units are a task each.)  Chunks, sums and merges are those of
+// stage_fx_attn_t, in its order.  Six portions of 64 rows behind 1000 to 1500 positions, 32 q / 8 kv heads of 128: 96 us as a stage, portion by portion;
+// a unit a task 68, now 50.
+struct FxGroupRows {
+  int row[MK_GROUP];     // a lane's rows as the first token of a request in a portion; row tiles up to its own << 8, tasks << 20
+  int tiles, parts;      // of portion `lane`: row tiles; tasks of a kv head, and those of the portions in front
+  int per_task, tasks;   // units of a task at most; of all portions, a kv head
+};
+// False: another form of the stage (long heads, long page lists, or too few units: a workgroup would be alone with all chunks of one), portion by portion.
+__device__ __forceinline__ bool fx_attn_group_rows(CStage &st, const Ctx &c, const MkRuntime &rt, int portions, const int *sh_rows, FxGroupRows &g) {
+  if ((rt.max_seq + rt.page_size - 1) / rt.page_size > MK_ATTN_PAIR_PAGES || st.head_dim > st.k_tiles * FxType<uint16_t>::KW) return false;
+  const int lane = threadIdx.x & 63, qpk = st.num_q_heads / st.num_kv_heads, nvb = (st.v_dim + 15) / 16, nvs = (nvb + st.v_tiles - 1) / st.v_tiles;
+  int units = 0, begins[MK_GROUP];
+  g.tiles = 0;
+#pragma unroll
+  for (int p = 0; p < MK_GROUP; p++) begins[p] = ldc_i32(&rt.tok_first[min(p, portions - 1) * MK_MAX_TOKENS + lane]);  // (of rows that are none, looked at by nobody)
+#pragma unroll
+  for (int p = 0; p < MK_GROUP; p++) {
+    const int M = p < portions ? __builtin_amdgcn_readfirstlane(sh_rows[p]) : 0;
+    const bool first = lane < M && begins[p] == lane;
+    const unsigned long long fm = __ballot(first), later = lane < 63 ? fm >> (lane + 1) : 0ull;
+    const int n = first ? (later ? (int)__ffsll(later) : M - lane) : 0, incl = wave_incl_scan((n * qpk + 15) / 16, lane);
+    g.row[p] = n | incl << 8;
+    const int tiles = wave_bcast(incl, 63);
+    if (lane == p) g.tiles = tiles;
+    units += tiles * nvs * st.num_kv_heads;
+  }
+  g.per_task = units > c.G ? 2 : 1;
+  int parts = 0;
+#pragma unroll
+  for (int p = 0; p < MK_GROUP; p++) {
+    const int incl = wave_incl_scan((((g.row[p] & 0xff) * qpk + 15) / 16 + g.per_task - 1) / g.per_task, lane);
+    g.row[p] |= incl << 20;
+    if (lane == p) parts = wave_bcast(incl, 63) * nvs;
+  }
+  g.parts = wave_incl_scan(parts, lane);
+  g.tasks = wave_bcast(g.parts, 63);
+  return 2 * units >= c.G;
+}
+template <typename E, int KC, int VB>
+__device__ __forceinline__ void fx_attn_group(Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, const FxGroupRows &rows, char *smem) {
+  using X = FxType<E>;
+  static_assert(sizeof(E) == 2, "16-bit activations");
+  constexpr int EPC = X::EPC, KW = X::KW, TP = X::TP, SUB = X::SUB, NU = 2, ROWS = MK_GROUP * MK_MAX_TOKENS;
+  constexpr int PSTR = VB * 16 + 4, PST = VB * 16 + 32, QUADS = 16 * VB * 4, NE = QUADS / MK_THREADS, CHUNKS = 3, QMAX = KC * 64, PG = MK_ATTN_PAIR_PAGES / MK_THREADS;
+  static_assert(QUADS % MK_THREADS == 0, "a merged chunk is whole quads of all threads");
+  // LDS: query operands of this task and the next, page lists of both, the tokens' positions, first page-table entries and FxGroupRows::row, the wavefronts' sums, chunks
+  u32x4 *const q_at = (u32x4 *)smem;
+  int *const pages_at = (int *)(q_at + 2 * NU * QMAX), *const tab = pages_at + 2 * MK_ATTN_PAIR_PAGES;
+  int *const row_at = tab + 2 * ROWS;
+  float *const part = (float *)(row_at + ROWS), *const ml = part + NU * MK_WAVES * 16 * PSTR, *const chunk_ml = ml + NU * 128;
+  f32x4 *const chunk_at = (f32x4 *)(chunk_ml + NU * MK_ATTN_MAX_CHUNKS * 32);
+  static_assert((2 * NU * QMAX + NU * CHUNKS * QUADS) * 16 + (2 * MK_ATTN_PAIR_PAGES + 3 * ROWS + NU * (MK_WAVES * 16 * PSTR + 128 + MK_ATTN_MAX_CHUNKS * 32)) * 4 <= MK_LDS_BYTES, "attention scratch exceeds the LDS window");
+  const int tid = c.tid, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  CStage &st = mk_portion_stages(rt, 0)[s];
+  const int nkv = st.num_kv_heads, qpk = st.num_q_heads / nkv, D = st.head_dim, DV = st.v_dim;
+  const int nkc = (D + KW - 1) / KW, nvb = (DV + 15) / 16, nvs = (nvb + VB - 1) / VB, ps = rt.page_size;
+  const u32x4 *kc = (const u32x4 *)st.k_cache, *vc = (const u32x4 *)st.v_cache;
+  const int win = MK_HAVE_HYB ? st.window : 0, keep = MK_HAVE_HYB ? st.keep_first : 0;
+  if (wave == 0) {
+#pragma unroll
+    for (int p = 0; p < MK_GROUP; p++) row_at[p * MK_MAX_TOKENS + lane] = rows.row[p];
+  }
+  group_tokens(rt, portions, sh_rows, tab, tab + ROWS);
+  const int n_tasks = rows.tasks * nkv;
+  // Units from row r0 of a request on (its first row and position: t0, p0): query rows, none for the second where there is no such unit, and newest positions;
+  // tiles NT, those behind the first `kept` ones `gap` further on, in C chunks.  split: the units follow each other.
+  struct Task {
+    int g, vs, portion, t0, r0, p0, item, cmax, C, NT, kept, gap, n_pages, nrows[NU], newest[NU];
+    bool split;
+    const int *pages;
+  };
+  // kv head outermost, and every other round from its end (contexts differ): see stage_fx_attn_t
+  auto decode = [&](int u, int sub, Task &a) {
+    const int round0 = u / c.G * c.G, turned = (u / c.G) & 1 ? round0 + min(c.G, n_tasks - round0) - 1 - (u - round0) : u;
+    a.g = turned / rows.tasks;
+    int k = turned - a.g * rows.tasks;
+    // (looked up in a lane's registers and LDS: portions' numbers in scalar registers, and the choice among them, were spilled and fetched again for every task)
+    a.portion = __builtin_amdgcn_readfirstlane((int)__ffsll(__ballot(rows.parts > k)) - 1);
+    const int RT = wave_bcast(rows.tiles, a.portion), before = a.portion ? wave_bcast(rows.parts, a.portion - 1) : 0;
+    const int mine = row_at[a.portion * MK_MAX_TOKENS + lane], parts = (wave_bcast(rows.parts, a.portion) - before) / nvs;
+    k -= before;
+    a.vs = k / parts;
+    k -= a.vs * parts;
+    a.cmax = max(1, min(c.G / (RT * nkv * nvs), MK_ATTN_MAX_CHUNKS));
+    a.t0 = (int)__ffsll(__ballot((mine >> 20) > k)) - 1;
+    const int own = wave_bcast(mine, a.t0), n_rows = (own & 0xff) * qpk, tiles = (n_rows + 15) / 16;
+    const int tile = (k - ((own >> 20) - (tiles + rows.per_task - 1) / rows.per_task)) * rows.per_task;
+    a.r0 = tile * 16;
+    a.item = (a.g * nvs + a.vs) * RT + ((own >> 8) & 0xfff) - tiles + tile;
+    a.p0 = __builtin_amdgcn_readfirstlane(tab[a.portion * MK_MAX_TOKENS + a.t0]);
+    a.pages = rt.kv_indices + __builtin_amdgcn_readfirstlane(tab[ROWS + a.portion * MK_MAX_TOKENS + a.t0]);
+    int NT[NU], kept[NU], gap[NU];
+#pragma unroll
+    for (int e = 0; e < NU; e++) {
+      const int r = a.r0 + 16 * e;
+      a.nrows[e] = e < rows.per_task ? max(0, min(16, n_rows - r)) : 0;
+      a.newest[e] = a.p0 + (r + max(a.nrows[e], 1) - 1) / qpk;
+      NT[e] = a.newest[e] / TP + 1;
+      kept[e] = NT[e];
+      gap[e] = 0;
+      if (MK_HAVE_HYB) {
+        const int first = a.p0 + r / qpk;
+        int oldest = win ? max(0, first - win + 1) : 0;
+#if MK_HAVE_DUAL
+        if (st.chunk) oldest = max(oldest, first - first % st.chunk);
+        if (win || st.chunk) kept[e] = min((keep + TP - 1) / TP, NT[e]);
+#else
+        if (win) kept[e] = min((keep + TP - 1) / TP, NT[e]);
+#endif
+        gap[e] = max(0, oldest / TP - kept[e]);
+        NT[e] -= gap[e];
+      }
+    }
+    a.split = a.nrows[1] && (NT[0] != NT[1] || kept[0] != kept[1] || gap[0] != gap[1]);
+    a.NT = sub ? NT[1] : NT[0];
+    a.kept = sub ? kept[1] : kept[0];
+    a.gap = sub ? gap[1] : gap[0];
+    if (sub) {
+      a.r0 += 16;
+      a.item++;
+      a.nrows[0] = a.nrows[1];
+      a.newest[0] = a.newest[1];
+    }
+    if (a.split) a.nrows[1] = 0;
+    if (!a.nrows[1]) a.newest[1] = a.newest[0];
+    a.C = fx_chunks(a.NT, a.cmax);
+    a.n_pages = a.newest[1] / ps + 1;
+  };
+  auto phys = [](int tile, int kept, int gap) { return MK_HAVE_HYB && tile >= kept ? tile + gap : tile; };
+  constexpr int NQ = NU * QMAX / MK_THREADS;
+  static_assert(NU * QMAX % MK_THREADS == 0, "query operands of a unit, whole ones a thread");
+  u32x4 q_next[NQ];
+  int pg_next[PG];
+  auto request = [&](const Task &a) {
+    CStage &sp = mk_portion_stages(rt, a.portion)[s];
+    const int r = tid & 15;
+    unsigned row[NU];
+    const auto queries = dev_rows(sp.q_ws);
+#pragma unroll
+    for (int e = 0; e < NU; e++) {
+      const int R = a.r0 + e * 16 + min(r, max(a.nrows[e], 1) - 1), t = R / qpk;
+      row[e] = 2u * ((unsigned)(a.t0 + t) * st.ld_qws + (unsigned)(a.g * qpk + R - t * qpk) * nkc * KW + ((tid & 63) >> 4) * EPC);
+    }
+    // Behind a wait for everything: without it the compiler, which cannot see that the registers' last loads have landed, waits in front of each of these
+    // loads for all others.
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+#pragma unroll
+    for (int j = 0; j < NQ; j++) {
+      const int at = tid + j * MK_THREADS, i = at & (QMAX - 1);
+      q_next[j] = ldc_16B(queries, (at >= QMAX ? row[1] : row[0]) + 2 * min(i >> 6, nkc - 1) * KW);
+    }
+#pragma unroll
+    for (int i = 0; i < PG; i++) pg_next[i] = a.pages[min(tid + i * MK_THREADS, a.n_pages - 1)];
+  };
+  auto put = [&](const Task &a, int turn) {
+#pragma unroll
+    for (int j = 0; j < NQ; j++) {
+      const int at = tid + j * MK_THREADS, i = at & (QMAX - 1);
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      q_at[turn * (NU * QMAX) + at] = (tid & 15) < (at >= QMAX ? a.nrows[1] : a.nrows[0]) && (i >> 6) < nkc ? q_next[j] : z;
+    }
+#pragma unroll
+    for (int i = 0; i < PG; i++)
+      if (tid + i * MK_THREADS < a.n_pages) pages_at[turn * MK_ATTN_PAIR_PAGES + tid + i * MK_THREADS] = pg_next[i];
+  };
+  // Operands of a tile: keys, then values, each as soon as the registers are free (two sets of registers, and the tile's code twice, were
+  // longer in the fetching of instructions than any tile).  !ok: the same number of loads from one spot.
+  u32x4 k[SUB][KC], v[VB];
+  size_t pt = 0;
+  const int whole_shift = (ps & (ps - 1)) == 0 ? 31 - __builtin_clz(ps) : -1;
+  auto load_keys = [&](int g, int turn, int tile, bool ok) {
+    const int at = ok ? tile * TP : 0;
+    const int page = whole_shift >= 0 ? at >> whole_shift : at / ps;  // (a division is longer than what it finds takes to arrive)
+    pt = ok ? (size_t)__builtin_amdgcn_readfirstlane(pages_at[turn * MK_ATTN_PAIR_PAGES + page]) * ps + at - page * ps : 0;
+    const u32x4 *kp = kc + ((pt / 16) * nkv + g) * nkc * 64 + lane;
+    const int on = ok ? 64 : 0, su = ok ? nkv * nkc * 64 : 0;
+#pragma unroll
+    for (int u = 0; u < SUB; u++)
+#pragma unroll
+      for (int j = 0; j < KC; j++) k[u][j] = kp[u * su + min(j, nkc - 1) * on];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_values = [&](int g, int vs, bool ok) {  // of the tile whose keys were requested last
+    const u32x4 *vp = vc + ((pt / TP) * nkv + g) * nvb * 64 + lane;
+    const int on = ok ? 64 : 0;
+#pragma unroll
+    for (int b = 0; b < VB; b++) v[b] = vp[min(vs * VB + b, nvb - 1) * on];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_first = [&](int NT, int C, int kept, int gap, int g, int vs, int turn, int ci) {  // of a chunk, this wavefront's
+    const int tile = NT * ci / C + wave;
+    const bool ok = tile < NT * (ci + 1) / C;
+    load_keys(g, turn, phys(tile, kept, gap), ok);
+    load_values(g, vs, ok);
+  };
+  const float cap = st.softcap, sc1 = cap > 0.f ? st.sm_scale / cap : st.sm_scale, LOG2E = 1.4426950408889634f;
+  const float *sink = (const float *)st.sink;
+  Task next;
+  if (c.vid < n_tasks) decode(c.vid, 0, next);
+  barrier_wait(c);
+  c.wrote_through = true;
+  if (c.vid < n_tasks) {
+    request(next);
+    put(next, 0);
+    __syncthreads();
+    load_first(next.NT, next.C, next.kept, next.gap, next.g, next.vs, 0, 0);
+  }
+  for (int u = c.vid, sub = 0, turn = 0; u < n_tasks; turn ^= 1) {
+    const Task a = next;
+    if (a.split && !sub) {
+      sub = 1;
+    } else {
+      sub = 0;
+      u += c.G;
+    }
+    const bool goes_on = u < n_tasks;
+    if (goes_on) {
+      decode(u, sub, next);
+      request(next);
+    }
+    CStage &sp = mk_portion_stages(rt, a.portion)[s];
+    const u32x4 *qs = q_at + turn * (NU * QMAX);
+    int plim[NU], olim[NU];
+    float sc_row[NU];
+#pragma unroll
+    for (int e = 0; e < NU; e++) {
+      const int R = a.r0 + 16 * e + min(lr, max(a.nrows[e], 1) - 1);
+      plim[e] = a.p0 + R / qpk;
+#if MK_HAVE_DUAL
+      olim[e] = st.chunk ? plim[e] - plim[e] % st.chunk : 0;
+      sc_row[e] = sc1 * (st.temp ? st.temp[a.g * qpk + R % qpk] : 1.f);
+#else
+      olim[e] = 0;
+      sc_row[e] = sc1;
+#endif
+    }
+    const int dv0 = a.vs * VB * 16;
+    auto sink_of = [&](int e, int r) -> float { return sink ? sink[a.g * qpk + (a.r0 + 16 * e + min(r, max(e ? a.nrows[1] : a.nrows[0], 1) - 1)) % qpk] * LOG2E : -INFINITY; };
+    auto emit = [&](int e, int r, int d, const f32x4 &o) {
+      const int R = a.r0 + 16 * e + r;
+      const float q[4] = {o[0], o[1], o[2], o[3]};
+      fx_stc4((E *)sp.out + (size_t)(a.t0 + R / qpk) * st.ld_out + (size_t)(a.g * qpk + R % qpk) * DV, dv0 + d, DV, q);
+    };
+    float *const chunk_far = rt.group_attn_part + (size_t)a.portion * rt.group_attn + (size_t)a.item * a.cmax * 16 * PST;
+    auto far = [&](int e, int ci, int r, int d) { return (f32x4 *)(chunk_far + ((size_t)(e * a.cmax + ci) * 16 + r) * PST + d); };
+    for (int ci = 0; ci < a.C; ci++) {
+      const int tb = a.NT * ci / a.C, te = a.NT * (ci + 1) / a.C;
+      float m[NU], l[NU];
+      f32x4 acc[NU][VB], S[NU][SUB];
+#pragma unroll
+      for (int e = 0; e < NU; e++) {
+        m[e] = MK_FX_NEG;
+        l[e] = 0.f;
+#pragma unroll
+        for (int b = 0; b < VB; b++) acc[e][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+      // (see stage_fx_attn_t for what is done with a tile; the last one is requested again behind the end)
+      for (int tl = tb + wave; tl < te; tl += MK_WAVES) {
+        const int tile = phys(tl, a.kept, a.gap);
+        const bool more = tl + MK_WAVES < te;
+#pragma unroll
+        for (int e = 0; e < NU; e++)
+#pragma unroll
+          for (int u_ = 0; u_ < SUB; u_++) S[e][u_] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        u32x4 q[KC][NU];
+#pragma unroll
+        for (int j = 0; j < KC; j++)
+#pragma unroll
+          for (int e = 0; e < NU; e++) q[j][e] = qs[e * QMAX + j * 64 + lane];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < KC; j++)
+#pragma unroll
+          for (int u_ = 0; u_ < SUB; u_++)
+#pragma unroll
+            for (int e = 0; e < NU; e++) S[e][u_] = fx_mma_k(E(), k[u_][j], q[j][e], S[e][u_]);
+        load_keys(a.g, turn, phys(tl + MK_WAVES, a.kept, a.gap), more);
+        float sc[NU][SUB][4], tm[NU];
+        auto each = [&](auto f) {
+#pragma unroll
+          for (int e = 0; e < NU; e++)
+#pragma unroll
+            for (int u_ = 0; u_ < SUB; u_++)
+#pragma unroll
+              for (int i = 0; i < 4; i++) f(e, u_, i);
+        };
+        // (one branch: at every value of its own the values follow each other, 14 us of 55 in a thousand positions)
+        if (cap > 0.f) {
+          each([&](int e, int u_, int i) { sc[e][u_][i] = __builtin_amdgcn_exp2f(S[e][u_][i] * sc_row[e] * (2.f * LOG2E)); });
+          each([&](int e, int u_, int i) { sc[e][u_][i] = (cap * LOG2E) * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + sc[e][u_][i])); });
+        } else {
+          each([&](int e, int u_, int i) { sc[e][u_][i] = S[e][u_][i] * sc_row[e] * LOG2E; });
+        }
+        tm[0] = tm[1] = MK_FX_NEG;
+        each([&](int e, int u_, int i) {
+          const int at = tile * TP + u_ * 16 + lg * 4 + i;
+          bool seen = at <= plim[e];
+          if (MK_HAVE_HYB) seen = seen && (win == 0 || plim[e] - at < win || at < keep);
+#if MK_HAVE_DUAL
+          seen = seen && at >= olim[e];
+#endif
+          sc[e][u_][i] = seen ? sc[e][u_][i] : MK_FX_NEG;
+          tm[e] = fmaxf(tm[e], sc[e][u_][i]);
+        });
+#pragma unroll
+        for (int e = 0; e < NU; e++) tm[e] = groups_max(tm[e]);
+        if (__any(tm[0] > m[0] || tm[1] > m[1])) {
+#pragma unroll
+          for (int e = 0; e < NU; e++) {
+            const float nm = fmaxf(m[e], tm[e]), corr = fx_exp2(E(), m[e] - nm);
+            m[e] = nm;
+            l[e] *= corr;
+#pragma unroll
+            for (int b = 0; b < VB; b++) acc[e][b] *= corr;
+          }
+        }
+        u32x4 hi[NU], lo[NU];
+#pragma unroll
+        for (int e = 0; e < NU; e++) {
+#pragma unroll
+          for (int u_ = 0; u_ < SUB; u_++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              sc[e][u_][i] = sc[e][u_][i] > 0.5f * MK_FX_NEG ? fx_exp2(E(), sc[e][u_][i] - m[e]) : 0.f;
+              l[e] += sc[e][u_][i];
+            }
+#pragma unroll
+          for (int w = 0; w < 4; w++) {
+            const float x0 = sc[e][w >> 1][(w & 1) * 2], x1 = sc[e][w >> 1][(w & 1) * 2 + 1];
+            hi[e][w] = pack2(x0, x1);
+            lo[e][w] = pack2(x0 - bf_lo(hi[e][w]), x1 - bf_hi(hi[e][w]));
+          }
+        }
+        const bool edge = (tile + 1) * TP - 1 > a.newest[0];
+#pragma unroll
+        for (int e = NU - 1; e >= 0; e--) {
+          if (edge) {  // values behind the newest position belong to nobody (the first unit's is not behind the second's)
+#pragma unroll
+            for (int b = 0; b < VB; b++)
+#pragma unroll
+              for (int w = 0; w < 4; w++) {
+                const int q = tile * TP + (w >> 1) * 16 + lg * 4 + (w & 1) * 2;
+                v[b][w] = q > a.newest[e] ? 0u : (q + 1 > a.newest[e] ? v[b][w] & 0xffffu : v[b][w]);
+              }
+          }
+#pragma unroll
+          for (int b = 0; b < VB; b += 4) fx_add_products(acc[e][b], acc[e][b + 1], acc[e][b + 2], acc[e][b + 3], v[b], v[b + 1], v[b + 2], v[b + 3], hi[e], lo[e]);
+        }
+        load_values(a.g, a.vs, more);
+      }
+      // ---- wavefronts of the workgroup
+      const bool last = ci == a.C - 1;
+      if (last && goes_on) put(next, turn ^ 1);
+#pragma unroll
+      for (int e = 0; e < NU; e++) l[e] = groups_sum(l[e]);
+      lds_barrier();  // (sums of the chunk in front have been read, and what was put is there)
+      if (!last || goes_on)
+        load_first(last ? next.NT : a.NT, last ? next.C : a.C, last ? next.kept : a.kept, last ? next.gap : a.gap, last ? next.g : a.g, last ? next.vs : a.vs, last ? turn ^ 1 : turn, last ? 0 : ci + 1);
+#pragma unroll
+      for (int e = 0; e < NU; e++) {
+#pragma unroll
+        for (int b = 0; b < VB; b++) *(f32x4 *)(part + ((e * MK_WAVES + wave) * 16 + lr) * PSTR + b * 16 + lg * 4) = acc[e][b];
+        if (lg == 0) {
+          ml[e * 128 + wave * 16 + lr] = m[e];
+          ml[e * 128 + 64 + wave * 16 + lr] = l[e];
+        }
+      }
+      lds_barrier();
+#pragma unroll 1
+      for (int i = tid; i < (a.nrows[1] ? 2 : 1) * QUADS; i += MK_THREADS) {
+        const int e = i >= QUADS, q = i - e * QUADS, r = q / (VB * 4), d = (q - r * (VB * 4)) * 4;
+        const float *const mr = ml + e * 128 + r, *const pr = part + (e * MK_WAVES * 16 + r) * PSTR + d;
+        float M_ = MK_FX_NEG, L_ = 0.f, fin[MK_WAVES];
+#pragma unroll
+        for (int w = 0; w < MK_WAVES; w++) M_ = fmaxf(M_, mr[w * 16]);
+#pragma unroll
+        for (int w = 0; w < MK_WAVES; w++) {
+          fin[w] = exp2f(mr[w * 16] - M_);
+          L_ += mr[64 + w * 16] * fin[w];
+        }
+        if (a.C == 1) {
+          const float inv = 1.f / (L_ + exp2f(sink_of(e, r) - M_));
+#pragma unroll
+          for (int w = 0; w < MK_WAVES; w++) fin[w] *= inv;
+        } else if (d == 0) {
+          float *const cml = chunk_ml + (e * MK_ATTN_MAX_CHUNKS + ci) * 32 + r;
+          cml[0] = M_;
+          cml[16] = L_;
+        }
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < MK_WAVES; w++) o += *(const f32x4 *)(pr + w * 16 * PSTR) * fin[w];
+        if (a.C > 1) {  // (not one address for both: it would be a generic one)
+          if (ci < CHUNKS) chunk_at[(e * CHUNKS + ci) * QUADS + q] = o;
+          else *far(e, ci, r, d) = o;
+        } else if (r < (e ? a.nrows[1] : a.nrows[0]) && dv0 + d < DV) {
+          emit(e, r, d, o);
+        }
+      }
+    }
+    if (a.C == 1) continue;
+    // ---- chunks
+    lds_barrier();
+#pragma unroll 1
+    for (int i = tid; i < (a.nrows[1] ? 2 : 1) * QUADS; i += MK_THREADS) {
+      const int e = i >= QUADS, q = i - e * QUADS, r = q / (VB * 4), d = (q - r * (VB * 4)) * 4;
+      if (r >= (e ? a.nrows[1] : a.nrows[0]) || dv0 + d >= DV) continue;
+      const float *const cml = chunk_ml + e * MK_ATTN_MAX_CHUNKS * 32 + r;
+      float M_ = MK_FX_NEG, L_ = 0.f;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int ci = 0; ci < a.C; ci++) M_ = fmaxf(M_, cml[ci * 32]);
+#pragma unroll 1
+      for (int ci = 0; ci < a.C; ci++) {
+        const float f = exp2f(cml[ci * 32] - M_);
+        f32x4 x;
+        if (ci < CHUNKS) x = chunk_at[(e * CHUNKS + ci) * QUADS + q];
+        else x = *far(e, ci, r, d);
+        L_ += cml[ci * 32 + 16] * f;
+        o += x * f;
+      }
+      emit(e, r, d, o * (1.f / (L_ + exp2f(sink_of(e, r) - M_))));
+    }
+  }
+}
+template <typename E>
+__device__ __forceinline__ void stage_fx_attn_group(CStage &st, Ctx &c, const MkRuntime &rt, int s, int portions, const int *sh_rows, const FxGroupRows &rows, char *smem) {
+  if (st.v_tiles == 4) {
+    if (st.k_tiles == 2) fx_attn_group<E, 2, 4>(c, rt, s, portions, sh_rows, rows, smem);
+    else fx_attn_group<E, 4, 4>(c, rt, s, portions, sh_rows, rows, smem);
+  } else {
+    fx_attn_group<E, 4, 8>(c, rt, s, portions, sh_rows, rows, smem);
+  }
+}
+#endif
 template <typename E>
 __device__ __forceinline__ void stage_fx_attn(CStage &st, Ctx &c, const MkRuntime &rt, int M, bool single, char *smem) {
   if constexpr (sizeof(E) == 2) {

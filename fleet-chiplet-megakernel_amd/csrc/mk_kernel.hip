@@ -4905,6 +4905,15 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
           e += (int)(ent >> MK_PAIR_BACK_SHIFT);
         }
       }
+#if MK_HAVE_FLEX
+      FxGroupRows fx_tasks;
+      if constexpr (FX) {
+        if ((ent & MK_PAIR_BOTH) && (op == MK_OP_FX_PREP || op == MK_OP_FX_ATTN)) {
+          if (any_single || (op == MK_OP_FX_ATTN && !fx_attn_group_rows(st, c, rt, portions, sh_rows, fx_tasks))) continue;  // (as above)
+          e += (int)(ent >> MK_PAIR_BACK_SHIFT);
+        }
+      }
+#endif
 #endif
       c.st = &st;
       const long long t_in = (long long)wall_clock64();
@@ -4920,8 +4929,24 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
 #endif
           if constexpr (FX) stage_fx_addnorm<E>(st, c, M, smem);
           break;
-        case MK_OP_FX_PREP: if constexpr (FX) stage_fx_prep<E>(st, c, rt, M, smem); break;
-        case MK_OP_FX_ATTN: if constexpr (FX) stage_fx_attn<E>(st, c, rt, M, MAXM == 1 || single, smem); break;
+        case MK_OP_FX_PREP:
+#if MK_PAIR
+          if (ent & MK_PAIR_BOTH) {
+            if constexpr (FX) stage_fx_prep_group<E>(c, rt, s, portions, sh_rows, smem);
+            break;
+          }
+#endif
+          if constexpr (FX) stage_fx_prep<E>(st, c, rt, M, smem);
+          break;
+        case MK_OP_FX_ATTN:
+#if MK_PAIR
+          if (ent & MK_PAIR_BOTH) {
+            if constexpr (FX) stage_fx_attn_group<E>(st, c, rt, s, portions, sh_rows, fx_tasks, smem);
+            break;
+          }
+#endif
+          if constexpr (FX) stage_fx_attn<E>(st, c, rt, M, MAXM == 1 || single, smem);
+          break;
         case MK_OP_LINEAR_F32:
           if constexpr (F32) stage_fx_linear_f32(st, c, M, smem);
           break;

@@ -84,6 +84,29 @@ def test_session(family):
             assert torch.isfinite(a).all() and torch.equal(a, b) and ga == gb
 
 
+# flex attention: more chunks than LDS holds, units in pairs; five queries a kv head and two slices of value dims; units one by one; a window and kept positions
+# whose tiles lie apart; positions in chunks.  Requests that begin inside a portion: units whose tiles are not the same ones
+@pytest.mark.parametrize("family,sizes", [
+    ("suborax", dict(heads=16, kv_heads=4)), ("suborax", dict(heads=20, kv_heads=4, dim=96, vdim=160)), ("suborax", dict(heads=8, kv_heads=2, dim=64, vdim=64)),
+    ("suborax", dict(heads=16, kv_heads=8, dim=160)), ("bukatar", dict(window=100, keep_first=40)), ("vizonex", dict(chunk=128))])
+def test_flex_attention(family, sizes):
+    import generate
+    from mirage.mpk import ServingSession
+    make, base = generate.SHAPES[family + "-2k"]
+    torch.manual_seed(7)
+    model = generate.random_model(make(**{**base, **sizes}, layers={"suborax": 2}.get(family, 4), vocab=1000, **({"positions": 1024} if family == "vizonex" else {})))[0]
+    g = torch.Generator().manual_seed(9)
+    lengths = (64 * 9 + 5, 333, 70)
+    prompts, outs = [torch.randint(0, 1000, (n,), generator=g).tolist() for n in lengths], []
+    for together in (8, 0):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 64, max_requests=3, max_seq_length=640)
+        assert s.mpk.persistent_kernel.stats()["paired_portions"]
+        s._second, s._together = s._second if together else 0, together
+        outs.append([s.step(list(enumerate(prompts)), [[n - 1] for n in lengths])[0].cpu(), s.step([(r, [3]) for r in range(3)], [[0]] * 3)[0].cpu()])
+        s.finalize()
+    assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*outs))
+
+
 def test_portions_of_single_rows():
     """Portions in which every request brings one row append keys and values in the attention itself, beside portions whose rows are prepared ahead of it."""
     from mirage.mpk import ServingSession
