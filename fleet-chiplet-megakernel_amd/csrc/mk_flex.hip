@@ -1344,7 +1344,7 @@ __device__ __forceinline__ void fx_attn_group(Ctx &c, const MkRuntime &rt, int s
     const auto queries = dev_rows(sp.q_ws);
 #pragma unroll
     for (int e = 0; e < NU; e++) {
-      const int R = a.r0 + e * 16 + min(r, max(a.nrows[e], 1) - 1), t = R / qpk;
+      const int R = a.nrows[e] ? a.r0 + e * 16 + min(r, a.nrows[e] - 1) : a.r0, t = R / qpk;  // (a unit that is none: the first one's first row, as none may follow)
       row[e] = 2u * ((unsigned)(a.t0 + t) * st.ld_qws + (unsigned)(a.g * qpk + R - t * qpk) * nkc * KW + ((tid & 63) >> 4) * EPC);
     }
     // Behind a wait for everything: without it the compiler, which cannot see that the registers' last loads have landed, waits in front of each of these
