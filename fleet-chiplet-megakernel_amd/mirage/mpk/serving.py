@@ -251,7 +251,7 @@ class ServingSession:
 
     def _put(self, at, ids, desc):
         """A description in pinned memory, from word `at` on; its length."""
-        n, host = 2 * self.max_rows, self._words.numpy()[at:]
+        n, host = 2 * self.max_rows, (self._host if self._words is None else self._words).numpy()[at:]
         # plain numbers as they are; what else torch takes for ids (tensors of one value among it) by way of torch, which costs 6.5 us
         host[:2 * len(ids)].view("int64")[:] = ids if set(map(type, ids)) == {int} else torch.tensor(ids, dtype=torch.int64).numpy()
         host[n:n + len(desc)] = desc
