@@ -2285,7 +2285,9 @@ int tail_stage(const mk_graph *g) {
 // Several portions inside prompts as one iteration (MkPairEntry): linears that run for all portions at once, and between two of them the stages of
 // the first portion, then those of the second, and so on, as iterations of their own would run them.  What a cache or a state gets from a portion is
 // written back and read anew in front of the next one; stages that only take rows to rows run for one portion after the other without a barrier, and so do
-// stages that put keys and values into pages and, behind them all, the attention over those pages, which looks at no position behind a row's own.
+// stages that put keys and values into pages and, behind them all, the attention over those pages, which looks at no position behind a row's own.  Norms by
+// rows run for all portions at once, and so does attention with what prepares its rows, unless the portions ask for another form: then the entries
+// behind, portion by portion, are the ones that run.
 // Empty: the graph does not run portions that way.
 //
 // *worth: pairs at the beginning of an offline launch that pay for the kernel they run in, which is 42 us of launch and handshake.  A pair gains, against its
@@ -3339,7 +3341,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   if (!rt) rt = &g->h_rt;
   const MkRuntime *rtp = g->d_rt;
   void *args[] = {(void *)rt, (void *)&rtp, (void *)&max_iters, (void *)&run_scheduler};
-  // Two portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions and the other kernel
+  // Several portions an iteration: a kernel of their own.  Where the GPU schedules, it runs until an iteration is none of two portions or more and the other kernel
   // goes on; a launch begins with it where the requests' prompts, as they were when the last one ended or the requests began, say that enough pairs come
   // first to pay for it (only speed is lost where prompts were changed since).
   const bool both = rt->batch_n > 0;
@@ -3348,7 +3350,7 @@ int do_launch(mk_graph *g, hipStream_t stream, int max_iters, int run_scheduler,
   auto enqueue = [&](MkLaunchPart part) -> int {
     switch (part) {
       case MK_PART_PAIRS:
-        what = "kernel of two portions";
+        what = "kernel of several portions";
         return hipLaunchCooperativeKernel(pair_kernel_of(g), dim3(g->G), dim3(MK_THREADS), args, MK_LDS_BYTES, stream);
       case MK_PART_RESUME:
         what = "hand-over";

@@ -90,7 +90,7 @@ typedef const __attribute__((address_space(4))) MkWeight CWeight;
 #define MK_HAVE_MIX 0
 #endif
 
-// kernels that run iterations of two portions inside prompts, and nothing else
+// kernels that run iterations of several portions inside prompts, and nothing else
 #if defined(MK_KERNEL_DENSE_PAIR) || defined(MK_KERNEL_FLEX_PAIR) || defined(MK_KERNEL_MIX_PAIR) || defined(MK_KERNEL_HYB_PAIR) || defined(MK_KERNEL_DUAL_PAIR)
 #define MK_PAIR 1
 #else
@@ -5389,7 +5389,7 @@ extern "C" __global__ __launch_bounds__(MK_THREADS, 1) void mk_persistent_kernel
   mk_kernel_body<1, void>(rt, rtp, max_iters, run_scheduler);
 }
 #endif
-// Iterations of two portions inside prompts, and nothing else: a launch of the offline scheduler that begins inside prompts runs this kernel up to its
+// Iterations of two portions inside prompts or more, and nothing else: a launch of the offline scheduler that begins inside prompts runs this kernel up to its
 // first iteration that is none, which the kernel of several tokens goes on from (MK_SCHED_RESUME).  Two kernels, as registers are allotted to
 // all stages of one together: decode steps that ran here too were up to 3.7 % longer (qwen3-8b, 8 layers, rows for portions of 64, 24 requests
 // 883 -> 915 us, 8 requests 807 -> 826), and with the pairs as a function beside the other stages both were slower (690 -> 1010, prompts 32.3 -> 36.0 ms).

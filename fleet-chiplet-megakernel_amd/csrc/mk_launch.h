@@ -4,7 +4,7 @@
 
 enum MkLaunchPart { MK_PART_PAIRS, MK_PART_RESUME, MK_PART_MAIN, MK_PART_DONE };
 
-// `first`: the kernel of two portions runs in front of the main one; `both`: in its place.  enqueue(part) returns 0 or an error.  What has been
+// `first`: the kernel of several portions runs in front of the main one; `both`: in its place.  enqueue(part) returns 0 or an error.  What has been
 // enqueued when a call fails runs all the same, so undo(lost) has to wait for it and clear the counters that the missing last part would have
 // cleared: the next launch's workgroups would count on from them.  `lost`: the kernel in front has scheduled an iteration that nobody runs.
 template <class Enqueue, class Undo>

@@ -357,7 +357,7 @@ enum MkSchedMode {
   MK_SCHED_OFFLINE = 1,      // on-GPU continuous batching over `tokens` (MODE_OFFLINE)
   MK_SCHED_FROM_META = 2,    // derived on the GPU from the qo / paged-kv meta tensors the host filled (MODE_ONLINE_NOTOKEN, MODE_ONEPASS)
   MK_SCHED_ONLINE = 3,       // one request, host-written tokens consumed num_new_tokens[0] at a time (MODE_ONLINE)
-  MK_SCHED_RESUME = 5,       // MK_SCHED_OFFLINE from iteration MkSched::resume_it on, which has been scheduled: the launch began with pairs of portions
+  MK_SCHED_RESUME = 5,       // MK_SCHED_OFFLINE from iteration MkSched::resume_it on, which has been scheduled: the launch began with iterations of several portions
   MK_SCHED_INGEST = 4,       // MK_SCHED_FROM_META, and nobody reads the logits or sampled tokens of the batch (mk_enqueue_ingest)
 };
 
@@ -376,11 +376,12 @@ struct MkSched {
 #define MK_GROUP_SINGLE 0x10000
 
 // What an iteration of several portions runs, one after another: a stage's index with these bits.  Linears that stream their weights through the matrix
-// cores run for all portions at once (MK_PAIR_BOTH); the stages between two of them run for the first portion, then for the second one, and so on.
+// cores run for all portions at once (MK_PAIR_BOTH), and so do attention over pages, what prepares its rows, and norms; other stages between two linears run for the
+// first portion, then for the second one, and so on.
 enum MkPairEntry {
   MK_PAIR_STAGE = 0xffff,
   MK_PAIR_SECOND = 1 << 16,   // for the second portion, and each one behind it
-  MK_PAIR_BOTH = 1 << 17,     // for all at once; 128-wide attention (MK_OP_ATTN): where the portions allow it, and the `back` entries behind it, for one after the other, are skipped
+  MK_PAIR_BOTH = 1 << 17,     // for all at once; attention and the preparation of its rows: where the portions allow it, and the `back` entries behind it, for one after the other, are skipped
   MK_PAIR_ON = 1 << 18,       // the next portion's run of this stage follows without a barrier
   MK_PAIR_RELEASE = 1 << 19,  // caches or states may have been written, here or by the stages in front, for the next portion to read: write back ...
   MK_PAIR_ACQUIRE = 1 << 20,  // ... and, no stage, drop what the caches of the dies hold

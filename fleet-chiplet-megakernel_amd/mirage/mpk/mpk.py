@@ -72,7 +72,7 @@ class MPKMetadata:
     eos_token_id: Optional[int] = None
     max_tokens_per_request: Optional[int] = None
     single_weight_copy: Optional[bool] = None  # keep every linear weight once, in tile order (see PersistentKernel)
-    pair_portions: bool = True  # two portions inside prompts may run as one iteration, where the model's builder says so (GraphBuilder.pair_portions)
+    pair_portions: bool = True  # portions inside prompts, eight at most, may run as one iteration, where the model's builder says so (GraphBuilder.pair_portions)
     dtype: torch.dtype = torch.bfloat16  # activations, weights and caches; the builder refuses what its model cannot run in
 
     def check_valid(self):

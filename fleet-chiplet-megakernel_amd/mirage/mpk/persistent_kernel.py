@@ -62,7 +62,7 @@ class PersistentKernel:
         `single_weight_copy` (no counterpart in the reference; None takes FLEET_MK_SINGLE_WEIGHT_COPY, else False): a graph
         with max_num_batched_tokens >= 2 then keeps every linear weight ONCE, in the matrix-core tile layout compile()
         makes; `release_row_major_weights()` afterwards drops the attached tensors nothing reads any more.
-        `pair_portions`: the caller's word that no stage reads rows its iteration has not written, token ids apart; two portions inside prompts may then
+        `pair_portions`: the caller's word that no stage reads rows its iteration has not written, token ids apart; portions inside prompts, eight at most, may then
         run as one iteration (fleet_mk.h, MK_CFG_PAIR_PORTIONS).
         `binding`: "ctypes" or "cython" -- which binding of the C ABI carries the calls (None: FLEET_MK_BINDING, else ctypes)."""
         self.__finalized__ = False
