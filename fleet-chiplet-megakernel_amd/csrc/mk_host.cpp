@@ -22,6 +22,7 @@
 #include "../../include/fleet_mk.h"
 #include "mk_types.h"
 #include "mk_launch.h"
+#include "mk_pairs.h"
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -2282,13 +2283,7 @@ int tail_stage(const mk_graph *g) {
   return tail;
 }
 
-// Several portions inside prompts as one iteration (MkPairEntry): linears that run for all portions at once, and between two of them the stages of
-// the first portion, then those of the second, and so on, as iterations of their own would run them.  What a cache or a state gets from a portion is
-// written back and read anew in front of the next one; stages that only take rows to rows run for one portion after the other without a barrier, and so do
-// stages that put keys and values into pages and, behind them all, the attention over those pages, which looks at no position behind a row's own.  Norms by
-// rows run for all portions at once, and so does attention with what prepares its rows, unless the portions ask for another form: then the entries
-// behind, portion by portion, are the ones that run.
-// Empty: the graph does not run portions that way.
+// What iterations of several portions run (mk_pair_program).  Empty: the graph does not run portions that way.
 //
 // *worth: pairs at the beginning of an offline launch that pay for the kernel they run in, which is 42 us of launch and handshake.  A pair gains, against its
 // portions one by one, about 8 us for every linear that runs for both and 0.05 us for every megabyte of their weights, and loses 7.5 where one portion
@@ -2304,87 +2299,8 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
   if (c.max_num_batched_tokens <= 32 || c.max_num_batched_tokens > MK_MAX_TOKENS || c.max_tokens_per_request <= 8) return prog;
   if (c.mode != MK_MODE_OFFLINE && std::any_of(g->stages.begin(), g->stages.end(), [](const MkStage &s) { return (s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED) && (s.flags & MK_F_EMBED_FROM_TOKENS); }))
     return prog;  // (the rows of requests that the host does not describe)
-  auto keeps_nothing = [&](const MkStage &s) { return !s.k_cache && !s.v_cache && !s.tail && !s.conv_w; };
-  auto row_wise = [&](const MkStage &s) {
-    return keeps_nothing(s) && (s.op == MK_OP_NORM || s.op == MK_OP_FX_ADDNORM || s.op == MK_OP_MX_PRENORM || s.op == MK_OP_EMBED || s.op == MK_OP_FX_EMBED);
-  };
-  auto passes = [&](const MkStage &s) {  // (leaves nothing for another iteration)
-    switch (s.op) {
-      case MK_OP_NORM: case MK_OP_FX_ADDNORM: case MK_OP_MX_PRENORM: case MK_OP_EMBED: case MK_OP_FX_EMBED: case MK_OP_LINEAR: case MK_OP_SILU_MUL: case MK_OP_MOE_TOPK: case MK_OP_MOE_LINEAR:
-      case MK_OP_MOE_COMBINE: case MK_OP_MX_HEAD_LINEAR: case MK_OP_HY_ROUTE: case MK_OP_HY_EXPERTS: case MK_OP_COPY: return keeps_nothing(s);
-      default: return false;
-    }
-  };
-  auto left_out = [&](const MkStage &s) {  // (by iterations in which nobody has several rows, or nothing was split)
-    return s.op == MK_OP_FX_PREP || s.op == MK_OP_DU_CONV || s.op == MK_OP_MX_LATENT_MERGE || s.op == MK_OP_MX_DELTA_OUT;
-  };
-  std::vector<char> both(n, 0);
-  for (int i = 0; i < n; i++) {
-    MkStage s = g->stages[i];
-    both[i] = s.op == MK_OP_LINEAR && keeps_nothing(s) && (s.k & 63) == 0 && mk_xres_plan(s, g->G).S >= 1;
-  }
-  // what says where a sum is that was left to the stage behind says so of the last linear that left one, and is kept until all portions have read it: by a
-  // stage that runs for all of them at once, or with no other linear in between
-  for (int i = n - 1; i >= 0; i--) {
-    if (!both[i] || !(g->stages[i].flags & MK_F_DEFER_SUM) || (i + 1 < n && row_wise(g->stages[i + 1]))) continue;
-    for (int j = i + 1; j < n && !both[j]; j++)
-      if (g->stages[j].op == MK_OP_LINEAR) both[i] = 0;
-  }
-  if (std::count(both.begin(), both.end(), 1) == 0) return prog;
-  for (int i = 0; i < n;) {
-    if (both[i]) {
-      prog.push_back(i++ | MK_PAIR_BOTH);
-      continue;
-    }
-    int j = i;
-    while (j < n && !both[j]) j++;
-    // a run [q0, q1) for one portion after the other; the first stage of all may find a sum that the linear in front has left
-    auto in_turn = [&](int q0, int q1, bool on) {
-      bool carries = false;
-      for (int q = q0; q < q1; q++) carries = carries || !(on || passes(g->stages[q]));
-      // One write-back of the caches is enough, behind the last of these stages that no iteration leaves out, or behind later ones that may write.
-      // (Each is 2 to 4 us.  Behind every stage, pairs were slower than their portions one by one where few linears run for both, us a pair: dodonex-2k
-      // + 53, vizonex-8b + 50, vizonex-2k + 63, bukatar-2k + 37; now - 7, - 15, - 14, - 21, and suborax-8b - 174 -> - 184, dodonex-8b - 37 -> - 93.)
-      int last = q1 - 1;
-      while (last >= q0 && left_out(g->stages[last])) last--;
-      auto entry = [&](int q) { return q | (on ? MK_PAIR_ON : 0) | (carries && (q == last || (q > last && !passes(g->stages[q]))) ? MK_PAIR_RELEASE : 0); };
-      for (int q = q0; q < q1; q++) prog.push_back(entry(q));
-      const size_t again = prog.size();
-      if (carries) prog.push_back(MK_PAIR_ACQUIRE);
-      for (int q = q0; q < q1; q++) prog.push_back(entry(q) | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
-      prog.back() |= MK_PAIR_LOOP | (unsigned)(prog.size() - 1 - again) << MK_PAIR_BACK_SHIFT;
-    };
-    auto prepared = [&](int q) {  // attention over pages, all of whose new rows the stage in front has put there
-      const MkStage &s = g->stages[q];
-      return s.op == MK_OP_FX_ATTN && q > i && g->stages[q - 1].op == MK_OP_FX_PREP && g->stages[q - 1].k_cache == s.k_cache && g->stages[q - 1].v_cache == s.v_cache;
-    };
-    // (not a stage that may find a sum which a stage of the same run has left)
-    auto first = [&](int q) { return q == i || !(g->stages[q - 1].flags & MK_F_DEFER_SUM); };
-    auto normed = [&](const MkStage &s) { return row_wise(s) && ((s.op == MK_OP_NORM && mk_norm_by_rows(s)) || s.op == MK_OP_FX_ADDNORM); };
-    auto attends = [&](int q) {  // attention that may run for all portions at once, and what prepares its rows
-      const MkStage &s = g->stages[q];
-      if (prepared(q) || (q + 1 < j && prepared(q + 1))) return first(q);
-      return s.op == MK_OP_ATTN && first(q) && (s.num_q_heads == 4 * s.num_kv_heads || s.num_q_heads == 8 * s.num_kv_heads);
-    };
-    auto alone = [&](int q) { return first(q) && (row_wise(g->stages[q]) || prepared(q) || (q + 1 < j && prepared(q + 1))); };
-    for (int q = i; q < j;) {
-      int e = q + 1;
-      if (first(q) && normed(g->stages[q])) {
-        prog.push_back(q | MK_PAIR_BOTH);
-      } else if (attends(q)) {
-        const size_t at = prog.size();
-        prog.push_back(q | MK_PAIR_BOTH);
-        in_turn(q, e, alone(q));
-        prog[at] |= (unsigned)(prog.size() - at - 1) << MK_PAIR_BACK_SHIFT;
-      } else {
-        if (!alone(q))
-          while (e < j && !alone(e) && !attends(e) && !(first(e) && normed(g->stages[e]))) e++;
-        in_turn(q, e, alone(q));
-      }
-      q = e;
-    }
-    i = j;
-  }
+  prog = mk_pair_program(g->stages.data(), n, g->G);
+  if (prog.empty()) return prog;
   double gain = 0;
   for (const unsigned e : prog) {
     const MkStage &s = g->stages[e & MK_PAIR_STAGE];
