@@ -1,4 +1,4 @@
-// What an iteration of several portions of prompts runs (MkPairEntry).  No HIP: the CPU can run it as well.
+// What an iteration of several portions of prompts runs (MkPairEntry).  No HIP: tests/test_pair_program.py runs the same code on the CPU.
 #pragma once
 #include <algorithm>
 #include <vector>
@@ -64,12 +64,15 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
       for (int q = q0; q < q1; q++) prog.push_back(entry(q) | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
       prog.back() |= MK_PAIR_LOOP | (unsigned)(prog.size() - 1 - again) << MK_PAIR_BACK_SHIFT;
     };
-    auto prepared = [&](int q) {  // attention over pages, all of whose new rows the stage in front has put there
-      const MkStage &s = stages[q];
-      return s.op == MK_OP_FX_ATTN && q > i && stages[q - 1].op == MK_OP_FX_PREP && stages[q - 1].k_cache == s.k_cache && stages[q - 1].v_cache == s.v_cache;
-    };
     // (not a stage that may find a sum which a stage of the same run has left)
     auto first = [&](int q) { return q == i || !(stages[q - 1].flags & MK_F_DEFER_SUM); };
+    // Attention over pages, all of whose new rows the stage in front has put there.  A portion in which every request brings one row leaves the stage in front out,
+    // and what a linear of the same run has left to that one lies where the next portion's run of the linear puts its own: linear, preparation and attention
+    // then run together, portion by portion.
+    auto prepared = [&](int q) {
+      const MkStage &s = stages[q];
+      return s.op == MK_OP_FX_ATTN && q > i && first(q - 1) && stages[q - 1].op == MK_OP_FX_PREP && stages[q - 1].k_cache == s.k_cache && stages[q - 1].v_cache == s.v_cache;
+    };
     auto normed = [&](const MkStage &s) { return row_wise(s) && ((s.op == MK_OP_NORM && mk_norm_by_rows(s)) || s.op == MK_OP_FX_ADDNORM); };
     auto attends = [&](int q) {  // attention that may run for all portions at once, and what prepares its rows
       const MkStage &s = stages[q];

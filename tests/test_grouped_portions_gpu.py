@@ -170,3 +170,25 @@ def test_out_of_pages_behind_some_passes():
         outs.append([c.clone().cpu() for c in s.mpk.model_builder.k_cache] + [torch.tensor([r.length for r in s.requests.values()])])
         s.finalize()
     assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_single_rows_whose_sums_lie_apart():
+    """As above where the projection runs portion by portion, since the output one streams no weights (2560 values, 128 tiles): its slices are the next portion's a moment later."""
+    import generate
+    from mirage.mpk import ServingSession
+    make, base = generate.SHAPES["suborax-2k"]
+    torch.manual_seed(7)
+    model, outs = generate.random_model(make(**{**base, "heads": 16, "kv_heads": 8, "dim": 160}, layers=2, vocab=1000))[0], []
+    for grouped in (True, False):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 64, max_requests=40, max_seq_length=512)
+        assert s.mpk.persistent_kernel.stats()["paired_portions"]
+        passes = [[(r, [r + 1]) for r in range(40)], [(0, list(range(50)))], [(r, [r + 7]) for r in range(40)], [(r, [r + 9]) for r in range(36)]]
+        if grouped:
+            s._passes(passes)
+        else:
+            for p in passes:
+                s._unread = True
+                s._pass(p)
+        outs.append([c.clone().cpu() for c in s.mpk.model_builder.k_cache + s.mpk.model_builder.v_cache] + [s.step([(0, [5]), (1, [6]), (3, [7])], [[0]] * 3)[0].cpu()])
+        s.finalize()
+    assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*outs))
