@@ -4840,11 +4840,7 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       }
 #endif
       if (portion != shown) {
-        if (portion && portion != held) {
-          mk_portion_rows(rt, tok + 4 * MK_MAX_TOKENS, (int)threadIdx.x, M, portion);
-          held = portion;
-          __syncthreads();
-        }
+        mk_hold_portion(portion, held, [&]() { mk_portion_rows(rt, tok + 4 * MK_MAX_TOKENS, (int)threadIdx.x, M, portion); }, []() { __syncthreads(); });
         c.sh_tok = portion ? tok + 4 * MK_MAX_TOKENS : tok;
         shown = portion;
         one_each();

@@ -320,6 +320,17 @@ MK_HOST_DEVICE inline int mk_rows_ahead(int dealt, int G) {
 }
 MK_HOST_DEVICE inline int mk_first_row(int at, int ahead, int G) { return at >= ahead ? at - ahead : at - ahead + G; }
 
+// Tokens of one portion lie behind the first one's in LDS: `held` says whose.  load() puts another portion's there, by one wavefront, behind a barrier of the
+// workgroup, as a stage that was left out has none behind its look at them, and in front of one for those who read them.
+template <class Load, class Sync>
+MK_HOST_DEVICE inline void mk_hold_portion(int portion, int &held, Load load, Sync sync) {
+  if (portion == 0 || portion == held) return;
+  sync();
+  load();
+  held = portion;
+  sync();
+}
+
 // LDS map of MX_LATENT_ATTN, in bytes: query operands, one tile of cached rows, weights of the tile's positions, row statistics,
 // page-table entries.  RT: 16-row query tiles per unit; nkc: operand rows of a cached latent; sub: 16-position sub-tiles of a tile.
 struct MkLatentLds {

@@ -179,3 +179,24 @@ int main() {
 }
 ''')
     assert bad == 0 and programs == 1 and slices_left > 1
+
+
+def test_tokens_of_a_portion_replaced_behind_a_barrier(tmp_path):
+    """A left-out stage looks at its portion's tokens and has no barrier: another portion's take their place behind one, and are read behind one."""
+    src, exe = tmp_path / "hold.cpp", tmp_path / "hold"
+    src.write_text(r'''
+#include "mk_types.h"
+#include <stdio.h>
+#include <vector>
+int main() {
+  int held = 1;
+  for (int portion : {0, 1, 2, 2, 0, 2, 3, 1}) {
+    printf("%d", portion);
+    mk_hold_portion(portion, held, []() { printf("L"); }, []() { printf("|"); });
+    printf(" ");
+  }
+}
+''')
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "fleet-chiplet-megakernel_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split() == ["0", "1", "2|L|", "2", "0", "2", "3|L|", "1|L|"]
