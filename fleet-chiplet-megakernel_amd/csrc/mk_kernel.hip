@@ -136,6 +136,7 @@ struct Ctx {
   int defer_stage;         // the linear itself (its residual rows are each portion's own)
   int rows_ahead;          // where the running stage has dealt rows of portions in front already: mk_rows_ahead of them
   int portion;             // that the running stage runs for
+  bool keeps_sum;          // the running linear leaves no sum (mk_keeps_sum)
 #endif
 #if MK_HAVE_MIX
   bool mx_split;  // the latent attention (delta rule) that just ran left some request in chunks (its heads in slices)
@@ -2113,7 +2114,10 @@ __device__ __forceinline__ void stage_linear_mfma_xres(CStage &st, Ctx &c, const
   u32x4 *xpair = xl + 2 * XBUF + 16;  // a gate/up pair that two wavefronts hold
   u32x4 *part = (u32x4 *)rt.splitk_part;
   // hand the K-slice sum to the norm stage that follows, if there is one and the rows fit the partial buffer
-  const bool defer = (st.flags & MK_F_DEFER_SUM) && S > 1 && (size_t)S * (MT * 16) * st.n * 4 <= (size_t)c.G * 65536;
+  bool defer = (st.flags & MK_F_DEFER_SUM) && S > 1 && (size_t)S * (MT * 16) * st.n * 4 <= (size_t)c.G * 65536;
+#if MK_PAIR
+  defer = defer && !c.keeps_sum;
+#endif
   if (defer) {
     c.defer_S = S;
     c.defer_rows = MT * 16;
@@ -4801,8 +4805,8 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
     };
     one_each();
 #if MK_PAIR
-    int sum_S = 0, prep_S = 0;  // what the last linear for all portions left to the stage behind it; what was left to the last stage that prepares rows
-    bool all_through = true;
+    int sum_S = 0, prep_S = 0;  // what the last linear for all portions left to the stage behind it; what such a one left to the last stage that prepares rows
+    bool all_through = true, together = false;  // together: the last linear ran for all portions
     int again = 1, held = 1, shown = 0;  // the portion that entries for the second one and those behind it run for; whose tokens lie behind the first one's; c.sh_tok's
     for (int e = 0; e < rt.pair_n && !c.dead; e++) {
       const unsigned ent = (unsigned)__builtin_amdgcn_readfirstlane((int)((const __attribute__((address_space(4))) unsigned *)(unsigned long long)rt.pair_prog)[e]);
@@ -4861,7 +4865,11 @@ __device__ __forceinline__ void run_stage_program(const MkRuntime &rt, const MkR
       // reads normalised rows from the NORM stage's output: that stage then runs for one and two tokens as well)
 #if MK_PAIR
       // (a portion whose rows nobody prepares leaves its sum to the attention, which comes behind other portions' preparation)
-      if (FX && op == MK_OP_FX_PREP) prep_S = c.defer_S;
+      if (FX && op == MK_OP_LINEAR) {
+        c.keeps_sum = mk_keeps_sum(single, s + 1 < rt.num_stages ? (&st)[1].op : 0);
+        together = ent & MK_PAIR_BOTH;
+      }
+      if (FX && op == MK_OP_FX_PREP) prep_S = together ? c.defer_S : 0;
       if (FX && op == MK_OP_FX_ATTN && (ent & MK_PAIR_ON) && single) {
         c.defer_S = prep_S;
         c.defer_part = rt.group_part + (size_t)portion * MK_MAX_TOKENS * c.defer_n;
@@ -5173,6 +5181,7 @@ __device__ __forceinline__ void mk_kernel_body(const MkRuntime &rt, const MkRunt
   c.defer_n = 0;
   c.defer_stage = 0;
   c.portion = 0;
+  c.keeps_sum = false;
 #endif
   c.wrote_through = false;
   c.arrive_w0 = false;

@@ -66,12 +66,10 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
     };
     // (not a stage that may find a sum which a stage of the same run has left)
     auto first = [&](int q) { return q == i || !(stages[q - 1].flags & MK_F_DEFER_SUM); };
-    // Attention over pages, all of whose new rows the stage in front has put there.  A portion in which every request brings one row leaves the stage in front out,
-    // and what a linear of the same run has left to that one lies where the next portion's run of the linear puts its own: linear, preparation and attention
-    // then run together, portion by portion.
+    // attention over pages, all of whose new rows the stage in front has put there (or, of single rows, puts there itself: see mk_keeps_sum)
     auto prepared = [&](int q) {
       const MkStage &s = stages[q];
-      return s.op == MK_OP_FX_ATTN && q > i && first(q - 1) && stages[q - 1].op == MK_OP_FX_PREP && stages[q - 1].k_cache == s.k_cache && stages[q - 1].v_cache == s.v_cache;
+      return s.op == MK_OP_FX_ATTN && q > i && stages[q - 1].op == MK_OP_FX_PREP && stages[q - 1].k_cache == s.k_cache && stages[q - 1].v_cache == s.v_cache;
     };
     auto normed = [&](const MkStage &s) { return row_wise(s) && ((s.op == MK_OP_NORM && mk_norm_by_rows(s)) || s.op == MK_OP_FX_ADDNORM); };
     auto attends = [&](int q) {  // attention that may run for all portions at once, and what prepares its rows

@@ -320,6 +320,10 @@ MK_HOST_DEVICE inline int mk_rows_ahead(int dealt, int G) {
 }
 MK_HOST_DEVICE inline int mk_first_row(int at, int ahead, int G) { return at >= ahead ? at - ahead : at - ahead + G; }
 
+// Whether a portion's own run of a linear makes its sum itself, whatever the stage behind takes: a portion in which every request brings one row leaves the
+// preparation of its rows out, and the attention that reads them instead runs behind other portions' linears, which use the same partial sums.
+MK_HOST_DEVICE inline bool mk_keeps_sum(bool single, int next_op) { return single && next_op == MK_OP_FX_PREP; }
+
 // Tokens of one portion lie behind the first one's in LDS: `held` says whose.  load() puts another portion's there, by one wavefront, behind a barrier of the
 // workgroup, as a stage that was left out has none behind its look at them, and in front of one for those who read them.
 template <class Load, class Sync>

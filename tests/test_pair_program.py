@@ -15,10 +15,12 @@ static int slices(MkStage s) { return s.op == MK_OP_LINEAR && !(s.k & 63) ? mk_x
 static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &st, int portions, unsigned single, bool grouped) {
   const int n = (int)st.size();
   int bad = 0, steps = 0, defer = 0, sum = 0, prep = 0, group = -1, again = 1;  // group: the linear whose slices lie with those of all portions
+  bool together = false;                 // the last linear ran for all portions
   bool own = false;                      // what is left lies in the portion's own place ...
   int own_stage = -1, own_portion = -1;  // ... which holds this linear's
   int at = 0;                            // portion whose slices are looked at
   std::vector<int> next(portions, 0);    // stages that have run, in order
+  std::vector<int> kept(portions, -1);   // the portion's own linear that has made its sum itself
   auto ran = [&](int s, int p) { bad += next[p] != s; next[p] = s + 1; };
   auto left_by = [&](int s) {  // the linear whose sum a stage finds, or none
     int l = s - 1;
@@ -27,7 +29,7 @@ static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &s
   };
   auto takes = [&](int s, int p, bool all) {
     const int l = left_by(s);
-    if (l < 0) bad += defer != 0;
+    if (l < 0 || (!all && kept[p] == l)) bad += defer != 0;
     else if (all) bad += !defer || own || group != l;
     else bad += !defer || (own ? own_stage != l || own_portion != p : group != l || at != p);
     defer = 0;
@@ -53,7 +55,8 @@ static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &s
       own = false;
       at = p;
     }
-    if (op == MK_OP_FX_PREP) prep = defer;
+    if (op == MK_OP_LINEAR) together = all;
+    if (op == MK_OP_FX_PREP) prep = together ? defer : 0;
     if (op == MK_OP_FX_ATTN && (ent & MK_PAIR_ON) && one) {
       defer = prep;
       own = false;
@@ -89,7 +92,8 @@ static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &s
         bad += defer != 0;
         const int S = slices(st[s]);
         if (S > 1) own_stage = s, own_portion = p;
-        if (S > 1 && (st[s].flags & MK_F_DEFER_SUM)) defer = S, own = true;
+        if (S > 1 && (st[s].flags & MK_F_DEFER_SUM) && !mk_keeps_sum(one, s + 1 < n ? st[s + 1].op : 0)) defer = S, own = true;
+        else kept[p] = s;
       } else if (norm_op(op) || op == MK_OP_ATTN || op == MK_OP_FX_PREP || (op == MK_OP_FX_ATTN && one)) {
         takes(s, p, false);
       }
