@@ -1201,8 +1201,8 @@ __device__ __forceinline__ void fx_add_products(f32x4 &o0, f32x4 &o1, f32x4 &o2,
 //
 // Bound by round trips, hand-overs and chains of dependent instructions: a unit of stage_fx_attn_t waits for its page entries, its queries and its first tile,
 // for each tile's maximum, then for the other chunks' workgroups and what those have stored.  Here a task is two units, neighbouring row tiles of a
-// request, whose chains cover each other over the same tiles, with all of their chunks, whose partial results stay in LDS (those behind CHUNKS in memory
-// that only this workgroup reads); pages and queries of the next task are requested while one runs, and the first tile of the next chunk or task before
+// request, whose chains cover each other over the same tiles, with all of their chunks, whose partial results stay in LDS (those behind CHUNKS in memory,
+// written through: other layers' attention, with other units or portion by portion, uses the same words from other dies); pages and queries of the next task are requested while one runs, and the first tile of the next chunk or task before
 // sums are merged.  (Units whose chunks end at different tiles follow each other; few units are a task each.)  Chunks, sums and merges are those of
 // stage_fx_attn_t, in its order.  Six portions of 64 rows behind 1000 to 1500 positions, 32 q / 8 kv heads of 128: 96 us as a stage, portion by portion;
 // a unit a task 68, now 50.
@@ -1598,7 +1598,7 @@ __device__ __forceinline__ void fx_attn_group(Ctx &c, const MkRuntime &rt, int s
         for (int w = 0; w < MK_WAVES; w++) o += *(const f32x4 *)(pr + w * 16 * PSTR) * fin[w];
         if (a.C > 1) {  // (not one address for both: it would be a generic one)
           if (ci < CHUNKS) chunk_at[(e * CHUNKS + ci) * QUADS + q] = o;
-          else *far(e, ci, r, d) = o;
+          else stc_16B((u32x4 *)far(e, ci, r, d), __builtin_bit_cast(u32x4, o));
         } else if (r < (e ? a.nrows[1] : a.nrows[0]) && dv0 + d < DV) {
           emit(e, r, d, o);
         }
@@ -1621,7 +1621,7 @@ __device__ __forceinline__ void fx_attn_group(Ctx &c, const MkRuntime &rt, int s
         const float f = exp2f(cml[ci * 32] - M_);
         f32x4 x;
         if (ci < CHUNKS) x = chunk_at[(e * CHUNKS + ci) * QUADS + q];
-        else x = *far(e, ci, r, d);
+        else x = __builtin_bit_cast(f32x4, ldc_16B((const u32x4 *)far(e, ci, r, d)));
         L_ += cml[ci * 32 + 16] * f;
         o += x * f;
       }

@@ -192,3 +192,27 @@ def test_single_rows_whose_sums_lie_apart():
         outs.append([c.clone().cpu() for c in s.mpk.model_builder.k_cache + s.mpk.model_builder.v_cache] + [s.step([(0, [5]), (1, [6]), (3, [7])], [[0]] * 3)[0].cpu()])
         s.finalize()
     assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_attention_layers_of_unequal_shape():
+    """Heads of 128, attended for all portions at once with more chunks than LDS holds, and of 160, portion by portion, by turns: both leave partial results in the same words, and little is
+    streamed between them (two layers have a feed-forward)."""
+    import generate
+    from mirage.mpk import ServingSession
+    make, base = generate.SHAPES["suborax-2k"]
+    torch.manual_seed(7)
+    cfg = make(**{**base, "heads": 16, "kv_heads": 4}, layers=1, vocab=1000)
+    narrow = {**cfg["layers"][0], "mlp": None}
+    wide = {**narrow, "mixer": {**narrow["mixer"], "dim": 160}}
+    cfg["layers"] = [{**narrow, "mlp": cfg["layers"][0]["mlp"]}, wide, narrow, wide, narrow, {**wide, "mlp": cfg["layers"][0]["mlp"]}, narrow]
+    model, g = generate.random_model(cfg)[0], torch.Generator().manual_seed(9)
+    lengths, outs = (64 * 16 + 5, 64 * 9), []
+    prompts = [torch.randint(0, 1000, (n,), generator=g).tolist() for n in lengths]
+    for together in (8, 0):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=64 * 64, max_requests=2, max_seq_length=1088)
+        assert s.mpk.persistent_kernel.stats()["paired_portions"]
+        s._second, s._together = s._second if together else 0, together
+        outs.append([s.step([(i, p)], [[len(p) - 1]])[0].cpu() for i, p in enumerate(prompts)] + [s.step([(r, [3]) for r in range(2)], [[0]] * 2)[0].cpu()])
+        outs[-1] += [c.clone().cpu() for c in s.mpk.model_builder.k_cache + s.mpk.model_builder.v_cache]
+        s.finalize()
+    assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*outs))
