@@ -11,7 +11,7 @@
 // stages that put keys and values into pages and, behind them all, the attention over those pages, which looks at no position behind a row's own.  Norms by
 // rows run for all portions at once, and so does attention with what prepares its rows, unless the portions ask for another form: then the entries
 // behind, portion by portion, are the ones that run.
-// stages [0, n) on G workgroups.  Empty: no linear runs that way.
+// stages [0, n) on G workgroups.  Empty: no linear runs that way, or a run is longer than an entry can say.
 inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G) {
   std::vector<unsigned> prog;
   auto keeps_nothing = [&](const MkStage &s) { return !s.k_cache && !s.v_cache && !s.tail && !s.conv_w; };
@@ -41,6 +41,11 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
       if (stages[j].op == MK_OP_LINEAR) both[i] = 0;
   }
   if (std::count(both.begin(), both.end(), 1) == 0) return prog;
+  bool fits = true;
+  auto back = [&](size_t entries) -> unsigned {  // (all that is above the other bits)
+    fits = fits && entries < 1u << (32 - MK_PAIR_BACK_SHIFT);
+    return (unsigned)entries << MK_PAIR_BACK_SHIFT;
+  };
   for (int i = 0; i < n;) {
     if (both[i]) {
       prog.push_back(i++ | MK_PAIR_BOTH);
@@ -62,7 +67,7 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
       const size_t again = prog.size();
       if (carries) prog.push_back(MK_PAIR_ACQUIRE);
       for (int q = q0; q < q1; q++) prog.push_back(entry(q) | MK_PAIR_SECOND | (q == i && i > 0 ? MK_PAIR_AGAIN : 0));
-      prog.back() |= MK_PAIR_LOOP | (unsigned)(prog.size() - 1 - again) << MK_PAIR_BACK_SHIFT;
+      prog.back() |= MK_PAIR_LOOP | back(prog.size() - 1 - again);
     };
     // (not a stage that may find a sum which a stage of the same run has left)
     auto first = [&](int q) { return q == i || !(stages[q - 1].flags & MK_F_DEFER_SUM); };
@@ -86,7 +91,7 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
         const size_t at = prog.size();
         prog.push_back(q | MK_PAIR_BOTH);
         in_turn(q, e, alone(q));
-        prog[at] |= (unsigned)(prog.size() - at - 1) << MK_PAIR_BACK_SHIFT;
+        prog[at] |= back(prog.size() - at - 1);
       } else {
         if (!alone(q))
           while (e < j && !alone(e) && !attends(e) && !(first(e) && normed(stages[e]))) e++;
@@ -96,5 +101,6 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
     }
     i = j;
   }
+  if (!fits) prog.clear();
   return prog;
 }

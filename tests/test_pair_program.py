@@ -204,3 +204,20 @@ int main() {
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "fleet-chiplet-megakernel_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split() == ["0", "1", "2|L|", "2", "0", "2", "3|L|", "1|L|"]
+
+
+def test_runs_longer_than_an_entry_can_say(tmp_path):
+    """Stages between two linears for one portion after the other: as many as an entry's nine bits can go back over, or portions one by one."""
+    bad, short, long_ = _run(tmp_path, r'''
+int main() {
+  long bad = 0, programs[2] = {0, 0};
+  for (int len = 490; len < 700; len++)
+    for (int op : {(int)MK_OP_SILU_MUL, (int)MK_OP_HY_SCAN}) {
+      std::vector<MkStage> st(len, stage(op));
+      st.push_back(stage(MK_OP_LINEAR, 24576, 4096));
+      bad += walks(st, &programs[len > 512]);
+    }
+  printf("%ld %ld %ld\n", bad, programs[0], programs[1]);
+}
+''')
+    assert bad == 0 and short >= 44 and long_ == 0
