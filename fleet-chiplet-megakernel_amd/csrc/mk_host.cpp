@@ -3872,6 +3872,7 @@ int mk_init_requests(mk_graph *g) {
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending");
   HIP_TRY(hipSetDevice(g->cfg.device));
   const MkRuntime &rt = g->h_rt;
+  g->held.clear();
   HIP_TRY(hipDeviceSynchronize());
   HIP_TRY(hipMemset(rt.step, 0, sizeof(int) * rt.total_requests));
   HIP_TRY(hipMemset(rt.request_ids, 0xFF, sizeof(int) * rt.max_requests));
@@ -4047,8 +4048,10 @@ int mk_set_more_batches(mk_graph *g, int64_t words) {
 
 int mk_hold_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2) {
   if (const int rc = check_batches(g, at, words, second, words2)) return rc;
-  if (g->held.empty() != (at == 0)) return fail(MK_EINVAL, "the first batches are described from word 0 on, others behind them");
+  if (at == 0) g->held.clear();  // (what a caller that failed in between has left)
+  if (g->held.empty() && at) return fail(MK_EINVAL, "the first batches are described from word 0 on, others behind them");
   if ((int)g->held.size() + 2 > g->h_rt.group) return fail(MK_EINVAL, "this graph runs %d batches together at most (mk_stats.portions_together)", g->h_rt.group);
+  if (at && at < g->held.back().at + g->held.back().words) return fail(MK_EINVAL, "batches from word %lld on, behind those that end at word %lld", (long long)at, (long long)(g->held.back().at + g->held.back().words));
   g->held.push_back({at, words});
   g->held.push_back({at + second, words2});
   return MK_OK;

@@ -187,7 +187,8 @@ int mk_enqueue_batch(mk_graph *g, void *stream, int64_t words, int ingest);
 int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second, int64_t words2);
 /* More than two such batches as one launch, mk_stats.portions_together at most.  mk_set_more_batches: both places that mk_set_host_batch named go on for
  * `words` more words.  mk_hold_batches: two batches, described from word `at` (even) and from word `at + second` on, run with the next mk_enqueue_held,
- * behind those held so far; the first ones' `at` is 0.  mk_enqueue_held launches them and holds none from then on (neither does naming other words). */
+ * behind those held so far, whose descriptions end in front of word `at`.  Word 0: none are held so far, whatever a caller that failed has left.
+ * mk_enqueue_held launches them and holds none from then on (neither do mk_init_requests and naming other words). */
 int mk_set_more_batches(mk_graph *g, int64_t words);
 int mk_hold_batches(mk_graph *g, int64_t at, int64_t words, int64_t second, int64_t words2);
 int mk_enqueue_held(mk_graph *g, void *stream);

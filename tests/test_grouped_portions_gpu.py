@@ -216,3 +216,30 @@ def test_attention_layers_of_unequal_shape():
         outs[-1] += [c.clone().cpu() for c in s.mpk.model_builder.k_cache + s.mpk.model_builder.v_cache]
         s.finalize()
     assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_batches_that_a_failed_caller_has_left():
+    """Held batches of a caller that failed before it could launch them: the next one's first batches, from word 0 on, begin anew, and so do requests; descriptions that overlap are refused."""
+    from mirage import _capi
+    from mirage.mpk import ServingSession
+    model, outs = _model("suborax"), []
+    toks = torch.randint(0, 1000, (64 * 6 + 9,), generator=torch.Generator().manual_seed(9)).tolist()
+    for left in (False, True):
+        s = ServingSession.open(model_config=model, dtype=torch.bfloat16, max_tokens=2048, max_requests=2, max_seq_length=512)
+        pk, at, apart = s.mpk.persistent_kernel, s._second, s._apart
+        if left:
+            words = [s._put(i // 2 * apart + i % 2 * at, *s._describe([("gone", list(range(64)))])[:2]) for i in range(4)]
+            s.end("gone")
+            pk.enqueue_batches(words[0], at, words[1], hold=True)
+            with pytest.raises(_capi.MkError, match="behind those that end at word"):
+                pk.enqueue_batches(words[2], at, words[3], at=at, hold=True)
+            pk.enqueue_batches(words[2], at, words[3], at=apart, hold=True)
+        outs.append([s.step([("a", toks)], [[len(toks) - 1]])[0].cpu()] + [c.clone().cpu() for c in s.mpk.model_builder.k_cache])
+        assert pk.stats()["iterations"] == 7
+        if left:
+            pk.enqueue_batches(words[0], at, words[1], hold=True)
+            pk._g.init_requests()
+            with pytest.raises(_capi.MkError, match="no batches are held"):
+                pk._g.enqueue_held(pk._stream_ptr(None))
+        s.finalize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
