@@ -3999,9 +3999,9 @@ static int check_batches(mk_graph *g, int64_t at, int64_t words, int64_t second,
   if (!g->compiled) return fail(MK_ESTATE, "mk_compile has not been called");
   if (!g->h_rt.pair_n || g->h_rt.profiler) return fail(MK_EUNSUPPORTED, "this graph runs portions of prompts one by one");
   const int64_t cap = g->batch_cap + (at ? g->batch_more : 0);
-  if (words < 1 || words2 < 1 || second < words || at < 0 || at + second + words2 > cap || ((second | at) & 1))
+  if (words < 1 || words2 < 1 || second < words || at < 0 || at > cap || second > cap || words2 > cap || at + second + words2 > cap || ((second | at) & 1))  // (one by one: sums of any three may wrap)
     return fail(MK_EINVAL, "batches of %lld words from word %lld and of %lld from word %lld on, mk_set_host_batch named %lld", (long long)words, (long long)at, (long long)words2,
-                (long long)(at + second), (long long)cap);
+                (long long)((unsigned long long)at + (unsigned long long)second), (long long)cap);
   // the descriptions are read `at` and `at + second` words behind every tensor of the graph: all of that is in the named words
   auto named = [&](const void *p, size_t bytes) { return !p || ((const char *)p >= (const char *)g->batch_dst && (const char *)p + 4 * (at + second) + bytes <= (const char *)(g->batch_dst + cap)); };
   const mk_config &c = g->cfg;
@@ -4036,7 +4036,7 @@ int mk_enqueue_batches(mk_graph *g, void *stream, int64_t words, int64_t second,
 int mk_set_more_batches(mk_graph *g, int64_t words) {
   if (!g) return fail(MK_EINVAL, "null argument");
   if (g->launch_pending) return fail(MK_ESTATE, "a launch is still pending");
-  if (!g->batch_cap || words < 0 || g->batch_cap + words > (1ll << 28)) return fail(MK_EINVAL, "%lld words behind those that mk_set_host_batch named (%lld)", (long long)words, (long long)g->batch_cap);
+  if (!g->batch_cap || words < 0 || words > (1ll << 28) - g->batch_cap) return fail(MK_EINVAL, "%lld words behind those that mk_set_host_batch named (%lld)", (long long)words, (long long)g->batch_cap);
   HIP_TRY(hipSetDevice(g->cfg.device));
   const size_t bytes = 4 * (size_t)(g->batch_cap + words);
   if (device_view(g->batch_host, bytes, hipMemoryTypeHost, g->cfg.device) != (void *)g->batch_src || device_view(g->batch_dst, bytes, hipMemoryTypeDevice, g->cfg.device) != (void *)g->batch_dst)

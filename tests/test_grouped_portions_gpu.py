@@ -243,3 +243,21 @@ def test_batches_that_a_failed_caller_has_left():
                 pk._g.enqueue_held(pk._stream_ptr(None))
         s.finalize()
     assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_numbers_of_words_whose_sums_wrap():
+    from mirage import _capi
+    from mirage.mpk import ServingSession
+    s = ServingSession.open(model_config=_model("suborax"), max_tokens=1024, max_requests=2, max_seq_length=512)
+    pk, at, apart, most = s.mpk.persistent_kernel, s._second, s._apart, 2 ** 63 - 2
+    for words, second, words2 in ((4, at, most), (4, most, 4), (most, most, 4), (4, most, most)):
+        with pytest.raises(_capi.MkError, match="mk_set_host_batch named"):
+            pk.enqueue_batches(words, second, words2)
+        for far in (0, apart, most):
+            with pytest.raises(_capi.MkError, match="mk_set_host_batch named"):
+                pk._g.hold_batches(far, words, second, words2)
+    with pytest.raises(_capi.MkError, match="mk_set_host_batch named"):
+        pk._g.hold_batches(most, 4, at, 4)
+    with pytest.raises(_capi.MkError, match="words behind those"):
+        pk.attach_more_batches(most)
+    s.finalize()
