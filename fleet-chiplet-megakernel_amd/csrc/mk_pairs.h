@@ -33,6 +33,11 @@ inline std::vector<unsigned> mk_pair_program(const MkStage *stages, int n, int G
     MkStage s = stages[i];
     both[i] = s.op == MK_OP_LINEAR && keeps_nothing(s) && (s.k & 63) == 0 && mk_xres_plan(s, G).S >= 1;
   }
+  // a convolution reads the request's last inputs, which the scan behind it writes: for a portion that must be those of the one in front, so nothing between the two
+  // runs for all portions
+  for (int i = 0; i < n; i++)
+    for (int j = n - 1; j > i && stages[i].tail; j--)
+      if (stages[j].tail == stages[i].tail) std::fill(both.begin() + i, both.begin() + j, 0);
   // what says where a sum is that was left to the stage behind says so of the last linear that left one, and is kept until all portions have read it: by a
   // stage that runs for all of them at once, or with no other linear in between
   for (int i = n - 1; i >= 0; i--) {

@@ -21,7 +21,11 @@ static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &s
   int at = 0;                            // portion whose slices are looked at
   std::vector<int> next(portions, 0);    // stages that have run, in order
   std::vector<int> kept(portions, -1);   // the portion's own linear that has made its sum itself
-  auto ran = [&](int s, int p) { bad += next[p] != s; next[p] = s + 1; };
+  auto ran = [&](int s, int p) {
+    bad += next[p] != s;
+    next[p] = s + 1;
+    for (int j = s + 1; j < n && p; j++) bad += st[s].tail && st[j].tail == st[s].tail && next[p - 1] <= j;  // (reads what the portion in front leaves there)
+  };
   auto left_by = [&](int s) {  // the linear whose sum a stage finds, or none
     int l = s - 1;
     if (st[s].op == MK_OP_FX_ATTN && l >= 0 && st[l].op == MK_OP_FX_PREP) l--;
@@ -104,7 +108,7 @@ static int walk(const std::vector<unsigned> &prog, const std::vector<MkStage> &s
   for (int q = 0; q < portions; q++) bad += next[q] != n;
   return bad;
 }
-static char caches[8];
+static char caches[64];
 static MkStage stage(int op, int n = 0, int k = 0, unsigned flags = 0) {
   MkStage s;
   memset(&s, 0, sizeof(s));
@@ -113,7 +117,6 @@ static MkStage stage(int op, int n = 0, int k = 0, unsigned flags = 0) {
   s.k = k;
   s.flags = flags;
   if (op == MK_OP_FX_PREP || op == MK_OP_FX_ATTN || op == MK_OP_ATTN) s.k_cache = caches, s.v_cache = caches + 1, s.num_q_heads = 32, s.num_kv_heads = 8;
-  if (op == MK_OP_HY_SCAN) s.tail = caches + 2;
   return s;
 }
 static int walks(const std::vector<MkStage> &st, long *programs) {
@@ -138,7 +141,7 @@ def _run(tmp_path, main):
 
 
 def test_programs_of_any_stages(tmp_path):
-    """Sequences of norms, linears (whole, in slices, none that stream; their sums left to the stage behind or not), attention with its preparation, and others."""
+    """Sequences of norms, linears (whole, in slices, none that stream; their sums left to the stage behind or not), attention with its preparation, convolutions and scans, and others."""
     bad, programs = _run(tmp_path, r'''
 int main() {
   long bad = 0, programs = 0;
@@ -149,14 +152,22 @@ int main() {
     std::vector<MkStage> st;
     const bool fx = draw(2);
     for (int len = 3 + draw(14); (int)st.size() < len;) {
-      switch (draw(6)) {
+      switch (draw(7)) {
         case 0: st.push_back(stage(fx ? MK_OP_FX_ADDNORM : MK_OP_NORM, 2048, draw(4) ? 2048 : 2044)); break;
         case 1: if (fx) st.push_back(stage(MK_OP_MX_PRENORM, 2048)); break;
         case 2:
           if (fx) st.push_back(stage(MK_OP_FX_PREP));
           st.push_back(stage(fx ? MK_OP_FX_ATTN : MK_OP_ATTN));
           break;
-        case 3: st.push_back(stage(draw(2) ? MK_OP_SILU_MUL : MK_OP_HY_SCAN)); break;
+        case 3: st.push_back(stage(draw(2) ? MK_OP_SILU_MUL : MK_OP_HY_STEP)); break;
+        case 4:  // (a convolution reads the request's last inputs, which the scan behind it writes)
+          st.push_back(stage(MK_OP_HY_CONV));
+          st.back().tail = caches + st.size();
+          if (draw(3)) st.push_back(stage(MK_OP_LINEAR, ns[draw(5)], ks[draw(6)]));
+          if (draw(2)) st.push_back(stage(MK_OP_HY_STEP));
+          st.push_back(stage(MK_OP_HY_SCAN));
+          for (size_t i = st.size() - 1; st[i].op != MK_OP_HY_CONV; i--) st.back().tail = st[i - 1].tail;
+          break;
         default: st.push_back(stage(MK_OP_LINEAR, ns[draw(5)], ks[draw(6)]));
       }
     }
