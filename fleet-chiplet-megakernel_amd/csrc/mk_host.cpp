@@ -2359,7 +2359,7 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions) {
   }
   size_t bytes = 0;
   for (const auto &e : rows.at) bytes += (e.second - e.first + 255) / 256 * 256;
-  int P = MK_GROUP;
+  int P = mk_most_portions(g->G);
   void *block = nullptr;
   for (; P > 1; P /= 2) {  // (the ids in front)
     if (dev_alloc(g, &block, (size_t)(P - 1) * (sizeof(int64_t) * MK_MAX_TOKENS + bytes), false) == MK_OK) break;

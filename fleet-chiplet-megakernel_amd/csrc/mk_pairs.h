@@ -5,6 +5,13 @@
 
 #include "mk_types.h"
 
+// Portions that run together on G workgroups at most: a wavefront prepares rows of one portion for the attention of all, so every portion needs one.
+inline int mk_most_portions(int G) {
+  int portions = MK_GROUP;
+  while (portions > G * MK_WAVES) portions /= 2;
+  return portions;
+}
+
 // Several portions inside prompts as one iteration (MkPairEntry): linears that run for all portions at once, and between two of them the stages of
 // the first portion, then those of the second, and so on, as iterations of their own would run them.  What a cache or a state gets from a portion is
 // written back and read anew in front of the next one; stages that only take rows to rows run for one portion after the other without a barrier, and so do

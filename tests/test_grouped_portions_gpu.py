@@ -266,12 +266,22 @@ def test_numbers_of_words_whose_sums_wrap():
 @pytest.mark.parametrize("workgroups", [2, 8, 16])
 def test_convolutions_that_read_what_scans_leave(workgroups):
     """Where few workgroups have the small linear between a convolution and its scan run for all portions: not before the portion in front has left its last inputs."""
+    _offline_grid("bukatar", workgroups, 8)
+
+
+@pytest.mark.parametrize("family", ["suborax", "bukatar"])
+def test_fewer_wavefronts_than_portions(family):
+    """One workgroup has four wavefronts, each of which prepares rows of one portion: no more portions run together."""
+    _offline_grid(family, 1, 4)
+
+
+def _offline_grid(family, workgroups, together):
     import generate
-    model, outs = _model("bukatar"), []
+    model, outs = _model(family), []
     prompt = torch.randint(0, 1000, (64 * 9 + 5,), generator=torch.Generator().manual_seed(6))
     for pairs in (True, False):
         gen = generate.Generator(600, model_config=model, batch=1, max_num_batched_tokens=64, max_tokens_per_request=64, page_size=64, eos_token_id=-1, pair_portions=pairs, num_workers=workgroups)
-        assert gen.mpk.stats()["paired_portions"] == pairs
+        assert gen.mpk.stats()["portions_together"] == (together if pairs else 1)
         gen.load_prompts([prompt])
         gen.mpk.run_steps(10)
         outs.append([t.clone().cpu() for t in [gen.logits()[:5], *_kept(gen.model.model_builder)]])

@@ -217,6 +217,11 @@ int main() {
     assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split() == ["0", "1", "2|L|", "2", "0", "2", "3|L|", "1|L|"]
 
 
+def test_every_portion_has_a_wavefront(tmp_path):
+    most = _run(tmp_path, 'int main() { for (int G : {1, 2, 3, 256}) printf("%d ", mk_most_portions(G)); }')
+    assert most == [4, 8, 8, 8]
+
+
 def test_runs_longer_than_an_entry_can_say(tmp_path):
     """Stages between two linears for one portion after the other: as many as an entry's nine bits can go back over, or portions one by one."""
     bad, short, long_ = _run(tmp_path, r'''
