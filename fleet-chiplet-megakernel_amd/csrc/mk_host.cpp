@@ -2313,10 +2313,38 @@ std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
   return prog;
 }
 
+constexpr size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+
+// Scratch of iterations of several portions, in one piece: what lies where, in bytes.
+struct GroupScratch {
+  size_t stages, prog, part, attn, q, cnt, bytes;
+};
+GroupScratch group_scratch(const mk_graph *g, int portions) {
+  size_t part = 0;  // floats of partial sums
+  int heads = 0;    // of queries prepared ahead of the attention
+  for (const unsigned e : g->pair_prog) {
+    if (!(e & MK_PAIR_BOTH)) continue;
+    MkStage s = g->stages[e & MK_PAIR_STAGE];
+    if (s.op == MK_OP_ATTN) heads = std::max(heads, s.num_q_heads);
+    if (s.op != MK_OP_LINEAR) continue;
+    const XresPlan plan = mk_xres_plan(s, g->G);
+    if (plan.S > 1) part = std::max(part, (size_t)plan.S * portions * MK_MAX_TOKENS * std::max(plan.wt * 16, s.n));
+  }
+  GroupScratch at;
+  at.stages = 0;
+  at.prog = align256(sizeof(MkStage) * (portions - 1) * g->stages.size());
+  at.part = at.prog + align256(sizeof(unsigned) * g->pair_prog.size());
+  at.attn = at.part + align256(part * sizeof(float));
+  at.q = at.attn + portions * align256(g->flex_part * sizeof(float));
+  at.cnt = at.q + align256((size_t)portions * MK_MAX_TOKENS * heads * 256);
+  at.bytes = at.cnt + portions * g->flex_items * 32 * sizeof(unsigned);
+  return at;
+}
+
 // The stages as they run for the second portion and those behind it: over rows of their own, in copies of the memory that stages write rows to.  *portions:
 // as many run together at most, fewer where memory is short; 1: some stage could not be told apart from the first portion's, or not even one copy fits, and
-// portions run one by one.
-int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions) {
+// portions run one by one.  *scratch: what they need beside those rows (group_scratch), in the same piece of memory, so that all of it is there or none.
+int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions, char **scratch) {
   const mk_config &c = g->cfg;
   *portions = 1;
   Extents held, rows;  // tensors and allocations; those among them that stages write rows to
@@ -2361,11 +2389,13 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions) {
   for (const auto &e : rows.at) bytes += (e.second - e.first + 255) / 256 * 256;
   int P = mk_most_portions(g->G);
   void *block = nullptr;
-  for (; P > 1; P /= 2) {  // (the ids in front)
-    if (dev_alloc(g, &block, (size_t)(P - 1) * (sizeof(int64_t) * MK_MAX_TOKENS + bytes), false) == MK_OK) break;
+  auto own_bytes = [&](int P) { return (size_t)(P - 1) * (sizeof(int64_t) * MK_MAX_TOKENS + bytes); };  // (the ids in front)
+  for (; P > 1; P /= 2) {
+    if (dev_alloc(g, &block, own_bytes(P) + group_scratch(g, P).bytes, false) == MK_OK) break;
     (void)hipGetLastError();
   }
   if (P < 2) return MK_OK;
+  *scratch = (char *)block + own_bytes(P);
   int64_t *ids = (int64_t *)block;
   g->h_rt.ids2 = (long long *)ids;
   char *const first_rows = (char *)(ids + (size_t)(P - 1) * MK_MAX_TOKENS), *to = first_rows;
@@ -3338,7 +3368,6 @@ int do_wait(mk_graph *g, hipStream_t stream, int *finished_out) {
 // sampling stages' per-workgroup partials -- taken from this file-scope device array instead of from the buffers
 // mk_compile allocated.  Each GPU the library runs on holds its own copy of the array until the process ends.
 // Sizes are for the largest launch the entry point accepts (256 workgroups, 64 tokens x 8 kv heads, 8 q heads per kv head).
-constexpr size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 constexpr int MK_STATIC_MAX_WG = 256;
 constexpr int MK_STATIC_MAX_ITEMS = MK_MAX_TOKENS * 8;  // (token, kv head) pairs
 constexpr int MK_STATIC_MAX_QPK = 8;
@@ -3822,41 +3851,23 @@ int mk_compile(mk_graph *g) {
   if (pairs) {  // (behind all other memory that the graph needs: where this does not fit, portions run one by one)
     std::vector<MkStage> second;
     int portions;
-    if ((rc = second_stages(g, second, &portions))) return rc;
-    while (portions > 1) {
-      const size_t bytes = sizeof(MkStage) * (portions - 1) * g->stages.size(), prog = align256(sizeof(unsigned) * g->pair_prog.size());
-      size_t part = 0;  // floats of partial sums
-      int heads = 0;    // of queries prepared ahead of the attention
-      for (const unsigned e : g->pair_prog) {
-        if (!(e & MK_PAIR_BOTH)) continue;
-        MkStage &s = g->stages[e & MK_PAIR_STAGE];
-        if (s.op == MK_OP_ATTN) heads = std::max(heads, s.num_q_heads);
-        if (s.op != MK_OP_LINEAR) continue;
-        const XresPlan plan = mk_xres_plan(s, g->G);
-        if (plan.S > 1) part = std::max(part, (size_t)plan.S * portions * MK_MAX_TOKENS * std::max(plan.wt * 16, s.n));
-      }
-      const size_t attn = align256(g->flex_part * sizeof(float)), items = g->flex_items;
-      const size_t at_prog = align256(bytes), at_part = at_prog + prog, at_attn = at_part + align256(part * sizeof(float)), at_q = at_attn + portions * attn, at_cnt = at_q + align256((size_t)portions * MK_MAX_TOKENS * heads * 256),
-                   cnt = portions * items * 32 * sizeof(unsigned);
-      if (dev_alloc(g, &p, at_cnt + cnt, false) != MK_OK) {
-        (void)hipGetLastError();
-        portions /= 2;
-        continue;
-      }
-      HIP_TRY(hipMemcpy(p, second.data(), bytes, hipMemcpyHostToDevice));
-      HIP_TRY(hipMemcpy((char *)p + at_prog, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
-      rt.stages2 = (const MkStage *)p;
-      rt.pair_prog = (const unsigned *)((char *)p + at_prog);
-      rt.group_part = (float *)((char *)p + at_part);
-      rt.group_q = (uint16_t *)((char *)p + at_q);
-      rt.group_attn_part = (float *)((char *)p + at_attn);
-      rt.group_attn = (long long)(attn / sizeof(float));
-      rt.group_attn_cnt = (unsigned *)((char *)p + at_cnt);
-      rt.group_cnt = (long long)items;
-      g->group_cnt_bytes = cnt;
+    char *at;
+    if ((rc = second_stages(g, second, &portions, &at))) return rc;
+    if (portions > 1) {
+      const GroupScratch lies = group_scratch(g, portions);
+      HIP_TRY(hipMemcpy(at + lies.stages, second.data(), sizeof(MkStage) * second.size(), hipMemcpyHostToDevice));
+      HIP_TRY(hipMemcpy(at + lies.prog, g->pair_prog.data(), sizeof(unsigned) * g->pair_prog.size(), hipMemcpyHostToDevice));
+      rt.stages2 = (const MkStage *)(at + lies.stages);
+      rt.pair_prog = (const unsigned *)(at + lies.prog);
+      rt.group_part = (float *)(at + lies.part);
+      rt.group_q = (uint16_t *)(at + lies.q);
+      rt.group_attn_part = (float *)(at + lies.attn);
+      rt.group_attn = (long long)(align256(g->flex_part * sizeof(float)) / sizeof(float));
+      rt.group_attn_cnt = (unsigned *)(at + lies.cnt);
+      rt.group_cnt = (long long)g->flex_items;
+      g->group_cnt_bytes = lies.bytes - lies.cnt;
       rt.pair_n = (int)g->pair_prog.size();
       rt.group = portions;
-      break;
     }
   }
   if ((rc = upload_runtime(g))) return rc;
