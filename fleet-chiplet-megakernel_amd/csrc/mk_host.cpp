@@ -2387,13 +2387,13 @@ int second_stages(mk_graph *g, std::vector<MkStage> &out, int *portions, char **
   }
   size_t bytes = 0;
   for (const auto &e : rows.at) bytes += (e.second - e.first + 255) / 256 * 256;
-  int P = mk_most_portions(g->G);
   void *block = nullptr;
   auto own_bytes = [&](int P) { return (size_t)(P - 1) * (sizeof(int64_t) * MK_MAX_TOKENS + bytes); };  // (the ids in front)
-  for (; P > 1; P /= 2) {
-    if (dev_alloc(g, &block, own_bytes(P) + group_scratch(g, P).bytes, false) == MK_OK) break;
+  const int P = mk_portions_that_fit(g->G, [&](int P) {
+    if (dev_alloc(g, &block, own_bytes(P) + group_scratch(g, P).bytes, false) == MK_OK) return true;
     (void)hipGetLastError();
-  }
+    return false;
+  });
   if (P < 2) return MK_OK;
   *scratch = (char *)block + own_bytes(P);
   int64_t *ids = (int64_t *)block;

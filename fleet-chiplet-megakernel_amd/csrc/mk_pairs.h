@@ -11,6 +11,13 @@ inline int mk_most_portions(int G) {
   while (portions > G * MK_WAVES) portions /= 2;
   return portions;
 }
+// As many of them as allocate(portions) finds memory for: all, a half, a quarter; 1: not even for two.
+template <class Allocate>
+inline int mk_portions_that_fit(int G, Allocate allocate) {
+  int portions = mk_most_portions(G);
+  while (portions > 1 && !allocate(portions)) portions /= 2;
+  return portions;
+}
 
 // Several portions inside prompts as one iteration (MkPairEntry): linears that run for all portions at once, and between two of them the stages of
 // the first portion, then those of the second, and so on, as iterations of their own would run them.  What a cache or a state gets from a portion is

@@ -287,58 +287,3 @@ def _offline_grid(family, workgroups, together):
         outs.append([t.clone().cpu() for t in [gen.logits()[:5], *_kept(gen.model.model_builder)]])
         gen.finalize()
     assert all(torch.equal(a, b) for a, b in zip(*outs))
-
-
-def test_as_many_portions_as_fit_the_memory(monkeypatch):
-    """Rows and scratch of eight portions, four or two are there whole or not at all: a graph of fewer keeps no rows of the others, and its results are the same."""
-    import gc
-    import generate
-    from mirage import _capi
-    from mirage.mpk import MPK
-    model, compile_, free = _model("suborax"), MPK.compile, lambda: torch.cuda.mem_get_info()[0]
-    prompt = torch.randint(0, 1000, (64 * 9 + 5,), generator=torch.Generator().manual_seed(6))
-    used = {}
-
-    def fill(leave):
-        gc.collect()
-        torch.cuda.empty_cache()
-        torch.cuda.synchronize()
-        held = []
-        while free() > leave + (4 << 20) and len(held) < 8:  # (a large piece takes less than it says)
-            held.append(torch.empty(free() - leave, dtype=torch.uint8, device="cuda"))
-        return held
-
-    def run(pairs, leave):
-        def compiled(mpk):  # (only this has so little memory)
-            held, before = fill(leave), free()
-            compile_(mpk)
-            used[pairs and mpk.persistent_kernel.stats()["portions_together"]] = before - free()
-            held.clear()
-            torch.cuda.empty_cache()
-        monkeypatch.setattr(MPK, "compile", compiled)
-        gen = generate.Generator(600, model_config=model, batch=1, max_num_batched_tokens=64, max_tokens_per_request=64, page_size=64, eos_token_id=-1, pair_portions=pairs)
-        together = gen.mpk.stats()["portions_together"]
-        gen.load_prompts([prompt])
-        gen.mpk.run_steps(10)
-        out = [t.clone().cpu() for t in [gen.logits()[:5], *_kept(gen.model.model_builder)]]
-        gen.finalize()
-        return together, out
-
-    most = fill(4 << 30)
-    run(True, 1 << 30)  # (the first one of a process has the runtime's own on top)
-    for _ in range(2):
-        alone = run(False, 288 << 20)[1]
-    seen = []
-    for leave in range(320 << 20, 0, -(8 << 20)):
-        try:
-            together, out = run(True, leave)
-        except _capi.MkError:  # (the weights' copies do not fit any more)
-            break
-        seen.append(together)
-        assert all(torch.equal(a, b) for a, b in zip(out, alone))
-        if together == 1:
-            break
-    del most
-    assert {8, 4} <= set(seen) <= {8, 4, 2, 1}
-    assert used[4] < used[False] + 0.55 * (used[8] - used[False])  # (a half, and what pieces are rounded up to)
-    assert 1 not in used or used[1] < used[False] + (4 << 20)

@@ -222,6 +222,19 @@ def test_every_portion_has_a_wavefront(tmp_path):
     assert most == [4, 8, 8, 8]
 
 
+def test_as_many_portions_as_fit_the_memory(tmp_path):
+    """Rows and scratch are asked for in one piece, for as many portions as a grid can have, then half of them and so on, until a piece is there."""
+    tried = _run(tmp_path, r'''
+int main() {
+  for (int G : {256, 1})
+    for (int room : {8, 7, 4, 3, 2, 1, 0}) printf("%d 0 ", mk_portions_that_fit(G, [&](int p) { printf("%d ", p); return p <= room; }));
+}
+''')
+    wide = [[8, 8], [8, 4, 4], [8, 4, 4], [8, 4, 2, 2], [8, 4, 2, 2], [8, 4, 2, 1], [8, 4, 2, 1]]
+    narrow = [[4, 4]] * 3 + [[4, 2, 2], [4, 2, 2], [4, 2, 1], [4, 2, 1]]
+    assert tried == [x for t in wide + narrow for x in t + [0]]
+
+
 def test_runs_longer_than_an_entry_can_say(tmp_path):
     """Stages between two linears for one portion after the other: as many as an entry's nine bits can go back over, or portions one by one."""
     bad, short, long_ = _run(tmp_path, r'''
