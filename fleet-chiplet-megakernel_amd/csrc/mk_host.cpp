@@ -4156,6 +4156,7 @@ int mk_run_once(mk_graph *g, void *stream, int num_tokens, const int32_t *tok_sl
   return do_wait(g, s, nullptr);
 }
 
+static_assert(sizeof(mk_stats) == 72, "callers built before portions_together, which lies where their struct was padded, have as many bytes");
 int mk_get_stats(mk_graph *g, mk_stats *out) {
   if (!g || !out) return fail(MK_EINVAL, "null argument");
   memset(out, 0, sizeof(*out));
