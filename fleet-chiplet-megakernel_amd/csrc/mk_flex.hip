@@ -1247,7 +1247,7 @@ __device__ __forceinline__ void fx_attn_group(Ctx &c, const MkRuntime &rt, int s
   using X = FxType<E>;
   static_assert(sizeof(E) == 2, "16-bit activations");
   constexpr int EPC = X::EPC, KW = X::KW, TP = X::TP, SUB = X::SUB, NU = 2, ROWS = MK_GROUP * MK_MAX_TOKENS;
-  constexpr int PSTR = VB * 16 + 4, PST = VB * 16 + 32, QUADS = 16 * VB * 4, NE = QUADS / MK_THREADS, CHUNKS = 3, QMAX = KC * 64, PG = MK_ATTN_PAIR_PAGES / MK_THREADS;
+  constexpr int PSTR = VB * 16 + 4, PST = VB * 16 + 32, QUADS = 16 * VB * 4, CHUNKS = 3, QMAX = KC * 64, PG = MK_ATTN_PAIR_PAGES / MK_THREADS;
   static_assert(QUADS % MK_THREADS == 0, "a merged chunk is whole quads of all threads");
   // LDS: query operands of this task and the next, page lists of both, the tokens' positions, first page-table entries and FxGroupRows::row, the wavefronts' sums, chunks
   u32x4 *const q_at = (u32x4 *)smem;

@@ -440,7 +440,8 @@ __device__ __forceinline__ void stage_norm_group(CStage &st, Ctx &c, const MkRun
 //
 // First every portion's rows are prepared (q/k norm, rotation; keys and values into their pages, queries into a scratch), then, behind a barrier, all
 // portions' tokens are attended at once, everything out of the pages.  Portions one after the other, each with a barrier, a write-back and an invalidate in
-// between, prepared a portion's key and value rows in every unit of sixteen query rows: 512 tokens behind 1540 of 32 q / 8 kv heads 377 us as a stage, now 132.
+// between, prepared a portion's key and value rows in every unit of sixteen query rows: 512 tokens of 32 q / 8 kv heads, as a stage, were 377 us
+// behind 1540 positions; now 132 behind about 2000 (112 behind 1536, by themselves).
 //
 // A task is up to two units of stage_attn_tiles, neighbouring token groups of one request and kv head: a cached tile, once in LDS, is scored against all
 // their queries, and its values, read back transposed, are packed once.  Sums are made as that stage makes them: a unit's chunks are as many and end where

@@ -2287,9 +2287,10 @@ int tail_stage(const mk_graph *g) {
 //
 // *worth: pairs at the beginning of an offline launch that pay for the kernel they run in, which is 42 us of launch and handshake.  A pair gains, against its
 // portions one by one, about 8 us for every linear that runs for both and 0.05 us for every megabyte of their weights, and loses 7.5 where one portion
-// hands over to the other; expert linears of many tokens are 6 us faster in that kernel.  By that rule / measured, us a pair (25 portions of one
-// prompt, four layers): qwen3-8b 134 / 174, its width with 1536 columns 69 / 74, 2048 wide with 6144 columns and 2 / 6 kv heads 2 / 4 and 11 / 12, qwen3-30b-a3b
-// 90 / 96, suborax-8b 134 / 188, -2k 64 / 55, dodonex-8b 61 / 97, -2k 17 / 10, bukatar-8b 103 / 132, -2k 25 / 25, vizonex-8b 39 / 18, -2k 9 / 17.
+// hands over to the other; expert linears of many tokens are 6 us faster in that kernel.  The figures are of iterations of two portions: those of more, norms and
+// attention for all portions at once, and hand-overs that such attention leaves out are not in them, so that launches begin this way later than pays rather than
+// sooner.  By that rule / measured, us a pair, when no more than two ran together (25 portions of one prompt, four layers): qwen3-8b 134 / 174, its width with
+// 1536 columns 69 / 74, 2048 wide with 6144 columns and 2 / 6 kv heads 2 / 4 and 11 / 12, qwen3-30b-a3b 90 / 96, suborax-8b 134 / 188, -2k 64 / 55, dodonex-8b 61 / 97, -2k 17 / 10, bukatar-8b 103 / 132, -2k 25 / 25, vizonex-8b 39 / 18, -2k 9 / 17.
 std::vector<unsigned> pair_program(const mk_graph *g, int *worth) {
   std::vector<unsigned> prog;
   const mk_config &c = g->cfg;
