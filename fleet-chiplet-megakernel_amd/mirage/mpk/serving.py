@@ -322,7 +322,8 @@ class ServingSession:
     # ------------------------------------------------------------------ greedy generation
     def generate(self, prompts: Sequence[Sequence[int]], max_new_tokens: int, eos_token_id: int = -1) -> List[List[int]]:
         """Greedy continuation of every prompt, continuously batched: a request is admitted when a batch slot and the pages
-        for its whole length are free; prompts enter in portions beside the running requests' tokens."""
+        for its whole length are free; prompts enter in portions beside the running requests' tokens, a pass a step (no two run
+        together, as they do in one step over a whole prompt)."""
         out = [list(p) for p in prompts]
         need = [-(-(len(p) + max_new_tokens) // self.page_size) for p in prompts]
         for i, p in enumerate(prompts):
